@@ -1,0 +1,199 @@
+// Float32 matrix products out [M, N] (+)= a [M, K] w[N, K]^T (+ bias) on the matrix cores.
+//
+// The float32 matrix instruction multiplies and adds float32 values as fused multiply-adds in ascending k, subnormal
+// numbers included: 16x16x4 gives, bit for bit, the chain of fmaf that a thread would make (checked over normal products,
+// subnormal products and subnormal inputs).  So every output here is the sum over k ascending from zero whatever kernel,
+// tile or number of rows made it, and equals the tiled kernel's in gemm.hip, which serves what this file does not take
+// (K no multiple of 32, rows not 16-byte aligned): a row's result does not depend on what else is in the batch.
+#include "common.h"
+
+int lrs_gemm_f32(float* out, bool add, const float* a, const float* w, const float* bias, int m, int n, int k, int lda, int ldc, hipStream_t s);
+
+namespace {
+
+// Waits until at most PENDING fetches are on their way and this wave has what it read from LDS, then for the workgroup.
+template <int PENDING>
+__device__ __forceinline__ void fetched_and_read_then_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(PENDING) : "memory");
+}
+
+// Memory straight into LDS as fetch_to_lds (common.h) has it, for a base that the compiler holds in scalar registers already.
+__device__ __forceinline__ void fetch_from(uint64_t base, unsigned lane_offset, unsigned lds_address) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds_address), "v"(lane_offset), "s"(base) : "memory");
+}
+
+// WN x WM waves side by side along weight rows and input rows, TN x TM tiles of 16 x 16 outputs a wave; slices of BK of both
+// operands lie in LDS, written there by memory itself (STAGES slices).  A tile's rows lie piece by piece, the 16 bytes of its
+// rows at one place of K after each other: the 64 single floats that a fragment read takes (16 rows, four consecutive k) meet
+// every bank once, and all of a slice's reads go by one address register.  A slice's fragments are read into registers while
+// the slice before is multiplied, between the products: what a wave does besides them has to fit the 32 cycles of a 16x16x4,
+// for a wave whose sums are one chain has nothing else to wait for (K = 3,072 in 64 workgroups: 54 cycles a product with an
+// address worked out for every read and fetch).
+// WR, AR: 8 where a tile has only 8 rows of weights or inputs to bring (its other outputs are copies that nobody stores).
+// A wave's fragment of the weights is the instruction's first operand: its lanes end with four consecutive output columns.
+template <int BK, int WN, int WM, int TN, int TM, int STAGES, int WR, int AR>
+__global__ __launch_bounds__(WN * WM * WAVE) void gemm_f32_mfma_kernel(float* __restrict__ out, int add, const float* __restrict__ a,
+                                                                       const float* __restrict__ w, const float* __restrict__ bias, int m,
+                                                                       int n, int k, int lda, int ldc, int tiles_m, int wide_stores) {
+  static_assert((BK == 32 || BK == 64) && (WR == 8 || WR == 16) && (AR == 8 || AR == 16), "what the layout is made for");
+  constexpr int WAVES = WN * WM, BN = WN * TN * WR, BM = WM * TM * AR;
+  constexpr int CHUNKS = BK / 4;                                           // a row's pieces of 16 bytes
+  constexpr int STAGE = (BN + BM) * BK, EACH = (BN + BM) * BK / 256 / WAVES;   // floats; fetches a wave and slice (a fetch brings 64 pieces)
+  constexpr int W_FETCHES = CHUNKS * WR / 64, A_FETCHES = CHUNKS * AR / 64;    // for the rows of a tile
+  static_assert((BN + BM) * BK / 256 % WAVES == 0 && STAGES * EACH < 64, "every wave brings as much, counted in vmcnt");
+  __shared__ __attribute__((aligned(128))) float slices[STAGES * STAGE];
+  const int tid = threadIdx.x, lane = tid % WAVE, wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / WAVE);
+  int id = blockIdx.x;
+  if (gridDim.x % 8 == 0) id = (id % 8) * (gridDim.x / 8) + id / 8;        // an XCD takes neighbouring weight rows, which it then reads once
+  const int m0 = (id % tiles_m) * BM, n0 = (id / tiles_m) * BN;
+  unsigned offset[EACH];
+#pragma unroll
+  for (int i = 0; i < EACH; ++i) {
+    const int fetch = wave + i * WAVES;                                    // the weights' tiles first, then the inputs'
+    if (fetch < BN / WR * W_FETCHES) {
+      const int row = fetch / W_FETCHES * WR + lane % WR, chunk = fetch % W_FETCHES * (64 / WR) + lane / WR, last = n - 1 - n0;
+      offset[i] = ((unsigned)(row < last ? row : last) * (unsigned)k + (unsigned)chunk * 4u) * 4u;
+    } else {
+      const int mine = fetch - BN / WR * W_FETCHES;
+      const int row = mine / A_FETCHES * AR + lane % AR, chunk = mine % A_FETCHES * (64 / AR) + lane / AR, last = m - 1 - m0;
+      offset[i] = ((unsigned)(row < last ? row : last) * (unsigned)lda + (unsigned)chunk * 4u) * 4u;
+    }
+  }
+  const int steps = k / BK;
+  const unsigned slices_address = (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)slices + (unsigned)wave * 1024u;
+  uint64_t w_at = (uint64_t)(uintptr_t)(w + (int64_t)n0 * k), a_at = (uint64_t)(uintptr_t)(a + (int64_t)m0 * lda);   // of the slice to fetch next
+  auto fetch = [&](int stage, int i) {
+    const uint64_t base = wave + i * WAVES < BN / WR * W_FETCHES ? w_at : a_at;
+    fetch_from(base, offset[i], slices_address + (unsigned)(stage * (STAGE * 4) + i * WAVES * 1024));
+  };
+  auto advance = [&](int kt) {                                             // kt: the slice to fetch next; past the end the last one once more, read by nobody
+    const unsigned by = kt < steps ? BK * 4u : 0u;
+    w_at += by, a_at += by;
+  };
+  struct Fragments {
+    float w[CHUNKS][TN], a[CHUNKS][TM];
+  };
+  const int r = lane & 15, g = lane >> 4;
+  const int wave_n = (wave % WN) * TN * WR, wave_m = (wave / WN) * TM * AR;
+  const float* w_mine = slices + wave_n * BK + (r % WR) * 4 + g;
+  const float* a_mine = slices + (BN + wave_m) * BK + (r % AR) * 4 + g;
+  auto read = [&](int stage, int c, Fragments& f) {                       // four k of a slice
+#pragma unroll
+    for (int i = 0; i < TN; ++i) f.w[c][i] = w_mine[stage * STAGE + i * WR * BK + c * WR * 4];
+#pragma unroll
+    for (int j = 0; j < TM; ++j) f.a[c][j] = a_mine[stage * STAGE + j * AR * BK + c * AR * 4];
+  };
+  floatx4 acc[TN][TM];
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int kt = 0; kt < STAGES; ++kt) {
+#pragma unroll
+    for (int i = 0; i < EACH; ++i) fetch(kt, i);
+    advance(kt + 1);
+  }
+  Fragments even, odd;
+  fetched_and_read_then_barrier<(STAGES - 1) * EACH>();
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) read(0, c, even);
+  int stage = 0;                                                           // of slice kt
+  auto turn = [&](int kt, const Fragments& now, Fragments& next) {
+    // slice kt + 1 is there, and every wave holds slice kt in registers: its stage may be filled again
+    fetched_and_read_then_barrier<(STAGES - 2) * EACH>();
+    const int free = stage;
+    stage = stage == STAGES - 1 ? 0 : stage + 1;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      // the matrix unit works on these while the wave asks for the rest: reads in the first half, so that they are there by the end
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.w[c][i], now.a[c][j], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (c < CHUNKS / 2) read(stage, 2 * c, next), read(stage, 2 * c + 1, next);
+      if (c < EACH) fetch(free, c);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    advance(kt + STAGES + 1);
+  };
+  for (int kt = 0; kt < steps; kt += 2) {
+    turn(kt, even, odd);
+    if (kt + 1 < steps) turn(kt + 1, odd, even);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                         // the fetches past K
+#pragma unroll
+  for (int j = 0; j < TM; ++j) {
+    const int token = m0 + wave_m + j * AR + r;
+    if (token >= m || r >= AR) continue;
+#pragma unroll
+    for (int i = 0; i < TN; ++i) {
+      const int col = n0 + wave_n + i * WR + 4 * g;
+      if (4 * g >= WR) continue;
+      float* to = out + (int64_t)token * ldc + col;
+      floatx4 v = acc[i][j];
+      if (wide_stores && col + 3 < n) {
+        if (bias)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] += bias[col + e];
+        if (add) v = *(const floatx4*)to + v;
+        *(floatx4*)to = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (col + e >= n) break;
+          float x = v[e];
+          if (bias) x += bias[col + e];
+          to[e] = add ? to[e] + x : x;
+        }
+      }
+    }
+  }
+}
+
+// Measured on the MI355X (us; the FMA kernels that made the same sums before, 64 x 64 tiles and a thread an output):
+//   rows 509: N 4,096 K 1,024 39 (169 before), N 1,024 K 2,048 28 and K 3,072 38 (408 on average), N 6,144 K 1,024 56 (179);
+//   rows 2,048: N 24,576 K 4,096 2,978, 138 TFLOP/s of the 139 that the instruction alone reaches in a loop;
+//   rows 8: N 1,024 K 3,072 15.7 and K 2,048 11.3 (33.5 on average), N 4,096 K 1,024 9.9 (15.1), N 151,936 K 1,024 143 (141).
+// What bounds them: many rows the matrix units; few rows and few weight rows the chain of a sum, 13.3 ns for four k where nothing
+// else is in the way (16.5 here); the head memory.
+// What a launch of BN x BM tiles costs, by the outputs of the compute unit that has the most of them; `per_output` is how much
+// longer a small tile takes an output (it reads more from the L2s for each).
+int tile_cost(int m, int n, int bn, int bm, int per_output) {
+  const int tiles = ((n + bn - 1) / bn) * ((m + bm - 1) / bm);
+  return (tiles + 255) / 256 * (bn * bm / 64) * per_output;
+}
+
+}  // namespace
+
+// K % 32 == 0; a, w and rows of lda floats 16-byte aligned.
+int lrs_gemm_f32(float* out, bool add, const float* a, const float* w, const float* bias, int m, int n, int k, int lda, int ldc, hipStream_t s) {
+  const int wide_stores = ldc % 4 == 0 && (uintptr_t)out % 16 == 0;
+#define TILES(BK, WN, WM, TN, TM, STAGES, WR, AR)                                                                                  \
+  do {                                                                                                                             \
+    const int tiles_m = (m + WM * TM * AR - 1) / (WM * TM * AR), tiles_n = (n + WN * TN * WR - 1) / (WN * TN * WR);                \
+    gemm_f32_mfma_kernel<BK, WN, WM, TN, TM, STAGES, WR, AR><<<tiles_m * tiles_n, WN * WM * WAVE, 0, s>>>(                         \
+        out, add, a, w, bias, m, n, k, lda, ldc, tiles_m, wide_stores);                                                            \
+  } while (0)
+  if (m <= 16) {
+    // Few rows: memory and the chains bound it.  As many workgroups as there are tiles of 16 weight rows, of 8 where those are
+    // fewer than half the compute units (N under 2,048), with slices of 64 deep in flight; a head's many rows in workgroups of
+    // 64, which share the input rows (one wave a workgroup: 197 us, its tiles of 16 weight rows as half lines 147).
+    const bool pairs = k % 64 == 0, half = m <= 8;
+    if (n > 16384 && pairs) TILES(64, 4, 1, 2, 1, 4, 8, 16);
+    else if (!pairs) TILES(32, 1, 1, 1, 1, 15, 16, 16);
+    else if (n >= 2048) { if (half) TILES(64, 1, 1, 1, 1, 8, 16, 8); else TILES(64, 1, 1, 1, 1, 7, 16, 16); }
+    else if (half) TILES(64, 1, 1, 1, 1, 15, 8, 8);
+    else TILES(64, 1, 1, 1, 1, 10, 8, 16);
+  } else {
+    // Many rows: the tile whose busiest compute unit has least to do, small tiles marked up by what they measured
+    const int small = tile_cost(m, n, 16, 32, 18), middle = tile_cost(m, n, 64, 32, 13), large = tile_cost(m, n, 64, 64, 11), largest = tile_cost(m, n, 128, 128, 10);
+    if (small <= middle && small <= large && small <= largest) TILES(32, 1, 2, 1, 1, 12, 16, 16);
+    else if (middle <= large && middle <= largest) TILES(32, 2, 2, 2, 1, 8, 16, 16);
+    else if (large <= largest) TILES(32, 2, 2, 2, 2, 3, 16, 16);
+    else TILES(32, 2, 4, 4, 2, 3, 16, 16);
+  }
+#undef TILES
+  return 0;
+}
