@@ -1,0 +1,237 @@
+// Float32 attention over the paged cache on the matrix cores (the rules of attention.hip: what a token sees, the pages'
+// layout, rounding that depends on positions alone).
+//
+// The keys of a sequence are cut into pieces of 64 positions counted from position 0.  A wave takes a piece for up to 16
+// queries (tokens times the kv group's heads, the columns of its products): scores, their maximum, weights and weighted sum of
+// that piece alone, as if there were no other.  A query's result is its pieces' partial results merged one after the
+// other in the order of their positions, by the same operations however many queries
+// share a workgroup's eight waves, which take eight pieces at a time.
+//
+// A piece is 512 products of 32 cycles at 128 dims whatever columns are in use, 6.8 us for the two waves of a SIMD: that bounds a
+// prompt (2,048 tokens, 16 heads of 128: 305 us, 56 TFLOP/s; 3,174 us with a workgroup a (token, head) and plain FMAs) and,
+// with one trip to memory before it, a decode step (8 tokens at 509: 18 us, 35 before).  A block of 16 keys, and one of
+// values, is asked for while the one before is multiplied; the registers this takes leave one workgroup a compute unit.
+#include "common.h"
+
+int lrs_attention_f32(float* out, int out_stride, const float* q, int q_stride, const float* k_pages, const float* v_pages, const int* block_table,
+                      int table_stride, const int* token_request, const int* positions, int tokens, int nq, int nkv, int d, int page_size,
+                      float scale, int window, int together, hipStream_t s);
+bool lrs_attention_f32_takes(const void* out, int out_stride, const void* q, int q_stride, const void* k_pages, const void* v_pages, int nq, int nkv,
+                             int d, int dv, int page_size);
+
+namespace {
+
+constexpr int PIECE = 64, COLUMNS = 16, WAVES = 8;
+
+// What is left of a partial result when its reference point moves to `top`.
+__device__ __forceinline__ float moved(float from, float top) { return from == -INFINITY ? 0.f : expf(from - top); }
+
+// 16 keys' weighted values where some values are not finite (perhaps in slots that nothing was written to): such a value counts
+// only where its weight is not zero, which a product of tiles cannot tell.  It is left out of the products, and three more
+// products say which sums see an infinity or a NaN.
+__device__ __forceinline__ void add_odd_values(floatx4 values, floatx4 weights, floatx4& acc) {
+  floatx4 plus = {0.f, 0.f, 0.f, 0.f}, minus = plus, none = plus;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const float v = values[t], seen = weights[t] != 0.f ? 1.f : 0.f;
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(isfinite(v) ? v : 0.f, weights[t], acc, 0, 0, 0);
+    plus = __builtin_amdgcn_mfma_f32_16x16x4f32(v == INFINITY ? 1.f : 0.f, seen, plus, 0, 0, 0);
+    minus = __builtin_amdgcn_mfma_f32_16x16x4f32(v == -INFINITY ? 1.f : 0.f, seen, minus, 0, 0, 0);
+    none = __builtin_amdgcn_mfma_f32_16x16x4f32(v != v ? 1.f : 0.f, seen, none, 0, 0, 0);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (plus[e] > 0.f) acc[e] += INFINITY;
+    if (minus[e] > 0.f) acc[e] -= INFINITY;
+    if (none[e] > 0.f) acc[e] = NAN;
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// One workgroup: `together` tokens (as many as fit 16 columns with the kv group's heads) of one kv head, taken request by
+// request should they not all belong to one.
+template <int D>
+__global__ __launch_bounds__(WAVES * WAVE) void attention_f32_mfma_kernel(
+    float* __restrict__ out, int out_stride, const float* __restrict__ q, int q_stride, const float* __restrict__ k_pages,
+    const float* __restrict__ v_pages, const int* __restrict__ block_table, int table_stride, const int* __restrict__ token_request,
+    const int* __restrict__ positions, int tokens, int heads, int nkv, int page_size, float scale, int window, int together) {
+  constexpr int PITCH = D + 4, TILES = D / 16;   // floats from column to column of a partial result; its tiles of 16 dims
+  extern __shared__ __attribute__((aligned(16))) float parts[];           // [WAVES][columns][PITCH], then maxima and sums [WAVES][16][2]
+  const int columns = together * heads;
+  float* maxima = parts + WAVES * columns * PITCH;
+  const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int r = lane & 15, g = lane >> 4;
+  const int kv_head = blockIdx.y;
+  // the last tokens of a prompt, which see most, begin first
+  const int begin = ((int)gridDim.x - 1 - (int)blockIdx.x) * together, end = begin + together < tokens ? begin + together : tokens;
+  const unsigned key_lane = (unsigned)(r * D + 4 * g), value_lane = (unsigned)(r * page_size + 4 * g);     // floats from a block's first
+  const int my_token = begin + r / heads;                                  // of this lane's column
+  // the thread that merges: column and four dims
+  const int item = tid, item_column = item / (D / 4), item_dim = item % (D / 4) * 4;
+  for (int first = begin; first < end;) {
+    const int request = token_request[first];
+    int last = first + 1, highest = positions[first], lowest = first_seen(highest, window);
+    for (; last < end && token_request[last] == request; ++last) {
+      const int pos = positions[last], from = first_seen(pos, window);
+      highest = pos > highest ? pos : highest, lowest = from < lowest ? from : lowest;
+    }
+    const bool mine = r < columns && my_token >= first && my_token < last;
+    const int token = mine ? my_token : first, head = kv_head * heads + (mine ? r % heads : 0);
+    const int pos = mine ? positions[token] : -1, from = mine ? first_seen(pos, window) : 0;
+    const int* table = block_table + (int64_t)request * table_stride;
+    // the query, as the products' second operand: product 4 j + t multiplies dims 16 j + 4 g + t
+    floatx4 qf[TILES];
+#pragma unroll
+    for (int j = 0; j < TILES; ++j) qf[j] = *(const floatx4*)(q + (int64_t)token * q_stride + head * D + 16 * j + 4 * g);
+    float run_max = -INFINITY, run_sum = 0.f;
+    floatx4 run = {0.f, 0.f, 0.f, 0.f};
+    const int last_piece = highest / PIECE;
+    for (int piece0 = lowest / PIECE; piece0 <= last_piece; piece0 += WAVES) {
+      const int piece = piece0 + wave;
+      if (piece <= last_piece) {
+        floatx4 score[4], ahead[2][TILES];                                 // ahead: 16 keys, or their values, asked for a block ahead
+        int64_t page[4];                                                   // the (page, kv head) block of 16 keys, and the slot they begin at
+        int slot[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          // a block that nobody sees (perhaps without a page) stands for the nearest that somebody does: its weights will be zero
+          int key0 = piece * PIECE + b * 16;
+          key0 = key0 < (lowest & ~15) ? lowest & ~15 : key0 > (highest & ~15) ? highest & ~15 : key0;
+          page[b] = (int64_t)table[key0 / page_size] * nkv + kv_head;
+          slot[b] = key0 % page_size;
+        }
+        auto load_keys = [&](int b) {
+          const float* keys = k_pages + (page[b] * page_size + slot[b]) * D;
+#pragma unroll
+          for (int j = 0; j < TILES; ++j) ahead[b & 1][j] = *(const floatx4*)(keys + (key_lane + 16 * j));
+        };
+        auto load_values = [&](int b) {
+          const float* values = v_pages + page[b] * D * page_size + slot[b];                      // [dim][slot]
+#pragma unroll
+          for (int i = 0; i < TILES; ++i) ahead[b & 1][i] = *(const floatx4*)(values + (int64_t)(16 * i) * page_size + value_lane);
+        };
+        load_keys(0);
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          if (b < 3) load_keys(b + 1);
+          else load_values(0);
+          __builtin_amdgcn_sched_barrier(0);
+          score[b] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int j = 0; j < TILES; ++j)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) score[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(ahead[b & 1][j][t], qf[j][t], score[b], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        // this lane: keys 16 b + 4 g + t of its column
+        float top = -INFINITY;
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const int key = piece * PIECE + b * 16 + 4 * g + t;
+            score[b][t] = key <= pos && key >= from ? score[b][t] * scale : -INFINITY;
+            top = fmaxf(top, score[b][t]);
+          }
+        top = fmaxf(top, __shfl_xor(top, 16, WAVE));
+        top = fmaxf(top, __shfl_xor(top, 32, WAVE));
+        float sum = 0.f;
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const int key = piece * PIECE + b * 16 + 4 * g + t;
+            score[b][t] = key <= pos && key >= from ? expf(score[b][t] - top) : 0.f;
+            sum += score[b][t];
+            if (t == 3) __builtin_amdgcn_sched_barrier(0);
+          }
+        sum += __shfl_xor(sum, 16, WAVE);
+        sum += __shfl_xor(sum, 32, WAVE);
+        floatx4 acc[TILES];
+#pragma unroll
+        for (int i = 0; i < TILES; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          if (b < 3) load_values(b + 1);
+          __builtin_amdgcn_sched_barrier(0);
+          const floatx4(&vf)[TILES] = ahead[b & 1];
+          float finite = 0.f;
+#pragma unroll
+          for (int i = 0; i < TILES; ++i)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) finite = fmaf(vf[i][t], 0.f, finite);
+          if (__any(finite != 0.f)) {
+#pragma unroll
+            for (int i = 0; i < TILES; ++i) add_odd_values(vf[i], score[b], acc[i]);
+          } else {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+              for (int i = 0; i < TILES; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][t], score[b][t], acc[i], 0, 0, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (r < columns) {
+          float* to = parts + (wave * columns + r) * PITCH + 4 * g;
+#pragma unroll
+          for (int i = 0; i < TILES; ++i) *(floatx4*)(to + 16 * i) = acc[i];
+          if (g == 0) maxima[(wave * COLUMNS + r) * 2] = top, maxima[(wave * COLUMNS + r) * 2 + 1] = sum;
+        }
+      }
+      __syncthreads();
+      if (item_column < columns) {
+        const int here = last_piece - piece0 + 1 < WAVES ? last_piece - piece0 + 1 : WAVES;
+        for (int p = 0; p < here; ++p) {
+          const float top = maxima[(p * COLUMNS + item_column) * 2], sum = maxima[(p * COLUMNS + item_column) * 2 + 1];
+          const floatx4 part = *(const floatx4*)(parts + (p * columns + item_column) * PITCH + item_dim);
+          const float now = fmaxf(run_max, top), keep = moved(run_max, now), take = moved(top, now);
+          run_sum = fmaf(run_sum, keep, sum * take);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) run[e] = fmaf(run[e], keep, part[e] * take);
+          run_max = now;
+        }
+      }
+      __syncthreads();
+    }
+    const int item_token = begin + item_column / heads;
+    if (item_column < columns && item_token >= first && item_token < last) {
+      const float inv = 1.f / run_sum;
+      *(floatx4*)(out + (int64_t)item_token * out_stride + (kv_head * heads + item_column % heads) * D + item_dim) = run * inv;
+    }
+    first = last;
+  }
+}
+
+template <int D>
+void launch(float* out, int out_stride, const float* q, int q_stride, const float* k_pages, const float* v_pages, const int* block_table, int table_stride,
+            const int* token_request, const int* positions, int tokens, int heads, int nkv, int page_size, float scale, int window, int together,
+            hipStream_t s) {
+  const dim3 grid((tokens + together - 1) / together, nkv);
+  const int columns = together * heads;
+  attention_f32_mfma_kernel<D><<<grid, WAVES * WAVE, sizeof(float) * WAVES * (columns * (D + 4) + COLUMNS * 2), s>>>(
+      out, out_stride, q, q_stride, k_pages, v_pages, block_table, table_stride, token_request, positions, tokens, heads, nkv, page_size, scale, window, together);
+}
+
+}  // namespace
+
+bool lrs_attention_f32_takes(const void* out, int out_stride, const void* q, int q_stride, const void* k_pages, const void* v_pages, int nq, int nkv,
+                             int d, int dv, int page_size) {
+  const uintptr_t places = (uintptr_t)out | (uintptr_t)q | (uintptr_t)k_pages | (uintptr_t)v_pages;
+  return d == dv && (d == 32 || d == 64 || d == 96 || d == 128) && nq / nkv <= COLUMNS && page_size % 16 == 0 && places % 16 == 0 && out_stride % 4 == 0 && q_stride % 4 == 0;
+}
+
+// together: the most consecutive tokens that may share a workgroup (1: a step in which every request brings one token).
+int lrs_attention_f32(float* out, int out_stride, const float* q, int q_stride, const float* k_pages, const float* v_pages, const int* block_table,
+                      int table_stride, const int* token_request, const int* positions, int tokens, int nq, int nkv, int d, int page_size,
+                      float scale, int window, int together, hipStream_t s) {
+  const int heads = nq / nkv, fit = COLUMNS / heads;
+  if (together > fit) together = fit;
+  if (together < 1) together = 1;
+#define SIZE(D) launch<D>(out, out_stride, q, q_stride, k_pages, v_pages, block_table, table_stride, token_request, positions, tokens, heads, nkv, page_size, scale, window, together, s)
+  if (d == 32) SIZE(32);
+  else if (d == 64) SIZE(64);
+  else if (d == 96) SIZE(96);
+  else SIZE(128);
+#undef SIZE
+  return lrs_check_launch("attention");
+}

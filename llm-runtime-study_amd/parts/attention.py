@@ -364,9 +364,21 @@ class GQAAttention(Part):
                                   ctx.qblock_token0, ctx.qblock_count, nq, self.scale, self.reach, ctx.max_qblock, ctx.max_k_bound,
                                   splits, part_o, part_ml, queries_raw)
         else:
-            ops.attention(out, qkv, cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot, ctx.positions,
-                          nq, self.scale, self.reach)
+            self._attend(ctx, out, qkv, cache, group)
         return linear(ctx, residual, out, self.w_o, accumulate=accumulate, then_norm=then_norm)
+
+    def _attend(self, ctx, out, qkv, cache, group, gates=None, **more):
+        """Attention by the kernels for any shape and dtype; the single tokens at the head of a mixed step (each of a request of
+        its own) in a launch of their own, so that a prompt's tokens behind them share workgroups."""
+        singles = 0 if ctx.all_decode else ctx.single_rows
+        if not singles:
+            ops.attention(out, qkv, cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot, ctx.positions, self.num_heads, self.scale,
+                          self.reach, self.keep_first, gates=gates, together=1 if ctx.all_decode else 16, **more)
+            return
+        for first, end, together in ((0, singles, 1), (singles, out.shape[0], 16)):
+            ops.attention(out[first:end], qkv[first:end], cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot[first:end],
+                          ctx.positions[first:end], self.num_heads, self.scale, self.reach, self.keep_first,
+                          gates=None if gates is None else gates[first:end], together=together, **more)
 
     def _forward_whole_rows(self, ctx, x, residual, cache, group, cos, sin, then_norm, accumulate):
         """The forms whose heads `qkv_norm_prep` prepares: one product for q, k, v (and the gate), the norms over the whole
@@ -432,8 +444,7 @@ class GQAAttention(Part):
                                   ctx.qblock_token0, ctx.qblock_count, nq, self.scale, self.reach, ctx.max_qblock, ctx.max_k_bound,
                                   splits, part_o, part_ml, None, keep_first=self.keep_first, gates=None if gates is None else gates[singles:], **more)
         else:
-            ops.attention(out, qkv, cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot, ctx.positions, nq, self.scale,
-                          self.reach, self.keep_first, gates=gates, **more)
+            self._attend(ctx, out, qkv, cache, group, gates=gates, **more)
         if self.output_gate is True:
             ops.sigmoid_gate(out, qkv[:, gate_at:gate_at + self.gate_width])
         return linear(ctx, residual, out, self.w_o, accumulate=accumulate, then_norm=then_norm)

@@ -1,5 +1,8 @@
-"""The float32 products on the matrix cores, alone: against float64 and, bit for bit, against the kernel for any shape (which a
-row stride that is no multiple of four sends them to)."""
+"""The float32 kernels on the matrix cores, alone: products against float64 and, bit for bit, against the kernel for any shape
+(which a row stride that is no multiple of four sends them to); attention against float64, and the same bits however the
+queries share workgroups."""
+
+import math
 
 import pytest
 import torch
@@ -44,3 +47,71 @@ def test_float32_product(ops, m, n, k):
     ops.gemm(strided[:, :n], a, w, accumulate=True)
     ops.gemm(plain, wide[:, :k], w)
     assert torch.equal(added, plain + 0.25) and torch.equal(strided[:, :n], added) and (strided[:, n:] == 0.25).all()
+
+
+# (cached tokens, new tokens): pieces of 64 keys cut at every place, several requests among 16 neighbouring tokens, more pieces
+# than a workgroup has waves
+REQUESTS = [(0, 70), (130, 1), (63, 2), (600, 17), (1030, 3), (64, 1)]
+
+
+@pytest.mark.parametrize("nq,nkv,d,page,window", [(4, 2, 128, 16, 0), (8, 2, 64, 32, 0), (3, 1, 96, 16, 40), (16, 1, 32, 48, 0), (2, 2, 128, 64, 130), (6, 2, 64, 16, -128)])
+def test_float32_attention(ops, nq, nkv, d, page, window):
+    g = torch.Generator().manual_seed(nq * 31 + d)
+    blocks = [-(-(a + b) // page) for a, b in REQUESTS]
+    perm = torch.randperm(sum(blocks) + 2, generator=g).tolist()
+    # slots that nothing was written to hold what they like
+    k_pages, v_pages = torch.full((len(perm), nkv, page, d), float("nan")), torch.full((len(perm), nkv, d, page), float("inf"))
+    table = torch.full((len(REQUESTS), max(blocks)), -1, dtype=torch.int32)
+    rows, of, at, want = [], [], [], []
+    for r, (before, new) in enumerate(REQUESTS):
+        k, v, q = (torch.randn(before + new, nkv, d, generator=g) for _ in range(2)), None, torch.randn(new, nq, d, generator=g) * 2
+        k, v = k
+        for b in range(blocks[r]):
+            table[r, b] = perm.pop()
+            n = min(page, before + new - b * page)
+            k_pages[table[r, b], :, :n] = k[b * page:b * page + n].transpose(0, 1)
+            v_pages[table[r, b], :, :, :n] = v[b * page:b * page + n].permute(1, 2, 0)
+        for i in range(new):
+            pos = before + i
+            first = 0 if window == 0 else max(0, pos - window + 1) if window > 0 else pos - pos % -window
+            keys, values = (t[first:pos + 1].double().repeat_interleave(nq // nkv, 1) for t in (k, v))
+            share = torch.softmax(torch.einsum("khd,hd->hk", keys, q[i].double()) / math.sqrt(d), -1)
+            want.append(torch.einsum("hk,khd->hd", share, values).flatten())
+        rows.append(q.reshape(new, nq * d))
+        of += [r] * new
+        at += list(range(before, before + new))
+    q, want = torch.cat(rows), torch.stack(want)
+    wide = torch.zeros(len(q), nq * d + 8)
+    wide[:, :nq * d] = q
+    wide, k_pages, v_pages, table, of, at = dev(wide), dev(k_pages), dev(v_pages), dev(table), dev(torch.tensor(of, dtype=torch.int32)), dev(torch.tensor(at, dtype=torch.int32))
+    results = []
+    for together in (16, 1, 5):
+        out = torch.empty(len(q), nq * d, device="cuda")
+        ops.attention(out, wide, k_pages, v_pages, table, of, at, nq, 1 / math.sqrt(d), window, together=together)
+        results.append(out)
+    # scores of size s are off by at most (d + 2) 2^-24 |q||k| scale (here below 2e-5), weights by as much in proportion, sums likewise
+    torch.testing.assert_close(results[0].cpu().double(), want, rtol=2e-5, atol=2e-5)
+    assert torch.equal(results[0], results[1]) and torch.equal(results[0], results[2])
+
+
+def test_float32_attention_keeps_odd_values_to_those_who_see_them(ops):
+    """An infinite value and a NaN in a prompt: tokens before them give what they give without them, those behind see them."""
+    g = torch.Generator().manual_seed(3)
+    n, d = 90, 64
+    q, k, v = (torch.randn(n, d, generator=g) for _ in range(3))
+    pages, table, of, at = -(-n // 16), torch.arange(-(-n // 16), dtype=torch.int32)[None], torch.zeros(n, dtype=torch.int32), torch.arange(n, dtype=torch.int32)
+
+    def run(v):
+        k_pages, v_pages = torch.zeros(pages * 16, d), torch.zeros(pages * 16, d)
+        k_pages[:n], v_pages[:n] = k, v
+        out = torch.empty(n, d, device="cuda")
+        ops.attention(out, dev(q), dev(k_pages.view(pages, 1, 16, d)), dev(v_pages.view(pages, 1, 16, d).transpose(2, 3).contiguous()), dev(table), dev(of), dev(at),
+                      1, 0.125, together=16)
+        return out.cpu()
+
+    plain, odd = run(v), v.clone()
+    odd[50, 7], odd[71, 9], odd[73, 8] = float("inf"), float("nan"), float("-inf")
+    got = run(odd)
+    expected = plain.clone()
+    expected[50:, 7], expected[71:, 9], expected[73:, 8] = float("inf"), float("nan"), float("-inf")
+    assert torch.equal(got.nan_to_num(nan=12345.0), expected.nan_to_num(nan=12345.0))
