@@ -1280,7 +1280,14 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void attention_prefill_bf16_
 // nothing, a cap (softcap * tanh(score / softcap) of the scaled scores), a bias by distance (in the form with a logarithm, or the
 // linear one, which without a cap is what the products are added to and costs nothing), or the cap and then the bias.
 enum { SCORES_PLAIN = 0, SCORES_CAPPED = 1, SCORES_DISTANCE = 2, SCORES_BOTH = 3, SCORES_LINEAR = 4, SCORES_CAPPED_LINEAR = 5 };
-template <int QB, bool MANY_WAVES, bool IDLE_WAVES, int SCORES>
+// SPREAD: how a kv group's heads meet the waves: a wave a head (in several passes if there are more heads than waves); the same with
+// waves that have no head in some pass; and for two heads, which left half of the waves idle, a wave a (head, block of 16 queries) or,
+// where neighbouring groups are one request's, a wave a (head, group of 32).  A turn of the walk is bound by its tile's way from the
+// L2s (16 KB a turn and workgroup, 9 TB/s with two workgroups a unit), so a pair walking together does twice as much with it:
+// 16 heads on 8, 2,048 tokens after 14,336: 569 us with idle waves, 444 with halves, 322 in pairs with the keys divided by two;
+// 8,192 tokens 584 / 385 / 390; 2,048 after 2,048 142 / 136 / 100.
+enum { SPREAD_HEADS = 0, SPREAD_SOME_IDLE = 1, SPREAD_HALVES = 2, SPREAD_PAIRS = 3 };
+template <int QB, bool MANY_WAVES, int SPREAD, int SCORES>
 __global__ __launch_bounds__(MANY_WAVES ? 512 : 256, MANY_WAVES ? 1 : QB == 1 && (SCORES & SCORES_LINEAR) ? 3 : 2) void attention_prefill_d128_bf16_kernel(
     bf16* __restrict__ out, int out_stride, const bf16* __restrict__ q, int q_stride,
     const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
@@ -1291,6 +1298,9 @@ __global__ __launch_bounds__(MANY_WAVES ? 512 : 256, MANY_WAVES ? 1 : QB == 1 &&
     const float* __restrict__ sinks, float softcap, const bf16* __restrict__ gates, int gate_stride, int dv,
     const float* __restrict__ distance) {
   constexpr bool CAPPED = (SCORES & SCORES_CAPPED) != 0, DISTANCE = (SCORES & SCORES_DISTANCE) != 0, LINEAR = (SCORES & SCORES_LINEAR) != 0;
+  constexpr bool IDLE_WAVES = SPREAD == SPREAD_SOME_IDLE, HALVES = SPREAD == SPREAD_HALVES, PAIRS = SPREAD == SPREAD_PAIRS;
+  static_assert(!HALVES || (QB == 1 && !MANY_WAVES), "two heads and two blocks of 16 queries are four waves' work");
+  static_assert(!PAIRS || (QB == 2 && !MANY_WAVES), "two heads and two groups of 32 queries are four waves' work");
   constexpr int D = 128, DS = D / 32, DB = D / 16, STAGES = 3;
   constexpr int KBLOCK = 1024 + 32, KBYTES = 8 * KBLOCK, VHALF = 16 * D * 2 + 16, VBYTES = 2 * VHALF;
   constexpr int VSTAGE = (VBYTES + 63) / 64 * 64;
@@ -1301,14 +1311,18 @@ __global__ __launch_bounds__(MANY_WAVES ? 512 : 256, MANY_WAVES ? 1 : QB == 1 &&
   const int col = lane & 15, g = lane >> 4;
   const int key_chunk = ((g & 1) << 1) | (g >> 1);                 // m: the eight keys this lane group holds weights of
   const int group = nq / nkv;
-  const int work = blockIdx.x % (n_blocks * nkv), split = blockIdx.x / (n_blocks * nkv);
+  const int n_walks = PAIRS ? (n_blocks + 1) / 2 : n_blocks;       // PAIRS: two neighbouring groups of one request walk together
+  const int work = blockIdx.x % (n_walks * nkv), split = blockIdx.x / (n_walks * nkv);
   const int which_chunk = work / chunk, in_chunk = work % chunk;
   const int chunk_block0 = which_chunk * (chunk / nkv);
-  const int chunk_blocks = n_blocks - chunk_block0 < chunk / nkv ? n_blocks - chunk_block0 : chunk / nkv;
+  const int chunk_blocks = n_walks - chunk_block0 < chunk / nkv ? n_walks - chunk_block0 : chunk / nkv;
   const int kvh = in_chunk % nkv;
-  const int qblock = chunk_block0 + ((which_chunk & 1) ? chunk_blocks - 1 - in_chunk / nkv : in_chunk / nkv);
-  const int token0 = qblock_token0[qblock], count = qblock_count[qblock];
-  const int pos_first = positions[token0], pos_last = positions[token0 + count - 1];
+  const int walk = chunk_block0 + ((which_chunk & 1) ? chunk_blocks - 1 - in_chunk / nkv : in_chunk / nkv);
+  // groups stand from a request's last tokens to its first
+  const int later = PAIRS ? 2 * walk : walk, earlier = PAIRS && later + 1 < n_blocks ? later + 1 : later;
+  const int qblock = PAIRS && wave >= 2 ? earlier : later;
+  const int token0 = qblock_token0[qblock], count = PAIRS && wave >= 2 && earlier == later ? 0 : qblock_count[qblock];
+  const int pos_first = positions[qblock_token0[earlier]], pos_last = positions[qblock_token0[later] + qblock_count[later] - 1];
   const int lo_first = first_seen(pos_first, window);
   const int lo_last = first_seen(pos_last, window);
   const int* table = block_table + (int64_t)token_request[token0] * table_stride;
@@ -1392,8 +1406,12 @@ __global__ __launch_bounds__(MANY_WAVES ? 512 : 256, MANY_WAVES ? 1 : QB == 1 &&
 
   // kv groups of more than four heads take several passes over the keys
   const int waves = blockDim.x / WAVE;
+  // two heads: a wave has one of them and one of the group's two blocks of 16 queries (beginning at query0), or one of two groups
+  const int query0 = HALVES ? (wave >> 1) * 16 : 0;
+  // waves without a head sit on other SIMDs in the workgroup that shares the compute unit (the 256th from here)
+  const int my_wave = HALVES || PAIRS ? wave & 1 : IDLE_WAVES && !MANY_WAVES ? (wave + (blockIdx.x >> 8 & 1) * 2) & 3 : wave;
   for (int head0 = kvh * group; head0 < (kvh + 1) * group; head0 += waves) {
-    const int head = head0 + wave;
+    const int head = head0 + my_wave;
     const bool active = head < (kvh + 1) * group;
     bf16x8 qf[QB][DS];
     floatx4 o[QB][DB];
@@ -1402,8 +1420,8 @@ __global__ __launch_bounds__(MANY_WAVES ? 512 : 256, MANY_WAVES ? 1 : QB == 1 &&
     bool live[QB];
 #pragma unroll
     for (int b = 0; b < QB; ++b) {
-      live[b] = active && b * 16 + col < count;
-      const int token = token0 + (live[b] ? b * 16 + col : 0);
+      live[b] = active && query0 + b * 16 + col < count;
+      const int token = token0 + (live[b] ? query0 + b * 16 + col : 0);
       pos[b] = live[b] ? positions[token] : -1;                // a dead column sees no key
       lo[b] = first_seen(pos[b], window);
       run_max[b] = -INFINITY;
@@ -1739,7 +1757,7 @@ __global__ __launch_bounds__(MANY_WAVES ? 512 : 256, MANY_WAVES ? 1 : QB == 1 &&
       total += __shfl_xor(total, 16, WAVE);
       total += __shfl_xor(total, 32, WAVE);
       if (live[b] && slots > 1) {
-        const int64_t slot = ((int64_t)(token0 + b * 16 + col) * nq + head) * slots + split;
+        const int64_t slot = ((int64_t)(token0 + query0 + b * 16 + col) * nq + head) * slots + split;
 #pragma unroll
         for (int e = 0; e < DB; ++e)
           if (e * 16 < dv) *(floatx4*)(part_o + slot * dv + e * 16 + g * 4) = o[b][e];
@@ -1749,8 +1767,8 @@ __global__ __launch_bounds__(MANY_WAVES ? 512 : 256, MANY_WAVES ? 1 : QB == 1 &&
         }
       } else if (live[b]) {
         const float keep = sinks ? with_sink(sinks[head] * LOG2E, run_max[b] * scale2, total) : 1.f;
-        const float inv = keep / total * head_gate(gates, gate_stride, token0 + b * 16 + col, head);
-        bf16* dst = out + (int64_t)(token0 + b * 16 + col) * out_stride + (int64_t)head * dv + g * 4;
+        const float inv = keep / total * head_gate(gates, gate_stride, token0 + query0 + b * 16 + col, head);
+        bf16* dst = out + (int64_t)(token0 + query0 + b * 16 + col) * out_stride + (int64_t)head * dv + g * 4;
 #pragma unroll
         for (int e = 0; e < DB; ++e) {
           if (e * 16 >= dv) break;
@@ -1809,7 +1827,7 @@ LRS_API int lrs_attention_prefill(void* out, int out_stride, const void* q, int 
                                   int nkv, int d, int page_size, float scale, int window, int keep_first, int tokens, int splits,
                                   float* part_o, float* part_ml, int prepare, const void* q_weight, int w_dtype, float eps,
                                   const float* cosv, const float* sinv, const float* sinks, float softcap, const void* gates,
-                                  int gate_stride, int dv, const float* distance, int distance_form, void* stream) {
+                                  int gate_stride, int dv, const float* distance, int distance_form, int one_request, void* stream) {
   LRS_REQUIRE(distance_form == DISTANCE_LOG || distance_form == DISTANCE_LINEAR, "attention_prefill: unknown form %d of the bias by distance", distance_form);
   LRS_REQUIRE(dv > 0 && dv % 16 == 0 && dv <= d, "attention_prefill: values of %d dims beside keys of %d are not served (a multiple of 16, at most the keys')", dv, d);
   LRS_REQUIRE(n_blocks > 0 && nq > 0 && nkv > 0 && nq % nkv == 0, "attention_prefill: bad sizes blocks=%d nq=%d nkv=%d", n_blocks, nq, nkv);
@@ -1872,26 +1890,30 @@ LRS_API int lrs_attention_prefill(void* out, int out_stride, const void* q, int 
       {
         const bool many = nq / nkv > 4 && (int64_t)n_blocks * nkv * splits <= 2 * compute_units();
         if (many) block = dim3((nq / nkv < 8 ? nq / nkv : 8) * WAVE);
-#define D128(QB, MANY, IDLE)                                                                                                      \
+#define D128(QB, MANY, SPREAD)                                                                                                      \
         const bool linear = distance && distance_form == DISTANCE_LINEAR;                                                             \
-        if (softcap > 0.f && linear) D128C(QB, MANY, IDLE, SCORES_CAPPED_LINEAR);                                                     \
-        else if (linear) D128C(QB, MANY, IDLE, SCORES_LINEAR);                                                                        \
-        else if (softcap > 0.f && distance) D128C(QB, MANY, IDLE, SCORES_BOTH);                                                       \
-        else if (softcap > 0.f) D128C(QB, MANY, IDLE, SCORES_CAPPED);                                                                 \
-        else if (distance) D128C(QB, MANY, IDLE, SCORES_DISTANCE);                                                                    \
-        else D128C(QB, MANY, IDLE, SCORES_PLAIN)
-#define D128C(QB, MANY, IDLE, SCORES)                                                                                             \
-        attention_prefill_d128_bf16_kernel<QB, MANY, IDLE, SCORES><<<grid, block, 0, s>>>(                                            \
+        if (softcap > 0.f && linear) D128C(QB, MANY, SPREAD, SCORES_CAPPED_LINEAR);                                                     \
+        else if (linear) D128C(QB, MANY, SPREAD, SCORES_LINEAR);                                                                        \
+        else if (softcap > 0.f && distance) D128C(QB, MANY, SPREAD, SCORES_BOTH);                                                       \
+        else if (softcap > 0.f) D128C(QB, MANY, SPREAD, SCORES_CAPPED);                                                                 \
+        else if (distance) D128C(QB, MANY, SPREAD, SCORES_DISTANCE);                                                                    \
+        else D128C(QB, MANY, SPREAD, SCORES_PLAIN)
+#define D128C(QB, MANY, SPREAD, SCORES)                                                                                             \
+        attention_prefill_d128_bf16_kernel<QB, MANY, SPREAD, SCORES><<<grid, block, 0, s>>>(                                            \
             (bf16*)out, out_stride, (const bf16*)q, q_stride, (const bf16*)k_pages, (const bf16*)v_pages, block_table, table_stride, \
             token_request, positions, qblock_token0, qblock_count, n_blocks, chunk, nq, nkv, page_size, scale, window, splits, slots, part_o, part_ml, \
             prepare, prep, own_sinks, softcap, own_gates, gate_stride, dv, distance)
 #define D128_OF(QB)                                        \
-        if (many && idle) { D128(QB, true, true); }        \
-        else if (many) { D128(QB, true, false); }          \
-        else if (idle) { D128(QB, false, true); }          \
-        else { D128(QB, false, false); }
+        if (many && idle) { D128(QB, true, SPREAD_SOME_IDLE); }  \
+        else if (many) { D128(QB, true, SPREAD_HEADS); }         \
+        else if (idle) { D128(QB, false, SPREAD_SOME_IDLE); }    \
+        else { D128(QB, false, SPREAD_HEADS); }
         const bool idle = (nq / nkv) % (int)(block.x / WAVE) != 0;   // some wave of some pass has no head
         if (max_count <= 16) { D128_OF(1); }
+        else if (nq / nkv == 2 && one_request) {
+          grid = dim3((n_blocks + 1) / 2 * nkv * splits);
+          D128(2, false, SPREAD_PAIRS);
+        } else if (nq / nkv == 2) { D128(1, false, SPREAD_HALVES); }
         else { D128_OF(2); }
 #undef D128_OF
 #undef D128

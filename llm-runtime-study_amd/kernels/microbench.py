@@ -67,7 +67,7 @@ def attention_prefill(args) -> None:
                 part_ml = torch.empty(tokens, nq * splits * 2, device="cuda") if splits > 1 else None
                 seconds = _time(lambda i: ops.attention_prefill(out, q, k_pages, v_pages, table, request, positions, token0, count,
                                                                 nq, 1 / math.sqrt(d), args.window, size, before + tokens,
-                                                                splits, part_o, part_ml), args.repeats)
+                                                                splits, part_o, part_ml, one_request=True), args.repeats)
                 print(f"attention_prefill tokens={tokens} after={before} group={size} splits={splits}: {seconds * 1e6:9.1f} us  "
                       f"{flops / seconds / 1e12:7.1f} TFLOP/s (keys a query may see)", flush=True)
 

@@ -155,7 +155,7 @@ _SIGNATURES = {
                                      c_void_p, c_void_p, c_int, c_float, c_void_p, c_void_p, c_int, c_void_p, c_float, c_void_p, c_int, c_int, c_void_p, c_int, c_void_p]),
     "lrs_attention_prefill": (c_int, [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                                       c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int,
-                                      c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_int, c_float, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int, c_int, c_void_p, c_int, c_void_p]),
+                                      c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_int, c_float, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_void_p]),
     "lrs_attention_prefill_prepares": (c_int, [c_int]),
     "lrs_compute_units": (c_int, []),
     "lrs_gemm_lines_width": (c_int, [c_int, c_int, c_int]),
@@ -1277,7 +1277,8 @@ def attention_prefill(out: torch.Tensor, q: torch.Tensor, k_pages: torch.Tensor,
                       nq: int, scale: float, window: int = 0, max_count: int | None = None, max_context: int | None = None,
                       splits: int = 1, part_o: torch.Tensor | None = None, part_ml: torch.Tensor | None = None,
                       prepare: "DecodePrepare | None" = None, keep_first: int = 0, sinks: torch.Tensor | None = None,
-                      softcap: float = 0.0, gates: torch.Tensor | None = None, distance: torch.Tensor | None = None) -> None:
+                      softcap: float = 0.0, gates: torch.Tensor | None = None, distance: torch.Tensor | None = None,
+                      one_request: bool = False) -> None:
     """attention() on matrix cores for any bfloat16 step.  qblock_token0 / qblock_count list groups of at
     most attention_prefill_group() consecutive tokens of one request that together cover every token of
     the step once; `max_count` is the largest count among them (the group limit if not given) and
@@ -1288,7 +1289,9 @@ def attention_prefill(out: torch.Tensor, q: torch.Tensor, k_pages: torch.Tensor,
     them their norm and rotation itself (q_weight, eps, cos, sin of DecodePrepare; kv_heads 0: the keys and values are in
     the pages already, from qk_prep(skip_q=True)).
     keep_first (with a window and prepared heads): the first positions of a sequence stay visible behind the window; their
-    share is one more partial result, so the buffers hold splits + 1 and are needed whatever `splits` is."""
+    share is one more partial result, so the buffers hold splits + 1 and are needed whatever `splits` is.
+    one_request: the groups are one request's, listed from its last tokens to its first without a gap, so that neighbouring
+    ones may walk their keys together (a matter of speed)."""
     tokens = out.shape[0]
     _need(k_pages.dim() == 4 and k_pages.is_contiguous() and v_pages.is_contiguous(), "attention_prefill: pages must be contiguous")
     _, nkv, page_size, d = k_pages.shape
@@ -1329,7 +1332,7 @@ def attention_prefill(out: torch.Tensor, q: torch.Tensor, k_pages: torch.Tensor,
         block_table.shape[1] * page_size if max_context is None else max_context, nq, nkv, d, page_size, scale, window, keep_first,
         tokens, splits, None if slots == 1 else _dev(part_o, "part_o"), None if slots == 1 else _dev(part_ml, "part_ml"), *fused,
         _sinks(sinks, nq, "attention_prefill"), float(softcap), *_gates(gates, tokens, nq, q.dtype, "attention_prefill"), dv,
-        *_distance(distance, nq, "attention_prefill"), _stream())
+        *_distance(distance, nq, "attention_prefill"), 1 if one_request else 0, _stream())
 
 
 def attention_prefill_prepares(d: int) -> bool:

@@ -228,7 +228,13 @@ class GQAAttention(Part):
         return max(1, min(wanted, length_class(longest) // 256, 64), -(-bound // (4096 * page_size)))
 
     @staticmethod
-    def _prefill_splits(workgroups: int, longest: int, outputs: int, heads_per_group: int = 4, tokens: int = 0) -> int:
+    def _walks_in_pairs(ctx, heads_per_group: int, head_dim: int) -> bool:
+        """Whether the kernel for ragged steps lets two neighbouring query groups walk their keys together (attention_prefill's
+        `one_request`): two heads a kv group, groups of more than 16 tokens, all of one request."""
+        return heads_per_group == 2 and head_dim == 128 and ctx.max_qblock > 16 and ctx.R - ctx.single_rows == 1
+
+    @staticmethod
+    def _prefill_splits(workgroups: int, longest: int, outputs: int, heads_per_group: int = 4, tokens: int = 0, paired: bool = False) -> int:
         """Into how many workgroups the keys of every query group of a ragged step are divided: one, unless
         the groups alone leave compute units idle (a last portion of a prompt, a short portion after a long
         context), and never from two workgroups a unit on.  Partial results (float32, `outputs` values per split)
@@ -252,6 +258,14 @@ class GQAAttention(Part):
         for long contexts holds for them too (512 tokens after 32,256: 697 us undivided, 617 with 8)."""
         units = ops.compute_units()
         within = (64 << 20) // max(outputs, 1)
+        if paired:
+            # Two heads a kv group, groups of 32 that walk in pairs (csrc/attention.hip, SPREAD_PAIRS): a walk is as long as its keys
+            # whatever it works on, so two workgroups a unit are the aim behind any context (16 heads on 8: 2,048 tokens after 14,336
+            # 567 us undivided, 322 with 2, 382 with 3, 313 with 4; after 2,048 136 / 100 / - / 103; 1,024 after 15,360 551 us
+            # undivided, 290 / 178 / 184 with 2 / 4 / 8; but 8,192 tokens, two a unit without, 390 and 404 with 2)
+            if workgroups >= 2 * units:
+                return 1
+            return max(1, min(-(-2 * units // workgroups), longest // 256, 32, within))
         if workgroups >= 2 * units:      # (2,048 tokens in groups of 32 after 30,720: 1,071 us undivided, 1,115 with 2)
             return 1
         if longest < 16384 and longest < 4 * tokens:
@@ -355,14 +369,16 @@ class GQAAttention(Part):
                 rest = ctx.memo["rows_after_singles"] = (ctx.token_slot[singles:], ctx.positions[singles:])
             if queries_raw is not None and singles and cos is not None:
                 queries_raw = ops.DecodePrepare(self.q_norm, None, self.qk_norm_eps, parted[2], parted[3], 0)
-            splits = self._prefill_splits(ctx.num_qblocks * kv_heads, longest, (t - singles) * nq * d, nq // kv_heads, t - singles)
+            paired = self._walks_in_pairs(ctx, nq // kv_heads, d)
+            splits = self._prefill_splits((-(-ctx.num_qblocks // 2) if paired else ctx.num_qblocks) * kv_heads, longest, (t - singles) * nq * d,
+                                          nq // kv_heads, t - singles, paired)
             part_o = part_ml = None
             if splits > 1:
                 part_o = ctx.scratch("attn_part_o", (t - singles, nq * splits * d), torch.float32)
                 part_ml = ctx.scratch("attn_part_ml", (t - singles, nq * splits * 2), torch.float32)
             ops.attention_prefill(out[singles:], qkv[singles:], cache.k_pages, cache.v_pages, group.block_table, rest[0], rest[1],
                                   ctx.qblock_token0, ctx.qblock_count, nq, self.scale, self.reach, ctx.max_qblock, ctx.max_k_bound,
-                                  splits, part_o, part_ml, queries_raw)
+                                  splits, part_o, part_ml, queries_raw, one_request=paired)
         else:
             self._attend(ctx, out, qkv, cache, group)
         return linear(ctx, residual, out, self.w_o, accumulate=accumulate, then_norm=then_norm)
@@ -435,14 +451,17 @@ class GQAAttention(Part):
             rest = ctx.memo.get("rows_after_singles")
             if rest is None:
                 rest = ctx.memo["rows_after_singles"] = (ctx.token_slot[singles:], ctx.positions[singles:])
-            splits = self._prefill_splits(ctx.num_qblocks * nkv, longest, (t - singles) * nq * dv, nq // nkv, t - singles)
+            paired = self._walks_in_pairs(ctx, nq // nkv, d)
+            splits = self._prefill_splits((-(-ctx.num_qblocks // 2) if paired else ctx.num_qblocks) * nkv, longest, (t - singles) * nq * dv,
+                                          nq // nkv, t - singles, paired)
             part_o = part_ml = None
             if splits + extra > 1:
                 part_o = ctx.scratch("attn_part_o", (t - singles, nq * (splits + extra) * dv), torch.float32)
                 part_ml = ctx.scratch("attn_part_ml", (t - singles, nq * (splits + extra) * 2), torch.float32)
             ops.attention_prefill(out[singles:], qkv[singles:], cache.k_pages, cache.v_pages, group.block_table, rest[0], rest[1],
                                   ctx.qblock_token0, ctx.qblock_count, nq, self.scale, self.reach, ctx.max_qblock, ctx.max_k_bound,
-                                  splits, part_o, part_ml, None, keep_first=self.keep_first, gates=None if gates is None else gates[singles:], **more)
+                                  splits, part_o, part_ml, None, keep_first=self.keep_first, gates=None if gates is None else gates[singles:],
+                                  one_request=paired, **more)
         else:
             self._attend(ctx, out, qkv, cache, group, gates=gates, **more)
         if self.output_gate is True:
