@@ -109,3 +109,8 @@ template <int PENDING>
 __device__ __forceinline__ void fetched_then_barrier() {
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(PENDING) : "memory");
 }
+// ... and until this wave has what it read from LDS as well: others may then fill what it read from.
+template <int PENDING>
+__device__ __forceinline__ void fetched_and_read_then_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(PENDING) : "memory");
+}

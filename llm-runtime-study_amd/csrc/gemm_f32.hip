@@ -11,12 +11,6 @@ int lrs_gemm_f32(float* out, bool add, const float* a, const float* w, const flo
 
 namespace {
 
-// Waits until at most PENDING fetches are on their way and this wave has what it read from LDS, then for the workgroup.
-template <int PENDING>
-__device__ __forceinline__ void fetched_and_read_then_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(PENDING) : "memory");
-}
-
 // Memory straight into LDS as fetch_to_lds (common.h) has it, for a base that the compiler holds in scalar registers already.
 __device__ __forceinline__ void fetch_from(uint64_t base, unsigned lane_offset, unsigned lds_address) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds_address), "v"(lane_offset), "s"(base) : "memory");

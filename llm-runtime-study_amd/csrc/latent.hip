@@ -478,6 +478,208 @@ __global__ __launch_bounds__(256) void latent_attention_bf16_kernel(
   }
 }
 
+// The same for latent rows of 128, 256 or 512 values with 64 rotated dims behind them (CT tiles of 16 latent columns), whose tiles go from
+// memory straight into LDS: a workgroup's four waves (16 rows each) share them, and three tiles of 32 keys are on their way while one
+// is worked on.  The kernel above waits for memory four times a tile, 9 us in all; 16 tokens of 32 heads at 3,072
+// positions took 71-81 us with their merge, 31 here (a prompt of 2,048 tokens 1,535 and 322).  A tile is read once for both products: as rows for the scores (keys x queries:
+// a lane ends with eight keys' scores of one query, which are the second product's operand as they stand), and through the transposing
+// LDS read for the values (columns x queries: a lane's sums are of the same query), so the copy by columns is not read at all.
+// Piece c (16 bytes) of key row k lies at place c ^ turn(k): eight consecutive rows then meet every bank once, for whole pieces
+// and for the halves that the transposing read takes.  One wave a SIMD: its turn of some 3,000 cycles, 1,088 of them products, bounds
+// a prompt; a decode step the trips to memory before the first tile, 1.4 us a tile and the merge.
+template <int CT>
+__global__ __launch_bounds__(256) void latent_attention_shared_kernel(
+    bf16* __restrict__ out, int out_stride, float* __restrict__ part_o, float* __restrict__ part_ml, const bf16* __restrict__ queries,
+    int query_stride, const bf16* __restrict__ pages, const int* __restrict__ block_table, int table_stride,
+    const int* __restrict__ token_request, const int* __restrict__ positions, const int* __restrict__ group_token0,
+    const int* __restrict__ group_count, const float* __restrict__ sink, const bf16* __restrict__ gate, int gate_stride, int heads,
+    int page_size, float scale, int window, int splits) {
+  constexpr int RANK = 16 * CT, WIDTH = RANK + 64, KS = WIDTH / 32, PIECES = WIDTH / 8, ROW = WIDTH * 2;     // ROW: bytes
+  constexpr int STAGE = 32 * ROW, STAGES = 4, FETCHES = WIDTH / 16, EACH = FETCHES / 4, AHEAD = 6;
+  static_assert(PIECES % 16 == 8 && FETCHES % 4 == 0, "what the layout is made for");
+  __shared__ __attribute__((aligned(128))) unsigned char tiles[STAGES * STAGE];
+  const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), col = lane & 15, g = lane >> 4;
+  const int group = blockIdx.x, split = blockIdx.z;
+  const int token0 = group_token0 ? group_token0[group] : group;
+  const int rows = (group_count ? group_count[group] : 1) * heads;
+  const int block_row0 = blockIdx.y * 64;
+  if (block_row0 >= rows) return;
+  const int last_row = (block_row0 + 63 < rows ? block_row0 + 63 : rows - 1);
+  const int* table = block_table + (int64_t)token_request[token0] * table_stride;
+  const int pos_first = positions[token0 + block_row0 / heads], pos_last = positions[token0 + last_row / heads];
+  const int lo = first_seen(pos_first, window);
+  const int first_tile = lo / 32, last_tile = pos_last / 32, first_run = lo / 16, last_run = pos_last / 16;
+  const int per_split = (last_tile - first_tile + splits) / splits;
+  const int tile_begin = first_tile + split * per_split;
+  const int tile_end = tile_begin + per_split <= last_tile + 1 ? tile_begin + per_split : last_tile + 1;
+
+  // this lane's row: a (token, head) pair
+  const int row0 = block_row0 + wave * 16;
+  const bool works = row0 < rows;                                          // a wave without rows only brings tiles in
+  const int mine = row0 + col;
+  const bool live = mine < rows;
+  const int token = token0 + (live ? mine / heads : 0), head = live ? mine % heads : 0;
+  const int pos = live ? positions[token] : -1, from = live ? first_seen(pos, window) : 0;
+  bf16x8 qf[KS];
+  const bf16x8 zero = {};
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+    qf[ks] = live ? *(const bf16x8*)(queries + (int64_t)token * query_stride + (int64_t)head * WIDTH + ks * 32 + g * 8) : zero;
+
+  // the queries are there before the walk begins: the compiler would wait for them, and with them for every fetch, inside it
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[ks]));
+
+  // What this lane brings of a tile: piece p = (wave + 4 i) * 64 + lane of the first run's 16 rows, then the second's
+  auto turn_of = [](int row) { return ((row >> 1) & 3) << 1; };
+  unsigned offset[EACH];
+#pragma unroll
+  for (int i = 0; i < EACH; ++i) {
+    const int at = ((wave + 4 * i) * 64 + lane) % (16 * PIECES), row = at / PIECES, place = at % PIECES;
+    offset[i] = (unsigned)(row * ROW + (place ^ turn_of(row)) * 16);
+  }
+  const unsigned tiles_address = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)tiles;
+  // a run of keys that nobody sees stands for the nearest that somebody does: its scores are masked
+  auto run_of = [&](int tile, int half) {
+    const int run = tile * 2 + half;
+    return run < first_run ? first_run : run > last_run ? last_run : run;
+  };
+  int page_ahead[2];                                                       // of the tile to fetch next
+  auto look_up = [&](int tile) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) page_ahead[half] = table[run_of(tile, half) * 16 / page_size];
+  };
+  auto fetch = [&](int tile, int stage) {
+    const char* base[2];
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+      base[half] = (const char*)(pages + ((int64_t)page_ahead[half] * page_size + run_of(tile, half) * 16 % page_size) * WIDTH);
+#pragma unroll
+    for (int i = 0; i < EACH; ++i)
+      fetch_to_lds(base[wave + 4 * i < FETCHES / 2 ? 0 : 1], offset[i], tiles_address + (unsigned)(stage * STAGE + (wave + 4 * i) * 1024));
+  };
+  // where this lane reads: key row `col` (and col + 16) for the scores; four keys 4 g .. (and 16 on), four columns for the values
+  const int swap = turn_of(col);
+  const int key_at[2] = {col * ROW + ((g ^ swap) * 16), col * ROW + (((4 + g) ^ swap) * 16)};           // even and odd steps of 32 dims
+  const int value_row = 4 * g + (col >> 2);
+  int value_at[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) value_at[c] = value_row * ROW + (((2 * c + ((col & 3) >> 1)) ^ turn_of(value_row)) * 16) + (col & 1) * 8;
+
+  floatx4 acc[CT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c) acc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const float scale2 = scale * LOG2E;
+  float top = -INFINITY, total = 0.f;                                      // in powers of two; total: of this lane's keys
+  constexpr float STEP = 8.f;                                              // how far a maximum may pass the reference before that moves
+  if (tile_begin < tile_end) {
+#pragma unroll
+    for (int i = 0; i < STAGES - 1; ++i) {
+      look_up(tile_begin + i);
+      fetch(tile_begin + i, i);
+    }
+    look_up(tile_begin + STAGES - 1);
+  }
+  int stage = 0;
+  for (int tile = tile_begin; tile < tile_end; ++tile) {
+    // this tile is there, and the stage of the one before has been read by everyone
+    fetched_and_read_then_barrier<(STAGES - 2) * EACH>();
+    fetch(tile + STAGES - 1, (stage + STAGES - 1) % STAGES);               // past the end: the last run once more
+    look_up(tile + STAGES);
+    const unsigned char* at = tiles + stage * STAGE;
+    stage = (stage + 1) % STAGES;
+    if (!works) continue;
+    // fragments are asked for AHEAD products before their own; the fences keep the order (left alone, the compiler waits for each)
+    floatx4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    bf16x8 kf[AHEAD];
+    auto keys = [&](int f) { return *(const bf16x8*)(at + key_at[f >> 1 & 1] + (f >> 2) * 128 + (f & 1) * 16 * ROW); };
+#pragma unroll
+    for (int f = 0; f < AHEAD; ++f) kf[f] = keys(f);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int f = 0; f < 2 * KS; ++f) {
+      s[f & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[f % AHEAD], qf[f >> 1], s[f & 1], 0, 0, 0);
+      if (f + AHEAD < 2 * KS) kf[f % AHEAD] = keys(f + AHEAD);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    bf16x4 vf[AHEAD][2];
+    auto values = [&](int c, bf16x4 (&v)[2]) {
+      typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+      typedef __attribute__((address_space(3))) const unsigned char lds_byte;
+      lds_byte* from_lds = (lds_byte*)(at + value_at[c & 3] + (c >> 2) * 128);
+      v[0] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)from_lds);
+      v[1] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(from_lds + 16 * ROW));
+    };
+#pragma unroll
+    for (int c = 0; c < AHEAD; ++c) values(c, vf[c]);
+    __builtin_amdgcn_sched_barrier(0);
+    float most = -INFINITY;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int key = tile * 32 + h * 16 + 4 * g + i;
+        s[h][i] = key <= pos && key >= from ? s[h][i] * scale2 : -INFINITY;
+        most = fmaxf(most, s[h][i]);
+      }
+    most = fmaxf(most, __shfl_xor(most, 16, WAVE));
+    most = fmaxf(most, __shfl_xor(most, 32, WAVE));
+    const float now = most > top + STEP || top == -INFINITY ? most : top;
+    const float ref = now == -INFINITY ? 0.f : now;                        // a row that has seen no key yet
+    const float shrink = now == top ? 1.f : __builtin_amdgcn_exp2f(top - ref);
+    top = now;
+    bf16x8 weights;
+    float sum = 0.f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float e = __builtin_amdgcn_exp2f(s[h][i] - ref);
+        sum += e;
+        weights[h * 4 + i] = (bf16)e;
+      }
+    total = total * shrink + sum;
+    if (__any(shrink != 1.f)) {
+#pragma unroll
+      for (int c = 0; c < CT; ++c) acc[c] *= shrink;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      const bf16x4 first = vf[c % AHEAD][0], second = vf[c % AHEAD][1];
+      const bf16x8 v = {first[0], first[1], first[2], first[3], second[0], second[1], second[2], second[3]};
+      acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, weights, acc[c], 0, 0, 0);
+      if (c + AHEAD < CT) values(c + AHEAD, vf[c % AHEAD]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                         // the fetches past the end
+  total += __shfl_xor(total, 16, WAVE);
+  total += __shfl_xor(total, 32, WAVE);
+  if (!live) return;
+  if (splits > 1) {
+    const int64_t part = ((int64_t)token * heads + head) * splits + split;
+    if (g == 0) part_ml[part * 2] = top, part_ml[part * 2 + 1] = total;
+#pragma unroll
+    for (int c = 0; c < CT; ++c) *(floatx4*)(part_o + part * RANK + 16 * c + 4 * g) = acc[c];
+    return;
+  }
+  // the sink, one more term of the denominator, and the gate
+  float shrunk = 1.f, denominator = total;
+  if (sink) {
+    const float s2 = sink[head] * LOG2E, most = fmaxf(top, s2);
+    shrunk = __builtin_amdgcn_exp2f(top - most);
+    denominator = total * shrunk + __builtin_amdgcn_exp2f(s2 - most);
+  }
+  float factor = shrunk / denominator;
+  if (gate) factor *= 1.0f / (1.0f + expf(-(float)gate[(int64_t)token * gate_stride + head]));
+#pragma unroll
+  for (int c = 0; c < CT; ++c) {
+    const bf16x4 y = {(bf16)(acc[c][0] * factor), (bf16)(acc[c][1] * factor), (bf16)(acc[c][2] * factor), (bf16)(acc[c][3] * factor)};
+    *(bf16x4*)(out + (int64_t)token * out_stride + (int64_t)head * RANK + 16 * c + 4 * g) = y;
+  }
+}
+
 // What the parts of one (token, head) left, put together: maxima and sums in powers of two.
 __global__ __launch_bounds__(256) void latent_merge_kernel(bf16* __restrict__ out, int out_stride, const float* __restrict__ part_o,
                                                            const float* __restrict__ part_ml, const float* __restrict__ sink,
@@ -604,6 +806,11 @@ LRS_API int lrs_latent_attention_groups_takes(int rank, int width, int page_size
   return rank > 0 && rank <= 512 && width >= rank && width % 8 == 0 && page_size % 8 == 0;
 }
 
+// Whether its tiles go through LDS that a workgroup shares (one workgroup a compute unit) rather than into every wave's registers.
+LRS_API int lrs_latent_attention_groups_shares(int rank, int width, int page_size) {
+  return (rank == 128 || rank == 256 || rank == 512) && width == rank + 64 && page_size % 16 == 0;
+}
+
 // The same attention on the matrix cores, bfloat16: the step's tokens come as query groups (group_token0 / group_count
 // [groups]: consecutive tokens of one request, at most max_count; both null: every token a group of its own), the keys of a
 // group may be divided between `splits` workgroups (part_o [tokens, heads, splits, rank], part_ml [tokens, heads, splits, 2]
@@ -629,7 +836,15 @@ LRS_API int lrs_latent_attention_groups(void* out, int out_stride, const void* q
                                                         positions, group_token0, group_count, sink, (const bf16*)gate, gate_stride, heads, rank, \
                                                         width, page_size, scale, window, splits)
   const int ct = (rank + 15) / 16;
-  if (ct <= 2) LRS_LA(2);
+#define LRS_LS(CT)                                                                                                                        \
+  latent_attention_shared_kernel<CT><<<grid, 256, 0, s>>>((bf16*)out, out_stride, part_o, part_ml, (const bf16*)queries, query_stride,    \
+                                                          (const bf16*)pages, block_table, table_stride, token_request, positions, group_token0, \
+                                                          group_count, sink, (const bf16*)gate, gate_stride, heads, page_size, scale, window, splits)
+  if (lrs_latent_attention_groups_shares(rank, width, page_size) && out_stride % 4 == 0 && (uintptr_t)out % 8 == 0 && (uintptr_t)part_o % 16 == 0) {
+    if (rank == 128) LRS_LS(8);
+    else if (rank == 256) LRS_LS(16);
+    else LRS_LS(32);
+  } else if (ct <= 2) LRS_LA(2);
   else if (ct <= 4) LRS_LA(4);
   else if (ct <= 6) LRS_LA(6);
   else if (ct <= 8) LRS_LA(8);
@@ -637,6 +852,7 @@ LRS_API int lrs_latent_attention_groups(void* out, int out_stride, const void* q
   else if (ct <= 16) LRS_LA(16);
   else if (ct <= 24) LRS_LA(24);
   else LRS_LA(32);
+#undef LRS_LS
 #undef LRS_LA
   if (int rc = lrs_check_launch("latent_attention_groups")) return rc;
   if (splits > 1) {

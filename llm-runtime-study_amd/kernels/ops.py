@@ -188,6 +188,7 @@ _SIGNATURES = {
     "lrs_latent_prep": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_float, c_void_p, c_void_p,
                                 c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p]),
     "lrs_latent_attention_groups_takes": (c_int, [c_int, c_int, c_int]),
+    "lrs_latent_attention_groups_shares": (c_int, [c_int, c_int, c_int]),
     "lrs_latent_attention_groups": (c_int, [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
                                             c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int,
                                             c_void_p, c_void_p, c_void_p]),
@@ -1832,6 +1833,12 @@ def latent_attention(out: torch.Tensor, queries: torch.Tensor, pages: torch.Tens
 def latent_attention_groups_takes(dtype: torch.dtype, rank: int, width: int, page_size: int) -> bool:
     """Whether latent_attention_groups() takes the shape (else latent_attention())."""
     return dtype == torch.bfloat16 and bool(library().lrs_latent_attention_groups_takes(rank, width, page_size))
+
+
+def latent_attention_groups_shares(rank: int, width: int, page_size: int) -> bool:
+    """Whether latent_attention_groups() brings a workgroup's tiles into LDS for all its waves (one workgroup a compute unit; else
+    two, every wave by itself)."""
+    return bool(library().lrs_latent_attention_groups_shares(rank, width, page_size))
 
 
 def latent_attention_groups(out: torch.Tensor, queries: torch.Tensor, pages: torch.Tensor, value_pages: torch.Tensor, block_table: torch.Tensor,
