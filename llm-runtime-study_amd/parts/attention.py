@@ -227,6 +227,23 @@ class GQAAttention(Part):
             wanted = 2
         return max(1, min(wanted, length_class(longest) // 256, 64), -(-bound // (4096 * page_size)))
 
+    @classmethod
+    def _decode_shape(cls, workgroups: int, longest: int, bound: int, page_size: int, head_dim: int) -> tuple[int, int]:
+        """(splits, form) of attention_decode(): workgroups of four waves, two a unit (form 1), divided as _decode_splits says;
+        or, while the batch alone has no more than one workgroup a unit, of eight waves (form 2; heads of up to 128), one a unit
+        and undivided under 1,024 tokens.  A unit streams its workgroup's keys at some 40 GB/s whatever is on its way at once,
+        and a merge costs 3-4 us and the gap before it, so eight waves finish a short context sooner than a merge would: us
+        with four waves / with eight, parts in brackets, merge and gap counted: 16 heads on 8, batch 1 and 16 at 509 tokens 13.5 [1] /
+        11.2 [1] and 14.8 [1] / 12.6 [1], batch 32 at 600 27.4 [2] / 19.8 [1], batch 16 at 1,500 29.0 [4] / 28.1 [2]; 32 heads on 8,
+        batch 1 at 2,048 14.5 [8] / 13.2 [8], batch 8 24.5 [8] / 23.4 [4], batch 24 at 1,500 33.5 [1] / 30.8 [1], batch 8 at 8,192
+        58.2 [8] / 56.1 [4]; but batch 40 at 600 28.3 / 32.6 and batch 64 at 1,500 73.1 / 75.9."""
+        units = ops.compute_units()
+        if workgroups > units or head_dim > 128:
+            return cls._decode_splits(workgroups, longest, bound, page_size), 1
+        reach = length_class(longest)
+        wanted = 1 if reach < 1024 else min(-(-units // workgroups), reach // 256, 64)
+        return max(wanted, -(-bound // (4096 * page_size))), 2
+
     @staticmethod
     def _walks_in_pairs(ctx, heads_per_group: int, head_dim: int) -> bool:
         """Whether the kernel for ragged steps lets two neighbouring query groups walk their keys together (attention_prefill's
@@ -332,14 +349,14 @@ class GQAAttention(Part):
             longest, bound = ctx.max_k, ctx.max_k_bound
             if self.span is not None:
                 longest, bound = min(longest, self.span + 32), min(bound, self.span + 64)
-            splits = self._decode_splits(t * kv_heads, longest, bound, group.page_size)
+            splits, form = self._decode_shape(t * kv_heads, longest, bound, group.page_size, d)
             part_o = part_ml = None
             if splits > 1:
                 part_o = ctx.scratch("attn_part_o", (t, nq * splits * d), torch.float32)
                 part_ml = ctx.scratch("attn_part_ml", (t, nq * splits * 2), torch.float32)
             ops.attention_decode(out, qkv, cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot, ctx.positions,
                                  nq, self.scale, self.reach, splits, part_o, part_ml, ctx.max_k_bound, prepare,
-                                 form=1)   # the next tile on its way while one is worked on, the first one before the query is prepared (measured: 0.6 % of a step)
+                                 form=form)   # the next tile on its way while one is worked on, the first one before the query is prepared (measured: 0.6 % of a step)
         elif ops.attention_decode_supported(ctx.dtype, nq, kv_heads, d, group.page_size):
             # sized by the step's coarse bound of the longest context, the same for every step of one shape
             longest = ctx.max_k_bound if self.span is None else min(ctx.max_k_bound, self.span + 64)
@@ -348,7 +365,7 @@ class GQAAttention(Part):
                 # the single tokens at the head of a mixed step (decoding requests beside a prompt portion) go to the
                 # kernel of decode steps, which divides one token's keys between waves and workgroups; as rows of
                 # the other kernel each would walk its whole context in one workgroup
-                splits = self._decode_splits(singles * kv_heads, longest, ctx.max_k_bound, group.page_size)
+                splits, form = self._decode_shape(singles * kv_heads, longest, ctx.max_k_bound, group.page_size, d)
                 part_o = part_ml = None
                 if splits > 1:
                     part_o = ctx.scratch("attn_single_part_o", (singles, nq * splits * d), torch.float32)
@@ -363,7 +380,7 @@ class GQAAttention(Part):
                     first = ops.DecodePrepare(self.q_norm, self.k_norm, self.qk_norm_eps, None if parted is None else parted[0],
                                               None if parted is None else parted[1], 0)
                 ops.attention_decode(out[:singles], qkv[:singles], cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot,
-                                     ctx.positions, nq, self.scale, self.reach, splits, part_o, part_ml, ctx.max_k_bound, first, form=1)
+                                     ctx.positions, nq, self.scale, self.reach, splits, part_o, part_ml, ctx.max_k_bound, first, form=form)
             rest = ctx.memo.get("rows_after_singles")
             if rest is None:
                 rest = ctx.memo["rows_after_singles"] = (ctx.token_slot[singles:], ctx.positions[singles:])
@@ -428,25 +445,25 @@ class GQAAttention(Part):
             longest, bound = ctx.max_k, ctx.max_k_bound
             if self.span is not None:
                 longest, bound = min(longest, self.span + 32), min(bound, self.span + 64)
-            splits = self._decode_splits(t * nkv, longest, bound, group.page_size)
+            splits, form = self._decode_shape(t * nkv, longest, bound, group.page_size, d)
             part_o = part_ml = None
             if splits + extra > 1:
                 part_o = ctx.scratch("attn_part_o", (t, nq * (splits + extra) * dv), torch.float32)
                 part_ml = ctx.scratch("attn_part_ml", (t, nq * (splits + extra) * 2), torch.float32)
             ops.attention_decode(out, qkv, cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot, ctx.positions,
-                                 nq, self.scale, self.reach, splits, part_o, part_ml, ctx.max_k_bound, prepare, form=1,
+                                 nq, self.scale, self.reach, splits, part_o, part_ml, ctx.max_k_bound, prepare, form=form,
                                  keep_first=self.keep_first, gates=gates, **more)
         elif cores:
             longest = ctx.max_k_bound if self.span is None else min(ctx.max_k_bound, self.span + 64)
             singles = ctx.single_rows
             if singles:
-                splits = self._decode_splits(singles * nkv, longest, ctx.max_k_bound, group.page_size)
+                splits, form = self._decode_shape(singles * nkv, longest, ctx.max_k_bound, group.page_size, d)
                 part_o = part_ml = None
                 if splits + extra > 1:
                     part_o = ctx.scratch("attn_single_part_o", (singles, nq * (splits + extra) * dv), torch.float32)
                     part_ml = ctx.scratch("attn_single_part_ml", (singles, nq * (splits + extra) * 2), torch.float32)
                 ops.attention_decode(out[:singles], qkv[:singles], cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot,
-                                     ctx.positions, nq, self.scale, self.reach, splits, part_o, part_ml, ctx.max_k_bound, None, form=1,
+                                     ctx.positions, nq, self.scale, self.reach, splits, part_o, part_ml, ctx.max_k_bound, None, form=form,
                                      keep_first=self.keep_first, gates=None if gates is None else gates[:singles], **more)
             rest = ctx.memo.get("rows_after_singles")
             if rest is None:
