@@ -310,8 +310,16 @@ __device__ __forceinline__ void prepare_head(bf16x8 (&r)[D / 32], const bf16* __
 // the pages hold there, and writes both into the pages (see DecodePrep).
 // MORE: values narrower than keys and a bias by distance (dv and distance are looked at); instances of their own, so that the
 // others are spared the checks.
+template <int D, int WAVES>
+struct DecodeLds {
+  float sm_m[WAVES][16], sm_l[WAVES][16];
+  float sm_o[WAVES][D][16];
+  __attribute__((aligned(16))) bf16 own_k[D];
+  bf16 own_v[D];
+};
 template <int D, bool PREP, int WAVES, bool AHEAD, bool MORE>
-__global__ __launch_bounds__(WAVES * 64) void attention_decode_bf16_kernel(
+__device__ __forceinline__ void attention_decode_part(
+    DecodeLds<D, WAVES>& lds, int* page_ids, int split, int kvh, int token,
     bf16* __restrict__ out, int out_stride, float* __restrict__ part_o, float* __restrict__ part_ml,
     const bf16* __restrict__ q, int q_stride, bf16* __restrict__ k_pages,
     bf16* __restrict__ v_pages, const int* __restrict__ block_table, int table_stride,
@@ -322,11 +330,10 @@ __global__ __launch_bounds__(WAVES * 64) void attention_decode_bf16_kernel(
   constexpr int DS = D / 32, DB = D / 16, THREADS = WAVES * 64;
   const int dv = MORE ? dv_given : D;
   const float* __restrict__ distance = MORE ? distance_given : nullptr;
-  __shared__ float sm_m[WAVES][16], sm_l[WAVES][16];
-  __shared__ float sm_o[WAVES][D][16];
+  auto &sm_m = lds.sm_m, &sm_l = lds.sm_l;
+  auto& sm_o = lds.sm_o;
   const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
   const int col = lane & 15, g = lane >> 4;
-  const int split = blockIdx.x, kvh = blockIdx.y, token = blockIdx.z;
   const int group = nq / nkv;
   const int pos = positions[token];
   const int lo = first_seen(pos, window);
@@ -354,7 +361,6 @@ __global__ __launch_bounds__(WAVES * 64) void attention_decode_bf16_kernel(
 
   // the block table entries of this workgroup's tiles, in LDS: the address of a key must not
   // wait for a trip to memory of its own
-  extern __shared__ int page_ids[];
   const int first_block = tile_begin * 32 / page_size;
   const int last_key = tile_end * 32 - 1 < pos ? tile_end * 32 - 1 : pos;
   if (tile_begin < tile_end)
@@ -416,8 +422,7 @@ __global__ __launch_bounds__(WAVES * 64) void attention_decode_bf16_kernel(
   // The workgroup that walks the token's own position prepares the new key once (its last wave,
   // which is dealt the fewest tiles), leaves it and the new value in LDS for the wave that meets
   // the position, and writes both into the pages.
-  __shared__ __attribute__((aligned(16))) bf16 own_k[D];
-  __shared__ bf16 own_v[D];
+  auto &own_k = lds.own_k, &own_v = lds.own_v;
   const bool holds_own = PREP && prep.kv_columns > 0 && tile_begin <= last_tile && last_tile < tile_end;
   if (holds_own && wave == WAVES - 1) {
     bf16x8 kn[DS];
@@ -578,6 +583,20 @@ __global__ __launch_bounds__(WAVES * 64) void attention_decode_bf16_kernel(
       }
     }
   }
+}
+
+template <int D, bool PREP, int WAVES, bool AHEAD, bool MORE>
+__global__ __launch_bounds__(WAVES * 64) void attention_decode_bf16_kernel(
+    bf16* __restrict__ out, int out_stride, float* __restrict__ part_o, float* __restrict__ part_ml,
+    const bf16* __restrict__ q, int q_stride, bf16* __restrict__ k_pages,
+    bf16* __restrict__ v_pages, const int* __restrict__ block_table, int table_stride,
+    const int* __restrict__ token_request, const int* __restrict__ positions, int nq, int nkv,
+    int page_size, float scale, int window, int splits, int slots, DecodePrep prep, const float* __restrict__ sinks,
+    float softcap, const bf16* __restrict__ gates, int gate_stride, int dv_given, const float* __restrict__ distance_given,
+    int distance_form) {
+  __shared__ DecodeLds<D, WAVES> lds;
+  extern __shared__ int page_ids[];
+  attention_decode_part<D, PREP, WAVES, AHEAD, MORE>(lds, page_ids, blockIdx.x, blockIdx.y, blockIdx.z, out, out_stride, part_o, part_ml, q, q_stride, k_pages, v_pages, block_table, table_stride, token_request, positions, nq, nkv, page_size, scale, window, splits, slots, prep, sinks, softcap, gates, gate_stride, dv_given, distance_given, distance_form);
 }
 
 // Merges the partial results of the splits of one (token, head): out = sum_s o_s 2^(m_s - m) / sum_s l_s 2^(m_s - m).
@@ -1287,9 +1306,15 @@ enum { SCORES_PLAIN = 0, SCORES_CAPPED = 1, SCORES_DISTANCE = 2, SCORES_BOTH = 3
 // 16 heads on 8, 2,048 tokens after 14,336: 569 us with idle waves, 444 with halves, 322 in pairs with the keys divided by two;
 // 8,192 tokens 584 / 385 / 390; 2,048 after 2,048 142 / 136 / 100.
 enum { SPREAD_HEADS = 0, SPREAD_SOME_IDLE = 1, SPREAD_HALVES = 2, SPREAD_PAIRS = 3 };
+struct PrefillLds {
+  static constexpr int D = 128, STAGES = 3, KBLOCK = 1024 + 32, KBYTES = 8 * KBLOCK, VHALF = 16 * D * 2 + 16;
+  static constexpr int VSTAGE = (2 * VHALF + 63) / 64 * 64;
+  __attribute__((aligned(64))) unsigned char key_tiles[STAGES * KBYTES];
+  __attribute__((aligned(64))) unsigned char value_tiles[STAGES * VSTAGE];
+};
 template <int QB, bool MANY_WAVES, int SPREAD, int SCORES>
-__global__ __launch_bounds__(MANY_WAVES ? 512 : 256, MANY_WAVES ? 1 : QB == 1 && (SCORES & SCORES_LINEAR) ? 3 : 2) void attention_prefill_d128_bf16_kernel(
-    bf16* __restrict__ out, int out_stride, const bf16* __restrict__ q, int q_stride,
+__device__ __forceinline__ void attention_prefill_d128_part(
+    PrefillLds& lds, int block, bf16* __restrict__ out, int out_stride, const bf16* __restrict__ q, int q_stride,
     const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
     const int* __restrict__ block_table, int table_stride, const int* __restrict__ token_request,
     const int* __restrict__ positions, const int* __restrict__ qblock_token0,
@@ -1302,17 +1327,17 @@ __global__ __launch_bounds__(MANY_WAVES ? 512 : 256, MANY_WAVES ? 1 : QB == 1 &&
   static_assert(!HALVES || (QB == 1 && !MANY_WAVES), "two heads and two blocks of 16 queries are four waves' work");
   static_assert(!PAIRS || (QB == 2 && !MANY_WAVES), "two heads and two groups of 32 queries are four waves' work");
   constexpr int D = 128, DS = D / 32, DB = D / 16, STAGES = 3;
-  constexpr int KBLOCK = 1024 + 32, KBYTES = 8 * KBLOCK, VHALF = 16 * D * 2 + 16, VBYTES = 2 * VHALF;
-  constexpr int VSTAGE = (VBYTES + 63) / 64 * 64;
-  __shared__ __attribute__((aligned(64))) unsigned char key_tiles[STAGES * KBYTES];
-  __shared__ __attribute__((aligned(64))) unsigned char value_tiles[STAGES * VSTAGE];
+  constexpr int KBLOCK = PrefillLds::KBLOCK, KBYTES = PrefillLds::KBYTES, VHALF = PrefillLds::VHALF, VSTAGE = PrefillLds::VSTAGE;
+  static_assert(D == PrefillLds::D && STAGES == PrefillLds::STAGES, "what the tiles' place is made for");
+  auto& key_tiles = lds.key_tiles;
+  auto& value_tiles = lds.value_tiles;
   const int tid = threadIdx.x;
   const int lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int col = lane & 15, g = lane >> 4;
   const int key_chunk = ((g & 1) << 1) | (g >> 1);                 // m: the eight keys this lane group holds weights of
   const int group = nq / nkv;
   const int n_walks = PAIRS ? (n_blocks + 1) / 2 : n_blocks;       // PAIRS: two neighbouring groups of one request walk together
-  const int work = blockIdx.x % (n_walks * nkv), split = blockIdx.x / (n_walks * nkv);
+  const int work = block % (n_walks * nkv), split = block / (n_walks * nkv);
   const int which_chunk = work / chunk, in_chunk = work % chunk;
   const int chunk_block0 = which_chunk * (chunk / nkv);
   const int chunk_blocks = n_walks - chunk_block0 < chunk / nkv ? n_walks - chunk_block0 : chunk / nkv;
@@ -1405,11 +1430,11 @@ __global__ __launch_bounds__(MANY_WAVES ? 512 : 256, MANY_WAVES ? 1 : QB == 1 &&
   const int value_fragment = (g & 1) * VHALF + col * 32 + (g >> 1) * 16;                // + e * 512
 
   // kv groups of more than four heads take several passes over the keys
-  const int waves = blockDim.x / WAVE;
+  const int waves = MANY_WAVES ? blockDim.x / WAVE : 4;
   // two heads: a wave has one of them and one of the group's two blocks of 16 queries (beginning at query0), or one of two groups
   const int query0 = HALVES ? (wave >> 1) * 16 : 0;
   // waves without a head sit on other SIMDs in the workgroup that shares the compute unit (the 256th from here)
-  const int my_wave = HALVES || PAIRS ? wave & 1 : IDLE_WAVES && !MANY_WAVES ? (wave + (blockIdx.x >> 8 & 1) * 2) & 3 : wave;
+  const int my_wave = HALVES || PAIRS ? wave & 1 : IDLE_WAVES && !MANY_WAVES ? (wave + (block >> 8 & 1) * 2) & 3 : wave;
   for (int head0 = kvh * group; head0 < (kvh + 1) * group; head0 += waves) {
     const int head = head0 + my_wave;
     const bool active = head < (kvh + 1) * group;
@@ -1780,6 +1805,53 @@ __global__ __launch_bounds__(MANY_WAVES ? 512 : 256, MANY_WAVES ? 1 : QB == 1 &&
   }
 }
 
+template <int QB, bool MANY_WAVES, int SPREAD, int SCORES>
+__global__ __launch_bounds__(MANY_WAVES ? 512 : 256, MANY_WAVES ? 1 : QB == 1 && (SCORES & SCORES_LINEAR) ? 3 : 2) void attention_prefill_d128_bf16_kernel(
+    bf16* __restrict__ out, int out_stride, const bf16* __restrict__ q, int q_stride,
+    const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
+    const int* __restrict__ block_table, int table_stride, const int* __restrict__ token_request,
+    const int* __restrict__ positions, const int* __restrict__ qblock_token0,
+    const int* __restrict__ qblock_count, int n_blocks, int chunk, int nq, int nkv, int page_size, float scale,
+    int window, int splits, int slots, float* __restrict__ part_o, float* __restrict__ part_ml, int prepare_q, DecodePrep prep,
+    const float* __restrict__ sinks, float softcap, const bf16* __restrict__ gates, int gate_stride, int dv,
+    const float* __restrict__ distance) {
+  __shared__ PrefillLds lds;
+  attention_prefill_d128_part<QB, MANY_WAVES, SPREAD, SCORES>(lds, blockIdx.x, out, out_stride, q, q_stride, k_pages, v_pages, block_table, table_stride, token_request, positions, qblock_token0, qblock_count, n_blocks, chunk, nq, nkv, page_size, scale, window, splits, slots, part_o, part_ml, prepare_q, prep, sinks, softcap, gates, gate_stride, dv, distance);
+}
+
+// --------------------------------- a mixed step's two kinds of rows in one launch
+// The single tokens at the head of a mixed step (decoding requests) and the prompt portion behind them are independent, but
+// as two launches one waits for the other: 24 tokens at 1,500 are bound by their keys' way from memory, 488 tokens behind as
+// many by the length of a walk in fewer workgroups than the chip has room for.  Here the first single_blocks workgroups
+// (token by token, the kv heads in turn) do what attention_decode_bf16_kernel does with four waves, the others what the
+// kernel above does: 37 and 39 us a layer in two launches (32 heads on 8), 41 in one.  Heads of 128, plain scores, undivided keys.
+template <int QB, int SPREAD, bool PREP>
+__global__ __launch_bounds__(256, 2) void attention_mixed_d128_kernel(
+    bf16* __restrict__ out, int out_stride, const bf16* __restrict__ q, int q_stride, bf16* __restrict__ k_pages, bf16* __restrict__ v_pages,
+    const int* __restrict__ block_table, int table_stride, const int* __restrict__ token_request, const int* __restrict__ positions,
+    const int* __restrict__ qblock_token0, const int* __restrict__ qblock_count, int n_blocks, int chunk, int nq, int nkv, int page_size,
+    float scale, int window, DecodePrep prep, int singles) {
+  __shared__ union Place {
+    DecodeLds<128, 4> single;
+    PrefillLds portion;
+  } lds;
+  extern __shared__ int page_ids[];
+  const int single_blocks = singles * nkv;
+  if ((int)blockIdx.x < single_blocks) {
+    attention_decode_part<128, PREP, 4, true, false>(lds.single, page_ids, 0, blockIdx.x % nkv, blockIdx.x / nkv, out, out_stride, nullptr, nullptr,
+                                                     q, q_stride, k_pages, v_pages, block_table, table_stride, token_request, positions, nq, nkv,
+                                                     page_size, scale, window, 1, 1, prep, nullptr, 0.f, nullptr, 0, 128, nullptr, 0);
+    return;
+  }
+  DecodePrep rest = prep;                                                  // the tables' rows of the tokens behind
+  if (prep.cosv) rest.cosv += (int64_t)singles * 64, rest.sinv += (int64_t)singles * 64;
+  attention_prefill_d128_part<QB, false, SPREAD, SCORES_PLAIN>(lds.portion, blockIdx.x - single_blocks, out + (int64_t)singles * out_stride, out_stride,
+                                                               q + (int64_t)singles * q_stride, q_stride, k_pages, v_pages, block_table, table_stride,
+                                                               token_request + singles, positions + singles, qblock_token0, qblock_count, n_blocks,
+                                                               chunk, nq, nkv, page_size, scale, window, 1, 1, nullptr, nullptr, PREP, rest, nullptr,
+                                                               0.f, nullptr, 0, 128, nullptr);
+}
+
 // Compute units of the current device (asked once).
 static int compute_units() {
   static int units = 0;
@@ -1937,6 +2009,52 @@ LRS_API int lrs_attention_prefill(void* out, int out_stride, const void* q, int 
     return lrs_check_launch("attention_merge");
   }
   return 0;
+}
+
+// lrs_attention_decode for the first `singles` tokens and lrs_attention_prefill for those behind them (qblock_token0 counts from
+// there) in one launch: heads of 128, plain scores, undivided keys; prepare as there (the keys are in the pages already).
+LRS_API int lrs_attention_mixed(void* out, int out_stride, const void* q, int q_stride, void* k_pages, void* v_pages, const int* block_table,
+                                int table_stride, const int* token_request, const int* positions, const int* qblock_token0, const int* qblock_count,
+                                int n_blocks, int max_count, int max_context, int nq, int nkv, int page_size, float scale, int window, int singles,
+                                int prepare, const void* q_weight, int w_dtype, float eps, const float* cosv, const float* sinv, int one_request,
+                                void* stream) {
+  LRS_REQUIRE(singles > 0 && n_blocks > 0 && nq > 0 && nkv > 0 && nq % nkv == 0 && nq / nkv <= 16, "attention_mixed: bad sizes singles=%d blocks=%d nq=%d nkv=%d",
+              singles, n_blocks, nq, nkv);
+  LRS_REQUIRE(max_count >= 1 && max_count <= 32, "attention_mixed: query groups hold 1..32 tokens, got %d", max_count);
+  LRS_REQUIRE(page_size > 0 && page_size % 16 == 0, "attention_mixed: page size %d is not a multiple of 16", page_size);
+  LRS_REQUIRE(q_stride % 8 == 0 && ((uintptr_t)q % 16) == 0 && out_stride % 4 == 0 && ((uintptr_t)out % 8) == 0, "attention_mixed: q rows must be 16-byte and out rows 8-byte aligned");
+  LRS_REQUIRE(max_context >= 1, "attention_mixed: max_context must be the longest context length of the step");
+  if (prepare) {
+    LRS_REQUIRE(q_weight == nullptr || eps > 0.f, "attention_mixed: eps must be positive");
+    LRS_REQUIRE((cosv == nullptr) == (sinv == nullptr), "attention_mixed: cos and sin tables must come together");
+    LRS_REQUIRE((uintptr_t)q_weight % 16 == 0 && (uintptr_t)cosv % 16 == 0 && (uintptr_t)sinv % 16 == 0, "attention_mixed: norm weight and rotation tables must be 16-byte aligned");
+  }
+  const int reach = window < 0 ? -window : window;
+  const int span = reach > 0 && reach + 64 < max_context ? reach + 64 : max_context;
+  const size_t table_lds = sizeof(int) * (size_t)((span / 32 + 1) * 32 / page_size + 4);
+  LRS_REQUIRE(table_lds <= 24 * 1024, "attention_mixed: a context of %d tokens needs more block table entries than fit LDS", max_context);
+  const DecodePrep prep{q_weight, nullptr, w_dtype == LRS_F32, eps, cosv, sinv, 0};
+  const int chunk = nkv >= compute_units() ? nkv : compute_units() / nkv * nkv;
+  const int heads = nq / nkv;
+  hipStream_t s = (hipStream_t)stream;
+#define MIXED(QB, SPREAD, WALKS)                                                                                                          \
+  do {                                                                                                                                    \
+    const dim3 grid(singles * nkv + (WALKS) * nkv);                                                                                       \
+    if (prepare) attention_mixed_d128_kernel<QB, SPREAD, true><<<grid, 256, table_lds, s>>>(MIXED_ARGS);                                  \
+    else attention_mixed_d128_kernel<QB, SPREAD, false><<<grid, 256, table_lds, s>>>(MIXED_ARGS);                                         \
+  } while (0)
+#define MIXED_ARGS                                                                                                                        \
+  (bf16*)out, out_stride, (const bf16*)q, q_stride, (bf16*)k_pages, (bf16*)v_pages, block_table, table_stride, token_request, positions,  \
+      qblock_token0, qblock_count, n_blocks, chunk, nq, nkv, page_size, scale, window, prep, singles
+  const bool idle = heads % 4 != 0;
+  if (max_count <= 16) { if (idle) MIXED(1, SPREAD_SOME_IDLE, n_blocks); else MIXED(1, SPREAD_HEADS, n_blocks); }
+  else if (heads == 2 && one_request) MIXED(2, SPREAD_PAIRS, (n_blocks + 1) / 2);
+  else if (heads == 2) MIXED(1, SPREAD_HALVES, n_blocks);
+  else if (idle) MIXED(2, SPREAD_SOME_IDLE, n_blocks);
+  else MIXED(2, SPREAD_HEADS, n_blocks);
+#undef MIXED
+#undef MIXED_ARGS
+  return lrs_check_launch("attention_mixed");
 }
 
 // Compute units of the device, for callers that size their launches by it.

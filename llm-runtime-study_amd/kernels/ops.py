@@ -156,6 +156,9 @@ _SIGNATURES = {
     "lrs_attention_prefill": (c_int, [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                                       c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int,
                                       c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_int, c_float, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_void_p]),
+    "lrs_attention_mixed": (c_int, [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
+                                    c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_void_p, c_int, c_float, c_void_p, c_void_p,
+                                    c_int, c_void_p]),
     "lrs_attention_prefill_prepares": (c_int, [c_int]),
     "lrs_compute_units": (c_int, []),
     "lrs_gemm_lines_width": (c_int, [c_int, c_int, c_int]),
@@ -234,7 +237,7 @@ def library():
 # PLAN_OPS fixes the number of each entry point inside a plan; csrc/plan_dispatch.inc, made from this list
 # and _SIGNATURES by kernels/plan_codegen.py, is the other side (a test keeps the two in step).
 PLAN_OPS = ("lrs_activation", "lrs_add_gathered", "lrs_add_into", "lrs_add_rmsnorm", "lrs_advance_decode", "lrs_advance_slots", "lrs_attention", "lrs_attention_decode",
-            "lrs_attention_prefill", "lrs_axpby", "lrs_choose_tokens", "lrs_choose_tokens_split", "lrs_copy_to_pinned", "lrs_delta_rule", "lrs_delta_rule_channels", "lrs_embed", "lrs_fill_i32",
+            "lrs_attention_mixed", "lrs_attention_prefill", "lrs_axpby", "lrs_choose_tokens", "lrs_choose_tokens_split", "lrs_copy_to_pinned", "lrs_delta_rule", "lrs_delta_rule_channels", "lrs_embed", "lrs_fill_i32",
             "lrs_filter_logits", "lrs_gated_clamped", "lrs_gated_norm_add", "lrs_gather_rows", "lrs_gemm", "lrs_gemm_lines_add_rmsnorm", "lrs_gemm_mid_add_norm_begin", "lrs_gemm_mid_qk_prep", "lrs_gemm_mid_scaled",
             "lrs_gemm_norm_chain", "lrs_head_gemm", "lrs_latent_attention", "lrs_latent_attention_groups", "lrs_latent_prep", "lrs_layernorm", "lrs_library_gemm", "lrs_mlstm", "lrs_mlstm_chunks", "lrs_moe_align", "lrs_moe_combine", "lrs_moe_experts", "lrs_moe_route", "lrs_moe_route_align", "lrs_norm_add",
             "lrs_qk_prep", "lrs_qkv_norm_prep", "lrs_rmsnorm", "lrs_rope_table", "lrs_rotate_unit_prep", "lrs_round_rows", "lrs_scale_add_layernorm", "lrs_scale_rows", "lrs_scale_values", "lrs_sigmoid_gate", "lrs_silu_mul", "lrs_soft_cap", "lrs_ssm", "lrs_xielu")
@@ -1334,6 +1337,44 @@ def attention_prefill(out: torch.Tensor, q: torch.Tensor, k_pages: torch.Tensor,
         tokens, splits, None if slots == 1 else _dev(part_o, "part_o"), None if slots == 1 else _dev(part_ml, "part_ml"), *fused,
         _sinks(sinks, nq, "attention_prefill"), float(softcap), *_gates(gates, tokens, nq, q.dtype, "attention_prefill"), dv,
         *_distance(distance, nq, "attention_prefill"), 1 if one_request else 0, _stream())
+
+
+def attention_mixed(out: torch.Tensor, q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, block_table: torch.Tensor, token_request: torch.Tensor,
+                    positions: torch.Tensor, singles: int, qblock_token0: torch.Tensor, qblock_count: torch.Tensor, nq: int, scale: float, window: int = 0,
+                    max_count: int | None = None, max_context: int | None = None, prepare: "DecodePrepare | None" = None, one_request: bool = False) -> None:
+    """attention_decode() for the first `singles` tokens of a step and attention_prefill() for those behind them (whose groups
+    count from there), in one launch: bfloat16 heads of 128, plain scores, undivided keys.  prepare: q_weight, eps, cos and sin for all tokens
+    (kv_heads 0: the keys and values are in the pages already)."""
+    tokens = out.shape[0]
+    _need(k_pages.dim() == 4 and k_pages.is_contiguous() and v_pages.is_contiguous(), "attention_mixed: pages must be contiguous")
+    _, nkv, page_size, d = k_pages.shape
+    _need(d == 128 and v_pages.shape == (k_pages.shape[0], nkv, d, page_size), "attention_mixed: key pages must be [P, nkv, page, 128] and value pages [P, nkv, 128, page]")
+    _need(attention_decode_supported(q.dtype, nq, nkv, d, page_size), f"attention_mixed: unsupported shape nq={nq} nkv={nkv} page={page_size} {q.dtype}")
+    _need(0 < singles < tokens and out.shape[1] == nq * d and q.shape[0] == tokens and q.shape[1] >= nq * d, "attention_mixed: q/out widths do not match nq*d, or no tokens of one kind")
+    _need(q.dtype == k_pages.dtype == v_pages.dtype == out.dtype, "attention_mixed: q, pages and out must share a dtype")
+    _need(block_table.dim() == 2 and block_table.dtype == torch.int32 and block_table.stride(1) == 1, "attention_mixed: block_table must be int32 [R, blocks]")
+    for name, t in (("token_request", token_request), ("positions", positions)):
+        _need(t.dtype == torch.int32 and t.numel() >= tokens and t.is_contiguous(), f"attention_mixed: {name} must be int32 [T]")
+    n_blocks = qblock_token0.numel()
+    _need(n_blocks > 0 and qblock_count.numel() == n_blocks and qblock_token0.dtype == qblock_count.dtype == torch.int32
+          and qblock_token0.is_contiguous() and qblock_count.is_contiguous(), "attention_mixed: query blocks must be two int32 vectors of one length")
+    fused = [0, None, 0, 0.0, None, None]
+    if prepare is not None:
+        _need(prepare.kv_heads == 0, "attention_mixed: prepares the queries only (kv_heads must be 0)")
+        w = prepare.q_weight
+        _need(w is None or (w.numel() == d and w.is_contiguous() and prepare.eps > 0), "attention_mixed: q_weight must hold head_dim values, eps be positive")
+        for name, t in (("cos", prepare.cos), ("sin", prepare.sin)):
+            _need((t is None) == (prepare.cos is None) and (t is None or (t.dtype == torch.float32 and t.dim() == 2 and t.shape[0] >= tokens
+                                                                       and t.shape[1] == d // 2 and t.is_contiguous())),
+                  f"attention_mixed: {name} must be float32 [{tokens}, {d // 2}]")
+        fused = [1, None if w is None else _dev(w, "q_weight"), 0 if w is None else dtype_code(w.dtype), prepare.eps,
+                 None if prepare.cos is None else _dev(prepare.cos, "cos"), None if prepare.sin is None else _dev(prepare.sin, "sin")]
+    _launch("lrs_attention_mixed",
+        _dev(out, "out"), _rows(out, "out"), _dev(q, "q"), _rows(q, "q"), _dev(k_pages, "k_pages"), _dev(v_pages, "v_pages"),
+        _dev(block_table, "block_table"), block_table.stride(0), _dev(token_request, "token_request"), _dev(positions, "positions"),
+        _dev(qblock_token0, "qblock_token0"), _dev(qblock_count, "qblock_count"), n_blocks, attention_prefill_group() if max_count is None else max_count,
+        block_table.shape[1] * page_size if max_context is None else max_context, nq, nkv, page_size, scale, window, singles, *fused,
+        1 if one_request else 0, _stream())
 
 
 def attention_prefill_prepares(d: int) -> bool:

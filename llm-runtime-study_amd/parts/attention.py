@@ -361,11 +361,21 @@ class GQAAttention(Part):
             # sized by the step's coarse bound of the longest context, the same for every step of one shape
             longest = ctx.max_k_bound if self.span is None else min(ctx.max_k_bound, self.span + 64)
             singles = ctx.single_rows
+            paired = self._walks_in_pairs(ctx, nq // kv_heads, d)
+            rest_splits = self._prefill_splits((-(-ctx.num_qblocks // 2) if paired else ctx.num_qblocks) * kv_heads, longest, (t - singles) * nq * d,
+                                               nq // kv_heads, t - singles, paired)
+            splits, form = self._decode_shape(singles * kv_heads, longest, ctx.max_k_bound, group.page_size, d) if singles else (1, 1)
+            if (singles and d == 128 and (splits == 1 or 2 * singles * kv_heads > ops.compute_units()) and rest_splits == 1 and ctx.max_k_bound <= 4096 * group.page_size):
+                # both kinds of rows in one launch: neither fills the chip by itself, and two launches would wait for each other
+                # (24 tokens at 1,500 beside 488 behind 488: 37 + 39 us a layer, 41 in one launch).  Single tokens whose keys would be
+                # divided come along where they are half a workgroup a unit and more: the portion's workgroups fill the rest
+                ops.attention_mixed(out, qkv, cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot, ctx.positions, singles, ctx.qblock_token0,
+                                    ctx.qblock_count, nq, self.scale, self.reach, ctx.max_qblock, ctx.max_k_bound, queries_raw, one_request=paired)
+                return linear(ctx, residual, out, self.w_o, accumulate=accumulate, then_norm=then_norm)
             if singles:
                 # the single tokens at the head of a mixed step (decoding requests beside a prompt portion) go to the
                 # kernel of decode steps, which divides one token's keys between waves and workgroups; as rows of
                 # the other kernel each would walk its whole context in one workgroup
-                splits, form = self._decode_shape(singles * kv_heads, longest, ctx.max_k_bound, group.page_size, d)
                 part_o = part_ml = None
                 if splits > 1:
                     part_o = ctx.scratch("attn_single_part_o", (singles, nq * splits * d), torch.float32)
@@ -386,9 +396,7 @@ class GQAAttention(Part):
                 rest = ctx.memo["rows_after_singles"] = (ctx.token_slot[singles:], ctx.positions[singles:])
             if queries_raw is not None and singles and cos is not None:
                 queries_raw = ops.DecodePrepare(self.q_norm, None, self.qk_norm_eps, parted[2], parted[3], 0)
-            paired = self._walks_in_pairs(ctx, nq // kv_heads, d)
-            splits = self._prefill_splits((-(-ctx.num_qblocks // 2) if paired else ctx.num_qblocks) * kv_heads, longest, (t - singles) * nq * d,
-                                          nq // kv_heads, t - singles, paired)
+            splits = rest_splits
             part_o = part_ml = None
             if splits > 1:
                 part_o = ctx.scratch("attn_part_o", (t - singles, nq * splits * d), torch.float32)
