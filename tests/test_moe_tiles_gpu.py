@@ -1,0 +1,34 @@
+"""The grouped products of large steps deal the tiles in use to the dies, whose number only the device knows: lists whose
+used part ends anywhere, among them lists longer than one look of a wave."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# experts, choices, tokens, how many experts are chosen at all: one tile, few of many, all, more than 64 in the list
+@pytest.mark.parametrize("count,top,tokens,chosen", [(2, 1, 96, 1), (6, 2, 145, 6), (16, 2, 400, 2), (40, 4, 640, 40), (70, 1, 3500, 3), (70, 1, 3500, 70), (3, 1, 9000, 3)])
+def test_every_tile_in_use_is_made_once(count, top, tokens, chosen):
+    from llm_runtime_study_amd.kernels import ops
+
+    n, k = 260, 64
+    g = torch.Generator().manual_seed(count + tokens)
+    x = torch.randn(tokens, k, generator=g).to(torch.bfloat16)
+    w = torch.randn(count, n, k, generator=g).to(torch.bfloat16)
+    ids = torch.stack([torch.randperm(chosen, generator=g)[:top] for _ in range(tokens)]).to(torch.int32)
+    tile, tiles = ops.moe_tile_rows(tokens * top, count), ops.moe_max_tiles(tokens * top, count)
+    assert tile == 128
+    sorted_pairs, place = torch.empty(tiles * tile, dtype=torch.int32, device="cuda"), torch.empty(tokens * top, dtype=torch.int32, device="cuda")
+    tile_expert = torch.empty(tiles, dtype=torch.int32, device="cuda")
+    ops.moe_align(ids.cuda(), count, sorted_pairs, place, tile_expert)
+    out = torch.full((tiles * tile, n), -7.0, device="cuda")
+    ops.moe_experts(out, x.cuda(), w.cuda(), sorted_pairs, tile_expert, tile, top, gather=True, relu_squared=False)
+    got, listed = out.cpu(), sorted_pairs.cpu()
+    assert (got[listed < 0] == -7.0).all()                      # rows that only pad are not written
+    rows = got[place.cpu().long()].double().view(tokens, top, n)
+    for e in range(chosen):
+        t, c = (ids == e).nonzero(as_tuple=True)
+        want = x[t].double() @ w[e].double().T
+        size = x[t].double().abs() @ w[e].double().abs().T
+        assert ((rows[t, c] - want).abs() <= k * 2.0 ** -23 * size).all()        # float32 sums of k exact products, whatever their order
