@@ -1,0 +1,28 @@
+"""Products of many bfloat16 rows with at most 64 weight rows: remainders of rows, outputs and K, strides, and what is done
+with the sum."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 4, 32), (17, 16, 256), (128, 64, 4096), (129, 12, 96), (100, 16, 64), (300, 20, 1056), (257, 36, 2016), (511, 64, 544), (2048, 32, 4096), (9000, 60, 160)])
+def test_few_outputs_of_many_rows(m, n, k):
+    from llm_runtime_study_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k + 8, generator=g).to(torch.bfloat16).cuda()[:, :k]
+    w = torch.randn(n, k, generator=g).to(torch.bfloat16).cuda()
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    bound = k * 2.0 ** -23 * size                  # float32 sums of k exact products, whatever their order
+    wide = torch.full((m + 1, n + 4), -7.0, device="cuda")
+    ops.gemm(wide[:m, :n], x, w)
+    assert ((wide[:m, :n].double() - want).abs() <= bound).all()
+    assert (wide[m] == -7.0).all() and (wide[:, n:] == -7.0).all()
+    added = torch.ones(m, n, device="cuda")
+    ops.gemm(added, x, w, accumulate=True)
+    assert ((added.double() - 1.0 - want).abs() <= bound + 2.0 ** -23 * (1.0 + want.abs())).all()
+    short = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+    ops.gemm(short, x, w)
+    assert ((short.double() - want).abs() <= bound + 2.0 ** -8 * (want.abs() + bound)).all()
