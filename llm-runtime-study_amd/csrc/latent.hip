@@ -478,15 +478,29 @@ __global__ __launch_bounds__(256) void latent_attention_bf16_kernel(
   }
 }
 
+// a of lanes 0-31 plus a of lanes 32-63 in the former, b likewise in the latter.
+__device__ __forceinline__ float add_halves(float a, float b) {
+  const auto swapped = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(swapped[0]) + __uint_as_float(swapped[1]);
+}
+// The same within each pair of rows of 16 lanes: a's sum in even rows, b's in odd ones.
+__device__ __forceinline__ float add_rows(float a, float b) {
+  const auto swapped = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(swapped[0]) + __uint_as_float(swapped[1]);
+}
+
 // The same for latent rows of 128, 256 or 512 values with 64 rotated dims behind them (CT tiles of 16 latent columns), whose tiles go from
 // memory straight into LDS: a workgroup's four waves (16 rows each) share them, and three tiles of 32 keys are on their way while one
 // is worked on.  The kernel above waits for memory four times a tile, 9 us in all; 16 tokens of 32 heads at 3,072
-// positions took 71-81 us with their merge, 31 here (a prompt of 2,048 tokens 1,535 and 322).  A tile is read once for both products: as rows for the scores (keys x queries:
-// a lane ends with eight keys' scores of one query, which are the second product's operand as they stand), and through the transposing
-// LDS read for the values (columns x queries: a lane's sums are of the same query), so the copy by columns is not read at all.
-// Piece c (16 bytes) of key row k lies at place c ^ turn(k): eight consecutive rows then meet every bank once, for whole pieces
-// and for the halves that the transposing read takes.  One wave a SIMD: its turn of some 3,000 cycles, 1,088 of them products, bounds
-// a prompt; a decode step the trips to memory before the first tile, 1.4 us a tile and the merge.
+// positions took 70 us in 16 parts and 81 in 32 with their merge, 34 and 47 here (a prompt of 2,048 tokens 1,534 and 451).  A tile is read
+// once for both products: as rows for the scores (keys x queries: a lane ends with eight keys' scores of one query, which are the second
+// product's operand as they stand), and through the transposing LDS read for the values (columns x queries: a lane's sums are of the same
+// query), so the copy by columns is not read at all.  Piece c (16 bytes) of key row k lies at place c ^ turn(k): the eight rows that are read
+// together then meet every bank once, for whole pieces and for the halves that the transposing read takes.  One wave a SIMD: its turn of
+// some 4,000 cycles, 1,088 of them products, bounds a prompt; a decode step the trips to memory before the first tile, 1.7 us a tile and the merge.
+// The results are the kernel above's bit for bit: a tile's keys meet the products in its order, maxima and sums move as there, and the keys are
+// divided as there.  With sums in another order and maxima that moved in steps of 2^8 a prompt took 317 us and the tokens 29 and 43, but
+// scores of experts behind such layers that were nearly equal came out in the other order now and then.
 template <int CT>
 __global__ __launch_bounds__(256) void latent_attention_shared_kernel(
     bf16* __restrict__ out, int out_stride, float* __restrict__ part_o, float* __restrict__ part_ml, const bf16* __restrict__ queries,
@@ -504,18 +518,26 @@ __global__ __launch_bounds__(256) void latent_attention_shared_kernel(
   const int rows = (group_count ? group_count[group] : 1) * heads;
   const int block_row0 = blockIdx.y * 64;
   if (block_row0 >= rows) return;
-  const int last_row = (block_row0 + 63 < rows ? block_row0 + 63 : rows - 1);
   const int* table = block_table + (int64_t)token_request[token0] * table_stride;
-  const int pos_first = positions[token0 + block_row0 / heads], pos_last = positions[token0 + last_row / heads];
-  const int lo = first_seen(pos_first, window);
-  const int first_tile = lo / 32, last_tile = pos_last / 32, first_run = lo / 16, last_run = pos_last / 16;
-  const int per_split = (last_tile - first_tile + splits) / splits;
-  const int tile_begin = first_tile + split * per_split;
-  const int tile_end = tile_begin + per_split <= last_tile + 1 ? tile_begin + per_split : last_tile + 1;
+  // A wave divides the keys that its own rows see, as the kernel above does, so that their sums are the same; the workgroup walks
+  // the tiles that some wave works on.
+  const int row_here = block_row0 + lane < rows ? block_row0 + lane : rows - 1;
+  const int pos_here = positions[token0 + row_here / heads];               // of row block_row0 + lane
+  const int lo = first_seen(__builtin_amdgcn_readlane(pos_here, 0), window), pos_last = __builtin_amdgcn_readlane(pos_here, 63);
+  const int first_run = lo / 16, last_run = pos_last / 16;
+  int tile_begin = pos_last / 32 + 1, tile_end = 0, my_begin = 0, my_end = 0;      // my_end 0: a wave without rows only brings tiles in
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    if (block_row0 + 16 * w >= rows) break;
+    const int first_tile = first_seen(__builtin_amdgcn_readlane(pos_here, 16 * w), window) / 32, last_tile = __builtin_amdgcn_readlane(pos_here, 16 * w + 15) / 32;
+    const int per_split = (last_tile - first_tile + splits) / splits, begin = first_tile + split * per_split;
+    const int end = begin + per_split <= last_tile + 1 ? begin + per_split : last_tile + 1;
+    if (w == wave) my_begin = begin, my_end = end;
+    if (begin < end) tile_begin = begin < tile_begin ? begin : tile_begin, tile_end = end > tile_end ? end : tile_end;
+  }
 
   // this lane's row: a (token, head) pair
   const int row0 = block_row0 + wave * 16;
-  const bool works = row0 < rows;                                          // a wave without rows only brings tiles in
   const int mine = row0 + col;
   const bool live = mine < rows;
   const int token = token0 + (live ? mine / heads : 0), head = live ? mine % heads : 0;
@@ -531,7 +553,7 @@ __global__ __launch_bounds__(256) void latent_attention_shared_kernel(
   for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[ks]));
 
   // What this lane brings of a tile: piece p = (wave + 4 i) * 64 + lane of the first run's 16 rows, then the second's
-  auto turn_of = [](int row) { return ((row >> 1) & 3) << 1; };
+  auto turn_of = [](int row) { return (row & 2) | (row >> 1 & 4); };
   unsigned offset[EACH];
 #pragma unroll
   for (int i = 0; i < EACH; ++i) {
@@ -558,10 +580,11 @@ __global__ __launch_bounds__(256) void latent_attention_shared_kernel(
     for (int i = 0; i < EACH; ++i)
       fetch_to_lds(base[wave + 4 * i < FETCHES / 2 ? 0 : 1], offset[i], tiles_address + (unsigned)(stage * STAGE + (wave + 4 * i) * 1024));
   };
-  // where this lane reads: key row `col` (and col + 16) for the scores; four keys 4 g .. (and 16 on), four columns for the values
-  const int swap = turn_of(col);
-  const int key_at[2] = {col * ROW + ((g ^ swap) * 16), col * ROW + (((4 + g) ^ swap) * 16)};           // even and odd steps of 32 dims
-  const int value_row = 4 * g + (col >> 2);
+  // where this lane reads: for the scores the first four keys of eight (and the four behind them), so that a lane group ends with
+  // the scores of eight keys in a row; for the values the same keys, 8 g .. and the four behind, at four columns
+  const int key_row = 8 * (col >> 2) + (col & 3), swap = turn_of(key_row);
+  const int key_at[2] = {key_row * ROW + ((g ^ swap) * 16), key_row * ROW + (((4 + g) ^ swap) * 16)};   // even and odd steps of 32 dims
+  const int value_row = 8 * g + (col >> 2);
   int value_at[4];
 #pragma unroll
   for (int c = 0; c < 4; ++c) value_at[c] = value_row * ROW + (((2 * c + ((col & 3) >> 1)) ^ turn_of(value_row)) * 16) + (col & 1) * 8;
@@ -570,8 +593,7 @@ __global__ __launch_bounds__(256) void latent_attention_shared_kernel(
 #pragma unroll
   for (int c = 0; c < CT; ++c) acc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
   const float scale2 = scale * LOG2E;
-  float top = -INFINITY, total = 0.f;                                      // in powers of two; total: of this lane's keys
-  constexpr float STEP = 8.f;                                              // how far a maximum may pass the reference before that moves
+  float top = -INFINITY, total = 0.f;                                      // in powers of two
   if (tile_begin < tile_end) {
 #pragma unroll
     for (int i = 0; i < STAGES - 1; ++i) {
@@ -584,15 +606,23 @@ __global__ __launch_bounds__(256) void latent_attention_shared_kernel(
   for (int tile = tile_begin; tile < tile_end; ++tile) {
     // this tile is there, and the stage of the one before has been read by everyone
     fetched_and_read_then_barrier<(STAGES - 2) * EACH>();
+    unsigned char* at = tiles + stage * STAGE;
+    if (tile * 32 < lo || tile * 32 + 31 > pos_last) {
+      // keys that no row sees: a slot that nothing was written to may hold a NaN, which a weight of zero does not take away
+      for (int piece = threadIdx.x; piece < 32 * PIECES; piece += 256) {
+        const int key = tile * 32 + piece / PIECES;
+        if (key < lo || key > pos_last) *(bf16x8*)(at + piece * 16) = zero;
+      }
+      fetched_and_read_then_barrier<(STAGES - 2) * EACH>();
+    }
     fetch(tile + STAGES - 1, (stage + STAGES - 1) % STAGES);               // past the end: the last run once more
     look_up(tile + STAGES);
-    const unsigned char* at = tiles + stage * STAGE;
     stage = (stage + 1) % STAGES;
-    if (!works) continue;
+    if (tile < my_begin || tile >= my_end) continue;
     // fragments are asked for AHEAD products before their own; the fences keep the order (left alone, the compiler waits for each)
     floatx4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
     bf16x8 kf[AHEAD];
-    auto keys = [&](int f) { return *(const bf16x8*)(at + key_at[f >> 1 & 1] + (f >> 2) * 128 + (f & 1) * 16 * ROW); };
+    auto keys = [&](int f) { return *(const bf16x8*)(at + key_at[f >> 1 & 1] + (f >> 2) * 128 + (f & 1) * 4 * ROW); };
 #pragma unroll
     for (int f = 0; f < AHEAD; ++f) kf[f] = keys(f);
     __builtin_amdgcn_sched_barrier(0);
@@ -608,7 +638,7 @@ __global__ __launch_bounds__(256) void latent_attention_shared_kernel(
       typedef __attribute__((address_space(3))) const unsigned char lds_byte;
       lds_byte* from_lds = (lds_byte*)(at + value_at[c & 3] + (c >> 2) * 128);
       v[0] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)from_lds);
-      v[1] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(from_lds + 16 * ROW));
+      v[1] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(from_lds + 4 * ROW));
     };
 #pragma unroll
     for (int c = 0; c < AHEAD; ++c) values(c, vf[c]);
@@ -618,27 +648,28 @@ __global__ __launch_bounds__(256) void latent_attention_shared_kernel(
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int key = tile * 32 + h * 16 + 4 * g + i;
+        const int key = tile * 32 + 8 * g + h * 4 + i;
         s[h][i] = key <= pos && key >= from ? s[h][i] * scale2 : -INFINITY;
         most = fmaxf(most, s[h][i]);
       }
     most = fmaxf(most, __shfl_xor(most, 16, WAVE));
     most = fmaxf(most, __shfl_xor(most, 32, WAVE));
-    const float now = most > top + STEP || top == -INFINITY ? most : top;
+    const float now = fmaxf(top, most);
     const float ref = now == -INFINITY ? 0.f : now;                        // a row that has seen no key yet
-    const float shrink = now == top ? 1.f : __builtin_amdgcn_exp2f(top - ref);
+    const float shrink = __builtin_amdgcn_exp2f(top - ref);                // 0 while the old maximum is -inf
     top = now;
     bf16x8 weights;
-    float sum = 0.f;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float e = __builtin_amdgcn_exp2f(s[h][i] - ref);
-        sum += e;
-        weights[h * 4 + i] = (bf16)e;
+        s[h][i] = __builtin_amdgcn_exp2f(s[h][i] - ref);
+        weights[h * 4 + i] = (bf16)s[h][i];
       }
-    total = total * shrink + sum;
+    // The weights' sum over the tile's 32 keys in the order in which the kernel above adds them: keys 16 apart, then 8, 4, 2, 1.  A
+    // swap of halves (or of neighbouring rows of 16 lanes) and an addition do two numbers' step, and leave half of the lanes with either.
+    // They lie between the products, which leave the vector unit time for them.
+    float half[4], quarter[2], sum;
     if (__any(shrink != 1.f)) {
 #pragma unroll
       for (int c = 0; c < CT; ++c) acc[c] *= shrink;
@@ -650,12 +681,16 @@ __global__ __launch_bounds__(256) void latent_attention_shared_kernel(
       const bf16x8 v = {first[0], first[1], first[2], first[3], second[0], second[1], second[2], second[3]};
       acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, weights, acc[c], 0, 0, 0);
       if (c + AHEAD < CT) values(c + AHEAD, vf[c % AHEAD]);
+      if (c < 4) half[c] = add_halves(s[0][c], s[1][c]);                               // lanes 0-31 hold keys 8 g + c, the others 8 g + 4 + c
+      else if (c == 4) quarter[0] = add_rows(half[0], half[2]), quarter[1] = add_rows(half[1], half[3]);        // odd rows hold the second
+      else if (c == 5) sum = add_halves(quarter[0], quarter[1]);                       // 4 apart; lanes 0-31 hold the first
+      else if (c == 6) sum = add_rows(sum, sum);
+      else if (c == 7) sum = add_halves(sum, sum);
       __builtin_amdgcn_sched_barrier(0);
     }
+    total = total * shrink + sum;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                         // the fetches past the end
-  total += __shfl_xor(total, 16, WAVE);
-  total += __shfl_xor(total, 32, WAVE);
   if (!live) return;
   if (splits > 1) {
     const int64_t part = ((int64_t)token * heads + head) * splits + split;

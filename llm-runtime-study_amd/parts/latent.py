@@ -185,14 +185,14 @@ class LatentAttention(Part):
 
 
     @staticmethod
-    def _splits_alone(workgroups: int, longest: int, a_unit: int = 2) -> int:
-        """Into how many workgroups the keys of a single token are divided: towards as many workgroups a compute unit as the kernel
-        has room for (`a_unit`), at least 64 keys each (two tiles; a power of two that follows the length's class, so that eager steps and graph replays agree);
+    def _splits_alone(workgroups: int, longest: int) -> int:
+        """Into how many workgroups the keys of a single token are divided: towards two workgroups a compute unit, at least
+        64 keys each (two tiles; a power of two that follows the length's class, so that eager steps and graph replays agree);
         a workgroup walks its tiles one after the other, so a long context in few workgroups is a matter of latency."""
         units = ops.compute_units()
-        if workgroups >= a_unit * units:
+        if workgroups >= 2 * units:
             return 1
-        return max(1, min(-(-a_unit * units // workgroups), length_class(longest) // 64, 64))
+        return max(1, min(-(-2 * units // workgroups), length_class(longest) // 64, 64))
 
     def _attend_groups(self, ctx, latent, queries, gate, cache, group):
         """The matrix-core kernel: decode steps token by token, the single tokens at the head of a mixed step likewise, the
@@ -211,7 +211,7 @@ class LatentAttention(Part):
             longest = ctx.max_k if ctx.all_decode else ctx.max_k_bound
             if self.span is not None:
                 longest = min(longest, self.span + 32)
-            splits = self._splits_alone(rows * tiles, longest, 1 if ops.latent_attention_groups_shares(r, self.width, group.page_size) else 2)
+            splits = self._splits_alone(rows * tiles, longest)
             part_o, part_ml = parts("single", rows, splits)
             ops.latent_attention_groups(latent[:rows], queries[:rows], cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot, ctx.positions,
                                         None, None, 1, r, self.scale, sink=self.sink, gate=None if gate is None else gate[:rows], window=window,
