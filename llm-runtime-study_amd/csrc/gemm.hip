@@ -431,67 +431,61 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_lines_kernel(void* __restric
 // ------------------------------------------------- bf16 kernel for many rows and few outputs
 // Products of a step's rows with at most 64 weight rows (a router's logits, a gate's): the time is the time to read x
 // once, and a tile of 128 rows x 256 outputs is mostly padding on a handful of workgroups.  One workgroup owns 16 rows of
-// x and all the outputs; its eight waves take the 128-byte lines of K in turn and add their partial sums through LDS
-// in a fixed order.  The weights (256 KB at 32 x 4096) are read again by every workgroup, from L2, which is what bounds
-// it.  n 32, k 4096, before and now: 64 rows 24 and 12 us, 136 rows 58 and 12, 2,048 rows 59 and 13; n 64, 2,048 rows 59
-// and 20; n 8, k 2048, 2,048 rows 31 and 5.
+// x and all the outputs.  Memory writes slices of 256 of K into LDS, a wave's share the 32 of one product: 16 rows at 32 of K are
+// a fragment, which lies there lane by lane.  A wave for each 16 outputs multiplies, its sums one chain over K: the bits of the
+// kernel above for many rows, which this one stands in for (experts with nearly equal scores are told apart by the last one).
+// What bounds it is a workgroup's way from the L2s, x and all the weights once.  us of the kernel above and of this one: 2,048 rows n 8
+// k 2,048 31 and 6, n 32 k 4,096 59 and 16, n 64 k 4,096 59 and 23; 128 rows n 8 k 2,048 30 and 6.  With K dealt to the eight waves and their
+// sums added up n 32 took 13 us and n 64 20, in another order.
 constexpr int NARROW_MAX = 64, NARROW_WAVES = 8;
 template <int NT, int MODE>
 __global__ __launch_bounds__(NARROW_WAVES* WAVE) void gemm_bf16_narrow_kernel(void* __restrict__ out, const bf16* __restrict__ x,
                                                                               const bf16* __restrict__ w, int m, int n, int k, int lda, int ldc) {
-  constexpr int STRIDE = NT * 16 + 4, AHEAD = NT <= 2 ? 4 : 2;         // lines asked for before any is used
-  __shared__ __attribute__((aligned(16))) float part[NARROW_WAVES][16][STRIDE];
-  const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE, r = lane & 15, g = lane >> 4;
-  const int m0 = blockIdx.x * 16, row = m0 + r < m ? m0 + r : m - 1;
-  const bf16* xp = x + (int64_t)row * lda + g * 8;
-  const bf16* wp[NT];
+  constexpr int STEPS = NARROW_WAVES, BLOCK = 512, STAGE = STEPS * (1 + NT) * BLOCK, STAGES = NT <= 2 ? 6 : 4, EACH = 1 + NT;   // elements
+  __shared__ __attribute__((aligned(64))) bf16 slices[STAGES * STAGE];
+  const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), r = lane & 15, g = lane >> 4;
+  const int m0 = blockIdx.x * 16;
+  const unsigned x_lane = (unsigned)((m0 + r < m ? r : m - 1 - m0) * lda + g * 8) * 2u;
+  unsigned w_lane[NT];
 #pragma unroll
-  for (int j = 0; j < NT; ++j) wp[j] = w + (int64_t)(j * 16 + r < n ? j * 16 + r : n - 1) * k + g * 8;
-  floatx4 acc[NT];
+  for (int j = 0; j < NT; ++j) w_lane[j] = (unsigned)((j * 16 + r < n ? j * 16 + r : n - 1) * k + g * 8) * 2u;
+  const int steps = k / 32, rounds = (steps + STEPS - 1) / STEPS;
+  const unsigned to = (unsigned)(uintptr_t)(__attribute__((address_space(3))) bf16*)slices + (unsigned)(wave * (1 + NT) * BLOCK * 2);
+  auto fetch = [&](int round, int stage) {
+    const int step = round * STEPS + wave;
+    const int64_t at = (step < steps ? step : steps - 1) * 64;            // past K the last step once more, not multiplied
+    fetch_to_lds((const char*)(x + (int64_t)m0 * lda) + at, x_lane, to + (unsigned)(stage * STAGE * 2));
 #pragma unroll
-  for (int j = 0; j < NT; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const int steps = k / 32, whole = steps / 2;                          // steps of 32; lines of 64 that are whole
-  auto walk = [&](int first, auto lines) {                              // lines first, first + 8, ...
-    constexpr int L = decltype(lines)::value;
-    bf16x8 xf[L][2], wf[L][2][NT];
+    for (int j = 0; j < NT; ++j) fetch_to_lds((const char*)w + at, w_lane[j], to + (unsigned)(stage * STAGE * 2 + (1 + j) * BLOCK * 2));
+  };
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int u = 0; u < L; ++u)
+  for (int round = 0; round < STAGES - 1; ++round) fetch(round, round);
+  int stage = 0;
+  for (int round = 0; round < rounds; ++round) {
+    fetched_and_read_then_barrier<(STAGES - 2) * EACH>();                 // this slice is there, and the one before was read by everyone
+    fetch(round + STAGES - 1, stage == 0 ? STAGES - 1 : stage - 1);
+    if (wave < NT) {
+      const bf16* at = slices + stage * STAGE + lane * 8;
+      bf16x8 xf[STEPS], wf[STEPS];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int at = (first + u * NARROW_WAVES) * 64 + h * 32;
-        xf[u][h] = *(const bf16x8*)(xp + at);
-#pragma unroll
-        for (int j = 0; j < NT; ++j) wf[u][h][j] = *(const bf16x8*)(wp[j] + at);
+      for (int u = 0; u < STEPS; ++u) {
+        xf[u] = *(const bf16x8*)(at + u * (1 + NT) * BLOCK);
+        wf[u] = *(const bf16x8*)(at + (u * (1 + NT) + 1 + wave) * BLOCK);
       }
 #pragma unroll
-    for (int u = 0; u < L; ++u)
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][h][j], xf[u][h], acc[j], 0, 0, 0);
-  };
-  int line = wave;
-  for (; line + (AHEAD - 1) * NARROW_WAVES < whole; line += AHEAD * NARROW_WAVES) walk(line, std::integral_constant<int, AHEAD>());
-  for (; line < whole; line += NARROW_WAVES) walk(line, std::integral_constant<int, 1>());
-  if (steps % 2 && wave == whole % NARROW_WAVES) {                      // the half line at the end of K
-    const bf16x8 xf = *(const bf16x8*)(xp + whole * 64);
-#pragma unroll
-    for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(wp[j] + whole * 64), xf, acc[j], 0, 0, 0);
+      for (int u = 0; u < STEPS; ++u)
+        if (round * STEPS + u < steps) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u], xf[u], acc, 0, 0, 0);
+    }
+    stage = stage == STAGES - 1 ? 0 : stage + 1;
   }
-#pragma unroll
-  for (int j = 0; j < NT; ++j) *(floatx4*)&part[wave][r][j * 16 + 4 * g] = acc[j];
-  __syncthreads();
-  for (int e = tid; e < 16 * NT * 4; e += NARROW_WAVES * WAVE) {
-    const int token = m0 + e / (NT * 4), col = e % (NT * 4) * 4;
-    if (token >= m || col >= n) continue;
-    floatx4 v = *(const floatx4*)&part[0][e / (NT * 4)][col];
-#pragma unroll
-    for (int p = 1; p < NARROW_WAVES; ++p) v += *(const floatx4*)&part[p][e / (NT * 4)][col];
-    const int64_t at = (int64_t)token * ldc + col;
-    if constexpr (MODE == OUT_STORE) *(bf16x4*)((bf16*)out + at) = bf16x4{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
-    else if constexpr (MODE == OUT_STORE_F32) *(floatx4*)((float*)out + at) = v;
-    else *(floatx4*)((float*)out + at) = *(const floatx4*)((const float*)out + at) + v;
-  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                        // the fetches past K
+  const int token = m0 + r, col = wave * 16 + 4 * g;
+  if (wave >= NT || token >= m || col >= n) return;
+  const int64_t at = (int64_t)token * ldc + col;
+  if constexpr (MODE == OUT_STORE) *(bf16x4*)((bf16*)out + at) = bf16x4{(bf16)acc[0], (bf16)acc[1], (bf16)acc[2], (bf16)acc[3]};
+  else if constexpr (MODE == OUT_STORE_F32) *(floatx4*)((float*)out + at) = acc;
+  else *(floatx4*)((float*)out + at) = *(const floatx4*)((const float*)out + at) + acc;
 }
 
 // ------------------------------------------------- bf16 kernel for few rows
@@ -1814,23 +1808,7 @@ LRS_API int lrs_gemm(void* out, int mode, const void* a, const void* w, const vo
   } else if (dtype == LRS_BF16) {
     const bool mid = aligned && m > 16 && m <= 128 && !normed && !bias && tune.mid && k % 256 == 0 && n % 16 == 0 && ldc % 4 == 0 &&
                      (uintptr_t)out % 16 == 0;
-    // few outputs of more rows than the few-rows kernel's, where the kernel of whole lines does not divide K (4,096 rows,
-    // n 64, k 4096: 16 us divided, 21 here); up to 32 rows the middle kernel is ahead with more than 32 outputs (k 4096:
-    // 17 us against 19; n 32: 17 against 12)
-    const bool narrow = aligned && n <= NARROW_MAX && n % 4 == 0 && k % 32 == 0 && ldc % 4 == 0 && (uintptr_t)out % 16 == 0 && !normed && !swiglu &&
-                        !bias && (m > 64 || (mid && (m > 32 || n <= 32))) && !(m > 128 && (lrs_gemm_lines_splits(m, n, k) || lrs_gemm_lines_width(m, n, k)));
-    if (narrow) {
-#define NARROW(NT, MODE) gemm_bf16_narrow_kernel<NT, MODE><<<(m + 15) / 16, NARROW_WAVES * WAVE, 0, s>>>(out, (const bf16*)a, (const bf16*)w, m, n, k, lda, ldc)
-#define NARROW_OF(NT)                                    \
-      if (mode == OUT_STORE) NARROW(NT, OUT_STORE);        \
-      else if (mode == OUT_STORE_F32) NARROW(NT, OUT_STORE_F32); \
-      else NARROW(NT, OUT_ADD_F32)
-      if (n <= 16) { NARROW_OF(1); }
-      else if (n <= 32) { NARROW_OF(2); }
-      else { NARROW_OF(4); }
-#undef NARROW_OF
-#undef NARROW
-    } else if (aligned && (m <= 64 || mid)) {
+    if (aligned && (m <= 64 || mid)) {
       const bf16 *wp = (const bf16*)w, *bp = (const bf16*)bias;
       const NormInput norm{(const float*)a, rows, norm_weight, norm_weight_dtype == LRS_F32, eps};
       const bf16* ap = normed ? nullptr : (const bf16*)a;
@@ -1868,6 +1846,17 @@ LRS_API int lrs_gemm(void* out, int mode, const void* a, const void* w, const vo
         else { LINES_OF(128); }
 #undef LINES_OF
 #undef LINES
+      } else if (n <= NARROW_MAX && !swiglu) {
+#define NARROW(NT, MODE) gemm_bf16_narrow_kernel<NT, MODE><<<(m + 15) / 16, NARROW_WAVES * WAVE, 0, s>>>(out, (const bf16*)a, (const bf16*)w, m, n, k, lda, ldc)
+#define NARROW_OF(NT)                                    \
+        if (mode == OUT_STORE) NARROW(NT, OUT_STORE);        \
+        else if (mode == OUT_STORE_F32) NARROW(NT, OUT_STORE_F32); \
+        else NARROW(NT, OUT_ADD_F32)
+        if (n <= 16) { NARROW_OF(1); }
+        else if (n <= 32) { NARROW_OF(2); }
+        else { NARROW_OF(4); }
+#undef NARROW_OF
+#undef NARROW
       } else {
         const int tiles_m = (m + 127) / 128, tiles_n = (n + 255) / 256;
 #define WIDE(SW, MODE) gemm_bf16_wide_kernel<SW, MODE><<<tiles_m * tiles_n, 256, 0, s>>>(out, (const bf16*)a, (const bf16*)w, m, n, k, lda, ldc, tiles_m, tiles_n)

@@ -26,3 +26,16 @@ def test_few_outputs_of_many_rows(m, n, k):
     short = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
     ops.gemm(short, x, w)
     assert ((short.double() - want).abs() <= bound + 2.0 ** -8 * (want.abs() + bound)).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 4, 32), (70, 64, 224), (129, 12, 96), (100, 16, 64), (300, 20, 1056), (257, 36, 2016), (2048, 32, 4096), (2048, 64, 2048), (1000, 8, 544)])
+def test_few_outputs_have_the_bits_of_many(m, n, k):
+    """A row's outputs are the same whether its weight rows stand alone or among more than one such kernel takes."""
+    from llm_runtime_study_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w = torch.randn(m, k, generator=g).to(torch.bfloat16).cuda(), torch.randn(128, k, generator=g).to(torch.bfloat16).cuda()
+    few, many = torch.empty(m, n, device="cuda"), torch.empty(m, 128, device="cuda")
+    ops.gemm(few, x, w[:n])
+    ops.gemm(many, x, w)
+    assert torch.equal(few, many[:, :n])
