@@ -66,6 +66,13 @@ class ScratchArena:
         # address down (a captured graph, a recorded plan) then holds a stale address.  A buffer made for
         # the first time moves nothing.
         self.generation = 0
+        self._library = None
+
+    def library(self) -> "ops.LibraryState":
+        """What this runner's products by the vendor's library share, made when the first of them is."""
+        if self._library is None:
+            self._library = ops.LibraryState()
+        return self._library
 
     def get(self, name: str, shape: tuple, dtype: torch.dtype, zeroed: bool = False) -> torch.Tensor:
         """The buffer `name` with at least shape[0] rows.  zeroed: all zero when it is made (for buffers whose
@@ -138,6 +145,9 @@ class StepContext:
 
     def scratch(self, name: str, shape: tuple, dtype: torch.dtype) -> torch.Tensor:
         return self._runner.arena.get(name, shape, dtype)
+
+    def library_state(self) -> "ops.LibraryState":
+        return self._runner.arena.library()
 
     def group(self, index: int) -> GroupStep:
         return self._groups[index]

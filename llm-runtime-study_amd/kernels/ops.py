@@ -14,6 +14,7 @@ import threading
 from dataclasses import dataclass
 import ctypes
 import struct
+import weakref
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p, POINTER, byref
 
 import torch
@@ -114,7 +115,9 @@ _SIGNATURES = {
     "lrs_probe_lines": (c_int, [c_void_p, c_size_t, c_void_p, c_int, c_int, c_size_t, c_int, c_void_p]),
     "lrs_gemm_prepare": (c_int, []),
     "lrs_library_gemm_prepare": (c_int, []),
-    "lrs_library_gemm": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p]),
+    "lrs_library_open": (c_int, [POINTER(c_void_p)]),
+    "lrs_library_close": (c_int, [c_void_p]),
+    "lrs_library_gemm": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p]),
     "lrs_host_device_pointer": (c_int, [c_void_p, POINTER(c_void_p)]),
     "lrs_gemm_mid_shape": (c_int, [c_int, c_int, c_int, c_void_p, c_void_p]),
     "lrs_gemm_mid_deal": (c_int, [c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p]),
@@ -896,16 +899,28 @@ def gemm_lines_add_rmsnorm(residual: torch.Tensor, a: torch.Tensor, w: torch.Ten
             *_workspace(workspace, "gemm_lines_add_rmsnorm"), _stream())
 
 
-def library_gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> None:
+class LibraryState:
+    """The handle and the workspace of the vendor's matrix library for products that follow each other on one stream: a runner
+    has one of its own, since products that run at the same time must not share one.  Given back with the object."""
+
+    def __init__(self):
+        address = c_void_p()
+        _check(library().lrs_library_open(byref(address)))
+        self.address = address.value
+        weakref.finalize(self, library().lrs_library_close, self.address).atexit = False
+
+
+def library_gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, state: LibraryState | None = None) -> None:
     """out [M, N] = a [M, K] @ w[N, K].T by the vendor's matrix library (bfloat16 inputs, float32 sums; out bfloat16
-    or float32): for products of more rows than this package's own kernels are made for."""
+    or float32): for products of more rows than this package's own kernels are made for.  state: the caller's own (unless given,
+    the one the process keeps: products on one stream only)."""
     m, k = a.shape
     n = w.shape[0]
     _need(a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] == k and w.is_contiguous(),
           f"library_gemm: a and w must be bfloat16, w contiguous [N, {k}]")
     _need(out.shape == (m, n) and out.dtype in (torch.bfloat16, torch.float32), f"library_gemm: out must be bfloat16 or float32 [{m}, {n}]")
     _launch("lrs_library_gemm", _dev(out, "out"), 1 if out.dtype == torch.float32 else 0, _dev(a, "a"), _dev(w, "w"), m, n, k,
-                                      _rows(a, "a"), _rows(out, "out"), _stream())
+                                      _rows(a, "a"), _rows(out, "out"), None if state is None else state.address, _stream())
 
 
 NORM_CHAIN_MAX_ROWS = 16

@@ -91,6 +91,12 @@ def workspace_of(ctx) -> tuple:
     return known
 
 
+def library_of(ctx) -> "ops.LibraryState | None":
+    """What the step's products by the vendor's library share (one per runner likewise)."""
+    state = getattr(ctx, "library_state", None)
+    return None if state is None else state()
+
+
 ROUTES = ("chain", "mid_scaled", "fused_norm", "mid_begin", "mid", "split_norm", "library", "own")
 
 
@@ -200,10 +206,10 @@ def linear(ctx, out, x, weight, bias=None, accumulate: bool = False, swiglu: boo
         return normed
     if route == "library":
         if not (accumulate or swiglu):
-            ops.library_gemm(out, x, weight)                      # bfloat16, or the float32 logits of many rows
+            ops.library_gemm(out, x, weight, state=library_of(ctx))                      # bfloat16, or the float32 logits of many rows
             return None
         y = ctx.scratch("library_gemm_out", (m, n), torch.bfloat16)
-        ops.library_gemm(y, x, weight)
+        ops.library_gemm(y, x, weight, state=library_of(ctx))
         if swiglu:
             ops.silu_mul(out, y, interleaved=True)
             return None
