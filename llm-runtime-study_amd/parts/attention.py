@@ -230,19 +230,29 @@ class GQAAttention(Part):
     @classmethod
     def _decode_shape(cls, workgroups: int, longest: int, bound: int, page_size: int, head_dim: int) -> tuple[int, int]:
         """(splits, form) of attention_decode(): workgroups of four waves, two a unit (form 1), divided as _decode_splits says;
-        or, while the batch alone has no more than one workgroup a unit, of eight waves (form 2; heads of up to 128), one a unit
-        and undivided under 1,024 tokens.  A unit streams its workgroup's keys at some 40 GB/s whatever is on its way at once,
-        and a merge costs 3-4 us and the gap before it, so eight waves finish a short context sooner than a merge would: us
-        with four waves / with eight, parts in brackets, merge and gap counted: 16 heads on 8, batch 1 and 16 at 509 tokens 13.5 [1] /
-        11.2 [1] and 14.8 [1] / 12.6 [1], batch 32 at 600 27.4 [2] / 19.8 [1], batch 16 at 1,500 29.0 [4] / 28.1 [2]; 32 heads on 8,
-        batch 1 at 2,048 14.5 [8] / 13.2 [8], batch 8 24.5 [8] / 23.4 [4], batch 24 at 1,500 33.5 [1] / 30.8 [1], batch 8 at 8,192
-        58.2 [8] / 56.1 [4]; but batch 40 at 600 28.3 / 32.6 and batch 64 at 1,500 73.1 / 75.9."""
+        or, while the batch alone has no more than one workgroup a unit, of eight waves (form 2; heads of up to 128), one a unit.
+        A unit streams its workgroup's keys at some 40 GB/s whatever is on its way at once, and a merge costs 3-4 us and the gap
+        before it, so eight waves finish a short context sooner than a merge would.  us with four waves / with eight, parts in
+        brackets, merge counted, 32 heads on 8: batch 1 at 2,048 tokens 14.5 [8] / 13.2 [8], batch 8 24.5 [8] / 23.4 [4], batch 8 at 8,192
+        58.2 [8] / 56.1 [4]; but batch 40 at 600 28.3 / 32.6 and batch 64 at 1,500 73.1 / 75.9.
+          * As many parts as one round of workgroups has room for: a second round that is partly empty costs more than the shorter
+            walks give (batch 24 at 1,500, 192 workgroups: 35.2 [1] / 32.8 [1], 40.8 [2]; 96 workgroups, 32 heads on 4: 24.1 [4] / 21.2 [2],
+            30.4 [3]; 24 workgroups at 8,000, 16 heads on 1: 30.2 [16] / 26.4 [8], 36.4 [11]).
+          * But three for 129 to 160 workgroups from 2,048 tokens on, nearly two full rounds (144 at 3,000: 52.8 [4] / 51.2 [3], 53.8 [1];
+            at 8,000 122 [4] / 111 [3], 128 [1]; at 1,500 32.9 [4] / 30.8 [1], 33.7 [3]).
+          * At least 256 keys each (batch 1 at 900: 14.1 [2] / 12.5 [2], 15.1 [1]; batch 16 at 520, 640, 768 and 900 15.5 / 14.4 [2] 13.4 [1],
+            16.8 / 15.5 16.1, 18.2 / 17.3 18.6, 20.5 / 19.1 21.9), and under 1,024 tokens undivided for smaller heads, whose keys are
+            fewer bytes (64 dims, batch 4 at 520 and 768 10.2 [2] / 8.4 [1] 8.9 [2] and 10.4 / 9.1 9.8)."""
         units = ops.compute_units()
         if workgroups > units or head_dim > 128:
             return cls._decode_splits(workgroups, longest, bound, page_size), 1
         reach = length_class(longest)
-        wanted = 1 if reach < 1024 else min(-(-units // workgroups), reach // 256, 64)
-        return max(wanted, -(-bound // (4096 * page_size))), 2
+        wanted = units // workgroups
+        if 2 * workgroups > units and 8 * workgroups <= 5 * units and reach >= 2048:
+            wanted = 3
+        if head_dim < 128 and reach < 1024:
+            wanted = 1
+        return max(1, min(wanted, reach // 256, 64), -(-bound // (4096 * page_size))), 2
 
     @staticmethod
     def _walks_in_pairs(ctx, heads_per_group: int, head_dim: int) -> bool:

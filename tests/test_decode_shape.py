@@ -1,0 +1,22 @@
+"""Into how many workgroups a decode token's keys are divided: what the rule may not do, over batches, contexts and head sizes."""
+
+import pytest
+
+from llm_runtime_study_amd.kernels import ops
+from llm_runtime_study_amd.parts.attention import GQAAttention
+
+
+@pytest.mark.parametrize("head_dim", [32, 64, 96, 128, 192])
+def test_parts_of_a_decode_step(monkeypatch, head_dim):
+    monkeypatch.setattr(ops, "compute_units", lambda: 256)
+    for workgroups in list(range(1, 300)) + [512, 2048]:
+        for longest in (1, 255, 256, 511, 512, 600, 1023, 1024, 2047, 2048, 5000, 8192, 40000, 140000):
+            splits, form = GQAAttention._decode_shape(workgroups, longest, longest, 16, head_dim)
+            fits = -(-longest // (4096 * 16))                  # what one workgroup's block table entries ask for
+            assert splits >= fits
+            if workgroups > 256 or head_dim > 128:
+                assert (splits, form) == (GQAAttention._decode_splits(workgroups, longest, longest, 16), 1)
+                continue
+            assert form == 2 and (splits <= max(1, longest // 256, fits))
+            # one round of workgroups, or two that are nearly full
+            assert splits == fits or splits * workgroups <= 256 or (splits == 3 and longest >= 2048 and 384 < 3 * workgroups <= 480)
