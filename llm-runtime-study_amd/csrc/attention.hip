@@ -1824,7 +1824,8 @@ __global__ __launch_bounds__(MANY_WAVES ? 512 : 256, MANY_WAVES ? 1 : QB == 1 &&
 // as two launches one waits for the other: 24 tokens at 1,500 are bound by their keys' way from memory, 488 tokens behind as
 // many by the length of a walk in fewer workgroups than the chip has room for.  Here the first single_blocks workgroups
 // (token by token, the kv heads in turn) do what attention_decode_bf16_kernel does with four waves, the others what the
-// kernel above does: 37 and 39 us a layer in two launches (32 heads on 8), 41 in one.  Heads of 128, plain scores, undivided keys.
+// kernel above does with four waves: 77 us a layer in two launches (32 heads on 8), 43 in one; which steps come here: _one_launch in
+// parts/attention.py.  Heads of 128, plain scores, undivided keys.
 template <int QB, int SPREAD, bool PREP>
 __global__ __launch_bounds__(256, 2) void attention_mixed_d128_kernel(
     bf16* __restrict__ out, int out_stride, const bf16* __restrict__ q, int q_stride, bf16* __restrict__ k_pages, bf16* __restrict__ v_pages,

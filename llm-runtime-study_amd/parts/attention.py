@@ -261,6 +261,24 @@ class GQAAttention(Part):
         return heads_per_group == 2 and head_dim == 128 and ctx.max_qblock > 16 and ctx.R - ctx.single_rows == 1
 
     @staticmethod
+    def _one_launch(workgroups: int, splits: int, rest: int, group_size: int, heads_per_group: int, longest: int) -> bool:
+        """Whether a mixed step's single tokens (`workgroups`, divided into `splits` by themselves) and the portion behind them (`rest`
+        workgroups) go in one launch (attention_mixed), the single tokens' keys undivided: neither fills the chip by itself, and two
+        launches wait for each other.  us a layer in two launches / in one, `a` beside `b` tokens after `c`: 32 heads on 8, 24 at 1,500 beside
+        488 after 488 77 / 43; 40 on 8 78 / 60; 64 on 8 80 / 63; 20 at 8,192 beside 2,028 after 0 254 / 163, 295 / 206 and 306 / 213.
+        Not so
+          * single tokens that would be divided, unless they are half a workgroup a unit and more, which the portion's workgroups
+            fill up, and no context is much longer than the others need be: 17 on 8 kv heads, one at 8,192 and the others at 500, beside
+            2,028 145 / 120; at 16,000 171 / 206, at 32,000 224 / 380 (all 17 at 16,000: 348 / 253);
+          * five heads a group and more beside a long portion in groups of 32, whose launch alone has a wave for every head and
+            walks its keys once (csrc/attention.hip, MANY_WAVES), while no context is longer than that walk: 32 on 4, 33 at 500, 1,500
+            and 4,000 beside 2,028 115 / 130, 141 / 130 and 178 / 134, 64 at 500 and 1,500 112 / 138 and 146 / 152."""
+        units = ops.compute_units()
+        if heads_per_group > 4 and group_size > 16 and rest <= units and longest <= 3072:
+            return False
+        return splits == 1 or (2 * workgroups > units and longest <= 8192)
+
+    @staticmethod
     def _prefill_splits(workgroups: int, longest: int, outputs: int, heads_per_group: int = 4, tokens: int = 0, paired: bool = False) -> int:
         """Into how many workgroups the keys of every query group of a ragged step are divided: one, unless
         the groups alone leave compute units idle (a last portion of a prompt, a short portion after a long
@@ -375,10 +393,8 @@ class GQAAttention(Part):
             rest_splits = self._prefill_splits((-(-ctx.num_qblocks // 2) if paired else ctx.num_qblocks) * kv_heads, longest, (t - singles) * nq * d,
                                                nq // kv_heads, t - singles, paired)
             splits, form = self._decode_shape(singles * kv_heads, longest, ctx.max_k_bound, group.page_size, d) if singles else (1, 1)
-            if (singles and d == 128 and (splits == 1 or 2 * singles * kv_heads > ops.compute_units()) and rest_splits == 1 and ctx.max_k_bound <= 4096 * group.page_size):
-                # both kinds of rows in one launch: neither fills the chip by itself, and two launches would wait for each other
-                # (24 tokens at 1,500 beside 488 behind 488: 37 + 39 us a layer, 41 in one launch).  Single tokens whose keys would be
-                # divided come along where they are half a workgroup a unit and more: the portion's workgroups fill the rest
+            if (singles and d == 128 and rest_splits == 1 and ctx.max_k_bound <= 4096 * group.page_size
+                    and self._one_launch(singles * kv_heads, splits, ctx.num_qblocks * kv_heads, ctx.max_qblock, nq // kv_heads, longest)):
                 ops.attention_mixed(out, qkv, cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot, ctx.positions, singles, ctx.qblock_token0,
                                     ctx.qblock_count, nq, self.scale, self.reach, ctx.max_qblock, ctx.max_k_bound, queries_raw, one_request=paired)
                 return linear(ctx, residual, out, self.w_o, accumulate=accumulate, then_norm=then_norm)

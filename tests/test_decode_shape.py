@@ -20,3 +20,18 @@ def test_parts_of_a_decode_step(monkeypatch, head_dim):
             assert form == 2 and (splits <= max(1, longest // 256, fits))
             # one round of workgroups, or two that are nearly full
             assert splits == fits or splits * workgroups <= 256 or (splits == 3 and longest >= 2048 and 384 < 3 * workgroups <= 480)
+
+
+def test_which_mixed_steps_go_in_one_launch(monkeypatch):
+    monkeypatch.setattr(ops, "compute_units", lambda: 256)
+
+    def one(singles, nq, nkv, bound, portion, size):
+        splits, _ = GQAAttention._decode_shape(singles * nkv, bound, bound, 16, 128)
+        return GQAAttention._one_launch(singles * nkv, splits, -(-portion // size) * nkv, size, nq // nkv, bound)
+
+    assert one(24, 32, 8, 1536, 488, 16) and one(24, 40, 8, 1536, 488, 16) and one(24, 32, 8, 60160, 2028, 32)
+    assert not one(8, 32, 8, 1536, 488, 16)
+    # a decoding request far on among short ones: its keys are divided in a launch of their own
+    assert one(17, 32, 8, 8192, 2028, 32) and not one(17, 32, 8, 16128, 2028, 32) and not one(19, 32, 8, 60160, 2028, 32)
+    # many heads a group beside a long portion, whose own launch walks its keys once
+    assert not one(33, 32, 4, 2048, 2028, 32) and not one(100, 12, 2, 2048, 2028, 32) and one(40, 32, 4, 8192, 2028, 32) and one(66, 12, 2, 1536, 1100, 16)
