@@ -135,13 +135,14 @@ __global__ __launch_bounds__(WAVES * WAVE) void attention_f32_mfma_kernel(
           }
         top = fmaxf(top, __shfl_xor(top, 16, WAVE));
         top = fmaxf(top, __shfl_xor(top, 32, WAVE));
+        const float ref = top == -INFINITY ? 0.f : top;                    // all that is seen of the piece scores minus infinity: no weight
         float sum = 0.f;
 #pragma unroll
         for (int b = 0; b < 4; ++b)
 #pragma unroll
           for (int t = 0; t < 4; ++t) {
             const int key = piece * PIECE + b * 16 + 4 * g + t;
-            score[b][t] = key <= pos && key >= from ? expf(score[b][t] - top) : 0.f;
+            score[b][t] = key <= pos && key >= from ? expf(score[b][t] - ref) : 0.f;
             sum += score[b][t];
             if (t == 3) __builtin_amdgcn_sched_barrier(0);
           }

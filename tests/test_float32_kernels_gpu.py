@@ -115,3 +115,21 @@ def test_float32_attention_keeps_odd_values_to_those_who_see_them(ops):
     expected = plain.clone()
     expected[50:, 7], expected[71:, 9], expected[73:, 8] = float("inf"), float("nan"), float("-inf")
     assert torch.equal(got.nan_to_num(nan=12345.0), expected.nan_to_num(nan=12345.0))
+
+
+def test_float32_attention_gives_a_score_of_minus_infinity_no_weight(ops):
+    """Keys whose scores overflow to minus infinity, alone in their piece of 64 and among others: as if they were not there."""
+    g = torch.Generator().manual_seed(4)
+    n, d = 200, 64
+    q, k, v = (torch.randn(n, d, generator=g) for _ in range(3))
+    q[:, 0], k[:, 0] = 1e20, 0.0
+    k[5, 0] = k[64:130, 0] = k[199, 0] = -1e20
+    pages, table, of, at = -(-n // 16), torch.arange(-(-n // 16), dtype=torch.int32)[None], torch.zeros(n, dtype=torch.int32), torch.arange(n, dtype=torch.int32)
+    k_pages, v_pages = torch.zeros(pages * 16, d), torch.zeros(pages * 16, d)
+    k_pages[:n], v_pages[:n] = k, v
+    out = torch.empty(n, d, device="cuda")
+    ops.attention(out, dev(q), dev(k_pages.view(pages, 1, 16, d)), dev(v_pages.view(pages, 1, 16, d).transpose(2, 3).contiguous()), dev(table), dev(of), dev(at), 1, 0.125, together=16)
+    scores = (q[:, 1:].double() @ k[:, 1:].double().T) * 0.125
+    scores[:, k[:, 0] < 0] = -math.inf
+    scores[torch.ones(n, n, dtype=torch.bool).triu(1)] = -math.inf
+    torch.testing.assert_close(out.cpu().double(), torch.softmax(scores, -1) @ v.double(), rtol=2e-5, atol=2e-5)
