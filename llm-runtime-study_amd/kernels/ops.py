@@ -1050,6 +1050,11 @@ def attention(out: torch.Tensor, q: torch.Tensor, k_pages: torch.Tensor, v_pages
         *_gates(gates, tokens, nq, q.dtype, "attention"), *_distance(distance, nq, "attention"), together, _stream())
 
 
+def attention_shares(dtype: torch.dtype, nq: int, nkv: int, d: int, dv: int, page_size: int, plain: bool) -> bool:
+    """Whether attention() lets tokens share a workgroup (`together`): float32, and `plain`: no kept positions, sinks, cap, gates or bias."""
+    return dtype == torch.float32 and plain and d == dv and d in (32, 64, 96, 128) and nq // nkv <= 16 and page_size % 16 == 0
+
+
 def qkv_norm_prep(qkv: torch.Tensor, nq: int, nkv: int, d: int, dv: int, q_weight, k_weight, eps: float, cos, sin,
                   k_pages: torch.Tensor, v_pages: torch.Tensor, slots: torch.Tensor, page_size: int, bias: torch.Tensor | None = None,
                   temperature: tuple | None = None, positions: torch.Tensor | None = None, first_values: torch.Tensor | None = None,

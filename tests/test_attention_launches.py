@@ -1,0 +1,36 @@
+"""How many launches the attention of a mixed step takes where the kernels for any shape serve it: two only where the tokens of the
+portion can share workgroups."""
+
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from llm_runtime_study_amd.kernels import ops
+from llm_runtime_study_amd.parts.attention import GQAAttention
+
+
+@pytest.mark.parametrize("form,launches", [("plain", 2), ("bfloat16", 1), ("heads of 160", 1), ("gates", 1), ("kept", 1), ("sinks", 1), ("capped", 1), ("distance", 1), ("narrow values", 1),
+                                           ("all decode", 1), ("no singles", 1)])
+def test_launches(monkeypatch, form, launches):
+    calls = []
+    monkeypatch.setattr(ops, "attention", lambda out, q, k, v, table, of, at, *a, together=1, **more: calls.append((out.shape[0], of.tolist()[:out.shape[0]], together, more)))
+    part = GQAAttention.__new__(GQAAttention)
+    torch.nn.Module.__init__(part) if isinstance(part, torch.nn.Module) else None
+    d = 160 if form == "heads of 160" else 64
+    part.num_heads, part.head_dim, part.value_dim, part.scale, part.reach, part.keep_first = 4, d, 32 if form == "narrow values" else d, 0.125, 0, 4 if form == "kept" else 0
+    dtype = torch.bfloat16 if form == "bfloat16" else torch.float32
+    of = torch.tensor([3, 1, 2, 0, 0, 0, 0], dtype=torch.int32)
+    ctx = SimpleNamespace(all_decode=form == "all decode", single_rows=0 if form == "no singles" else 3, dtype=dtype, memo={}, token_slot=of, positions=of + 9)
+    cache = SimpleNamespace(k_pages=torch.zeros(1, 2, 16, d), v_pages=torch.zeros(1, 2, part.value_dim, 16))
+    more = {"sinks": None, "softcap": 0.0, "distance": None}
+    if form in ("sinks", "distance"):
+        more[form] = torch.ones(4)
+    if form == "capped":
+        more["softcap"] = 30.0
+    gates = torch.zeros(7, 4) if form == "gates" else None
+    part._attend(ctx, torch.zeros(7, 4 * part.value_dim), torch.zeros(7, 8 * d), cache, SimpleNamespace(block_table=None, page_size=16), gates=gates, **more)
+    assert [c[0] for c in calls] == ([3, 4] if launches == 2 else [7])
+    assert sum((c[1] for c in calls), []) == of.tolist()
+    if launches == 2:
+        assert [c[2] for c in calls] == [1, 16]
