@@ -16,7 +16,7 @@
 
 int lrs_attention_f32(float* out, int out_stride, const float* q, int q_stride, const float* k_pages, const float* v_pages, const int* block_table,
                       int table_stride, const int* token_request, const int* positions, int tokens, int nq, int nkv, int d, int page_size,
-                      float scale, int window, int together, hipStream_t s);
+                      float scale, int window, int together, int longest, hipStream_t s);
 bool lrs_attention_f32_takes(const void* out, int out_stride, const void* q, int q_stride, const void* k_pages, const void* v_pages, int nq, int nkv,
                              int d, int dv, int page_size);
 
@@ -2067,8 +2067,8 @@ LRS_API int lrs_attention(void* out, int out_stride, const void* q, int q_stride
                           const int* token_request, const int* positions, int dtype, int tokens,
                           int nq, int nkv, int d, int dv, int page_size, float scale, int window, int keep_first,
                           const float* sinks, float softcap, const void* gates, int gate_stride, const float* distance, int distance_form,
-                          int together, void* stream) {
-  // value pages [P, nkv, dv, page]; out rows hold nq heads of dv values; together: attention_f32.hip
+                          int together, int longest, void* stream) {
+  // value pages [P, nkv, dv, page]; out rows hold nq heads of dv values; together, longest: attention_f32.hip
   LRS_REQUIRE(tokens > 0 && nq > 0 && nkv > 0 && d > 0 && dv > 0 && page_size > 0, "attention: bad sizes tokens=%d nq=%d nkv=%d d=%d dv=%d page=%d", tokens, nq, nkv, d, dv, page_size);
   LRS_REQUIRE(nq % nkv == 0, "attention: %d query heads do not divide into %d kv heads", nq, nkv);
   LRS_REQUIRE(d <= 512 && dv <= 512, "attention: head sizes %d and %d above the supported 512", d, dv);
@@ -2085,7 +2085,7 @@ LRS_API int lrs_attention(void* out, int out_stride, const void* q, int q_stride
   if (dtype == LRS_F32 && !sinks && softcap == 0.f && !gates && !distance && keep_first == 0 &&
       lrs_attention_f32_takes(out, out_stride, q, q_stride, k_pages, v_pages, nq, nkv, d, dv, page_size))
     return lrs_attention_f32((float*)out, out_stride, (const float*)q, q_stride, (const float*)k_pages, (const float*)v_pages, block_table, table_stride,
-                             token_request, positions, tokens, nq, nkv, d, page_size, scale, window, together, s);
+                             token_request, positions, tokens, nq, nkv, d, page_size, scale, window, together, longest, s);
   if (dtype == LRS_F32)
     attention_generic_kernel<float, THREADS><<<grid, THREADS, lds, s>>>(
         (float*)out, out_stride, (const float*)q, q_stride, (const float*)k_pages, (const float*)v_pages,

@@ -5,23 +5,25 @@
 // queries (tokens times the kv group's heads, the columns of its products): scores, their maximum, weights and weighted sum of
 // that piece alone, as if there were no other.  A query's result is its pieces' partial results merged one after the
 // other in the order of their positions, by the same operations however many queries
-// share a workgroup's eight waves, which take eight pieces at a time.
+// share a workgroup's waves (eight, or fewer over short contexts), which take a piece each at a time.
 //
-// A piece is 512 products of 32 cycles at 128 dims whatever columns are in use, 6.8 us for the two waves of a SIMD: that bounds a
+// A piece is 256 products of 32 cycles at 128 dims whatever columns are in use, 6.8 us for the two waves of a SIMD: that bounds a
 // prompt (2,048 tokens, 16 heads of 128: 305 us, 56 TFLOP/s; 3,174 us with a workgroup a (token, head) and plain FMAs) and,
 // with one trip to memory before it, a decode step (8 tokens at 509: 18 us, 35 before).  A block of 16 keys, and one of
 // values, is asked for while the one before is multiplied; the registers this takes leave one workgroup a compute unit.
 #include "common.h"
 
+LRS_API int lrs_compute_units();
+
 int lrs_attention_f32(float* out, int out_stride, const float* q, int q_stride, const float* k_pages, const float* v_pages, const int* block_table,
                       int table_stride, const int* token_request, const int* positions, int tokens, int nq, int nkv, int d, int page_size,
-                      float scale, int window, int together, hipStream_t s);
+                      float scale, int window, int together, int longest, hipStream_t s);
 bool lrs_attention_f32_takes(const void* out, int out_stride, const void* q, int q_stride, const void* k_pages, const void* v_pages, int nq, int nkv,
                              int d, int dv, int page_size);
 
 namespace {
 
-constexpr int PIECE = 64, COLUMNS = 16, WAVES = 8;
+constexpr int PIECE = 64, COLUMNS = 16;
 
 // What is left of a partial result when its reference point moves to `top`.
 __device__ __forceinline__ float moved(float from, float top) { return from == -INFINITY ? 0.f : expf(from - top); }
@@ -48,10 +50,11 @@ __device__ __forceinline__ void add_odd_values(floatx4 values, floatx4 weights, 
   __builtin_amdgcn_sched_barrier(0);
 }
 
+// SHORT: blocks of 16 keys that nobody sees are left out rather than multiplied with weights of zero.
 // One workgroup: `together` tokens (as many as fit 16 columns with the kv group's heads) of one kv head, taken request by
 // request should they not all belong to one.
-template <int D>
-__global__ __launch_bounds__(WAVES * WAVE) void attention_f32_mfma_kernel(
+template <int D, int WAVES, bool SHORT>
+__global__ __launch_bounds__(WAVES * WAVE, WAVES == 8 ? 1 : 2) void attention_f32_mfma_kernel(
     float* __restrict__ out, int out_stride, const float* __restrict__ q, int q_stride, const float* __restrict__ k_pages,
     const float* __restrict__ v_pages, const int* __restrict__ block_table, int table_stride, const int* __restrict__ token_request,
     const int* __restrict__ positions, int tokens, int heads, int nkv, int page_size, float scale, int window, int together) {
@@ -92,10 +95,12 @@ __global__ __launch_bounds__(WAVES * WAVE) void attention_f32_mfma_kernel(
         floatx4 score[4], ahead[2][TILES];                                 // ahead: 16 keys, or their values, asked for a block ahead
         int64_t page[4];                                                   // the (page, kv head) block of 16 keys, and the slot they begin at
         int slot[4];
+        bool seen[4];
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
           // a block that nobody sees (perhaps without a page) stands for the nearest that somebody does: its weights will be zero
           int key0 = piece * PIECE + b * 16;
+          seen[b] = !SHORT || (key0 <= highest && key0 + 15 >= lowest);
           key0 = key0 < (lowest & ~15) ? lowest & ~15 : key0 > (highest & ~15) ? highest & ~15 : key0;
           page[b] = (int64_t)table[key0 / page_size] * nkv + kv_head;
           slot[b] = key0 % page_size;
@@ -117,10 +122,11 @@ __global__ __launch_bounds__(WAVES * WAVE) void attention_f32_mfma_kernel(
           else load_values(0);
           __builtin_amdgcn_sched_barrier(0);
           score[b] = floatx4{0.f, 0.f, 0.f, 0.f};
+          if (seen[b])
 #pragma unroll
-          for (int j = 0; j < TILES; ++j)
+            for (int j = 0; j < TILES; ++j)
 #pragma unroll
-            for (int t = 0; t < 4; ++t) score[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(ahead[b & 1][j][t], qf[j][t], score[b], 0, 0, 0);
+              for (int t = 0; t < 4; ++t) score[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(ahead[b & 1][j][t], qf[j][t], score[b], 0, 0, 0);
           __builtin_amdgcn_sched_barrier(0);
         }
         // this lane: keys 16 b + 4 g + t of its column
@@ -155,20 +161,22 @@ __global__ __launch_bounds__(WAVES * WAVE) void attention_f32_mfma_kernel(
         for (int b = 0; b < 4; ++b) {
           if (b < 3) load_values(b + 1);
           __builtin_amdgcn_sched_barrier(0);
-          const floatx4(&vf)[TILES] = ahead[b & 1];
-          float finite = 0.f;
+          if (seen[b]) {
+            const floatx4(&vf)[TILES] = ahead[b & 1];
+            float finite = 0.f;
 #pragma unroll
-          for (int i = 0; i < TILES; ++i)
+            for (int i = 0; i < TILES; ++i)
 #pragma unroll
-            for (int t = 0; t < 4; ++t) finite = fmaf(vf[i][t], 0.f, finite);
-          if (__any(finite != 0.f)) {
+              for (int t = 0; t < 4; ++t) finite = fmaf(vf[i][t], 0.f, finite);
+            if (__any(finite != 0.f)) {
 #pragma unroll
-            for (int i = 0; i < TILES; ++i) add_odd_values(vf[i], score[b], acc[i]);
-          } else {
+              for (int i = 0; i < TILES; ++i) add_odd_values(vf[i], score[b], acc[i]);
+            } else {
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
+              for (int t = 0; t < 4; ++t)
 #pragma unroll
-              for (int i = 0; i < TILES; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][t], score[b][t], acc[i], 0, 0, 0);
+                for (int i = 0; i < TILES; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][t], score[b][t], acc[i], 0, 0, 0);
+            }
           }
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -203,13 +211,13 @@ __global__ __launch_bounds__(WAVES * WAVE) void attention_f32_mfma_kernel(
   }
 }
 
-template <int D>
+template <int D, int WAVES, bool SHORT>
 void launch(float* out, int out_stride, const float* q, int q_stride, const float* k_pages, const float* v_pages, const int* block_table, int table_stride,
             const int* token_request, const int* positions, int tokens, int heads, int nkv, int page_size, float scale, int window, int together,
             hipStream_t s) {
   const dim3 grid((tokens + together - 1) / together, nkv);
   const int columns = together * heads;
-  attention_f32_mfma_kernel<D><<<grid, WAVES * WAVE, sizeof(float) * WAVES * (columns * (D + 4) + COLUMNS * 2), s>>>(
+  attention_f32_mfma_kernel<D, WAVES, SHORT><<<grid, WAVES * WAVE, sizeof(float) * WAVES * (columns * (D + 4) + COLUMNS * 2), s>>>(
       out, out_stride, q, q_stride, k_pages, v_pages, block_table, table_stride, token_request, positions, tokens, heads, nkv, page_size, scale, window, together);
 }
 
@@ -222,17 +230,35 @@ bool lrs_attention_f32_takes(const void* out, int out_stride, const void* q, int
 }
 
 // together: the most consecutive tokens that may share a workgroup (1: a step in which every request brings one token).
+// longest: no token's position + 1 is beyond it (0: not known).  Speed alone depends on either.
 int lrs_attention_f32(float* out, int out_stride, const float* q, int q_stride, const float* k_pages, const float* v_pages, const int* block_table,
                       int table_stride, const int* token_request, const int* positions, int tokens, int nq, int nkv, int d, int page_size,
-                      float scale, int window, int together, hipStream_t s) {
+                      float scale, int window, int together, int longest, hipStream_t s) {
   const int heads = nq / nkv, fit = COLUMNS / heads;
   if (together > fit) together = fit;
   if (together < 1) together = 1;
-#define SIZE(D) launch<D>(out, out_stride, q, q_stride, k_pages, v_pages, block_table, table_stride, token_request, positions, tokens, heads, nkv, page_size, scale, window, together, s)
+  // Short contexts: blocks of keys that nobody sees are left out (SHORT; a branch a block, 0.7 us a launch where none are), up to 32
+  // tokens, and more workgroups than units over a few pieces each have two waves, four times as many one: most of eight would wait
+  // with nothing to do.  us of 64 tokens at 30 and at 100, eight waves before / now (the kernel for any shape): 32 heads of 128 on 32 58 / 17
+  // (15) and 63 / 37 (36), 32 on 8 16 / 8 (12) and 18 / 16 (29), 16 heads of 64 on 16 21 / 7 (8) and 23 / 12 (17); one token at 10, 32 on 8 8.4 / 6.5 (5.3).
+  const int64_t workgroups = (int64_t)((tokens + together - 1) / together) * nkv;
+  const bool few_pieces = longest > 0 && longest <= 4 * PIECE;
+  const int items = together * heads * (d / 4);                            // what the merge has to do, one a thread
+#define CALL(D, WAVES, SHORT)                                                                                                                  \
+  launch<D, WAVES, SHORT>(out, out_stride, q, q_stride, k_pages, v_pages, block_table, table_stride, token_request, positions, tokens, heads, nkv, \
+                          page_size, scale, window, together, s)
+#define SIZE(D)                                                  \
+  do {                                                           \
+    if (few_pieces && workgroups > 4 * lrs_compute_units() && items <= WAVE) CALL(D, 1, true);     \
+    else if (few_pieces && workgroups > lrs_compute_units() && items <= 2 * WAVE) CALL(D, 2, true); \
+    else if (longest > 0 && longest <= 32) CALL(D, 8, true);     \
+    else CALL(D, 8, false);                                      \
+  } while (0)
   if (d == 32) SIZE(32);
   else if (d == 64) SIZE(64);
   else if (d == 96) SIZE(96);
   else SIZE(128);
 #undef SIZE
+#undef CALL
   return lrs_check_launch("attention");
 }

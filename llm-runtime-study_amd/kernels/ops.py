@@ -127,7 +127,7 @@ _SIGNATURES = {
                                             c_void_p, c_int64, c_void_p]),
     "lrs_norm_begin_parts": (c_int, [c_int]),
     "lrs_attention": (c_int, [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
-                              c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_float, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p]),
+                              c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_float, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_void_p]),
     "lrs_qkv_norm_prep": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p,
                                   c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_float, c_int, c_void_p, c_void_p, c_void_p]),
     "lrs_gated_norm_add": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_float, c_int, c_int, c_void_p, c_float,
@@ -1022,7 +1022,7 @@ def _distance(distance: torch.Tensor | None, nq: int, who: str):
 def attention(out: torch.Tensor, q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, block_table: torch.Tensor,
               token_request: torch.Tensor, positions: torch.Tensor, nq: int, scale: float, window: int = 0, keep_first: int = 0,
               sinks: torch.Tensor | None = None, softcap: float = 0.0, gates: torch.Tensor | None = None,
-              distance: torch.Tensor | None = None, together: int = 1) -> None:
+              distance: torch.Tensor | None = None, together: int = 1, longest: int = 0) -> None:
     """out [T, nq*dv]; q [T, >= nq*d] (leading nq*d columns of each row); key pages [P, nkv, page, d],
     value pages [P, nkv, dv, page].  window: a token at p sees keys above p - window; keep_first: and those below keep_first.
     sinks (float32 [nq]): the softmax's denominator of head h has one more term exp(sinks[h]), without key or value.
@@ -1032,7 +1032,7 @@ def attention(out: torch.Tensor, q: torch.Tensor, k_pages: torch.Tensor, v_pages
     [nq]: it loses distance[h] * x.  A negative window stands for chunks of -window positions counted from position 0: a token sees
     those of its own chunk (here and in every function that takes a window).
     together: the most consecutive tokens that may share a workgroup; speed alone depends on it (1 suits a step in which every
-    request brings one token, 16 a prompt)."""
+    request brings one token, 16 a prompt).  longest: the longest context (position + 1) among the tokens, if known; likewise."""
     tokens = out.shape[0]
     _need(k_pages.dim() == 4 and v_pages.dim() == 4 and k_pages.is_contiguous() and v_pages.is_contiguous(), "attention: pages must be contiguous")
     _, nkv, page_size, d = k_pages.shape
@@ -1047,7 +1047,7 @@ def attention(out: torch.Tensor, q: torch.Tensor, k_pages: torch.Tensor, v_pages
         _dev(out, "out"), _rows(out, "out"), _dev(q, "q"), _rows(q, "q"), _dev(k_pages, "k_pages"), _dev(v_pages, "v_pages"),
         _dev(block_table, "block_table"), block_table.stride(0), _dev(token_request, "token_request"), _dev(positions, "positions"),
         dtype_code(q.dtype), tokens, nq, nkv, d, dv, page_size, scale, window, keep_first, _sinks(sinks, nq, "attention"), float(softcap),
-        *_gates(gates, tokens, nq, q.dtype, "attention"), *_distance(distance, nq, "attention"), together, _stream())
+        *_gates(gates, tokens, nq, q.dtype, "attention"), *_distance(distance, nq, "attention"), together, longest, _stream())
 
 
 def attention_shares(dtype: torch.dtype, nq: int, nkv: int, d: int, dv: int, page_size: int, plain: bool) -> bool:

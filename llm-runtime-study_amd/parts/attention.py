@@ -438,17 +438,19 @@ class GQAAttention(Part):
         """Attention by the kernels for any shape and dtype; where tokens can share a workgroup, the single tokens at the head of a
         mixed step (each of a request of its own) go in a launch of their own, so that a prompt's tokens behind them do."""
         singles = 0 if ctx.all_decode else ctx.single_rows
+        longest = ctx.max_k if length_class(ctx.max_k) == 0 else 0        # of short contexts, a class that a shape's steps share
         plain = gates is None and not self.keep_first and not more.get("softcap") and more.get("sinks") is None and more.get("distance") is None
         if not singles or not ops.attention_shares(ctx.dtype, self.num_heads, cache.k_pages.shape[1], self.head_dim, self.value_dim, group.page_size, plain):
             ops.attention(out, qkv, cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot, ctx.positions, self.num_heads, self.scale,
-                          self.reach, self.keep_first, gates=gates, together=1 if ctx.all_decode else 16, **more)
+                          self.reach, self.keep_first, gates=gates, together=1 if ctx.all_decode else 16, longest=longest, **more)
             return
         rest = ctx.memo.get("rows_after_singles")
         if rest is None:
             rest = ctx.memo["rows_after_singles"] = (ctx.token_slot[singles:], ctx.positions[singles:])
         ops.attention(out[:singles], qkv[:singles], cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot, ctx.positions, self.num_heads,
-                      self.scale, self.reach, together=1)
-        ops.attention(out[singles:], qkv[singles:], cache.k_pages, cache.v_pages, group.block_table, *rest, self.num_heads, self.scale, self.reach, together=16)
+                      self.scale, self.reach, together=1, longest=longest)
+        ops.attention(out[singles:], qkv[singles:], cache.k_pages, cache.v_pages, group.block_table, *rest, self.num_heads, self.scale, self.reach, together=16,
+                      longest=longest)
 
     def _forward_whole_rows(self, ctx, x, residual, cache, group, cos, sin, then_norm, accumulate):
         """The forms whose heads `qkv_norm_prep` prepares: one product for q, k, v (and the gate), the norms over the whole

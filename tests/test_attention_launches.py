@@ -21,7 +21,7 @@ def test_launches(monkeypatch, form, launches):
     part.num_heads, part.head_dim, part.value_dim, part.scale, part.reach, part.keep_first = 4, d, 32 if form == "narrow values" else d, 0.125, 0, 4 if form == "kept" else 0
     dtype = torch.bfloat16 if form == "bfloat16" else torch.float32
     of = torch.tensor([3, 1, 2, 0, 0, 0, 0], dtype=torch.int32)
-    ctx = SimpleNamespace(all_decode=form == "all decode", single_rows=0 if form == "no singles" else 3, dtype=dtype, memo={}, token_slot=of, positions=of + 9)
+    ctx = SimpleNamespace(all_decode=form == "all decode", single_rows=0 if form == "no singles" else 3, dtype=dtype, memo={}, max_k=20, token_slot=of, positions=of + 9)
     cache = SimpleNamespace(k_pages=torch.zeros(1, 2, 16, d), v_pages=torch.zeros(1, 2, part.value_dim, 16))
     more = {"sinks": None, "softcap": 0.0, "distance": None}
     if form in ("sinks", "distance"):

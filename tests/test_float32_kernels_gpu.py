@@ -133,3 +133,22 @@ def test_float32_attention_gives_a_score_of_minus_infinity_no_weight(ops):
     scores[:, k[:, 0] < 0] = -math.inf
     scores[torch.ones(n, n, dtype=torch.bool).triu(1)] = -math.inf
     torch.testing.assert_close(out.cpu().double(), torch.softmax(scores, -1) @ v.double(), rtol=2e-5, atol=2e-5)
+
+
+@pytest.mark.parametrize("nq,nkv,d,batch", [(32, 32, 128, 40), (8, 8, 128, 70), (32, 8, 64, 70), (6, 2, 96, 200), (16, 16, 32, 80), (4, 4, 64, 300), (16, 1, 128, 300)])
+@pytest.mark.parametrize("window", [0, 20])
+def test_float32_attention_over_short_contexts(ops, nq, nkv, d, batch, window):
+    """Steps that workgroups of one and two waves take, and those that leave blocks out: the bits of eight waves, whatever is told."""
+    g = torch.Generator().manual_seed(nq + d + batch)
+    page, per = 16, 16
+    lengths = [(i * 37) % 256 + 1 for i in range(batch)]
+    pages = torch.randn(batch * per, nkv, page, d, generator=g).cuda(), torch.randn(batch * per, nkv, d, page, generator=g).cuda()
+    table = torch.arange(batch * per, dtype=torch.int32).view(batch, per).cuda()
+    q = torch.randn(batch, nq * d, generator=g).cuda()
+    of = torch.arange(batch, dtype=torch.int32)
+    for most in (256, 32):
+        at = torch.tensor([min(n, most) - 1 for n in lengths], dtype=torch.int32).cuda()
+        outs = [torch.empty(batch, nq * d, device="cuda") for _ in range(4)]
+        for out, (longest, together) in zip(outs, ((0, 1), (most, 1), (most, 16), (most, 3))):
+            ops.attention(out, q, *pages, table, of.cuda(), at, nq, 1 / math.sqrt(d), window, together=together, longest=longest)
+        assert all(torch.equal(out, outs[0]) for out in outs[1:])
