@@ -1798,8 +1798,9 @@ LRS_API int lrs_gemm(void* out, int mode, const void* a, const void* w, const vo
     LRS_REQUIRE(!normed || eps > 0.f, "gemm: eps must be positive");
   }
   LRS_REQUIRE(normed || rows == nullptr, "gemm: a row gather needs the fused norm input");
-  if (dtype == LRS_F32 && k % 32 == 0 && lda % 4 == 0 && ((uintptr_t)a % 16) == 0 && ((uintptr_t)w % 16) == 0) {
-    // on the matrix cores, with the bits of the tiled kernel below (gemm_f32.hip)
+  if (dtype == LRS_F32 && k % 32 == 0 && lda % 4 == 0 && ((uintptr_t)a % 16) == 0 && ((uintptr_t)w % 16) == 0 &&
+      (int64_t)128 * (lda > k ? lda : k) < (1ll << 30)) {
+    // on the matrix cores, with the bits of the tiled kernel below (gemm_f32.hip, whose byte offsets inside a tile of up to 128 rows are 32 bits)
     lrs_gemm_f32((float*)out, mode == OUT_ADD_F32, (const float*)a, (const float*)w, (const float*)bias, m, n, k, lda, ldc, s);
   } else if (dtype == LRS_F32) {
     dim3 grid((n + 63) / 64, (m + 63) / 64);

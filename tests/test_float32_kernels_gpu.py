@@ -152,3 +152,16 @@ def test_float32_attention_over_short_contexts(ops, nq, nkv, d, batch, window):
         for out, (longest, together) in zip(outs, ((0, 1), (most, 1), (most, 16), (most, 3))):
             ops.attention(out, q, *pages, table, of.cuda(), at, nq, 1 / math.sqrt(d), window, together=together, longest=longest)
         assert all(torch.equal(out, outs[0]) for out in outs[1:])
+
+
+def test_float32_product_of_rows_far_apart(ops):
+    """Rows whose distance, times the rows of a tile, does not fit 32 bits of bytes."""
+    m, n, k, stride = 16, 40, 64, 72_000_000
+    g = torch.Generator().manual_seed(9)
+    a, w = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g)
+    wide = torch.empty(m, stride, device="cuda")
+    wide[:, :k] = a.cuda()
+    far, near = torch.empty(m, n, device="cuda"), torch.empty(m, n, device="cuda")
+    ops.gemm(far, wide[:, :k], w.cuda())
+    ops.gemm(near, a.cuda(), w.cuda())
+    assert torch.equal(far, near)
