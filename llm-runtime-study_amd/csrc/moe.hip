@@ -539,18 +539,27 @@ __global__ __launch_bounds__(256) void moe_experts_bf16_wide_kernel(TO* __restri
   }
 }
 
-// How many tiles of the list are in use: they come first (the others hold -1).  A wave looks at 64 places a turn.
-__device__ __forceinline__ int tiles_in_use(const int* __restrict__ tile_expert, int tiles, int lane) {
-  int first = 0, count = tiles;                             // the end lies in [first, first + count]
-  while (count > 0) {
-    const int apart = (count + WAVE - 1) / WAVE, at = lane * apart;
-    const int before = __popcll(__ballot(at < count && tile_expert[first + (at < count ? at : 0)] >= 0));
-    if (before == 0) break;
-    const int skipped = (before - 1) * apart + 1;            // the last place seen in use is the last of these
-    count = count - skipped < apart - 1 ? count - skipped : apart - 1;
-    first += skipped;
+// The tiles of the list that are in use (the others hold -1): how many, and the place of the nth.  moe_align lists them first; lists with
+// gaps are looked through once more.  A wave looks at 64 places a turn.
+__device__ __forceinline__ int tiles_in_use(const int* __restrict__ tile_expert, int tiles, int lane, bool& gaps) {
+  int used = 0, end = 0;
+  for (int at = 0; at < tiles; at += WAVE) {
+    const unsigned long long mask = __ballot(at + lane < tiles && tile_expert[at + lane < tiles ? at + lane : 0] >= 0);
+    used += __popcll(mask);
+    if (mask) end = at + WAVE - __clzll(mask);
   }
-  return first;
+  gaps = end != used;
+  return used;
+}
+__device__ __forceinline__ int nth_in_use(const int* __restrict__ tile_expert, int tiles, int lane, int n) {
+  for (int at = 0; at < tiles; at += WAVE) {
+    const bool here = at + lane < tiles && tile_expert[at + lane < tiles ? at + lane : 0] >= 0;
+    const unsigned long long mask = __ballot(here);
+    const int before = __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0));
+    if (n < __popcll(mask)) return at + __ffsll(__ballot(here && before == n)) - 1;
+    n -= __popcll(mask);
+  }
+  return 0;
 }
 
 // The grouped product for large steps the way this package's many-rows product is made (gemm_bf16_wide in gemm.hip):
@@ -579,13 +588,14 @@ __global__ __launch_bounds__(256, 2) void moe_experts_bf16_fetch_kernel(TO* __re
   // unit, and how fast the L2s hand out the slices).  Two tiles of an expert in one workgroup of eight waves (256 x 256,
   // two stages of 64 KB) read a third less and took 1.3 times as long: with one workgroup on a compute unit nothing
   // runs while a slice arrives.
-  const int used = tiles_in_use(tile_expert, tiles_m, lane), in_use = used * tiles_n;
+  bool gaps;
+  const int used = tiles_in_use(tile_expert, tiles_m, lane, gaps), in_use = used * tiles_n;
   if ((int)blockIdx.x >= in_use) return;
   const int die = blockIdx.x % 8, left = in_use % 8;
   const int id = die * (in_use / 8) + (die < left ? die : left) + blockIdx.x / 8;
   const int band = id / (4 * tiles_n), within = id % (4 * tiles_n);
   const int band_rows = used - band * 4 < 4 ? used - band * 4 : 4;
-  const int tile_m = band * 4 + within % band_rows;
+  const int nth = band * 4 + within % band_rows, tile_m = gaps ? nth_in_use(tile_expert, tiles_m, lane, nth) : nth;
   const int expert = tile_expert[tile_m];
   const int m0 = tile_m * BM, n0 = (within / band_rows) * BN;
   const bf16* we = w + (int64_t)expert * n * k;

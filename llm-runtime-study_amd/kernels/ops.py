@@ -1750,7 +1750,7 @@ def moe_experts(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, sorted_pair
                 gather: bool, relu_squared: bool, silu_pairs: bool = False, clamped_pairs: tuple | None = None,
                 pair_weights: torch.Tensor | None = None) -> None:
     """out [tiles * tile rows, N] = rows of `a` times w[expert of the tile] [N, K], transposed, for every tile in use.
-    tile: rows of a tile, as moe_tile_rows() gave them for the step that was sorted; the tiles in use come first, as moe_align lists them.
+    tile: rows of a tile, as moe_tile_rows() gave them for the step that was sorted.
     gather: the row of a sorted pair is a[pair // top] (tokens); else `a` is in sorted order itself.
     silu_pairs: w holds a gate row 2j and an up row 2j + 1 for every feature j, and out [*, N / 2] = silu(gate) * up.
     clamped_pairs (alpha, limit): the same rows, out = g * sigmoid(alpha * g) * (u + 1) with g = min(p * gate, limit) and

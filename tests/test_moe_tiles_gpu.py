@@ -32,3 +32,31 @@ def test_every_tile_in_use_is_made_once(count, top, tokens, chosen):
         want = x[t].double() @ w[e].double().T
         size = x[t].double().abs() @ w[e].double().abs().T
         assert ((rows[t, c] - want).abs() <= k * 2.0 ** -23 * size).all()        # float32 sums of k exact products, whatever their order
+
+
+@pytest.mark.parametrize("count,top,tokens", [(6, 2, 145), (40, 4, 640), (70, 1, 3500)])
+def test_lists_with_tiles_not_in_use_between_those_in_use(count, top, tokens):
+    from llm_runtime_study_amd.kernels import ops
+
+    n, k, tile = 260, 64, 128
+    g = torch.Generator().manual_seed(count)
+    x, w = torch.randn(tokens, k, generator=g).to(torch.bfloat16).cuda(), torch.randn(count, n, k, generator=g).to(torch.bfloat16).cuda()
+    ids = torch.stack([torch.randperm(count, generator=g)[:top] for _ in range(tokens)]).to(torch.int32).cuda()
+    tiles = ops.moe_max_tiles(tokens * top, count)
+    assert ops.moe_tile_rows(tokens * top, count) == tile
+    sorted_pairs, place = torch.empty(tiles * tile, dtype=torch.int32, device="cuda"), torch.empty(tokens * top, dtype=torch.int32, device="cuda")
+    tile_expert = torch.empty(tiles, dtype=torch.int32, device="cuda")
+    ops.moe_align(ids, count, sorted_pairs, place, tile_expert)
+    # every tile two or three places further on than the one before it
+    to = torch.cumsum(torch.randint(1, 4, (tiles,), generator=g), 0)
+    spread = int(to[-1]) + 2
+    wide_expert, wide_pairs = torch.full((spread,), -1, dtype=torch.int32), torch.full((spread, tile), -1, dtype=torch.int32)
+    wide_expert[to], wide_pairs[to] = tile_expert.cpu(), sorted_pairs.view(tiles, tile).cpu()
+    want, got = torch.full((tiles * tile, n), -7.0, device="cuda"), torch.full((spread * tile, n), -7.0, device="cuda")
+    ops.moe_experts(want, x, w, sorted_pairs, tile_expert, tile, top, gather=True, relu_squared=False)
+    ops.moe_experts(got, x, w, wide_pairs.flatten().cuda(), wide_expert.cuda(), tile, top, gather=True, relu_squared=False)
+    got = got.view(spread, tile, n)
+    assert torch.equal(got[to.cuda()].view(tiles * tile, n), want)
+    between = torch.ones(spread, dtype=torch.bool)
+    between[to] = False
+    assert (got[between.cuda()] == -7.0).all()
