@@ -161,6 +161,15 @@ int tile_cost(int m, int n, int bn, int bm, int per_output) {
 
 }  // namespace
 
+// The tile of a product of more than 16 rows, weight rows times 1,024 plus input rows: the one whose busiest compute unit has least to
+// do, small tiles marked up by what they measured.
+LRS_API int lrs_gemm_f32_tile(int m, int n) {
+  const int small = tile_cost(m, n, 16, 32, 18), middle = tile_cost(m, n, 64, 32, 13), large = tile_cost(m, n, 64, 64, 11), largest = tile_cost(m, n, 128, 128, 10);
+  if (small <= middle && small <= large && small <= largest) return 16 * 1024 + 32;
+  if (middle <= large && middle <= largest) return 64 * 1024 + 32;
+  return large <= largest ? 64 * 1024 + 64 : 128 * 1024 + 128;
+}
+
 // K % 32 == 0; a, w and rows of lda floats 16-byte aligned.
 int lrs_gemm_f32(float* out, bool add, const float* a, const float* w, const float* bias, int m, int n, int k, int lda, int ldc, hipStream_t s) {
   const int wide_stores = ldc % 4 == 0 && (uintptr_t)out % 16 == 0;
@@ -181,12 +190,12 @@ int lrs_gemm_f32(float* out, bool add, const float* a, const float* w, const flo
     else if (half) TILES(64, 1, 1, 1, 1, 15, 8, 8);
     else TILES(64, 1, 1, 1, 1, 10, 8, 16);
   } else {
-    // Many rows: the tile whose busiest compute unit has least to do, small tiles marked up by what they measured
-    const int small = tile_cost(m, n, 16, 32, 18), middle = tile_cost(m, n, 64, 32, 13), large = tile_cost(m, n, 64, 64, 11), largest = tile_cost(m, n, 128, 128, 10);
-    if (small <= middle && small <= large && small <= largest) TILES(32, 1, 2, 1, 1, 12, 16, 16);
-    else if (middle <= large && middle <= largest) TILES(32, 2, 2, 2, 1, 8, 16, 16);
-    else if (large <= largest) TILES(32, 2, 2, 2, 2, 3, 16, 16);
-    else TILES(32, 2, 4, 4, 2, 3, 16, 16);
+    switch (lrs_gemm_f32_tile(m, n)) {
+      case 16 * 1024 + 32: TILES(32, 1, 2, 1, 1, 12, 16, 16); break;
+      case 64 * 1024 + 32: TILES(32, 2, 2, 2, 1, 8, 16, 16); break;
+      case 64 * 1024 + 64: TILES(32, 2, 2, 2, 2, 3, 16, 16); break;
+      default: TILES(32, 2, 4, 4, 2, 3, 16, 16);
+    }
   }
 #undef TILES
   return 0;

@@ -99,6 +99,7 @@ _SIGNATURES = {
     "lrs_gemm": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
                          c_int, c_float, c_int, c_int, c_void_p, c_int64, c_void_p]),
     "lrs_gemm_workspace_bytes": (c_int64, []),
+    "lrs_gemm_f32_tile": (c_int, [c_int, c_int]),
     "lrs_gemm_lines_add_rmsnorm": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_float, c_void_p, c_int,
                                            c_void_p, c_int64, c_void_p]),
     "lrs_gemm_norm_chain": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
@@ -575,6 +576,12 @@ def qk_prep(qkv: torch.Tensor, nq: int, nkv: int, d: int, q_weight, k_weight, ep
 
 
 @functools.lru_cache(maxsize=1)
+def gemm_f32_tile(m: int, n: int) -> tuple[int, int]:
+    """The tile (weight rows, input rows) of a float32 product of m > 16 rows with n weight rows."""
+    tile = library().lrs_gemm_f32_tile(m, n)
+    return tile // 1024, tile % 1024
+
+
 def gemm_workspace_bytes() -> int:
     """Bytes of device memory a caller brings as `workspace` to the products that divide K between workgroups."""
     return int(library().lrs_gemm_workspace_bytes())

@@ -23,8 +23,8 @@ def dev(t):
     return t.cuda()
 
 
-# every tile of the dispatch: few rows with few and many weight rows, K a multiple of 64 or of 32 only, 16 x 32 to 128 x 128 outputs,
-# ragged in both directions; K shorter than the slices that are on their way at once
+# few rows with few and many weight rows, K a multiple of 64 or of 32 only, tiles of 16 x 32 to 64 x 64 outputs (each of them and 128 x 128
+# below), ragged in both directions; K shorter than the slices that are on their way at once
 @pytest.mark.parametrize("m", [1, 8, 9, 16, 17, 33, 100, 300, 1030])
 @pytest.mark.parametrize("n,k", [(5, 32), (200, 64), (1027, 96), (2050, 320), (4096, 1024), (16401, 96), (16416, 128)])
 def test_float32_product(ops, m, n, k):
@@ -165,3 +165,27 @@ def test_float32_product_of_rows_far_apart(ops):
     ops.gemm(far, wide[:, :k], w.cuda())
     ops.gemm(near, a.cuda(), w.cuda())
     assert torch.equal(far, near)
+
+
+@pytest.mark.parametrize("m,n,tile", [(33, 1027, (16, 32)), (2047, 5, (16, 32)), (100, 2050, (64, 32)), (509, 4099, (64, 32)), (2047, 200, (64, 32)), (100, 4099, (64, 64)),
+                                      (1500, 1027, (64, 64)), (100, 24577, (128, 128)), (509, 6145, (128, 128)), (1500, 2050, (128, 128)), (2049, 16416, (128, 128))])
+@pytest.mark.parametrize("k", [32, 64, 96, 416])
+def test_float32_product_of_every_tile(ops, m, n, tile, k):
+    """Remainders in both directions, K shorter than, as long as and longer than the slices on their way, strided stores and sums: against
+    float64, and bit for bit against the kernel for any shape."""
+    assert ops.gemm_f32_tile(m, n) == tile
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, w, bias = (torch.randn(*shape, generator=g, device="cuda") for shape in ((m, k), (n, k), (n,)))
+    # k roundings of the sum of the products' sizes, one for the bias
+    want = a.double() @ w.double().T + bias.double()
+    bound = (k + 1) * 2.0 ** -24 * (a.abs().double() @ w.abs().double().T + bias.abs().double())
+    out, plain, strided = torch.empty(m, n, device="cuda"), torch.empty(m, n, device="cuda"), torch.full((m, n + 3), 0.25, device="cuda")
+    ops.gemm(out, a, w, bias)
+    assert ((out.double() - want).abs() <= bound).all()
+    wide = torch.zeros(m, k + 1, device="cuda")
+    wide[:, :k] = a
+    ops.gemm(plain, wide[:, :k], w, bias)
+    assert torch.equal(out, plain)
+    ops.gemm(strided[:, :n], a, w, accumulate=True)
+    ops.gemm(plain, wide[:, :k], w)
+    assert torch.equal(strided[:, :n], plain + 0.25) and (strided[:, n:] == 0.25).all()
