@@ -492,12 +492,13 @@ __device__ __forceinline__ float add_rows(float a, float b) {
 // The same for latent rows of 128, 256 or 512 values with 64 rotated dims behind them (CT tiles of 16 latent columns), whose tiles go from
 // memory straight into LDS: a workgroup's four waves (16 rows each) share them, and three tiles of 32 keys are on their way while one
 // is worked on.  The kernel above waits for memory four times a tile, 9 us in all; 16 tokens of 32 heads at 3,072
-// positions took 70 us in 16 parts and 81 in 32 with their merge, 34 and 47 here (a prompt of 2,048 tokens 1,534 and 451).  A tile is read
+// positions took 66 us in 16 parts and 77 in 32 with their merge, 30 and 43 here (a prompt of 2,048 tokens 1,418 and 355).  A tile is read
 // once for both products: as rows for the scores (keys x queries: a lane ends with eight keys' scores of one query, which are the second
 // product's operand as they stand), and through the transposing LDS read for the values (columns x queries: a lane's sums are of the same
 // query), so the copy by columns is not read at all.  Piece c (16 bytes) of key row k lies at place c ^ turn(k): the eight rows that are read
 // together then meet every bank once, for whole pieces and for the halves that the transposing read takes.  One wave a SIMD: its turn of
-// some 4,000 cycles, 1,088 of them products, bounds a prompt; a decode step the trips to memory before the first tile, 1.7 us a tile and the merge.
+// some 3,400 cycles, 1,088 of them products, bounds a prompt; a decode step the trips to memory before the first tile, 1.4 us a tile and the merge.
+// The sums' rescaling comes before the products: between them, where a product would hide it, it made them wait (455 us).
 // The results are the kernel above's bit for bit: a tile's keys meet the products in its order, maxima and sums move as there, and the keys are
 // divided as there.  With sums in another order and maxima that moved in steps of 2^8 a prompt took 317 us and the tokens 29 and 43, but
 // scores of experts behind such layers that were nearly equal came out in the other order now and then.

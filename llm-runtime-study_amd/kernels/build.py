@@ -28,6 +28,10 @@ ARCH = "gfx950"
 # -packed-fp32-ops: keep the compiler from forming packed float32 instructions.
 DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 FLAGS = [f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wno-unused-command-line-argument"] + DEVICE_FLAGS
+# Sources with flags of their own.  latent.hip: matrix products leave their sums in vector registers, not in accumulation registers, which a
+# running softmax that rescales some 128 of them at most tiles would read and write back one by one (a prompt of 2,048 tokens 355 us a layer
+# for 451, of the kernel of waves by themselves 1,418 for 1,530).
+FILE_FLAGS = {"latent.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 # the vendor's matrix library, for bfloat16 products of many rows (csrc/library_gemm.hip)
 ROCM_LIB = Path(os.environ.get("ROCM_PATH", "/opt/rocm")) / "lib"
 LINK_FLAGS = [f"-L{ROCM_LIB}", "-lhipblaslt", f"-Wl,-rpath,{ROCM_LIB}"]
@@ -47,6 +51,7 @@ def source_hash() -> str:
         digest.update(path.name.encode())
         digest.update(path.read_bytes())
     digest.update(" ".join(FLAGS + LINK_FLAGS).encode())
+    digest.update(repr(sorted(FILE_FLAGS.items())).encode())
     return digest.hexdigest()
 
 
@@ -77,7 +82,7 @@ def _say(message: str) -> None:
 def _compile_one(hipcc: str, src: Path, obj: Path) -> None:
     _say(f"compiling {src.name} ...")
     started = time.time()
-    proc = subprocess.run([hipcc, *FLAGS, "-c", str(src), "-o", str(obj)], capture_output=True, text=True)
+    proc = subprocess.run([hipcc, *FLAGS, *FILE_FLAGS.get(src.name, ()), "-c", str(src), "-o", str(obj)], capture_output=True, text=True)
     if proc.returncode != 0:
         raise BuildError(f"hipcc failed on {src.name}:\n{proc.stderr}")
     _say(f"compiled {src.name} in {time.time() - started:.1f} s")
