@@ -235,11 +235,16 @@ class GQAAttention(Part):
         before it, so eight waves finish a short context sooner than a merge would.  us with four waves / with eight, parts in
         brackets, merge counted, 32 heads on 8: batch 1 at 2,048 tokens 14.5 [8] / 13.2 [8], batch 8 24.5 [8] / 23.4 [4], batch 8 at 8,192
         58.2 [8] / 56.1 [4]; but batch 40 at 600 28.3 / 32.6 and batch 64 at 1,500 73.1 / 75.9.
-          * As many parts as one round of workgroups has room for: a second round that is partly empty costs more than the shorter
-            walks give (batch 24 at 1,500, 192 workgroups: 35.2 [1] / 32.8 [1], 40.8 [2]; 96 workgroups, 32 heads on 4: 24.1 [4] / 21.2 [2],
-            30.4 [3]; 24 workgroups at 8,000, 16 heads on 1: 30.2 [16] / 26.4 [8], 36.4 [11]).
-          * But three for 129 to 160 workgroups from 2,048 tokens on, nearly two full rounds (144 at 3,000: 52.8 [4] / 51.2 [3], 53.8 [1];
-            at 8,000 122 [4] / 111 [3], 128 [1]; at 1,500 32.9 [4] / 30.8 [1], 33.7 [3]).
+          * As many parts as one round of workgroups has room for: a second round that is partly empty costs more than the shorter walks
+            give (192 workgroups at 1,500: 34.9 [1] / 32.7 [1], 40.9 [2]; 96: 24.1 [4] / 20.8 [2], 29.8 [3], 27.3 [4]).
+          * Two rounds over contexts long enough for a request that is far longer than the others, which a step waits for, to count, where
+            one round is not full: from 4,096 tokens on, from 2,048 where one round has room for two parts and less, from 1,024 where it
+            has for one (while the four waves' rule divides).  96 workgroups at 3,000 40.3 [6] / 37.1 [5], 35.2 [2], at 8,000 88.7 [6] / 77.8 [5], 75.5 [2]; of 12
+            requests one at 32,000 and the others at 500 85 [6] / 86 [5], 190 [2]; 136 workgroups at 1,500 33.2 [4] / 32.9 [3], 28.2 [1].
+          * Two or three beyond that, the fuller, from 8,192 tokens on (192 workgroups: of 24 requests one at 32,000 430 [1] / 105 [4], 364 [1];
+            all at 8,000 146 [1] / 144 [4], 138 [1]).
+          * Four waves again from 4,096 tokens on where one round is full: a unit's stream is the limit, so one long context among short
+            ones wants units, not waves (64 workgroups, one request of 8 at 32,000 67 [8] / 102 [4]; all at 8,000 52.8 [8] / 51.6 [4]).
           * At least 256 keys each (batch 1 at 900: 14.1 [2] / 12.5 [2], 15.1 [1]; batch 16 at 520, 640, 768 and 900 15.5 / 14.4 [2] 13.4 [1],
             16.8 / 15.5 16.1, 18.2 / 17.3 18.6, 20.5 / 19.1 21.9), and under 1,024 tokens undivided for smaller heads, whose keys are
             fewer bytes (64 dims, batch 4 at 520 and 768 10.2 [2] / 8.4 [1] 8.9 [2] and 10.4 / 9.1 9.8)."""
@@ -247,12 +252,21 @@ class GQAAttention(Part):
         if workgroups > units or head_dim > 128:
             return cls._decode_splits(workgroups, longest, bound, page_size), 1
         reach = length_class(longest)
-        wanted = units // workgroups
-        if 2 * workgroups > units and 8 * workgroups <= 5 * units and reach >= 2048:
-            wanted = 3
+        most = min(reach // 256, 64)
+        wanted, twice, few = units // workgroups, 2 * units // workgroups, 8 * workgroups <= 5 * units
         if head_dim < 128 and reach < 1024:
             wanted = 1
-        return max(1, min(wanted, reach // 256, 64), -(-bound // (4096 * page_size))), 2
+        elif units % workgroups == 0:
+            if reach >= 4096 and 8 * workgroups >= units and 2 * workgroups <= units:
+                return cls._decode_splits(workgroups, longest, bound, page_size), 1
+        elif few:
+            # (160 workgroups, the last that the other rule divides, are as well off undivided under 2,048 tokens)
+            counts = reach >= 4096 or (reach >= 2048 and wanted < 3) or (reach >= 1024 and wanted < 2 and 8 * workgroups < 5 * units)
+            wanted = twice if counts and twice <= min(most, 32) else wanted
+        elif reach >= 8192:
+            thrice = 3 * units // workgroups
+            wanted = thrice if 2 * thrice > 3 * twice else twice
+        return max(1, min(wanted, most), -(-bound // (4096 * page_size))), 2
 
     @staticmethod
     def _walks_in_pairs(ctx, heads_per_group: int, head_dim: int) -> bool:

@@ -17,9 +17,16 @@ def test_parts_of_a_decode_step(monkeypatch, head_dim):
             if workgroups > 256 or head_dim > 128:
                 assert (splits, form) == (GQAAttention._decode_splits(workgroups, longest, longest, 16), 1)
                 continue
-            assert form == 2 and (splits <= max(1, longest // 256, fits))
-            # one round of workgroups, or two that are nearly full
-            assert splits == fits or splits * workgroups <= 256 or (splits == 3 and longest >= 2048 and 384 < 3 * workgroups <= 480)
+            if form == 1:      # one round is full and contexts are long: as for workgroups of four waves in every respect
+                assert longest >= 4096 and 256 % workgroups == 0 and splits == GQAAttention._decode_splits(workgroups, longest, longest, 16)
+                continue
+            assert splits <= max(1, longest // 256, fits)
+            # one round of workgroups; over longer contexts two or three, as full as they can be
+            rounds = -(-splits * workgroups // 256)
+            assert splits == fits or rounds == 1 or (longest >= 1024 and rounds == 2) or (longest >= 8192 and rounds == 3)
+            assert splits == fits or rounds == 1 or (splits + 1) * workgroups > 256 * rounds
+            # a context that is far longer than the others is not left to few workgroups
+            assert longest < 4096 or splits >= 0.45 * GQAAttention._decode_splits(workgroups, longest, longest, 16)
 
 
 def test_which_mixed_steps_go_in_one_launch(monkeypatch):
@@ -29,7 +36,7 @@ def test_which_mixed_steps_go_in_one_launch(monkeypatch):
         splits, _ = GQAAttention._decode_shape(singles * nkv, bound, bound, 16, 128)
         return GQAAttention._one_launch(singles * nkv, splits, -(-portion // size) * nkv, size, nq // nkv, bound)
 
-    assert one(24, 32, 8, 1536, 488, 16) and one(24, 40, 8, 1536, 488, 16) and one(24, 32, 8, 60160, 2028, 32)
+    assert one(24, 32, 8, 1536, 488, 16) and one(24, 40, 8, 1536, 488, 16) and one(24, 32, 8, 8192, 2028, 32) and not one(24, 32, 8, 60160, 2028, 32)
     assert not one(8, 32, 8, 1536, 488, 16)
     # a decoding request far on among short ones: its keys are divided in a launch of their own
     assert one(17, 32, 8, 8192, 2028, 32) and not one(17, 32, 8, 16128, 2028, 32) and not one(19, 32, 8, 60160, 2028, 32)
