@@ -1706,11 +1706,11 @@ __device__ __forceinline__ void attention_prefill_d128_part(
       if (first_tile + 1 <= last_tile) fetch_values(values_ahead, 1), pending += 2;
       values_ahead[0] = vbase[0], values_ahead[1] = vbase[1];
       pages_of(std::false_type{}, first_tile + 3, pages_ahead);
-      if (pending == 4) fetched_then_barrier<4>();
-      else if (pending == 2) fetched_then_barrier<2>();
-      else fetched_then_barrier<0>();
+      if (pending == 4) fetched_and_read_then_barrier<4>();
+      else if (pending == 2) fetched_and_read_then_barrier<2>();
+      else fetched_and_read_then_barrier<0>();
       if (!IDLE_WAVES || active) scores(first_tile, 0, sa);
-      asm volatile("s_barrier" ::: "memory");                  // everyone has read the first keys: their stage may be filled again
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // everyone has read the first keys: their stage may be filled again
     }
     int tile = first_tile, stage = 0;                          // stage = (tile - first_tile) % 3
     // the turn's fetches, and how many they are; EVERY: tile + 3 is not past the last, so all of them happen
@@ -1726,9 +1726,9 @@ __device__ __forceinline__ void attention_prefill_d128_part(
       return pending;
     };
     auto turn_over = [&](int pending) {
-      if (pending == 4) fetched_then_barrier<4>();
-      else if (pending == 2) fetched_then_barrier<2>();
-      else fetched_then_barrier<0>();
+      if (pending == 4) fetched_and_read_then_barrier<4>();
+      else if (pending == 2) fetched_and_read_then_barrier<2>();
+      else fetched_and_read_then_barrier<0>();
       stage = stage == STAGES - 1 ? 0 : stage + 1;
       ++tile;
     };

@@ -94,7 +94,7 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
 // Memory straight into LDS (global_load_lds_dwordx4): lane l of the wave fetches the 16 bytes at
 // base + lane_offset (base the same for the whole wave) and they land at LDS byte address lds_address +
 // 16 l; nothing passes through registers and the wave goes on at once.  The compiler does not know these
-// fetches: whoever reads the LDS they fill waits for them with fetched_then_barrier (they finish in the
+// fetches: whoever reads the LDS they fill waits for them with fetched_and_read_then_barrier (they finish in the
 // order they were asked for, and count in vmcnt).  LDS that only they write must still be named as an
 // address here, which is what tells the compiler that its contents change.
 __device__ __forceinline__ void fetch_to_lds(const void* base, unsigned lane_offset, unsigned lds_address) {
@@ -104,12 +104,9 @@ __device__ __forceinline__ void fetch_to_lds(const void* base, unsigned lane_off
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                :: "s"(__builtin_amdgcn_readfirstlane(lds_address)), "v"(lane_offset), "s"(uniform_base) : "memory");
 }
-// Waits until at most `PENDING` of this wave's fetches are still on their way, then for the workgroup.
-template <int PENDING>
-__device__ __forceinline__ void fetched_then_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(PENDING) : "memory");
-}
-// ... and until this wave has what it read from LDS as well: others may then fill what it read from.
+// Waits until at most `PENDING` of this wave's fetches are still on their way and this wave has what it read from LDS, then for the
+// workgroup.  The reads as well: behind the barrier others ask memory to fill what was read from, and a read that waits its turn in
+// a busy compute unit can take as long as a fetch that its L2 answers.
 template <int PENDING>
 __device__ __forceinline__ void fetched_and_read_then_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(PENDING) : "memory");

@@ -248,12 +248,12 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_wide_kernel(void* __restrict
   int m0_opaque = m0;
   fetch(0, 0);
   fetch(1, 1);
-  fetched_then_barrier<6>();
+  fetched_and_read_then_barrier<6>();
   int stage = 0;
   for (int kt = 0; kt < steps; ++kt) {
     fetch(kt + 2, stage == 0 ? 2 : stage - 1);
     multiply(stage);
-    fetched_then_barrier<6>();
+    fetched_and_read_then_barrier<6>();
     stage = stage == STAGES - 1 ? 0 : stage + 1;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");               // the fetches past K that nobody reads
@@ -389,12 +389,12 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_lines_kernel(void* __restric
   int m0_opaque = m0;
   fetch(0, 0);
   if (STAGES == 3) fetch(1, 1);
-  fetched_then_barrier<PENDING>();
+  fetched_and_read_then_barrier<PENDING>();
   int stage = 0;
   for (int kt = 0; kt < steps; ++kt) {
     fetch(kt + STAGES - 1, stage == 0 ? STAGES - 1 : stage - 1);
     multiply(stage);
-    fetched_then_barrier<PENDING>();
+    fetched_and_read_then_barrier<PENDING>();
     stage = stage == STAGES - 1 ? 0 : stage + 1;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");               // the fetches past K that nobody reads

@@ -648,12 +648,12 @@ __global__ __launch_bounds__(256, 2) void moe_experts_bf16_fetch_kernel(TO* __re
   int m0_opaque = m0;
   fetch(0, 0);
   fetch(1, 1);
-  fetched_then_barrier<6>();
+  fetched_and_read_then_barrier<6>();
   int stage = 0;
   for (int kt = 0; kt < steps; ++kt) {
     fetch(kt + 2, stage == 0 ? 2 : stage - 1);
     multiply(stage);
-    fetched_then_barrier<6>();
+    fetched_and_read_then_barrier<6>();
     stage = stage == STAGES - 1 ? 0 : stage + 1;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");               // the fetches past K that nobody reads
