@@ -1295,22 +1295,32 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void attention_prefill_bf16_
 // The wave that fetched a tile waits for its own fetches (vmcnt) before the barrier that opens the
 // tile to the others; the fetches of the tile after it stay in flight.  The fetches are written in
 // assembly because the compiler would wait for all of them before any LDS read it cannot tell apart.
+// What bounds a walk is the instructions a wave issues beside its products (one every four cycles at most): 32 products of a turn
+// of 32 queries come with 80 vector, 33 scalar and 18 LDS instructions, and the chip's clock is at 2.1 GHz meanwhile.  Turns of
+// 215 instructions that also waited for the fetches they had just made, for scalar loads of the block table and for every value
+// fragment in turn took 1.40 us with two workgroups a unit behind contexts in memory, these 1.11 (16 heads on 8, 2,048 tokens after
+// 14,336: 360 -> 284 us a layer; 32 on 8 691 -> 486; 32,768 tokens 8.95 -> 7.64 ms, 1.15 PFLOP/s; 2,048 after 2,048 152 -> 115).
 // SCORES: what happens to the scores before the softmax, by instances of their own so that the others keep their registers:
 // nothing, a cap (softcap * tanh(score / softcap) of the scaled scores), a bias by distance (in the form with a logarithm, or the
 // linear one, which without a cap is what the products are added to and costs nothing), or the cap and then the bias.
 enum { SCORES_PLAIN = 0, SCORES_CAPPED = 1, SCORES_DISTANCE = 2, SCORES_BOTH = 3, SCORES_LINEAR = 4, SCORES_CAPPED_LINEAR = 5 };
 // SPREAD: how a kv group's heads meet the waves: a wave a head (in several passes if there are more heads than waves); the same with
 // waves that have no head in some pass; and for two heads, which left half of the waves idle, a wave a (head, block of 16 queries) or,
-// where neighbouring groups are one request's, a wave a (head, group of 32).  A turn of the walk is bound by its tile's way from the
-// L2s (16 KB a turn and workgroup, 9 TB/s with two workgroups a unit), so a pair walking together does twice as much with it:
-// 16 heads on 8, 2,048 tokens after 14,336: 569 us with idle waves, 444 with halves, 322 in pairs with the keys divided by two;
-// 8,192 tokens 584 / 385 / 390; 2,048 after 2,048 142 / 136 / 100.
+// where neighbouring groups are one request's, a wave a (head, group of 32).  A turn of the walk costs its tile's way from the
+// L2s (16 KB a turn and workgroup) and its barrier whatever is done with them, so a pair walking together does twice as much with it
+// (before turns were made shorter: 16 heads on 8, 2,048 tokens after 14,336: 569 us with idle waves, 444 with halves, 322 in pairs with
+// the keys divided by two; 8,192 tokens 584 / 385 / 390; 2,048 after 2,048 142 / 136 / 100).
 enum { SPREAD_HEADS = 0, SPREAD_SOME_IDLE = 1, SPREAD_HALVES = 2, SPREAD_PAIRS = 3 };
 struct PrefillLds {
   static constexpr int D = 128, STAGES = 3, KBLOCK = 1024 + 32, KBYTES = 8 * KBLOCK, VHALF = 16 * D * 2 + 16;
   static constexpr int VSTAGE = (2 * VHALF + 63) / 64 * 64;
   __attribute__((aligned(64))) unsigned char key_tiles[STAGES * KBYTES];
   __attribute__((aligned(64))) unsigned char value_tiles[STAGES * VSTAGE];
+  // where runs of 16 keys lie in memory, and their values: rings of two blocks of 64 runs (the values' a tile further on, so that
+  // one place in both holds what a turn asks for: the keys of one tile and the values of the tile before it)
+  static constexpr int BLOCK_RUNS = 64, RUNS = 2 * BLOCK_RUNS;
+  __attribute__((aligned(16))) uint64_t key_runs[RUNS];
+  __attribute__((aligned(16))) uint64_t value_runs[RUNS];
 };
 template <int QB, bool MANY_WAVES, int SPREAD, int SCORES>
 __device__ __forceinline__ void attention_prefill_d128_part(
@@ -1375,55 +1385,53 @@ __device__ __forceinline__ void attention_prefill_d128_part(
   const unsigned value_offset = (unsigned)(((value_dim * page_size) + (lane & 1) * 8) * 2);
   const unsigned keys_address = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)key_tiles;
   const unsigned values_address = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)value_tiles;
-  // Where a run of 16 keys lies in memory.  Everything about it is the same for the whole workgroup, so the
-  // page comes from the block table by a scalar load and the rest is a handful of scalar instructions; a
-  // tile's two pages are asked for a turn before its addresses are wanted.  A run no query sees is masked:
-  // any page with numbers in it will do, so runs are clamped to those the queries do see.
-  const unsigned page_bytes = (unsigned)(nkv * page_size * D * 2);   // from page to page of keys ...
-  const unsigned value_page_bytes = (unsigned)(nkv * page_size * dv * 2);   // ... and of values
+  // Where a run of 16 keys lies in memory: a page from the block table and a place in it.  A run no query sees is masked: any page
+  // with numbers in it will do, so runs are clamped to those the queries do see.
+  const uint64_t page_bytes = (uint64_t)nkv * page_size * D * 2;            // from page to page of keys ...
+  const uint64_t value_page_bytes = (uint64_t)nkv * page_size * dv * 2;     // ... and of values
   const char* const k_head = (const char*)(k_pages + (int64_t)kvh * page_size * D);
   const char* const v_head = (const char*)(v_pages + (int64_t)kvh * page_size * dv);
-  // INSIDE: the tile lies behind the first of the walk, so that only the far end needs the clamp
-  auto run_in_reach = [&](auto inside, int tile, int half) {
-    const int run = tile * 2 + half;
-    if (decltype(inside)::value) return run > last_run ? last_run : run;
-    return run < first_run ? first_run : run > last_run ? last_run : run;
+  auto locate = [&](int run, uint64_t& keys, uint64_t& values) {
+    run = run < first_run ? first_run : run > last_run ? last_run : run;
+    const int entry = pages16 > 1 ? (int)__umulhi((unsigned)run, magic) : run;
+    const uint64_t page = (uint64_t)(unsigned)table[entry];
+    const unsigned in_page = (unsigned)(run - entry * pages16) * 16u;
+    keys = (uint64_t)(uintptr_t)k_head + page * page_bytes + in_page * (unsigned)(D * 2);
+    values = (uint64_t)(uintptr_t)v_head + page * value_page_bytes + in_page * 2u;
   };
-  auto pages_of = [&](auto inside, int tile, int (&pages)[2]) {
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const int run = run_in_reach(inside, tile, half);
-      pages[half] = table[pages16 > 1 ? (int)__umulhi((unsigned)run, magic) : run];
-    }
+  // A wave's lanes look up a block of 64 runs at a time and leave the addresses in LDS, from where every turn takes its four: the
+  // same work done by every wave in every turn with scalar instructions (loads of the block table among them, which LDS reads cannot
+  // be waited for apart from) was 60 of a turn's 215 instructions.
+  constexpr int BLOCK_RUNS = PrefillLds::BLOCK_RUNS, RUNS = PrefillLds::RUNS;
+  auto locate_block = [&](int which) {
+    uint64_t keys, values;
+    locate(first_tile * 2 + which * BLOCK_RUNS + lane, keys, values);
+    const int at = (which & 1) * BLOCK_RUNS + lane;
+    lds.key_runs[at] = keys;
+    lds.value_runs[(at + 2) & (RUNS - 1)] = values;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");             // there before this wave comes to the next barrier
   };
-  auto locate = [&](auto inside, int tile, const int (&pages)[2], const char* (&kbase)[2], const char* (&vbase)[2]) {
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const uint64_t at = (uint64_t)(unsigned)pages[half] * page_bytes, value_at = (uint64_t)(unsigned)pages[half] * value_page_bytes;
-      if (pages16 > 1) {
-        const int run = run_in_reach(inside, tile, half);
-        const unsigned off = (unsigned)(run - (int)__umulhi((unsigned)run, magic) * pages16) * 16u;
-        kbase[half] = k_head + at + off * (unsigned)(D * 2);
-        vbase[half] = v_head + value_at + off * 2u;
-      } else {
-        kbase[half] = k_head + at;
-        vbase[half] = v_head + value_at;
-      }
-    }
+  struct Pair {
+    uint64_t run[2];
+  };
+  auto runs_at = [&](const uint64_t (&ring)[RUNS], int place) {
+    typedef uint64_t pair __attribute__((ext_vector_type(2)));
+    const pair at = *(const pair*)&ring[place];
+    return Pair{{at[0], at[1]}};
   };
   // (a kv group of five to eight heads brings as many waves, so that one walk over the keys serves them all;
   // the first four waves bring the tiles in)
-  auto fetch_keys = [&](const char* const (&kbase)[2], int stage) {      // two fetches a wave
-    if (wave >= 4) return;
+  auto fetch_keys = [&](const Pair& from, int stage) {      // two fetches a wave
+    if (MANY_WAVES && wave >= 4) return;
 #pragma unroll
     for (int half = 0; half < 2; ++half)
-      fetch_to_lds(kbase[half], key_offset, keys_address + (unsigned)(stage * KBYTES + (wave + 4 * half) * KBLOCK));
+      fetch_lanes_to_lds(from.run[half] + key_offset, keys_address + (unsigned)(stage * KBYTES + (wave + 4 * half) * KBLOCK));
   };
-  auto fetch_values = [&](const char* const (&vbase)[2], int stage) {    // two fetches a wave
-    if (wave >= 4) return;
+  auto fetch_values = [&](const Pair& from, int stage) {    // two fetches a wave
+    if (MANY_WAVES && wave >= 4) return;
 #pragma unroll
     for (int half = 0; half < 2; ++half)
-      fetch_to_lds(vbase[half], value_offset, values_address + (unsigned)(stage * VSTAGE + half * VHALF + wave * 1024));
+      fetch_lanes_to_lds(from.run[half] + value_offset, values_address + (unsigned)(stage * VSTAGE + half * VHALF + wave * 1024));
   };
   // where this lane's fragments lie in a stage
   const int key_fragment = (col & 7) * KBLOCK + (col >> 3) * 256 + g * 16;              // + h * 512 + c * 64
@@ -1438,6 +1446,25 @@ __device__ __forceinline__ void attention_prefill_d128_part(
   for (int head0 = kvh * group; head0 < (kvh + 1) * group; head0 += waves) {
     const int head = head0 + my_wave;
     const bool active = head < (kvh + 1) * group;
+    // the first tiles are asked for before the queries, whose way to the registers is as long
+    __syncthreads();                                           // the stages of an earlier pass are done with
+    int pending = 0;
+    if (first_tile <= last_tile) {
+      Pair keys[3], values[2];
+#pragma unroll
+      for (int n = 0; n < 3; ++n)
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          uint64_t at;
+          locate((first_tile + n) * 2 + half, keys[n].run[half], n < 2 ? values[n].run[half] : at);
+        }
+      fetch_keys(keys[0], 0);
+      fetch_values(values[0], 0);
+      if (first_tile + 1 <= last_tile) fetch_keys(keys[1], 1);
+      if (first_tile + 2 <= last_tile) fetch_keys(keys[2], 2), pending += 2;
+      if (first_tile + 1 <= last_tile) fetch_values(values[1], 1), pending += 2;
+      if (wave < 2 && first_tile + 2 <= last_tile) locate_block(wave);
+    }
     bf16x8 qf[QB][DS];
     floatx4 o[QB][DB];
     float run_max[QB], run_sum[QB];
@@ -1466,6 +1493,14 @@ __device__ __forceinline__ void attention_prefill_d128_part(
       }
 #pragma unroll
       for (int e = 0; e < DB; ++e) o[b][e] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    // The queries and positions are waited for here.  Left to the compiler the wait stands before their first use, in the walk's
+    // inner loop, where it waits for every fetch just asked for as well, in every turn.
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+      asm volatile("" : "+v"(pos[b]));
+#pragma unroll
+      for (int c = 0; c < DS; ++c) asm volatile("" : "+v"(qf[b][c]));
     }
 
     // the cap, in units of the unscaled scores (the scale enters with the exponent)
@@ -1614,9 +1649,14 @@ __device__ __forceinline__ void attention_prefill_d128_part(
     // three or four vector instructions of a weight cost nothing.  A head of 128 has as many products a tile
     // (8 for every 16 queries) as a lane has weights.  Returns false, and has changed nothing but pf and
     // next, if a weight sum says the reference point will not do.
-    auto weights_beside_scores = [&](int next_tile, int stage, floatx4 (&sc)[QB][2], floatx4 (&next)[QB][2], bf16x8 (&pf)[QB]) -> bool {
-      const unsigned char* kt = key_tiles + stage * KBYTES + key_fragment;
-      constexpr int FRAGMENTS = 2 * DS, READ_AHEAD = 3;
+    // The fragments of keys, and those of the tile's own values for the products that follow (values_read_ahead), are asked for
+    // READ_AHEAD ahead of their products.
+    constexpr int READ_AHEAD = 3;
+    auto weights_beside_scores = [&](int next_tile, int key_stage, int value_stage, floatx4 (&sc)[QB][2], floatx4 (&next)[QB][2],
+                                     bf16x8 (&pf)[QB], bf16x8 (&vf)[DB]) -> bool {
+      const unsigned char* kt = key_tiles + key_stage * KBYTES + key_fragment;
+      const unsigned char* vt = value_tiles + value_stage * VSTAGE + value_fragment;
+      constexpr int FRAGMENTS = 2 * DS;
       static_assert(FRAGMENTS * QB == QB * 8, "one weight for every product");
       bf16x8 kf[FRAGMENTS];
 #pragma unroll
@@ -1634,6 +1674,7 @@ __device__ __forceinline__ void attention_prefill_d128_part(
         const int f = n / QB, b = n % QB;
         if (b == 0 && f + READ_AHEAD < FRAGMENTS)
           kf[f + READ_AHEAD] = *(const bf16x8*)(kt + ((f + READ_AHEAD) / DS) * 512 + ((f + READ_AHEAD) % DS) * 64);
+        else if (b == 0) vf[f + READ_AHEAD - FRAGMENTS] = *(const bf16x8*)(vt + (f + READ_AHEAD - FRAGMENTS) * 512);
         next[b][f / DS] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[f], qf[b][f % DS], next[b][f / DS], 0, 0, 0);
         const int wb = n / 8, wh = (n / 4) % 2, wi = n % 4;      // the n-th weight of the lane
         weight[n] = fast_exp2(fmaf(sc[wb][wh][wi], scale2, shift[wb]));
@@ -1644,10 +1685,12 @@ __device__ __forceinline__ void attention_prefill_d128_part(
         }
         __builtin_amdgcn_sched_barrier(0);
       }
+#pragma unroll
+      for (int b = 0; b < QB; ++b) asm volatile("" : "+v"(pf[b]));       // packed before the way parts: half the registers
       bool again = false;
 #pragma unroll
       for (int b = 0; b < QB; ++b) again |= !(tile_sum[b] <= 0x1p60f);   // too large, infinite or not a number
-      if (__any(again)) return false;
+      if (__builtin_amdgcn_ballot_w64(again) != 0) return false;
 #pragma unroll
       for (int b = 0; b < QB; ++b) run_sum[b] += tile_sum[b];
       if constexpr (RAISES) {
@@ -1672,6 +1715,18 @@ __device__ __forceinline__ void attention_prefill_d128_part(
       }
     };
 
+    // ... whose first fragments are on their way
+    auto values_read_ahead = [&](int stage, const bf16x8 (&pf)[QB], bf16x8 (&vf)[DB]) {
+      const unsigned char* vt = value_tiles + stage * VSTAGE + value_fragment;
+#pragma unroll
+      for (int e = 0; e < DB; ++e) {
+        if (e + READ_AHEAD < DB) vf[e + READ_AHEAD] = *(const bf16x8*)(vt + (e + READ_AHEAD) * 512);
+#pragma unroll
+        for (int b = 0; b < QB; ++b) o[b][e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[e], pf[b], o[b][e], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+
     // Tiles [whole_begin, whole_end) need no mask: every query of the group sees every key of theirs.
     int whole_begin = (lo_last + 31) / 32, whole_end = (pos_first + 1) / 32;
     if (whole_begin < first_tile) whole_begin = first_tile;
@@ -1684,45 +1739,38 @@ __device__ __forceinline__ void attention_prefill_d128_part(
     // stage was last read a turn ago, for the scores of t) and the values of t + 2 (likewise), computes the
     // scores of t + 1 beside the weights of t, adds the values of t, and before the barrier waits until only
     // what it asked for itself is still on its way: the keys of t + 2 and the values of t + 1 are then in LDS.
-    __syncthreads();                                           // the stages of an earlier pass are done with
     floatx4 sa[QB][2], sb[QB][2];
     bf16x8 pf[QB];
-    int pages_ahead[2];                                        // the pages of tile + 3 at the top of a turn
-    const char* values_ahead[2];                               // where the values of tile + 2 lie
+    Pair keys_ahead, values_ahead;                             // at the top of a turn: where the keys of tile + 3 and the values of tile + 2 lie
     if (first_tile <= last_tile) {
-      int pages[2];
-      const char *kbase[2], *vbase[2];
-      pages_of(std::false_type{}, first_tile, pages);
-      locate(std::false_type{}, first_tile, pages, kbase, vbase);
-      fetch_keys(kbase, 0);
-      fetch_values(vbase, 0);
-      pages_of(std::false_type{}, first_tile + 1, pages);
-      locate(std::false_type{}, first_tile + 1, pages, kbase, values_ahead);
-      if (first_tile + 1 <= last_tile) fetch_keys(kbase, 1);
-      int pending = 0;
-      pages_of(std::false_type{}, first_tile + 2, pages);
-      locate(std::false_type{}, first_tile + 2, pages, kbase, vbase);
-      if (first_tile + 2 <= last_tile) fetch_keys(kbase, 2), pending += 2;
-      if (first_tile + 1 <= last_tile) fetch_values(values_ahead, 1), pending += 2;
-      values_ahead[0] = vbase[0], values_ahead[1] = vbase[1];
-      pages_of(std::false_type{}, first_tile + 3, pages_ahead);
       if (pending == 4) fetched_and_read_then_barrier<4>();
       else if (pending == 2) fetched_and_read_then_barrier<2>();
       else fetched_and_read_then_barrier<0>();
+      keys_ahead = runs_at(lds.key_runs, 6);
+      values_ahead = runs_at(lds.value_runs, 6);
       if (!IDLE_WAVES || active) scores(first_tile, 0, sa);
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // everyone has read the first keys: their stage may be filled again
     }
     int tile = first_tile, stage = 0;                          // stage = (tile - first_tile) % 3
+    int place = 6;                                             // where the addresses of the tiles ahead stand in their rings
+    // the third block and those after it are looked up two turns into the block before them, the last one that holds a tile too
+    const int last_locate = last_tile - (BLOCK_RUNS / 2 - 2);
+    int locate_at = first_tile + BLOCK_RUNS / 2 + 2 <= last_locate ? first_tile + BLOCK_RUNS / 2 + 2 : -1;
     // the turn's fetches, and how many they are; EVERY: tile + 3 is not past the last, so all of them happen
     auto ask_ahead = [&](auto every) -> int {
       constexpr bool EVERY = decltype(every)::value;
       int pending = 0;
-      const char *kbase[2], *vbase[2];
-      locate(std::true_type{}, tile + 3, pages_ahead, kbase, vbase);
-      if (EVERY || tile + 3 <= last_tile) fetch_keys(kbase, stage), pending += 2;
+      if (tile == locate_at) {
+        // the block of runs behind the one that the walk is in takes the place of the one before it, which the walk left two turns ago
+        if (wave == 0) locate_block((tile - first_tile) / (BLOCK_RUNS / 2) + 1);
+        locate_at += BLOCK_RUNS / 2;
+        if (locate_at > last_locate) locate_at = -1;
+      }
+      if (EVERY || tile + 3 <= last_tile) fetch_keys(keys_ahead, stage), pending += 2;
       if (EVERY || tile + 2 <= last_tile) fetch_values(values_ahead, stage == 0 ? STAGES - 1 : stage - 1), pending += 2;
-      values_ahead[0] = vbase[0], values_ahead[1] = vbase[1];
-      pages_of(std::true_type{}, tile + 4, pages_ahead);        // wanted a turn from now
+      place = (place + 2) & (RUNS - 1);
+      keys_ahead = runs_at(lds.key_runs, place);                // wanted a turn from now
+      values_ahead = runs_at(lds.value_runs, place);
       return pending;
     };
     auto turn_over = [&](int pending) {
@@ -1746,15 +1794,17 @@ __device__ __forceinline__ void attention_prefill_d128_part(
     }
     for (;;) {
       bool asked = false;                                      // the turn's fetches have been asked for already
+      const int fast_until = tile >= fast_begin ? fast_end : tile;
       // one way out of the inner loop only, at its top, before anything of the turn has happened to the accumulators
       for (;;) {
-        if (asked || tile < fast_begin || tile >= fast_end || (RAISES && grown)) break;
+        if (asked || tile >= fast_until || (RAISES && grown)) break;
         ask_ahead(std::true_type{});
-        if (!weights_beside_scores(tile + 1, stage == STAGES - 1 ? 0 : stage + 1, sa, sb, pf)) {
+        bf16x8 vf[DB];
+        if (!weights_beside_scores(tile + 1, stage == STAGES - 1 ? 0 : stage + 1, stage, sa, sb, pf, vf)) {
           asked = true;
           continue;
         }
-        values(stage, pf);
+        values_read_ahead(stage, pf, vf);
         turn_over(4);
 #pragma unroll
         for (int b = 0; b < QB; ++b) sa[b][0] = sb[b][0], sa[b][1] = sb[b][1];
@@ -1767,12 +1817,12 @@ __device__ __forceinline__ void attention_prefill_d128_part(
       }
       const bool unfinished = tile <= last_tile;
       if (!unfinished) break;
-      const int pending = asked ? 4 : ask_ahead(std::false_type{});
+      const int on_their_way = asked ? 4 : ask_ahead(std::false_type{});
       if (tile < last_tile) scores(tile + 1, stage == STAGES - 1 ? 0 : stage + 1, sb);
       if (tile >= whole_begin && tile < whole_end) weights_with_maximum(tile, sa, std::false_type{}, pf);
       else weights_with_maximum(tile, sa, std::true_type{}, pf);
       values(stage, pf);
-      turn_over(pending);
+      turn_over(on_their_way);
 #pragma unroll
       for (int b = 0; b < QB; ++b) sa[b][0] = sb[b][0], sa[b][1] = sb[b][1];
     }
@@ -1806,7 +1856,7 @@ __device__ __forceinline__ void attention_prefill_d128_part(
 }
 
 template <int QB, bool MANY_WAVES, int SPREAD, int SCORES>
-__global__ __launch_bounds__(MANY_WAVES ? 512 : 256, MANY_WAVES ? 1 : QB == 1 && (SCORES & SCORES_LINEAR) ? 3 : 2) void attention_prefill_d128_bf16_kernel(
+__global__ __launch_bounds__(MANY_WAVES ? 512 : 256, MANY_WAVES ? 1 : QB == 1 ? 3 : 2) void attention_prefill_d128_bf16_kernel(
     bf16* __restrict__ out, int out_stride, const bf16* __restrict__ q, int q_stride,
     const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
     const int* __restrict__ block_table, int table_stride, const int* __restrict__ token_request,

@@ -104,6 +104,11 @@ __device__ __forceinline__ void fetch_to_lds(const void* base, unsigned lane_off
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                :: "s"(__builtin_amdgcn_readfirstlane(lds_address)), "v"(lane_offset), "s"(uniform_base) : "memory");
 }
+// The same from an address of each lane's own.
+__device__ __forceinline__ void fetch_lanes_to_lds(uint64_t address, unsigned lds_address) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :: "s"(__builtin_amdgcn_readfirstlane(lds_address)), "v"(address) : "memory");
+}
 // Waits until at most `PENDING` of this wave's fetches are still on their way and this wave has what it read from LDS, then for the
 // workgroup.  The reads as well: behind the barrier others ask memory to fill what was read from, and a read that waits its turn in
 // a busy compute unit can take as long as a fetch that its L2 answers.
