@@ -14,6 +14,7 @@
 //   moe_combine   per token: the weighted sum of its experts' rows in the order of its choices, and, when a norm
 //                 weight is given, the RMS norm of that sum added into the residual stream.
 #include "common.h"
+#include "lines_walk.h"
 
 LRS_API int lrs_compute_units();
 
@@ -562,7 +563,42 @@ __device__ __forceinline__ int nth_in_use(const int* __restrict__ tile_expert, i
   return 0;
 }
 
-// The grouped product for large steps the way this package's many-rows product is made (gemm_bf16_wide in gemm.hip):
+// A wave's sums into the output: rows m0 + 16 jt .. in sorted order, columns n0 + 16 it ..; rows that only pad are not written.
+template <int IT, int JT, typename TO>
+__device__ __forceinline__ void store_expert_tile(floatx4 (&acc)[IT][JT], TO* __restrict__ out, int ldc, int m0, int n0, int n,
+                                                  const int* __restrict__ sorted, int act, const PairAct& pa) {
+  const int lane = threadIdx.x % WAVE, r = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int jt = 0; jt < JT; ++jt) {
+    const int at = m0 + jt * 16 + r;
+    const bool pair = sorted[at] >= 0;
+    const float pw = pair && act == ACT_CLAMPED_PAIRS ? weight_of_row(pa, sorted, at) : 1.f;
+    const int64_t row_at = (int64_t)at * ldc;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int row0 = n0 + it * 16 + 4 * g;                  // this lane's four weight rows = output columns
+      if (pair && row0 < n) {
+        floatx4 v = acc[it][jt];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = __shfl(v[i], lane, WAVE);      // keeps the loop above free of spills, as in the dense kernel
+        if (act == ACT_RELU_SQUARED) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = v[i] > 0.f ? v[i] * v[i] : 0.f;
+        }
+        if (act >= ACT_SILU_PAIRS) {
+          const float first = pair_times(act, v[0], v[1], pw, pa), second = pair_times(act, v[2], v[3], pw, pa);
+          if constexpr (sizeof(TO) == 2) *(bf16x2*)((bf16*)out + row_at + row0 / 2) = bf16x2{(bf16)first, (bf16)second};
+          else ((float*)out)[row_at + row0 / 2] = first, ((float*)out)[row_at + row0 / 2 + 1] = second;
+        } else if constexpr (sizeof(TO) == 2) *(bf16x4*)((bf16*)out + row_at + row0) = bf16x4{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
+        else *(floatx4*)((float*)out + row_at + row0) = v;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
+// The grouped product for large steps whose K is 32 more than a multiple of 64 (the kernel below takes multiples), the way this
+// package's many-rows product is made (gemm_bf16_wide in gemm.hip):
 // 128 sorted rows x 256 columns of one expert per workgroup of four waves, a wave 64 rows x 128 columns; memory writes
 // slices of 32 of K straight into LDS (fetch_to_lds), three stages, in a layout whose rows swap places and whose chunks
 // are turned round by the row number so that every fragment read touches every bank once; no registers hold a slice on
@@ -658,33 +694,122 @@ __global__ __launch_bounds__(256, 2) void moe_experts_bf16_fetch_kernel(TO* __re
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");               // the fetches past K that nobody reads
   asm volatile("" : "+s"(ldc), "+s"(m0_opaque));
-#pragma unroll
-  for (int jt = 0; jt < 4; ++jt) {
-    const int at = m0_opaque + wm + jt * 16 + r;
-    const bool pair = sorted[at] >= 0;
-    const float pw = pair && act == ACT_CLAMPED_PAIRS ? weight_of_row(pa, sorted, at) : 1.f;
-    const int64_t row_at = (int64_t)at * ldc;
-#pragma unroll
-    for (int it = 0; it < 8; ++it) {
-      const int row0 = n0 + wn + it * 16 + 4 * g;                  // this lane's four weight rows = output columns
-      if (pair && row0 < n) {
-        floatx4 v = acc[it][jt];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = __shfl(v[i], lane, WAVE);      // keeps the loop above free of spills, as in the dense kernel
-        if (act == ACT_RELU_SQUARED) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) v[i] = v[i] > 0.f ? v[i] * v[i] : 0.f;
-        }
-        if (act >= ACT_SILU_PAIRS) {
-          const float first = pair_times(act, v[0], v[1], pw, pa), second = pair_times(act, v[2], v[3], pw, pa);
-          if constexpr (sizeof(TO) == 2) *(bf16x2*)((bf16*)out + row_at + row0 / 2) = bf16x2{(bf16)first, (bf16)second};
-          else ((float*)out)[row_at + row0 / 2] = first, ((float*)out)[row_at + row0 / 2 + 1] = second;
-        } else if constexpr (sizeof(TO) == 2) *(bf16x4*)((bf16*)out + row_at + row0) = bf16x4{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
-        else *(floatx4*)((float*)out + row_at + row0) = v;
-      }
-      __builtin_amdgcn_sched_barrier(0);
+  store_expert_tile<8, 4>(acc, out, ldc, m0_opaque + wm, n0 + wn, n, sorted, act, pa);
+}
+
+// The list's tiles two by two: a pair is two neighbouring tiles of one expert, counted from the first of its run; the last of an odd
+// run stands alone.  COUNT: how many pairs there are (first) and how many tiles alone; else the first tile of the nth pair, or the nth
+// tile alone.  A wave looks at 64 places a turn.
+struct TilesUsed {
+  int pairs, alone;
+};
+template <bool COUNT>
+__device__ __forceinline__ TilesUsed tiles_by_two(const int* __restrict__ tile_expert, int tiles, int lane, int n, bool paired) {
+  int before = -2, start = 0;                                          // the expert of the place before, where its run began
+  TilesUsed used{0, 0};
+  for (int at = 0; at < tiles; at += WAVE) {
+    const int place = at + lane, expert = place < tiles ? tile_expert[place] : -1, right = place + 1 < tiles ? tile_expert[place + 1] : -1;
+    int left = __shfl_up(expert, 1, WAVE);
+    if (lane == 0) left = before;
+    const unsigned long long starts = __ballot(expert != left), here = starts & (~0ull >> (63 - lane));
+    const int run = here ? at + 63 - __clzll(here) : start;
+    const bool first = expert >= 0 && ((place - run) & 1) == 0;
+    const unsigned long long two = __ballot(first && right == expert), one = __ballot(first && right != expert);
+    if (!COUNT) {
+      const unsigned long long mask = paired ? two : one;
+      const int earlier = __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0));
+      if (n < __popcll(mask)) return TilesUsed{at + __ffsll(__ballot((mask >> lane & 1) != 0 && earlier == n)) - 1, 0};
+      n -= __popcll(mask);
     }
+    used.pairs += __popcll(two);
+    used.alone += __popcll(one);
+    before = __shfl(expert, 63, WAVE);
+    if (starts) start = at + 63 - __clzll(starts);
   }
+  return used;
+}
+
+// The grouped product for large steps whose K is a multiple of 64: two tiles of an expert (256 rows) x 256 columns a workgroup of
+// eight waves, a wave 128 rows x 64 columns, two stages of 64 KB; the last tile of an odd run alone, a wave 64 x 64, three stages of
+// 48 KB.  Slices of 64 of K (lines_walk.h): the kernel above takes half lines, of which the L2s hand out half as many bytes (17 TB/s
+// against 34, measured with nothing but fetches), and its tiles of 128 x 256 take half as much again for every product.  What bounds
+// it: few rows an expert, the weights' way from memory; many, the clock (some 2 GHz with the matrix cores this busy), the rows that
+// pad runs to tiles and the last round of workgroups.  Pairs before tiles alone: in the list's order a late pair made a round of its
+// own (612 tokens 218 us for 160).  32 experts of 8 choices, 4,096 -> 2,304 features and back, this kernel against that one: 200
+// tokens 176 / 194 and 132 / 138 us, 612 160 / 190 and 197 / 225, 1,200 247 / 322 and 270 / 321, 2,048 415 / 501 and 429 / 507, 8,192
+// 1,167 / 1,422; at 500 tokens 160 / 184 and 194 / 186.
+template <int TILES, int STAGES, typename TO>
+__device__ __forceinline__ void experts_tile(bf16* slices, TO* __restrict__ out, int ldc, const bf16* __restrict__ x, int lda,
+                                             const bf16* __restrict__ w, int n, int k, const int* __restrict__ sorted, int m0, int n0,
+                                             int top, int gather, int act, const PairAct& pa) {
+  constexpr int BM = 128 * TILES, BN = 256, BK = LINES_BK, IT = 4, JT = 4 * TILES;
+  constexpr int XL = BM / 8 / 8, WL = BN / 8 / 8, STAGE_ELEMENTS = (BM + BN) * BK;
+  const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int wm = (wave >> 2) * (16 * JT), wn = (wave & 3) * 64;
+  const int place_row = lines_place_row(lane), place_chunk = lines_place_chunk(lane);
+  const int first_pair = sorted[m0];                                 // a tile in use begins with a row in use
+  const int fallback = gather ? first_pair / top : m0;
+  unsigned xoff[XL], woff[WL];
+#pragma unroll
+  for (int i = 0; i < XL; ++i) {
+    const int at = m0 + 8 * (wave + 8 * i) + place_row, pair = sorted[at];
+    const int row = pair < 0 ? fallback : (gather ? pair / top : at);
+    xoff[i] = (unsigned)((row * lda + place_chunk * 8) * 2);
+  }
+#pragma unroll
+  for (int i = 0; i < WL; ++i) {
+    const int row = n0 + 8 * (wave + 8 * i) + place_row;
+    woff[i] = (unsigned)(((row < n ? row : n - 1) * k + place_chunk * 8) * 2);
+  }
+  floatx4 acc[IT][JT];
+#pragma unroll
+  for (int it = 0; it < IT; ++it)
+#pragma unroll
+    for (int jt = 0; jt < JT; ++jt) acc[it][jt] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int steps = k / BK;
+  const unsigned slices_address = (unsigned)(uintptr_t)(__attribute__((address_space(3))) bf16*)slices;
+  auto fetch = [&](int kt, int stage) {
+    const int at = (kt < steps ? kt : steps - 1) * BK * 2;
+    const unsigned to = slices_address + (unsigned)(stage * STAGE_ELEMENTS * 2 + wave * 1024);
+#pragma unroll
+    for (int i = 0; i < XL; ++i) fetch_to_lds((const char*)x + at, xoff[i], to + (unsigned)(i * 8192));
+#pragma unroll
+    for (int i = 0; i < WL; ++i) fetch_to_lds((const char*)w + at, woff[i], to + (unsigned)(BM * BK * 2 + i * 8192));
+  };
+  int m0_opaque = m0;
+  lines_walk<STAGES, XL + WL>(acc, slices, BM, BN, wm, wn, steps, fetch);
+  asm volatile("" : "+s"(ldc), "+s"(m0_opaque));
+  store_expert_tile<IT, JT>(acc, out, ldc, m0_opaque + wm, n0 + wn, n, sorted, act, pa);
+}
+template <typename TO>
+__global__ __launch_bounds__(512, 1) void moe_experts_bf16_pairs_kernel(TO* __restrict__ out, int ldc, const bf16* __restrict__ x, int lda,
+                                                                        const bf16* __restrict__ w, int n, int k, const int* __restrict__ sorted,
+                                                                        const int* __restrict__ tile_expert, int tiles_m, int tiles_n, int top,
+                                                                        int gather, int act, const PairAct pa) {
+  __shared__ __attribute__((aligned(64))) bf16 slices[3 * (128 + 256) * LINES_BK];
+  static_assert(sizeof(slices) >= 2 * (256 + 256) * LINES_BK * sizeof(bf16), "two stages of two tiles");
+  const int lane = threadIdx.x % WAVE;
+  // Every die has an equal run of the pairs' tiles and one of those alone, and begins with the pairs, which take twice as long: the
+  // last to start are short.
+  const TilesUsed used = tiles_by_two<true>(tile_expert, tiles_m, lane, 0, false);
+  const int die = blockIdx.x % 8, paired_items = used.pairs * tiles_n, alone_items = used.alone * tiles_n;
+  const int paired_here = paired_items / 8 + (die < paired_items % 8), alone_here = alone_items / 8 + (7 - die < alone_items % 8);
+  int id = blockIdx.x / 8;
+  if (id >= paired_here + alone_here) return;
+  const bool paired = id < paired_here;
+  if (paired) id += die * (paired_items / 8) + (die < paired_items % 8 ? die : paired_items % 8);
+  else id += die * (alone_items / 8) + (alone_items % 8 > 8 - die ? alone_items % 8 - (8 - die) : 0) - paired_here;
+  const int rows = paired ? used.pairs : used.alone;
+  const int band = id / (4 * tiles_n), within = id % (4 * tiles_n);
+  const int band_rows = rows - band * 4 < 4 ? rows - band * 4 : 4;
+  const int tile_m = __builtin_amdgcn_readfirstlane(tiles_by_two<false>(tile_expert, tiles_m, lane, band * 4 + within % band_rows, paired).pairs);
+  const int expert = tile_expert[tile_m];
+  const bf16* we = w + (int64_t)expert * n * k;
+  const int n0 = (within / band_rows) * 256;
+  if (paired)
+    experts_tile<2, 2>(slices, out, ldc, x, lda, we, n, k, sorted, tile_m * 128, n0, top, gather, act, pa);
+  else
+    experts_tile<1, 3>(slices, out, ldc, x, lda, we, n, k, sorted, tile_m * 128, n0, top, gather, act, pa);
 }
 
 // What becomes of a token's weighted sum y of its experts' rows:
@@ -985,10 +1110,20 @@ LRS_API int lrs_moe_experts(void* out, int out_dtype, int ldc, const void* a, co
   LRS_REQUIRE(act < ACT_SILU_PAIRS || n % 4 == 0, "moe_experts: pairs of gate and up rows come four rows at a time, got %d rows", n);
   hipStream_t s = (hipStream_t)stream;
   const bool cores = dtype == LRS_BF16 && k % GK == 0 && lda % 8 == 0 && ((uintptr_t)a % 16) == 0 && ((uintptr_t)w % 16) == 0;
-  // large steps of shapes the fetching kernel takes: whole slices of 32 of K, rows of the output 16 bytes aligned, offsets
+  // large steps of shapes the fetching kernels take: whole slices of 32 of K, rows of the output 16 bytes aligned, offsets
   // that fit 32 bits
   const bool fetching = cores && tile == WM && k % 32 == 0 && n % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)out % 16) == 0 && k >= 64 &&
                         (int64_t)n * k < (1ll << 30) && (gather ? (int64_t)max_tiles * tile / top + 1 : (int64_t)max_tiles * tile) * lda < (1ll << 30);
+  if (fetching && k % LINES_BK == 0) {
+    const int tiles_n = (n + 255) / 256;
+    if (out_dtype == LRS_BF16)
+      moe_experts_bf16_pairs_kernel<bf16><<<max_tiles * tiles_n + 16, 512, 0, s>>>((bf16*)out, ldc, (const bf16*)a, lda, (const bf16*)w, n, k, sorted, tile_expert, max_tiles, tiles_n, top, gather, act, pa);
+    else if (out_dtype == LRS_F32)
+      moe_experts_bf16_pairs_kernel<float><<<max_tiles * tiles_n + 16, 512, 0, s>>>((float*)out, ldc, (const bf16*)a, lda, (const bf16*)w, n, k, sorted, tile_expert, max_tiles, tiles_n, top, gather, act, pa);
+    else
+      return lrs_fail("moe_experts: unknown output dtype %d", out_dtype);
+    return lrs_check_launch("moe_experts");
+  }
   if (fetching) {
     const int tiles_n = (n + 255) / 256;
     if (out_dtype == LRS_BF16)

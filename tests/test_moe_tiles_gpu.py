@@ -60,3 +60,44 @@ def test_lists_with_tiles_not_in_use_between_those_in_use(count, top, tokens):
     between = torch.ones(spread, dtype=torch.bool)
     between[to] = False
     assert (got[between.cuda()] == -7.0).all()
+
+
+# runs of one tile, two, an odd and an even number of them, one of more than 64 tiles, and few or many columns; K of one slice of 64, two
+# and more (and of half a slice more, which another kernel takes); rows gathered and rows as they are
+@pytest.mark.parametrize("rows,n,k", [((1,), 256, 64), ((128, 129, 256, 257, 1), 260, 128), ((384, 0, 500, 128), 516, 192), ((9000, 130, 640), 68, 448), ((300,) * 70, 256, 320),
+                                      ((200, 700), 260, 96)])
+@pytest.mark.parametrize("gather,kind", [(True, "bf16"), (True, "pairs"), (False, "f32")])
+def test_two_tiles_and_one(rows, n, k, gather, kind):
+    from llm_runtime_study_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(n + k)
+    count, tile = len(rows), 128
+    tiles = [-(-m // tile) for m in rows]
+    total = sum(tiles)
+    spare = 3                                                    # tiles not in use at the end
+    listed = torch.full((total + spare, tile), -1, dtype=torch.int32)
+    experts, pair, at = torch.full((total + spare,), -1, dtype=torch.int32), 0, 0
+    order = torch.randperm(sum(rows), generator=g).to(torch.int32)
+    for e, m in enumerate(rows):
+        experts[at:at + tiles[e]] = e
+        listed[at:at + tiles[e]].view(-1)[:m] = order[pair:pair + m]
+        at, pair = at + tiles[e], pair + m
+    x = torch.randn(sum(rows) if gather else listed.numel(), k, generator=g).to(torch.bfloat16)
+    w = torch.randn(count, n, k, generator=g).to(torch.bfloat16)
+    out = torch.full((listed.numel(), n // 2 if kind == "pairs" else n), -7.0, device="cuda", dtype=torch.float32 if kind == "f32" else torch.bfloat16)
+    ops.moe_experts(out, x.cuda(), w.cuda(), listed.flatten().cuda(), experts.cuda(), tile, 1, gather=gather, relu_squared=False, silu_pairs=kind == "pairs")
+    got, flat = out.cpu().double(), listed.flatten()
+    assert (got[flat < 0] == -7.0).all()
+    for e in range(count):
+        rows_of = ((experts == e).repeat_interleave(tile) & (flat >= 0)).nonzero().flatten()
+        a = x[flat[rows_of].long()] if gather else x[rows_of]
+        want, size = a.double() @ w[e].double().T, a.double().abs() @ w[e].double().abs().T
+        bound = k * 2.0 ** -23 * size                            # float32 sums of k exact products, whatever their order
+        if kind == "pairs":
+            # silu' is at most 1.1; a rounding to bfloat16 of at most 2^-8 at the end, exp and division in float32 below it
+            gate, up = want[:, 0::2], want[:, 1::2]
+            bound = 1.1 * bound[:, 0::2] * up.abs() + gate.abs() * bound[:, 1::2] + 1e-6 * (gate * up).abs()
+            want = torch.nn.functional.silu(gate) * up
+        if kind != "f32":
+            bound = bound + (want.abs() + bound) * 2.0 ** -8
+        assert ((got[rows_of] - want).abs() <= bound + 1e-30).all()
