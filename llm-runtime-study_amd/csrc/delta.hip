@@ -21,7 +21,11 @@
 //   S of head h at h * rows * vdim * 16 floats, element (i, j) at ((i % rows) * vdim + j) * 16 + i / rows with
 //   rows = 4, 8 or 16 (dim over the 16 lanes of a column, padded): the order in which the scan's threads hold it,
 //   so that loading and storing it are whole lines; then [taps - 1, channels], oldest first.
+// (delta_chunks.hip has the form of the scan for long portions on the matrix cores.)
 #include "common.h"
+
+void lrs_delta_chunk_walk(const float* qkv, const float* gates, const int* cu, const int* slot_ids, int tokens, int requests, float* state,
+                          int64_t state_stride, int G, int H, int d, int dv, float* raw, float* packs, hipStream_t s);
 
 namespace {
 
@@ -496,11 +500,12 @@ namespace {
 // head and key channel from decay_rank values (decay_up [decay_rank, H*d], dt_bias [H*d], decays [tokens, H*d] scratch);
 // gate_rank > 0: a sigmoid gate from gate_rank values (gate_up [gate_rank, H*dv]); 0: silu of H*dv columns.  A rank below 0:
 // the inputs were made by a product of the caller's: decays [tokens, H*d] holds the decays' inputs, gate_up [tokens, H*dv] the gate's.
+// packs: null, or the scratch with which the requests behind the step's first `singles` (one token each) take the form in chunks.
 int delta_launch(void* out, int out_dtype, const void* proj, int proj_dtype, int ld, int tokens, int requests,
                  const int* token_request, const int* cu, const int* slot_ids, float* state, int64_t state_stride,
                  const float* conv_w, int taps, int G, int H, int d, int dv, const float* a_log, const float* dt_bias,
                  const float* norm_w, float eps, float* qkv, float* gates, float* raw, int gate_at, int beta_at, int decay_at,
-                 int decay_rank, const float* decay_up, float* decays, int gate_rank, const float* gate_up, void* stream) {
+                 int decay_rank, const float* decay_up, float* decays, int gate_rank, const float* gate_up, float* packs, int singles, void* stream) {
   LRS_REQUIRE(tokens > 0 && requests > 0 && requests <= tokens, "delta_rule: bad sizes tokens=%d requests=%d", tokens, requests);
   LRS_REQUIRE(G > 0 && H > 0 && H % G == 0 && d > 0 && dv > 0 && taps >= 1, "delta_rule: bad sizes G=%d H=%d d=%d dv=%d taps=%d", G, H, d, dv, taps);
   LRS_REQUIRE(d <= 256, "delta_rule: takes keys of up to 256 values, got %d", d);
@@ -515,6 +520,9 @@ int delta_launch(void* out, int out_dtype, const void* proj, int proj_dtype, int
   LRS_REQUIRE(((uintptr_t)qkv % 16) == 0 && ((uintptr_t)decays % 16) == 0, "delta_rule: the scratch rows must be 16 bytes aligned");
   LRS_REQUIRE(decay_rank == 0 || ((decay_up || decay_rank < 0) && decays), "delta_rule: decays per channel need their matrix and scratch rows");
   LRS_REQUIRE(gate_rank == 0 || gate_up, "delta_rule: a gate of low rank needs its matrix or its inputs");
+  LRS_REQUIRE(!packs || (decay_rank == 0 && d <= 128 && ((uintptr_t)packs % 16) == 0),
+              "delta_rule: the form in chunks takes one decay a head, keys of up to 128 values and scratch that is 16 bytes aligned");
+  LRS_REQUIRE(!packs || (singles >= 0 && singles < requests), "delta_rule: %d single tokens leave no portion among %d requests", singles, requests);
   hipStream_t s = (hipStream_t)stream;
   dim3 pgrid(tokens, 2 * G + H), kgrid(requests, (channels + 255) / 256), sgrid(requests, H, (dv + COLUMNS - 1) / COLUMNS);
   const int64_t pairs = (int64_t)tokens * H;
@@ -528,7 +536,12 @@ int delta_launch(void* out, int out_dtype, const void* proj, int proj_dtype, int
       delta_conv_keep_kernel<TP><<<kgrid, 256, 0, s>>>((const TP*)proj, ld, cu, slot_ids, state, state_stride, conv_offset,  \
                                                        taps, channels, 0);                                                    \
     if (decay_rank != 0) launch_scan<RULE_DELTA_CHANNELS>(rows, single, sgrid, s, qkv, gates, cu, slot_ids, state, state_stride, G, H, d, dv, raw, decays); \
-    else launch_scan<RULE_DELTA>(rows, single, sgrid, s, qkv, gates, cu, slot_ids, state, state_stride, G, H, d, dv, raw, nullptr);                    \
+    else if (!packs) launch_scan<RULE_DELTA>(rows, single, sgrid, s, qkv, gates, cu, slot_ids, state, state_stride, G, H, d, dv, raw, nullptr); \
+    else {                                                                                                                    \
+      if (singles > 0)                                                                                                        \
+        launch_scan<RULE_DELTA>(rows, true, dim3(singles, sgrid.y, sgrid.z), s, qkv, gates, cu, slot_ids, state, state_stride, G, H, d, dv, raw, nullptr); \
+      lrs_delta_chunk_walk(qkv, gates, cu + singles, slot_ids + singles, tokens, requests - singles, state, state_stride, G, H, d, dv, raw, packs, s); \
+    }                                                                                                                         \
     delta_gate_kernel<TP, TO><<<(unsigned)((pairs + 3) / 4), 256, 0, s>>>(raw, (const TP*)proj, ld, gate_at, norm_w, eps, tokens, H, dv, (TO*)out, \
                                                                           gate_rank, gate_up);                                \
   } while (0)
@@ -551,7 +564,22 @@ LRS_API int lrs_delta_rule(void* out, int out_dtype, const void* proj, int proj_
   const int channels = 2 * G * d + H * dv;
   return delta_launch(out, out_dtype, proj, proj_dtype, ld, tokens, requests, token_request, cu, slot_ids, state, state_stride, conv_w, taps,
                       G, H, d, dv, a_log, dt_bias, norm_w, eps, qkv, gates, raw, channels, channels + H * dv, channels + H * dv + H, 0, nullptr,
-                      nullptr, 0, nullptr, stream);
+                      nullptr, 0, nullptr, nullptr, 0, stream);
+}
+
+// The same with the form in chunks for the requests behind the first `singles`, which bring one token each (their tokens are the
+// step's first): packs holds lrs_delta_pack_floats(tokens, requests, H, d, dv) floats, d is at most 128.
+LRS_API int lrs_delta_rule_chunks(void* out, int out_dtype, const void* proj, int proj_dtype, int ld, int tokens, int requests,
+                                  const int* token_request, const int* cu, const int* slot_ids, float* state, int64_t state_stride,
+                                  const float* conv_w, int taps, int G, int H, int d, int dv, const float* a_log,
+                                  const float* dt_bias, const float* norm_w, float eps, float* qkv, float* gates, float* raw,
+                                  float* packs, int singles, void* stream) {
+  LRS_REQUIRE(packs, "delta_rule_chunks: needs the packs' scratch");
+  LRS_REQUIRE(tokens > requests, "delta_rule_chunks: %d tokens of %d requests hold no portion", tokens, requests);
+  const int channels = 2 * G * d + H * dv;
+  return delta_launch(out, out_dtype, proj, proj_dtype, ld, tokens, requests, token_request, cu, slot_ids, state, state_stride, conv_w, taps,
+                      G, H, d, dv, a_log, dt_bias, norm_w, eps, qkv, gates, raw, channels, channels + H * dv, channels + H * dv + H, 0, nullptr,
+                      nullptr, 0, nullptr, packs, singles, stream);
 }
 
 // The rule with a decay per head and key channel and a sigmoid gate, both from inputs of low rank.  proj columns:
@@ -568,7 +596,7 @@ LRS_API int lrs_delta_rule_channels(void* out, int out_dtype, const void* proj, 
   const int channels = 2 * G * d + H * dv;
   return delta_launch(out, out_dtype, proj, proj_dtype, ld, tokens, requests, token_request, cu, slot_ids, state, state_stride, conv_w, taps,
                       G, H, d, dv, a_log, dt_bias, norm_w, eps, qkv, gates, raw, channels + H + decay_rank, channels, channels + H, decay_rank,
-                      decay_up, decays, gate_rank, gate_up, stream);
+                      decay_up, decays, gate_rank, gate_up, nullptr, 0, stream);
 }
 
 // One step of the state space recurrence for a ragged batch.  proj [tokens, ld]: z (H*dv) | x (H*dv) | B (G*N) | C (G*N) | dt (H).

@@ -181,6 +181,10 @@ _SIGNATURES = {
     "lrs_delta_state_rows": (c_int, [c_int]),
     "lrs_delta_rule": (c_int, [c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int64,
                                c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "lrs_delta_pack_floats": (c_int64, [c_int, c_int, c_int, c_int, c_int]),
+    "lrs_delta_rule_chunks": (c_int, [c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int64,
+                                      c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p,
+                                      c_void_p, c_int, c_void_p]),
     "lrs_moe_tile_rows": (c_int, [c_int, c_int]),
     "lrs_moe_max_tiles": (c_int, [c_int, c_int]),
     "lrs_moe_route": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p]),
@@ -241,7 +245,7 @@ def library():
 # PLAN_OPS fixes the number of each entry point inside a plan; csrc/plan_dispatch.inc, made from this list
 # and _SIGNATURES by kernels/plan_codegen.py, is the other side (a test keeps the two in step).
 PLAN_OPS = ("lrs_activation", "lrs_add_gathered", "lrs_add_into", "lrs_add_rmsnorm", "lrs_advance_decode", "lrs_advance_slots", "lrs_attention", "lrs_attention_decode",
-            "lrs_attention_mixed", "lrs_attention_prefill", "lrs_axpby", "lrs_choose_tokens", "lrs_choose_tokens_split", "lrs_copy_to_pinned", "lrs_delta_rule", "lrs_delta_rule_channels", "lrs_embed", "lrs_fill_i32",
+            "lrs_attention_mixed", "lrs_attention_prefill", "lrs_axpby", "lrs_choose_tokens", "lrs_choose_tokens_split", "lrs_copy_to_pinned", "lrs_delta_rule", "lrs_delta_rule_channels", "lrs_delta_rule_chunks", "lrs_embed", "lrs_fill_i32",
             "lrs_filter_logits", "lrs_gated_clamped", "lrs_gated_norm_add", "lrs_gather_rows", "lrs_gemm", "lrs_gemm_lines_add_rmsnorm", "lrs_gemm_mid_add_norm_begin", "lrs_gemm_mid_qk_prep", "lrs_gemm_mid_scaled",
             "lrs_gemm_norm_chain", "lrs_head_gemm", "lrs_latent_attention", "lrs_latent_attention_groups", "lrs_latent_prep", "lrs_layernorm", "lrs_library_gemm", "lrs_mlstm", "lrs_mlstm_chunks", "lrs_moe_align", "lrs_moe_combine", "lrs_moe_experts", "lrs_moe_route", "lrs_moe_route_align", "lrs_norm_add",
             "lrs_qk_prep", "lrs_qkv_norm_prep", "lrs_rmsnorm", "lrs_rope_table", "lrs_rotate_unit_prep", "lrs_round_rows", "lrs_scale_add_layernorm", "lrs_scale_rows", "lrs_scale_values", "lrs_sigmoid_gate", "lrs_silu_mul", "lrs_soft_cap", "lrs_ssm", "lrs_xielu")
@@ -1499,13 +1503,20 @@ def delta_state_floats(heads: int, kv_heads: int, dim: int, vdim: int, taps: int
     return heads * rows * 16 * vdim + (taps - 1) * (2 * kv_heads * dim + heads * vdim)
 
 
+def delta_pack_floats(tokens: int, requests: int, heads: int, dim: int, vdim: int) -> int:
+    """Floats of delta_rule()'s packs for a step of that shape."""
+    return library().lrs_delta_pack_floats(tokens, requests, heads, dim, vdim)
+
+
 def delta_rule(out: torch.Tensor, proj: torch.Tensor, state: torch.Tensor, token_request: torch.Tensor, cu_seqlens: torch.Tensor,
                slot_ids: torch.Tensor, requests: int, conv_weight: torch.Tensor, kv_heads: int, heads: int, dim: int, vdim: int,
                a_log: torch.Tensor, dt_bias: torch.Tensor, norm_weight: torch.Tensor, eps: float, qkv: torch.Tensor, gates: torch.Tensor,
-               raw: torch.Tensor) -> None:
+               raw: torch.Tensor, packs: torch.Tensor | None = None, singles: int = 0) -> None:
     """One step of the gated delta rule for a ragged batch.  proj [T, >= C] holds each token's projections, columns
     q (kv_heads*dim) | k (kv_heads*dim) | v (heads*vdim) | output gate (heads*vdim) | step size (heads) | decay input
-    (heads); state [slots, floats] float32 is read and written at the rows slot_ids names; out [T, heads*vdim]."""
+    (heads); state [slots, floats] float32 is read and written at the rows slot_ids names; out [T, heads*vdim].  With packs
+    (float32 scratch of delta_pack_floats(), dim at most 128) the recurrence is worked out in chunks of 64 tokens on the matrix
+    cores, but for the first `singles` requests, which bring one token each."""
     tokens = out.shape[0]
     channels = 2 * kv_heads * dim + heads * vdim
     taps = conv_weight.shape[1]
@@ -1522,10 +1533,17 @@ def delta_rule(out: torch.Tensor, proj: torch.Tensor, state: torch.Tensor, token
     _need(qkv.dtype == torch.float32 and qkv.is_contiguous() and qkv.numel() >= tokens * channels, "delta_rule: qkv scratch too small")
     _need(gates.dtype == torch.float32 and gates.is_contiguous() and gates.numel() >= tokens * 2 * heads, "delta_rule: gates scratch too small")
     _need(raw.dtype == torch.float32 and raw.is_contiguous() and raw.numel() >= tokens * heads * vdim, "delta_rule: read-out scratch too small")
-    _launch("lrs_delta_rule", _dev(out, "out"), dtype_code(out.dtype), _dev(proj, "proj"), dtype_code(proj.dtype), _rows(proj, "proj"), tokens,
-            requests, _dev(token_request, "token_request"), _dev(cu_seqlens, "cu_seqlens"), _dev(slot_ids, "slot_ids"), _dev(state, "state"),
-            state.stride(0), _dev(conv_weight, "conv_weight"), taps, kv_heads, heads, dim, vdim, _dev(a_log, "a_log"), _dev(dt_bias, "dt_bias"),
-            _dev(norm_weight, "norm_weight"), eps, _dev(qkv, "qkv"), _dev(gates, "gates"), _dev(raw, "raw"), _stream())
+    chunked = ()
+    if packs is not None:
+        _need(0 <= singles < requests < tokens, f"delta_rule: {singles} single tokens leave no portion among {requests} requests with {tokens} tokens")
+        _need(dim <= 128, f"delta_rule: the form in chunks takes keys of up to 128 values, got {dim}")
+        _need(packs.dtype == torch.float32 and packs.is_contiguous() and packs.numel() >= delta_pack_floats(tokens, requests, heads, dim, vdim),
+              "delta_rule: the packs are too small")
+        chunked = (_dev(packs, "packs"), singles)
+    _launch("lrs_delta_rule_chunks" if chunked else "lrs_delta_rule", _dev(out, "out"), dtype_code(out.dtype), _dev(proj, "proj"), dtype_code(proj.dtype),
+            _rows(proj, "proj"), tokens, requests, _dev(token_request, "token_request"), _dev(cu_seqlens, "cu_seqlens"), _dev(slot_ids, "slot_ids"),
+            _dev(state, "state"), state.stride(0), _dev(conv_weight, "conv_weight"), taps, kv_heads, heads, dim, vdim, _dev(a_log, "a_log"),
+            _dev(dt_bias, "dt_bias"), _dev(norm_weight, "norm_weight"), eps, _dev(qkv, "qkv"), _dev(gates, "gates"), _dev(raw, "raw"), *chunked, _stream())
 
 
 def delta_rule_channels(out: torch.Tensor, proj: torch.Tensor, state: torch.Tensor, token_request: torch.Tensor, cu_seqlens: torch.Tensor,

@@ -18,6 +18,10 @@ size.  The second matrices are applied in float32: as two products of their own,
 handful of multiply-adds an output cost less than two more launches), inside the recurrence's kernels.  A rank of None is read from
 the checkpoint's tensors when they are bound.
 
+The recurrence is a scan, sequential over a request's tokens.  bfloat16 runs take another form for long portions, chunks of 64 tokens on
+the float32 matrix cores (csrc/delta_chunks.hip; float32 as the scan, in another order).  float32 runs always scan, so that how a prompt
+was cut changes no bit of them.
+
 All six input projections are one stacked product.  What a request keeps between steps is one float32 row: the
 matrices of all heads, then the convolution's last taps - 1 inputs of every channel (`StateNeed`); the cache
 manager hands out the rows, clears a row at admission and the kernels find a request's row by its slot.
@@ -126,6 +130,22 @@ class GatedDeltaRule(Part):
     def cache_need(self):
         return StateNeed((self.state_floats(),), torch.float32)
 
+    def in_chunks(self, tokens: int, requests: int, singles: int) -> bool:
+        """Whether the form in chunks is the faster one for a step of that many tokens and requests, the first `singles` with one each.
+
+        The scan is a chain, 0.25 us a token of a portion, as long as there are few portions; many fill each other's waits, down to
+        0.10 us a token and workgroup on a compute unit.  The chunks' matrices take 19 us for every 256 heads of chunks and the walk
+        3 us a chunk, 3.6 with workgroups in turn (32 heads of 128 x 128: 2,048 tokens of one request 514 us in the scan, 180 in
+        chunks; 256 tokens 66 and 40; 128 tokens 34 and 34; four requests of 512 209 and 206; sixteen of 128 204 and 310).  Only what
+        a recorded step's shape tells is asked: the longest portion is at least as long as the mean."""
+        portions, rows = requests - singles, tokens - singles
+        if self.head_dim > 128 or tokens <= requests or portions <= 0:
+            return False
+        groups = self.num_heads * -(-self.value_dim // 16) / 256          # workgroups a request and compute unit
+        chunks = rows / 64 + portions / 2
+        scan = max(0.25 * rows / portions, 0.10 * rows * groups)
+        return 12 + 19 * max(1.0, chunks * self.num_heads / 256) + 3 * max(chunks / portions, 1.2 * chunks * groups) < 0.9 * scan
+
     def forward(self, ctx, x, residual, cache, then_norm=None, accumulate: bool = True):
         if cache is None or cache.state is None:
             raise ValueError("the gated delta rule needs a state row per request")
@@ -152,8 +172,12 @@ class GatedDeltaRule(Part):
                                     decay_up, decays, gate_up, gate_in)
             linear(ctx, residual, out, self.w_o, accumulate=accumulate)
             return None
+        packs = None
+        if ctx.dtype == torch.bfloat16 and self.in_chunks(t, ctx.R, ctx.single_rows):
+            packs = ctx.scratch("delta_packs", (ops.delta_pack_floats(t, ctx.R, self.num_heads, self.head_dim, self.value_dim),), torch.float32)
         ops.delta_rule(out, proj, cache.state, ctx.token_request, ctx.cu_seqlens_q, ctx.slot_ids, ctx.R, self.conv, self.num_kv_heads,
-                       self.num_heads, self.head_dim, self.value_dim, self.a_log, self.dt_bias, self.norm, self.norm_eps, qkv, gates, raw)
+                       self.num_heads, self.head_dim, self.value_dim, self.a_log, self.dt_bias, self.norm, self.norm_eps, qkv, gates, raw,
+                       packs, ctx.single_rows if packs is not None else 0)
         linear(ctx, residual, out, self.w_o, accumulate=accumulate)
         return None
 

@@ -1,0 +1,137 @@
+"""The gated delta rule in chunks on the matrix cores against the recurrence in 64 bits, beside the scan on the same numbers."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def recurrence(qkv, gates, begun, lengths, groups, heads, d, e):
+    """Read-outs [T, heads, e] and last states [R, heads, d, e] in 64 bits."""
+    q, k, v = qkv.double().split((groups * d, groups * d, heads * e), 1)
+    of = torch.arange(heads) // (heads // groups)
+    q, k, v = q.view(-1, groups, d)[:, of], k.view(-1, groups, d)[:, of], v.view(-1, heads, e)
+    beta, decay = gates.double().view(-1, 2, heads).unbind(1)
+    outs, states, t = [], [], 0
+    for r, n in enumerate(lengths):
+        S = begun[r].clone()
+        for t in range(t, t + n):
+            S = decay[t, :, None, None] * S
+            u = beta[t, :, None] * (v[t] - torch.einsum("hde,hd->he", S, k[t]))
+            S = S + k[t, :, :, None] * u[:, None, :]
+            outs.append(torch.einsum("hde,hd->he", S, q[t]))
+        t, states = t + 1, states + [S]
+    return torch.stack(outs), torch.stack(states)
+
+
+def matrices(rows, heads, d, e):
+    """The heads' matrices [R, heads, d, e] of state rows: element (i, j) at ((i % rows) * e + j) * 16 + i / rows."""
+    per = 4 if d <= 64 else 8
+    S = rows[:, :heads * per * e * 16].view(-1, heads, per, e, 16).permute(0, 1, 4, 2, 3)
+    return S.reshape(len(rows), heads, 16 * per, e)
+
+
+@pytest.mark.parametrize("heads,groups,d,e,lengths,singles,kind", [
+    (4, 2, 24, 40, (130, 1, 64, 65), 0, "slow"), (2, 1, 128, 128, (200, 3), 0, "slow"), (6, 2, 128, 96, (64, 128, 5, 1, 63), 0, "fast"),
+    (1, 1, 100, 17, (1,) * 70 + (300,), 0, "slow"), (1, 1, 101, 17, (1,) * 70 + (300, 1, 2), 70, "fast"), (4, 4, 64, 50, (1, 1, 1, 90), 2, "zero"),
+    (3, 3, 65, 1, (256,), 0, "zero"), (2, 2, 10, 7, (17, 66), 0, "alike"), (8, 1, 128, 128, (511,), 0, "alike")])
+def test_chunks_against_the_recurrence_in_64_bits(heads, groups, d, e, lengths, singles, kind):
+    """Portions that end inside, at and behind a chunk, twice in a row over one state; keys' sizes at the edges of blocks; single
+    tokens before the portions; decays near one, far from one and of exactly zero, keys that are nearly all alike with step sizes
+    near one (every token then rewrites what the one before wrote)."""
+    from llm_runtime_study_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(len(lengths) + d)
+    tokens, requests, taps = sum(lengths), len(lengths), 4
+    channels = 2 * groups * d + heads * e
+    proj = torch.randn(tokens, channels + heads * e + 2 * heads + 3, generator=g)
+    if kind == "alike":
+        proj[:, groups * d:2 * groups * d] = 3 + 0.05 * proj[:, groups * d:2 * groups * d]
+        proj[:, channels + heads * e:channels + heads * e + heads] += 4
+    proj = proj.cuda()
+    conv = (torch.randn(channels, taps, generator=g).abs() * 0.5).cuda()
+    a_log = {"slow": -5.0, "fast": 0.5, "zero": 6.0, "alike": -4.0}[kind] + torch.randn(heads, generator=g)
+    if kind == "zero":
+        proj[::3, channels + heads * e + heads:channels + heads * e + 2 * heads] -= 12.0        # zeros among decays near one
+    a_log, dt_bias, norm = a_log.cuda(), torch.randn(heads, generator=g).cuda(), (torch.rand(e, generator=g) + 0.5).cuda()
+    floats = ops.delta_state_floats(heads, groups, d, e, taps)
+    begun = 0.3 * torch.randn(requests + 1, floats, generator=g)
+    per = 4 if d <= 64 else 8
+    padding = torch.ones(heads * per * e * 16).view(1, heads, per, e, 16)
+    padding = (torch.arange(16)[:, None] * per + torch.arange(per) < d).float().t().reshape(1, 1, per, 1, 16) * padding       # rows past d are zero
+    begun[:, :padding.numel()] *= padding.reshape(1, -1)
+    cu = torch.tensor([0] + list(np.cumsum(lengths)), dtype=torch.int32, device="cuda")
+    of = torch.repeat_interleave(torch.arange(requests), torch.tensor(lengths)).int().cuda()
+    slots = torch.randperm(requests, generator=g)
+    qkv, gates = torch.empty(tokens, channels, device="cuda"), torch.empty(tokens, 2 * heads, device="cuda")
+    raw = torch.empty(tokens, heads * e, device="cuda")
+    errors = []
+    for chunked in (False, True):
+        out, state = torch.zeros(tokens, heads * e, dtype=torch.bfloat16, device="cuda"), begun.cuda()
+        worst = [0.0, 0.0]
+        for _ in range(2):
+            before = state.cpu()
+            packs = torch.full((ops.delta_pack_floats(tokens, requests, heads, d, e),), float("nan"), device="cuda") if chunked else None
+            ops.delta_rule(out, proj, state, of, cu, slots.int().cuda(), requests, conv, groups, heads, d, e, a_log, dt_bias, norm, 1e-5, qkv, gates, raw,
+                           packs, singles if chunked else 0)
+            torch.cuda.synchronize()
+            want, S = recurrence(qkv.cpu(), gates.cpu(), matrices(before.double(), heads, d, e)[slots][:, :, :d], lengths, groups, heads, d, e)
+            got = matrices(state.cpu().double(), heads, d, e)[slots]
+            assert torch.isfinite(raw).all() and not got[:, :, d:].any()
+            worst[0] = max(worst[0], float((raw.cpu().double().view(want.shape) - want).norm() / want.norm()))
+            worst[1] = max(worst[1], float((got[:, :, :d] - S).norm() / S.norm()))
+        assert torch.equal(state[requests].cpu(), begun[requests])
+        errors.append(worst)
+    print(kind, d, e, "scan %.2e %.2e, chunks %.2e %.2e" % (*errors[0], *errors[1]))
+    # 24 bits: a unit in the last place is 6e-8; a sum of up to 128 products, the one of 64 tokens behind it and the product with the
+    # chunk's inverse add independent roundings, some ten units at the most
+    assert max(errors[1]) < 2e-6, errors
+
+
+@pytest.mark.parametrize("lengths,chunked", [((1, 1, 400), True), ((1, 300, 40), False), ((255, 256), True), ((700,), True), ((64, 64, 64), False)])
+def test_the_part_chooses_and_both_forms_agree(lengths, chunked):
+    """Steps on either side of the rule, the second on the state that the first left: the part's bfloat16 rows against its own scan.
+    Differences of the last places of 24 bits turn few roundings to 8 bits: an 8-bit unit is 2^-8 at most, in one value of some hundred."""
+    from llm_runtime_study_amd.parts import PartSpec, create
+
+    from tests.test_nobodra_gpu import bf16_values
+    from tests.test_parts_gpu import PartHarness
+
+    part = create("mixer", PartSpec("gated_delta_rule", {"hidden_size": 64, "num_heads": 4, "num_kv_heads": 2, "head_dim": 96, "value_dim": 48,
+                                                        "conv_taps": 4, "norm_eps": 1e-5}))
+    w = {name: bf16_values(*spec.shape, scale=spec.shape[-1] ** -0.5 if len(spec.shape) == 2 else 0.5, seed=i) for i, (name, spec) in enumerate(part.tensors().items())}
+    w["A_log"] = w["A_log"] - 2.0
+    part.bind({name: t.to(torch.bfloat16).cuda() for name, t in w.items()}, torch.bfloat16)
+    assert part.in_chunks(sum(lengths), len(lengths), next(i for i, n in enumerate(lengths) if n > 1)) is chunked
+    rule, rows = part.in_chunks, []
+    for choose in (rule, lambda *a: False):
+        part.in_chunks = choose
+        harness = PartHarness([part.cache_need()], torch.bfloat16, max_step_tokens=1408)
+        live = [harness.cache.admit(str(i)) for i in range(len(lengths))]
+        for turn in range(2):
+            x = bf16_values(sum(lengths), 64, seed=7 + turn).to(torch.bfloat16).cuda()
+            out = torch.zeros(sum(lengths), 64, device="cuda")
+            ctx = harness.context([(seq, [0] * n) for seq, n in zip(live, lengths)])
+            part.forward(ctx, x, out, ctx.layer_cache(0))
+        torch.cuda.synchronize()
+        rows.append(out.double().cpu())
+    part.in_chunks = rule
+    assert (rows[0] - rows[1]).norm() < 2.0 ** -8 * 0.1 * rows[1].norm()
+
+
+def test_chunks_refuse_what_they_do_not_serve():
+    from llm_runtime_study_amd.kernels import ops
+
+    def call(d, tokens, requests, singles, floats):
+        heads, e, taps = 1, 16, 2
+        channels = 2 * d + e
+        t = lambda *shape: torch.zeros(*shape, device="cuda")
+        ops.delta_rule(t(tokens, e).bfloat16(), t(tokens, channels + e + 2), t(requests, ops.delta_state_floats(heads, 1, d, e, taps)), t(tokens).int(),
+                       t(requests + 1).int(), t(requests).int(), requests, t(channels, taps), 1, heads, d, e, t(heads), t(heads), t(e), 1e-5,
+                       t(tokens, channels), t(tokens, 2), t(tokens, e), t(floats), singles)
+
+    plenty = 1 << 20
+    for case in ((129, 20, 1, 0, plenty), (64, 20, 2, 2, plenty), (64, 2, 2, 0, plenty), (64, 20, 1, 0, 64)):
+        with pytest.raises(Exception, match="delta_rule"):
+            call(*case)
