@@ -226,15 +226,46 @@ struct DecodePrep {
 // One head row, raw -> normalised and rotated, in the operand layout of the 16x16x32 products: the
 // lane holds dims c*32 + g*8 .. +8 of every 32-dim chunk c, the four lanes g = 0..3 with equal
 // lane % 16 hold one head between them.  All 64 lanes must call it together.
-// head_from_values: the same from values already in registers (a row asked for earlier, so that its trip to memory
-// ran beside other work).
+// What it needs besides the row is asked for on its own (HeadWeights, HeadTables), so that a kernel can do so before
+// anything makes it wait; head_from_values: from a row already in registers.
 template <int D>
-__device__ __forceinline__ void head_from_values(bf16x8 (&r)[D / 32], float (&x)[D / 32][8], int g,
-                                                 const void* __restrict__ weight, int weight_is_f32, float eps,
-                                                 const float* __restrict__ cosrow, const float* __restrict__ sinrow) {
+struct HeadWeights {      // the norm's weights of the lane's dims; left alone without a norm
+  floatx4 raw[D / 32][2];
+  __device__ __forceinline__ void fetch(const void* __restrict__ weight, int is_f32, int g) {
+    if (!weight) return;
+    // 16-byte loads (the host checks the alignment); bfloat16 weights need one for eight and load it twice: no branch around a load
+    const int size = is_f32 ? 4 : 2;
+#pragma unroll
+    for (int c = 0; c < D / 32; ++c) {
+      const char* from = (const char*)weight + (c * 32 + g * 8) * size;
+      raw[c][0] = *(const floatx4*)from;
+      raw[c][1] = *(const floatx4*)(from + (is_f32 ? 16 : 0));
+    }
+  }
+  __device__ __forceinline__ float value(int c, int j, int is_f32) const {
+    union { floatx4 f; bf16x8 b; } whole{raw[c][0]};
+    return is_f32 ? raw[c][j / 4][j % 4] : (float)whole.b[j];
+  }
+};
+template <int D>
+struct HeadTables {       // the rotation's cosines and sines of the lane's dims; left alone without a rotation
+  floatx4 cs[D < 64 ? 1 : D / 64][2], sn[D < 64 ? 1 : D / 64][2];
+  __device__ __forceinline__ void fetch(const float* __restrict__ cosrow, const float* __restrict__ sinrow, int g) {
+    if (!cosrow) return;
+#pragma unroll
+    for (int c = 0; c < D / 64; ++c)
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        cs[c][n] = *(const floatx4*)(cosrow + c * 32 + g * 8 + 4 * n);
+        sn[c][n] = *(const floatx4*)(sinrow + c * 32 + g * 8 + 4 * n);
+      }
+  }
+};
+template <int D>
+__device__ __forceinline__ void head_from_values(bf16x8 (&r)[D / 32], float (&x)[D / 32][8], bool normed, const HeadWeights<D>& weights,
+                                                 int weight_is_f32, float eps, bool rotated, const HeadTables<D>& tables) {
   constexpr int DS = D / 32;
-  // weights and tables come in 16-byte loads (the host checks their alignment)
-  if (weight) {
+  if (normed) {
     float ss = 0.f;
 #pragma unroll
     for (int c = 0; c < DS; ++c)
@@ -244,34 +275,20 @@ __device__ __forceinline__ void head_from_values(bf16x8 (&r)[D / 32], float (&x)
     ss += __shfl_xor(ss, 32, WAVE);
     const float inv = 1.0f / sqrtf(ss / (float)D + eps);
 #pragma unroll
-    for (int c = 0; c < DS; ++c) {
-      float w[8];
-      if (weight_is_f32) {
-        const floatx4 w0 = *(const floatx4*)((const float*)weight + c * 32 + g * 8), w1 = *(const floatx4*)((const float*)weight + c * 32 + g * 8 + 4);
+    for (int c = 0; c < DS; ++c)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) { w[j] = w0[j]; w[4 + j] = w1[j]; }
-      } else {
-        const bf16x8 wb = *(const bf16x8*)((const bf16*)weight + c * 32 + g * 8);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) w[j] = (float)wb[j];
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) x[c][j] = x[c][j] * inv * w[j];
-    }
+      for (int j = 0; j < 8; ++j) x[c][j] = x[c][j] * inv * weights.value(c, j, weight_is_f32);
   }
-  if (cosrow) {
+  if (rotated) {
 #pragma unroll
-    for (int c = 0; c < DS / 2; ++c) {
-      const floatx4 c0 = *(const floatx4*)(cosrow + c * 32 + g * 8), c1 = *(const floatx4*)(cosrow + c * 32 + g * 8 + 4);
-      const floatx4 s0 = *(const floatx4*)(sinrow + c * 32 + g * 8), s1 = *(const floatx4*)(sinrow + c * 32 + g * 8 + 4);
+    for (int c = 0; c < D / 64; ++c)
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const float cs = j < 4 ? c0[j & 3] : c1[j & 3], sn = j < 4 ? s0[j & 3] : s1[j & 3];
+        const float cs = tables.cs[c][j / 4][j % 4], sn = tables.sn[c][j / 4][j % 4];
         const float a = x[c][j], b = x[c + DS / 2][j];
         x[c][j] = a * cs - b * sn;
         x[c + DS / 2][j] = b * cs + a * sn;
       }
-    }
   }
 #pragma unroll
   for (int c = 0; c < DS; ++c)
@@ -290,7 +307,11 @@ __device__ __forceinline__ void prepare_head(bf16x8 (&r)[D / 32], const bf16* __
 #pragma unroll
     for (int j = 0; j < 8; ++j) x[c][j] = (float)raw[j];
   }
-  head_from_values<D>(r, x, g, weight, weight_is_f32, eps, cosrow, sinrow);
+  HeadWeights<D> weights;
+  HeadTables<D> tables;
+  weights.fetch(weight, weight_is_f32, g);
+  tables.fetch(cosrow, sinrow, g);
+  head_from_values<D>(r, x, weight, weights, weight_is_f32, eps, cosrow, tables);
 }
 
 // One query token per request (a decode step).  A workgroup of four waves owns one
@@ -313,7 +334,7 @@ __device__ __forceinline__ void prepare_head(bf16x8 (&r)[D / 32], const bf16* __
 template <int D, int WAVES>
 struct DecodeLds {
   float sm_m[WAVES][16], sm_l[WAVES][16];
-  float sm_o[WAVES][D][16];
+  __attribute__((aligned(16))) float sm_o[WAVES][16][D + 4];     // a head's dims side by side, heads four banks apart
   __attribute__((aligned(16))) bf16 own_k[D];
   bf16 own_v[D];
 };
@@ -342,120 +363,111 @@ __device__ __forceinline__ void attention_decode_part(
   const int per_split = (last_tile - first_tile + splits) / splits;
   const int tile_begin = first_tile + split * per_split;
   const int tile_end = tile_begin + per_split <= last_tile + 1 ? tile_begin + per_split : last_tile + 1;
-  // PREP: the wave that may have to prepare the token's new key asks for the raw key and value rows now, before
-  // anything here waits for memory: the rows are then there when their turn comes, two trips to memory later
-  // (they are the token's own, whichever workgroup turns out to walk its position)
+  // PREP: the raw rows, the norms' weights and the rotation's tables are asked for now, before anything here waits for
+  // memory: they are there when the first keys are on their way.  (The new key's and value's by every wave, since which
+  // one walks the token's position is not known yet; they are the token's own, whichever workgroup does.)
   const bf16* q_row = q + (int64_t)token * q_stride;
-  bf16x8 raw_k[DS];
+  const bool normed = PREP && prep.q_weight, rotated = PREP && prep.cosv;
+  bf16x8 qf[DS], raw_k[DS];
   bf16 raw_v[(D + WAVE - 1) / WAVE];
+  HeadWeights<D> q_weights, k_weights;
+  HeadTables<D> tables;
+#pragma unroll
+  for (int c = 0; c < DS; ++c) qf[c] = *(const bf16x8*)(q_row + (int64_t)(kvh * group + (col < group ? col : 0)) * D + c * 32 + g * 8);
   if constexpr (PREP) {
-    if (prep.kv_columns > 0 && wave == WAVES - 1) {
+    q_weights.fetch(prep.q_weight, prep.weight_is_f32, g);
+    if (rotated) tables.fetch(prep.cosv + (int64_t)token * (D / 2), prep.sinv + (int64_t)token * (D / 2), g);
+    if (prep.kv_columns > 0) {
 #pragma unroll
       for (int c = 0; c < DS; ++c) raw_k[c] = *(const bf16x8*)(q_row + (int64_t)(nq + kvh) * D + c * 32 + g * 8);
       const bf16* v_row = q_row + (int64_t)(nq + prep.kv_columns + kvh) * D;
 #pragma unroll
-      for (int n = 0; n < (D + WAVE - 1) / WAVE; ++n)
-        if (lane + n * WAVE < D) raw_v[n] = v_row[lane + n * WAVE];
+      for (int n = 0; n < (D + WAVE - 1) / WAVE; ++n) raw_v[n] = v_row[min(lane + n * WAVE, D - 1)];
+      k_weights.fetch(prep.k_weight, prep.weight_is_f32, g);
     }
   }
 
   // the block table entries of this workgroup's tiles, in LDS: the address of a key must not
-  // wait for a trip to memory of its own
-  const int first_block = tile_begin * 32 / page_size;
-  const int last_key = tile_end * 32 - 1 < pos ? tile_end * 32 - 1 : pos;
-  if (tile_begin < tile_end)
-    for (int i = tid; i <= last_key / page_size - first_block; i += THREADS) page_ids[i] = table[first_block + i];
+  // wait for a trip to memory of its own.  (A split that has no tiles left looks the last one's up.)
+  const int first_block = min(tile_begin, last_tile) * 32 / page_size;
+  const int last_key = min(max(tile_end, min(tile_begin, last_tile) + 1) * 32 - 1, pos);
+  for (int i = tid; i <= last_key / page_size - first_block; i += THREADS) page_ids[i] = table[first_block + i];
+  __syncthreads();
 
   const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
   // Every key and value fragment of a tile is requested before any is used, so a tile costs one
   // trip to memory instead of two.  Which of the tile's 32 keys a row of the two key blocks stands
   // for is chosen so that a lane ends up with the weights of eight consecutive keys, g*8 .. g*8+7:
   // block h, row 4*r + i is key 8*r + 4*h + i.  The values of those eight keys lie side by side in
-  // the (transposed) page, one 16-byte load a dim.
+  // the (transposed) page, one 16-byte load a dim.  A key or eight keys that the token does not see
+  // are read from the nearest it does see, not branched around (three branches were three trips to
+  // memory one after the other): their scores are replaced, their values zeroed (work, below).
   const int key_of_row = (col >> 2) * 8 + (col & 3);           // + 4*h
   auto fetch = [&](int tile, bf16x8 (&kf)[2][DS], bf16x8 (&vf)[DB]) {
+    const bf16* kp[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int key = tile * 32 + key_of_row + 4 * h;
-      if (key <= pos && key >= lo) {
-        const int64_t page = page_ids[key / page_size - first_block];
-        const bf16* kp = k_pages + ((page * nkv + kvh) * page_size + key % page_size) * D + g * 8;
-#pragma unroll
-        for (int c = 0; c < DS; ++c) kf[h][c] = *(const bf16x8*)(kp + c * 32);
-      } else {
-#pragma unroll
-        for (int c = 0; c < DS; ++c) kf[h][c] = zero8;
-      }
+      const int key = max(lo, min(pos, tile * 32 + key_of_row + 4 * h));
+      const int64_t page = page_ids[key / page_size - first_block];
+      kp[h] = k_pages + ((page * nkv + kvh) * page_size + key % page_size) * D + g * 8;
     }
-    const int key8 = tile * 32 + g * 8;                        // this lane's eight keys; pages hold multiples of 16
-    if (key8 <= pos && key8 + 7 >= lo) {
-      const int64_t page = page_ids[key8 / page_size - first_block];
-      const bf16* vp = v_pages + (page * nkv + kvh) * (int64_t)dv * page_size + (int64_t)col * page_size + key8 % page_size;
-      // (values narrower than keys: the blocks behind them repeat the last one, and nothing of them is written)
+    const int key8 = max(lo & ~7, min(pos & ~7, tile * 32 + g * 8));         // this lane's eight keys; pages hold multiples of 16
+    const int64_t page = page_ids[key8 / page_size - first_block];
+    const bf16* vp = v_pages + (page * nkv + kvh) * (int64_t)dv * page_size + (int64_t)col * page_size + key8 % page_size;
 #pragma unroll
-      for (int b = 0; b < DB; ++b) vf[b] = *(const bf16x8*)(vp + (int64_t)(b * 16 < dv ? b * 16 : dv - 16) * page_size);
-    } else {
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int b = 0; b < DB; ++b) vf[b] = zero8;
-    }
+      for (int c = 0; c < DS; ++c) kf[h][c] = *(const bf16x8*)(kp[h] + c * 32);
+    // (values narrower than keys: the blocks behind them repeat the last one, and nothing of them is written)
+#pragma unroll
+    for (int b = 0; b < DB; ++b) vf[b] = *(const bf16x8*)(vp + (int64_t)(b * 16 < dv ? b * 16 : dv - 16) * page_size);
   };
   // AHEAD: the wave's first tile is asked for as soon as the page ids are there, before the query (and
-  // the new key) are prepared, so that the first trip to memory runs beside that work.
+  // the new key) are prepared, so that the first trip to memory runs beside that work.  No branch around it, a wave
+  // without a tile asks for the last one: where loads may or may not be on their way, the compiler waits for all.
   bf16x8 kf_a[AHEAD ? 2 : 1][AHEAD ? DS : 1], vf_a[AHEAD ? DB : 1];
   if constexpr (AHEAD) {
-    __syncthreads();
-    if (tile_begin + wave < tile_end) fetch(tile_begin + wave, (bf16x8(&)[2][DS])kf_a, (bf16x8(&)[DB])vf_a);
+    fetch(min(tile_begin + wave, max(tile_end - 1, min(tile_begin, last_tile))), (bf16x8(&)[2][DS])kf_a, (bf16x8(&)[DB])vf_a);
   }
-  bf16x8 qf[DS];
-  if (PREP) {
-    const float* cosrow = prep.cosv ? prep.cosv + (int64_t)token * (D / 2) : nullptr;
-    const float* sinrow = prep.sinv ? prep.sinv + (int64_t)token * (D / 2) : nullptr;
-    prepare_head<D>(qf, q_row + (int64_t)(kvh * group + (col < group ? col : 0)) * D, g, prep.q_weight, prep.weight_is_f32,
-                    prep.eps, cosrow, sinrow);
-#pragma unroll
-    for (int c = 0; c < DS; ++c) qf[c] = col < group ? qf[c] : zero8;
-  } else {
+  auto prepare = [&](bf16x8 (&row)[DS], const HeadWeights<D>& weights) {
+    float x[DS][8];
 #pragma unroll
     for (int c = 0; c < DS; ++c)
-      qf[c] = col < group ? *(const bf16x8*)(q_row + (int64_t)(kvh * group + col) * D + c * 32 + g * 8) : zero8;
-  }
-  // The workgroup that walks the token's own position prepares the new key once (its last wave,
-  // which is dealt the fewest tiles), leaves it and the new value in LDS for the wave that meets
-  // the position, and writes both into the pages.
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[c][j] = (float)row[c][j];
+    head_from_values<D>(row, x, normed, weights, prep.weight_is_f32, prep.eps, rotated, tables);
+  };
+  if constexpr (PREP) prepare(qf, q_weights);
+#pragma unroll
+  for (int c = 0; c < DS; ++c) qf[c] = col < group ? qf[c] : zero8;
+  // The wave that walks the token's own position prepares the new key, passes it and the new value through LDS of its own
+  // into the fragments when it meets the position (no other wave waits for it), and writes both into the pages.
   auto &own_k = lds.own_k, &own_v = lds.own_v;
-  const bool holds_own = PREP && prep.kv_columns > 0 && tile_begin <= last_tile && last_tile < tile_end;
-  if (holds_own && wave == WAVES - 1) {
-    bf16x8 kn[DS];
-    float kx[DS][8];
-#pragma unroll
-    for (int c = 0; c < DS; ++c)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) kx[c][j] = (float)raw_k[c][j];
-    head_from_values<D>(kn, kx, g, prep.k_weight, prep.weight_is_f32, prep.eps,
-                        prep.cosv ? prep.cosv + (int64_t)token * (D / 2) : nullptr,
-                        prep.sinv ? prep.sinv + (int64_t)token * (D / 2) : nullptr);
-    // (among this workgroup's entries, since it walks the position; they are in LDS once a barrier has been passed)
-    const int64_t page = AHEAD ? page_ids[pos / page_size - first_block] : table[pos / page_size];
+  const bool holds_own = PREP && prep.kv_columns > 0 && tile_begin <= last_tile && last_tile < tile_end && (last_tile - tile_begin) % WAVES == wave;
+  if (holds_own) {
+    prepare(raw_k, k_weights);
+    const int64_t page = page_ids[pos / page_size - first_block];
     const int off = pos % page_size;
     if (col == 0) {
       bf16* kdst = k_pages + ((page * nkv + kvh) * page_size + off) * D + g * 8;
 #pragma unroll
       for (int c = 0; c < DS; ++c) {
-        *(bf16x8*)&own_k[c * 32 + g * 8] = kn[c];
-        if (page >= 0) *(bf16x8*)(kdst + c * 32) = kn[c];
+        *(bf16x8*)&own_k[c * 32 + g * 8] = raw_k[c];
+        if (page >= 0) *(bf16x8*)(kdst + c * 32) = raw_k[c];
       }
     }
 #pragma unroll
     for (int n = 0; n < (D + WAVE - 1) / WAVE; ++n) {
       const int i = lane + n * WAVE;
       if (i < D) {
-        const bf16 vn = raw_v[n];
-        own_v[i] = vn;
-        if (page >= 0) v_pages[(page * nkv + kvh) * (int64_t)D * page_size + (int64_t)i * page_size + off] = vn;
+        own_v[i] = raw_v[n];
+        if (page >= 0) v_pages[(page * nkv + kvh) * (int64_t)D * page_size + (int64_t)i * page_size + off] = raw_v[n];
       }
     }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
-  __syncthreads();
 
   floatx4 o[DB];
 #pragma unroll
@@ -468,6 +480,12 @@ __device__ __forceinline__ void attention_decode_part(
   const float rate2 = distance ? distance[biased] * (linear ? LOG2E : 1.f) : 0.f, reach = distance && !linear ? distance[nq + biased] : 0.f;
 
   auto work = [&](int tile, bf16x8 (&kf)[2][DS], bf16x8 (&vf)[DB]) {
+    if (tile * 32 < lo || tile * 32 + 31 > pos) {
+      const int key8 = tile * 32 + g * 8;
+      const bool seen = key8 <= pos && key8 + 7 >= lo;
+#pragma unroll
+      for (int b = 0; b < DB; ++b) vf[b] = seen ? vf[b] : zero8;
+    }
     if (holds_own && tile == last_tile) {
       // the token's own key and value take the place of what the pages hold at its position
       const int own = pos % 32;
@@ -532,12 +550,20 @@ __device__ __forceinline__ void attention_decode_part(
     bf16x8 (&kf_first)[2][DS] = (bf16x8(&)[2][DS])kf_a;
     bf16x8 (&vf_first)[DB] = (bf16x8(&)[DB])vf_a;
     bf16x8 kf_b[2][DS], vf_b[DB];
-    for (int tile = tile_begin + wave; tile < tile_end; tile += 2 * WAVES) {
-      if (tile + WAVES < tile_end) fetch(tile + WAVES, kf_b, vf_b);
+    // (no fetch that may or may not be made before a use, see above: the last two tiles stand by themselves)
+    int tile = tile_begin + wave;
+    for (; tile + 2 * WAVES < tile_end; tile += 2 * WAVES) {
+      fetch(tile + WAVES, kf_b, vf_b);
       work(tile, kf_first, vf_first);
-      if (tile + WAVES >= tile_end) break;
-      if (tile + 2 * WAVES < tile_end) fetch(tile + 2 * WAVES, kf_first, vf_first);
+      fetch(tile + 2 * WAVES, kf_first, vf_first);
       work(tile + WAVES, kf_b, vf_b);
+    }
+    if (tile + WAVES < tile_end) {
+      fetch(tile + WAVES, kf_b, vf_b);
+      work(tile, kf_first, vf_first);
+      work(tile + WAVES, kf_b, vf_b);
+    } else if (tile < tile_end) {
+      work(tile, kf_first, vf_first);
     }
   } else {
     for (int tile = tile_begin + wave; tile < tile_end; tile += WAVES) {
@@ -552,14 +578,13 @@ __device__ __forceinline__ void attention_decode_part(
     sm_m[wave][col] = run_max;
     sm_l[wave][col] = run_sum;
   }
+  if (col < group) {
 #pragma unroll
-  for (int b = 0; b < DB; ++b)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sm_o[wave][b * 16 + g * 4 + i][col] = o[b][i];
+    for (int b = 0; b < DB; ++b) *(floatx4*)&sm_o[wave][col][b * 16 + g * 4] = o[b];
+  }
   __syncthreads();
-  for (int e = tid; e < dv * 16; e += THREADS) {
-    const int dim = e / 16, h = e % 16;
-    if (h >= group) continue;
+  for (int e = tid; e < dv * group; e += THREADS) {
+    const int h = e / dv, dim = e % dv;
     float top = sm_m[0][h];
 #pragma unroll
     for (int w = 1; w < WAVES; ++w) top = fmaxf(top, sm_m[w][h]);
@@ -567,7 +592,7 @@ __device__ __forceinline__ void attention_decode_part(
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
       const float weight = top == -INFINITY ? 0.f : fast_exp2(sm_m[w][h] - top);
-      acc += sm_o[w][dim][h] * weight;
+      acc += sm_o[w][h][dim] * weight;
       total += sm_l[w][h] * weight;
     }
     const int head = kvh * group + h;
@@ -586,7 +611,7 @@ __device__ __forceinline__ void attention_decode_part(
 }
 
 template <int D, bool PREP, int WAVES, bool AHEAD, bool MORE>
-__global__ __launch_bounds__(WAVES * 64) void attention_decode_bf16_kernel(
+__global__ __launch_bounds__(WAVES * 64, WAVES == 4 && D == 128 ? 2 : 1) void attention_decode_bf16_kernel(
     bf16* __restrict__ out, int out_stride, float* __restrict__ part_o, float* __restrict__ part_ml,
     const bf16* __restrict__ q, int q_stride, bf16* __restrict__ k_pages,
     bf16* __restrict__ v_pages, const int* __restrict__ block_table, int table_stride,
