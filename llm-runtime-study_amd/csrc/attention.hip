@@ -338,6 +338,8 @@ struct DecodeLds {
   __attribute__((aligned(16))) bf16 own_k[D];
   bf16 own_v[D];
 };
+struct Inner { static constexpr bool value = false; };
+struct End { static constexpr bool value = true; };
 template <int D, bool PREP, int WAVES, bool AHEAD, bool MORE>
 __device__ __forceinline__ void attention_decode_part(
     DecodeLds<D, WAVES>& lds, int* page_ids, int split, int kvh, int token,
@@ -479,14 +481,17 @@ __device__ __forceinline__ void attention_decode_part(
   const bool linear = MORE && distance_form == DISTANCE_LINEAR;
   const float rate2 = distance ? distance[biased] * (linear ? LOG2E : 1.f) : 0.f, reach = distance && !linear ? distance[nq + biased] : 0.f;
 
-  auto work = [&](int tile, bf16x8 (&kf)[2][DS], bf16x8 (&vf)[DB]) {
-    if (tile * 32 < lo || tile * 32 + 31 > pos) {
+  // END: the wave's last tile, which may hold the token's own position or reach behind it (the others cannot: less code)
+  auto work = [&](auto END, int tile, bf16x8 (&kf)[2][DS], bf16x8 (&vf)[DB]) {
+    constexpr bool end = decltype(END)::value;
+    const bool cut = tile * 32 < lo || (end && tile * 32 + 31 > pos);
+    if (cut) {
       const int key8 = tile * 32 + g * 8;
       const bool seen = key8 <= pos && key8 + 7 >= lo;
 #pragma unroll
       for (int b = 0; b < DB; ++b) vf[b] = seen ? vf[b] : zero8;
     }
-    if (holds_own && tile == last_tile) {
+    if (end && holds_own && tile == last_tile) {
       // the token's own key and value take the place of what the pages hold at its position
       const int own = pos % 32;
       const int own_h = (own % 8) / 4, own_col = (own / 8) * 4 + own % 4, own_g = own / 8, own_j = own % 8;
@@ -510,18 +515,29 @@ __device__ __forceinline__ void attention_decode_part(
 #pragma unroll
       for (int c = 0; c < DS; ++c) s[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[h][c], qf[c], s[h], 0, 0, 0);
     }
-    float tile_max = -INFINITY;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int key = tile * 32 + g * 8 + h * 4 + i;
-        const bool valid = key <= pos && key >= lo;
         float scaled = softcap > 0.f ? capped(s[h][i] * scale, softcap) * LOG2E : s[h][i] * scale2;
         if (distance) scaled -= linear ? rate2 * (float)(pos - key) : distance_loss(rate2, reach, (float)(pos - key));
-        s[h][i] = valid ? scaled : -INFINITY;
-        tile_max = fmaxf(tile_max, s[h][i]);
+        s[h][i] = scaled;
       }
+    if (cut) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = tile * 32 + g * 8 + h * 4 + i;
+          s[h][i] = key <= pos && key >= lo ? s[h][i] : -INFINITY;
+        }
+    }
+    float tile_max = -INFINITY;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) tile_max = fmaxf(tile_max, s[h][i]);
     tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, WAVE));
     tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, WAVE));
     const float new_max = tile_max > run_max + RESCALE_STEP ? tile_max : run_max;   // see RESCALE_STEP
@@ -554,22 +570,22 @@ __device__ __forceinline__ void attention_decode_part(
     int tile = tile_begin + wave;
     for (; tile + 2 * WAVES < tile_end; tile += 2 * WAVES) {
       fetch(tile + WAVES, kf_b, vf_b);
-      work(tile, kf_first, vf_first);
+      work(Inner{}, tile, kf_first, vf_first);
       fetch(tile + 2 * WAVES, kf_first, vf_first);
-      work(tile + WAVES, kf_b, vf_b);
+      work(Inner{}, tile + WAVES, kf_b, vf_b);
     }
     if (tile + WAVES < tile_end) {
       fetch(tile + WAVES, kf_b, vf_b);
-      work(tile, kf_first, vf_first);
-      work(tile + WAVES, kf_b, vf_b);
+      work(Inner{}, tile, kf_first, vf_first);
+      work(End{}, tile + WAVES, kf_b, vf_b);
     } else if (tile < tile_end) {
-      work(tile, kf_first, vf_first);
+      work(End{}, tile, kf_first, vf_first);
     }
   } else {
     for (int tile = tile_begin + wave; tile < tile_end; tile += WAVES) {
       bf16x8 kf[2][DS], vf[DB];
       fetch(tile, kf, vf);
-      work(tile, kf, vf);
+      work(End{}, tile, kf, vf);
     }
   }
   run_sum += __shfl_xor(run_sum, 16, WAVE);
