@@ -329,6 +329,11 @@ __device__ __forceinline__ void prepare_head(bf16x8 (&r)[D / 32], const bf16* __
 // PREP: q holds the raw rows of the q/k/v product; the kernel prepares q itself, and the wave that
 // meets the token's own position prepares the new key, takes it and the new value in place of what
 // the pages hold there, and writes both into the pages (see DecodePrep).
+// What bounds a walk of few keys is the chain of trips to memory (position, block table, keys) and what stands between them;
+// so nothing that is asked for hides behind a branch, rows, weights and tables are asked for first, and only the wave that
+// meets the new key waits for it.  A step of the 0.6B shape (28 layers, 16 heads on 8), one request at 509 tokens: 1,166 ->
+// 1,076 us, 16 requests 1,276 -> 1,176; of the 8B shape (36 layers, 32 heads on 8) at 2,048 tokens, 8 requests 3,968 -> 3,879,
+// 64 requests 7,040 -> 6,930: two and a half to three and a half microseconds a layer.
 // MORE: values narrower than keys and a bias by distance (dv and distance are looked at); instances of their own, so that the
 // others are spared the checks.
 template <int D, int WAVES>
