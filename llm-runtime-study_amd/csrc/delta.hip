@@ -57,18 +57,57 @@ __global__ void delta_prepare_kernel(const TP* __restrict__ proj, int ld, const 
   const int c0 = is_v ? 2 * G * d + (unit - 2 * G) * dv : unit * d, n = is_v ? dv : d;
   float* out = qkv + (int64_t)t * channels + c0;
   float ss = 0.f;
-  for (int i = lane; i < n; i += WAVE) {
-    const int c = c0 + i;
-    float acc = 0.f;
-    for (int j = 0; j < taps; ++j) {
-      const int s = at - (taps - 1 - j);
-      const float x = s >= 0 ? to_float(proj[(int64_t)(start + s) * ld + c]) : kept[(int64_t)(taps - 1 + s) * channels + c];
-      acc = fmaf(conv_w[(int64_t)c * taps + j], x, acc);
-      if (keep_inside && j > 0) kept[(int64_t)(j - 1) * channels + c] = x;      // input j of this token's window is entry j - 1 of the next one's
+  constexpr int TAPS = 4;
+  if (taps <= TAPS) {
+    // Two channels a lane at a time and every input and weight of both asked for before any is used: a load behind a branch (from
+    // this step or from the request's state) is waited for by itself, eight trips to memory a wave of 128 channels.
+    for (int i = lane; i < n; i += 2 * WAVE) {
+      float x[2][TAPS], w[2][TAPS];
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const int c = c0 + min(i + p * WAVE, n - 1);
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) {
+          const int tap = min(j, taps - 1), s = at - (taps - 1 - tap);
+          const float* before = kept + (int64_t)(taps - 1 + min(s, -1)) * channels + c;
+          const TP* here = proj + (int64_t)(start + max(s, 0)) * ld + c;
+          if constexpr (sizeof(TP) == sizeof(float)) x[p][j] = *(s >= 0 ? (const float*)here : before);
+          else x[p][j] = s >= 0 ? to_float(*here) : *before;
+          w[p][j] = conv_w[(int64_t)c * taps + tap];
+        }
+      }
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        if (i + p * WAVE < n) {
+          const int c = c0 + i + p * WAVE;
+          float acc = 0.f;
+#pragma unroll
+          for (int j = 0; j < TAPS; ++j) {
+            if (j < taps) {
+              acc = fmaf(w[p][j], x[p][j], acc);
+              if (keep_inside && j > 0) kept[(int64_t)(j - 1) * channels + c] = x[p][j];      // (as below)
+            }
+          }
+          const float y = silu_f(acc);
+          out[i + p * WAVE] = y;
+          ss = fmaf(y, y, ss);
+        }
+      }
     }
-    const float y = silu_f(acc);
-    out[i] = y;
-    ss = fmaf(y, y, ss);
+  } else {
+    for (int i = lane; i < n; i += WAVE) {
+      const int c = c0 + i;
+      float acc = 0.f;
+      for (int j = 0; j < taps; ++j) {
+        const int s = at - (taps - 1 - j);
+        const float x = s >= 0 ? to_float(proj[(int64_t)(start + s) * ld + c]) : kept[(int64_t)(taps - 1 + s) * channels + c];
+        acc = fmaf(conv_w[(int64_t)c * taps + j], x, acc);
+        if (keep_inside && j > 0) kept[(int64_t)(j - 1) * channels + c] = x;      // input j of this token's window is entry j - 1 of the next one's
+      }
+      const float y = silu_f(acc);
+      out[i] = y;
+      ss = fmaf(y, y, ss);
+    }
   }
   if (!is_v) {
     ss = wave_sum(ss);
