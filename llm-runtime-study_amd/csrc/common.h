@@ -97,11 +97,14 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
 // fetches: whoever reads the LDS they fill waits for them with fetched_and_read_then_barrier (they finish in the
 // order they were asked for, and count in vmcnt).  LDS that only they write must still be named as an
 // address here, which is what tells the compiler that its contents change.
+// Between a vector instruction that writes a scalar register (a lane read into the base, or a base kept in a vector register for
+// want of scalar ones) and a memory instruction that reads it, five wait states have to pass.  The compiler does not look into
+// assembly, so they stand here, whatever the base comes from: the move's own and four.  (m0 needs one of them.)
 __device__ __forceinline__ void fetch_to_lds(const void* base, unsigned lane_offset, unsigned lds_address) {
   const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)base);
   const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)((uintptr_t)base >> 32));
   const unsigned long long uniform_base = ((unsigned long long)hi << 32) | lo;
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2"
                :: "s"(__builtin_amdgcn_readfirstlane(lds_address)), "v"(lane_offset), "s"(uniform_base) : "memory");
 }
 // The same from an address of each lane's own.
