@@ -12,6 +12,7 @@
 //   delta_walk  per (request, head, 16 columns of S): walks the chunks with its part of S in accumulators.
 // Precision: everything is float32 as in the scan, sums included; only their order differs.  Decays are multiplied as the scan does
 // and never divided, so decays of zero are no special case; the inverse holds products of contractions (1 - beta k k^T), none above one.
+// A token whose inputs are infinite or NaN spoils itself and what comes after it, as in the scan, and no token before it.
 //
 // The matrix instructions are 16 x 16 x 4: of a block of 16 rows, lane 16 g + r gives or gets row r (column r) and, of every 16 of
 // the inner size, the four 4 g .. 4 g + 3 in four instructions.  Sums come out with lane 16 g + r holding column r of the rows
@@ -210,6 +211,24 @@ __global__ __launch_bounds__(256, 2) void delta_pack_kernel(const float* __restr
       la[b * (b + 1) / 2 + c] = *(const floatx4*)(low + (b * 16 + col) * TLD + c * 16 + 4 * g);
       pa[b * (b + 1) / 2 + c] = *(const floatx4*)(seen + (b * 16 + col) * TLD + c * 16 + 4 * g);
     }
+  // A diagonal block of either triangle times a block of x, added to c.  A product multiplies the zeros above the diagonal with the
+  // rows of later tokens as well, which makes NaN of an infinity or NaN there: a column of x with one in it is then worked out value by
+  // value, below the diagonal only, so that it reaches no token before its own, as in the scan.
+  auto on_diagonal = [&](const float* triangle, int b, const floatx4& block, const floatx4& rows, floatx4 c) {
+    const float probe = fmaf(rows[0], 0.f, fmaf(rows[1], 0.f, fmaf(rows[2], 0.f, rows[3] * 0.f)));      // 0, or NaN
+    if (__builtin_amdgcn_ballot_w64(probe != 0.f) == 0) return product(block, rows, c);
+    const float* a = triangle + (b * 16 + 4 * g) * TLD + b * 16;
+#pragma unroll 1
+    for (int from = 0; from < 4; ++from)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float row = __shfl(rows[j], from * 16 + col, WAVE);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (4 * from + j <= 4 * g + i) c[i] = fmaf(a[i * TLD + 4 * from + j], row, c[i]);
+      }
+    return c;
+  };
   // a tile's queries (W' and Q') or values (V' and O'), asked for a tile ahead
   floatx4 next[4];
   auto fetch = [&](int tile) {
@@ -245,9 +264,10 @@ __global__ __launch_bounds__(256, 2) void delta_pack_kernel(const float* __restr
 #pragma unroll
       for (int c = 0; c < b; ++c) above.add(c, la[b * (b + 1) / 2 + c], x[c]);
       if (b > 0) x[b] += above.total();
-      x[b] = product(la[b * (b + 1) / 2 + b], x[b], floatx4{0.f, 0.f, 0.f, 0.f});
+      x[b] = on_diagonal(low, b, la[b * (b + 1) / 2 + b], x[b], floatx4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-      for (int c = 0; c <= b; ++c) read.add(c, pa[b * (b + 1) / 2 + c], x[c]);
+      for (int c = 0; c < b; ++c) read.add(c, pa[b * (b + 1) / 2 + c], x[c]);
+      read.part[b] = on_diagonal(seen, b, pa[b * (b + 1) / 2 + b], x[b], read.part[b]);
       y[b] += read.total();
     }
 #pragma unroll

@@ -120,6 +120,42 @@ def test_the_part_chooses_and_both_forms_agree(lengths, chunked):
     assert (rows[0] - rows[1]).norm() < 2.0 ** -8 * 0.1 * rows[1].norm()
 
 
+@pytest.mark.parametrize("what,value", [("q", "nan"), ("k", "inf"), ("k", "nan"), ("v", "inf"), ("v", "nan"), ("beta", "nan"), ("decay", "nan")])
+@pytest.mark.parametrize("token", [0, 5, 37, 63, 79])
+@pytest.mark.parametrize("d", [64, 128])
+def test_a_token_that_is_not_finite_spoils_no_token_before_it(what, value, token, d):
+    """An infinity or NaN in one column of one token: the same read-outs are finite as in the scan (those of every token before it, of
+    the other request, of the other columns if it is a value's, of later tokens if it is a query's) and agree with it."""
+    from llm_runtime_study_amd.kernels import ops
+
+    heads, groups, e, taps, lengths = 2, 2, 24, 4, (100, 70)
+    g = torch.Generator().manual_seed(token + d)
+    tokens, requests, channels = sum(lengths), len(lengths), 2 * groups * d + heads * e
+    proj = torch.randn(tokens, channels + heads * e + 2 * heads, generator=g)
+    proj[token, {"q": 3, "k": groups * d + 3, "v": 2 * groups * d + 3, "beta": channels + heads * e, "decay": channels + heads * e + heads}[what]] = float(value)
+    conv = torch.randn(channels, taps, generator=g).abs() * 0.5 + 0.01
+    a_log, dt_bias, norm = torch.randn(heads, generator=g) - 3, torch.randn(heads, generator=g), torch.rand(e, generator=g) + 0.5
+    proj, conv, a_log, dt_bias, norm = (t.cuda() for t in (proj, conv, a_log, dt_bias, norm))
+    cu = torch.tensor([0] + list(np.cumsum(lengths)), dtype=torch.int32, device="cuda")
+    of = torch.repeat_interleave(torch.arange(requests), torch.tensor(lengths)).int().cuda()
+    raws, states = [], []
+    for chunked in (False, True):
+        state = torch.zeros(requests, ops.delta_state_floats(heads, groups, d, e, taps), device="cuda")
+        raw, out = torch.empty(tokens, heads * e, device="cuda"), torch.empty(tokens, heads * e, dtype=torch.bfloat16, device="cuda")
+        packs = torch.empty(ops.delta_pack_floats(tokens, requests, heads, d, e), device="cuda") if chunked else None
+        ops.delta_rule(out, proj, state, of, cu, torch.arange(requests, dtype=torch.int32, device="cuda"), requests, conv, groups, heads, d, e, a_log, dt_bias,
+                       norm, 1e-5, torch.empty(tokens, channels, device="cuda"), torch.empty(tokens, 2 * heads, device="cuda"), raw, packs)
+        torch.cuda.synchronize()
+        raws.append(raw.cpu().double())
+        states.append(matrices(state.cpu().double(), heads, d, e))
+    scan, chunks = raws
+    assert torch.isfinite(scan[:token]).all() and torch.isfinite(scan[lengths[0]:]).all() and not torch.isfinite(scan[token]).all()
+    assert torch.equal(torch.isfinite(chunks), torch.isfinite(scan)) and torch.equal(torch.isfinite(states[1]), torch.isfinite(states[0]))
+    for got, want in ((chunks, scan), (states[1], states[0])):
+        kept = torch.isfinite(want)
+        assert (got[kept] - want[kept]).norm() <= 4e-6 * want[kept].norm()       # twice what either may be from 64 bits, above
+
+
 def test_chunks_refuse_what_they_do_not_serve():
     from llm_runtime_study_amd.kernels import ops
 
