@@ -1395,6 +1395,10 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void attention_prefill_bf16_
 // 215 instructions that also waited for the fetches they had just made, for scalar loads of the block table and for every value
 // fragment in turn took 1.40 us with two workgroups a unit behind contexts in memory, these 1.11 (16 heads on 8, 2,048 tokens after
 // 14,336: 360 -> 284 us a layer; 32 on 8 691 -> 486; 32,768 tokens 8.95 -> 7.64 ms, 1.15 PFLOP/s; 2,048 after 2,048 152 -> 115).
+// A walk of a few tiles (short prompts, windows) is bound by what stands before its first turn.  us with the longer turns of that
+// time / with these and a chain of waits before them / with all asked for at once and nothing spilled: 16 heads on 8, 2,048 tokens,
+// window of 128 21.4 / 29.1 / 21.9, linear bias 26.1 / 42.9 / 26.7; 100 tokens 8.5 / 9.3 / 8.6; 32 on 8, linear bias, 32 tokens 7.1 /
+// 8.9 / 7.3, 2,048 in a window of 512 51 / 61 / 47; plain, 2,048 tokens 63.7 / 62.2 / 57.6, 2,048 after 2,048 165 / 124 / 116.
 // SCORES: what happens to the scores before the softmax, by instances of their own so that the others keep their registers:
 // nothing, a cap (softcap * tanh(score / softcap) of the scaled scores), a bias by distance (in the form with a logarithm, or the
 // linear one, which without a cap is what the products are added to and costs nothing), or the cap and then the bias.
@@ -1437,9 +1441,8 @@ __device__ __forceinline__ void attention_prefill_d128_part(
   auto& key_tiles = lds.key_tiles;
   auto& value_tiles = lds.value_tiles;
   const int tid = threadIdx.x;
-  const int lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-  const int col = lane & 15, g = lane >> 4;
-  const int key_chunk = ((g & 1) << 1) | (g >> 1);                 // m: the eight keys this lane group holds weights of
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  int lane = tid % WAVE;                                           // (set anew in every pass over the keys: see there)
   const int group = nq / nkv;
   const int n_walks = PAIRS ? (n_blocks + 1) / 2 : n_blocks;       // PAIRS: two neighbouring groups of one request walk together
   const int work = block % (n_walks * nkv), split = block / (n_walks * nkv);
@@ -1472,12 +1475,6 @@ __device__ __forceinline__ void attention_prefill_d128_part(
   // (or first slot) never changes; the run's page is looked up once a wave.
   const int pages16 = page_size / 16;                            // runs of 16 keys in a page
   const unsigned magic = pages16 > 1 ? 0xFFFFFFFFu / (unsigned)pages16 + 1u : 0u;   // run / pages16 = umulhi(run, magic)
-  // lane l of a key block brings row l / 16 (h = row / 2, k = row % 2), piece l % 16: key 8 k + 4 h + wave of its run
-  const unsigned key_offset = (unsigned)(((((lane >> 4) & 1) * 8 + (lane >> 5) * 4 + wave) * D + (lane & 15) * 8) * 2);
-  // lane l of a value block brings dimension 32 wave + l / 2, keys 8 (l % 2) .. + 7 of the run
-  // (values narrower than keys: the dims behind them repeat the last one)
-  const int value_dim = wave * 32 + (lane >> 1) < dv ? wave * 32 + (lane >> 1) : dv - 1;
-  const unsigned value_offset = (unsigned)(((value_dim * page_size) + (lane & 1) * 8) * 2);
   const unsigned keys_address = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)key_tiles;
   const unsigned values_address = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)value_tiles;
   // Where a run of 16 keys lies in memory: a page from the block table and a place in it.  A run no query sees is masked: any page
@@ -1486,51 +1483,19 @@ __device__ __forceinline__ void attention_prefill_d128_part(
   const uint64_t value_page_bytes = (uint64_t)nkv * page_size * dv * 2;     // ... and of values
   const char* const k_head = (const char*)(k_pages + (int64_t)kvh * page_size * D);
   const char* const v_head = (const char*)(v_pages + (int64_t)kvh * page_size * dv);
-  auto locate = [&](int run, uint64_t& keys, uint64_t& values) {
+  struct Run {
+    int number, entry;
+  };
+  auto run_in_reach = [&](int run) {
     run = run < first_run ? first_run : run > last_run ? last_run : run;
-    const int entry = pages16 > 1 ? (int)__umulhi((unsigned)run, magic) : run;
-    const uint64_t page = (uint64_t)(unsigned)table[entry];
-    const unsigned in_page = (unsigned)(run - entry * pages16) * 16u;
-    keys = (uint64_t)(uintptr_t)k_head + page * page_bytes + in_page * (unsigned)(D * 2);
-    values = (uint64_t)(uintptr_t)v_head + page * value_page_bytes + in_page * 2u;
+    return Run{run, pages16 > 1 ? (int)__umulhi((unsigned)run, magic) : run};
   };
-  // A wave's lanes look up a block of 64 runs at a time and leave the addresses in LDS, from where every turn takes its four: the
-  // same work done by every wave in every turn with scalar instructions (loads of the block table among them, which LDS reads cannot
-  // be waited for apart from) was 60 of a turn's 215 instructions.
+  auto locate = [&](const Run& run, int page, uint64_t& keys, uint64_t& values) {
+    const unsigned in_page = (unsigned)(run.number - run.entry * pages16) * 16u;
+    keys = (uint64_t)(uintptr_t)k_head + (uint64_t)(unsigned)page * page_bytes + in_page * (unsigned)(D * 2);
+    values = (uint64_t)(uintptr_t)v_head + (uint64_t)(unsigned)page * value_page_bytes + in_page * 2u;
+  };
   constexpr int BLOCK_RUNS = PrefillLds::BLOCK_RUNS, RUNS = PrefillLds::RUNS;
-  auto locate_block = [&](int which) {
-    uint64_t keys, values;
-    locate(first_tile * 2 + which * BLOCK_RUNS + lane, keys, values);
-    const int at = (which & 1) * BLOCK_RUNS + lane;
-    lds.key_runs[at] = keys;
-    lds.value_runs[(at + 2) & (RUNS - 1)] = values;
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");             // there before this wave comes to the next barrier
-  };
-  struct Pair {
-    uint64_t run[2];
-  };
-  auto runs_at = [&](const uint64_t (&ring)[RUNS], int place) {
-    typedef uint64_t pair __attribute__((ext_vector_type(2)));
-    const pair at = *(const pair*)&ring[place];
-    return Pair{{at[0], at[1]}};
-  };
-  // (a kv group of five to eight heads brings as many waves, so that one walk over the keys serves them all;
-  // the first four waves bring the tiles in)
-  auto fetch_keys = [&](const Pair& from, int stage) {      // two fetches a wave
-    if (MANY_WAVES && wave >= 4) return;
-#pragma unroll
-    for (int half = 0; half < 2; ++half)
-      fetch_lanes_to_lds(from.run[half] + key_offset, keys_address + (unsigned)(stage * KBYTES + (wave + 4 * half) * KBLOCK));
-  };
-  auto fetch_values = [&](const Pair& from, int stage) {    // two fetches a wave
-    if (MANY_WAVES && wave >= 4) return;
-#pragma unroll
-    for (int half = 0; half < 2; ++half)
-      fetch_lanes_to_lds(from.run[half] + value_offset, values_address + (unsigned)(stage * VSTAGE + half * VHALF + wave * 1024));
-  };
-  // where this lane's fragments lie in a stage
-  const int key_fragment = (col & 7) * KBLOCK + (col >> 3) * 256 + g * 16;              // + h * 512 + c * 64
-  const int value_fragment = (g & 1) * VHALF + col * 32 + (g >> 1) * 16;                // + e * 512
 
   // kv groups of more than four heads take several passes over the keys
   const int waves = MANY_WAVES ? blockDim.x / WAVE : 4;
@@ -1541,51 +1506,124 @@ __device__ __forceinline__ void attention_prefill_d128_part(
   for (int head0 = kvh * group; head0 < (kvh + 1) * group; head0 += waves) {
     const int head = head0 + my_wave;
     const bool active = head < (kvh + 1) * group;
-    // the first tiles are asked for before the queries, whose way to the registers is as long
+    // What follows from the lane is worked out in every pass.  Left alone the compiler takes all of it, addresses of loads before and
+    // behind the walk too, for values to keep through all passes, and has no registers for them: 14 to 63 were spilled, and each one's
+    // way back waits for every fetch asked for before it.
+    int begin = first_tile;
+    asm volatile("" : "+v"(lane), "+s"(begin));
+    const int col = lane & 15, g = lane >> 4;
+    const int key_chunk = ((g & 1) << 1) | (g >> 1);           // m: the eight keys this lane group holds weights of
+    // lane l of a key block brings row l / 16 (h = row / 2, k = row % 2), piece l % 16: key 8 k + 4 h + wave of its run
+    const unsigned key_offset = (unsigned)(((((lane >> 4) & 1) * 8 + (lane >> 5) * 4 + wave) * D + (lane & 15) * 8) * 2);
+    // lane l of a value block brings dimension 32 wave + l / 2, keys 8 (l % 2) .. + 7 of the run
+    // (values narrower than keys: the dims behind them repeat the last one)
+    const int value_dim = wave * 32 + (lane >> 1) < dv ? wave * 32 + (lane >> 1) : dv - 1;
+    const unsigned value_offset = (unsigned)(((value_dim * page_size) + (lane & 1) * 8) * 2);
+    // where this lane's fragments lie in a stage
+    const int key_fragment = (col & 7) * KBLOCK + (col >> 3) * 256 + g * 16;              // + h * 512 + c * 64
+    const int value_fragment = (g & 1) * VHALF + col * 32 + (g >> 1) * 16;                // + e * 512
+
+    // A wave's lanes look up a block of 64 runs at a time and leave the addresses in LDS, from where every turn takes its four: the
+    // same work done by every wave in every turn with scalar instructions (loads of the block table among them, which LDS reads cannot
+    // be waited for apart from) was 60 of a turn's 215 instructions.
+    auto leave_block = [&](int which, const Run& run, int page) {
+      uint64_t keys, values;
+      locate(run, page, keys, values);
+      const int at = (which & 1) * BLOCK_RUNS + lane;
+      lds.key_runs[at] = keys;
+      lds.value_runs[(at + 2) & (RUNS - 1)] = values;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");             // there before this wave comes to the next barrier
+    };
+    struct Pair {
+      uint64_t run[2];
+    };
+    auto runs_at = [&](const uint64_t (&ring)[RUNS], int place) {
+      typedef uint64_t pair __attribute__((ext_vector_type(2)));
+      const pair at = *(const pair*)&ring[place];
+      return Pair{{at[0], at[1]}};
+    };
+    // (a kv group of five to eight heads brings as many waves, so that one walk over the keys serves them all;
+    // the first four waves bring the tiles in)
+    auto fetch_keys = [&](const Pair& from, int stage) {      // two fetches a wave
+      if (MANY_WAVES && wave >= 4) return;
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+        fetch_lanes_to_lds(from.run[half] + key_offset, keys_address + (unsigned)(stage * KBYTES + (wave + 4 * half) * KBLOCK));
+    };
+    auto fetch_values = [&](const Pair& from, int stage) {    // two fetches a wave
+      if (MANY_WAVES && wave >= 4) return;
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+        fetch_lanes_to_lds(from.run[half] + value_offset, values_address + (unsigned)(stage * VSTAGE + half * VHALF + wave * 1024));
+    };
+    // What a walk begins with is asked for before anything is waited for: the pages of the first two blocks of runs, positions and
+    // raw rows, and behind them the first tiles, whose addresses come by scalar loads.  A wait in between is a trip to memory of its
+    // own, since a wave's loads come back in the order they were asked for, and short walks are little else.
     __syncthreads();                                           // the stages of an earlier pass are done with
+    bf16x8 qf[QB][DS];
+    int pos[QB], lo[QB];
+    bool live[QB];
+    const Run my_run = run_in_reach(begin * 2 + (wave & 1) * BLOCK_RUNS + lane);
+    const int my_page = table[my_run.entry];
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+      live[b] = active && query0 + b * 16 + col < count;
+      const int token = token0 + (live[b] ? query0 + b * 16 + col : 0);      // (a dead column takes its group's first token and drops the result)
+      pos[b] = positions[token];
+      const bf16* row = q + (int64_t)token * q_stride + (int64_t)(active ? head : head0) * D + g * 8;
+#pragma unroll
+      for (int c = 0; c < DS; ++c) qf[b][c] = *(const bf16x8*)(row + c * 32);
+    }
     int pending = 0;
     if (first_tile <= last_tile) {
-      Pair keys[3], values[2];
+      const char *keys[3][2], *values[3][2];
 #pragma unroll
       for (int n = 0; n < 3; ++n)
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
-          uint64_t at;
-          locate((first_tile + n) * 2 + half, keys[n].run[half], n < 2 ? values[n].run[half] : at);
+          const Run run = run_in_reach((begin + n) * 2 + half);
+          uint64_t key_at, value_at;
+          locate(run, table[run.entry], key_at, value_at);
+          keys[n][half] = (const char*)(uintptr_t)key_at, values[n][half] = (const char*)(uintptr_t)value_at;
         }
-      fetch_keys(keys[0], 0);
-      fetch_values(values[0], 0);
-      if (first_tile + 1 <= last_tile) fetch_keys(keys[1], 1);
-      if (first_tile + 2 <= last_tile) fetch_keys(keys[2], 2), pending += 2;
-      if (first_tile + 1 <= last_tile) fetch_values(values[1], 1), pending += 2;
-      if (wave < 2 && first_tile + 2 <= last_tile) locate_block(wave);
+      auto first_keys = [&](int n) {
+        if (MANY_WAVES && wave >= 4) return;
+#pragma unroll
+        for (int half = 0; half < 2; ++half) fetch_to_lds(keys[n][half], key_offset, keys_address + (unsigned)(n * KBYTES + (wave + 4 * half) * KBLOCK));
+      };
+      auto first_values = [&](int n) {
+        if (MANY_WAVES && wave >= 4) return;
+#pragma unroll
+        for (int half = 0; half < 2; ++half) fetch_to_lds(values[n][half], value_offset, values_address + (unsigned)(n * VSTAGE + half * VHALF + wave * 1024));
+      };
+      first_keys(0);
+      first_values(0);
+      if (first_tile + 1 <= last_tile) first_keys(1);
+      if (first_tile + 2 <= last_tile) first_keys(2), pending += 2;
+      if (first_tile + 1 <= last_tile) first_values(1), pending += 2;
+      if (wave < 2 && first_tile + 2 <= last_tile) leave_block(wave, my_run, my_page);
     }
-    bf16x8 qf[QB][DS];
     floatx4 o[QB][DB];
     float run_max[QB], run_sum[QB];
-    int pos[QB], lo[QB];
-    bool live[QB];
 #pragma unroll
     for (int b = 0; b < QB; ++b) {
-      live[b] = active && query0 + b * 16 + col < count;
-      const int token = token0 + (live[b] ? query0 + b * 16 + col : 0);
-      pos[b] = live[b] ? positions[token] : -1;                // a dead column sees no key
+      pos[b] = live[b] ? pos[b] : -1;                          // a dead column sees no key
       lo[b] = first_seen(pos[b], window);
       run_max[b] = -INFINITY;
       run_sum[b] = 0.f;
+      // q holds the raw rows of the q/k/v product: the head is normalised and rotated here, in the registers it stays in
       if (prepare_q) {
-        // q holds the raw rows of the q/k/v product: the head is normalised and rotated here, on its way into
-        // the registers it stays in (a dead column prepares its group's first token and drops the result)
-        prepare_head<D>(qf[b], q + (int64_t)token * q_stride + (int64_t)(active ? head : head0) * D, g, prep.q_weight, prep.weight_is_f32,
-                        prep.eps, prep.cosv ? prep.cosv + (int64_t)token * (D / 2) : nullptr,
-                        prep.sinv ? prep.sinv + (int64_t)token * (D / 2) : nullptr);
-#pragma unroll
-        for (int c = 0; c < DS; ++c) qf[b][c] = live[b] ? qf[b][c] : zero8;
-      } else {
+        float x[DS][8];
 #pragma unroll
         for (int c = 0; c < DS; ++c)
-          qf[b][c] = live[b] ? *(const bf16x8*)(q + (int64_t)token * q_stride + (int64_t)head * D + c * 32 + g * 8) : zero8;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) x[c][j] = (float)qf[b][c][j];
+        const int token = token0 + (live[b] ? query0 + b * 16 + col : 0);
+        head_from_values<D>(qf[b], x, g, prep.q_weight, prep.weight_is_f32, prep.eps, prep.cosv ? prep.cosv + (int64_t)token * (D / 2) : nullptr,
+                            prep.sinv ? prep.sinv + (int64_t)token * (D / 2) : nullptr);
       }
+#pragma unroll
+      for (int c = 0; c < DS; ++c) qf[b][c] = live[b] ? qf[b][c] : zero8;
 #pragma unroll
       for (int e = 0; e < DB; ++e) o[b][e] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
@@ -1836,7 +1874,7 @@ __device__ __forceinline__ void attention_prefill_d128_part(
     // what it asked for itself is still on its way: the keys of t + 2 and the values of t + 1 are then in LDS.
     floatx4 sa[QB][2], sb[QB][2];
     bf16x8 pf[QB];
-    Pair keys_ahead, values_ahead;                             // at the top of a turn: where the keys of tile + 3 and the values of tile + 2 lie
+    Pair keys_ahead, values_ahead;                             // where the keys of tile + 3 and the values of tile + 2 lie: known at the top of a turn
     if (first_tile <= last_tile) {
       if (pending == 4) fetched_and_read_then_barrier<4>();
       else if (pending == 2) fetched_and_read_then_barrier<2>();
@@ -1857,16 +1895,23 @@ __device__ __forceinline__ void attention_prefill_d128_part(
       int pending = 0;
       if (tile == locate_at) {
         // the block of runs behind the one that the walk is in takes the place of the one before it, which the walk left two turns ago
-        if (wave == 0) locate_block((tile - first_tile) / (BLOCK_RUNS / 2) + 1);
+        if (wave == 0) {
+          const int which = (tile - first_tile) / (BLOCK_RUNS / 2) + 1;
+          const Run run = run_in_reach(first_tile * 2 + which * BLOCK_RUNS + lane);
+          leave_block(which, run, table[run.entry]);
+        }
         locate_at += BLOCK_RUNS / 2;
         if (locate_at > last_locate) locate_at = -1;
       }
       if (EVERY || tile + 3 <= last_tile) fetch_keys(keys_ahead, stage), pending += 2;
       if (EVERY || tile + 2 <= last_tile) fetch_values(values_ahead, stage == 0 ? STAGES - 1 : stage - 1), pending += 2;
-      place = (place + 2) & (RUNS - 1);
-      keys_ahead = runs_at(lds.key_runs, place);                // wanted a turn from now
-      values_ahead = runs_at(lds.value_runs, place);
       return pending;
+    };
+    // the addresses for the next turn's fetches, read late in a turn, where registers are free
+    auto look_ahead = [&]() {
+      place = (place + 2) & (RUNS - 1);
+      keys_ahead = runs_at(lds.key_runs, place);
+      values_ahead = runs_at(lds.value_runs, place);
     };
     auto turn_over = [&](int pending) {
       if (pending == 4) fetched_and_read_then_barrier<4>();
@@ -1884,7 +1929,11 @@ __device__ __forceinline__ void attention_prefill_d128_part(
     // so that the others keep their registers) only brings its share of the tiles in and keeps the workgroup's
     // barriers: one a tile, as the others.
     if (IDLE_WAVES && !active) {
-      while (tile <= last_tile) turn_over(ask_ahead(std::false_type{}));
+      while (tile <= last_tile) {
+        const int on_their_way = ask_ahead(std::false_type{});
+        look_ahead();
+        turn_over(on_their_way);
+      }
       continue;
     }
     for (;;) {
@@ -1899,6 +1948,7 @@ __device__ __forceinline__ void attention_prefill_d128_part(
           asked = true;
           continue;
         }
+        look_ahead();
         values_read_ahead(stage, pf, vf);
         turn_over(4);
 #pragma unroll
@@ -1916,6 +1966,7 @@ __device__ __forceinline__ void attention_prefill_d128_part(
       if (tile < last_tile) scores(tile + 1, stage == STAGES - 1 ? 0 : stage + 1, sb);
       if (tile >= whole_begin && tile < whole_end) weights_with_maximum(tile, sa, std::false_type{}, pf);
       else weights_with_maximum(tile, sa, std::true_type{}, pf);
+      look_ahead();
       values(stage, pf);
       turn_over(on_their_way);
 #pragma unroll
@@ -1951,7 +2002,7 @@ __device__ __forceinline__ void attention_prefill_d128_part(
 }
 
 template <int QB, bool MANY_WAVES, int SPREAD, int SCORES>
-__global__ __launch_bounds__(MANY_WAVES ? 512 : 256, MANY_WAVES ? 1 : QB == 1 ? 3 : 2) void attention_prefill_d128_bf16_kernel(
+__global__ __launch_bounds__(MANY_WAVES ? 512 : 256, MANY_WAVES ? 1 : QB == 1 && (SCORES & SCORES_LINEAR) ? 3 : 2) void attention_prefill_d128_bf16_kernel(
     bf16* __restrict__ out, int out_stride, const bf16* __restrict__ q, int q_stride,
     const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
     const int* __restrict__ block_table, int table_stride, const int* __restrict__ token_request,
