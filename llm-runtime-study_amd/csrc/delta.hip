@@ -607,7 +607,8 @@ LRS_API int lrs_delta_rule(void* out, int out_dtype, const void* proj, int proj_
 }
 
 // The same with the form in chunks for the requests behind the first `singles`, which bring one token each (their tokens are the
-// step's first): packs holds lrs_delta_pack_floats(tokens, requests, H, d, dv) floats, d is at most 128.
+// step's first): packs holds lrs_delta_pack_floats(tokens, requests - singles, H, d, dv) floats, d is at
+// most 128.
 LRS_API int lrs_delta_rule_chunks(void* out, int out_dtype, const void* proj, int proj_dtype, int ld, int tokens, int requests,
                                   const int* token_request, const int* cu, const int* slot_ids, float* state, int64_t state_stride,
                                   const float* conv_w, int taps, int G, int H, int d, int dv, const float* a_log,

@@ -421,7 +421,7 @@ __global__ __launch_bounds__(256, 1) void delta_walk_kernel(const float* __restr
 
 }  // namespace
 
-// Floats of the packs that a step of so many tokens and requests needs.
+// Floats of the packs that a step of so many tokens needs, `requests` of whose requests take the form in chunks.
 LRS_API int64_t lrs_delta_pack_floats(int tokens, int requests, int H, int d, int dv) {
   return (int64_t)(tokens / L + requests + 1) * H * pack_floats(SPLIT * lrs_delta_state_rows(d), (dv + 15) / 16);
 }

@@ -1504,7 +1504,7 @@ def delta_state_floats(heads: int, kv_heads: int, dim: int, vdim: int, taps: int
 
 
 def delta_pack_floats(tokens: int, requests: int, heads: int, dim: int, vdim: int) -> int:
-    """Floats of delta_rule()'s packs for a step of that shape."""
+    """Floats of delta_rule()'s packs for a step of so many tokens; requests: those behind the `singles`."""
     return library().lrs_delta_pack_floats(tokens, requests, heads, dim, vdim)
 
 
@@ -1537,7 +1537,7 @@ def delta_rule(out: torch.Tensor, proj: torch.Tensor, state: torch.Tensor, token
     if packs is not None:
         _need(0 <= singles < requests < tokens, f"delta_rule: {singles} single tokens leave no portion among {requests} requests with {tokens} tokens")
         _need(dim <= 128, f"delta_rule: the form in chunks takes keys of up to 128 values, got {dim}")
-        _need(packs.dtype == torch.float32 and packs.is_contiguous() and packs.numel() >= delta_pack_floats(tokens, requests, heads, dim, vdim),
+        _need(packs.dtype == torch.float32 and packs.is_contiguous() and packs.numel() >= delta_pack_floats(tokens, requests - singles, heads, dim, vdim),
               "delta_rule: the packs are too small")
         chunked = (_dev(packs, "packs"), singles)
     _launch("lrs_delta_rule_chunks" if chunked else "lrs_delta_rule", _dev(out, "out"), dtype_code(out.dtype), _dev(proj, "proj"), dtype_code(proj.dtype),

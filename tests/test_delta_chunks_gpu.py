@@ -89,6 +89,62 @@ def test_chunks_against_the_recurrence_in_64_bits(heads, groups, d, e, lengths, 
     assert max(errors[1]) < 2e-6, errors
 
 
+def test_packs_are_as_large_as_the_walked_requests_need():
+    """Single tokens before a portion take no room in the packs: the part's buffer is the portion's, and a buffer of just that size,
+    with a guard behind it, gives the read-outs that a larger one gives.  Where there is no memory for it the scan runs."""
+    from types import SimpleNamespace
+
+    from llm_runtime_study_amd.kernels import ops
+    from llm_runtime_study_amd.parts import PartSpec, create
+
+    heads, d, e, taps, portion = 4, 64, 32, 4, 700
+    part = create("mixer", PartSpec("gated_delta_rule", {"hidden_size": 64, "num_heads": heads, "num_kv_heads": heads, "head_dim": d, "value_dim": e, "conv_taps": taps, "norm_eps": 1e-5}))
+    g = torch.Generator().manual_seed(5)
+    part.bind({name: (torch.randn(spec.shape, generator=g) * 0.1).to(torch.bfloat16).cuda() for name, spec in part.tensors().items()}, torch.bfloat16)
+    sizes = []
+    for singles, room in ((0, True), (64, True), (0, False)):
+        tokens, requests, sized = singles + portion, singles + 1, {}
+
+        def scratch(name, shape, dtype):
+            if name == "delta_packs" and not room:
+                raise torch.OutOfMemoryError("no room")
+            sized[name] = torch.zeros(shape, dtype=dtype, device="cuda")
+            return sized[name]
+
+        lengths = torch.tensor([1] * singles + [portion])
+        cu = torch.cat((torch.zeros(1), lengths.cumsum(0))).int().cuda()
+        ctx = SimpleNamespace(dtype=torch.bfloat16, R=requests, single_rows=singles, scratch=scratch, kernels=ops.KernelChoice(library=False), cu_seqlens_q=cu,
+                              token_request=torch.repeat_interleave(torch.arange(requests), lengths).int().cuda(), slot_ids=torch.arange(requests).int().cuda())
+        cache = SimpleNamespace(state=torch.zeros(requests, part.state_floats(), device="cuda"))
+        assert part.in_chunks(tokens, requests, singles)
+        out = torch.zeros(tokens, 64, device="cuda")
+        part.forward(ctx, torch.randn(tokens, 64, generator=g).bfloat16().cuda(), out, cache)
+        torch.cuda.synchronize()
+        assert torch.isfinite(out).all() and out.any()
+        if room:
+            sizes.append(sized["delta_packs"].numel())
+    assert sizes[1] - sizes[0] <= -(-64 // 64) * ops.delta_pack_floats(0, 0, heads, d, e)      # 64 tokens more are a chunk more at most
+
+    singles = 64
+    tokens, requests = singles + portion, singles + 1
+    lengths = torch.tensor([1] * singles + [portion])
+    cu = torch.cat((torch.zeros(1), lengths.cumsum(0))).int().cuda()
+    of = torch.repeat_interleave(torch.arange(requests), lengths).int().cuda()
+    channels, raws = 2 * heads * d + heads * e, []
+    args = (cu, torch.arange(requests).int().cuda(), requests, torch.rand(channels, taps, generator=g).cuda(), heads, heads, d, e, torch.zeros(heads).cuda() - 2,
+            torch.zeros(heads).cuda(), torch.ones(e).cuda(), 1e-5)
+    proj = torch.randn(tokens, channels + heads * e + 2 * heads, generator=g).cuda()
+    for floats, guard in ((ops.delta_pack_floats(tokens, 1, heads, d, e), 4096), (ops.delta_pack_floats(tokens, requests, heads, d, e), 0)):
+        room, raw = torch.full((floats + guard,), -7.0, device="cuda"), torch.empty(tokens, heads * e, device="cuda")
+        state = torch.zeros(requests, ops.delta_state_floats(heads, heads, d, e, taps), device="cuda")
+        ops.delta_rule(torch.empty(tokens, heads * e, dtype=torch.bfloat16, device="cuda"), proj, state, of, *args,
+                       torch.empty(tokens, channels, device="cuda"), torch.empty(tokens, 2 * heads, device="cuda"), raw, room[:floats], singles)
+        torch.cuda.synchronize()
+        assert (room[floats:] == -7.0).all()
+        raws.append(raw.cpu())
+    assert torch.equal(raws[0], raws[1])
+
+
 @pytest.mark.parametrize("lengths,chunked", [((1, 1, 400), True), ((1, 300, 40), False), ((255, 256), True), ((700,), True), ((64, 64, 64), False)])
 def test_the_part_chooses_and_both_forms_agree(lengths, chunked):
     """Steps on either side of the rule, the second on the state that the first left: the part's bfloat16 rows against its own scan.
