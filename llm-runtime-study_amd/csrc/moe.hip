@@ -597,7 +597,7 @@ __device__ __forceinline__ void store_expert_tile(floatx4 (&acc)[IT][JT], TO* __
   }
 }
 
-// The grouped product for large steps whose K is 32 more than a multiple of 64 (the kernel below takes multiples), the way this
+// The grouped product for large steps whose K is 32 more than a multiple of 64 (the kernel below takes multiples) or short, the way this
 // package's many-rows product is made (gemm_bf16_wide in gemm.hip):
 // 128 sorted rows x 256 columns of one expert per workgroup of four waves, a wave 64 rows x 128 columns; memory writes
 // slices of 32 of K straight into LDS (fetch_to_lds), three stages, in a layout whose rows swap places and whose chunks
@@ -698,14 +698,15 @@ __global__ __launch_bounds__(256, 2) void moe_experts_bf16_fetch_kernel(TO* __re
 }
 
 // The list's tiles two by two: a pair is two neighbouring tiles of one expert, counted from the first of its run; the last of an odd
-// run stands alone.  COUNT: how many pairs there are (first) and how many tiles alone; else the first tile of the nth pair, or the nth
-// tile alone.  A wave looks at 64 places a turn.
+// run stands alone, and so do both tiles of the pairs behind the first `keep`.  COUNT: how many pairs there are (first) and how many
+// tiles alone; else the first tile of the nth pair, or the nth tile alone.  A wave looks at 64 places a turn.
 struct TilesUsed {
   int pairs, alone;
 };
 template <bool COUNT>
-__device__ __forceinline__ TilesUsed tiles_by_two(const int* __restrict__ tile_expert, int tiles, int lane, int n, bool paired) {
+__device__ __forceinline__ TilesUsed tiles_by_two(const int* __restrict__ tile_expert, int tiles, int lane, int n, bool paired, int keep) {
   int before = -2, start = 0;                                          // the expert of the place before, where its run began
+  unsigned long long second = 0;                                       // place 0 is the second tile of a pair that is not kept
   TilesUsed used{0, 0};
   for (int at = 0; at < tiles; at += WAVE) {
     const int place = at + lane, expert = place < tiles ? tile_expert[place] : -1, right = place + 1 < tiles ? tile_expert[place + 1] : -1;
@@ -713,20 +714,33 @@ __device__ __forceinline__ TilesUsed tiles_by_two(const int* __restrict__ tile_e
     if (lane == 0) left = before;
     const unsigned long long starts = __ballot(expert != left), here = starts & (~0ull >> (63 - lane));
     const int run = here ? at + 63 - __clzll(here) : start;
-    const bool first = expert >= 0 && ((place - run) & 1) == 0;
-    const unsigned long long two = __ballot(first && right == expert), one = __ballot(first && right != expert);
+    const bool first = expert >= 0 && ((place - run) & 1) == 0, of_two = first && right == expert;
+    const unsigned long long all_twos = __ballot(of_two);
+    const int twos_before = used.pairs + __builtin_amdgcn_mbcnt_hi((unsigned)(all_twos >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)all_twos, 0));
+    const unsigned long long two = __ballot(of_two && twos_before < keep), parted = all_twos & ~two;
+    const unsigned long long one = __ballot(first && !of_two) | parted | parted << 1 | second;
+    second = parted >> 63;
     if (!COUNT) {
       const unsigned long long mask = paired ? two : one;
       const int earlier = __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0));
       if (n < __popcll(mask)) return TilesUsed{at + __ffsll(__ballot((mask >> lane & 1) != 0 && earlier == n)) - 1, 0};
       n -= __popcll(mask);
     }
-    used.pairs += __popcll(two);
+    used.pairs += __popcll(all_twos);
     used.alone += __popcll(one);
     before = __shfl(expert, 63, WAVE);
     if (starts) start = at + 63 - __clzll(starts);
   }
   return used;
+}
+
+// How many of the pairs stay pairs.  A compute unit works on one item at a time, on a pair some 1.7 times as long as on a tile alone:
+// pairs left over from whole rounds of the chip are parted where their tiles fit one round beside those that stand alone anyway (8
+// experts of 2 choices, 1,024 -> 2,048 features: 300 to 1,200 tokens 31-35 us with all pairs kept, 22-23 so, 24-26 in the kernel above;
+// 4,096 tokens 68 / 56 / 60; back to 1,024 2,048 tokens 54 / 34.5 / 40).
+__device__ __forceinline__ int pairs_to_keep(const TilesUsed& used, int tiles_n, int units) {
+  const int keep = used.pairs * tiles_n / units * units / tiles_n;
+  return (2 * (used.pairs - keep) + used.alone) * tiles_n <= units ? keep : used.pairs;
 }
 
 // The grouped product for large steps whose K is a multiple of 64: two tiles of an expert (256 rows) x 256 columns a workgroup of
@@ -735,9 +749,9 @@ __device__ __forceinline__ TilesUsed tiles_by_two(const int* __restrict__ tile_e
 // against 34, measured with nothing but fetches), and its tiles of 128 x 256 take half as much again for every product.  What bounds
 // it: few rows an expert, the weights' way from memory; many, the clock (some 2 GHz with the matrix cores this busy), the rows that
 // pad runs to tiles and the last round of workgroups.  Pairs before tiles alone: in the list's order a late pair made a round of its
-// own (612 tokens 218 us for 160).  32 experts of 8 choices, 4,096 -> 2,304 features and back, this kernel against that one: 200
-// tokens 176 / 194 and 132 / 138 us, 612 160 / 190 and 197 / 225, 1,200 247 / 322 and 270 / 321, 2,048 415 / 501 and 429 / 507, 8,192
-// 1,167 / 1,422; at 500 tokens 160 / 184 and 194 / 186.
+// own (612 tokens 218 us for 160).  32 experts of 8 choices, unequally loaded, 4,096 -> 2,304 features and back, this kernel against
+// that one: 200 tokens 172 / 190 and 131 / 134 us, 500 156 / 179 and 170 / 181, 612 183 / 188 and 194 / 219, 1,200 250 / 303 and 272 / 302,
+// 2,048 352 / 450 and 386 / 466, 4,096 612 / 754 and 710 / 790.
 template <int TILES, int STAGES, typename TO>
 __device__ __forceinline__ void experts_tile(bf16* slices, TO* __restrict__ out, int ldc, const bf16* __restrict__ x, int lda,
                                              const bf16* __restrict__ w, int n, int k, const int* __restrict__ sorted, int m0, int n0,
@@ -784,14 +798,17 @@ __device__ __forceinline__ void experts_tile(bf16* slices, TO* __restrict__ out,
 template <typename TO>
 __global__ __launch_bounds__(512, 1) void moe_experts_bf16_pairs_kernel(TO* __restrict__ out, int ldc, const bf16* __restrict__ x, int lda,
                                                                         const bf16* __restrict__ w, int n, int k, const int* __restrict__ sorted,
-                                                                        const int* __restrict__ tile_expert, int tiles_m, int tiles_n, int top,
-                                                                        int gather, int act, const PairAct pa) {
+                                                                        const int* __restrict__ tile_expert, int tiles_m, int tiles_n, int units,
+                                                                        int top, int gather, int act, const PairAct pa) {
   __shared__ __attribute__((aligned(64))) bf16 slices[3 * (128 + 256) * LINES_BK];
   static_assert(sizeof(slices) >= 2 * (256 + 256) * LINES_BK * sizeof(bf16), "two stages of two tiles");
   const int lane = threadIdx.x % WAVE;
   // Every die has an equal run of the pairs' tiles and one of those alone, and begins with the pairs, which take twice as long: the
   // last to start are short.
-  const TilesUsed used = tiles_by_two<true>(tile_expert, tiles_m, lane, 0, false);
+  TilesUsed used = tiles_by_two<true>(tile_expert, tiles_m, lane, 0, false, 1 << 30);
+  const int keep = pairs_to_keep(used, tiles_n, units);
+  used.alone += 2 * (used.pairs - keep);
+  used.pairs = keep;
   const int die = blockIdx.x % 8, paired_items = used.pairs * tiles_n, alone_items = used.alone * tiles_n;
   const int paired_here = paired_items / 8 + (die < paired_items % 8), alone_here = alone_items / 8 + (7 - die < alone_items % 8);
   int id = blockIdx.x / 8;
@@ -802,7 +819,7 @@ __global__ __launch_bounds__(512, 1) void moe_experts_bf16_pairs_kernel(TO* __re
   const int rows = paired ? used.pairs : used.alone;
   const int band = id / (4 * tiles_n), within = id % (4 * tiles_n);
   const int band_rows = rows - band * 4 < 4 ? rows - band * 4 : 4;
-  const int tile_m = __builtin_amdgcn_readfirstlane(tiles_by_two<false>(tile_expert, tiles_m, lane, band * 4 + within % band_rows, paired).pairs);
+  const int tile_m = __builtin_amdgcn_readfirstlane(tiles_by_two<false>(tile_expert, tiles_m, lane, band * 4 + within % band_rows, paired, keep).pairs);
   const int expert = tile_expert[tile_m];
   const bf16* we = w + (int64_t)expert * n * k;
   const int n0 = (within / band_rows) * 256;
@@ -1114,18 +1131,22 @@ LRS_API int lrs_moe_experts(void* out, int out_dtype, int ldc, const void* a, co
   // that fit 32 bits
   const bool fetching = cores && tile == WM && k % 32 == 0 && n % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)out % 16) == 0 && k >= 64 &&
                         (int64_t)n * k < (1ll << 30) && (gather ? (int64_t)max_tiles * tile / top + 1 : (int64_t)max_tiles * tile) * lda < (1ll << 30);
-  if (fetching && k % LINES_BK == 0) {
-    const int tiles_n = (n + 255) / 256;
+  const int tiles_n = (n + 255) / 256, units = lrs_compute_units();
+  // Two tiles a workgroup are one workgroup a compute unit, whose first slices and whose stores stand by themselves: under some ten
+  // slices that is what a product of several rounds of the chip is made of.  us, the kernel of pairs / the other one: 32 experts of 8
+  // choices, 512 -> 1,024 features 400 tokens (one round) 18.9 / 19.5, 1,200 29.4 / 28.2, 1,800 36 / 31, 2,048 42.6 / 42.1; 384 -> 1,024 1,800
+  // 33 / 29; 640 -> 2,048 300 tokens 30.6 / 32.7, 612 35.6 / 33.5, 2,048 77 / 78, 4,096 160 / 176; 1,024 -> 2,048 300 40 / 43, 612 44 / 42.5, 2,048
+  // 107 / 118; 1,152 -> 2,048 612 47.9 / 47.2, 1,500 85 / 105, 2,048 118 / 138.
+  if (fetching && k % LINES_BK == 0 && (k >= 640 || max_tiles * tiles_n <= units)) {
     if (out_dtype == LRS_BF16)
-      moe_experts_bf16_pairs_kernel<bf16><<<max_tiles * tiles_n + 16, 512, 0, s>>>((bf16*)out, ldc, (const bf16*)a, lda, (const bf16*)w, n, k, sorted, tile_expert, max_tiles, tiles_n, top, gather, act, pa);
+      moe_experts_bf16_pairs_kernel<bf16><<<max_tiles * tiles_n + 16, 512, 0, s>>>((bf16*)out, ldc, (const bf16*)a, lda, (const bf16*)w, n, k, sorted, tile_expert, max_tiles, tiles_n, units, top, gather, act, pa);
     else if (out_dtype == LRS_F32)
-      moe_experts_bf16_pairs_kernel<float><<<max_tiles * tiles_n + 16, 512, 0, s>>>((float*)out, ldc, (const bf16*)a, lda, (const bf16*)w, n, k, sorted, tile_expert, max_tiles, tiles_n, top, gather, act, pa);
+      moe_experts_bf16_pairs_kernel<float><<<max_tiles * tiles_n + 16, 512, 0, s>>>((float*)out, ldc, (const bf16*)a, lda, (const bf16*)w, n, k, sorted, tile_expert, max_tiles, tiles_n, units, top, gather, act, pa);
     else
       return lrs_fail("moe_experts: unknown output dtype %d", out_dtype);
     return lrs_check_launch("moe_experts");
   }
   if (fetching) {
-    const int tiles_n = (n + 255) / 256;
     if (out_dtype == LRS_BF16)
       moe_experts_bf16_fetch_kernel<bf16><<<max_tiles * tiles_n, 256, 0, s>>>((bf16*)out, ldc, (const bf16*)a, lda, (const bf16*)w, n, k, sorted, tile_expert, max_tiles, tiles_n, top, gather, act, pa);
     else if (out_dtype == LRS_F32)

@@ -101,3 +101,12 @@ def test_two_tiles_and_one(rows, n, k, gather, kind):
         if kind != "f32":
             bound = bound + (want.abs() + bound) * 2.0 ** -8
         assert ((got[rows_of] - want).abs() <= bound + 1e-30).all()
+
+
+# more items than 256 compute units work on at once: all pairs kept, the last ones of some rounds parted (in the middle of a run, at the
+# end of 64 places of the list, all of a small expert's), and whole rounds of nothing but pairs; and a K too short for pairs of so many items
+@pytest.mark.parametrize("rows,n,k", [((9000, 130, 640), 1028, 640), ((9000, 130, 640), 2052, 640), ((300, 8000, 1, 257, 256), 2308, 704), ((256,) * 96, 772, 640),
+                                      ((512,) * 32 + (3,), 1024, 640), ((9000, 130, 640), 1028, 576)])
+@pytest.mark.parametrize("gather,kind", [(True, "pairs"), (False, "f32")])
+def test_pairs_kept_and_parted(rows, n, k, gather, kind):
+    test_two_tiles_and_one(rows, n, k, gather, kind)
