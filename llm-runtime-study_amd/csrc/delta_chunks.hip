@@ -10,16 +10,21 @@
 // left for the walk are U = V' + W' S0, O = O' + Q' S0 and the update of S.
 //   delta_pack  per (chunk, head): those matrices, as operands of the walk's products;
 //   delta_walk  per (request, head, 16 columns of S): walks the chunks with its part of S in accumulators.
-// Precision: everything is float32 as in the scan, sums included; only their order differs.  Decays are multiplied as the scan does
-// and never divided, so decays of zero are no special case; the inverse holds products of contractions (1 - beta k k^T), none above one.
+// Precision: float32 as in the scan, sums in another order, and with it the queries' products with keys would make read-outs half as far
+// again from those of 64 bits as the scan's.  So the nearest tokens' are made in 64 bits, a token's u is rounded as often as in the scan
+// (exact_sum) and the state's update adds the last tokens one by one on top of the earlier ones (U's order).  Distance from 64 bits,
+// here / in the scan, read-outs and states: a Nobodra layer's inputs (decays about 0.5) 6.4e-8 / 6.7e-8 and 4.9e-8 / 5.0e-8 (1.0e-7 and
+// 6.6e-8 without all that); decays near one 1.5e-7 / 1.9e-7 and 1.1e-7 / 1.5e-7; keys that are nearly all alike under step sizes near one
+// 4.0e-7 / 2.5e-7 and 5.9e-7 / 6.5e-7.  Decays are multiplied as the scan does and never divided, so decays of zero are no special case;
+// the inverse holds products of contractions (1 - beta k k^T), none above one.
 // A token whose inputs are infinite or NaN spoils itself and what comes after it, as in the scan, and no token before it.
 //
 // The matrix instructions are 16 x 16 x 4: of a block of 16 rows, lane 16 g + r gives or gets row r (column r) and, of every 16 of
 // the inner size, the four 4 g .. 4 g + 3 in four instructions.  Sums come out with lane 16 g + r holding column r of the rows
 // 4 g .. 4 g + 3, so a block of sums is at once a right operand of the next product.
 //
-// 32 heads of 128 x 128, one request of 2,048 tokens: 514 us in the scan, a chain of 2,048 turns with two lane sums each; here 75 us for
-// the packs and 95 for the walk.  Where the scan is the faster one (many portions, short ones) the part says.
+// 32 heads of 128 x 128, one request of 2,048 tokens: 514 us in the scan, a chain of 2,048 turns with two lane sums each; here, inside a
+// prompt, 81 us for the packs (78 with all products in float32) and 103 for the walk.  Where the scan is the faster one (many portions, short ones) the part says.
 #include "common.h"
 
 extern "C" int lrs_delta_state_rows(int d);
@@ -33,6 +38,8 @@ constexpr int BLOCK = 16 * 16;    // floats of a block of operands or sums
 // A request's chunks lie side by side in the packs: request r's chunk c in slot cu[r] / L + r + c (requests never share one).
 __device__ __forceinline__ int first_slot(const int* __restrict__ cu, int r) { return cu[r] / L + r; }
 
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
 __device__ __forceinline__ floatx4 mfma(float a, float b, floatx4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 // c + a b for a block of 16 x 16 x 16
@@ -43,7 +50,7 @@ __device__ __forceinline__ floatx4 product(const floatx4& a, const floatx4& b, f
 }
 
 // A sum over many blocks, in four parts: a part's roundings are a quarter as many and of smaller numbers (with one chain the read-outs
-// were twice as far from those of 64 bits as the scan's, 3.7e-7 and 1.9e-7).
+// were twice as far from those of 64 bits as the scan's).
 struct Sums {
   floatx4 part[4] = {};
   __device__ __forceinline__ void add(int j, const floatx4& a, const floatx4& b) { part[j % 4] = product(a, b, part[j % 4]); }
@@ -58,6 +65,27 @@ struct Sums {
   __device__ __forceinline__ floatx4 total() const { return (part[0] + part[1]) + (part[2] + part[3]); }
 };
 
+// The four values of lane group g and the lane groups change places: value i of group g goes to value g of group i.
+__device__ __forceinline__ floatx4 groups_for_values(floatx4 v) {
+  typedef unsigned two __attribute__((ext_vector_type(2)));
+  const two a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[0]), __float_as_uint(v[1]), false, false);
+  const two b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[2]), __float_as_uint(v[3]), false, false);
+  const two c = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false), d = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+  return floatx4{__uint_as_float(c[0]), __uint_as_float(d[0]), __uint_as_float(c[1]), __uint_as_float(d[1])};
+}
+
+// s times x plus c, as a sum and what its rounding left out of it.
+struct Pair {
+  float sum, rest;
+};
+__device__ __forceinline__ Pair exact_sum(float s, float x, float c) {
+#pragma clang fp contract(off)
+  const float p = s * x, p_rest = fmaf(s, x, -p), sum = p + c, back = sum - p;
+  return Pair{sum, ((p - (sum - back)) + (c - back)) + p_rest};
+}
+
+// U's order: lane group g's value i of a block is token g + 4 i, so that the four tokens of a matrix instruction of the state's update
+// are neighbours and the update adds them from the first to the last, as the scan does; W', V' and the keys are packed for that.
 // A (slot, head)'s floats: W' and Q' [L / 16][DP / 16] blocks of left operands, D_Ls k_s by rows of S [DP / 16][L / 16] blocks of left
 // operands, V' and O' [column blocks][L / 16] blocks of sums, and one line for c_L.
 __host__ __device__ inline int64_t pack_floats(int dp, int blocks) { return (int64_t)3 * L * dp + (int64_t)2 * L * 16 * blocks + 64; }
@@ -65,9 +93,9 @@ __host__ __device__ inline int64_t pack_floats(int dp, int blocks) { return (int
 // Four waves.  The products of keys with keys and queries (wave w takes row block w of the one and 3 - w of the other: ten blocks each
 // in all, five a wave), the inverses of A's diagonal blocks (a wave one, a lane a column), and then every wave solves for columns of
 // its own, block row by block row, each block of the solution at once an operand of the next.  480 matrix instructions a wave for
-// heads of 128 x 128, 7 us (139 TFLOP/s is what the float32 ones reach): 29 us for 1,024 heads of chunks if nothing else took time, 75 as
-// it is, two workgroups a compute unit filling each other's waits.  11 of them are the stores of W' and Q' in pieces of 16 bytes; loads
-// behind branches, one waited for after the other, had made it 117.
+// heads of 128 x 128, 32 of them in 64 bits and twice as long, 7 us (139 TFLOP/s is what the float32 ones reach): 31 us for 1,024 heads of
+// chunks if nothing else took time, 81 as it is inside a prompt, two workgroups a compute unit filling each other's waits.  11 of them are
+// the stores of W' and Q' in pieces of 16 bytes; loads behind branches, one waited for after the other, had made it 40 more.
 // WHOLE: every piece of four values is 16 bytes aligned.
 template <int DP, bool WHOLE>
 __global__ __launch_bounds__(256, 2) void delta_pack_kernel(const float* __restrict__ qkv, const float* __restrict__ gates,
@@ -75,7 +103,7 @@ __global__ __launch_bounds__(256, 2) void delta_pack_kernel(const float* __restr
                                                             float* __restrict__ packs) {
   constexpr int KB = DP / 16, LD = DP + 4, TLD = L + 4;        // rows four banks apart: 16-byte reads of 16 rows meet no conflict
   __shared__ __attribute__((aligned(16))) float ks[L * LD];
-  __shared__ __attribute__((aligned(16))) float low[L * TLD];  // D, then -A off the diagonal blocks and the inverses in them
+  __shared__ __attribute__((aligned(16))) float low[L * TLD];  // D, then -A off the diagonal blocks and the inverses less 1 in them
   __shared__ __attribute__((aligned(16))) float seen[L * TLD]; // D, then P
   __shared__ __attribute__((aligned(16))) float beta_of[L], decay_of[L], tail_of[L];
   const int slot = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), col = lane & 15, g = lane >> 4;
@@ -152,13 +180,18 @@ __global__ __launch_bounds__(256, 2) void delta_pack_kernel(const float* __restr
     for (int j = 0; j < KB; ++j) ka[j] = *(const floatx4*)(ks + (wave * 16 + col) * LD + 16 * j + 4 * g);
     // the sums of one row block's rows with the keys of block b
     auto with_keys = [&](const floatx4 (&rows)[KB], int b) {
-      Sums sums;
-      floatx4 keys[KB];
+      floatx4 part[KB] = {}, keys[KB];
 #pragma unroll
       for (int j = 0; j < KB; ++j) keys[j] = *(const floatx4*)(ks + (b * 16 + col) * LD + 16 * j + 4 * g);
 #pragma unroll
-      for (int j = 0; j < KB; j += 2) sums.add_two(j, rows, keys);
-      return sums.total();
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < KB; ++j) part[j] = mfma(rows[j][i], keys[j][i], part[j]);
+#pragma unroll
+      for (int apart = 1; apart < KB; apart *= 2)
+#pragma unroll
+        for (int j = 0; j < KB; j += 2 * apart) part[j] += part[j + apart];
+      return part[0];
     };
     for (int b = 0; b <= wave; ++b) {
       const floatx4 sums = with_keys(ka, b), beta4 = *(const floatx4*)(beta_of + wave * 16 + 4 * g);
@@ -170,20 +203,30 @@ __global__ __launch_bounds__(256, 2) void delta_pack_kernel(const float* __restr
         low[t * TLD + s] = b < wave ? -a : s < t ? a : 0.f;
       }
     }
-    for (int b = 0; b <= bq; ++b) {
+    for (int b = 0; b < bq; ++b) {
       const floatx4 sums = with_keys(qa, b);
-      const int s = b * 16 + col;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int t = bq * 16 + 4 * g + i;
-        const float p = seen[t * TLD + s] * sums[i];
-        seen[t * TLD + s] = s <= t ? p : 0.f;
-      }
+      for (int i = 0; i < 4; ++i) seen[(bq * 16 + 4 * g + i) * TLD + b * 16 + col] *= sums[i];
+    }
+    // The last block in 64 bits: a query's product with a key is where the terms cancel most, and the nearest tokens' are what
+    // read-outs are mostly made of.  (Sums come out with lane 16 g + r holding column r of the rows g, g + 4, g + 8 and g + 12.)
+    doublex4 sums[2] = {};
+#pragma unroll
+    for (int j = 0; j < KB; ++j) {
+      const floatx4 keys = *(const floatx4*)(ks + (bq * 16 + col) * LD + 16 * j + 4 * g);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sums[i % 2] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)qa[j][i], (double)keys[i], sums[i % 2], 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = g + 4 * i;
+      float* at = seen + (bq * 16 + row) * TLD + bq * 16 + col;
+      *at = col <= row ? (float)((double)*at * (sums[0][i] + sums[1][i])) : 0.f;
     }
   }
   __syncthreads();
   {
-    // column `col` of the inverse of 1 + A's block (wave, wave), by substitution from the top
+    // column `col` of the inverse of 1 + A's block (wave, wave) by substitution from the top; what is kept is the inverse less 1
     const float* a = low + (wave * 16) * TLD + wave * 16;
     float x[16];
 #pragma unroll
@@ -198,7 +241,7 @@ __global__ __launch_bounds__(256, 2) void delta_pack_kernel(const float* __restr
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < 16; ++t)
-      if (t / 4 == g) low[(wave * 16 + t) * TLD + wave * 16 + col] = x[t];
+      if (t / 4 == g) low[(wave * 16 + t) * TLD + wave * 16 + col] = t == col ? 0.f : x[t];
   }
   __syncthreads();
 
@@ -247,13 +290,12 @@ __global__ __launch_bounds__(256, 2) void delta_pack_kernel(const float* __restr
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
       const int t0 = b * 16 + 4 * g;
-      const floatx4 steps = *(const floatx4*)(beta_of + t0), kept = *(const floatx4*)(decay_of + t0);
+      const floatx4 kept = *(const floatx4*)(decay_of + t0);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float value = t0 + i < count && column < width ? next[b][i] : 0.f;
-        const float from_key = -steps[i] * (kept[i] * ks[(t0 + i) * LD + min(column, DP - 1)]), from_value = steps[i] * value, read = kept[i] * value;
-        x[b][i] = is_w ? from_key : from_value;
-        y[b][i] = is_w ? read : 0.f;
+        x[b][i] = is_w ? kept[i] * ks[(t0 + i) * LD + min(column, DP - 1)] : value;       // (times the step sizes below)
+        y[b][i] = is_w ? kept[i] * value : 0.f;
       }
     }
     fetch(min(tile + 4, KB + blocks - 1));
@@ -263,8 +305,16 @@ __global__ __launch_bounds__(256, 2) void delta_pack_kernel(const float* __restr
       Sums above, read;
 #pragma unroll
       for (int c = 0; c < b; ++c) above.add(c, la[b * (b + 1) / 2 + c], x[c]);
-      if (b > 0) x[b] += above.total();
-      x[b] = on_diagonal(low, b, la[b * (b + 1) / 2 + b], x[b], floatx4{0.f, 0.f, 0.f, 0.f});
+      // The right side less what the blocks above take of it, rounded and what the rounding left out, which joins the smaller part of
+      // the product with the inverse: a token's u is rounded twice, as in the scan.
+      const floatx4 steps = *(const floatx4*)(beta_of + b * 16 + 4 * g), taken = above.total();
+      floatx4 rest;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const Pair right = exact_sum(is_w ? -steps[i] : steps[i], x[b][i], taken[i]);
+        x[b][i] = right.sum, rest[i] = right.rest;
+      }
+      x[b] += on_diagonal(low, b, la[b * (b + 1) / 2 + b], x[b], rest);
 #pragma unroll
       for (int c = 0; c < b; ++c) read.add(c, pa[b * (b + 1) / 2 + c], x[c]);
       read.part[b] = on_diagonal(seen, b, pa[b * (b + 1) / 2 + b], x[b], read.part[b]);
@@ -273,16 +323,16 @@ __global__ __launch_bounds__(256, 2) void delta_pack_kernel(const float* __restr
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
       if (is_w) {
-        // as left operands: row 4 g + i, and column col of the block is lane group col / 4's value col % 4
+        // as left operands: row 4 g + i (of W' row 4 i + g: see U's order), and column col of the block is lane group col / 4's value col % 4
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int at = (b * KB + tile) * BLOCK + (col / 4 * 16 + 4 * g + i) * 4 + col % 4;
-          w_pack[at] = x[b][i];
-          q_pack[at] = y[b][i];
+          const int at = (b * KB + tile) * BLOCK + col / 4 * 64 + col % 4;
+          w_pack[at + (4 * i + g) * 4] = x[b][i];
+          q_pack[at + (4 * g + i) * 4] = y[b][i];
         }
       } else {
         const int at = ((tile - KB) * 4 + b) * BLOCK + lane * 4;
-        *(floatx4*)(v_pack + at) = x[b];
+        *(floatx4*)(v_pack + at) = groups_for_values(x[b]);
         *(floatx4*)(o_pack + at) = y[b];
       }
     }
@@ -292,7 +342,7 @@ __global__ __launch_bounds__(256, 2) void delta_pack_kernel(const float* __restr
     for (int j = 0; j < 4; ++j) {
       floatx4 v;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = ks[(16 * j + 4 * g + i) * LD + 16 * b + col] * tail_of[16 * j + 4 * g + i];
+      for (int i = 0; i < 4; ++i) v[i] = ks[(16 * j + g + 4 * i) * LD + 16 * b + col] * tail_of[16 * j + g + 4 * i];
       *(floatx4*)(k_pack + (b * 4 + j) * BLOCK + lane * 4) = v;
     }
 }
@@ -301,7 +351,7 @@ __global__ __launch_bounds__(256, 2) void delta_pack_kernel(const float* __restr
 // new S go through LDS, a barrier each; half of O's products stand before either barrier, with the old S still in registers.  A
 // chunk's operands (a wave's rows of the packs, 1,024 bytes a load) are asked for a chunk ahead, into a second set of registers: with
 // one wave a SIMD there are enough.  96 matrix instructions a wave and chunk, 3,072 cycles: 47 us for
-// 32 chunks, 95 as it is: 71 without the loads (96 KB a chunk and compute unit, 44 bytes a nanosecond is the most that any kernel here
+// 32 chunks, 95 by itself and 103 inside a prompt: 71 without the loads (96 KB a chunk and compute unit, 44 bytes a nanosecond is the most that any kernel here
 // has been seen to get), the rest the two barriers with a trip through LDS each.  Left to itself the compiler moves the loads to where
 // their registers are cheapest: 106 us.
 template <int DP>
@@ -378,15 +428,19 @@ __global__ __launch_bounds__(256, 1) void delta_walk_kernel(const float* __restr
 #pragma unroll
     for (int j = 0; j < 4; ++j) all[j] = u_room[j * WAVE + lane];
     read_out(1);
+    // the state and the first three blocks of tokens, each summed by itself, and the last block's chain, mostly the largest, on top
 #pragma unroll
-    for (int j = 0; j < 4; j += 2)
+    for (int b = 0; b < SB; ++b) s[b].add_two(0, x.k[b], all);
 #pragma unroll
-      for (int b = 0; b < SB; ++b) s[b].add_two(j, x.k[b], all);
+    for (int b = 0; b < SB; ++b) s[b].add(2, x.k[b][2], all[2]);
 #pragma unroll
-    for (int b = 0; b < SB; ++b) {
-      S[b] = x.end * S[b] + s[b].total();
-      s_room[(wave * SB + b) * WAVE + lane] = S[b];
-    }
+    for (int b = 0; b < SB; ++b) S[b] = x.end * S[b] + ((s[b].part[0] + s[b].part[1]) + s[b].part[2]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int b = 0; b < SB; ++b) S[b] = mfma(x.k[b][3][i], all[3][i], S[b]);
+#pragma unroll
+    for (int b = 0; b < SB; ++b) s_room[(wave * SB + b) * WAVE + lane] = S[b];
     read_out(2);
     __syncthreads();
     floatx4 now[KB];

@@ -134,7 +134,7 @@ class GatedDeltaRule(Part):
         """Whether the form in chunks is the faster one for a step of that many tokens and requests, the first `singles` with one each.
 
         The scan is a chain, 0.25 us a token of a portion, as long as there are few portions; many fill each other's waits, down to
-        0.10 us a token and workgroup on a compute unit.  The chunks' matrices take 19 us for every 256 heads of chunks and the walk
+        0.10 us a token and workgroup on a compute unit.  The chunks' matrices take 21 us for every 256 heads of chunks and the walk
         3 us a chunk, 3.6 with workgroups in turn (32 heads of 128 x 128: 2,048 tokens of one request 514 us in the scan, 180 in
         chunks; 256 tokens 66 and 40; 128 tokens 34 and 34; four requests of 512 209 and 206; sixteen of 128 204 and 310).  Only what
         a recorded step's shape tells is asked: the longest portion is at least as long as the mean."""
@@ -144,7 +144,7 @@ class GatedDeltaRule(Part):
         groups = self.num_heads * -(-self.value_dim // 16) / 256          # workgroups a request and compute unit
         chunks = rows / 64 + portions / 2
         scan = max(0.25 * rows / portions, 0.10 * rows * groups)
-        return 12 + 19 * max(1.0, chunks * self.num_heads / 256) + 3 * max(chunks / portions, 1.2 * chunks * groups) < 0.9 * scan
+        return 12 + 21 * max(1.0, chunks * self.num_heads / 256) + 3 * max(chunks / portions, 1.2 * chunks * groups) < 0.9 * scan
 
     def forward(self, ctx, x, residual, cache, then_norm=None, accumulate: bool = True):
         if cache is None or cache.state is None:
