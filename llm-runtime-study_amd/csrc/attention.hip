@@ -261,9 +261,10 @@ struct HeadTables {       // the rotation's cosines and sines of the lane's dims
       }
   }
 };
-template <int D>
-__device__ __forceinline__ void head_from_registers(bf16x8 (&r)[D / 32], float (&x)[D / 32][8], bool normed, const HeadWeights<D>& weights,
-                                                 int weight_is_f32, float eps, bool rotated, const HeadTables<D>& tables) {
+// One head's norm and rotation: weights_of(c, w) and tables_of(c, cs, sn) give a chunk's eight weights, cosines and sines.
+template <int D, typename Weights, typename Tables>
+__device__ __forceinline__ void norm_and_rotate(bf16x8 (&r)[D / 32], float (&x)[D / 32][8], bool normed, float eps, bool rotated,
+                                                const Weights& weights_of, const Tables& tables_of) {
   constexpr int DS = D / 32;
   if (normed) {
     float ss = 0.f;
@@ -275,71 +276,23 @@ __device__ __forceinline__ void head_from_registers(bf16x8 (&r)[D / 32], float (
     ss += __shfl_xor(ss, 32, WAVE);
     const float inv = 1.0f / sqrtf(ss / (float)D + eps);
 #pragma unroll
-    for (int c = 0; c < DS; ++c)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) x[c][j] = x[c][j] * inv * weights.value(c, j, weight_is_f32);
-  }
-  if (rotated) {
-#pragma unroll
-    for (int c = 0; c < D / 64; ++c)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float cs = tables.cs[c][j / 4][j % 4], sn = tables.sn[c][j / 4][j % 4];
-        const float a = x[c][j], b = x[c + DS / 2][j];
-        x[c][j] = a * cs - b * sn;
-        x[c + DS / 2][j] = b * cs + a * sn;
-      }
-  }
-#pragma unroll
-  for (int c = 0; c < DS; ++c)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) r[c][j] = (bf16)x[c][j];
-}
-
-// The same for the prompt kernels, whose waves prepare their queries once a walk and have no registers to spare: weights and
-// tables are loaded where they are used (with them asked for first a prompt of 2,048 tokens of the 8B shape took 1.5 % longer).
-template <int D>
-__device__ __forceinline__ void head_from_values(bf16x8 (&r)[D / 32], float (&x)[D / 32][8], int g,
-                                                 const void* __restrict__ weight, int weight_is_f32, float eps,
-                                                 const float* __restrict__ cosrow, const float* __restrict__ sinrow) {
-  constexpr int DS = D / 32;
-  // weights and tables come in 16-byte loads (the host checks their alignment)
-  if (weight) {
-    float ss = 0.f;
-#pragma unroll
-    for (int c = 0; c < DS; ++c)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) ss = fmaf(x[c][j], x[c][j], ss);
-    ss += __shfl_xor(ss, 16, WAVE);
-    ss += __shfl_xor(ss, 32, WAVE);
-    const float inv = 1.0f / sqrtf(ss / (float)D + eps);
-#pragma unroll
     for (int c = 0; c < DS; ++c) {
       float w[8];
-      if (weight_is_f32) {
-        const floatx4 w0 = *(const floatx4*)((const float*)weight + c * 32 + g * 8), w1 = *(const floatx4*)((const float*)weight + c * 32 + g * 8 + 4);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) { w[j] = w0[j]; w[4 + j] = w1[j]; }
-      } else {
-        const bf16x8 wb = *(const bf16x8*)((const bf16*)weight + c * 32 + g * 8);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) w[j] = (float)wb[j];
-      }
+      weights_of(c, w);
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[c][j] = x[c][j] * inv * w[j];
     }
   }
-  if (cosrow) {
+  if (rotated) {
 #pragma unroll
-    for (int c = 0; c < DS / 2; ++c) {
-      const floatx4 c0 = *(const floatx4*)(cosrow + c * 32 + g * 8), c1 = *(const floatx4*)(cosrow + c * 32 + g * 8 + 4);
-      const floatx4 s0 = *(const floatx4*)(sinrow + c * 32 + g * 8), s1 = *(const floatx4*)(sinrow + c * 32 + g * 8 + 4);
+    for (int c = 0; c < D / 64; ++c) {
+      float cs[8], sn[8];
+      tables_of(c, cs, sn);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const float cs = j < 4 ? c0[j & 3] : c1[j & 3], sn = j < 4 ? s0[j & 3] : s1[j & 3];
         const float a = x[c][j], b = x[c + DS / 2][j];
-        x[c][j] = a * cs - b * sn;
-        x[c + DS / 2][j] = b * cs + a * sn;
+        x[c][j] = a * cs[j] - b * sn[j];
+        x[c + DS / 2][j] = b * cs[j] + a * sn[j];
       }
     }
   }
@@ -348,19 +301,48 @@ __device__ __forceinline__ void head_from_values(bf16x8 (&r)[D / 32], float (&x)
 #pragma unroll
     for (int j = 0; j < 8; ++j) r[c][j] = (bf16)x[c][j];
 }
-
 template <int D>
-__device__ __forceinline__ void prepare_head(bf16x8 (&r)[D / 32], const bf16* __restrict__ head, int g,
-                                             const void* __restrict__ weight, int weight_is_f32, float eps,
-                                             const float* __restrict__ cosrow, const float* __restrict__ sinrow) {
-  float x[D / 32][8];
+__device__ __forceinline__ void head_from_registers(bf16x8 (&r)[D / 32], float (&x)[D / 32][8], bool normed, const HeadWeights<D>& weights,
+                                                    int weight_is_f32, float eps, bool rotated, const HeadTables<D>& tables) {
+  norm_and_rotate<D>(
+      r, x, normed, eps, rotated,
+      [&](int c, float (&w)[8]) {
 #pragma unroll
-  for (int c = 0; c < D / 32; ++c) {
-    const bf16x8 raw = *(const bf16x8*)(head + c * 32 + g * 8);
+        for (int j = 0; j < 8; ++j) w[j] = weights.value(c, j, weight_is_f32);
+      },
+      [&](int c, float (&cs)[8], float (&sn)[8]) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) x[c][j] = (float)raw[j];
-  }
-  head_from_values<D>(r, x, g, weight, weight_is_f32, eps, cosrow, sinrow);
+        for (int j = 0; j < 8; ++j) cs[j] = tables.cs[c][j / 4][j % 4], sn[j] = tables.sn[c][j / 4][j % 4];
+      });
+}
+
+// The same for the prompt kernels, whose waves prepare their queries once a walk and have no registers to spare: weights and
+// tables are loaded where they are used (asked for first they cost 30 to 90 spilled registers), in 16-byte loads (the host checks
+// their alignment).
+template <int D>
+__device__ __forceinline__ void head_from_memory(bf16x8 (&r)[D / 32], float (&x)[D / 32][8], int g, const void* __restrict__ weight,
+                                                 int weight_is_f32, float eps, const float* __restrict__ cosrow, const float* __restrict__ sinrow) {
+  norm_and_rotate<D>(
+      r, x, weight != nullptr, eps, cosrow != nullptr,
+      [&](int c, float (&w)[8]) {
+        if (weight_is_f32) {
+          const floatx4 w0 = *(const floatx4*)((const float*)weight + c * 32 + g * 8), w1 = *(const floatx4*)((const float*)weight + c * 32 + g * 8 + 4);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) w[j] = w0[j], w[4 + j] = w1[j];
+        } else {
+          const bf16x8 wb = *(const bf16x8*)((const bf16*)weight + c * 32 + g * 8);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) w[j] = (float)wb[j];
+        }
+      },
+      [&](int c, float (&cs)[8], float (&sn)[8]) {
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+          const floatx4 c4 = *(const floatx4*)(cosrow + c * 32 + g * 8 + 4 * n), s4 = *(const floatx4*)(sinrow + c * 32 + g * 8 + 4 * n);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) cs[4 * n + j] = c4[j], sn[4 * n + j] = s4[j];
+        }
+      });
 }
 
 // One query token per request (a decode step).  A workgroup of four waves owns one
@@ -1619,7 +1601,7 @@ __device__ __forceinline__ void attention_prefill_d128_part(
 #pragma unroll
           for (int j = 0; j < 8; ++j) x[c][j] = (float)qf[b][c][j];
         const int token = token0 + (live[b] ? query0 + b * 16 + col : 0);
-        head_from_values<D>(qf[b], x, g, prep.q_weight, prep.weight_is_f32, prep.eps, prep.cosv ? prep.cosv + (int64_t)token * (D / 2) : nullptr,
+        head_from_memory<D>(qf[b], x, g, prep.q_weight, prep.weight_is_f32, prep.eps, prep.cosv ? prep.cosv + (int64_t)token * (D / 2) : nullptr,
                             prep.sinv ? prep.sinv + (int64_t)token * (D / 2) : nullptr);
       }
 #pragma unroll
