@@ -13,9 +13,9 @@
 // Precision: float32 as in the scan, sums in another order, and with it the queries' products with keys would make read-outs half as far
 // again from those of 64 bits as the scan's.  So the nearest tokens' are made in 64 bits, a token's u is rounded as often as in the scan
 // (exact_sum) and the state's update adds the last tokens one by one on top of the earlier ones (U's order).  Distance from 64 bits,
-// here / in the scan, read-outs and states: a Nobodra layer's inputs (decays about 0.5) 6.4e-8 / 6.7e-8 and 4.9e-8 / 5.0e-8 (1.0e-7 and
+// here / in the scan, read-outs and states: a Nobodra layer's inputs (decays about 0.5) 6.4e-8 / 6.7e-8 and 4.8e-8 / 4.9e-8 (1.0e-7 and
 // 6.6e-8 without all that); decays near one 1.5e-7 / 1.9e-7 and 1.1e-7 / 1.5e-7; keys that are nearly all alike under step sizes near one
-// 4.0e-7 / 2.5e-7 and 5.9e-7 / 6.5e-7.  Decays are multiplied as the scan does and never divided, so decays of zero are no special case;
+// 4.2e-7 / 2.5e-7 and 5.9e-7 / 6.5e-7.  Decays are multiplied as the scan does and never divided, so decays of zero are no special case;
 // the inverse holds products of contractions (1 - beta k k^T), none above one.
 // A token whose inputs are infinite or NaN spoils itself and what comes after it, as in the scan, and no token before it.
 //
@@ -24,7 +24,8 @@
 // 4 g .. 4 g + 3, so a block of sums is at once a right operand of the next product.
 //
 // 32 heads of 128 x 128, one request of 2,048 tokens: 514 us in the scan, a chain of 2,048 turns with two lane sums each; here, inside a
-// prompt, 81 us for the packs (78 with all products in float32) and 103 for the walk.  Where the scan is the faster one (many portions, short ones) the part says.
+// prompt, 84 us for the packs, some 5 of them for the precision above, and 105 for the walk.  Where the scan is the faster one (many
+// portions, short ones) the part says.
 #include "common.h"
 
 extern "C" int lrs_delta_state_rows(int d);
@@ -94,7 +95,7 @@ __host__ __device__ inline int64_t pack_floats(int dp, int blocks) { return (int
 // in all, five a wave), the inverses of A's diagonal blocks (a wave one, a lane a column), and then every wave solves for columns of
 // its own, block row by block row, each block of the solution at once an operand of the next.  480 matrix instructions a wave for
 // heads of 128 x 128, 32 of them in 64 bits and twice as long, 7 us (139 TFLOP/s is what the float32 ones reach): 31 us for 1,024 heads of
-// chunks if nothing else took time, 81 as it is inside a prompt, two workgroups a compute unit filling each other's waits.  11 of them are
+// chunks if nothing else took time, 84 as it is inside a prompt, two workgroups a compute unit filling each other's waits.  11 of them are
 // the stores of W' and Q' in pieces of 16 bytes; loads behind branches, one waited for after the other, had made it 40 more.
 // WHOLE: every piece of four values is 16 bytes aligned.
 template <int DP, bool WHOLE>
@@ -351,7 +352,7 @@ __global__ __launch_bounds__(256, 2) void delta_pack_kernel(const float* __restr
 // new S go through LDS, a barrier each; half of O's products stand before either barrier, with the old S still in registers.  A
 // chunk's operands (a wave's rows of the packs, 1,024 bytes a load) are asked for a chunk ahead, into a second set of registers: with
 // one wave a SIMD there are enough.  96 matrix instructions a wave and chunk, 3,072 cycles: 47 us for
-// 32 chunks, 95 by itself and 103 inside a prompt: 71 without the loads (96 KB a chunk and compute unit, 44 bytes a nanosecond is the most that any kernel here
+// 32 chunks, 95 by itself and 105 inside a prompt: 71 without the loads (96 KB a chunk and compute unit, 44 bytes a nanosecond is the most that any kernel here
 // has been seen to get), the rest the two barriers with a trip through LDS each.  Left to itself the compiler moves the loads to where
 // their registers are cheapest: 106 us.
 template <int DP>
