@@ -441,6 +441,10 @@ __device__ __forceinline__ void attention_decode_part(
   // are read from the nearest it does see, not branched around (three branches were three trips to
   // memory one after the other): their scores are replaced, their values zeroed (work, below).
   const int key_of_row = (col >> 2) * 8 + (col & 3);           // + 4*h
+  // A key or value is read by one workgroup, once (load_once; 64 requests at 2,048 tokens, 8B sizes: 6,774 -> 6,618 us a step).  Not in
+  // the form of eight waves: its short contexts of a few requests stay in the last-level cache from step to step, which what is
+  // loaded with the hint does not (one request at 509 tokens, 0.6B sizes: 1,035 us a step, 1,078 with the hint).
+  constexpr bool ONCE = WAVES == 4;
   auto fetch = [&](int tile, bf16x8 (&kf)[2][DS], bf16x8 (&vf)[DB]) {
     const bf16* kp[2];
 #pragma unroll
@@ -455,10 +459,13 @@ __device__ __forceinline__ void attention_decode_part(
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int c = 0; c < DS; ++c) kf[h][c] = *(const bf16x8*)(kp[h] + c * 32);
+      for (int c = 0; c < DS; ++c) kf[h][c] = ONCE ? load_once((const bf16x8*)(kp[h] + c * 32)) : *(const bf16x8*)(kp[h] + c * 32);
     // (values narrower than keys: the blocks behind them repeat the last one, and nothing of them is written)
 #pragma unroll
-    for (int b = 0; b < DB; ++b) vf[b] = *(const bf16x8*)(vp + (int64_t)(b * 16 < dv ? b * 16 : dv - 16) * page_size);
+    for (int b = 0; b < DB; ++b) {
+      const bf16x8* at = (const bf16x8*)(vp + (int64_t)(b * 16 < dv ? b * 16 : dv - 16) * page_size);
+      vf[b] = ONCE ? load_once(at) : *at;
+    }
   };
   // AHEAD: the wave's first tile is asked for as soon as the page ids are there, before the query (and
   // the new key) are prepared, so that the first trip to memory runs beside that work.  No branch around it, a wave

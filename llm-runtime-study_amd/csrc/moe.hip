@@ -364,6 +364,8 @@ __global__ __launch_bounds__(256) void moe_experts_kernel(TO* __restrict__ out, 
 // multiplied.
 constexpr int GM = 32, GN = 128, GK = 64, GPAD = 8;
 
+// An expert of a step of few rows has one tile of them, so its weights are read once (load_once): eight steps of eight requests and their
+// prompts, 4 layers of the 8B sizes with 32 experts 14,425 -> 13,310 us; a step of 16 requests with gated experts 1,354 -> 1,240.
 // NT: columns per workgroup, 128 (a wave 32 of them) or 64 (a wave 16: twice the workgroups, for steps of so few rows
 // that 128 columns each would leave compute units without any).
 template <typename TO, int NT>
@@ -396,7 +398,7 @@ __global__ __launch_bounds__(256) void moe_experts_bf16_kernel(TO* __restrict__ 
 #pragma unroll
     for (int p = 0; p < NT / 32; ++p) {
       const int r = p * 32 + a_row;
-      b_reg[p] = col0 + r < n ? *(const bf16x8*)(we + (int64_t)(col0 + r) * k + k0 + a_col) : zero;
+      b_reg[p] = col0 + r < n ? load_once((const bf16x8*)(we + (int64_t)(col0 + r) * k + k0 + a_col)) : zero;
     }
   };
   floatx4 acc[2][WN] = {};
