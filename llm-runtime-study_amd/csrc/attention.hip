@@ -357,20 +357,23 @@ __device__ __forceinline__ void head_from_memory(bf16x8 (&r)[D / 32], float (&x)
 // S comes out of the first product with a head per lane column and four keys per lane, which
 // is exactly the operand layout the second product wants for P, so P never leaves registers.
 // Waves are merged through LDS, splits by attention_merge_kernel.
-// PREP: q holds the raw rows of the q/k/v product; the kernel prepares q itself, and the wave that
-// meets the token's own position prepares the new key, takes it and the new value in place of what
-// the pages hold there, and writes both into the pages (see DecodePrep).
+// PREP: q holds the raw rows of the q/k/v product; the kernel prepares q and the new key itself; the wave that
+// meets the token's own position takes that key and the new value in place of what the pages hold there, and
+// its workgroup writes both into the pages (see DecodePrep).
 // What bounds a walk of few keys is the chain of trips to memory (position, block table, keys) and what stands between them;
 // so nothing that is asked for hides behind a branch, rows, weights and tables are asked for first, and only the wave that
 // meets the new key waits for it.  A step of the 0.6B shape (28 layers, 16 heads on 8), one request at 509 tokens: 1,166 ->
 // 1,076 us, 16 requests 1,276 -> 1,176; of the 8B shape (36 layers, 32 heads on 8) at 2,048 tokens, 8 requests 3,968 -> 3,879,
-// 64 requests 7,040 -> 6,930: two and a half to three and a half microseconds a layer.
+// 64 requests 7,040 -> 6,930: two and a half to three and a half microseconds a layer.  One wave prepares queries and key for the
+// workgroup (all eight did, and the wave with the new key twice): 1,034 -> 1,000 us, 1,177 -> 1,161, 3,640 -> 3,606; of the 10.5 us that
+// were inside the kernel 2 passed before the keys could be asked for behind that work's loads, 0.7 preparing, 1.3 with the new key alone.
 // MORE: values narrower than keys and a bias by distance (dv and distance are looked at); instances of their own, so that the
 // others are spared the checks.
 template <int D, int WAVES>
 struct DecodeLds {
   float sm_m[WAVES][16], sm_l[WAVES][16];
   __attribute__((aligned(16))) float sm_o[WAVES][16][D + 4];     // a head's dims side by side, heads four banks apart
+  __attribute__((aligned(16))) bf16 queries[16][D + 8];           // prepared heads, four banks apart
   __attribute__((aligned(16))) bf16 own_k[D];
   bf16 own_v[D];
 };
@@ -404,24 +407,26 @@ __device__ __forceinline__ void attention_decode_part(
   // PREP: the raw rows, the norms' weights and the rotation's tables are asked for now, before anything here waits for
   // memory: they are there when the first keys are on their way.  (The new key's and value's by every wave, since which
   // one walks the token's position is not known yet; they are the token's own, whichever workgroup does.)
+  // One wave, the last, does so for the workgroup: eight that all did would ask their compute unit for 160 loads of rows, weights and
+  // tables before the first keys.  The new key is prepared where the queries are, in the column behind the group's heads (a group of 16
+  // leaves none: there it follows them).
   const bf16* q_row = q + (int64_t)token * q_stride;
-  const bool normed = PREP && prep.q_weight, rotated = PREP && prep.cosv;
-  bf16x8 qf[DS], raw_k[DS];
+  const bool normed = PREP && prep.q_weight, rotated = PREP && prep.cosv, brings_key = PREP && prep.kv_columns > 0;
+  const bool prepares = PREP && wave == WAVES - 1, key_column = brings_key && group < 16 && col == group;
+  bf16x8 qf[DS];
   bf16 raw_v[(D + WAVE - 1) / WAVE];
-  HeadWeights<D> q_weights, k_weights;
+  HeadWeights<D> weights;
   HeadTables<D> tables;
+  if (!PREP || prepares) {
+    const bf16* my_row = q_row + (int64_t)(key_column ? nq + kvh : kvh * group + (col < group ? col : 0)) * D + g * 8;
 #pragma unroll
-  for (int c = 0; c < DS; ++c) qf[c] = *(const bf16x8*)(q_row + (int64_t)(kvh * group + (col < group ? col : 0)) * D + c * 32 + g * 8);
-  if constexpr (PREP) {
-    q_weights.fetch(prep.q_weight, prep.weight_is_f32, g);
+    for (int c = 0; c < DS; ++c) qf[c] = *(const bf16x8*)(my_row + c * 32);
+    if (normed) weights.fetch(key_column ? prep.k_weight : prep.q_weight, prep.weight_is_f32, g);
     if (rotated) tables.fetch(prep.cosv + (int64_t)token * (D / 2), prep.sinv + (int64_t)token * (D / 2), g);
-    if (prep.kv_columns > 0) {
-#pragma unroll
-      for (int c = 0; c < DS; ++c) raw_k[c] = *(const bf16x8*)(q_row + (int64_t)(nq + kvh) * D + c * 32 + g * 8);
+    if (brings_key) {
       const bf16* v_row = q_row + (int64_t)(nq + prep.kv_columns + kvh) * D;
 #pragma unroll
       for (int n = 0; n < (D + WAVE - 1) / WAVE; ++n) raw_v[n] = v_row[min(lane + n * WAVE, D - 1)];
-      k_weights.fetch(prep.k_weight, prep.weight_is_f32, g);
     }
   }
 
@@ -440,22 +445,24 @@ __device__ __forceinline__ void attention_decode_part(
   // the (transposed) page, one 16-byte load a dim.  A key or eight keys that the token does not see
   // are read from the nearest it does see, not branched around (three branches were three trips to
   // memory one after the other): their scores are replaced, their values zeroed (work, below).
+  // A tile is two runs of 16 keys, each in one page (pages hold multiples of 16, tiles begin at multiples of 32), so pages are looked up
+  // for runs, with numbers that the whole wave shares; a run that the token does not see stands for the nearest that it does see.
   const int key_of_row = (col >> 2) * 8 + (col & 3);           // + 4*h
+  const int first_run = lo / 16, last_run = pos / 16, page_runs = page_size / 16;
   // A key or value is read by one workgroup, once (load_once; 64 requests at 2,048 tokens, 8B sizes: 6,774 -> 6,618 us a step).  Not in
   // the form of eight waves: its short contexts of a few requests stay in the last-level cache from step to step, which what is
   // loaded with the hint does not (one request at 509 tokens, 0.6B sizes: 1,035 us a step, 1,078 with the hint).
   constexpr bool ONCE = WAVES == 4;
   auto fetch = [&](int tile, bf16x8 (&kf)[2][DS], bf16x8 (&vf)[DB]) {
+    const int run0 = __builtin_amdgcn_readfirstlane(max(first_run, min(last_run, tile * 2)));
+    const int run1 = __builtin_amdgcn_readfirstlane(max(first_run, min(last_run, tile * 2 + 1)));
+    const int block0 = run0 / page_runs, block1 = run1 / page_runs;
+    const int slot0 = (run0 - block0 * page_runs) * 16, slot1 = (run1 - block1 * page_runs) * 16;
+    const int64_t key_page = page_ids[(col < 8 ? block0 : block1) - first_block], value_page = page_ids[(g < 2 ? block0 : block1) - first_block];
     const bf16* kp[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int key = max(lo, min(pos, tile * 32 + key_of_row + 4 * h));
-      const int64_t page = page_ids[key / page_size - first_block];
-      kp[h] = k_pages + ((page * nkv + kvh) * page_size + key % page_size) * D + g * 8;
-    }
-    const int key8 = max(lo & ~7, min(pos & ~7, tile * 32 + g * 8));         // this lane's eight keys; pages hold multiples of 16
-    const int64_t page = page_ids[key8 / page_size - first_block];
-    const bf16* vp = v_pages + (page * nkv + kvh) * (int64_t)dv * page_size + (int64_t)col * page_size + key8 % page_size;
+    kp[0] = k_pages + ((key_page * nkv + kvh) * page_size + (col < 8 ? slot0 : slot1) + key_of_row % 16) * D + g * 8;
+    kp[1] = kp[0] + 4 * D;
+    const bf16* vp = v_pages + (value_page * nkv + kvh) * (int64_t)dv * page_size + (int64_t)col * page_size + (g < 2 ? slot0 : slot1) + g % 2 * 8;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -474,7 +481,7 @@ __device__ __forceinline__ void attention_decode_part(
   if constexpr (AHEAD) {
     fetch(min(tile_begin + wave, max(tile_end - 1, min(tile_begin, last_tile))), (bf16x8(&)[2][DS])kf_a, (bf16x8(&)[DB])vf_a);
   }
-  auto prepare = [&](bf16x8 (&row)[DS], const HeadWeights<D>& weights) {
+  auto prepare = [&](bf16x8 (&row)[DS]) {
     float x[DS][8];
 #pragma unroll
     for (int c = 0; c < DS; ++c)
@@ -482,37 +489,52 @@ __device__ __forceinline__ void attention_decode_part(
       for (int j = 0; j < 8; ++j) x[c][j] = (float)row[c][j];
     head_from_registers<D>(row, x, normed, weights, prep.weight_is_f32, prep.eps, rotated, tables);
   };
-  if constexpr (PREP) prepare(qf, q_weights);
+  // The queries, the new key and the new value meet the waves in LDS; the workgroup that walks the token's own position writes key and
+  // value into the pages, and its wave that meets the position takes them in place of what the pages hold there.
+  auto &own_k = lds.own_k, &own_v = lds.own_v;
+  const bool own_here = brings_key && tile_begin <= last_tile && last_tile < tile_end;
+  const bool holds_own = own_here && (last_tile - tile_begin) % WAVES == wave;
+  if constexpr (PREP) {
+    if (prepares) {
+      prepare(qf);
+      if (col < group)
+#pragma unroll
+        for (int c = 0; c < DS; ++c) *(bf16x8*)&lds.queries[col][c * 32 + g * 8] = qf[c];
+      bool has_key = key_column;
+      if (own_here && group == 16) {
+#pragma unroll
+        for (int c = 0; c < DS; ++c) qf[c] = *(const bf16x8*)(q_row + (int64_t)(nq + kvh) * D + c * 32 + g * 8);
+        if (normed) weights.fetch(prep.k_weight, prep.weight_is_f32, g);
+        prepare(qf);
+        has_key = col == 0;
+      }
+      if (own_here) {
+        if (has_key)
+#pragma unroll
+          for (int c = 0; c < DS; ++c) *(bf16x8*)&own_k[c * 32 + g * 8] = qf[c];
+#pragma unroll
+        for (int n = 0; n < (D + WAVE - 1) / WAVE; ++n)
+          if (lane + n * WAVE < D) own_v[lane + n * WAVE] = raw_v[n];
+      }
+    }
+    __syncthreads();
+    if (prepares && own_here) {
+      const int64_t page = page_ids[pos / page_size - first_block];
+      const int off = pos % page_size;
+      if (page >= 0) {
+        bf16* kdst = k_pages + ((page * nkv + kvh) * page_size + off) * D;
+        bf16* vdst = v_pages + (page * nkv + kvh) * (int64_t)D * page_size + off;
+        if (lane < D / 8) *(bf16x8*)(kdst + lane * 8) = *(const bf16x8*)&own_k[lane * 8];
+#pragma unroll
+        for (int n = 0; n < (D + WAVE - 1) / WAVE; ++n)
+          if (lane + n * WAVE < D) vdst[(int64_t)(lane + n * WAVE) * page_size] = raw_v[n];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < DS; ++c) qf[c] = *(const bf16x8*)&lds.queries[col < group ? col : 0][c * 32 + g * 8];
+  }
 #pragma unroll
   for (int c = 0; c < DS; ++c) qf[c] = col < group ? qf[c] : zero8;
-  // The wave that walks the token's own position prepares the new key, passes it and the new value through LDS of its own
-  // into the fragments when it meets the position (no other wave waits for it), and writes both into the pages.
-  auto &own_k = lds.own_k, &own_v = lds.own_v;
-  const bool holds_own = PREP && prep.kv_columns > 0 && tile_begin <= last_tile && last_tile < tile_end && (last_tile - tile_begin) % WAVES == wave;
-  if (holds_own) {
-    prepare(raw_k, k_weights);
-    const int64_t page = page_ids[pos / page_size - first_block];
-    const int off = pos % page_size;
-    if (col == 0) {
-      bf16* kdst = k_pages + ((page * nkv + kvh) * page_size + off) * D + g * 8;
-#pragma unroll
-      for (int c = 0; c < DS; ++c) {
-        *(bf16x8*)&own_k[c * 32 + g * 8] = raw_k[c];
-        if (page >= 0) *(bf16x8*)(kdst + c * 32) = raw_k[c];
-      }
-    }
-#pragma unroll
-    for (int n = 0; n < (D + WAVE - 1) / WAVE; ++n) {
-      const int i = lane + n * WAVE;
-      if (i < D) {
-        own_v[i] = raw_v[n];
-        if (page >= 0) v_pages[(page * nkv + kvh) * (int64_t)D * page_size + (int64_t)i * page_size + off] = raw_v[n];
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  }
 
   floatx4 o[DB];
 #pragma unroll

@@ -102,3 +102,39 @@ def test_walk_against_64_bits(waves, form, d, splits, window, page):
     changed = (k.cpu() != k_pages).any(-1)
     assert not (changed & ~(k_want != k_pages).any(-1)).any()
     assert ((k.cpu().double() - k_want.double()).abs() <= 2.0 ** -7 * k_want.double().abs()).all()
+
+
+@pytest.mark.parametrize("form", [0, 1, 2])
+@pytest.mark.parametrize("nq,nkv,d,page,window", [(1, 1, 64, 16, 0), (15, 1, 128, 32, 0), (16, 1, 128, 48, 0), (32, 2, 64, 16, 40), (12, 4, 128, 16, 0)])
+def test_new_key_behind_any_number_of_heads(nq, nkv, d, page, window, form):
+    """The new key is prepared in the column behind a kv group's heads, after them where 16 leave none: pages and results against heads
+    and key prepared by qk_prep (the same norm and rotation but for the order of a sum: a last place of bfloat16)."""
+    from llm_runtime_study_amd.kernels import ops
+
+    lengths, splits = [1, 16, 17, 33, 255, 256, 300], 2
+    g = torch.Generator().manual_seed(nq + d)
+    tokens, most = len(lengths), -(-max(lengths) // page)
+    k_pages = torch.randn(tokens * most, nkv, page, d, generator=g).bfloat16().cuda()
+    v_pages = torch.randn(tokens * most, nkv, d, page, generator=g).bfloat16().cuda()
+    table = torch.randperm(tokens * most, generator=g).view(tokens, most).int().cuda()
+    raw = torch.randn(tokens, (nq + 2 * nkv) * d, generator=g).bfloat16().cuda()
+    angle = torch.rand(tokens, d // 2, generator=g) * 6.28
+    cos, sin = angle.cos().cuda(), angle.sin().cuda()
+    q_weight, k_weight = ((1 + 0.3 * torch.randn(d, generator=g)).bfloat16().cuda() for _ in range(2))
+    last = torch.tensor([n - 1 for n in lengths], dtype=torch.int32).cuda()
+    slots = (table[torch.arange(tokens).cuda(), (last // page).long()] * page + last % page).int()
+
+    def run(fused):
+        k, v, rows, out = k_pages.clone(), v_pages.clone(), raw.clone(), torch.full((tokens, nq * d), float("nan"), dtype=torch.bfloat16, device="cuda")
+        if not fused:
+            ops.qk_prep(rows, nq, nkv, d, q_weight, k_weight, 1e-5, cos, sin, k, v, slots, page)
+        ops.attention_decode(out, rows, k, v, table, torch.arange(tokens, dtype=torch.int32).cuda(), last, nq, 1 / math.sqrt(d), window, splits,
+                             torch.empty(tokens * nq * splits * d, device="cuda"), torch.empty(tokens * nq * splits * 2, device="cuda"),
+                             prepare=ops.DecodePrepare(q_weight, k_weight, 1e-5, cos, sin, nkv) if fused else None, form=form)
+        torch.cuda.synchronize()
+        return out.float(), k.float(), v
+
+    got, want = run(True), run(False)
+    assert torch.equal(got[2], want[2]) and not torch.equal(want[1], k_pages.float())
+    torch.testing.assert_close(got[1], want[1], rtol=2 ** -7, atol=1e-6)
+    torch.testing.assert_close(got[0], want[0], rtol=2 ** -6, atol=2 ** -6)
