@@ -396,10 +396,11 @@ __device__ __forceinline__ void attention_decode_part(
   auto& sm_o = lds.sm_o;
   const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
   const int col = lane & 15, g = lane >> 4;
+  const int pos = positions[token], request = token_request[token];
+  asm volatile("" :: "s"(pos), "s"(request));                               // asked for together: the compiler would put the second off
   const int group = nq / nkv;
-  const int pos = positions[token];
+  const int* table = block_table + (int64_t)request * table_stride;
   const int lo = first_seen(pos, window);
-  const int* table = block_table + (int64_t)token_request[token] * table_stride;
   const int first_tile = lo / 32, last_tile = pos / 32;
   const int per_split = (last_tile - first_tile + splits) / splits;
   const int tile_begin = first_tile + split * per_split;
@@ -693,13 +694,13 @@ __device__ __forceinline__ void attention_decode_part(
 
 template <int D, bool PREP, int WAVES, bool AHEAD, bool MORE>
 __global__ __launch_bounds__(WAVES * 64, WAVES == 4 && D == 128 ? 2 : 1) void attention_decode_bf16_kernel(
-    bf16* __restrict__ out, int out_stride, float* __restrict__ part_o, float* __restrict__ part_ml,
-    const bf16* __restrict__ q, int q_stride, bf16* __restrict__ k_pages,
-    bf16* __restrict__ v_pages, const int* __restrict__ block_table, int table_stride,
-    const int* __restrict__ token_request, const int* __restrict__ positions, int nq, int nkv,
-    int page_size, float scale, int window, int splits, int slots, DecodePrep prep, const float* __restrict__ sinks,
-    float softcap, const bf16* __restrict__ gates, int gate_stride, int dv_given, const float* __restrict__ distance_given,
-    int distance_form) {
+    const int* __restrict__ positions, const int* __restrict__ token_request, const int* __restrict__ block_table, const bf16* __restrict__ q,
+    int table_stride, int q_stride, int nq, int nkv, int page_size, int splits, bf16* __restrict__ out, int out_stride,
+    float* __restrict__ part_o, float* __restrict__ part_ml, bf16* __restrict__ k_pages, bf16* __restrict__ v_pages, float scale, int window,
+    int slots, DecodePrep prep, const float* __restrict__ sinks, float softcap, const bf16* __restrict__ gates, int gate_stride, int dv_given,
+    const float* __restrict__ distance_given, int distance_form) {
+  // What leads to the first keys comes first: fourteen words of the arguments are in registers when a wave begins (the file is
+  // compiled so), the others are a trip to memory away.
   __shared__ DecodeLds<D, WAVES> lds;
   extern __shared__ int page_ids[];
   attention_decode_part<D, PREP, WAVES, AHEAD, MORE>(lds, page_ids, blockIdx.x, blockIdx.y, blockIdx.z, out, out_stride, part_o, part_ml, q, q_stride, k_pages, v_pages, block_table, table_stride, token_request, positions, nq, nkv, page_size, scale, window, splits, slots, prep, sinks, softcap, gates, gate_stride, dv_given, distance_given, distance_form);
@@ -936,8 +937,8 @@ LRS_API int lrs_attention_decode(void* out, int out_stride, float* part_o, float
   // `form`: 0 = four waves, a tile at a time; 1 = four waves, 2 = eight waves, each wave with its next
   // tile on the way while it works (heads of 192 dims have no registers for that and stay with 0)
 #define ARGS                                                                                                 \
-  (bf16*)out, out_stride, part_o, part_ml, (const bf16*)q, q_stride, (bf16*)k_pages, (bf16*)v_pages, block_table, \
-      table_stride, token_request, positions, nq, nkv, page_size, scale, window, splits, slots, prep, slots == 1 ? sinks : nullptr, softcap, \
+  positions, token_request, block_table, (const bf16*)q, table_stride, q_stride, nq, nkv, page_size, splits, (bf16*)out, out_stride, part_o, \
+      part_ml, (bf16*)k_pages, (bf16*)v_pages, scale, window, slots, prep, slots == 1 ? sinks : nullptr, softcap, \
       slots == 1 ? (const bf16*)gates : nullptr, gate_stride, dv, distance, distance_form
 #define LAUNCH_PREP(D, PREP, MORE)                                                                           \
   do {                                                                                                       \

@@ -530,11 +530,17 @@ struct NormChain {
 };
 
 
-template <int MT, int RT, int WAVES, int UNROLL, bool NORM, bool SWIGLU, bool PARTIAL = false, bool LINES = false>
+template <int MT, int RT, int WAVES, int UNROLL, bool NORM, bool SWIGLU, bool PARTIAL = false, bool LINES = false, bool SCALED = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(
-    void* __restrict__ out, int mode, const bf16* __restrict__ x, NormInput norm,
-    const bf16* __restrict__ w, const bf16* __restrict__ bias, int m, int n, int k, int lda, int ldc,
-    float* __restrict__ split_sums, NormChain chain, int group_rows) {
+    const bf16* __restrict__ x, const bf16* __restrict__ w, const float* __restrict__ in_sumsq, int m, int n, int k, int lda, int in_parts,
+    int group_rows, void* __restrict__ out, int mode, int ldc, NormInput norm, const bf16* __restrict__ bias, float* __restrict__ split_sums,
+    NormChain chain) {
+  // What the first loads need comes first: fourteen words of the arguments are in registers when a wave begins (the file is
+  // compiled so), the others are a trip to memory away.
+  // Such a kernel is 4-5 us long, of which a trip is nearly one: nothing waits before the weights are asked for, neither for an argument
+  // nor for a load behind a branch (the sums of the norm before were), and those sums are added up while the weights are on their way.
+  // A step of the 0.6B sizes at batch 1 1,000 -> 915 us, at batch 16 1,161 -> 1,089, of the 8B sizes at batch 8 3,606 -> 3,516.
+  // SCALED (with LINES; the other instances look at in_sumsq): the product finishes a norm.
   // RT: row tiles of 16 weight rows per workgroup; every activation fragment is used RT times.
   // group_rows (16 * RT unless PARTIAL): the weight rows a workgroup owns; fewer than its tiles hold
   // when that divides the matrix evenly between the compute units (rows past them are neither
@@ -649,43 +655,66 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(
     return b;
   };
 
+  const int k_splits = LINES ? 1 : (int)gridDim.y;      // (the grid's own size is a trip to memory)
   const int all_steps = (k + 31) / 32;
-  const int per_split = (all_steps + gridDim.y - 1) / gridDim.y;
-  const int split_begin = blockIdx.y * per_split;
+  const int per_split = k_splits == 1 ? all_steps : (all_steps + k_splits - 1) / k_splits;
+  const int split_begin = k_splits == 1 ? 0 : blockIdx.y * per_split;
   const int split_end = split_begin + per_split < all_steps ? split_begin + per_split : all_steps;
   const int per_wave = (per_split + WAVES - 1) / WAVES;
   int s = split_begin + wave * per_wave;
   const int s_end = s + per_wave < split_end ? s + per_wave : split_end;
   const int full_end = k / 32 < s_end ? k / 32 : s_end;   // steps whose 32 k are all inside K
-  // What the epilogue will need from memory is asked for now, before the weights stream, so that it
-  // has long arrived by then: the partial sums of squares of the norm this product finishes, and
-  // the residual values and norm weights of the columns this thread will update.
-  const bool scaled_input = MT == 1 && !NORM && chain.in_sumsq != nullptr;
-  const bool feeds_norm = MT == 1 && !SWIGLU && chain.next_x != nullptr && mode == OUT_ADD_F32 && gridDim.y == 1;
-  constexpr int EARLY = 16;
-  const bool sums_early = scaled_input && chain.in_parts <= WAVES * 4 * EARLY;
+  // The partial sums of squares of the norm that this product finishes are asked for before the weights: they are added up while
+  // those are on their way.
+  const bool scaled_input = LINES ? SCALED : MT == 1 && !NORM && in_sumsq != nullptr;
+  constexpr int EARLY = 80 / WAVES;                              // up to 320 parts, 5,120 columns, at once
   float early_sums[EARLY];
-  if (sums_early) {
-    const int token = tid % 16, part = tid / 16;
+  if (scaled_input) {
+    // (a part or row that is not there stands for the last that is: no branch around a load, which is a wait for all before it)
+    const int token = tid % 16 < m ? tid % 16 : m - 1, part = tid / 16;
 #pragma unroll
     for (int j = 0; j < EARLY; ++j) {
       const int p = part + j * WAVES * 4;
-      early_sums[j] = (token < m && p < chain.in_parts) ? chain.in_sumsq[(int64_t)p * m + token] : 0.f;
+      early_sums[j] = in_sumsq[(p < in_parts ? p : in_parts - 1) * m + token];
     }
   }
-  float early_h[RT], early_w[RT];
-  if (feeds_norm && tid < WAVE * 4) {
-    const int l = tid / 4, i = tid % 4, token = l & 15;
+  bool feeds_norm = false;
+  float early_h[RT];
+  unsigned early_w[RT];                                          // as it is stored
+  // Behind the first weights asked for, once in every wave: the residual values and norm weights of the columns that this thread will
+  // update, and the sums above.
+  auto meanwhile = [&]() {
+    __builtin_amdgcn_sched_barrier(0);                           // nothing that waits for the other arguments before the weights
+    feeds_norm = MT == 1 && !SWIGLU && chain.next_x != nullptr && mode == OUT_ADD_F32 && k_splits == 1;
+    if (feeds_norm) {
+      const int l = tid / 4 % WAVE, i = tid % 4, token = (l & 15) < m ? l & 15 : m - 1;
 #pragma unroll
-    for (int q = 0; q < RT; ++q) {
-      const int gn = n0 + q * 16 + 4 * (l >> 4) + i;
-      const bool inside = token < m && gn < n_end;
-      early_h[q] = inside ? ((const float*)out)[(int64_t)token * ldc + gn] : 0.f;
-      early_w[q] = !inside ? 0.f : chain.next_weight_is_f32 ? ((const float*)chain.next_weight)[gn] : (float)((const bf16*)chain.next_weight)[gn];
+      for (int q = 0; q < RT; ++q) {
+        const int gn = n0 + q * 16 + 4 * (l >> 4) + i, at = gn < n_end ? gn : n_end - 1;
+        early_h[q] = ((const float*)out)[(int64_t)token * ldc + at];
+        if (chain.next_weight_is_f32) early_w[q] = ((const unsigned*)chain.next_weight)[at];
+        else early_w[q] = ((const unsigned short*)chain.next_weight)[at];
+      }
     }
-  }
+    if (scaled_input) {
+      const int token = tid % 16, part = tid / 16;
+      float v = 0.f;
+#pragma unroll
+      for (int j = 0; j < EARLY; ++j) v += part + j * WAVES * 4 < in_parts ? early_sums[j] : 0.f;
+      if (token < m)
+        for (int p = part + EARLY * WAVES * 4; p < in_parts; p += WAVES * 4) v += in_sumsq[(int64_t)p * m + token];
+      chain_parts[part][token] = v;
+      __syncthreads();
+      if (tid < 16) {
+        float q = 0.f;
+#pragma unroll
+        for (int p = 0; p < WAVES * 4; ++p) q += chain_parts[p][tid];
+        chain_scale[tid] = 1.0f / sqrtf(q / (float)k + chain.in_eps);
+      }
+    }
+  };
   // U steps of 32 k, all their loads asked for before any is used
-  auto steps_together = [&](int sb, auto count) {
+  auto steps_together = [&](int sb, auto count, auto&& behind_loads) {
     constexpr int U = decltype(count)::value;
     if constexpr (LINES && U % 4 == 0) {
       static_assert(MT == 1, "whole-line loads are for one block of tokens");
@@ -700,6 +729,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(
         rawb[p][0] = *(const bf16x8*)(xl[0] + (sb + 2 * p) * 32);
         rawb[p][1] = second ? *(const bf16x8*)(xl[1] + (sb + 2 * p) * 32) : zero;
       }
+      behind_loads();
 #pragma unroll
       for (int c4 = 0; c4 < U; c4 += 4) {
         bf16x8 b[4];
@@ -732,6 +762,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int t = 0; t < MT; ++t) b[u][t] = load_b(t, sb + u);
+    behind_loads();
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -744,20 +775,31 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(
   // depends on the column alone): all of them read the same activations, and in step they would
   // all ask the same few cache lines of the L2 at the same moment.
   const int batches = full_end > s ? (full_end - s) / UNROLL : 0;
-  const int s_first = s;
-  for (int j = 0; j < batches; ++j)
-    steps_together(s_first + ((j + (int)blockIdx.x) % batches) * UNROLL, std::integral_constant<int, UNROLL>{});
-  s = s_first + batches * UNROLL;
+  auto nothing = [] {};
+  if (batches > 0) {
+    int at = batches > 1 ? (int)(blockIdx.x % (unsigned)batches) : 0;
+    steps_together(s + at * UNROLL, std::integral_constant<int, UNROLL>{}, meanwhile);
+    for (int j = 1; j < batches; ++j) {
+      at = at + 1 == batches ? 0 : at + 1;
+      steps_together(s + at * UNROLL, std::integral_constant<int, UNROLL>{}, nothing);
+    }
+    s += batches * UNROLL;
+  } else if (UNROLL > 4 && full_end - s >= 4) {
+    steps_together(s, std::integral_constant<int, 4>{}, meanwhile);
+    s += 4;
+  } else {
+    meanwhile();
+  }
   // what is left of the whole steps, in shrinking groups (a step alone costs a trip to memory of its own)
   if constexpr (UNROLL > 4) {
     if (full_end - s >= 4) {
-      steps_together(s, std::integral_constant<int, 4>{});
+      steps_together(s, std::integral_constant<int, 4>{}, nothing);
       s += 4;
     }
   }
   if constexpr (UNROLL > 2) {
     if (full_end - s >= 2) {
-      steps_together(s, std::integral_constant<int, 2>{});
+      steps_together(s, std::integral_constant<int, 2>{}, nothing);
       s += 2;
     }
   }
@@ -782,24 +824,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(
       if (g == 0) sumsq[wave][t][r] = v;
     }
   }
-  if (scaled_input) {
-    const int token = tid % 16, part = tid / 16;
-    float v = 0.f;
-    if (sums_early) {
-#pragma unroll
-      for (int j = 0; j < EARLY; ++j) v += early_sums[j];      // the order of the loop below
-    } else if (token < m) {
-      for (int p = part; p < chain.in_parts; p += WAVES * 4) v += chain.in_sumsq[(int64_t)p * m + token];
-    }
-    chain_parts[part][token] = v;
-    __syncthreads();
-    if (tid < 16) {
-      float q = 0.f;
-#pragma unroll
-      for (int p = 0; p < WAVES * 4; ++p) q += chain_parts[p][tid];
-      chain_scale[tid] = 1.0f / sqrtf(q / (float)k + chain.in_eps);
-    }
-  }
   // accumulator layout: token = t*16 + lane % 16, weight row = tile row 4 * (lane / 16) + i
   auto total = [&](int t, int l, int i) -> float {
     float v = 0.f;
@@ -821,7 +845,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(
     for (int t = 0; t < MT; ++t) partial[wave][t][lane] = acc[q][t];
     __syncthreads();
     const int nq0 = n0 + q * 16;
-    if (gridDim.y > 1) {
+    if (k_splits > 1) {
       for (int e = tid; e < MT * WAVE * 4; e += WAVES * WAVE) {
         const int t = e / (WAVE * 4), l = (e / 4) % WAVE, i = e % 4;
         const int token = t * 16 + (l & 15), gn = nq0 + 4 * (l >> 4) + i;
@@ -847,7 +871,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(
         if (feeds_norm) {                                        // MT == 1: e == tid, the element asked for early
           const float updated = early_h[q] + v;
           ((float*)out)[(int64_t)token * ldc + gn] = updated;
-          chain.next_x[(int64_t)token * n + gn] = (bf16)(updated * early_w[q]);
+          chain.next_x[(int64_t)token * n + gn] = (bf16)(updated * __uint_as_float(chain.next_weight_is_f32 ? early_w[q] : early_w[q] << 16));
           chain_squares[l & 15][q * 16 + 4 * (l >> 4) + i] = updated * updated;
         } else {
           emit<bf16>(out, mode, (int64_t)token * ldc + gn, v);
@@ -1254,6 +1278,18 @@ static bool tune_ok(int word) {
 }
 static GemmTune tune_of(int word) { return GemmTune{(word & 1) != 0, (word & 2) != 0, (word >> 4) & 15, (word >> 8) & 31, (word >> 13) & 3}; }
 
+template <int RT, int WAVES, int UNROLL, bool SWIGLU, bool PARTIAL>
+static void launch_lines(void* out, int mode, const bf16* a, const bf16* w, const bf16* bias, int m, int n, int k, int lda, int ldc, hipStream_t s,
+                         NormChain chain, int group_rows) {
+  const dim3 grid((n + group_rows - 1) / group_rows);
+  if (chain.in_sumsq)
+    gemm_bf16_skinny_kernel<1, RT, WAVES, UNROLL, false, SWIGLU, PARTIAL, true, true><<<grid, WAVES * 64, 0, s>>>(
+        a, w, chain.in_sumsq, m, n, k, lda, chain.in_parts, group_rows, out, mode, ldc, NormInput{}, bias, nullptr, chain);
+  else
+    gemm_bf16_skinny_kernel<1, RT, WAVES, UNROLL, false, SWIGLU, PARTIAL, true><<<grid, WAVES * 64, 0, s>>>(
+        a, w, nullptr, m, n, k, lda, 0, group_rows, out, mode, ldc, NormInput{}, bias, nullptr, chain);
+}
+
 // Row tiles per workgroup: more of them means each activation fragment read from L2 serves more
 // weight rows, which matters once there are several token blocks; fewer means more workgroups.
 template <int MT, int RT, bool NORM, bool SWIGLU>
@@ -1264,22 +1300,22 @@ static void launch_skinny_rt(void* out, int mode, const bf16* a, NormInput norm,
   constexpr int UNROLL = (NORM ? 4 : 8) / (MT * RT > 4 ? 4 : (MT * RT > 1 ? 2 : 1));
   if (group_rows != 16 * RT) {
     if constexpr (MT == 1 && RT == 2 && !NORM && !SWIGLU) {
-      if (tune.lines && splits == 1 && k % 64 == 0 && (k / 32) % 16 == 0 && UNROLL % 4 == 0)
-        gemm_bf16_skinny_kernel<MT, RT, 8, UNROLL, NORM, SWIGLU, true, true><<<dim3(groups, 1), 8 * 64, 0, s>>>(out, mode, a, norm, w, bias, m, n, k, lda, ldc, split_sums, chain, group_rows);
+      if (tune.lines && splits == 1 && k % 64 == 0 && (k / 32) % 16 == 0)
+        launch_lines<RT, 8, UNROLL, SWIGLU, true>(out, mode, a, w, bias, m, n, k, lda, ldc, s, chain, group_rows);
       else
-        gemm_bf16_skinny_kernel<MT, RT, 8, UNROLL, NORM, SWIGLU, true><<<dim3(groups, splits), 8 * 64, 0, s>>>(out, mode, a, norm, w, bias, m, n, k, lda, ldc, split_sums, chain, group_rows);
+        gemm_bf16_skinny_kernel<MT, RT, 8, UNROLL, NORM, SWIGLU, true><<<dim3(groups, splits), 8 * 64, 0, s>>>(a, w, chain.in_sumsq, m, n, k, lda, chain.in_parts, group_rows, out, mode, ldc, norm, bias, split_sums, chain);
     }
   } else if (groups <= 2048) {
     if constexpr (MT == 1 && !NORM && UNROLL % 4 == 0) {
       if (tune.lines && splits == 1 && k % 64 == 0 && (k / 32) % 16 == 0) {   // every wave starts at an even step
-        gemm_bf16_skinny_kernel<MT, RT, 8, UNROLL, NORM, SWIGLU, false, true><<<dim3(groups, 1), 8 * 64, 0, s>>>(out, mode, a, norm, w, bias, m, n, k, lda, ldc, split_sums, chain, group_rows);
+        launch_lines<RT, 8, UNROLL, SWIGLU, false>(out, mode, a, w, bias, m, n, k, lda, ldc, s, chain, group_rows);
         return;
       }
     }
-    gemm_bf16_skinny_kernel<MT, RT, 8, UNROLL, NORM, SWIGLU><<<dim3(groups, splits), 8 * 64, 0, s>>>(out, mode, a, norm, w, bias, m, n, k, lda, ldc, split_sums, chain, group_rows);
+    gemm_bf16_skinny_kernel<MT, RT, 8, UNROLL, NORM, SWIGLU><<<dim3(groups, splits), 8 * 64, 0, s>>>(a, w, chain.in_sumsq, m, n, k, lda, chain.in_parts, group_rows, out, mode, ldc, norm, bias, split_sums, chain);
   }
   else
-    gemm_bf16_skinny_kernel<MT, RT, 4, UNROLL, NORM, SWIGLU><<<dim3(groups, splits), 4 * 64, 0, s>>>(out, mode, a, norm, w, bias, m, n, k, lda, ldc, split_sums, chain, group_rows);
+    gemm_bf16_skinny_kernel<MT, RT, 4, UNROLL, NORM, SWIGLU><<<dim3(groups, splits), 4 * 64, 0, s>>>(a, w, chain.in_sumsq, m, n, k, lda, chain.in_parts, group_rows, out, mode, ldc, norm, bias, split_sums, chain);
   if (splits > 1) {
     const int64_t total = (int64_t)m * (SWIGLU ? n / 2 : n);
     const int blocks = (int)((total + 255) / 256 < 1024 ? (total + 255) / 256 : 1024);
@@ -1542,10 +1578,10 @@ static void launch_skinny(void* out, int mode, const bf16* a, NormInput norm, co
     return;
   }
   if (MT == 1 && !NORM && n >= 16384) {  // measured: two row tiles and four waves stream wide matrices a little faster
-    if (tune.lines && k % 64 == 0 && (k / 32) % 8 == 0)
-      gemm_bf16_skinny_kernel<1, 2, 4, 4, NORM, SWIGLU, false, true><<<dim3((n + 31) / 32, 1), 4 * 64, 0, s>>>(out, mode, a, norm, w, bias, m, n, k, lda, ldc, nullptr, chain, 32);
+    if (!NORM && tune.lines && k % 64 == 0 && (k / 32) % 8 == 0)
+      launch_lines<2, 4, 4, SWIGLU, false>(out, mode, a, w, bias, m, n, k, lda, ldc, s, chain, 32);
     else
-      gemm_bf16_skinny_kernel<1, 2, 4, 4, NORM, SWIGLU><<<dim3((n + 31) / 32, 1), 4 * 64, 0, s>>>(out, mode, a, norm, w, bias, m, n, k, lda, ldc, nullptr, chain, 32);
+      gemm_bf16_skinny_kernel<1, 2, 4, 4, NORM, SWIGLU><<<dim3((n + 31) / 32, 1), 4 * 64, 0, s>>>(a, w, chain.in_sumsq, m, n, k, lda, chain.in_parts, 32, out, mode, ldc, norm, bias, nullptr, chain);
   }
   else if (MT == 1 && !NORM && !SWIGLU && even_group_rows(n) > 0) {
     if constexpr (MT == 1 && !NORM && !SWIGLU)

@@ -1,0 +1,44 @@
+"""Few-rows products that finish a norm: any number of parts of its sum of squares, rows and walks over K."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,k,swiglu", [(256, 512, False), (2048, 1536, True), (6144, 1024, False), (16416, 768, False), (272, 96, False)])
+@pytest.mark.parametrize("m,parts", [(1, 1), (3, 31), (16, 33), (9, 320), (16, 321), (2, 700)])
+def test_sums_of_squares_in_any_number_of_parts(m, parts, n, k, swiglu):
+    """Against 64 bits: the factor is right to 2^-20 whatever the parts (sums of 32 bits over at most 700), a product of K bfloat16 pairs
+    to 2^-20 of the sum of its terms' magnitudes, and the result is rounded to bfloat16 (2^-8; the gated activation twice)."""
+    from llm_runtime_study_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(n + parts + m)
+    x, w = torch.randn(m, k, generator=g).bfloat16(), (torch.randn(n, k, generator=g) * k ** -0.5).bfloat16()
+    sumsq = torch.rand(parts, m, generator=g) * 2 * k / parts
+    out = torch.full((m, n // 2 if swiglu else n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ops.gemm_norm_chain(out, x.cuda(), w.cuda(), swiglu=swiglu, in_sumsq=sumsq.cuda(), in_eps=1e-6)
+    factor = 1.0 / (sumsq.double().sum(0) / k + 1e-6).sqrt()
+    want = x.double() @ w.double().T * factor[:, None]
+    if swiglu:
+        pairs = want.view(m, n // 16, 2, 8)
+        gate, up = pairs[:, :, 0].reshape(m, -1), pairs[:, :, 1].reshape(m, -1)
+        want = gate * torch.sigmoid(gate) * up
+    torch.testing.assert_close(out.cpu().double(), want, rtol=2 ** -8 + 2 ** -18, atol=2 ** -14)
+
+
+@pytest.mark.parametrize("m,n,k,weight_dtype", [(1, 1024, 2048, torch.bfloat16), (16, 1024, 3072, torch.float32), (5, 512, 512, torch.bfloat16), (8, 40, 256, torch.float32)])
+def test_product_that_begins_the_next_norm(m, n, k, weight_dtype):
+    """The residual stream, the weighted row and the sums of squares that a product leaves, against 64 bits of the same values."""
+    from llm_runtime_study_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(n + k + m)
+    x, w = torch.randn(m, k, generator=g).bfloat16(), (torch.randn(n, k, generator=g) * k ** -0.5).bfloat16()
+    h, weight = torch.randn(m, n, generator=g), (1 + 0.3 * torch.randn(n, generator=g)).to(weight_dtype)
+    stream, next_x = h.cuda(), torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    sums = torch.full((ops.norm_chain_parts(n), m), float("nan"), device="cuda")
+    ops.gemm_norm_chain(stream, x.cuda(), w.cuda(), accumulate=True, next_x=next_x, next_sumsq=sums, next_weight=weight.cuda())
+    want = h.double() + x.double() @ w.double().T
+    torch.testing.assert_close(stream.cpu().double(), want, rtol=2 ** -18, atol=2 ** -16)
+    torch.testing.assert_close(next_x.cpu().double(), want * weight.double(), rtol=2 ** -8, atol=2 ** -14)
+    torch.testing.assert_close(sums.cpu().double().sum(0), want.pow(2).sum(1), rtol=2 ** -16, atol=0.0)
