@@ -55,9 +55,10 @@ __device__ __forceinline__ void add_odd_values(floatx4 values, floatx4 weights, 
 // request should they not all belong to one.
 template <int D, int WAVES, bool SHORT>
 __global__ __launch_bounds__(WAVES * WAVE, WAVES == 8 ? 1 : 2) void attention_f32_mfma_kernel(
-    float* __restrict__ out, int out_stride, const float* __restrict__ q, int q_stride, const float* __restrict__ k_pages,
-    const float* __restrict__ v_pages, const int* __restrict__ block_table, int table_stride, const int* __restrict__ token_request,
-    const int* __restrict__ positions, int tokens, int heads, int nkv, int page_size, float scale, int window, int together) {
+    const int* __restrict__ positions, const int* __restrict__ token_request, const int* __restrict__ block_table, const float* __restrict__ q,
+    int table_stride, int q_stride, int tokens, int together, int heads, int groups, const float* __restrict__ k_pages,
+    const float* __restrict__ v_pages, float* __restrict__ out, int out_stride, int nkv, int page_size, float scale, int window) {
+  // (what leads to the first keys comes first: those arguments are in registers when a wave begins, the file is compiled so)
   constexpr int PITCH = D + 4, TILES = D / 16;   // floats from column to column of a partial result; its tiles of 16 dims
   extern __shared__ __attribute__((aligned(16))) float parts[];           // [WAVES][columns][PITCH], then maxima and sums [WAVES][16][2]
   const int columns = together * heads;
@@ -66,7 +67,7 @@ __global__ __launch_bounds__(WAVES * WAVE, WAVES == 8 ? 1 : 2) void attention_f3
   const int r = lane & 15, g = lane >> 4;
   const int kv_head = blockIdx.y;
   // the last tokens of a prompt, which see most, begin first
-  const int begin = ((int)gridDim.x - 1 - (int)blockIdx.x) * together, end = begin + together < tokens ? begin + together : tokens;
+  const int begin = (groups - 1 - (int)blockIdx.x) * together, end = begin + together < tokens ? begin + together : tokens;
   const unsigned key_lane = (unsigned)(r * D + 4 * g), value_lane = (unsigned)(r * page_size + 4 * g);     // floats from a block's first
   const int my_token = begin + r / heads;                                  // of this lane's column
   // the thread that merges: column and four dims
@@ -218,7 +219,8 @@ void launch(float* out, int out_stride, const float* q, int q_stride, const floa
   const dim3 grid((tokens + together - 1) / together, nkv);
   const int columns = together * heads;
   attention_f32_mfma_kernel<D, WAVES, SHORT><<<grid, WAVES * WAVE, sizeof(float) * WAVES * (columns * (D + 4) + COLUMNS * 2), s>>>(
-      out, out_stride, q, q_stride, k_pages, v_pages, block_table, table_stride, token_request, positions, tokens, heads, nkv, page_size, scale, window, together);
+      positions, token_request, block_table, q, table_stride, q_stride, tokens, together, heads, (int)grid.x, k_pages, v_pages, out, out_stride, nkv, page_size,
+      scale, window);
 }
 
 }  // namespace

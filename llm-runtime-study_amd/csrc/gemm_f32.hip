@@ -27,9 +27,10 @@ __device__ __forceinline__ void fetch_from(uint64_t base, unsigned lane_offset, 
 // WR, AR: 8 where a tile has only 8 rows of weights or inputs to bring (its other outputs are copies that nobody stores).
 // A wave's fragment of the weights is the instruction's first operand: its lanes end with four consecutive output columns.
 template <int BK, int WN, int WM, int TN, int TM, int STAGES, int WR, int AR>
-__global__ __launch_bounds__(WN * WM * WAVE) void gemm_f32_mfma_kernel(float* __restrict__ out, int add, const float* __restrict__ a,
-                                                                       const float* __restrict__ w, const float* __restrict__ bias, int m,
-                                                                       int n, int k, int lda, int ldc, int tiles_m, int wide_stores) {
+__global__ __launch_bounds__(WN * WM * WAVE) void gemm_f32_mfma_kernel(const float* __restrict__ a, const float* __restrict__ w, int m, int n, int k,
+                                                                       int lda, int tiles_m, int tiles, float* __restrict__ out, int add, int ldc,
+                                                                       const float* __restrict__ bias, int wide_stores) {
+  // (the arguments that lead to the first fetches come first: they are in registers when a wave begins, the file is compiled so)
   static_assert((BK == 32 || BK == 64) && (WR == 8 || WR == 16) && (AR == 8 || AR == 16), "what the layout is made for");
   constexpr int WAVES = WN * WM, BN = WN * TN * WR, BM = WM * TM * AR;
   constexpr int CHUNKS = BK / 4;                                           // a row's pieces of 16 bytes
@@ -39,7 +40,7 @@ __global__ __launch_bounds__(WN * WM * WAVE) void gemm_f32_mfma_kernel(float* __
   __shared__ __attribute__((aligned(128))) float slices[STAGES * STAGE];
   const int tid = threadIdx.x, lane = tid % WAVE, wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / WAVE);
   int id = blockIdx.x;
-  if (gridDim.x % 8 == 0) id = (id % 8) * (gridDim.x / 8) + id / 8;        // an XCD takes neighbouring weight rows, which it then reads once
+  if (tiles % 8 == 0) id = (id % 8) * (tiles / 8) + id / 8;        // an XCD takes neighbouring weight rows, which it then reads once
   const int m0 = (id % tiles_m) * BM, n0 = (id / tiles_m) * BN;
   unsigned offset[EACH];
 #pragma unroll
@@ -178,7 +179,7 @@ int lrs_gemm_f32(float* out, bool add, const float* a, const float* w, const flo
   do {                                                                                                                             \
     const int tiles_m = (m + WM * TM * AR - 1) / (WM * TM * AR), tiles_n = (n + WN * TN * WR - 1) / (WN * TN * WR);                \
     gemm_f32_mfma_kernel<BK, WN, WM, TN, TM, STAGES, WR, AR><<<tiles_m * tiles_n, WN * WM * WAVE, 0, s>>>(                         \
-        out, add, a, w, bias, m, n, k, lda, ldc, tiles_m, wide_stores);                                                            \
+        a, w, m, n, k, lda, tiles_m, tiles_m * tiles_n, out, add, ldc, bias, wide_stores);                                                         \
   } while (0)
   if (m <= 16) {
     // Few rows: memory and the chains bound it.  As many workgroups as there are tiles of 16 weight rows, of 8 where those are

@@ -31,10 +31,10 @@ FLAGS = [f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-fvisibility=h
 # Sources with flags of their own.  latent.hip: matrix products leave their sums in vector registers, not in accumulation registers, which a
 # running softmax that rescales some 128 of them at most tiles would read and write back one by one (a prompt of 2,048 tokens 355 us a layer
 # for 451, of the kernel of waves by themselves 1,418 for 1,530).
-# gemm.hip, attention.hip: the first words of a kernel's arguments (fourteen, in the order of its parameters, up to the first that is a structure)
+# ARGUMENTS_IN_REGISTERS: the first words of a kernel's arguments (fourteen, in the order of its parameters, up to the first that is a structure)
 # are in registers when a wave begins, instead of a trip to memory away.
 ARGUMENTS_IN_REGISTERS = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
-FILE_FLAGS = {"gemm.hip": ARGUMENTS_IN_REGISTERS, "attention.hip": ARGUMENTS_IN_REGISTERS, "latent.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+FILE_FLAGS = {**{name: ARGUMENTS_IN_REGISTERS for name in ("gemm.hip", "attention.hip", "elementwise.hip", "gemm_f32.hip", "attention_f32.hip")}, "latent.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
               "delta_chunks.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 # the vendor's matrix library, for bfloat16 products of many rows (csrc/library_gemm.hip)
 ROCM_LIB = Path(os.environ.get("ROCM_PATH", "/opt/rocm")) / "lib"

@@ -42,3 +42,30 @@ def test_product_that_begins_the_next_norm(m, n, k, weight_dtype):
     torch.testing.assert_close(stream.cpu().double(), want, rtol=2 ** -18, atol=2 ** -16)
     torch.testing.assert_close(next_x.cpu().double(), want * weight.double(), rtol=2 ** -8, atol=2 ** -14)
     torch.testing.assert_close(sums.cpu().double().sum(0), want.pow(2).sum(1), rtol=2 ** -16, atol=0.0)
+
+
+@pytest.mark.parametrize("hidden", [4, 252, 256, 260, 1020, 1024, 1028, 4096, 4100, 8192])
+@pytest.mark.parametrize("weight_dtype,out_dtype", [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32), (torch.bfloat16, torch.float32)])
+def test_norms_of_rows_of_any_length(hidden, weight_dtype, out_dtype):
+    """Rows that end inside, at and behind the last chunk a thread owns: plain, gathered, and with a product's output added first (which
+    the stream keeps).  Against 64 bits: a sum of `hidden` squares in 32 bits, then the output's own rounding."""
+    from llm_runtime_study_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(hidden)
+    x, y = torch.randn(7, hidden, generator=g) * 3, torch.randn(7, hidden, generator=g).bfloat16()
+    weight, rows = (1 + 0.3 * torch.randn(hidden, generator=g)).to(weight_dtype), torch.tensor([6, 0, 0, 3], dtype=torch.int32)
+    near = dict(rtol=2 ** -8 if out_dtype == torch.bfloat16 else 2 ** -18, atol=2 ** -20)
+
+    def normed(v):
+        return v / (v.pow(2).mean(1, keepdim=True) + 1e-6).sqrt() * weight.double()
+
+    stream, out = x.cuda(), torch.full((7, hidden), float("nan"), dtype=out_dtype, device="cuda")
+    ops.rmsnorm(out, stream, weight.cuda(), 1e-6)
+    torch.testing.assert_close(out.cpu().double(), normed(x.double()), **near)
+    assert torch.equal(stream.cpu(), x)
+    gathered = torch.full((4, hidden), float("nan"), dtype=out_dtype, device="cuda")
+    ops.rmsnorm(gathered, stream, weight.cuda(), 1e-6, rows=rows.cuda())
+    assert torch.equal(gathered, out[rows.long().cuda()])
+    ops.add_rmsnorm(out, stream, y.cuda(), weight.cuda(), 1e-6)
+    assert torch.equal(stream.cpu(), x + y.float())
+    torch.testing.assert_close(out.cpu().double(), normed((x + y.float()).double()), **near)
