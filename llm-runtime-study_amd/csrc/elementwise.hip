@@ -169,29 +169,32 @@ LRS_API int lrs_rmsnorm(void* out, int out_dtype, const float* x, const void* we
 constexpr int NORM_BEGIN_COLUMNS = 1024;
 template <typename TW>
 __global__ __launch_bounds__(NORM_BEGIN_COLUMNS / 4) void split_add_norm_begin_kernel(
-    float* __restrict__ x, const float* __restrict__ sums, int splits, const TW* __restrict__ weight,
-    bf16* __restrict__ next_x, float* __restrict__ next_sumsq, int hidden) {
+    float* __restrict__ x, const float* __restrict__ sums, const TW* __restrict__ weight, int splits, int hidden, int rows,
+    bf16* __restrict__ next_x, float* __restrict__ next_sumsq) {
   __shared__ float scratch[16];
-  const int row = blockIdx.y, rows = gridDim.y, c = (blockIdx.x * (NORM_BEGIN_COLUMNS / 4) + threadIdx.x) * 4;
+  const int row = blockIdx.y, c = (blockIdx.x * (NORM_BEGIN_COLUMNS / 4) + threadIdx.x) * 4;
   float ss = 0.f;
   if (c < hidden) {
     const int64_t at = (int64_t)row * hidden + c;
     floatx4 v = *(const floatx4*)(x + at);
+    TW wc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) wc[i] = weight[c + i];
     floatx4 y = floatx4{0.f, 0.f, 0.f, 0.f};
     for (int sp0 = 0; sp0 < splits; sp0 += 8) {       // eight splits asked for at a time (usually all there are)
       floatx4 part[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i)
-        part[i] = sp0 + i < splits ? *(const floatx4*)(sums + ((int64_t)(sp0 + i) * rows) * hidden + at) : floatx4{0.f, 0.f, 0.f, 0.f};
+        part[i] = *(const floatx4*)(sums + ((int64_t)(sp0 + i < splits ? sp0 + i : splits - 1) * rows) * hidden + at);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) y += part[i];
+      for (int i = 0; i < 8; ++i) y += sp0 + i < splits ? part[i] : floatx4{0.f, 0.f, 0.f, 0.f};
     }
     v += y;
     *(floatx4*)(x + at) = v;
     bf16x4 nx;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      nx[i] = (bf16)(v[i] * to_float(weight[c + i]));
+      nx[i] = (bf16)(v[i] * to_float(wc[i]));
       ss += v[i] * v[i];
     }
     *(bf16x4*)(next_x + at) = nx;
@@ -211,8 +214,8 @@ LRS_API int lrs_split_add_norm_begin(float* x, const float* sums, int splits, co
   const dim3 grid(lrs_norm_begin_parts(hidden), n_rows);
   constexpr int threads = NORM_BEGIN_COLUMNS / 4;
   hipStream_t s = (hipStream_t)stream;
-  if (w_dtype == LRS_F32) split_add_norm_begin_kernel<float><<<grid, threads, 0, s>>>(x, sums, splits, (const float*)weight, (bf16*)next_x, next_sumsq, hidden);
-  else if (w_dtype == LRS_BF16) split_add_norm_begin_kernel<bf16><<<grid, threads, 0, s>>>(x, sums, splits, (const bf16*)weight, (bf16*)next_x, next_sumsq, hidden);
+  if (w_dtype == LRS_F32) split_add_norm_begin_kernel<float><<<grid, threads, 0, s>>>(x, sums, (const float*)weight, splits, hidden, n_rows, (bf16*)next_x, next_sumsq);
+  else if (w_dtype == LRS_BF16) split_add_norm_begin_kernel<bf16><<<grid, threads, 0, s>>>(x, sums, (const bf16*)weight, splits, hidden, n_rows, (bf16*)next_x, next_sumsq);
   else return lrs_fail("split_add_norm_begin: unknown weight dtype %d", w_dtype);
   return lrs_check_launch("split_add_norm_begin");
 }

@@ -954,8 +954,13 @@ struct MidScale {
 // first MT waves.
 template <int MT, int WAVES, bool SWIGLU, bool EXTRA = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_mid_kernel(
-    void* __restrict__ out, int mode, const bf16* __restrict__ x, const bf16* __restrict__ w,
-    int m, int n, int k, int lda, int ldc, float* __restrict__ split_sums, MidScale scale, int extras) {
+    const bf16* __restrict__ x, const bf16* __restrict__ w, const float* __restrict__ sumsq, int m, int n, int k, int lda, int per_split, int extras,
+    int parts, float eps, void* __restrict__ out, int mode, int ldc, float* __restrict__ split_sums) {
+  // The arguments that lead to the first loads come first (they are in registers when a wave begins, see gemm_bf16_skinny_kernel).  With
+  // that, the norm's sums behind the first weights and no branch before those, a layer's four products take, in us before -> after (whole
+  // lines loaded with the hint among it): 0.6B sizes 20 rows 35.5 -> 30.8, 64 rows 41.8 -> 38.4, 8B sizes 20 rows 91.8 -> 82.9, 64 rows
+  // 104.3 -> 99.3, 100 rows 134 -> 125.
+  // per_split: slices of 256 k a workgroup of the grid's y takes.  sumsq, parts, eps: see MidScale.
   static_assert(!EXTRA || ((WAVES == 4 || WAVES == 6 || WAVES == 8) && MT <= 4), "the extra tile needs 4, 6 or 8 waves and at most 64 rows");
   constexpr int STEPS = 8;                         // k steps of 32 in a slice
   constexpr int XS = EXTRA ? (STEPS + WAVES - 1) / WAVES : 1;    // most steps of the extra tile that a wave multiplies in a slice
@@ -985,7 +990,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_mid_kernel(
     rd_off[h] = spot_of(h, r, g);
   }
   const int slices = k / 256;
-  const int per_split = (slices + gridDim.y - 1) / gridDim.y;
   const int s0 = blockIdx.y * per_split;
   const int count = (s0 + per_split < slices ? s0 + per_split : slices) - s0;
   // Workgroups walk their slices from different starting points (round the ring): all of them read the
@@ -1021,20 +1025,24 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_mid_kernel(
     xp[i] = x + (int64_t)(tok < m ? tok : m - 1) * lda + chunk * 8;
     spot[i] = lds + place(chunk / 4, tok / 16, tok % 16, chunk % 4);
   }
-  // the factors of a norm begun before this product: one thread a token adds up the parts now (the loads run
-  // beside the weights') and keeps the factor; after the last slice they go through LDS to the lanes that need them
-  float my_scale = 1.f;
-  if (scale.sumsq && tid < m) {
-    float q = 0.f;
-    for (int p0 = 0; p0 < scale.parts; p0 += 8) {      // eight parts asked for at a time (usually all there are)
-      float part[8];
+  // the factors of a norm begun before this product: one thread a token adds up the parts, which are asked for before the weights (without
+  // a branch, so that nothing waits for them there; without a norm the same loads bring some input) and added up behind the first of them;
+  // after the last slice the factors go through LDS to the lanes that need them
+  constexpr int AT_ONCE = 8;
+  float early[AT_ONCE], my_scale = 1.f;
+  {
+    const float* from = (sumsq ? sumsq : (const float*)x) + (tid < m ? tid : m - 1);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) part[j] = p0 + j < scale.parts ? scale.sumsq[(int64_t)(p0 + j) * m + tid] : 0.f;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) q += part[j];
-    }
-    my_scale = 1.0f / sqrtf(q / (float)k + scale.eps);
+    for (int j = 0; j < AT_ONCE; ++j) early[j] = from[(j < parts ? j : parts > 0 ? parts - 1 : 0) * m];
   }
+  auto add_up = [&]() {
+    float q = 0.f;
+#pragma unroll
+    for (int j = 0; j < AT_ONCE; ++j) q += j < parts ? early[j] : 0.f;
+    if (sumsq && tid < m)
+      for (int p = AT_ONCE; p < parts; ++p) q += sumsq[(int64_t)p * m + tid];
+    my_scale = 1.0f / sqrtf(q / (float)k + eps);
+  };
   floatx4 acc[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -1129,20 +1137,20 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_mid_kernel(
   // set (slice c + 2) beyond, where registers are short.
   // (six waves with an extra tile at 64 rows have no registers for the second set either)
   constexpr bool TWO_SETS = MT <= 4 && !(EXTRA && WAVES == 6 && MT == 4);
+  // (the first loads are made whatever `count` is: behind branches they are waited for one after the other; a slice that is not there
+  // stands for the last that is)
+  auto there = [&](int c) -> int { return count > 0 ? slice_at(c < count ? c : count - 1) : slices - 1; };
   int c = 0;
   if constexpr (TWO_SETS) {
-    if (count > 0) {
-      load_w(slice_at(0), wa);
-      load_x(slice_at(0), xa);
-      load_acts(slice_at(0), sa);
-    }
-    if (count > 1) {
-      load_w(slice_at(1), wb);
-      load_x(slice_at(1), xb);
-      load_acts(slice_at(1), sb);
-    }
-    if (count > 0) store_acts(0, sa);
-    if (count > 2) load_acts(slice_at(2), sa);
+    load_w(there(0), wa);
+    load_x(there(0), xa);
+    load_acts(there(0), sa);
+    load_w(there(1), wb);
+    load_x(there(1), xb);
+    load_acts(there(1), sb);
+    add_up();
+    store_acts(0, sa);
+    load_acts(there(2), sa);
     // slice c: after the barrier LDS buffer c & 1 holds it and nobody reads the other buffer any more
     auto steady = [&](int c, bf16x8 (&a)[STEPS], bf16x8 (&xf)[XS], bf16x8 (&st)[MINE]) {
       __syncthreads();
@@ -1167,17 +1175,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_mid_kernel(
       ending(c + 1, wb, xb, sa);
     }
   } else {
-    if (count > 0) {
-      load_w(slice_at(0), wa);
-      load_x(slice_at(0), xa);
-      load_acts(slice_at(0), sa);
-    }
-    if (count > 1) {
-      load_w(slice_at(1), wb);
-      load_x(slice_at(1), xb);
-    }
-    if (count > 0) store_acts(0, sa);
-    if (count > 1) load_acts(slice_at(1), sa);
+    load_w(there(0), wa);
+    load_x(there(0), xa);
+    load_acts(there(0), sa);
+    load_w(there(1), wb);
+    load_x(there(1), xb);
+    add_up();
+    store_acts(0, sa);
+    load_acts(there(1), sa);
     auto steady = [&](int c, bf16x8 (&a)[STEPS], bf16x8 (&xf)[XS]) {
       __syncthreads();
       store_acts((c & 1) ^ 1, sa);                       // slice c + 1
@@ -1205,7 +1210,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_mid_kernel(
     }
   }
   // accumulator layout: token = t * 16 + lane % 16, weight rows row0 + 4 * (lane / 16) + 0..3
-  if (scale.sumsq) {
+  if (sumsq) {
     float* const row_scales = (float*)mid_lds;     // the activation buffers have done their work
     __syncthreads();
     if (tid < m) row_scales[tid] = my_scale;
@@ -1249,7 +1254,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_mid_kernel(
       if (wave < MT) {
         floatx4 v = meet[wave * WAVE + lane];
         for (int other = 1; other < WAVES; ++other) v += meet[(other * MT + wave) * WAVE + lane];
-        if (scale.sumsq) v *= ((const float*)mid_lds)[wave * 16 + r < m ? wave * 16 + r : 0];
+        if (sumsq) v *= ((const float*)mid_lds)[wave * 16 + r < m ? wave * 16 + r : 0];
         emit_block(wave, v, row_x);
       }
     }
@@ -1530,7 +1535,8 @@ static int launch_mid_mt(void* out, int mode, const bf16* a, const bf16* w, int 
       (void)hipFuncSetAttribute((const void*)gemm_bf16_mid_kernel<MT, WV, SWIGLU, EXTRA>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes); \
       asked = true;                                                                                                 \
     }                                                                                                               \
-    gemm_bf16_mid_kernel<MT, WV, SWIGLU, EXTRA><<<grid, WV * 64, bytes, s>>>(out, mode, a, w, m, n, k, lda, ldc, sums, scale, extras);    \
+    gemm_bf16_mid_kernel<MT, WV, SWIGLU, EXTRA><<<grid, WV * 64, bytes, s>>>(a, w, scale.sumsq, m, n, k, lda, (k / 256 + (int)grid.y - 1) / (int)grid.y, \
+                                                                              extras, scale.parts, scale.eps, out, mode, ldc, sums);        \
   } while (0)
   if constexpr (MT <= 4) {
     if (even && waves == 4) MID_LAUNCH(4, true);

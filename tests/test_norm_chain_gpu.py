@@ -69,3 +69,23 @@ def test_norms_of_rows_of_any_length(hidden, weight_dtype, out_dtype):
     ops.add_rmsnorm(out, stream, y.cuda(), weight.cuda(), 1e-6)
     assert torch.equal(stream.cpu(), x + y.float())
     torch.testing.assert_close(out.cpu().double(), normed((x + y.float()).double()), **near)
+
+
+@pytest.mark.parametrize("k", [256, 512, 768, 1280, 2304])
+@pytest.mark.parametrize("m,splits,waves", [(17, 1, 4), (33, 2, 8), (64, 4, 4), (64, 8, 6), (100, 3, 5), (128, 16, 8)])
+def test_slices_left_to_a_workgroup_of_17_to_128_rows(m, splits, waves, k):
+    """K splits whose workgroups have no slice of 256, one, and a few: against 64 bits (sums of 32 bits, then the output's rounding)."""
+    from llm_runtime_study_amd.kernels import ops
+
+    n = 96
+    g = torch.Generator().manual_seed(m + k)
+    x, w = torch.randn(m, k, generator=g).bfloat16(), (torch.randn(n, k, generator=g) * k ** -0.5).bfloat16()
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ops.gemm(out, x.cuda(), w.cuda(), choice=ops.KernelChoice(mid_splits=splits, mid_waves=waves))
+    torch.testing.assert_close(out.cpu().double(), x.double() @ w.double().T, rtol=2 ** -8, atol=2 ** -14)
+    parts = 11
+    sumsq = torch.rand(parts, m, generator=g) * 2 * k / parts
+    if splits == 1:
+        ops.gemm_mid_scaled(out, x.cuda(), w.cuda(), sumsq.cuda(), 1e-6, choice=ops.KernelChoice(mid_splits=splits, mid_waves=waves))
+        want = x.double() @ w.double().T / (sumsq.double().sum(0) / k + 1e-6).sqrt()[:, None]
+        torch.testing.assert_close(out.cpu().double(), want, rtol=2 ** -8 + 2 ** -18, atol=2 ** -14)
