@@ -181,15 +181,17 @@ __device__ __forceinline__ void route_token_scores(const float* __restrict__ log
       }
     const float w = __shfl(own, where % WAVE, WAVE);
     total += w;
-    chosen[k / WAVE] = lane == k % WAVE ? where : chosen[k / WAVE];
-    share[k / WAVE] = lane == k % WAVE ? w : share[k / WAVE];
+    if (lane == 0) {
+      ids[(int64_t)t * top + k] = where;
+      weights[(int64_t)t * top + k] = w;
+    }
   }
-#pragma unroll
-  for (int c = 0; c < ROUTE_MAX_PER_LANE; ++c) {
-    const int k = lane + WAVE * c;
-    if (k >= top) continue;
-    ids[(int64_t)t * top + k] = chosen[c];
-    weights[(int64_t)t * top + k] = rule.kind >= ROUTE_SIGMOID_SCORES ? (rule.scale != 1.f ? share[c] * rule.scale : share[c]) : share[c] / (total + 1e-20f) * rule.scale;
+  // the same lane wrote them: it reads its own stores
+  if (lane == 0 && rule.kind >= ROUTE_SIGMOID_SCORES) {
+    if (rule.scale != 1.f)
+      for (int k = 0; k < top; ++k) weights[(int64_t)t * top + k] *= rule.scale;
+  } else if (lane == 0) {
+    for (int k = 0; k < top; ++k) weights[(int64_t)t * top + k] = weights[(int64_t)t * top + k] / (total + 1e-20f) * rule.scale;
   }
 }
 
