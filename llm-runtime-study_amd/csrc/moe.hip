@@ -22,12 +22,27 @@ namespace {
 
 constexpr int ROUTE_MAX_PER_LANE = 8;     // experts up to 64 * 8
 
-// One token by one wave.
+// The largest of a wave's values, by moves between neighbouring lanes (six through LDS take several times as long, and a choice of eight
+// experts in four groups of eight needs fifty such searches one after the other).
+__device__ __forceinline__ float lanes_max(float v) {
+#define STEP(CONTROL) v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CONTROL, 0xf, 0xf, false)))
+  STEP(0x111);       // the lane before, 2, 4 and 8 before, of its row of 16: the row's last lane then holds the row's largest
+  STEP(0x112);
+  STEP(0x114);
+  STEP(0x118);
+  STEP(0x142);       // the last lane of the row before, then of the half before
+  STEP(0x143);
+#undef STEP
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), WAVE - 1));
+}
+
+// One token by one wave; PER_LANE: experts a lane looks after.
+template <int PER_LANE>
 __device__ __forceinline__ void route_token(const float* __restrict__ logits, int ld, const float* __restrict__ bias,
                                             int* ids, float* __restrict__ weights, int t, int experts, int top, int lane) {
-  float v[ROUTE_MAX_PER_LANE];
+  float v[PER_LANE];
 #pragma unroll
-  for (int c = 0; c < ROUTE_MAX_PER_LANE; ++c) {
+  for (int c = 0; c < PER_LANE; ++c) {
     const int e = lane + WAVE * c;
     v[c] = e < experts ? logits[(int64_t)t * ld + e] + (bias ? bias[e] : 0.f) : -INFINITY;
   }
@@ -36,17 +51,17 @@ __device__ __forceinline__ void route_token(const float* __restrict__ logits, in
   for (int k = 0; k < top; ++k) {
     float best = -INFINITY;
 #pragma unroll
-    for (int c = 0; c < ROUTE_MAX_PER_LANE; ++c) best = fmaxf(best, v[c]);
-    best = wave_max(best);
+    for (int c = 0; c < PER_LANE; ++c) best = fmaxf(best, v[c]);
+    best = lanes_max(best);
     int where = 1 << 30;
 #pragma unroll
-    for (int c = ROUTE_MAX_PER_LANE - 1; c >= 0; --c)
-      if (v[c] == best) where = lane + WAVE * c;
-#pragma unroll
-    for (int off = WAVE / 2; off > 0; off >>= 1) where = min(where, __shfl_xor(where, off, WAVE));
+    for (int c = PER_LANE - 1; c >= 0; --c) {
+      const unsigned long long there = __ballot(v[c] == best);
+      if (there) where = WAVE * c + __ffsll(there) - 1;
+    }
     if (where >= experts) where = k;    // logits that are not numbers: any expert, never an index outside the table
 #pragma unroll
-    for (int c = 0; c < ROUTE_MAX_PER_LANE; ++c)
+    for (int c = 0; c < PER_LANE; ++c)
       if (lane + WAVE * c == where) v[c] = -INFINITY;
     if (k == 0) first = best;
     const float w = expf(best - first);
@@ -85,29 +100,32 @@ struct RouteRule {
 };
 
 // The lowest index among the lanes' elements that equal `best` (1 << 30 if none).
-__device__ __forceinline__ int route_where(const float (&v)[ROUTE_MAX_PER_LANE], float best, int lane) {
+template <int PER_LANE>
+__device__ __forceinline__ int route_where(const float (&v)[PER_LANE], float best) {
   int where = 1 << 30;
 #pragma unroll
-  for (int c = ROUTE_MAX_PER_LANE - 1; c >= 0; --c)
-    if (v[c] == best) where = lane + WAVE * c;
-#pragma unroll
-  for (int off = WAVE / 2; off > 0; off >>= 1) where = min(where, __shfl_xor(where, off, WAVE));
+  for (int c = PER_LANE - 1; c >= 0; --c) {
+    const unsigned long long there = __ballot(v[c] == best);
+    if (there) where = WAVE * c + __ffsll(there) - 1;
+  }
   return where;
 }
-__device__ __forceinline__ float route_max(const float (&v)[ROUTE_MAX_PER_LANE]) {
+template <int PER_LANE>
+__device__ __forceinline__ float route_max(const float (&v)[PER_LANE]) {
   float best = -INFINITY;
 #pragma unroll
-  for (int c = 0; c < ROUTE_MAX_PER_LANE; ++c) best = fmaxf(best, v[c]);
-  return wave_max(best);
+  for (int c = 0; c < PER_LANE; ++c) best = fmaxf(best, v[c]);
+  return lanes_max(best);
 }
 
 // One token by one wave: every rule that chooses by scores of all experts.
+template <int PER_LANE>
 __device__ __forceinline__ void route_token_scores(const float* __restrict__ logits, int ld, const float* __restrict__ bias,
                                                     int* ids, float* __restrict__ weights, int t, int experts, int top, int lane,
                                                     const RouteRule rule) {
-  float s[ROUTE_MAX_PER_LANE], v[ROUTE_MAX_PER_LANE], zs[ROUTE_MAX_PER_LANE];
+  float s[PER_LANE], v[PER_LANE], zs[PER_LANE];
 #pragma unroll
-  for (int c = 0; c < ROUTE_MAX_PER_LANE; ++c) {
+  for (int c = 0; c < PER_LANE; ++c) {
     const int e = lane + WAVE * c;
     zs[c] = e < experts ? logits[(int64_t)t * ld + e] : -INFINITY;
   }
@@ -116,11 +134,11 @@ __device__ __forceinline__ void route_token_scores(const float* __restrict__ log
     highest = route_max(zs);
     all = 0.f;
 #pragma unroll
-    for (int c = 0; c < ROUTE_MAX_PER_LANE; ++c) all += lane + WAVE * c < experts ? expf(zs[c] - highest) : 0.f;
+    for (int c = 0; c < PER_LANE; ++c) all += lane + WAVE * c < experts ? expf(zs[c] - highest) : 0.f;
     all = wave_sum(all);
   }
 #pragma unroll
-  for (int c = 0; c < ROUTE_MAX_PER_LANE; ++c) {
+  for (int c = 0; c < PER_LANE; ++c) {
     const int e = lane + WAVE * c;
     const float z = zs[c];
     s[c] = e >= experts ? 0.f : rule.kind == ROUTE_SOFTMAX_SCORES ? expf(z - highest) / all : 1.0f / (1.0f + expf(-z));
@@ -130,68 +148,81 @@ __device__ __forceinline__ void route_token_scores(const float* __restrict__ log
   }
   if (rule.groups > 0 && rule.keep < rule.groups) {
     const int per = experts / rule.groups;
-    float score[ROUTE_MAX_PER_LANE];       // of group lane + WAVE * c
+    float score[PER_LANE];       // of group lane + WAVE * c
 #pragma unroll
-    for (int c = 0; c < ROUTE_MAX_PER_LANE; ++c) score[c] = -INFINITY;
+    for (int c = 0; c < PER_LANE; ++c) score[c] = -INFINITY;
     for (int g = 0; g < rule.groups; ++g) {
-      float mine[ROUTE_MAX_PER_LANE];
+      float mine[PER_LANE];
 #pragma unroll
-      for (int c = 0; c < ROUTE_MAX_PER_LANE; ++c) mine[c] = (lane + WAVE * c) / per == g ? v[c] : -INFINITY;
+      for (int c = 0; c < PER_LANE; ++c) mine[c] = (lane + WAVE * c) / per == g ? v[c] : -INFINITY;
       const float first = route_max(mine);
       float sum = first;
       if (per > 1) {
-        const int where = route_where(mine, first, lane);
+        const int where = route_where(mine, first);
 #pragma unroll
-        for (int c = 0; c < ROUTE_MAX_PER_LANE; ++c)
+        for (int c = 0; c < PER_LANE; ++c)
           if (lane + WAVE * c == where) mine[c] = -INFINITY;
         sum = first + route_max(mine);
       }
 #pragma unroll
-      for (int c = 0; c < ROUTE_MAX_PER_LANE; ++c)
+      for (int c = 0; c < PER_LANE; ++c)
         if (lane + WAVE * c == g) score[c] = sum;
     }
-    bool kept[ROUTE_MAX_PER_LANE];
+    bool kept[PER_LANE];
 #pragma unroll
-    for (int c = 0; c < ROUTE_MAX_PER_LANE; ++c) kept[c] = false;
+    for (int c = 0; c < PER_LANE; ++c) kept[c] = false;
     for (int k = 0; k < rule.keep; ++k) {
       const float best = route_max(score);
-      int where = route_where(score, best, lane);
+      int where = route_where(score, best);
       if (where >= rule.groups) where = k;   // scores that are not numbers: any group
 #pragma unroll
-      for (int c = 0; c < ROUTE_MAX_PER_LANE; ++c) {
+      for (int c = 0; c < PER_LANE; ++c) {
         if (lane + WAVE * c == where) score[c] = -INFINITY;
         if ((lane + WAVE * c) / per == where) kept[c] = true;
       }
     }
 #pragma unroll
-    for (int c = 0; c < ROUTE_MAX_PER_LANE; ++c)
+    for (int c = 0; c < PER_LANE; ++c)
       if (!kept[c]) v[c] = -INFINITY;
   }
-  float total = 0.f;
+  // a lane keeps the choices of its number (written and read again, each was a trip to memory: 27 us for 16 tokens, 8 of 32 experts in groups)
+  int chosen[PER_LANE];
+  float total = 0.f, share[PER_LANE];
   for (int k = 0; k < top; ++k) {
     const float best = route_max(v);
-    int where = route_where(v, best, lane);
+    int where = route_where(v, best);
     if (where >= experts) where = k;    // scores that are not numbers: any expert, never an index outside the table
     float own = 0.f;
 #pragma unroll
-    for (int c = 0; c < ROUTE_MAX_PER_LANE; ++c)
+    for (int c = 0; c < PER_LANE; ++c)
       if (lane + WAVE * c == where) {
         v[c] = -INFINITY;
         own = s[c];
       }
-    const float w = __shfl(own, where % WAVE, WAVE);
+    const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(own), where % WAVE));
     total += w;
-    if (lane == 0) {
-      ids[(int64_t)t * top + k] = where;
-      weights[(int64_t)t * top + k] = w;
-    }
+#pragma unroll
+    for (int c = 0; c < PER_LANE; ++c)
+      if (lane + WAVE * c == k) chosen[c] = where, share[c] = w;
   }
-  // the same lane wrote them: it reads its own stores
-  if (lane == 0 && rule.kind >= ROUTE_SIGMOID_SCORES) {
-    if (rule.scale != 1.f)
-      for (int k = 0; k < top; ++k) weights[(int64_t)t * top + k] *= rule.scale;
-  } else if (lane == 0) {
-    for (int k = 0; k < top; ++k) weights[(int64_t)t * top + k] = weights[(int64_t)t * top + k] / (total + 1e-20f) * rule.scale;
+#pragma unroll
+  for (int c = 0; c < PER_LANE; ++c) {
+    const int k = lane + WAVE * c;
+    if (k >= top) continue;
+    ids[(int64_t)t * top + k] = chosen[c];
+    weights[(int64_t)t * top + k] = rule.kind >= ROUTE_SIGMOID_SCORES ? (rule.scale != 1.f ? share[c] * rule.scale : share[c]) : share[c] / (total + 1e-20f) * rule.scale;
+  }
+}
+
+__device__ __forceinline__ void route_one(const float* __restrict__ logits, int ld, const float* __restrict__ bias, int* ids, float* __restrict__ weights,
+                                          int t, int experts, int top, int lane, const RouteRule rule) {
+  const bool few = experts <= WAVE;
+  if (rule.kind != ROUTE_SOFTMAX_CHOSEN) {
+    if (few) route_token_scores<1>(logits, ld, bias, ids, weights, t, experts, top, lane, rule);
+    else route_token_scores<ROUTE_MAX_PER_LANE>(logits, ld, bias, ids, weights, t, experts, top, lane, rule);
+  } else {
+    if (few) route_token<1>(logits, ld, bias, ids, weights, t, experts, top, lane);
+    else route_token<ROUTE_MAX_PER_LANE>(logits, ld, bias, ids, weights, t, experts, top, lane);
   }
 }
 
@@ -200,8 +231,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict_
                                                         int experts, int top, const RouteRule rule) {
   const int t = blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
   if (t >= tokens) return;
-  if (rule.kind != ROUTE_SOFTMAX_CHOSEN) route_token_scores(logits, ld, bias, ids, weights, t, experts, top, threadIdx.x % WAVE, rule);
-  else route_token(logits, ld, bias, ids, weights, t, experts, top, threadIdx.x % WAVE);
+  route_one(logits, ld, bias, ids, weights, t, experts, top, threadIdx.x % WAVE, rule);
 }
 
 // sorted [capacity]: the pair (token * top + choice) at each row of the sorted order, -1 for the rows that pad an
@@ -225,7 +255,18 @@ __device__ __forceinline__ void align_pairs(const int* ids, int pairs, int exper
     if (!itself(id)) atomicAdd(&count[min((unsigned)id, (unsigned)experts - 1)], 1);
   }
   __syncthreads();
-  if (tid == 0) {
+  if (experts <= WAVE) {                // a wave adds up what lies before each
+    if (tid < WAVE) {
+      const int rows = tid < experts ? (count[tid] + tile - 1) / tile * tile : 0;
+      int end = rows;
+      for (int step = 1; step < WAVE; step <<= 1) {
+        const int before = __shfl_up(end, step, WAVE);
+        if (tid >= step) end += before;
+      }
+      if (tid < experts) first[tid + 1] = end;
+      if (tid == 0) first[0] = 0;
+    }
+  } else if (tid == 0) {
     int at = 0;
     for (int e = 0; e < experts; ++e) {
       first[e] = at;
@@ -263,8 +304,7 @@ __global__ __launch_bounds__(1024) void moe_route_align_kernel(const float* __re
                                                                const RouteRule rule) {
   extern __shared__ int shared[];
   for (int t = threadIdx.x / WAVE; t < tokens; t += blockDim.x / WAVE) {
-    if (rule.kind != ROUTE_SOFTMAX_CHOSEN) route_token_scores(logits, ld, bias, ids, weights, t, experts + identity, top, threadIdx.x % WAVE, rule);
-    else route_token(logits, ld, bias, ids, weights, t, experts + identity, top, threadIdx.x % WAVE);
+    route_one(logits, ld, bias, ids, weights, t, experts + identity, top, threadIdx.x % WAVE, rule);
   }
   __syncthreads();          // the choices are in memory for every thread of the workgroup
   align_pairs(ids, tokens * top, experts, identity, tile, sorted, capacity, place, tile_expert, max_tiles, shared);
