@@ -307,66 +307,19 @@ __device__ __forceinline__ void filter_find_bin(const V* bins, int nbins, double
   __syncthreads();
 }
 
-__global__ __launch_bounds__(1024) void filter_logits_kernel(float* __restrict__ logits,
-                                                             int64_t row_stride, int vocab,
-                                                             const float* __restrict__ temperature,
-                                                             const int* __restrict__ top_k,
-                                                             const float* __restrict__ top_p) {
-  __shared__ float scratch[16];
-  __shared__ unsigned long long bins[FILTER_BINS];             // counts or masses
-  __shared__ int found_bin;
-  __shared__ double found_above;
-  const int row = blockIdx.x, tid = threadIdx.x;
-  float* z = logits + (int64_t)row * row_stride;
-  const float temp = temperature[row];
-  if (!(temp > 0.f)) return;
-  const int k = top_k ? top_k[row] : 0;
-  const float p = top_p ? top_p[row] : 1.f;
-  const bool use_k = k > 0 && k < vocab, use_p = p < 1.f;
-
-  // A pass over the row: body(index, logit) for each of this thread's values.  Four loads of 16 bytes are asked
-  // for before any is used (a thread's loads one after the other, each waited for, were what a pass took its
-  // time for); rows that do not begin on 16 bytes go one value at a time.  The patterns compared are those of the
-  // scaled values logit / temperature, as the reference compares them: two logits whose quotients round to one
-  // float32 are a tie there and are kept or dropped together.  The masses are exp((logit - largest logit) / temperature).
-  const bool in_fours = ((uintptr_t)z % 16) == 0;
-  auto walk = [&](auto&& body) {
-    const int fours = in_fours ? vocab / 4 : 0;
-    for (int first = tid; first < fours; first += 4 * (int)blockDim.x) {
-      floatx4 part[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int at = first + j * (int)blockDim.x;
-        part[j] = ((const floatx4*)z)[at < fours ? at : first];
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int at = first + j * (int)blockDim.x;
-        if (at < fours) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) body(at * 4 + e, part[j][e]);
-        }
-      }
-    }
-    for (int i = fours * 4 + tid; i < vocab; i += blockDim.x) body(i, z[i]);
-  };
-
-  // Every row of positive temperature is looked over once, filtered or not: a row that is not finite as it comes
-  // (the reference refuses it, mini_llm/sampling.py:104-113) gets a NaN that the token choice after this kernel
-  // refuses, since it can no longer tell a -inf that came from one that a filter left.
-  float zmax = -INFINITY;
-  int bad = 0;
-  walk([&](int, float v) {
-    zmax = fmaxf(zmax, v);
-    if (!(fabsf(v) < INFINITY)) bad = 1;
-  });
-  bad = __syncthreads_or(bad);
-  if (bad) {
-    if (tid == 0) z[0] = NAN;
-    return;
-  }
-  if (!use_k && !use_p) return;
-  zmax = block_max(zmax, scratch);
+// The LDS a selection needs.
+struct FilterLds {
+  unsigned long long bins[FILTER_BINS];                        // counts or masses
+  int found_bin;
+  double found_above;
+};
+// The smallest pattern that stays of values that `walk(body)` goes over, body(index, logit) for each of this thread's; the whole workgroup.
+template <typename Walk>
+__device__ __forceinline__ uint32_t filter_threshold(const Walk& walk, FilterLds& lds, float temp, float zmax, int k, bool use_k, float p, bool use_p) {
+  auto& bins = lds.bins;
+  int& found_bin = lds.found_bin;
+  double& found_above = lds.found_above;
+  const int tid = threadIdx.x;
   const float per_temp2 = 1.4426950408889634f / temp;          // exp(x / temp) = exp2(x * this)
 
   // One selection: MASS false: the largest pattern t with count(pattern >= t) >= need; MASS true: the largest
@@ -420,9 +373,254 @@ __global__ __launch_bounds__(1024) void filter_logits_kernel(float* __restrict__
   uint32_t threshold = 0;
   if (use_k) threshold = select(std::false_type{}, (double)k, 0u, 0.f);
   if (use_p) threshold = select(std::true_type{}, 0.0, threshold, p);
+  return threshold;
+}
+
+__global__ __launch_bounds__(1024) void filter_logits_kernel(float* __restrict__ logits,
+                                                             int64_t row_stride, int vocab,
+                                                             const float* __restrict__ temperature,
+                                                             const int* __restrict__ top_k,
+                                                             const float* __restrict__ top_p) {
+  __shared__ float scratch[16];
+  __shared__ FilterLds lds;
+  const int row = blockIdx.x, tid = threadIdx.x;
+  float* z = logits + (int64_t)row * row_stride;
+  const float temp = temperature[row];
+  if (!(temp > 0.f)) return;
+  const int k = top_k ? top_k[row] : 0;
+  const float p = top_p ? top_p[row] : 1.f;
+  const bool use_k = k > 0 && k < vocab, use_p = p < 1.f;
+
+  // A pass over the row: body(index, logit) for each of this thread's values.  Four loads of 16 bytes are asked
+  // for before any is used (a thread's loads one after the other, each waited for, were what a pass took its
+  // time for); rows that do not begin on 16 bytes go one value at a time.  The patterns compared are those of the
+  // scaled values logit / temperature, as the reference compares them: two logits whose quotients round to one
+  // float32 are a tie there and are kept or dropped together.  The masses are exp((logit - largest logit) / temperature).
+  const bool in_fours = ((uintptr_t)z % 16) == 0;
+  auto walk = [&](auto&& body) {
+    const int fours = in_fours ? vocab / 4 : 0;
+    for (int first = tid; first < fours; first += 4 * (int)blockDim.x) {
+      floatx4 part[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int at = first + j * (int)blockDim.x;
+        part[j] = ((const floatx4*)z)[at < fours ? at : first];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int at = first + j * (int)blockDim.x;
+        if (at < fours) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) body(at * 4 + e, part[j][e]);
+        }
+      }
+    }
+    for (int i = fours * 4 + tid; i < vocab; i += blockDim.x) body(i, z[i]);
+  };
+
+  // Every row of positive temperature is looked over once, filtered or not: a row that is not finite as it comes
+  // (the reference refuses it, mini_llm/sampling.py:104-113) gets a NaN that the token choice after this kernel
+  // refuses, since it can no longer tell a -inf that came from one that a filter left.
+  float zmax = -INFINITY;
+  int bad = 0;
+  walk([&](int, float v) {
+    zmax = fmaxf(zmax, v);
+    if (!(fabsf(v) < INFINITY)) bad = 1;
+  });
+  bad = __syncthreads_or(bad);
+  if (bad) {
+    if (tid == 0) z[0] = NAN;
+    return;
+  }
+  if (!use_k && !use_p) return;
+  zmax = block_max(zmax, scratch);
+  const uint32_t threshold = filter_threshold(walk, lds, temp, zmax, k, use_k, p, use_p);
   walk([&](int i, float v) {
     if (ordered_key(v / temp) < threshold) z[i] = -INFINITY;
   });
+}
+
+// The same in four launches over the chip, for large vocabularies and callers that bring a workspace of FILTER_WORDS words a row, all
+// zero before the first call (each call leaves it so): (1) slices of a row look for its largest value, for values that are not finite, and
+// count by the first digit; (2) the values from the k-th largest's bin up, usually a few dozen to a few hundred, are collected in a list;
+// (3) one workgroup a row selects among the list's, or among all of the row's where there is no k or the list is too short; (4) slices
+// drop what lies under the threshold and clear the workspace.  The thresholds are those of the one-kernel form: a list holds everything
+// at or above the k-th largest value, and a share of the mass is one of the values that the k leaves.  One workgroup a row reads 608 KB
+// at the rate of one compute unit, eight times over: 8 rows of 151,936 with k 50 and p 0.9 188 us a call, 48 here
+// (64 rows 209 / 68; a share of the mass alone 151 / 115).
+constexpr int FILTER_SLICE = 4096, FILTER_LIST = 4096, FILTER_THREADS = 256;
+constexpr int FILTER_HEAD = 16, FILTER_WORDS = FILTER_HEAD + FILTER_BINS + FILTER_LIST;
+enum { FILTER_MAX = 0, FILTER_BAD = 1, FILTER_COUNT = 2, FILTER_THRESHOLD = 3 };      // words of a row's head
+__device__ __forceinline__ float value_of_key(uint32_t key) { return __uint_as_float((key & 0x80000000U) ? key ^ 0x80000000U : ~key); }
+
+// body(index, value) for this thread's values of slice blockIdx.x: all loads asked for before any is used
+template <typename Body>
+__device__ __forceinline__ void walk_slice(const float* __restrict__ z, int vocab, const Body& body) {
+  constexpr int EACH = FILTER_SLICE / FILTER_THREADS / 4;
+  const int begin = blockIdx.x * FILTER_SLICE, tid = threadIdx.x;
+  if (((uintptr_t)z % 16) == 0) {
+    const int fours = vocab / 4, first = begin / 4 + tid;
+    floatx4 part[EACH];
+#pragma unroll
+    for (int j = 0; j < EACH; ++j) {
+      const int at = first + j * FILTER_THREADS;
+      part[j] = ((const floatx4*)z)[at < fours ? at : fours - 1];
+    }
+#pragma unroll
+    for (int j = 0; j < EACH; ++j) {
+      const int at = first + j * FILTER_THREADS;
+      if (at < fours)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) body(at * 4 + e, part[j][e]);
+    }
+    if (blockIdx.x == gridDim.x - 1)
+      for (int i = fours * 4 + tid; i < vocab; i += FILTER_THREADS) body(i, z[i]);
+  } else {
+    const int end = begin + FILTER_SLICE < vocab ? begin + FILTER_SLICE : vocab;
+    for (int i = begin + tid; i < end; i += FILTER_THREADS) body(i, z[i]);
+  }
+}
+
+__global__ __launch_bounds__(FILTER_THREADS) void filter_look_kernel(const float* __restrict__ logits, int64_t row_stride, int vocab, const float* __restrict__ temperature,
+                                                                     const int* __restrict__ top_k, uint32_t* __restrict__ space) {
+  __shared__ uint32_t counts[FILTER_BINS];
+  const int row = blockIdx.y, tid = threadIdx.x;
+  const float temp = temperature[row];
+  if (!(temp > 0.f)) return;
+  const int k = top_k ? top_k[row] : 0;
+  const bool use_k = k > 0 && k < vocab;
+  uint32_t* mine = space + (int64_t)row * FILTER_WORDS;
+  if (use_k)
+    for (int i = tid; i < FILTER_BINS; i += FILTER_THREADS) counts[i] = 0;
+  __syncthreads();
+  float zmax = -INFINITY;
+  bool bad = false;
+  walk_slice(logits + (int64_t)row * row_stride, vocab, [&](int, float v) {
+    zmax = fmaxf(zmax, v);
+    if (!(fabsf(v) < INFINITY)) bad = true;
+    if (use_k) atomicAdd(&counts[ordered_key(v / temp) >> 21], 1u);
+  });
+  zmax = wave_max(zmax);
+  bad = __any(bad);
+  if (tid % WAVE == 0) {
+    atomicMax(&mine[FILTER_MAX], ordered_key(zmax));
+    if (bad) atomicMax(&mine[FILTER_BAD], 1u);
+  }
+  if (!use_k) return;
+  __syncthreads();
+  for (int i = tid; i < FILTER_BINS; i += FILTER_THREADS)
+    if (counts[i]) atomicAdd(&mine[FILTER_HEAD + i], counts[i]);
+}
+
+__global__ __launch_bounds__(FILTER_THREADS) void filter_collect_kernel(const float* __restrict__ logits, int64_t row_stride, int vocab, const float* __restrict__ temperature,
+                                                                        const int* __restrict__ top_k, uint32_t* __restrict__ space) {
+  __shared__ uint32_t counts[FILTER_BINS];
+  __shared__ float list[FILTER_LIST];
+  __shared__ int found_bin, length, base;
+  __shared__ double found_above;
+  const int row = blockIdx.y, tid = threadIdx.x;
+  const float temp = temperature[row];
+  const int k = top_k ? top_k[row] : 0;
+  uint32_t* mine = space + (int64_t)row * FILTER_WORDS;
+  if (!(temp > 0.f) || !(k > 0 && k < vocab) || mine[FILTER_BAD]) return;
+  for (int i = tid; i < FILTER_BINS; i += FILTER_THREADS) counts[i] = mine[FILTER_HEAD + i];
+  if (tid == 0) length = 0;
+  __syncthreads();
+  filter_find_bin(counts, FILTER_BINS, (double)k, &found_bin, &found_above);
+  const uint32_t floor = (uint32_t)found_bin << 21;
+  walk_slice(logits + (int64_t)row * row_stride, vocab, [&](int, float v) {
+    if (ordered_key(v / temp) >= floor) list[atomicAdd(&length, 1)] = v;          // a slice has no more values than a list places
+  });
+  __syncthreads();
+  if (tid == 0) base = (int)atomicAdd(&mine[FILTER_COUNT], (uint32_t)length);
+  __syncthreads();
+  for (int i = tid; i < length && base + i < FILTER_LIST; i += FILTER_THREADS) mine[FILTER_HEAD + FILTER_BINS + base + i] = __float_as_uint(list[i]);
+}
+
+__global__ __launch_bounds__(1024) void filter_select_kernel(float* __restrict__ logits, int64_t row_stride, int vocab, const float* __restrict__ temperature,
+                                                             const int* __restrict__ top_k, const float* __restrict__ top_p, uint32_t* __restrict__ space) {
+  __shared__ FilterLds lds;
+  __shared__ float list[FILTER_LIST];
+  const int row = blockIdx.x, tid = threadIdx.x;
+  float* z = logits + (int64_t)row * row_stride;
+  const float temp = temperature[row];
+  if (!(temp > 0.f)) return;
+  uint32_t* mine = space + (int64_t)row * FILTER_WORDS;
+  const int k = top_k ? top_k[row] : 0;
+  const float p = top_p ? top_p[row] : 1.f;
+  const bool use_k = k > 0 && k < vocab, use_p = p < 1.f;
+  uint32_t threshold = 0;
+  if (mine[FILTER_BAD]) {
+    if (tid == 0) z[0] = NAN;                                  // as filter_logits_kernel leaves a row that was not finite
+  } else if (use_k || use_p) {
+    const float zmax = value_of_key(mine[FILTER_MAX]);
+    const int count = (int)mine[FILTER_COUNT];
+    if (use_k && count <= FILTER_LIST) {
+      for (int i = tid; i < count; i += blockDim.x) list[i] = __uint_as_float(mine[FILTER_HEAD + FILTER_BINS + i]);
+      __syncthreads();
+      threshold = filter_threshold([&](auto&& body) { for (int i = tid; i < count; i += (int)blockDim.x) body(i, list[i]); }, lds, temp, zmax, k, use_k, p, use_p);
+    } else {
+      const int fours = ((uintptr_t)z % 16) == 0 ? vocab / 4 : 0;
+      threshold = filter_threshold(
+          [&](auto&& body) {
+            for (int first = tid; first < fours; first += 4 * (int)blockDim.x) {
+              floatx4 part[4];
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                const int at = first + j * (int)blockDim.x;
+                part[j] = ((const floatx4*)z)[at < fours ? at : first];
+              }
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                const int at = first + j * (int)blockDim.x;
+                if (at < fours)
+#pragma unroll
+                  for (int e = 0; e < 4; ++e) body(at * 4 + e, part[j][e]);
+              }
+            }
+            for (int i = fours * 4 + tid; i < vocab; i += (int)blockDim.x) body(i, z[i]);
+          },
+          lds, temp, zmax, k, use_k, p, use_p);
+    }
+  }
+  if (tid == 0) mine[FILTER_THRESHOLD] = threshold;
+}
+
+__global__ __launch_bounds__(FILTER_THREADS) void filter_drop_kernel(float* __restrict__ logits, int64_t row_stride, int vocab, const float* __restrict__ temperature,
+                                                                     uint32_t* __restrict__ space) {
+  const int row = blockIdx.y, tid = threadIdx.x;
+  float* z = logits + (int64_t)row * row_stride;
+  const float temp = temperature[row];
+  if (!(temp > 0.f)) return;
+  uint32_t* mine = space + (int64_t)row * FILTER_WORDS;
+  const uint32_t threshold = mine[FILTER_THRESHOLD];
+  if (threshold)
+    walk_slice(z, vocab, [&](int i, float v) {
+      if (ordered_key(v / temp) < threshold) z[i] = -INFINITY;
+    });
+  for (int i = blockIdx.x * FILTER_THREADS + tid; i < FILTER_BINS; i += gridDim.x * FILTER_THREADS) mine[FILTER_HEAD + i] = 0;
+  if (blockIdx.x == 0 && tid <= FILTER_COUNT) mine[tid] = 0;
+}
+
+LRS_API int lrs_filter_words() { return FILTER_WORDS; }
+
+LRS_API int lrs_filter_logits_wide(float* logits, int64_t row_stride, int rows, int vocab, const float* temperature, const int* top_k,
+                                   const float* top_p, void* workspace, void* stream) {
+  LRS_REQUIRE(rows > 0 && rows <= 65535 && vocab >= 4, "filter_logits: rows=%d vocab=%d must be positive", rows, vocab);
+  LRS_REQUIRE(temperature != nullptr && workspace != nullptr, "filter_logits: temperature and a workspace are required");
+  const dim3 grid((vocab + FILTER_SLICE - 1) / FILTER_SLICE, rows);
+  hipStream_t s = (hipStream_t)stream;
+  uint32_t* space = (uint32_t*)workspace;
+  filter_look_kernel<<<grid, FILTER_THREADS, 0, s>>>(logits, row_stride, vocab, temperature, top_k, space);
+  if (lrs_check_launch("filter_look")) return 1;
+  if (top_k) {
+    filter_collect_kernel<<<grid, FILTER_THREADS, 0, s>>>(logits, row_stride, vocab, temperature, top_k, space);
+    if (lrs_check_launch("filter_collect")) return 1;
+  }
+  filter_select_kernel<<<rows, 1024, 0, s>>>(logits, row_stride, vocab, temperature, top_k, top_p, space);
+  if (lrs_check_launch("filter_select")) return 1;
+  filter_drop_kernel<<<grid, FILTER_THREADS, 0, s>>>(logits, row_stride, vocab, temperature, space);
+  return lrs_check_launch("filter_drop");
 }
 
 LRS_API int lrs_filter_logits(float* logits, int64_t row_stride, int rows, int vocab,

@@ -869,7 +869,7 @@ class ModelRunner:
             logits = self.model.logits(ctx, h)
             chosen = chosen_dev[i * stride:i * stride + ctx.T]
             if sampled:
-                ops.filter_logits(logits, temperature, top_k, top_p)
+                ops.filter_logits(logits, temperature, top_k, top_p, self.arena.get("filter", (ctx.T, ops.filter_words()), torch.int32, zeroed=True))
                 ops.choose_tokens(chosen, logits, temperature, seeds, draws, filtered=True)
             else:
                 ops.choose_tokens(chosen, logits)

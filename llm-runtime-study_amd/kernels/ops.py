@@ -176,6 +176,8 @@ _SIGNATURES = {
     "lrs_choose_tokens_static_init": (c_int, []),
     "lrs_choose_tokens_static_max_parts": (c_int, []),
     "lrs_filter_logits": (c_int, [c_void_p, c_int64, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "lrs_filter_logits_wide": (c_int, [c_void_p, c_int64, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "lrs_filter_words": (c_int, []),
     "lrs_round_rows": (c_int, [c_void_p, c_int, c_void_p, c_int64, c_void_p]),
     "lrs_norm_add": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_void_p, c_void_p]),
     "lrs_delta_state_rows": (c_int, [c_int]),
@@ -246,7 +248,7 @@ def library():
 # and _SIGNATURES by kernels/plan_codegen.py, is the other side (a test keeps the two in step).
 PLAN_OPS = ("lrs_activation", "lrs_add_gathered", "lrs_add_into", "lrs_add_rmsnorm", "lrs_advance_decode", "lrs_advance_slots", "lrs_attention", "lrs_attention_decode",
             "lrs_attention_mixed", "lrs_attention_prefill", "lrs_axpby", "lrs_choose_tokens", "lrs_choose_tokens_split", "lrs_copy_to_pinned", "lrs_delta_rule", "lrs_delta_rule_channels", "lrs_delta_rule_chunks", "lrs_embed", "lrs_fill_i32",
-            "lrs_filter_logits", "lrs_gated_clamped", "lrs_gated_norm_add", "lrs_gather_rows", "lrs_gemm", "lrs_gemm_lines_add_rmsnorm", "lrs_gemm_mid_add_norm_begin", "lrs_gemm_mid_qk_prep", "lrs_gemm_mid_scaled",
+            "lrs_filter_logits", "lrs_filter_logits_wide", "lrs_gated_clamped", "lrs_gated_norm_add", "lrs_gather_rows", "lrs_gemm", "lrs_gemm_lines_add_rmsnorm", "lrs_gemm_mid_add_norm_begin", "lrs_gemm_mid_qk_prep", "lrs_gemm_mid_scaled",
             "lrs_gemm_norm_chain", "lrs_head_gemm", "lrs_latent_attention", "lrs_latent_attention_groups", "lrs_latent_prep", "lrs_layernorm", "lrs_library_gemm", "lrs_mlstm", "lrs_mlstm_chunks", "lrs_moe_align", "lrs_moe_combine", "lrs_moe_experts", "lrs_moe_route", "lrs_moe_route_align", "lrs_norm_add",
             "lrs_qk_prep", "lrs_qkv_norm_prep", "lrs_rmsnorm", "lrs_rope_table", "lrs_rotate_unit_prep", "lrs_round_rows", "lrs_scale_add_layernorm", "lrs_scale_rows", "lrs_scale_values", "lrs_sigmoid_gate", "lrs_silu_mul", "lrs_soft_cap", "lrs_ssm", "lrs_xielu")
 _PLAN_INDEX = {name: index for index, name in enumerate(PLAN_OPS)}
@@ -1483,7 +1485,17 @@ def choose_tokens_static(out: torch.Tensor, logits: torch.Tensor, parts: int, te
         None if temperature is None else _dev(counters, "counters"), parts, int(bool(filtered)), _stream())
 
 
-def filter_logits(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor | None, top_p: torch.Tensor | None) -> None:
+def filter_words() -> int:
+    """Words of workspace that filter_logits() wants for a row."""
+    return library().lrs_filter_words()
+
+
+def filter_logits(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor | None, top_p: torch.Tensor | None,
+                  workspace: torch.Tensor | None = None) -> None:
+    """Drops (sets to -inf, in place) what top-k and top-p leave out of rows of positive temperature.
+
+    workspace: the caller's own device memory, int32 [R or more, filter_words()], all zero before its first use (every call leaves it
+    so) and used on one stream at a time: large vocabularies are then worked on by the whole chip."""
     rows, vocab = logits.shape
     stride = _rows(logits, "logits")
     _need(temperature.dtype == torch.float32 and temperature.numel() >= rows, "filter_logits: temperature must be float32 [R]")
@@ -1491,8 +1503,14 @@ def filter_logits(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.
         _need(top_k.dtype == torch.int32 and top_k.numel() >= rows, "filter_logits: top_k must be int32 [R]")
     if top_p is not None:
         _need(top_p.dtype == torch.float32 and top_p.numel() >= rows, "filter_logits: top_p must be float32 [R]")
-    _launch("lrs_filter_logits", _dev(logits, "logits", torch.float32), stride, rows, vocab, _dev(temperature, "temperature"),
-                                       None if top_k is None else _dev(top_k, "top_k"), None if top_p is None else _dev(top_p, "top_p"), _stream())
+    args = (_dev(logits, "logits", torch.float32), stride, rows, vocab, _dev(temperature, "temperature"),
+            None if top_k is None else _dev(top_k, "top_k"), None if top_p is None else _dev(top_p, "top_p"))
+    if workspace is not None:
+        _need(workspace.dtype == torch.int32 and workspace.is_contiguous() and workspace.numel() >= rows * filter_words(), f"filter_logits: workspace must be contiguous int32, {filter_words()} words a row")
+        if vocab >= 16384 and rows <= 65535:
+            _launch("lrs_filter_logits_wide", *args, _dev(workspace, "workspace"), _stream())
+            return
+    _launch("lrs_filter_logits", *args, _stream())
 
 
 # ------------------------------------------------------------------- gated delta rule

@@ -49,6 +49,7 @@ class Sampler:
         self._chosen_address = 0  # ... and where the device sees it
         self._settings_host = self._settings_dev = None   # the rows' sampling settings: pinned staging and its device copy
         self._settings_cap = 0
+        self._filter_space = None     # what filter_logits() leaves as it found it: all zero
 
     def _settings_room(self, rows: int) -> int:
         """Staging for `rows` rows' settings (six int32 words a row, in five arrays of `cap` rows); returns cap.  The
@@ -57,6 +58,7 @@ class Sampler:
             self._settings_cap = cap = max(64, -(-rows // 4) * 4)
             self._settings_host = torch.zeros(6 * cap, dtype=torch.int32, pin_memory=True)
             self._settings_dev = torch.zeros(6 * cap, dtype=torch.int32, device=self.device)
+            self._filter_space = None
         return self._settings_cap
 
     def _result(self, rows: int) -> torch.Tensor:
@@ -99,6 +101,8 @@ class Sampler:
         top_k, counters, seeds = dev[2 * cap:3 * cap][:n], dev[3 * cap:4 * cap][:n], dev[4 * cap:6 * cap].view(torch.int64)[:n]
         filtered = any((row.config.top_k is not None and row.config.top_k < vocab) or row.config.top_p < 1.0 for row in rows if not row.config.greedy)
         if filtered:
-            ops.filter_logits(logits, temperature, top_k, top_p)
+            if self._filter_space is None:
+                self._filter_space = torch.zeros(cap, ops.filter_words(), dtype=torch.int32, device=self.device)
+            ops.filter_logits(logits, temperature, top_k, top_p, self._filter_space)
         ops.choose_tokens(out, logits, temperature, seeds, counters, out_address=self._chosen_address, filtered=filtered)
         return self._read(out)
