@@ -409,9 +409,10 @@ constexpr int GM = 32, GN = 128, GK = 64, GPAD = 8;
 // NT: columns per workgroup, 128 (a wave 32 of them) or 64 (a wave 16: twice the workgroups, for steps of so few rows
 // that 128 columns each would leave compute units without any).
 template <typename TO, int NT>
-__global__ __launch_bounds__(256) void moe_experts_bf16_kernel(TO* __restrict__ out, int ldc, const bf16* __restrict__ a, int lda,
-                                                               const bf16* __restrict__ w, int n, int k, const int* __restrict__ sorted,
-                                                               const int* __restrict__ tile_expert, int top, int gather, int act, const PairAct pa) {
+__global__ __launch_bounds__(256) void moe_experts_bf16_kernel(const int* __restrict__ tile_expert, const int* __restrict__ sorted, const bf16* __restrict__ w,
+                                                               const bf16* __restrict__ a, int n, int k, int top, int gather, int lda,
+                                                               TO* __restrict__ out, int ldc, int act, const PairAct pa) {
+  // (what leads to the first loads comes first: those arguments are in registers when a wave begins, the file is compiled so)
   const int expert = tile_expert[blockIdx.x];
   if (expert < 0) return;
   __shared__ __attribute__((aligned(16))) bf16 a_s[GM][GK + GPAD];
@@ -420,29 +421,32 @@ __global__ __launch_bounds__(256) void moe_experts_bf16_kernel(TO* __restrict__ 
   const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
   constexpr int WN = NT / 64;                 // products of 16 columns a wave makes side by side
   const int row0 = blockIdx.x * GM, col0 = blockIdx.y * NT;
-  if (tid < GM) {
-    const int pair = sorted[row0 + tid];
-    row_of[tid] = pair < 0 ? -1 : (gather ? pair / top : row0 + tid);
-  }
-  __syncthreads();
   const bf16* we = w + (int64_t)expert * n * k;
   // a thread brings 8 values (16 bytes) of one row of the slice: 32 x 64 of the rows is one piece each, 128 x 64 of the
-  // weights four
+  // weights four (a row past the matrix is its last one, not stored); the first weights are asked for before the rows are known
   const int a_row = tid / 8, a_col = (tid % 8) * 8;
-  const int a_src = row_of[a_row];
-  const bf16* a_ptr = a_src >= 0 ? a + (int64_t)a_src * lda + a_col : nullptr;
   bf16x8 a_reg, b_reg[NT / 32];
   const bf16x8 zero = {};
-  auto fetch = [&](int k0) {
-    a_reg = a_ptr ? *(const bf16x8*)(a_ptr + k0) : zero;
+  auto fetch_weights = [&](int k0) {
 #pragma unroll
     for (int p = 0; p < NT / 32; ++p) {
-      const int r = p * 32 + a_row;
-      b_reg[p] = col0 + r < n ? load_once((const bf16x8*)(we + (int64_t)(col0 + r) * k + k0 + a_col)) : zero;
+      const int r = col0 + p * 32 + a_row;
+      b_reg[p] = load_once((const bf16x8*)(we + (int64_t)(r < n ? r : n - 1) * k + k0 + a_col));
     }
   };
+  const int my_pair = sorted[row0 + tid % GM];
+  fetch_weights(0);
+  if (tid < GM) row_of[tid] = my_pair < 0 ? -1 : (gather ? my_pair / top : row0 + tid);
+  __syncthreads();
+  const int a_src = row_of[a_row];
+  const bf16* a_ptr = a_src >= 0 ? a + (int64_t)a_src * lda + a_col : nullptr;
+  auto fetch_rows = [&](int k0) { a_reg = a_ptr ? *(const bf16x8*)(a_ptr + k0) : zero; };
+  auto fetch = [&](int k0) {
+    fetch_weights(k0);
+    fetch_rows(k0);
+  };
   floatx4 acc[2][WN] = {};
-  fetch(0);
+  fetch_rows(0);
   const int frag_row = lane % 16, frag_k = (lane / 16) * 8;
   for (int k0 = 0; k0 < k; k0 += GK) {
     *(bf16x8*)&a_s[a_row][a_col] = a_reg;
@@ -1211,7 +1215,7 @@ LRS_API int lrs_moe_experts(void* out, int out_dtype, int ldc, const void* a, co
     // few tiles (single tokens, short portions): 64 columns a workgroup, so that twice as many stream the weights
     const bool narrow = (int64_t)max_tiles * ((n + GN - 1) / GN) < 4 * lrs_compute_units();
     dim3 grid(max_tiles, narrow ? (n + 63) / 64 : (n + GN - 1) / GN);
-#define CORES(TO, NT) moe_experts_bf16_kernel<TO, NT><<<grid, 256, 0, s>>>((TO*)out, ldc, (const bf16*)a, lda, (const bf16*)w, n, k, sorted, tile_expert, top, gather, act, pa)
+#define CORES(TO, NT) moe_experts_bf16_kernel<TO, NT><<<grid, 256, 0, s>>>(tile_expert, sorted, (const bf16*)w, (const bf16*)a, n, k, top, gather, lda, (TO*)out, ldc, act, pa)
     if (out_dtype == LRS_BF16) { if (narrow) CORES(bf16, 64); else CORES(bf16, 128); }
     else if (out_dtype == LRS_F32) { if (narrow) CORES(float, 64); else CORES(float, 128); }
     else return lrs_fail("moe_experts: unknown output dtype %d", out_dtype);
