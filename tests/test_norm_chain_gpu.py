@@ -89,3 +89,17 @@ def test_slices_left_to_a_workgroup_of_17_to_128_rows(m, splits, waves, k):
         ops.gemm_mid_scaled(out, x.cuda(), w.cuda(), sumsq.cuda(), 1e-6, choice=ops.KernelChoice(mid_splits=splits, mid_waves=waves))
         want = x.double() @ w.double().T / (sumsq.double().sum(0) / k + 1e-6).sqrt()[:, None]
         torch.testing.assert_close(out.cpu().double(), want, rtol=2 ** -8 + 2 ** -18, atol=2 ** -14)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("tokens,hidden,offset", [(1, 8, 0), (3, 100, 0), (33, 1032, 0), (257, 16, 0), (5, 64, 4)])
+def test_rows_of_the_embedding(tokens, hidden, offset, dtype):
+    """Rows of whole and broken pieces of eight values, and a table that does not begin on 32 bytes: the table's rows times a factor."""
+    from llm_runtime_study_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(hidden)
+    table = torch.randn(50 * hidden + offset, generator=g).to(dtype).cuda()[offset:].view(50, hidden)
+    ids = torch.randint(0, 50, (tokens,), generator=g, dtype=torch.int32).cuda()
+    out = torch.full((tokens, hidden), float("nan"), device="cuda")
+    ops.embed(out, table, ids, 1.5)
+    assert torch.equal(out, table[ids.long()].float() * 1.5)
