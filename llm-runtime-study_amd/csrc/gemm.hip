@@ -561,7 +561,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(
   __shared__ bf16x8 act_patch_all[LINES ? WAVES : 1][128];
   __shared__ floatx4 partial[WAVES][MT][WAVE];
   __shared__ float sumsq[WAVES][MT][16];
-  __shared__ float chain_parts[WAVES * 4][16];   // in_sumsq, added up by WAVES * 4 threads per row
+  __shared__ __attribute__((aligned(16))) float chain_parts[16][WAVES * 4 + 4];   // in_sumsq, added up by WAVES * 4 threads per row
   __shared__ float chain_scale[16];
   __shared__ float chain_squares[16][RT * 16 + 1];
   const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
@@ -679,6 +679,22 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(
     }
   }
   bool feeds_norm = false;
+  // The factors of a norm that this product finishes, of what all waves left in chain_parts.  All waves of the workgroup come by the barrier on
+  // the same way: with LINES, whose waves walk equally many steps, behind the first weights; the ways of the others part there, since K
+  // need not be a multiple of what they walk together, and meet again behind the walk.
+  auto factors = [&]() {
+    __syncthreads();
+    if (tid < 16) {
+      float q = 0.f;
+#pragma unroll
+      for (int p = 0; p < WAVES; ++p) {
+        const floatx4 four = *(const floatx4*)&chain_parts[tid][p * 4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) q += four[i];
+      }
+      chain_scale[tid] = 1.0f / sqrtf(q / (float)k + chain.in_eps);
+    }
+  };
   float early_h[RT];
   unsigned early_w[RT];                                          // as it is stored
   // Behind the first weights asked for, once in every wave: the residual values and norm weights of the columns that this thread will
@@ -703,14 +719,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(
       for (int j = 0; j < EARLY; ++j) v += part + j * WAVES * 4 < in_parts ? early_sums[j] : 0.f;
       if (token < m)
         for (int p = part + EARLY * WAVES * 4; p < in_parts; p += WAVES * 4) v += in_sumsq[(int64_t)p * m + token];
-      chain_parts[part][token] = v;
-      __syncthreads();
-      if (tid < 16) {
-        float q = 0.f;
-#pragma unroll
-        for (int p = 0; p < WAVES * 4; ++p) q += chain_parts[p][tid];
-        chain_scale[tid] = 1.0f / sqrtf(q / (float)k + chain.in_eps);
-      }
+      chain_parts[token][part] = v;
+      if constexpr (LINES) factors();
     }
   };
   // U steps of 32 k, all their loads asked for before any is used
@@ -774,7 +784,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(
   // Workgroups walk their K slices from different starting points (the order of a column's sum
   // depends on the column alone): all of them read the same activations, and in step they would
   // all ask the same few cache lines of the L2 at the same moment.
-  const int batches = full_end > s ? (full_end - s) / UNROLL : 0;
+  // (LINES: the same number in every wave, of the arguments alone)
+  const int whole = LINES ? per_wave : full_end > s ? full_end - s : 0;
+  const int batches = whole / UNROLL;
   auto nothing = [] {};
   if (batches > 0) {
     int at = batches > 1 ? (int)(blockIdx.x % (unsigned)batches) : 0;
@@ -784,7 +796,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(
       steps_together(s + at * UNROLL, std::integral_constant<int, UNROLL>{}, nothing);
     }
     s += batches * UNROLL;
-  } else if (UNROLL > 4 && full_end - s >= 4) {
+  } else if (UNROLL > 4 && whole >= 4) {
     steps_together(s, std::integral_constant<int, 4>{}, meanwhile);
     s += 4;
   } else {
@@ -824,6 +836,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(
       if (g == 0) sumsq[wave][t][r] = v;
     }
   }
+  if constexpr (!LINES)
+    if (scaled_input) factors();
   // accumulator layout: token = t*16 + lane % 16, weight row = tile row 4 * (lane / 16) + i
   auto total = [&](int t, int l, int i) -> float {
     float v = 0.f;

@@ -6,7 +6,9 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n,k,swiglu", [(256, 512, False), (2048, 1536, True), (6144, 1024, False), (16416, 768, False), (272, 96, False)])
+# (K of 896, 1,152, 1,920 and 2,880, of 416 in the widest: the last of a workgroup's waves walks less than the others and takes another way)
+@pytest.mark.parametrize("n,k,swiglu", [(256, 512, False), (2048, 1536, True), (6144, 1024, False), (16416, 768, False), (272, 96, False),
+                                        (256, 896, False), (2048, 1152, True), (272, 1920, False), (256, 2880, False), (6144, 896, False), (16416, 416, False)])
 @pytest.mark.parametrize("m,parts", [(1, 1), (3, 31), (16, 33), (9, 320), (16, 321), (2, 700)])
 def test_sums_of_squares_in_any_number_of_parts(m, parts, n, k, swiglu):
     """Against 64 bits: the factor is right to 2^-20 whatever the parts (sums of 32 bits over at most 700), a product of K bfloat16 pairs
