@@ -404,72 +404,84 @@ __global__ __launch_bounds__(256) void moe_experts_kernel(TO* __restrict__ out, 
 // multiplied.
 constexpr int GM = 32, GN = 128, GK = 64, GPAD = 8;
 
-// An expert of a step of few rows has one tile of them, so its weights are read once (load_once): eight steps of eight requests and their
-// prompts, 4 layers of the 8B sizes with 32 experts 14,425 -> 13,310 us; a step of 16 requests with gated experts 1,354 -> 1,240.
+// The weights of an expert with one tile are read once (load_once): eight steps of eight requests and their prompts, 4 layers of the 8B sizes
+// with 32 experts 14,425 -> 13,310 us; a step of 16 requests with gated experts 1,354 -> 1,240.  Those of an expert with more are read by its
+// tiles side by side, and the hint would have each of them bring its own; which of the two a workgroup has, the tiles beside its own say.
+// us a product, 32 experts of 8 choices between widths of 4,096 and 2,304, without the hint / with it everywhere / as here: 64 tokens 126 / 110 / 110,
+// chosen unevenly 122 / 127 / 117; 96 unevenly 134 / 157 / 132; 160 tokens 187 / 227 / 190, unevenly 170 / 203 / 160.
 // NT: columns per workgroup, 128 (a wave 32 of them) or 64 (a wave 16: twice the workgroups, for steps of so few rows
 // that 128 columns each would leave compute units without any).
 template <typename TO, int NT>
 __global__ __launch_bounds__(256) void moe_experts_bf16_kernel(const int* __restrict__ tile_expert, const int* __restrict__ sorted, const bf16* __restrict__ w,
-                                                               const bf16* __restrict__ a, int n, int k, int top, int gather, int lda,
+                                                               const bf16* __restrict__ a, int n, int k, int top, int gather, int lda, int tiles,
                                                                TO* __restrict__ out, int ldc, int act, const PairAct pa) {
   // (what leads to the first loads comes first: those arguments are in registers when a wave begins, the file is compiled so)
-  const int expert = tile_expert[blockIdx.x];
+  const int tile = blockIdx.x, expert = tile_expert[tile];
+  const int before = tile_expert[tile > 0 ? tile - 1 : 0], behind = tile_expert[tile + 1 < tiles ? tile + 1 : tile];
   if (expert < 0) return;
+  const bool alone = (tile == 0 || before != expert) && (tile + 1 == tiles || behind != expert);
   __shared__ __attribute__((aligned(16))) bf16 a_s[GM][GK + GPAD];
   __shared__ __attribute__((aligned(16))) bf16 b_s[NT][GK + GPAD];
   __shared__ int row_of[GM];
   const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
   constexpr int WN = NT / 64;                 // products of 16 columns a wave makes side by side
-  const int row0 = blockIdx.x * GM, col0 = blockIdx.y * NT;
+  const int row0 = tile * GM, col0 = blockIdx.y * NT;
   const bf16* we = w + (int64_t)expert * n * k;
   // a thread brings 8 values (16 bytes) of one row of the slice: 32 x 64 of the rows is one piece each, 128 x 64 of the
   // weights four (a row past the matrix is its last one, not stored); the first weights are asked for before the rows are known
   const int a_row = tid / 8, a_col = (tid % 8) * 8;
-  bf16x8 a_reg, b_reg[NT / 32];
-  const bf16x8 zero = {};
-  auto fetch_weights = [&](int k0) {
-#pragma unroll
-    for (int p = 0; p < NT / 32; ++p) {
-      const int r = col0 + p * 32 + a_row;
-      b_reg[p] = load_once((const bf16x8*)(we + (int64_t)(r < n ? r : n - 1) * k + k0 + a_col));
-    }
-  };
-  const int my_pair = sorted[row0 + tid % GM];
-  fetch_weights(0);
-  if (tid < GM) row_of[tid] = my_pair < 0 ? -1 : (gather ? my_pair / top : row0 + tid);
-  __syncthreads();
-  const int a_src = row_of[a_row];
-  const bf16* a_ptr = a_src >= 0 ? a + (int64_t)a_src * lda + a_col : nullptr;
-  auto fetch_rows = [&](int k0) { a_reg = a_ptr ? *(const bf16x8*)(a_ptr + k0) : zero; };
-  auto fetch = [&](int k0) {
-    fetch_weights(k0);
-    fetch_rows(k0);
-  };
   floatx4 acc[2][WN] = {};
-  fetch_rows(0);
-  const int frag_row = lane % 16, frag_k = (lane / 16) * 8;
-  for (int k0 = 0; k0 < k; k0 += GK) {
-    *(bf16x8*)&a_s[a_row][a_col] = a_reg;
+  auto walk = [&](auto once) {
+    constexpr bool ONCE = decltype(once)::value;
+    bf16x8 a_reg, b_reg[NT / 32];
+    const bf16x8 zero = {};
+    auto fetch_weights = [&](int k0) {
 #pragma unroll
-    for (int p = 0; p < NT / 32; ++p) *(bf16x8*)&b_s[p * 32 + a_row][a_col] = b_reg[p];
+      for (int p = 0; p < NT / 32; ++p) {
+        const int r = col0 + p * 32 + a_row;
+        const bf16x8* at = (const bf16x8*)(we + (int64_t)(r < n ? r : n - 1) * k + k0 + a_col);
+        b_reg[p] = ONCE ? load_once(at) : *at;
+      }
+    };
+    const int my_pair = sorted[row0 + tid % GM];
+    fetch_weights(0);
+    if (tid < GM) row_of[tid] = my_pair < 0 ? -1 : (gather ? my_pair / top : row0 + tid);
     __syncthreads();
-    if (k0 + GK < k) fetch(k0 + GK);
+    const int a_src = row_of[a_row];
+    const bf16* a_ptr = a_src >= 0 ? a + (int64_t)a_src * lda + a_col : nullptr;
+    auto fetch_rows = [&](int k0) { a_reg = a_ptr ? *(const bf16x8*)(a_ptr + k0) : zero; };
+    auto fetch = [&](int k0) {
+      fetch_weights(k0);
+      fetch_rows(k0);
+    };
+    fetch_rows(0);
+    const int frag_row = lane % 16, frag_k = (lane / 16) * 8;
+    for (int k0 = 0; k0 < k; k0 += GK) {
+      *(bf16x8*)&a_s[a_row][a_col] = a_reg;
 #pragma unroll
-    for (int kk = 0; kk < GK; kk += 32) {
-      bf16x8 af[2], bfr[WN];
+      for (int p = 0; p < NT / 32; ++p) *(bf16x8*)&b_s[p * 32 + a_row][a_col] = b_reg[p];
+      __syncthreads();
+      if (k0 + GK < k) fetch(k0 + GK);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) af[i] = *(const bf16x8*)&a_s[i * 16 + frag_row][kk + frag_k];
+      for (int kk = 0; kk < GK; kk += 32) {
+        bf16x8 af[2], bfr[WN];
 #pragma unroll
-      for (int i = 0; i < WN; ++i) bfr[i] = *(const bf16x8*)&b_s[wave * 16 * WN + i * 16 + frag_row][kk + frag_k];
+        for (int i = 0; i < 2; ++i) af[i] = *(const bf16x8*)&a_s[i * 16 + frag_row][kk + frag_k];
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < WN; ++i) bfr[i] = *(const bf16x8*)&b_s[wave * 16 * WN + i * 16 + frag_row][kk + frag_k];
 #pragma unroll
-        for (int jj = 0; jj < WN; ++jj)
-          // the weights as the first operand: a lane then holds four consecutive columns of one output row
-          acc[i][jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[jj], af[i], acc[i][jj], 0, 0, 0);
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int jj = 0; jj < WN; ++jj)
+            // the weights as the first operand: a lane then holds four consecutive columns of one output row
+            acc[i][jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[jj], af[i], acc[i][jj], 0, 0, 0);
+      }
+      __syncthreads();
     }
-    __syncthreads();
-  }
+  };
+  // (the compiler takes the first slice of both out in front, without the hint)
+  if (alone) walk(std::true_type{});
+  else walk(std::false_type{});
   // lane l of a product holds output row (l % 16) and columns (l / 16) * 4 .. + 4 of its 16 x 16
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -1215,7 +1227,7 @@ LRS_API int lrs_moe_experts(void* out, int out_dtype, int ldc, const void* a, co
     // few tiles (single tokens, short portions): 64 columns a workgroup, so that twice as many stream the weights
     const bool narrow = (int64_t)max_tiles * ((n + GN - 1) / GN) < 4 * lrs_compute_units();
     dim3 grid(max_tiles, narrow ? (n + 63) / 64 : (n + GN - 1) / GN);
-#define CORES(TO, NT) moe_experts_bf16_kernel<TO, NT><<<grid, 256, 0, s>>>(tile_expert, sorted, (const bf16*)w, (const bf16*)a, n, k, top, gather, lda, (TO*)out, ldc, act, pa)
+#define CORES(TO, NT) moe_experts_bf16_kernel<TO, NT><<<grid, 256, 0, s>>>(tile_expert, sorted, (const bf16*)w, (const bf16*)a, n, k, top, gather, lda, max_tiles, (TO*)out, ldc, act, pa)
     if (out_dtype == LRS_BF16) { if (narrow) CORES(bf16, 64); else CORES(bf16, 128); }
     else if (out_dtype == LRS_F32) { if (narrow) CORES(float, 64); else CORES(float, 128); }
     else return lrs_fail("moe_experts: unknown output dtype %d", out_dtype);

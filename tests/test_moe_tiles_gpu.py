@@ -110,3 +110,24 @@ def test_two_tiles_and_one(rows, n, k, gather, kind):
 @pytest.mark.parametrize("gather,kind", [(True, "pairs"), (False, "f32")])
 def test_pairs_kept_and_parted(rows, n, k, gather, kind):
     test_two_tiles_and_one(rows, n, k, gather, kind)
+
+
+# tiles of 32 rows: an expert's tiles side by side or alone, at both ends of the list, beside tiles not in use (whose rows must stay as they are)
+@pytest.mark.parametrize("experts", [(0,), (1, 1), (0, 1, 1), (2, 2, 2, 0), (-1, 1, -1, 1, 1, -1), (0, 1, 2, -1, -1), (1, 0, 0, -1, 2, 2)])
+@pytest.mark.parametrize("n,k", [(64, 64), (132, 192), (4160, 128)])
+def test_experts_with_one_tile_of_32_rows_and_with_more(experts, n, k):
+    from llm_runtime_study_amd.kernels import ops
+
+    g, tile = torch.Generator().manual_seed(n + len(experts)), 32
+    x, w = torch.randn(len(experts) * tile, k, generator=g).to(torch.bfloat16), torch.randn(3, n, k, generator=g).to(torch.bfloat16)
+    listed = torch.randperm(len(experts) * tile, generator=g).to(torch.int32).view(len(experts), tile)
+    listed[:, 20:] = torch.where(torch.arange(len(experts))[:, None] % 2 == 0, listed[:, 20:], -1)
+    listed[torch.tensor(experts) < 0] = -1
+    out = torch.full((len(experts) * tile, n), -7.0, device="cuda")
+    ops.moe_experts(out, x.cuda(), w.cuda(), listed.flatten().cuda(), torch.tensor(experts, dtype=torch.int32).cuda(), tile, 1, gather=True, relu_squared=False)
+    got = out.cpu().view(len(experts), tile, n)
+    assert (got[listed < 0] == -7.0).all()
+    for i, e in enumerate(experts):
+        rows = x[listed[i][listed[i] >= 0].long()].double()
+        want, size = rows @ w[max(e, 0)].double().T, rows.abs() @ w[max(e, 0)].double().abs().T
+        assert ((got[i][listed[i] >= 0].double() - want).abs() <= k * 2.0 ** -23 * size).all()      # float32 sums of k exact products
