@@ -446,24 +446,25 @@ __device__ __forceinline__ void attention_decode_part(
   // the (transposed) page, one 16-byte load a dim.  A key or eight keys that the token does not see
   // are read from the nearest it does see, not branched around (three branches were three trips to
   // memory one after the other): their scores are replaced, their values zeroed (work, below).
-  // A tile is two runs of 16 keys, each in one page (pages hold multiples of 16, tiles begin at multiples of 32), so pages are looked up
-  // for runs, with numbers that the whole wave shares; a run that the token does not see stands for the nearest that it does see.
+  // (A tile is two runs of 16 keys, each in one page; looked up once for the wave, with numbers that it shares, pages cost more than every lane's
+  // own lookup: heads that come prepared, batch 128 at 64 tokens 11.7 us by lane / 13.1, 32 tokens 11.1 / 12.7, 300 27.2 / 27.7, one request at 40 4.5 / 4.9;
+  // heads prepared here, 16 requests seeing 128 of 4,000 7.8 / 8.0, others the same.)
   const int key_of_row = (col >> 2) * 8 + (col & 3);           // + 4*h
-  const int first_run = lo / 16, last_run = pos / 16, page_runs = page_size / 16;
   // A key or value is read by one workgroup, once (load_once; 64 requests at 2,048 tokens, 8B sizes: 6,774 -> 6,618 us a step).  Not in
   // the form of eight waves: its short contexts of a few requests stay in the last-level cache from step to step, which what is
   // loaded with the hint does not (one request at 509 tokens, 0.6B sizes: 1,035 us a step, 1,078 with the hint).
   constexpr bool ONCE = WAVES == 4;
   auto fetch = [&](int tile, bf16x8 (&kf)[2][DS], bf16x8 (&vf)[DB]) {
-    const int run0 = __builtin_amdgcn_readfirstlane(max(first_run, min(last_run, tile * 2)));
-    const int run1 = __builtin_amdgcn_readfirstlane(max(first_run, min(last_run, tile * 2 + 1)));
-    const int block0 = run0 / page_runs, block1 = run1 / page_runs;
-    const int slot0 = (run0 - block0 * page_runs) * 16, slot1 = (run1 - block1 * page_runs) * 16;
-    const int64_t key_page = page_ids[(col < 8 ? block0 : block1) - first_block], value_page = page_ids[(g < 2 ? block0 : block1) - first_block];
     const bf16* kp[2];
-    kp[0] = k_pages + ((key_page * nkv + kvh) * page_size + (col < 8 ? slot0 : slot1) + key_of_row % 16) * D + g * 8;
-    kp[1] = kp[0] + 4 * D;
-    const bf16* vp = v_pages + (value_page * nkv + kvh) * (int64_t)dv * page_size + (int64_t)col * page_size + (g < 2 ? slot0 : slot1) + g % 2 * 8;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int key = max(lo, min(pos, tile * 32 + key_of_row + 4 * h));
+      const int64_t page = page_ids[key / page_size - first_block];
+      kp[h] = k_pages + ((page * nkv + kvh) * page_size + key % page_size) * D + g * 8;
+    }
+    const int key8 = max(lo & ~7, min(pos & ~7, tile * 32 + g * 8));         // this lane's eight keys; pages hold multiples of 16
+    const int64_t page = page_ids[key8 / page_size - first_block];
+    const bf16* vp = v_pages + (page * nkv + kvh) * (int64_t)dv * page_size + (int64_t)col * page_size + key8 % page_size;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
