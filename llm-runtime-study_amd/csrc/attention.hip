@@ -379,7 +379,7 @@ struct DecodeLds {
 };
 struct Inner { static constexpr bool value = false; };
 struct End { static constexpr bool value = true; };
-template <int D, bool PREP, int WAVES, bool AHEAD, bool MORE>
+template <int D, bool PREP, int WAVES, bool AHEAD, bool MORE, bool ONCE>
 __device__ __forceinline__ void attention_decode_part(
     DecodeLds<D, WAVES>& lds, int* page_ids, int split, int kvh, int token,
     bf16* __restrict__ out, int out_stride, float* __restrict__ part_o, float* __restrict__ part_ml,
@@ -406,8 +406,8 @@ __device__ __forceinline__ void attention_decode_part(
   const int tile_begin = first_tile + split * per_split;
   const int tile_end = tile_begin + per_split <= last_tile + 1 ? tile_begin + per_split : last_tile + 1;
   // PREP: the raw rows, the norms' weights and the rotation's tables are asked for now, before anything here waits for
-  // memory: they are there when the first keys are on their way.  (The new key's and value's by every wave, since which
-  // one walks the token's position is not known yet; they are the token's own, whichever workgroup does.)
+  // memory: they are there when the first keys are on their way.  (The new key and value too, since which workgroup walks the token's
+  // position is not known yet; they are the token's own, whichever does.)
   // One wave, the last, does so for the workgroup: eight that all did would ask their compute unit for 160 loads of rows, weights and
   // tables before the first keys.  The new key is prepared where the queries are, in the column behind the group's heads (a group of 16
   // leaves none: there it follows them).
@@ -450,10 +450,7 @@ __device__ __forceinline__ void attention_decode_part(
   // own lookup: heads that come prepared, batch 128 at 64 tokens 11.7 us by lane / 13.1, 32 tokens 11.1 / 12.7, 300 27.2 / 27.7, one request at 40 4.5 / 4.9;
   // heads prepared here, 16 requests seeing 128 of 4,000 7.8 / 8.0, others the same.)
   const int key_of_row = (col >> 2) * 8 + (col & 3);           // + 4*h
-  // A key or value is read by one workgroup, once (load_once; 64 requests at 2,048 tokens, 8B sizes: 6,774 -> 6,618 us a step).  Not in
-  // the form of eight waves: its short contexts of a few requests stay in the last-level cache from step to step, which what is
-  // loaded with the hint does not (one request at 509 tokens, 0.6B sizes: 1,035 us a step, 1,078 with the hint).
-  constexpr bool ONCE = WAVES == 4;
+  // (ONCE: with the hint that says that a key or value is read by this workgroup alone, see lrs_attention_decode)
   auto fetch = [&](int tile, bf16x8 (&kf)[2][DS], bf16x8 (&vf)[DB]) {
     const bf16* kp[2];
 #pragma unroll
@@ -693,7 +690,7 @@ __device__ __forceinline__ void attention_decode_part(
   }
 }
 
-template <int D, bool PREP, int WAVES, bool AHEAD, bool MORE>
+template <int D, bool PREP, int WAVES, bool AHEAD, bool MORE, bool ONCE = false>
 __global__ __launch_bounds__(WAVES * 64, WAVES == 4 && D == 128 ? 2 : 1) void attention_decode_bf16_kernel(
     const int* __restrict__ positions, const int* __restrict__ token_request, const int* __restrict__ block_table, const bf16* __restrict__ q,
     int table_stride, int q_stride, int nq, int nkv, int page_size, int splits, bf16* __restrict__ out, int out_stride,
@@ -704,7 +701,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 && D == 128 ? 2 : 1) void at
   // compiled so), the others are a trip to memory away.
   __shared__ DecodeLds<D, WAVES> lds;
   extern __shared__ int page_ids[];
-  attention_decode_part<D, PREP, WAVES, AHEAD, MORE>(lds, page_ids, blockIdx.x, blockIdx.y, blockIdx.z, out, out_stride, part_o, part_ml, q, q_stride, k_pages, v_pages, block_table, table_stride, token_request, positions, nq, nkv, page_size, scale, window, splits, slots, prep, sinks, softcap, gates, gate_stride, dv_given, distance_given, distance_form);
+  attention_decode_part<D, PREP, WAVES, AHEAD, MORE, ONCE>(lds, page_ids, blockIdx.x, blockIdx.y, blockIdx.z, out, out_stride, part_o, part_ml, q, q_stride, k_pages, v_pages, block_table, table_stride, token_request, positions, nq, nkv, page_size, scale, window, splits, slots, prep, sinks, softcap, gates, gate_stride, dv_given, distance_given, distance_form);
 }
 
 // Merges the partial results of the splits of one (token, head): out = sum_s o_s 2^(m_s - m) / sum_s l_s 2^(m_s - m).
@@ -913,7 +910,7 @@ LRS_API int lrs_attention_decode(void* out, int out_stride, float* part_o, float
               "attention_decode: kept first positions (%d) need a window and prepared heads", keep_first);
   const int slots = splits + (keep_first > 0 ? 1 : 0);          // the kept keys' share is one more partial result
   LRS_REQUIRE(splits >= 1 && (slots == 1 || (part_o && part_ml)), "attention_decode: %d partial results need their buffers", slots);
-  LRS_REQUIRE(form >= 0 && form <= 2, "attention_decode: form must be 0, 1 or 2, got %d", form);
+  LRS_REQUIRE(form >= 0 && form <= 3, "attention_decode: form must be 0, 1, 2 or 3, got %d", form);
   LRS_REQUIRE(softcap >= 0.f, "attention_decode: the cap on the scores must be positive (0 = none), got %g", (double)softcap);
   LRS_REQUIRE(q_stride % 8 == 0 && ((uintptr_t)q % 16) == 0, "attention_decode: q rows must be 16-byte aligned");
   dim3 grid(splits, nkv, tokens);
@@ -935,8 +932,9 @@ LRS_API int lrs_attention_decode(void* out, int out_stride, float* part_o, float
                 "attention_decode: norm weights and rotation tables must be 16-byte aligned");
   }
   const DecodePrep prep{q_weight, k_weight, w_dtype == LRS_F32, eps, cosv, sinv, kv_columns};
-  // `form`: 0 = four waves, a tile at a time; 1 = four waves, 2 = eight waves, each wave with its next
-  // tile on the way while it works (heads of 192 dims have no registers for that and stay with 0)
+  // `form`: 0 = four waves, a tile at a time; 1 and 3 = four waves, 2 = eight waves, each wave with its next
+  // tile on the way while it works (heads of 192 dims have no registers for that and stay with 0); 3 loads keys and values with the
+  // streaming hint (load_once), which pays where a step's keys are many and a workgroup's as well: _keys_read_once in parts/attention.py
 #define ARGS                                                                                                 \
   positions, token_request, block_table, (const bf16*)q, table_stride, q_stride, nq, nkv, page_size, splits, (bf16*)out, out_stride, part_o, \
       part_ml, (bf16*)k_pages, (bf16*)v_pages, scale, window, slots, prep, slots == 1 ? sinks : nullptr, softcap, \
@@ -944,6 +942,7 @@ LRS_API int lrs_attention_decode(void* out, int out_stride, float* part_o, float
 #define LAUNCH_PREP(D, PREP, MORE)                                                                           \
   do {                                                                                                       \
     if (form == 2 && D <= 128) attention_decode_bf16_kernel<D, PREP, 8, (D <= 128), MORE><<<grid, 512, table_lds, s>>>(ARGS); \
+    else if (form == 3 && D <= 128) attention_decode_bf16_kernel<D, PREP, 4, (D <= 128), MORE, (D <= 128)><<<grid, 256, table_lds, s>>>(ARGS); \
     else if (form == 1 && D <= 128) attention_decode_bf16_kernel<D, PREP, 4, (D <= 128), MORE><<<grid, 256, table_lds, s>>>(ARGS); \
     else attention_decode_bf16_kernel<D, PREP, 4, false, MORE><<<grid, 256, table_lds, s>>>(ARGS);             \
   } while (0)
@@ -2048,9 +2047,16 @@ __global__ __launch_bounds__(256, 2) void attention_mixed_d128_kernel(
   extern __shared__ int page_ids[];
   const int single_blocks = singles * nkv;
   if ((int)blockIdx.x < single_blocks) {
-    attention_decode_part<128, PREP, 4, true, false>(lds.single, page_ids, 0, blockIdx.x % nkv, blockIdx.x / nkv, out, out_stride, nullptr, nullptr,
-                                                     q, q_stride, k_pages, v_pages, block_table, table_stride, token_request, positions, nq, nkv,
-                                                     page_size, scale, window, 1, 1, prep, nullptr, 0.f, nullptr, 0, 128, nullptr, 0);
+    // The hint (load_once) for pages whose lines a wave reads alone, see _keys_read_once in parts/attention.py; whole steps with it / without, 24 requests at
+    // 1,500 beside 488 tokens after 488 7,516 / 7,545 us (36 layers of the 4B sizes) and 4,241 / 4,177 (28 of the 1.7B), 40 at 800 beside 1,900 19,702 / 19,809
+    // and 8,662 / 8,787, 8 at 4,000 beside 1,000 12,345 / 12,335 and 5,954 / 5,924.  Larger pages have the kernel alone take 49.0 / 44.7 for the first.
+    auto one = [&](auto once) {
+      attention_decode_part<128, PREP, 4, true, false, decltype(once)::value>(
+          lds.single, page_ids, 0, blockIdx.x % nkv, blockIdx.x / nkv, out, out_stride, nullptr, nullptr, q, q_stride, k_pages, v_pages, block_table, table_stride,
+          token_request, positions, nq, nkv, page_size, scale, window, 1, 1, prep, nullptr, 0.f, nullptr, 0, 128, nullptr, 0);
+    };
+    if (page_size <= 32) one(std::true_type{});
+    else one(std::false_type{});
     return;
   }
   DecodePrep rest = prep;                                                  // the tables' rows of the tokens behind

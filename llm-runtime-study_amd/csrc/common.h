@@ -123,7 +123,8 @@ __device__ __forceinline__ void fetched_and_read_then_barrier() {
 // A load of what this launch reads once and nobody reads again soon (a decode step's weights and cached keys), with the hint that says
 // so: the L2s give its line up first.  Without it some 4 MB of weights a layer and die push out what the step keeps there, the rows that
 // travel between its kernels, norm weights and kernels' own arguments, and the next kernel begins by fetching those from far away: a
-// norm of 8 rows behind a plain read of 32 MB takes 4.05 us, behind a read with the hint 2.74 (2.80 by itself).  For loads of whole
-// 128-byte lines: the other half of a line that a later instruction asks for may be gone again.
+// norm of 8 rows behind a plain read of 32 MB takes 4.05 us, behind a read with the hint 2.74 (2.80 by itself).  For lines of 128 bytes
+// that one wave asks for whole, in an instruction or in a few that follow each other (a key's 256 bytes in four): the half that another wave or a
+// later tile asks for is gone again.  And not for what several workgroups read, or what a cache could keep until the next step.
 template <typename V>
 __device__ __forceinline__ V load_once(const V* at) { return __builtin_nontemporal_load(at); }

@@ -268,6 +268,23 @@ class GQAAttention(Part):
             wanted = thrice if 2 * thrice > 3 * twice else twice
         return max(1, min(wanted, most), -(-bound // (4096 * page_size))), 2
 
+    def _keys_read_once(self, splits: int, form: int, longest: int, page_size: int) -> int:
+        """`form` of a shape that _decode_shape() gave, 3 in place of 1 where keys and values are better loaded with the hint that they are read
+        once (csrc/common.h, load_once).  us without / with it, keys that no cache holds, heads of 128 on 8 kv heads unless it says otherwise:
+          * Workgroups that walk 128 keys and more, as their contexts' class or the window says: waves without a tile of their own bring
+            their workgroup's last once more, which the hint has them fetch again.  Contexts of a half up to all of 64, 150, 300 and 450 tokens:
+            batch 128 13.0 / 14.6, 18.1 / 17.4, 27.6 / 26.6, 38.1 / 36.6, batch 33 6.4 / 6.9, 8.4 / 8.5, 11.8 / 12.1, 16.4 / 16.8; batch 64 seeing 128 of 4,000
+            tokens 11.8 / 11.1, 512 29.7 / 27.6; batch 8 at 8,000 in 8 parts 52.0 / 47.9; heads of 64, batch 64 at 1,000 42.6 / 39.6.  (So many keys
+            of as many workgroups as go with four waves are tens of MB a layer: no cache keeps them until the next step.)
+          * Pages of up to 32, whose tiles have the lines of values to themselves; of larger ones the next tile, another wave's, has the other
+            half: batch 64 at 2,048 in pages of 16, 32, 64 and 256 99.1 / 87.1, 100.1 / 90.0, 105.8 / 110.1 and 107.2 / 114.4.
+          * Heads of up to 128: those of 192 bring a tile at a time (batch 40 at 600 31.1 / 33.7, batch 16 at 4,000 in 4 parts 68.5 / 65.5, one
+            request at 1,000 in 3 of 28 layers' keys 13.8 / 15.3).
+        Workgroups of eight waves walk contexts of few requests, which the last-level cache keeps from step to step unless they are
+        loaded so (one request at 509 tokens, 0.6B sizes, 1,035 us a step / 1,078)."""
+        seen = length_class(longest) if self.span is None else min(length_class(longest), self.span)
+        return 3 if form == 1 and self.head_dim <= 128 and page_size <= 32 and seen // splits >= 128 else form
+
     @staticmethod
     def _walks_in_pairs(ctx, heads_per_group: int, head_dim: int) -> bool:
         """Whether the kernel for ragged steps lets two neighbouring query groups walk their keys together (attention_prefill's
@@ -398,7 +415,7 @@ class GQAAttention(Part):
                 part_ml = ctx.scratch("attn_part_ml", (t, nq * splits * 2), torch.float32)
             ops.attention_decode(out, qkv, cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot, ctx.positions,
                                  nq, self.scale, self.reach, splits, part_o, part_ml, ctx.max_k_bound, prepare,
-                                 form=form)   # the next tile on its way while one is worked on, the first one before the query is prepared (measured: 0.6 % of a step)
+                                 form=self._keys_read_once(splits, form, ctx.max_k, group.page_size))   # the next tile on its way while one is worked on, the first one before the query is prepared (measured: 0.6 % of a step)
         elif ops.attention_decode_supported(ctx.dtype, nq, kv_heads, d, group.page_size):
             # sized by the step's coarse bound of the longest context, the same for every step of one shape
             longest = ctx.max_k_bound if self.span is None else min(ctx.max_k_bound, self.span + 64)
@@ -430,7 +447,8 @@ class GQAAttention(Part):
                     first = ops.DecodePrepare(self.q_norm, self.k_norm, self.qk_norm_eps, None if parted is None else parted[0],
                                               None if parted is None else parted[1], 0)
                 ops.attention_decode(out[:singles], qkv[:singles], cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot,
-                                     ctx.positions, nq, self.scale, self.reach, splits, part_o, part_ml, ctx.max_k_bound, first, form=form)
+                                     ctx.positions, nq, self.scale, self.reach, splits, part_o, part_ml, ctx.max_k_bound, first,
+                                     form=self._keys_read_once(splits, form, ctx.max_k_bound, group.page_size))
             rest = ctx.memo.get("rows_after_singles")
             if rest is None:
                 rest = ctx.memo["rows_after_singles"] = (ctx.token_slot[singles:], ctx.positions[singles:])
@@ -504,7 +522,8 @@ class GQAAttention(Part):
                 part_o = ctx.scratch("attn_part_o", (t, nq * (splits + extra) * dv), torch.float32)
                 part_ml = ctx.scratch("attn_part_ml", (t, nq * (splits + extra) * 2), torch.float32)
             ops.attention_decode(out, qkv, cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot, ctx.positions,
-                                 nq, self.scale, self.reach, splits, part_o, part_ml, ctx.max_k_bound, prepare, form=form,
+                                 nq, self.scale, self.reach, splits, part_o, part_ml, ctx.max_k_bound, prepare,
+                                 form=self._keys_read_once(splits, form, ctx.max_k, group.page_size),
                                  keep_first=self.keep_first, gates=gates, **more)
         elif cores:
             longest = ctx.max_k_bound if self.span is None else min(ctx.max_k_bound, self.span + 64)
@@ -516,7 +535,8 @@ class GQAAttention(Part):
                     part_o = ctx.scratch("attn_single_part_o", (singles, nq * (splits + extra) * dv), torch.float32)
                     part_ml = ctx.scratch("attn_single_part_ml", (singles, nq * (splits + extra) * 2), torch.float32)
                 ops.attention_decode(out[:singles], qkv[:singles], cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot,
-                                     ctx.positions, nq, self.scale, self.reach, splits, part_o, part_ml, ctx.max_k_bound, None, form=form,
+                                     ctx.positions, nq, self.scale, self.reach, splits, part_o, part_ml, ctx.max_k_bound, None,
+                                     form=self._keys_read_once(splits, form, ctx.max_k_bound, group.page_size),
                                      keep_first=self.keep_first, gates=None if gates is None else gates[:singles], **more)
             rest = ctx.memo.get("rows_after_singles")
             if rest is None:

@@ -29,6 +29,17 @@ def test_parts_of_a_decode_step(monkeypatch, head_dim):
             assert longest < 4096 or splits >= 0.45 * GQAAttention._decode_splits(workgroups, longest, longest, 16)
 
 
+@pytest.mark.parametrize("head_dim,page,longest,window,splits,form,wanted", [
+    (128, 16, 255, None, 1, 1, 1), (128, 16, 256, None, 1, 1, 3), (64, 32, 2048, None, 1, 1, 3), (128, 16, 2048, None, 4, 2, 2),      # short ones; eight waves
+    (128, 48, 2048, None, 1, 1, 1), (64, 64, 2048, None, 1, 1, 1), (192, 16, 8192, None, 2, 1, 1),                                  # pages and heads
+    (128, 16, 4096, None, 16, 1, 3), (128, 16, 4096, None, 64, 1, 1), (128, 16, 4096, 128, 1, 1, 3), (128, 16, 4096, 64, 1, 1, 1)])   # a workgroup's share
+def test_which_keys_are_loaded_as_read_once(head_dim, page, longest, window, splits, form, wanted):
+    """Form 3 where a workgroup walks 128 keys and more, of pages and heads whose lines it reads alone."""
+    part = GQAAttention.__new__(GQAAttention)
+    part.head_dim, part.span = head_dim, window
+    assert part._keys_read_once(splits, form, longest, page) == wanted
+
+
 def test_which_mixed_steps_go_in_one_launch(monkeypatch):
     monkeypatch.setattr(ops, "compute_units", lambda: 256)
 

@@ -1,5 +1,5 @@
-"""Weights that several workgroups read side by side are loaded without the hint that gives their lines up.  Read from the library as it
-was built."""
+"""What several workgroups read side by side, or a cache keeps until the next step, is loaded without the hint that gives its lines up.
+Read from the library as it was built."""
 
 import re
 import shutil
@@ -34,3 +34,14 @@ def test_experts_with_several_tiles_share_their_weights(tmp_path):
     for name, (once, shared) in found.items():
         weights = int(re.search(r"Li(\d+)E", name)[1]) // 32
         assert once >= weights and shared >= weights + 2, (name, once, shared)
+
+
+def test_decode_attention_has_both(tmp_path):
+    """Keys and values with the hint in the one form for it and without in the others; beside a prompt portion with and without, by the size
+    of the pages (eight values and eight keys a tile, asked for at two places and more)."""
+    found = wide_loads(tmp_path, "attention_decode_bf16_kernel")
+    asked = {name: counts for name, counts in found.items() if re.search(r"Lb[01]ELi4ELb[01]ELb[01]ELb1E", name)}
+    assert len(asked) >= 12 and all(once > 0 for once, _ in asked.values())
+    assert not any(once for name, (once, _) in found.items() if name not in asked)
+    mixed = wide_loads(tmp_path, "attention_mixed_d128_kernel")
+    assert mixed and all(once >= 32 and plain >= 32 for once, plain in mixed.values())
