@@ -46,7 +46,7 @@ def test_product_that_begins_the_next_norm(m, n, k, weight_dtype):
     torch.testing.assert_close(sums.cpu().double().sum(0), want.pow(2).sum(1), rtol=2 ** -16, atol=0.0)
 
 
-@pytest.mark.parametrize("hidden", [4, 252, 256, 260, 1020, 1024, 1028, 4096, 4100, 8192])
+@pytest.mark.parametrize("hidden", [4, 252, 256, 260, 600, 1020, 1024, 1028, 2052, 4096, 4100, 6148, 8192])
 @pytest.mark.parametrize("weight_dtype,out_dtype", [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32), (torch.bfloat16, torch.float32)])
 def test_norms_of_rows_of_any_length(hidden, weight_dtype, out_dtype):
     """Rows that end inside, at and behind the last chunk a thread owns: plain, gathered, and with a product's output added first (which
