@@ -716,26 +716,27 @@ __global__ __launch_bounds__(256) void latent_attention_shared_kernel(
   }
 }
 
-// What the parts of one (token, head) left, put together: maxima and sums in powers of two.  A thread four dims, sixteen parts asked for at
+// What the parts of one (token, head) left, put together: maxima and sums in powers of two.  A thread four dims, AT_ONCE parts asked for at
 // a time, the first of them before their weights are known: two trips to memory where a dim a thread and eight parts at a time made
-// eight (16 tokens, 32 heads of rank 512 in 32 parts 11.8 -> 8.2 us; the bytes are 6.4).
-constexpr int MERGE_THREADS = 128;
+// eight (16 tokens, 32 heads of rank 512 in 32 parts 11.8 -> 8.2 us; the bytes are 6.4).  Four at a time for up to four parts: a part that is not there
+// is a load all the same (16 tokens, rank 128 in two parts, the walk with it, 14.1 us with sixteen, 13.2).
+constexpr int MERGE_THREADS = 128;      // the ranks that lrs_latent_attention_groups takes, four dims each
+template <int AT_ONCE>
 __global__ __launch_bounds__(MERGE_THREADS) void latent_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml, int heads, int rank, int splits,
                                                                      int out_stride, bf16* __restrict__ out, const float* __restrict__ sink,
                                                                      const bf16* __restrict__ gate, int gate_stride) {
   __shared__ float weight[64];          // of each part: 2^(its maximum - the maximum of all), over the denominator, times the gate
-  constexpr int AT_ONCE = 16;
   const int token = blockIdx.x, head = blockIdx.y, lane = threadIdx.x;
   const int64_t base = ((int64_t)token * heads + head) * splits;
+  const int dim = lane * 4 < rank ? lane * 4 : rank - 4;
   floatx4 o[AT_ONCE];
-  auto ask = [&](int s0, int dim) {
+  auto ask = [&](int s0) {
 #pragma unroll
     for (int i = 0; i < AT_ONCE; ++i) o[i] = *(const floatx4*)(part_o + (base + (s0 + i < splits ? s0 + i : splits - 1)) * rank + dim);
   };
-  const int first = lane * 4 < rank ? lane * 4 : rank - 4;
   const int mine_at = lane < splits ? lane : splits - 1;
   const float mine_max = part_ml[(base + mine_at) * 2], mine_sum = part_ml[(base + mine_at) * 2 + 1];
-  ask(0, first);
+  ask(0);
   if (lane < WAVE) {                    // the first wave: a part a lane (splits <= 64)
     const float mine = lane < splits ? mine_max : -INFINITY;
     const float sum = lane < splits ? mine_sum : 0.f;
@@ -748,21 +749,19 @@ __global__ __launch_bounds__(MERGE_THREADS) void latent_merge_kernel(const float
     weight[lane] = w * factor;
   }
   __syncthreads();
-  for (int dim = lane * 4; dim < rank; dim += MERGE_THREADS * 4) {
-    if (dim != first) ask(0, dim);
-    floatx4 sum = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < splits; s0 += AT_ONCE) {
-      if (s0) ask(s0, dim);
+  if (lane * 4 >= rank) return;
+  floatx4 sum = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < splits; s0 += AT_ONCE) {
+    if (s0) ask(s0);
 #pragma unroll
-      for (int i = 0; i < AT_ONCE; ++i)
-        if (s0 + i < splits)
+    for (int i = 0; i < AT_ONCE; ++i)
+      if (s0 + i < splits)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) sum[e] = fmaf(o[i][e], weight[s0 + i], sum[e]);
-    }
-    bf16* to = out + (int64_t)token * out_stride + (int64_t)head * rank + dim;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) to[e] = (bf16)sum[e];
+        for (int e = 0; e < 4; ++e) sum[e] = fmaf(o[i][e], weight[s0 + i], sum[e]);
   }
+  bf16* to = out + (int64_t)token * out_stride + (int64_t)head * rank + dim;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) to[e] = (bf16)sum[e];
 }
 
 // The same for ranks and places that four dims a load do not fit.
@@ -888,7 +887,7 @@ LRS_API int lrs_latent_attention(void* out, int out_stride, const void* queries,
 
 // Whether lrs_latent_attention_groups takes the shape.
 LRS_API int lrs_latent_attention_groups_takes(int rank, int width, int page_size) {
-  return rank > 0 && rank <= 512 && width >= rank && width % 8 == 0 && page_size % 8 == 0;
+  return rank > 0 && rank <= MERGE_THREADS * 4 && width >= rank && width % 8 == 0 && page_size % 8 == 0;
 }
 
 // Whether its tiles go through LDS that a workgroup shares (one workgroup a compute unit) rather than into every wave's registers.
@@ -943,8 +942,10 @@ LRS_API int lrs_latent_attention_groups(void* out, int out_stride, const void* q
   if (splits > 1) {
     if (rank % 4 != 0 || (uintptr_t)part_o % 16 != 0)
       latent_merge_any_kernel<<<dim3(tokens, heads), 256, 0, s>>>((bf16*)out, out_stride, part_o, part_ml, sink, (const bf16*)gate, gate_stride, heads, rank, splits);
+    else if (splits <= 4)
+      latent_merge_kernel<4><<<dim3(tokens, heads), MERGE_THREADS, 0, s>>>(part_o, part_ml, heads, rank, splits, out_stride, (bf16*)out, sink, (const bf16*)gate, gate_stride);
     else
-      latent_merge_kernel<<<dim3(tokens, heads), MERGE_THREADS, 0, s>>>(part_o, part_ml, heads, rank, splits, out_stride, (bf16*)out, sink, (const bf16*)gate, gate_stride);
+      latent_merge_kernel<16><<<dim3(tokens, heads), MERGE_THREADS, 0, s>>>(part_o, part_ml, heads, rank, splits, out_stride, (bf16*)out, sink, (const bf16*)gate, gate_stride);
     return lrs_check_launch("latent_attention_groups merge");
   }
   return 0;

@@ -7,7 +7,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("rank,width", [(512, 576), (128, 192), (500, 504), (42, 48), (4, 8)])
-@pytest.mark.parametrize("splits", [2, 15, 17, 64])
+@pytest.mark.parametrize("splits", [2, 4, 5, 15, 17, 64])
 def test_parts_meet_as_if_undivided(rank, width, splits):
     """Against the same walk undivided: sums of 32 bits in another order, weights and results rounded to bfloat16 (2^-8 of values of order one,
     twice)."""
