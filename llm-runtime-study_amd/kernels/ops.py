@@ -1485,6 +1485,9 @@ def choose_tokens_static(out: torch.Tensor, logits: torch.Tensor, parts: int, te
         None if temperature is None else _dev(counters, "counters"), parts, int(bool(filtered)), _stream())
 
 
+FILTER_WIDE = 20000     # values of a row from which filter_logits() works on it with the whole chip
+
+
 def filter_words() -> int:
     """Words of workspace that filter_logits() wants for a row."""
     return library().lrs_filter_words()
@@ -1494,8 +1497,9 @@ def filter_logits(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.
                   workspace: torch.Tensor | None = None) -> None:
     """Drops (sets to -inf, in place) what top-k and top-p leave out of rows of positive temperature.
 
-    workspace: the caller's own device memory, int32 [R or more, filter_words()], all zero before its first use (every call leaves it
-    so) and used on one stream at a time: large vocabularies are then worked on by the whole chip."""
+    workspace: the caller's own device memory, int32 [R or more, filter_words()], all zero before its first use, left to these calls from
+    then on (each leaves zero what the next one counts in; the list and the threshold behind it stay written) and used on one stream at
+    a time: large vocabularies are then worked on by the whole chip."""
     rows, vocab = logits.shape
     stride = _rows(logits, "logits")
     _need(temperature.dtype == torch.float32 and temperature.numel() >= rows, "filter_logits: temperature must be float32 [R]")
@@ -1507,7 +1511,9 @@ def filter_logits(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.
             None if top_k is None else _dev(top_k, "top_k"), None if top_p is None else _dev(top_p, "top_p"))
     if workspace is not None:
         _need(workspace.dtype == torch.int32 and workspace.is_contiguous() and workspace.numel() >= rows * filter_words(), f"filter_logits: workspace must be contiguous int32, {filter_words()} words a row")
-        if vocab >= 16384 and rows <= 65535:
+        # us over the chip / in one kernel: 16,384 values of 64 rows k 50 23 / 20, p 0.9 29 / 24, both 32 / 35; 20,000 of them 18 / 22, 26 / 27 and 26 / 39, of one
+        # row 19 / 23, 28 / 26 and 28 / 40; 24,576 of 8 rows 17 / 24, 26 / 28 and 26 / 42
+        if vocab >= FILTER_WIDE and rows <= 65535:
             _launch("lrs_filter_logits_wide", *args, _dev(workspace, "workspace"), _stream())
             return
     _launch("lrs_filter_logits", *args, _stream())

@@ -1,4 +1,4 @@
-"""Top-k and top-p over the whole chip: bit for bit what the one-kernel form keeps, and a workspace left as it was found."""
+"""Top-k and top-p over the whole chip: bit for bit what the one-kernel form keeps, and a workspace left with zeros where the next call counts."""
 
 import pytest
 import torch
@@ -6,7 +6,8 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("vocab,stride,offset", [(151936, 151936, 0), (16384, 16384, 0), (16387, 16388, 0), (50257, 50257, 0), (20479, 20480, 1)])
+@pytest.mark.parametrize("vocab,stride,offset", [(151936, 151936, 0), (16384, 16384, 0), (16387, 16388, 0), (50257, 50257, 0), (20479, 20480, 1), (20000, 20000, 0),
+                                                 (20480, 20480, 0), (20483, 20484, 0)])
 def test_keeps_what_the_one_kernel_form_keeps(vocab, stride, offset):
     """Rows whose values spread, crowd into a bin (more than a list holds), tie at the threshold, or are not finite; greedy rows; k and p
     alone, together and off; rows that do not begin on 16 bytes.  Called twice: the second call finds the workspace zero."""
@@ -33,7 +34,10 @@ def test_keeps_what_the_one_kernel_form_keeps(vocab, stride, offset):
         want, got = (w.contiguous().view(torch.int32) for w in both)
         assert torch.equal(torch.isnan(both[0]), torch.isnan(both[1]))
         assert torch.equal(got.masked_fill(torch.isnan(both[1]), 0), want.masked_fill(torch.isnan(both[0]), 0))
-        assert not space[:, :4096 - 2048].clone().masked_fill_(torch.arange(2048, device="cuda") == 3, 0).any()
+        # the words before the list, but the threshold (whose place is the head's fourth): what the next call counts in
+        counted = ops.filter_words() - 4096
+        assert counted == 16 + 2048
+        assert not space[:, :counted].masked_fill(torch.arange(counted, device="cuda") == 3, 0).any()
     assert torch.isinf(both[1]).any()
 
 
