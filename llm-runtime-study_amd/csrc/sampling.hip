@@ -441,13 +441,14 @@ __global__ __launch_bounds__(1024) void filter_logits_kernel(float* __restrict__
 }
 
 // The same in four launches over the chip, for large vocabularies and callers that bring a workspace of FILTER_WORDS words a row, all
-// zero before the first call (each call leaves it so): (1) slices of a row look for its largest value, for values that are not finite, and
+// zero before the first call (each call leaves the counts and the words before FILTER_THRESHOLD so; the threshold and the list are
+// written before they are read): (1) slices of a row look for its largest value, for values that are not finite, and
 // count by the first digit; (2) the values from the k-th largest's bin up, usually a few dozen to a few hundred, are collected in a list;
 // (3) one workgroup a row selects among the list's, or among all of the row's where there is no k or the list is too short; (4) slices
-// drop what lies under the threshold and clear the workspace.  The thresholds are those of the one-kernel form: a list holds everything
+// drop what lies under the threshold and clear what was counted.  The thresholds are those of the one-kernel form: a list holds everything
 // at or above the k-th largest value, and a share of the mass is one of the values that the k leaves.  One workgroup a row reads 608 KB
-// at the rate of one compute unit, eight times over: 8 rows of 151,936 with k 50 and p 0.9 188 us a call, 48 here
-// (64 rows 209 / 68; a share of the mass alone 151 / 115).
+// at the rate of one compute unit, eight times over: 8 rows of 151,936 with k 50 and p 0.9 186 us a call, 34 here
+// (64 rows 200 / 64; a share of the mass alone 142 / 107).
 constexpr int FILTER_SLICE = 4096, FILTER_LIST = 4096, FILTER_THREADS = 256;
 constexpr int FILTER_HEAD = 16, FILTER_WORDS = FILTER_HEAD + FILTER_BINS + FILTER_LIST;
 enum { FILTER_MAX = 0, FILTER_BAD = 1, FILTER_COUNT = 2, FILTER_THRESHOLD = 3 };      // words of a row's head

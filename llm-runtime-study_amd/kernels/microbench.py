@@ -160,13 +160,15 @@ def sampling(args) -> None:
             top_k = torch.full((rows,), k, dtype=torch.int32, device="cuda")
             top_p = torch.full((rows,), p, device="cuda")
 
-            def call(i):
-                copies[i % 8].copy_(base)             # the filter writes into the logits: a fresh copy every time
-                ops.filter_logits(copies[i % 8], temperature, top_k, top_p)
-
             copy_only = _time(lambda i: copies[i % 8].copy_(base), args.repeats)
-            seconds = _time(call, args.repeats) - copy_only
-            print(f"sampling rows={rows:3d} vocab={vocab} filter_logits {name:20s} {seconds * 1e6:8.1f} us", flush=True)
+            # with a workspace, as steps and samplers call it (the whole chip for large vocabularies), and without (one kernel)
+            for form, workspace in (("with a workspace", torch.zeros(rows, ops.filter_words(), dtype=torch.int32, device="cuda")), ("without", None)):
+                def call(i):
+                    copies[i % 8].copy_(base)             # the filter writes into the logits: a fresh copy every time
+                    ops.filter_logits(copies[i % 8], temperature, top_k, top_p, workspace)
+
+                seconds = _time(call, args.repeats) - copy_only
+                print(f"sampling rows={rows:3d} vocab={vocab} filter_logits {name:20s} {form:16s} {seconds * 1e6:8.1f} us", flush=True)
         for name, drawn in (("greedy", False), ("drawn", True)):
             seconds = _time(lambda i: ops.choose_tokens(out, base, *((temperature, seeds, counters) if drawn else ())), args.repeats)
             print(f"sampling rows={rows:3d} vocab={vocab} choose_tokens {name:20s} {seconds * 1e6:8.1f} us", flush=True)

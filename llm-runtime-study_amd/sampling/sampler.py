@@ -49,7 +49,7 @@ class Sampler:
         self._chosen_address = 0  # ... and where the device sees it
         self._settings_host = self._settings_dev = None   # the rows' sampling settings: pinned staging and its device copy
         self._settings_cap = 0
-        self._filter_space = None     # what filter_logits() leaves as it found it: all zero
+        self._filter_space = None     # filter_logits()' workspace: zeroed when it is made, then its own
 
     def _settings_room(self, rows: int) -> int:
         """Staging for `rows` rows' settings (six int32 words a row, in five arrays of `cap` rows); returns cap.  The
