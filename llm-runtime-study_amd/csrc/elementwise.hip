@@ -14,21 +14,30 @@ __global__ void embed_kernel(float* __restrict__ out, const T* __restrict__ tabl
   for (int i = threadIdx.x; i < hidden; i += blockDim.x) dst[i] = to_float(src[i]) * multiplier;
 }
 
-// The same eight values a thread, 16 bytes a load: what bounds it is the trips to the token's id and to its row, which 4,096 columns in
-// one workgroup made sixteen of; of many tokens the bytes (graph nodes of 16 tokens of 4,096 3.4 -> 2.0 us, of 2,048 tokens 16.5 -> 12.5).
-template <typename T>
+// The same four or eight values a thread: what bounds it is the trips to the token's id and to its row, which 4,096 columns in one workgroup
+// made sixteen of; of many tokens the bytes.
+template <typename T, int EACH>
 __global__ __launch_bounds__(256) void embed_vec_kernel(const int* __restrict__ ids, const T* __restrict__ table, float* __restrict__ out, int pieces,
                                                         int per_row, float multiplier) {
-  typedef T vec __attribute__((ext_vector_type(8)));
+  typedef T vec __attribute__((ext_vector_type(EACH)));
   const int at = blockIdx.x * 256 + threadIdx.x;
   if (at >= pieces) return;
   const int64_t row = ids[at / per_row];
   const vec v = ((const vec*)table)[row * per_row + at % per_row];
-  floatx4 lo, hi;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) lo[i] = to_float(v[i]) * multiplier, hi[i] = to_float(v[4 + i]) * multiplier;
-  ((floatx4*)out)[(int64_t)at * 2] = lo;
-  ((floatx4*)out)[(int64_t)at * 2 + 1] = hi;
+  for (int h = 0; h < EACH / 4; ++h) {
+    floatx4 f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f[i] = to_float(v[h * 4 + i]) * multiplier;
+    ((floatx4*)out)[(int64_t)at * (EACH / 4) + h] = f;
+  }
+}
+
+template <int EACH>
+static void launch_embed_vec(float* out, const void* table, int dtype, const int* ids, int tokens, int hidden, float multiplier, hipStream_t s) {
+  const int per_row = hidden / EACH, pieces = tokens * per_row, groups = (pieces + 255) / 256;
+  if (dtype == LRS_F32) embed_vec_kernel<float, EACH><<<groups, 256, 0, s>>>(ids, (const float*)table, out, pieces, per_row, multiplier);
+  else embed_vec_kernel<bf16, EACH><<<groups, 256, 0, s>>>(ids, (const bf16*)table, out, pieces, per_row, multiplier);
 }
 
 LRS_API int lrs_embed(float* out, const void* table, int dtype, const int* ids, int tokens,
@@ -36,9 +45,13 @@ LRS_API int lrs_embed(float* out, const void* table, int dtype, const int* ids, 
   LRS_REQUIRE(tokens > 0 && hidden > 0, "embed: tokens=%d hidden=%d must be positive", tokens, hidden);
   dim3 grid(tokens), block(256);
   if (hidden % 8 == 0 && ((uintptr_t)table | (uintptr_t)out) % 32 == 0 && (int64_t)tokens * (hidden / 8) < (1ll << 30) && (dtype == LRS_F32 || dtype == LRS_BF16)) {
-    const int per_row = hidden / 8, pieces = tokens * per_row, groups = (pieces + 255) / 256;
-    if (dtype == LRS_F32) embed_vec_kernel<float><<<groups, 256, 0, (hipStream_t)stream>>>(ids, (const float*)table, out, pieces, per_row, multiplier);
-    else embed_vec_kernel<bf16><<<groups, 256, 0, (hipStream_t)stream>>>(ids, (const bf16*)table, out, pieces, per_row, multiplier);
+    // Four, so that a wave's store fills whole lines; eight for few rows, whose trips more workgroups only lengthen, and where what is written no longer
+    // stays in the last-level cache.  us, one value a thread / eight / four, bfloat16 rows: 1 of 4,096 3.2 / 1.87 / 2.05, 16 of 8,192 5.4 / 2.07 / 2.12; 512 of
+    // 1,024 2.24 / 2.23 / 2.15, 2,048 of 1,024 3.60 / 3.88 / 3.38, of 4,096 9.9 / 9.7 / 8.4, 12,288 of 4,096 (192 MB) 46.1 / 43.4 / 40.6; 6,144 float32 rows of 8,192 (the
+    // same) 89 / 58 / 62, 12,288 of 5,120 76 / 54 / 58, 8,192 of 8,192 109 / 66 / 84.
+    const int64_t written = (int64_t)tokens * hidden * (int64_t)sizeof(float);
+    if (written >= (1ll << 20) && written < (192ll << 20)) launch_embed_vec<4>(out, table, dtype, ids, tokens, hidden, multiplier, (hipStream_t)stream);
+    else launch_embed_vec<8>(out, table, dtype, ids, tokens, hidden, multiplier, (hipStream_t)stream);
     return lrs_check_launch("embed");
   }
   if (dtype == LRS_F32)
