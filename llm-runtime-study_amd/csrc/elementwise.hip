@@ -96,7 +96,9 @@ __global__ void rmsnorm_kernel(TO* __restrict__ out, float* __restrict__ x, cons
 // Every load of a row is asked for before any is used and none stands behind a branch (a chunk past the row's end is the last one
 // once more), and the arguments that lead to them come first (the file is compiled so that they are in registers): one trip to memory,
 // where a branch a chunk made four.  8 rows of 1,024 between the products of a float32 step 4.4 -> 2.7 us.
-template <typename TW, typename TO, int VEC>
+// SUMS: with a product's splits to add up (instances of their own: their two sets of loads take a thread of four chunks from under 64 registers to 94,
+// and a SIMD then holds five waves instead of eight: with one kernel for both, 2,048 bfloat16 rows of 4,096 took 9.5 us for 8.6, of 5,120 with an addend 1,024 rows 9.7 for 8.9).
+template <typename TW, typename TO, int VEC, bool SUMS>
 __global__ void rmsnorm_vec_kernel(float* __restrict__ x, const bf16* __restrict__ add, const TW* __restrict__ weight, const int* __restrict__ rows,
                                    const float* __restrict__ sums, int splits, int hidden, int threads, int n_rows, TO* __restrict__ out, float eps) {
   __shared__ float scratch[16];
@@ -123,7 +125,7 @@ __global__ void rmsnorm_vec_kernel(float* __restrict__ x, const bf16* __restrict
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[j][i] += (float)y[j][i];
   }
-  if (sums) {
+  if constexpr (SUMS) {
     // what the K splits of the product before left, [splits, rows, hidden], added up in split order, two splits asked for at a time
     floatx4 y[VEC];
 #pragma unroll
@@ -149,7 +151,7 @@ __global__ void rmsnorm_vec_kernel(float* __restrict__ x, const bf16* __restrict
 #pragma unroll
   for (int j = 0; j < VEC; ++j)
     if ((int)threadIdx.x + j * threads < chunks) {
-      if (add || sums) src[at[j]] = v[j];
+      if (add || SUMS) src[at[j]] = v[j];
       ss += v[j][0] * v[j][0] + v[j][1] * v[j][1] + v[j][2] * v[j][2] + v[j][3] * v[j][3];
     }
   ss = threads == WAVE ? wave_sum(ss) : block_sum(ss, scratch);
@@ -164,15 +166,15 @@ __global__ void rmsnorm_vec_kernel(float* __restrict__ x, const bf16* __restrict
 }
 
 // As many chunks a thread as the row has for it: a chunk behind the row's end is a load all the same, which many rows have time to feel (bfloat16
-// added to 2,048 rows of 2,048 and the norm, with four chunks whatever the row 8.3 us, with two 7.3; 1,024 rows of 5,120 10.5 / 9.7).
-template <typename TW, typename TO>
+// added to 2,048 rows of 2,048 and the norm, with four chunks whatever the row 8.3 us, with two 7.1; 1,024 rows of 5,120 10.2 / 8.9).
+template <bool SUMS, typename TW, typename TO>
 static void launch_rmsnorm_vec(float* x, const bf16* add, const TW* weight, const int* rows, const float* sums, int splits, int hidden, int threads, int n_rows,
                                TO* out, float eps, hipStream_t s) {
   switch ((hidden / 4 + threads - 1) / threads) {
-    case 1: rmsnorm_vec_kernel<TW, TO, 1><<<n_rows, threads, 0, s>>>(x, add, weight, rows, sums, splits, hidden, threads, n_rows, out, eps); break;
-    case 2: rmsnorm_vec_kernel<TW, TO, 2><<<n_rows, threads, 0, s>>>(x, add, weight, rows, sums, splits, hidden, threads, n_rows, out, eps); break;
-    case 3: rmsnorm_vec_kernel<TW, TO, 3><<<n_rows, threads, 0, s>>>(x, add, weight, rows, sums, splits, hidden, threads, n_rows, out, eps); break;
-    default: rmsnorm_vec_kernel<TW, TO, 4><<<n_rows, threads, 0, s>>>(x, add, weight, rows, sums, splits, hidden, threads, n_rows, out, eps); break;
+    case 1: rmsnorm_vec_kernel<TW, TO, 1, SUMS><<<n_rows, threads, 0, s>>>(x, add, weight, rows, sums, splits, hidden, threads, n_rows, out, eps); break;
+    case 2: rmsnorm_vec_kernel<TW, TO, 2, SUMS><<<n_rows, threads, 0, s>>>(x, add, weight, rows, sums, splits, hidden, threads, n_rows, out, eps); break;
+    case 3: rmsnorm_vec_kernel<TW, TO, 3, SUMS><<<n_rows, threads, 0, s>>>(x, add, weight, rows, sums, splits, hidden, threads, n_rows, out, eps); break;
+    default: rmsnorm_vec_kernel<TW, TO, 4, SUMS><<<n_rows, threads, 0, s>>>(x, add, weight, rows, sums, splits, hidden, threads, n_rows, out, eps); break;
   }
 }
 
@@ -185,7 +187,7 @@ static int launch_rmsnorm(void* out, int out_dtype, float* x, const bf16* add, c
   hipStream_t s = (hipStream_t)stream;
   if (hidden % 4 == 0 && hidden <= 4 * 4 * 512 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)add % 8) == 0) {
     const int threads = hidden <= 1024 ? 64 : (hidden <= 4096 ? 256 : 512);
-#define LAUNCH_VEC(TW, TO) launch_rmsnorm_vec<TW, TO>(x, add, (const TW*)weight, rows, nullptr, 0, hidden, threads, n_rows, (TO*)out, eps, s)
+#define LAUNCH_VEC(TW, TO) launch_rmsnorm_vec<false, TW, TO>(x, add, (const TW*)weight, rows, nullptr, 0, hidden, threads, n_rows, (TO*)out, eps, s)
     if (w_dtype == LRS_F32 && out_dtype == LRS_F32) LAUNCH_VEC(float, float);
     else if (w_dtype == LRS_BF16 && out_dtype == LRS_BF16) LAUNCH_VEC(bf16, bf16);
     else if (w_dtype == LRS_F32 && out_dtype == LRS_BF16) LAUNCH_VEC(float, bf16);
@@ -278,7 +280,7 @@ LRS_API int lrs_split_add_rmsnorm(void* out, int out_dtype, float* x, const floa
               "split_add_rmsnorm: needs hidden %% 4 == 0, at most 8192 columns and 16-byte aligned rows (hidden=%d)", hidden);
   const int threads = hidden <= 1024 ? 64 : (hidden <= 4096 ? 256 : 512);
   hipStream_t s = (hipStream_t)stream;
-#define LAUNCH_VEC(TW, TO) launch_rmsnorm_vec<TW, TO>(x, nullptr, (const TW*)weight, nullptr, sums, splits, hidden, threads, n_rows, (TO*)out, eps, s)
+#define LAUNCH_VEC(TW, TO) launch_rmsnorm_vec<true, TW, TO>(x, nullptr, (const TW*)weight, nullptr, sums, splits, hidden, threads, n_rows, (TO*)out, eps, s)
   if (w_dtype == LRS_F32 && out_dtype == LRS_F32) LAUNCH_VEC(float, float);
   else if (w_dtype == LRS_BF16 && out_dtype == LRS_BF16) LAUNCH_VEC(bf16, bf16);
   else if (w_dtype == LRS_F32 && out_dtype == LRS_BF16) LAUNCH_VEC(float, bf16);
