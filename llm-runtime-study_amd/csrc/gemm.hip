@@ -6,12 +6,13 @@
 // float32 run is float32 throughout.  The order of the sum over K for one output element of such a
 // product never depends on M, so a row's result does not depend on what else is in the batch.
 #include "common.h"
+#include "gemm_tiles.h"
 
 #include <type_traits>
 
 int lrs_gemm_f32(float* out, bool add, const float* a, const float* w, const float* bias, int m, int n, int k, int lda, int ldc, hipStream_t s);
 
-enum { OUT_STORE = 0, OUT_STORE_F32 = 1, OUT_ADD_F32 = 2 };
+enum { OUT_STORE = TILES_STORE, OUT_STORE_F32 = TILES_STORE_F32, OUT_ADD_F32 = TILES_ADD_F32 };
 
 template <typename T>
 __device__ __forceinline__ void emit(void* out, int mode, int64_t index, float value) {
@@ -286,139 +287,6 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_wide_kernel(void* __restrict
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           v[i] = __shfl(v[i], lane, WAVE);
-        if constexpr (MODE == OUT_STORE) *(bf16x4*)((bf16*)out + row_at + row0) = bf16x4{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
-        else if constexpr (MODE == OUT_STORE_F32) *(floatx4*)((float*)out + row_at + row0) = v;
-        else *(floatx4*)((float*)out + row_at + row0) = *(const floatx4*)((const float*)out + row_at + row0) + v;
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-}
-
-// ------------------------------------------ bf16 MFMA kernel for many rows, slices of whole lines
-// 256 tokens x BN weight rows per workgroup of eight waves, K walked in slices of 64, one workgroup a
-// compute unit.  BN = 256 (2 x 4 waves: a wave owns 128 tokens x 64 weight rows as 8 x 4 tiles of the
-// 16x16x32 product; two stages of 64 KB), BN = 192 (2 x 4 waves of 128 x 48; two stages of 56 KB) or
-// BN = 128 (4 x 2 waves of 64 x 64; three stages of 48 KB): whichever leaves the compute units the least
-// idle in the launch's last round (6,144 columns are 256 tiles of 192, one a unit).  Against the kernel above: a
-// slice holds whole 128-byte lines of every row, so a fetch touches 8 lines instead of 16 halves (the address
-// units in front of the L1 were busy 62 % of that kernel's time), and at BN = 256 a third less traffic from
-// memory per product.  The slice after next (BN = 128) or the next (BN = 256) is asked for before a slice
-// is multiplied.  K % 64 == 0; the kernel above takes the rest.
-// Where chunk c (8 k, 16 bytes) of tile row q lies in a stage: rows are 128 bytes, eight to a block of
-// 1,024 bytes (one fetch of one wave, whose lane l fills place l), and the chunks of a row are turned round
-// by twice (q / 2) % 4, so that the lanes LDS serves together (eight consecutive rows, chunks g and g + 1)
-// meet every bank once: place (q % 8) * 8 + (c ^ ((q >> 1 & 3) << 1)) of block q / 8.
-template <int BN, bool SWIGLU, int MODE>
-__global__ __launch_bounds__(512, 1) void gemm_bf16_lines_kernel(void* __restrict__ out, const bf16* __restrict__ x,
-                                                                 const bf16* __restrict__ w, int m, int n, int k, int lda,
-                                                                 int ldc, int tiles_m, int tiles_n, int splits) {
-  static_assert(BN == 256 || BN == 192 || BN == 128, "256, 192 or 128 weight rows a workgroup");
-  constexpr int BM = 256, BK = 64, STAGES = BN == 128 ? 3 : 2;
-  constexpr int WAVES_N = BN == 128 ? 2 : 4;                   // waves side by side along the weight rows
-  constexpr int IT = BN / WAVES_N / 16, JT = BM / (8 / WAVES_N) / 16;   // a wave's tiles: 4 x 8, 3 x 8 or 4 x 4
-  constexpr int XL = BM / 8 / 8, WL = BN / 8 / 8;             // blocks of 8 rows per wave: 4 of x, 4, 3 or 2 of w
-  constexpr int PENDING = STAGES == 2 ? 0 : XL + WL;          // fetches that may still be on their way at a barrier
-  constexpr int STAGE_ELEMENTS = (BM + BN) * BK;
-  __shared__ __attribute__((aligned(64))) bf16 slices[STAGES * STAGE_ELEMENTS];
-  const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-  const int r = lane & 15, g = lane >> 4;
-  const int tiles = tiles_m * tiles_n;
-  const int split = blockIdx.x / tiles;                            // which part of K (the launch is tiles x splits)
-  int id = blockIdx.x - split * tiles;
-  if (tiles % 8 == 0) id = (id % 8) * (tiles / 8) + id / 8;        // consecutive workgroups go to different XCDs
-  const int band = id / (4 * tiles_n), within = id % (4 * tiles_n);
-  const int band_rows = tiles_m - band * 4 < 4 ? tiles_m - band * 4 : 4;
-  const int m0 = (band * 4 + within % band_rows) * BM, n0 = (within / band_rows) * BN;
-  const int wm = (wave / WAVES_N) * (JT * 16), wn = (wave % WAVES_N) * (IT * 16);   // this wave's corner inside the tile
-  const int place_row = lane >> 3;                                  // the row whose piece lies at place l of a block
-  const int place_chunk = (lane & 7) ^ (((place_row >> 1) & 3) << 1);
-  unsigned xoff[XL], woff[WL];                                      // bytes from the matrix's first element
-#pragma unroll
-  for (int i = 0; i < XL; ++i) {
-    const int row = m0 + 8 * (wave + 8 * i) + place_row;
-    xoff[i] = (unsigned)(((row < m ? row : m - 1) * lda + place_chunk * 8) * 2);
-  }
-#pragma unroll
-  for (int i = 0; i < WL; ++i) {
-    const int row = n0 + 8 * (wave + 8 * i) + place_row;
-    woff[i] = (unsigned)(((row < n ? row : n - 1) * k + place_chunk * 8) * 2);
-  }
-  // this lane's fragment of rows 16 j .. 16 j + 15, k half c: row r, chunk 4 c + g
-  const int frag_row = (r >> 3) * 512 + (r & 7) * 64;               // elements; + 16 j * 64
-  const int turn = ((r >> 1) & 3) << 1;
-  const int frag0 = frag_row + ((g ^ turn) * 8), frag1 = frag_row + (((4 + g) ^ turn) * 8);
-  floatx4 acc[IT][JT];
-#pragma unroll
-  for (int it = 0; it < IT; ++it)
-#pragma unroll
-    for (int jt = 0; jt < JT; ++jt) acc[it][jt] = floatx4{0.f, 0.f, 0.f, 0.f};
-  // with K divided between workgroups, this one walks the slices step0 .. step0 + steps - 1 and leaves its sums
-  // in part `split` of out [splits, m, ldc]
-  const int steps_of_k = k / BK, steps_each = (steps_of_k + splits - 1) / splits, step0 = split * steps_each;
-  const int steps = steps_of_k - step0 < steps_each ? steps_of_k - step0 : steps_each;
-  const unsigned slices_address = (unsigned)(uintptr_t)(__attribute__((address_space(3))) bf16*)slices;
-  auto fetch = [&](int kt, int stage) {                             // XL + WL fetches a wave
-    const int at = (step0 + (kt < steps ? kt : steps - 1)) * BK * 2;
-    const unsigned to = slices_address + (unsigned)(stage * STAGE_ELEMENTS * 2 + wave * 1024);
-#pragma unroll
-    for (int i = 0; i < XL; ++i) fetch_to_lds((const char*)x + at, xoff[i], to + (unsigned)(i * 8192));
-#pragma unroll
-    for (int i = 0; i < WL; ++i) fetch_to_lds((const char*)w + at, woff[i], to + (unsigned)(BM * BK * 2 + i * 8192));
-  };
-  auto multiply = [&](int stage) {
-    const bf16* xs = slices + stage * STAGE_ELEMENTS;
-    const bf16* ws = xs + BM * BK;
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int frag = c ? frag1 : frag0;
-      bf16x8 xf[JT];
-#pragma unroll
-      for (int jt = 0; jt < JT; ++jt) xf[jt] = *(const bf16x8*)(xs + frag + (wm + jt * 16) * BK);
-#pragma unroll
-      for (int it = 0; it < IT; ++it) {
-        const bf16x8 wf = *(const bf16x8*)(ws + frag + (wn + it * 16) * BK);
-#pragma unroll
-        for (int jt = 0; jt < JT; ++jt) acc[it][jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf[jt], acc[it][jt], 0, 0, 0);
-      }
-    }
-  };
-  // Slice kt is multiplied from stage kt % STAGES while the slices after it arrive; a stage is filled again a
-  // barrier after it was last read.  Before the barrier a wave waits until only the fetches it asked for in
-  // this turn (none, with two stages) are still on their way: the next slice is then in LDS.
-  int m0_opaque = m0;
-  fetch(0, 0);
-  if (STAGES == 3) fetch(1, 1);
-  fetched_and_read_then_barrier<PENDING>();
-  int stage = 0;
-  for (int kt = 0; kt < steps; ++kt) {
-    fetch(kt + STAGES - 1, stage == 0 ? STAGES - 1 : stage - 1);
-    multiply(stage);
-    fetched_and_read_then_barrier<PENDING>();
-    stage = stage == STAGES - 1 ? 0 : stage + 1;
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");               // the fetches past K that nobody reads
-  asm volatile("" : "+s"(ldc), "+s"(m0_opaque));
-#pragma unroll
-  for (int jt = 0; jt < JT; ++jt) {
-    const int token = m0_opaque + wm + jt * 16 + r;
-    const int64_t row_at = ((int64_t)split * m + token) * ldc;
-#pragma unroll
-    for (int it = 0; it < IT; ++it) {
-      const int tile0 = n0 + wn + it * 16, row0 = tile0 + 4 * g;     // this lane's four weight rows = output columns
-      if (SWIGLU) {
-        floatx4 up;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) up[i] = __shfl(acc[it][jt][i], (lane + 32) % WAVE, WAVE);
-        if (g < 2 && token < m && tile0 + 15 < n) {
-          const floatx4 gate = acc[it][jt];
-          const bf16x4 y = {(bf16)(silu(gate[0]) * up[0]), (bf16)(silu(gate[1]) * up[1]), (bf16)(silu(gate[2]) * up[2]), (bf16)(silu(gate[3]) * up[3])};
-          *(bf16x4*)((bf16*)out + row_at + tile0 / 2 + 4 * g) = y;
-        }
-      } else if (token < m && row0 < n) {
-        floatx4 v = acc[it][jt];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = __shfl(v[i], lane, WAVE);    // as in the kernel above: keeps the loop free of spills
         if constexpr (MODE == OUT_STORE) *(bf16x4*)((bf16*)out + row_at + row0) = bf16x4{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
         else if constexpr (MODE == OUT_STORE_F32) *(floatx4*)((float*)out + row_at + row0) = v;
         else *(floatx4*)((float*)out + row_at + row0) = *(const floatx4*)((const float*)out + row_at + row0) + v;
@@ -1747,10 +1615,9 @@ LRS_API int lrs_gemm_mid_qk_prep(void* qkv, int row_stride, const void* a, const
                                v_pages, slots, page_size, split_sums_buffer(), splits, stream);
 }
 
-// Which tile width the kernel for many rows with slices of whole lines would take for this product, or 0 if
-// it does not take it: K a multiple of 64 and a tile of 256 x 128 for every compute unit; then the width
-// (256, 192 or 128 weight rows) whose launch takes the fewest rounds of the chip times its width, the wider
-// of two that tie (less traffic per product).
+// The width of 256-token tiles, of 256, 192 or 128 weight rows, whose launch takes the fewest rounds of the chip times its width (the
+// wider of two that tie), or 0 unless K is a multiple of 64 and there is a tile of 256 x 128 for every compute unit.  Says which products
+// of few outputs have tiles enough not to go to gemm_bf16_narrow; the tile that is taken is choose_tiles' (gemm_tiles.hip).
 LRS_API int lrs_gemm_lines_width(int m, int n, int k) {
   const int units = lrs_compute_units() > 0 ? lrs_compute_units() : 256;
   const int big_m = (m + 255) / 256;
@@ -1765,10 +1632,10 @@ LRS_API int lrs_gemm_lines_width(int m, int n, int k) {
   return width;
 }
 
-// Into how many parts that kernel divides K for a product with too few tiles of 256 x 128 to go round the
-// compute units, or 0 if it does not take the product that way (then lrs_gemm_lines_width says whether it takes
-// it whole): the number of parts, from 1 (just the tiles, if they fill half the units) to 8, that fills the
-// units best in one round, every part with 8 slices of 64 or more, and the parts' sums within the split buffer.
+// Into how many parts K would be divided for a product with too few tiles of 256 x 128 to go round the compute units, or 0 if there are
+// enough of them, or too few even so: the number of parts, from 1 (just the tiles, if they fill half the units) to 8, that fills the
+// units best in one round, every part with 8 slices of 64 or more, and the parts' sums within the split buffer.  Says which products
+// lrs_gemm_lines_add_rmsnorm takes; the parts that are made are choose_tiles'.
 LRS_API int lrs_gemm_lines_splits(int m, int n, int k) {
   const int units = lrs_compute_units() > 0 ? lrs_compute_units() : 256;
   if (m <= 128 || n <= 0 || k <= 0 || k % 64 != 0) return 0;
@@ -1783,12 +1650,9 @@ LRS_API int lrs_gemm_lines_splits(int m, int n, int k) {
   return splits && 2 * tiles * splits >= units ? splits : 0;
 }
 
-// Whether that divided form is the faster way for a product that could also go to the vendor library.  Measured
-// on MI355X at 256..1024 rows with the layer sizes of the 8B and 14B models, against the library's first choice:
-// products with a long K (the feed-forward's second: K three times N or more) take 0.4 to 0.9 of the library's
-// time at every such row count (14B at 512 rows: 102 against 171 us; 8B: 61 against 82); square and wide ones only
-// up to 256 rows, when every part still has 12 slices (14B q/k/v 41 against 54 us, o_proj 35 against 49; with 8
-// slices a part, 8B o_proj, 31 against 23).  Elsewhere the library is as fast or faster.
+// Whether such a product goes to this package's tiles rather than to the vendor library whatever follows it: a long K (the feed-forward's second
+// product: 14B at 512 rows 90 us against 174, 8B 61 against 86, norms included), square and wide ones up to 256 rows where every part would
+// have 12 slices (14B q/k/v 39 against 52).  lrs_gemm_tiles_pay says more, by what follows.
 LRS_API int lrs_gemm_lines_split_pays(int m, int n, int k) {
   const int splits = lrs_gemm_lines_splits(m, n, k);
   if (splits < 1 || n % 4 != 0) return 0;
@@ -1796,34 +1660,67 @@ LRS_API int lrs_gemm_lines_split_pays(int m, int n, int k) {
   return m <= 256 && splits >= 2 && (k / 64 + splits - 1) / splits >= 12;
 }
 
+// Whether the tiles of gemm_tiles.hip, with what follows the product in their epilogue or in the kernel that adds up their parts, are
+// faster than the vendor library and a kernel for what follows, for a product of more than 128 rows.  form: what follows.
+//   0  nothing (stored as bf16): up to 256 rows.  us of the tiles / the library at 256 rows: 0.6B q/k/v 8.2 / 9.7, 1.7B 11.5 / 11.3, 4B 17.4 / 24.8,
+//      8B 28.3 / 41.4, 14B 39.2 / 52.1; at 384 to 2,048 rows between a tenth slower and a twentieth faster (4B 384 23.6 / 21.7, 8B 1,536 65.8 / 70.0).
+//   1  the gated activation: always.  512 rows 0.6B 15.1 / 18.3, 1.7B 31.9 / 35.8, 4B 51.4 / 60.2, 8B 81.7 / 89.6, 14B 179 / 193; 2,048 rows 29.4 / 35.4,
+//      92 / 102, 189 / 218, 299 / 314, 579 / 627.
+//   2  the residual add and a norm: a K of twice the width (more than 1,024 wide), or up to 512 rows where K is divided.  Down 512 rows 1.7B 24.6 /
+//      26.0, 4B 39.7 / 53.7, 8B 60.6 / 86.0, 14B 89.9 / 174; 2,048 rows 59.8 / 66.2, 95.8 / 113, 170 / 189, 291 / 303; o at 512 rows 0.6B 13.0 / 14.0,
+//      1.7B 16.7 / 15.8 (not divided), 4B 24.1 / 25.7, 14B 43.8 / 53.2; at 768 8B 44.9 / 40.3.
+// Not at all for a K of less than 512: eight slices are mostly beginnings and ends.
+LRS_API int lrs_gemm_tiles_pay(int m, int n, int k, int form) {
+  if (m <= 128 || n <= NARROW_MAX || n % 4 != 0 || k < 512 || k % 64 != 0) return 0;
+  if (form == 0) return m <= 256;
+  if (form == 1) return n % 16 == 0;
+  if (form != 2 || n > 8192) return 0;
+  if (k >= 2 * n && n > 1024) return 1;
+  return m <= 512 && choose_tiles(m, n, k, SPLIT_SUMS_BYTES).splits > 1;
+}
+
 // Defined beside the norm kernels: x += the sum of the splits' sums, then out = RMSNorm(x), one pass over the rows.
 extern "C" int lrs_split_add_rmsnorm(void* out, int out_dtype, float* x, const float* sums, int splits, const void* weight,
                                      int w_dtype, int n_rows, int hidden, float eps, void* stream);
 
+extern "C" int lrs_rmsnorm(void* out, int out_dtype, const float* x, const void* weight, int w_dtype, const int* rows, int n_rows, int hidden,
+                           float eps, void* stream);
+
 // A product of more than 128 bf16 rows that adds into the float32 residual stream, and the RMSNorm that follows, as two
-// kernels: residual [M, N] += a [M, K] w[N, K]^T; normed [M, N] = RMSNorm(residual) with norm_weight and eps.  The
-// product is the many-rows kernel with slices of whole lines, its K divided between workgroups as lrs_gemm_lines_splits
-// says (which must take the shape); its sums stay in the workspace, and the kernel that adds them up also adds the
-// residual, writes it back and normalises the row: no kernel of its own for the add, none for the norm.
+// kernels: residual [M, N] += a [M, K] w[N, K]^T; normed [M, N] = RMSNorm(residual) with norm_weight and eps.  Where
+// choose_tiles divides K between workgroups, their sums stay in the workspace, and the kernel that adds them up also adds
+// the residual, writes it back and normalises the row: no kernel of its own for the add, none for the norm.  K % 64 == 0.
+LRS_API int lrs_gemm_tiles_add_rmsnorm(float* residual, const void* a, const void* w, int m, int n, int k, int lda,
+                                       const void* norm_weight, int norm_weight_dtype, float eps, void* normed, int normed_dtype,
+                                       void* workspace, int64_t workspace_bytes, void* stream) {
+  LRS_REQUIRE(m > 128 && n > 0 && k > 0 && lda >= k, "gemm_tiles_add_rmsnorm: takes more than 128 rows and positive sizes, got m=%d n=%d k=%d lda=%d", m, n, k, lda);
+  LRS_REQUIRE(workspace_ok(workspace, workspace_bytes), "gemm_tiles_add_rmsnorm: a workspace must be 16-byte aligned and hold lrs_gemm_workspace_bytes() bytes");
+  const UseSpace space(workspace, workspace_bytes);
+  LRS_REQUIRE(k % 64 == 0 && lda % 8 == 0 && n % 4 == 0 && n <= 8192 && ((uintptr_t)a % 16 == 0) && ((uintptr_t)w % 16 == 0) && ((uintptr_t)residual % 16 == 0) &&
+                  (int64_t)m * lda < (1ll << 31) && (int64_t)n * k < (1ll << 31),
+              "gemm_tiles_add_rmsnorm: needs K %% 64 == 0, 16-byte aligned rows, up to 8,192 outputs and sizes below 2^31 elements (m=%d n=%d k=%d lda=%d)", m, n, k, lda);
+  LRS_REQUIRE(residual && normed && norm_weight && eps > 0.f, "gemm_tiles_add_rmsnorm: needs the residual stream, the norm's weight, a positive eps and the output");
+  const TilesChoice choice = choose_tiles(m, n, k, split_sums_bytes());
+  const int splits = choice.splits;
+  if (splits == 1) {
+    // nothing to add up: the product adds into the stream itself (three passes over float32 rows instead of four)
+    launch_tiles(choice, residual, TILES_ADD_F32, (const bf16*)a, (const bf16*)w, m, n, k, lda, n, (hipStream_t)stream);
+    if (int rc = lrs_check_launch("gemm_tiles_add_rmsnorm")) return rc;
+    return lrs_rmsnorm(normed, normed_dtype, residual, norm_weight, norm_weight_dtype, nullptr, m, n, eps, stream);
+  }
+  float* sums = split_sums_buffer();
+  launch_tiles(choice, sums, TILES_STORE_F32, (const bf16*)a, (const bf16*)w, m, n, k, lda, n, (hipStream_t)stream);
+  if (int rc = lrs_check_launch("gemm_tiles_add_rmsnorm")) return rc;
+  return lrs_split_add_rmsnorm(normed, normed_dtype, residual, sums, splits, norm_weight, norm_weight_dtype, m, n, eps, stream);
+}
+
+// The same for shapes that lrs_gemm_lines_splits takes, with room for one part's sums.
 LRS_API int lrs_gemm_lines_add_rmsnorm(float* residual, const void* a, const void* w, int m, int n, int k, int lda,
                                        const void* norm_weight, int norm_weight_dtype, float eps, void* normed, int normed_dtype,
                                        void* workspace, int64_t workspace_bytes, void* stream) {
-  LRS_REQUIRE(m > 128 && n > 0 && k > 0 && lda >= k, "gemm_lines_add_rmsnorm: takes more than 128 rows and positive sizes, got m=%d n=%d k=%d lda=%d", m, n, k, lda);
-  LRS_REQUIRE(workspace_ok(workspace, workspace_bytes), "gemm_lines_add_rmsnorm: a workspace must be 16-byte aligned and hold lrs_gemm_workspace_bytes() bytes");
-  const UseSpace space(workspace, workspace_bytes);
-  const int splits = lrs_gemm_lines_splits(m, n, k);
-  LRS_REQUIRE(splits >= 1, "gemm_lines_add_rmsnorm: the divided product does not take m=%d n=%d k=%d (see lrs_gemm_lines_splits)", m, n, k);
-  LRS_REQUIRE(k % WIDE_BK == 0 && lda % 8 == 0 && n % 4 == 0 && ((uintptr_t)a % 16 == 0) && ((uintptr_t)w % 16 == 0) && ((uintptr_t)residual % 16 == 0) &&
-                  (int64_t)m * lda < (1ll << 31) && (int64_t)n * k < (1ll << 31),
-              "gemm_lines_add_rmsnorm: needs 16-byte aligned rows and sizes below 2^31 elements (m=%d n=%d k=%d lda=%d)", m, n, k, lda);
-  float* sums = split_sums_buffer();
-  LRS_REQUIRE(sums != nullptr && (size_t)splits * m * n * sizeof(float) <= split_sums_bytes(), "gemm_lines_add_rmsnorm: no room for the sums of %d K splits of %d x %d", splits, m, n);
-  LRS_REQUIRE(residual && normed && norm_weight && eps > 0.f, "gemm_lines_add_rmsnorm: needs the residual stream, the norm's weight, a positive eps and the output");
-  const int big_m = (m + 255) / 256, tiles_w = (n + 127) / 128;
-  gemm_bf16_lines_kernel<128, false, OUT_STORE_F32><<<big_m * tiles_w * splits, 512, 0, (hipStream_t)stream>>>(
-      sums, (const bf16*)a, (const bf16*)w, m, n, k, lda, n, big_m, tiles_w, splits);
-  if (int rc = lrs_check_launch("gemm_lines_add_rmsnorm")) return rc;
-  return lrs_split_add_rmsnorm(normed, normed_dtype, residual, sums, splits, norm_weight, norm_weight_dtype, m, n, eps, stream);
+  LRS_REQUIRE(lrs_gemm_lines_splits(m, n, k) >= 1 && (size_t)m * n * sizeof(float) <= SPLIT_SUMS_BYTES,
+              "gemm_lines_add_rmsnorm: the divided product does not take m=%d n=%d k=%d (see lrs_gemm_lines_splits)", m, n, k);
+  return lrs_gemm_tiles_add_rmsnorm(residual, a, w, m, n, k, lda, norm_weight, norm_weight_dtype, eps, normed, normed_dtype, workspace, workspace_bytes, stream);
 }
 
 // out [M, N] (row stride ldc) = a [M, K] (row stride lda) times w[N, K]^T.
@@ -1879,32 +1776,22 @@ LRS_API int lrs_gemm(void* out, int mode, const void* a, const void* w, const vo
       else launch_skinny_m<false, false>(out, mode, ap, norm, wp, bp, m, n, k, lda, ldc, s, tune);
     } else if (aligned && k % WIDE_BK == 0 && n % 4 == 0 && ldc % 4 == 0 && (uintptr_t)out % 16 == 0 && !bias &&
                (int64_t)m * lda < (1ll << 31) && (int64_t)n * k < (1ll << 31)) {
-      const int big_m = (m + 255) / 256, splits = lrs_gemm_lines_splits(m, n, k);
-      const int width = splits ? 128 : lrs_gemm_lines_width(m, n, k), tiles_w = width ? (n + width - 1) / width : 0;
-#define LINES(BN, SW, MODE, OUT, LDC, SPLITS) \
-  gemm_bf16_lines_kernel<BN, SW, MODE><<<big_m * tiles_w * SPLITS, 512, 0, s>>>(OUT, (const bf16*)a, (const bf16*)w, m, n, k, lda, LDC, big_m, tiles_w, SPLITS)
-      if (splits > 1) {
-        // K divided between workgroups: their sums go to the split buffer, and the kernel that adds them up
-        // writes the output with the epilogue that was asked for
-        float* sums = split_sums_buffer();
-        LRS_REQUIRE(sums != nullptr, "gemm: no memory for the sums of %d K splits", splits);
-        LINES(128, false, OUT_STORE_F32, sums, n, splits);
-        const int64_t total = (int64_t)m * (swiglu ? n / 2 : n);
-        const int blocks = (int)((total + 1023) / 1024 < 2048 ? (total + 1023) / 1024 : 2048);
-        if (swiglu) gemm_split_finish_kernel<true><<<blocks, 256, 0, s>>>(out, mode, sums, nullptr, m, n, ldc, splits);
-        else gemm_split_finish_kernel<false><<<blocks, 256, 0, s>>>(out, mode, sums, nullptr, m, n, ldc, splits);
-      } else if (width) {
-#define LINES_OF(BN)                                                           \
-        if (swiglu) LINES(BN, true, OUT_STORE, out, ldc, 1);                    \
-        else if (mode == OUT_STORE) LINES(BN, false, OUT_STORE, out, ldc, 1);   \
-        else if (mode == OUT_STORE_F32) LINES(BN, false, OUT_STORE_F32, out, ldc, 1); \
-        else LINES(BN, false, OUT_ADD_F32, out, ldc, 1)
-        if (width == 256) { LINES_OF(256); }
-        else if (width == 192) { LINES_OF(192); }
-        else { LINES_OF(128); }
-#undef LINES_OF
-#undef LINES
-      } else if (n <= NARROW_MAX && !swiglu) {
+      const bool narrow = n <= NARROW_MAX && !swiglu && !lrs_gemm_lines_width(m, n, k) && !lrs_gemm_lines_splits(m, n, k);
+      if (k % 64 == 0 && !narrow) {
+        const TilesChoice choice = choose_tiles(m, n, k, split_sums_bytes());
+        if (choice.splits > 1) {
+          // K divided between workgroups: their sums go to the split buffer, and the kernel that adds them up
+          // writes the output with the epilogue that was asked for
+          float* sums = split_sums_buffer();
+          launch_tiles(choice, sums, TILES_STORE_F32, (const bf16*)a, (const bf16*)w, m, n, k, lda, n, s);
+          const int64_t total = (int64_t)m * (swiglu ? n / 2 : n);
+          const int blocks = (int)((total + 1023) / 1024 < 2048 ? (total + 1023) / 1024 : 2048);
+          if (swiglu) gemm_split_finish_kernel<true><<<blocks, 256, 0, s>>>(out, mode, sums, nullptr, m, n, ldc, choice.splits);
+          else gemm_split_finish_kernel<false><<<blocks, 256, 0, s>>>(out, mode, sums, nullptr, m, n, ldc, choice.splits);
+        } else {
+          launch_tiles(choice, out, swiglu ? TILES_GATED : mode, (const bf16*)a, (const bf16*)w, m, n, k, lda, ldc, s);
+        }
+      } else if (narrow) {
 #define NARROW(NT, MODE) gemm_bf16_narrow_kernel<NT, MODE><<<(m + 15) / 16, NARROW_WAVES * WAVE, 0, s>>>(out, (const bf16*)a, (const bf16*)w, m, n, k, lda, ldc)
 #define NARROW_OF(NT)                                    \
         if (mode == OUT_STORE) NARROW(NT, OUT_STORE);        \

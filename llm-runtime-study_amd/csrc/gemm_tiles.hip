@@ -1,0 +1,263 @@
+// bf16 products of many rows: y = x W^T with both operands through LDS in slices of 64 k (whole 128-byte lines of every row), tiles of
+// 256 or 128 tokens x 64 to 256 weight rows, two groups of four waves in turn.
+#include "gemm_tiles.h"
+
+// A workgroup of eight waves owns WM * JT * 16 tokens x (8 / WM) * IT * 16 weight rows; a wave JT x IT tiles of the 16x16x32 product.
+// Slices of 64 * PANELS of K lie in STAGES places in LDS, which memory fills itself (fetch_to_lds).  A slice is taken whole, or in two
+// halves of the wave's tokens (HALVES: registers and LDS of the largest tiles): a step of reading (the fragments; those of the weights
+// stay in registers for the second half) and a step of multiplying, with a barrier behind each.  Waves 4..7 are one step behind waves
+// 0..3, and a SIMD has one of either: while one multiplies, the other reads LDS and asks memory for a slice to come.  So neither kind of
+// work waits for the other, where waves in step (the kernel that this one replaced) all read, then all multiplied.
+//
+// What may be asked for when.  A wave has what it read before the barrier that ends its step of reading.
+// Whole slices: waves 0..3 read slice s in step 2 s, waves 4..7 in step 2 s + 1.  Behind that its place is free, and every wave asks for
+// slice s + STAGES in its next step of reading (steps 2 s + 2 and 2 s + 3).  Before the barrier that ends a step of reading, of slice s, a
+// wave waits until only the last STAGES - 2 slices are on their way: slice s + 1 is then there (steps 2 s and 2 s + 1) before anyone reads
+// it (step 2 s + 2).
+// Halves: waves 0..3 read the first half of slice s in step 4 s and the second in step 4 s + 2, waves 4..7 in steps 4 s + 1 and 4 s + 3.  The
+// first half of x and the weights of s are read by everybody when step 4 s + 1 ends, and every wave asks for those of s + STAGES when it
+// reads the second half of s (steps 4 s + 2 and 4 s + 3); the second half of s is free when step 4 s + 3 ends, and is asked for again when
+// the first half of s + 1 is read (steps 4 s + 4 and 4 s + 5).  A wave waits until only the last STAGES - 1 slices' worth is on its way: at
+// the end of reading the second half of s (steps 4 s + 2 and 4 s + 3) the first half and the weights of s + 1 are there, read from step
+// 4 s + 4 on; at the end of reading the first half of s + 1 (steps 4 s + 4 and 4 s + 5) its second half, read from step 4 s + 6 on.
+// Once there are no more slices to ask for, a wave waits for all it has asked for.
+//
+// What bounds it: the large tiles by the matrix cores' power.  8B gate_up at 2,048 rows (three rounds of 256 x 256) 291 us (1.42 PFLOP/s; 327
+// before), on another card 317, there without fetches 280, without reads as well 262, the matrix instructions alone 259 (1.59); with
+// operands of zeros 259, 229, 218 and 215: what is left is the clock, not a wait.  The L2s hand out 22-26 TB/s to such fetches.  4B gate_up at
+// 512 rows (244 tiles of 256 x 160) 51 us (72), 8B down at 512 rows (256 x 128, K in four) with its norm 59 (66), 1.7B gate_up at
+// 2,048 (256 x 192) 90 (104).  32x32x16 products instead: a tenth slower.  The small tiles by their steps' beginnings, which is why
+// they take slices of 128 whole: 1.7B q/k/v at 256 rows (64 x 64) 12.2 us, in slices of 64 14.0, of 128 x 64 in halves 18.2.
+//
+// Fetches: a block of 8 rows x 128 bytes is one fetch of one wave, lane l fills place l.  Chunk c (16 bytes) of row q lies at place
+// (q % 8) * 8 + (c ^ ((q >> 1 & 3) << 1)) of block q / 8, so that the lanes LDS serves together (eight consecutive rows of a fragment,
+// chunks g and g + 1) meet every bank once.  Rows past a matrix are read from its last row and never written.
+// Needs K % (64 * PANELS) == 0, 16-byte aligned rows, N % 4 == 0, matrices of fewer than 2^31 elements.
+// With K divided (splits > 1) a workgroup walks its part of the slices and leaves its sums in part `split` of out [splits, m, ldc].
+// The sums of an output are one chain over its K in steps of 32, whatever the tile: bits depend on the parts alone.
+template <int N>
+__device__ __forceinline__ void wait_fetches() {
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
+}
+__device__ __forceinline__ void have_read_then_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+__device__ __forceinline__ void barrier_alone() { asm volatile("s_barrier" ::: "memory"); }
+__device__ __forceinline__ float silu_of(float v) { return v / (1.f + __expf(-v)); }
+
+template <int WM, int JT, int IT, int PANELS, int HALVES, int STAGES>
+__global__ __launch_bounds__(512, 1) void gemm_bf16_tiles_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, int m, int n, int k, int lda,
+                                                                 int tiles_m, int tiles_n, int splits, int chunk, void* __restrict__ out, int form, int ldc) {
+  constexpr int WN = 8 / WM, BM = WM * JT * 16, BN = WN * IT * 16, BK = 64 * PANELS, JH = JT / HALVES, STEPS = 2 * PANELS;
+  constexpr int X_BLOCKS = BM / 8 / HALVES, W_BLOCKS = BN / 8;   // blocks of 8 rows of a panel: of a part of the tokens, of the weights
+  static_assert(X_BLOCKS * PANELS % 8 == 0 && JT % HALVES == 0, "a part of the tokens is dealt evenly to eight waves");
+  constexpr int NX = X_BLOCKS * PANELS / 8, NW = W_BLOCKS * PANELS / 8, REST = W_BLOCKS * PANELS % 8;   // fetches a wave; REST: one more of the weights for the first waves
+  constexpr int STAGE_ELEMENTS = (BM + BN) * BK, EACH = HALVES * NX + NW, AHEAD = HALVES == 2 ? STAGES - 1 : STAGES - 2;
+  __shared__ __attribute__((aligned(64))) bf16 slices[STAGES * STAGE_ELEMENTS];   // a stage: the tokens' panels, then the weights'
+  const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int r = lane & 15, g = lane >> 4;
+  int id = (blockIdx.x % 8) * chunk + blockIdx.x / 8;            // consecutive workgroups go to different XCDs: a run of tiles to each
+  const int tiles = tiles_m * tiles_n;
+  if (id >= tiles * splits) return;
+  const int split = id / tiles;
+  id -= split * tiles;
+  const int band = id / (4 * tiles_n), within = id % (4 * tiles_n);
+  const int band_rows = tiles_m - band * 4 < 4 ? tiles_m - band * 4 : 4;
+  const int m0 = (band * 4 + within % band_rows) * BM, n0 = (within / band_rows) * BN;
+  const int wm = wave / WN, wn = wave % WN;
+  const int place_row = lane >> 3, place_chunk = (lane & 7) ^ (((place_row >> 1) & 3) << 1);
+  unsigned x_off[HALVES][NX], x_to[HALVES][NX], w_off[NW + 1];   // bytes from the matrix's first element, from the stage's first
+#pragma unroll
+  for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const int b = wave + 8 * i, panel = b / X_BLOCKS, of = b % X_BLOCKS;
+      const int first = HALVES == 2 ? ((of / JT) * 2 + h) * 8 * JT + (of % JT) * 8 : of * 8;   // a wave's half is JT blocks
+      const int row = m0 + first + place_row;
+      x_to[h][i] = (panel * BM + first) * 128;
+      x_off[h][i] = ((unsigned)(row < m ? row : m - 1) * (unsigned)lda + panel * 64 + place_chunk * 8) * 2u;
+    }
+#pragma unroll
+  for (int i = 0; i < NW + (REST ? 1 : 0); ++i) {
+    const int b = wave + 8 * i, panel = b / W_BLOCKS, row = n0 + 8 * (b % W_BLOCKS) + place_row;
+    w_off[i] = ((unsigned)(row < n ? row : n - 1) * (unsigned)k + panel * 64 + place_chunk * 8) * 2u;
+  }
+  // this lane's fragment of rows 16 j .. 16 j + 15, k half c of a panel: row r, chunk 4 c + g
+  const int frag_row = (r >> 3) * 512 + (r & 7) * 64, turn = ((r >> 1) & 3) << 1;
+  const int frag[2] = {frag_row + ((g ^ turn) * 8), frag_row + (((4 + g) ^ turn) * 8)};
+  floatx4 acc[IT][JT];
+#pragma unroll
+  for (int it = 0; it < IT; ++it)
+#pragma unroll
+    for (int jt = 0; jt < JT; ++jt) acc[it][jt] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int steps_of_k = k / BK, steps_each = (steps_of_k + splits - 1) / splits, step0 = split * steps_each;
+  const int steps = steps_of_k - step0 < steps_each ? steps_of_k - step0 : steps_each;
+  const unsigned slices_address = (unsigned)(uintptr_t)(__attribute__((address_space(3))) bf16*)slices;
+  const bool one_more = REST != 0 && wave < REST;
+  auto fetch_first = [&](int s, int stage) {                       // the first part of the tokens, and the weights
+    if (s >= steps) return;
+    const int at = (step0 + s) * BK * 2;
+    const unsigned to = slices_address + (unsigned)(stage * STAGE_ELEMENTS * 2), to_w = to + (unsigned)(BM * BK * 2 + wave * 1024);
+#pragma unroll
+    for (int i = 0; i < NX; ++i) fetch_to_lds((const char*)x + at, x_off[0][i], to + x_to[0][i]);
+#pragma unroll
+    for (int i = 0; i < NW; ++i) fetch_to_lds((const char*)w + at, w_off[i], to_w + (unsigned)(i * 8192));
+    if (REST != 0 && one_more) fetch_to_lds((const char*)w + at, w_off[NW], to_w + (unsigned)(NW * 8192));
+  };
+  auto fetch_second = [&](int s, int stage) {                      // the other half of the tokens
+    if (s >= steps) return;
+    const int at = (step0 + s) * BK * 2;
+    const unsigned to = slices_address + (unsigned)(stage * STAGE_ELEMENTS * 2);
+#pragma unroll
+    for (int i = 0; i < NX; ++i) fetch_to_lds((const char*)x + at, x_off[HALVES - 1][i], to + x_to[HALVES - 1][i]);
+  };
+  auto wait = [&](bool more_to_come) {
+    if (!more_to_come) wait_fetches<0>();
+    else if (REST != 0 && one_more) wait_fetches<AHEAD * (EACH + 1)>();
+    else wait_fetches<AHEAD * EACH>();
+  };
+  if constexpr (HALVES == 2) {
+#pragma unroll
+    for (int s = 0; s < STAGES; ++s) {
+      fetch_first(s, s);
+      if (s < STAGES - 1) fetch_second(s, s);
+    }
+    wait(STAGES - 1 < steps);
+  } else {
+#pragma unroll
+    for (int s = 0; s < STAGES - 1; ++s) fetch_first(s, s);
+    wait(STAGES - 2 < steps);
+  }
+  barrier_alone();
+  if (wave >= 4) barrier_alone();                                  // a step behind from here on
+  int stage = 0;
+  bf16x8 wf[STEPS][IT], xf[STEPS][JH];
+  auto multiply = [&](int first) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < STEPS; ++c)
+#pragma unroll
+      for (int it = 0; it < IT; ++it)
+#pragma unroll
+        for (int jt = 0; jt < JH; ++jt) acc[it][first + jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[c][it], xf[c][jt], acc[it][first + jt], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    barrier_alone();
+  };
+  for (int s = 0; s < steps; ++s) {
+    const bf16* xs = slices + stage * STAGE_ELEMENTS;
+    const bf16* ws = xs + BM * BK;
+    const int before = stage == 0 ? STAGES - 1 : stage - 1;
+#pragma unroll
+    for (int c = 0; c < STEPS; ++c) {
+#pragma unroll
+      for (int it = 0; it < IT; ++it) wf[c][it] = *(const bf16x8*)(ws + frag[c % 2] + (c / 2 * BN + (wn * IT + it) * 16) * 64);
+#pragma unroll
+      for (int jt = 0; jt < JH; ++jt) xf[c][jt] = *(const bf16x8*)(xs + frag[c % 2] + (c / 2 * BM + (wm * JT + jt) * 16) * 64);
+    }
+    if constexpr (HALVES == 2) fetch_second(s + STAGES - 1, before);
+    else fetch_first(s + STAGES - 1, before);
+    wait(s + STAGES - 1 < steps);
+    have_read_then_barrier();
+    multiply(0);
+    if constexpr (HALVES == 2) {
+#pragma unroll
+      for (int c = 0; c < STEPS; ++c)
+#pragma unroll
+        for (int jt = 0; jt < JH; ++jt) xf[c][jt] = *(const bf16x8*)(xs + frag[c % 2] + (c / 2 * BM + (wm * JT + JH + jt) * 16) * 64);
+      fetch_first(s + STAGES, stage);
+      wait(s + STAGES < steps);
+      have_read_then_barrier();
+      multiply(JH);
+    }
+    stage = stage == STAGES - 1 ? 0 : stage + 1;
+  }
+  if (wave < 4) barrier_alone();                                   // as many barriers for every wave
+  int m0_opaque = m0;                                              // nothing of what follows is worked out before the loop ends
+  asm volatile("" : "+s"(ldc), "+s"(m0_opaque));
+#pragma unroll
+  for (int jt = 0; jt < JT; ++jt) {
+    const int token = m0_opaque + (wm * JT + jt) * 16 + r;
+    const int64_t row_at = ((int64_t)split * m + token) * ldc;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int tile0 = n0 + (wn * IT + it) * 16, row0 = tile0 + 4 * g;   // this lane's four weight rows = output columns
+      const floatx4 v = acc[it][jt];
+      if (form == TILES_GATED) {
+        // a tile's 16 weight rows are 8 gate rows and the 8 up rows of the same features: the up values of a lane's gate rows are
+        // held by the lane 32 further on
+        floatx4 up;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) up[i] = __shfl(v[i], (lane + 32) % WAVE, WAVE);
+        if (g < 2 && token < m && tile0 + 15 < n)
+          *(bf16x4*)((bf16*)out + row_at + tile0 / 2 + 4 * g) =
+              bf16x4{(bf16)(silu_of(v[0]) * up[0]), (bf16)(silu_of(v[1]) * up[1]), (bf16)(silu_of(v[2]) * up[2]), (bf16)(silu_of(v[3]) * up[3])};
+      } else if (token < m && row0 < n) {
+        if (form == TILES_STORE) *(bf16x4*)((bf16*)out + row_at + row0) = bf16x4{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
+        else if (form == TILES_STORE_F32) *(floatx4*)((float*)out + row_at + row0) = v;
+        else *(floatx4*)((float*)out + row_at + row0) = *(const floatx4*)((const float*)out + row_at + row0) + v;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
+// The tiles, and what a launch of them takes: us = rounds of the chip * (fixed + slices of 64 k * (slice + crowd * share of the chip in use)),
+// fitted to 106 to 617 launches of each, at 144 to 2,048 rows of the 0.6B, 1.7B, 4B and 8B layers' products with K in 1 to 8 parts (half
+// of them within 5 %, nine in ten within 12 %; a fuller chip runs slower: its clock).  What the least of these takes is within 0.3 % of
+// the best of all launches on the mean, 6 % at most.  panels: slices of 64 k a step (K a multiple of so many).
+struct TileShape { int bm, bn, panels; float fixed, slice, crowd; };
+constexpr TileShape TILES[] = {{256, 256, 1, 12.0f, 0.81f, 0.66f}, {256, 192, 1, 9.7f, 0.69f, 0.51f}, {256, 160, 1, 8.9f, 0.58f, 0.45f},
+                               {256, 128, 1, 7.7f, 0.50f, 0.38f}, {128, 256, 1, 8.1f, 0.52f, 0.37f}, {128, 192, 1, 6.5f, 0.48f, 0.25f},
+                               {128, 128, 2, 5.8f, 0.37f, 0.17f}, {64, 128, 2, 4.1f, 0.28f, 0.08f}, {64, 64, 2, 3.0f, 0.23f, 0.03f}};
+// Sums of parts: a kernel more, or more work for the one that adds the residual, and every part's sums written and read once, most of it in the caches.
+constexpr float PARTS_FIXED = 2.f, PARTS_BYTES_A_US = 14e6f;
+
+// Few outputs stay undivided: a router's logits (gemm_bf16_narrow) keep the bits they have beside more weight rows.
+constexpr int UNDIVIDED = 128;
+
+TilesChoice choose_tiles(int m, int n, int k, size_t sums_bytes) {
+  const int units = lrs_compute_units() > 0 ? lrs_compute_units() : 256, steps = k / 64;
+  TilesChoice best{0, 1, 0.f};
+  for (int t = 0; t < (int)(sizeof(TILES) / sizeof(TILES[0])); ++t) {
+    const TileShape& shape = TILES[t];
+    if (k % (64 * shape.panels) != 0) continue;
+    const int64_t tiles = (int64_t)((m + shape.bm - 1) / shape.bm) * ((n + shape.bn - 1) / shape.bn);
+    for (int parts = 1; parts <= (n <= UNDIVIDED ? 1 : 8); ++parts) {
+      const int each = (steps / shape.panels + parts - 1) / parts * shape.panels;   // slices of the longest part
+      const double sums = (double)parts * m * n * sizeof(float);
+      // every part has work, and eight slices of it: shorter walks are mostly beginnings
+      if (parts > 1 && (each < 8 || (parts - 1) * each >= steps || sums > (double)sums_bytes || tiles * parts > units)) continue;
+      const int64_t rounds = (tiles * parts + units - 1) / units;
+      const float share = (float)(tiles * parts) / (float)(rounds * units);
+      float us = (float)rounds * (shape.fixed + (float)each * (shape.slice + shape.crowd * share));
+      if (parts > 1) us += PARTS_FIXED + 2.f * (float)sums / PARTS_BYTES_A_US;
+      if (best.us == 0.f || us < best.us) best = TilesChoice{t, parts, us};
+    }
+  }
+  return best;
+}
+
+void launch_tiles(const TilesChoice& choice, void* out, int form, const bf16* x, const bf16* w, int m, int n, int k, int lda, int ldc, hipStream_t s) {
+  const TileShape& shape = TILES[choice.tile];
+  const int tiles_m = (m + shape.bm - 1) / shape.bm, tiles_n = (n + shape.bn - 1) / shape.bn, chunk = (tiles_m * tiles_n * choice.splits + 7) / 8;
+#define TILES_OF(...) gemm_bf16_tiles_kernel<__VA_ARGS__><<<chunk * 8, 512, 0, s>>>(x, w, m, n, k, lda, tiles_m, tiles_n, choice.splits, chunk, out, form, ldc)
+  switch (choice.tile) {
+    case 0: TILES_OF(2, 8, 4, 1, 2, 2); break;
+    case 1: TILES_OF(2, 8, 3, 1, 2, 2); break;
+    case 2: TILES_OF(4, 4, 5, 1, 1, 3); break;
+    case 3: TILES_OF(4, 4, 4, 1, 1, 3); break;
+    case 4: TILES_OF(2, 4, 4, 1, 1, 3); break;
+    case 5: TILES_OF(2, 4, 3, 1, 1, 4); break;
+    case 6: TILES_OF(2, 4, 2, 2, 2, 2); break;
+    case 7: TILES_OF(2, 2, 2, 2, 1, 3); break;
+    default: TILES_OF(4, 1, 2, 2, 1, 4); break;
+  }
+#undef TILES_OF
+}
+
+// (tokens, weight rows) of the tile and the parts of K for a product, with `sums_bytes` of room for the parts' sums; a choice of this process's
+// device, the same at every call.
+LRS_API int lrs_gemm_tiles_choice(int m, int n, int k, int64_t sums_bytes, int* bm, int* bn, int* splits) {
+  LRS_REQUIRE(m > 0 && n > 0 && k > 0 && k % 64 == 0 && sums_bytes >= 0 && bm && bn && splits, "gemm_tiles_choice: takes positive sizes, K %% 64 == 0, got m=%d n=%d k=%d", m, n, k);
+  const TilesChoice choice = choose_tiles(m, n, k, (size_t)sums_bytes);
+  *bm = TILES[choice.tile].bm, *bn = TILES[choice.tile].bn, *splits = choice.splits;
+  return 0;
+}

@@ -24,8 +24,9 @@ name of a route and `linear()` runs it.  The routes:
   split_norm more than 128 rows adding into the residual stream before an RMSNorm, of a shape whose K this package's
              many-rows kernel divides between workgroups: the kernel that adds up their sums also adds the residual
              and normalises the rows (gemm_lines_add_rmsnorm)
-  library    more rows than these kernels are made for, if the step may use the vendor library; the
-             residual add (with the norm that follows) or the gated activation take one more small kernel
+  library    more rows than these kernels are made for, if the step may use the vendor library: where they are faster with
+             what follows, this package's tiles all the same (gemm_tiles_pay: gemm, gemm_tiles_add_rmsnorm), else the library,
+             where the residual add (with the norm that follows) or the gated activation take one more small kernel
   own        everything else, and every float32 product (gemm picks the kernel by shape)
 """
 
@@ -205,6 +206,17 @@ def linear(ctx, out, x, weight, bias=None, accumulate: bool = False, swiglu: boo
         ops.gemm_lines_add_rmsnorm(out, x, weight, following[0], following[1], normed, workspace=workspace_of(ctx))
         return normed
     if route == "library":
+        fused = following is not None and out.is_contiguous()
+        if not (x.data_ptr() | out.data_ptr() | weight.data_ptr()) % 16 and m * k < 2 ** 31 and n * k < 2 ** 31:
+            # what the tiles with the rest in their epilogue are faster at
+            if swiglu or (not accumulate and out.dtype == torch.bfloat16):
+                if ops.gemm_tiles_pay(m, n, k, "gate" if swiglu else "nothing"):
+                    ops.gemm(out, x, weight, swiglu=swiglu, choice=choice, workspace=workspace_of(ctx))
+                    return None
+            elif fused and ops.gemm_tiles_pay(m, n, k, "norm"):
+                normed = ctx.scratch("norm_after_add", (m, n), ctx.dtype)
+                ops.gemm_tiles_add_rmsnorm(out, x, weight, following[0], following[1], normed, workspace=workspace_of(ctx))
+                return normed
         if not (accumulate or swiglu):
             ops.library_gemm(out, x, weight, state=library_of(ctx))                      # bfloat16, or the float32 logits of many rows
             return None
@@ -213,7 +225,7 @@ def linear(ctx, out, x, weight, bias=None, accumulate: bool = False, swiglu: boo
         if swiglu:
             ops.silu_mul(out, y, interleaved=True)
             return None
-        if following is not None and out.is_contiguous():
+        if fused:
             # the residual add and the norm that follows it in one pass over the rows
             normed = ctx.scratch("norm_after_add", (m, n), ctx.dtype)
             ops.add_rmsnorm(normed, out, y, following[0], following[1])
