@@ -2,25 +2,10 @@
 // 256 or 128 tokens x 64 to 256 weight rows, two groups of four waves in turn.
 #include "gemm_tiles.h"
 
+#include "lines_walk.h"
+
 // A workgroup of eight waves owns WM * JT * 16 tokens x (8 / WM) * IT * 16 weight rows; a wave JT x IT tiles of the 16x16x32 product.
-// Slices of 64 * PANELS of K lie in STAGES places in LDS, which memory fills itself (fetch_to_lds).  A slice is taken whole, or in two
-// halves of the wave's tokens (HALVES: registers and LDS of the largest tiles): a step of reading (the fragments; those of the weights
-// stay in registers for the second half) and a step of multiplying, with a barrier behind each.  Waves 4..7 are one step behind waves
-// 0..3, and a SIMD has one of either: while one multiplies, the other reads LDS and asks memory for a slice to come.  So neither kind of
-// work waits for the other, where waves in step (the kernel that this one replaced) all read, then all multiplied.
-//
-// What may be asked for when.  A wave has what it read before the barrier that ends its step of reading.
-// Whole slices: waves 0..3 read slice s in step 2 s, waves 4..7 in step 2 s + 1.  Behind that its place is free, and every wave asks for
-// slice s + STAGES in its next step of reading (steps 2 s + 2 and 2 s + 3).  Before the barrier that ends a step of reading, of slice s, a
-// wave waits until only the last STAGES - 2 slices are on their way: slice s + 1 is then there (steps 2 s and 2 s + 1) before anyone reads
-// it (step 2 s + 2).
-// Halves: waves 0..3 read the first half of slice s in step 4 s and the second in step 4 s + 2, waves 4..7 in steps 4 s + 1 and 4 s + 3.  The
-// first half of x and the weights of s are read by everybody when step 4 s + 1 ends, and every wave asks for those of s + STAGES when it
-// reads the second half of s (steps 4 s + 2 and 4 s + 3); the second half of s is free when step 4 s + 3 ends, and is asked for again when
-// the first half of s + 1 is read (steps 4 s + 4 and 4 s + 5).  A wave waits until only the last STAGES - 1 slices' worth is on its way: at
-// the end of reading the second half of s (steps 4 s + 2 and 4 s + 3) the first half and the weights of s + 1 are there, read from step
-// 4 s + 4 on; at the end of reading the first half of s + 1 (steps 4 s + 4 and 4 s + 5) its second half, read from step 4 s + 6 on.
-// Once there are no more slices to ask for, a wave waits for all it has asked for.
+// K is walked in slices of 64 * PANELS, whole or in two halves of the wave's tokens (HALVES), STAGES of them in LDS (lines_walk.h).
 //
 // What bounds it: the large tiles by the matrix cores' power.  8B gate_up at 2,048 rows (three rounds of 256 x 256) 291 us (1.42 PFLOP/s; 327
 // before), on another card 317, there without fetches 280, without reads as well 262, the matrix instructions alone 259 (1.59); with
@@ -29,18 +14,10 @@
 // 2,048 (256 x 192) 90 (104).  32x32x16 products instead: a tenth slower.  The small tiles by their steps' beginnings, which is why
 // they take slices of 128 whole: 1.7B q/k/v at 256 rows (64 x 64) 12.2 us, in slices of 64 14.0, of 128 x 64 in halves 18.2.
 //
-// Fetches: a block of 8 rows x 128 bytes is one fetch of one wave, lane l fills place l.  Chunk c (16 bytes) of row q lies at place
-// (q % 8) * 8 + (c ^ ((q >> 1 & 3) << 1)) of block q / 8, so that the lanes LDS serves together (eight consecutive rows of a fragment,
-// chunks g and g + 1) meet every bank once.  Rows past a matrix are read from its last row and never written.
+// Rows past a matrix are read from its last row and never written.
 // Needs K % (64 * PANELS) == 0, 16-byte aligned rows, N % 4 == 0, matrices of fewer than 2^31 elements.
 // With K divided (splits > 1) a workgroup walks its part of the slices and leaves its sums in part `split` of out [splits, m, ldc].
 // The sums of an output are one chain over its K in steps of 32, whatever the tile: bits depend on the parts alone.
-template <int N>
-__device__ __forceinline__ void wait_fetches() {
-  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
-}
-__device__ __forceinline__ void have_read_then_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-__device__ __forceinline__ void barrier_alone() { asm volatile("s_barrier" ::: "memory"); }
 __device__ __forceinline__ float silu_of(float v) { return v / (1.f + __expf(-v)); }
 
 template <int WM, int JT, int IT, int PANELS, int HALVES, int STAGES>
@@ -50,7 +27,7 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_tiles_kernel(const bf16* __r
   constexpr int X_BLOCKS = BM / 8 / HALVES, W_BLOCKS = BN / 8;   // blocks of 8 rows of a panel: of a part of the tokens, of the weights
   static_assert(X_BLOCKS * PANELS % 8 == 0 && JT % HALVES == 0, "a part of the tokens is dealt evenly to eight waves");
   constexpr int NX = X_BLOCKS * PANELS / 8, NW = W_BLOCKS * PANELS / 8, REST = W_BLOCKS * PANELS % 8;   // fetches a wave; REST: one more of the weights for the first waves
-  constexpr int STAGE_ELEMENTS = (BM + BN) * BK, EACH = HALVES * NX + NW, AHEAD = HALVES == 2 ? STAGES - 1 : STAGES - 2;
+  constexpr int STAGE_ELEMENTS = (BM + BN) * BK;
   __shared__ __attribute__((aligned(64))) bf16 slices[STAGES * STAGE_ELEMENTS];   // a stage: the tokens' panels, then the weights'
   const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int r = lane & 15, g = lane >> 4;
@@ -63,7 +40,7 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_tiles_kernel(const bf16* __r
   const int band_rows = tiles_m - band * 4 < 4 ? tiles_m - band * 4 : 4;
   const int m0 = (band * 4 + within % band_rows) * BM, n0 = (within / band_rows) * BN;
   const int wm = wave / WN, wn = wave % WN;
-  const int place_row = lane >> 3, place_chunk = (lane & 7) ^ (((place_row >> 1) & 3) << 1);
+  const int place_row = lines_place_row(lane), place_chunk = lines_place_chunk(lane);
   unsigned x_off[HALVES][NX], x_to[HALVES][NX], w_off[NW + 1];   // bytes from the matrix's first element, from the stage's first
 #pragma unroll
   for (int h = 0; h < HALVES; ++h)
@@ -80,9 +57,6 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_tiles_kernel(const bf16* __r
     const int b = wave + 8 * i, panel = b / W_BLOCKS, row = n0 + 8 * (b % W_BLOCKS) + place_row;
     w_off[i] = ((unsigned)(row < n ? row : n - 1) * (unsigned)k + panel * 64 + place_chunk * 8) * 2u;
   }
-  // this lane's fragment of rows 16 j .. 16 j + 15, k half c of a panel: row r, chunk 4 c + g
-  const int frag_row = (r >> 3) * 512 + (r & 7) * 64, turn = ((r >> 1) & 3) << 1;
-  const int frag[2] = {frag_row + ((g ^ turn) * 8), frag_row + (((4 + g) ^ turn) * 8)};
   floatx4 acc[IT][JT];
 #pragma unroll
   for (int it = 0; it < IT; ++it)
@@ -92,84 +66,20 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_tiles_kernel(const bf16* __r
   const int steps = steps_of_k - step0 < steps_each ? steps_of_k - step0 : steps_each;
   const unsigned slices_address = (unsigned)(uintptr_t)(__attribute__((address_space(3))) bf16*)slices;
   const bool one_more = REST != 0 && wave < REST;
-  auto fetch_first = [&](int s, int stage) {                       // the first part of the tokens, and the weights
-    if (s >= steps) return;
-    const int at = (step0 + s) * BK * 2;
-    const unsigned to = slices_address + (unsigned)(stage * STAGE_ELEMENTS * 2), to_w = to + (unsigned)(BM * BK * 2 + wave * 1024);
-#pragma unroll
-    for (int i = 0; i < NX; ++i) fetch_to_lds((const char*)x + at, x_off[0][i], to + x_to[0][i]);
-#pragma unroll
-    for (int i = 0; i < NW; ++i) fetch_to_lds((const char*)w + at, w_off[i], to_w + (unsigned)(i * 8192));
-    if (REST != 0 && one_more) fetch_to_lds((const char*)w + at, w_off[NW], to_w + (unsigned)(NW * 8192));
-  };
-  auto fetch_second = [&](int s, int stage) {                      // the other half of the tokens
-    if (s >= steps) return;
+  auto fetch_x = [&](int h, int s, int stage) {
     const int at = (step0 + s) * BK * 2;
     const unsigned to = slices_address + (unsigned)(stage * STAGE_ELEMENTS * 2);
 #pragma unroll
-    for (int i = 0; i < NX; ++i) fetch_to_lds((const char*)x + at, x_off[HALVES - 1][i], to + x_to[HALVES - 1][i]);
+    for (int i = 0; i < NX; ++i) fetch_to_lds((const char*)x + at, x_off[h][i], to + x_to[h][i]);
   };
-  auto wait = [&](bool more_to_come) {
-    if (!more_to_come) wait_fetches<0>();
-    else if (REST != 0 && one_more) wait_fetches<AHEAD * (EACH + 1)>();
-    else wait_fetches<AHEAD * EACH>();
+  auto fetch_w = [&](int s, int stage) {
+    const int at = (step0 + s) * BK * 2;
+    const unsigned to = slices_address + (unsigned)((stage * STAGE_ELEMENTS + BM * BK) * 2 + wave * 1024);
+#pragma unroll
+    for (int i = 0; i < NW; ++i) fetch_to_lds((const char*)w + at, w_off[i], to + (unsigned)(i * 8192));
+    if (REST != 0 && one_more) fetch_to_lds((const char*)w + at, w_off[NW], to + (unsigned)(NW * 8192));
   };
-  if constexpr (HALVES == 2) {
-#pragma unroll
-    for (int s = 0; s < STAGES; ++s) {
-      fetch_first(s, s);
-      if (s < STAGES - 1) fetch_second(s, s);
-    }
-    wait(STAGES - 1 < steps);
-  } else {
-#pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s) fetch_first(s, s);
-    wait(STAGES - 2 < steps);
-  }
-  barrier_alone();
-  if (wave >= 4) barrier_alone();                                  // a step behind from here on
-  int stage = 0;
-  bf16x8 wf[STEPS][IT], xf[STEPS][JH];
-  auto multiply = [&](int first) {
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int c = 0; c < STEPS; ++c)
-#pragma unroll
-      for (int it = 0; it < IT; ++it)
-#pragma unroll
-        for (int jt = 0; jt < JH; ++jt) acc[it][first + jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[c][it], xf[c][jt], acc[it][first + jt], 0, 0, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    barrier_alone();
-  };
-  for (int s = 0; s < steps; ++s) {
-    const bf16* xs = slices + stage * STAGE_ELEMENTS;
-    const bf16* ws = xs + BM * BK;
-    const int before = stage == 0 ? STAGES - 1 : stage - 1;
-#pragma unroll
-    for (int c = 0; c < STEPS; ++c) {
-#pragma unroll
-      for (int it = 0; it < IT; ++it) wf[c][it] = *(const bf16x8*)(ws + frag[c % 2] + (c / 2 * BN + (wn * IT + it) * 16) * 64);
-#pragma unroll
-      for (int jt = 0; jt < JH; ++jt) xf[c][jt] = *(const bf16x8*)(xs + frag[c % 2] + (c / 2 * BM + (wm * JT + jt) * 16) * 64);
-    }
-    if constexpr (HALVES == 2) fetch_second(s + STAGES - 1, before);
-    else fetch_first(s + STAGES - 1, before);
-    wait(s + STAGES - 1 < steps);
-    have_read_then_barrier();
-    multiply(0);
-    if constexpr (HALVES == 2) {
-#pragma unroll
-      for (int c = 0; c < STEPS; ++c)
-#pragma unroll
-        for (int jt = 0; jt < JH; ++jt) xf[c][jt] = *(const bf16x8*)(xs + frag[c % 2] + (c / 2 * BM + (wm * JT + JH + jt) * 16) * 64);
-      fetch_first(s + STAGES, stage);
-      wait(s + STAGES < steps);
-      have_read_then_barrier();
-      multiply(JH);
-    }
-    stage = stage == STAGES - 1 ? 0 : stage + 1;
-  }
-  if (wave < 4) barrier_alone();                                   // as many barriers for every wave
+  walk_in_turns<HALVES, PANELS, STAGES, NX, NW, REST != 0>(acc, slices, BM, BN, wm * JT * 16, wn * IT * 16, steps, one_more, fetch_x, fetch_w);
   int m0_opaque = m0;                                              // nothing of what follows is worked out before the loop ends
   asm volatile("" : "+s"(ldc), "+s"(m0_opaque));
 #pragma unroll

@@ -815,19 +815,23 @@ __device__ __forceinline__ void experts_tile(bf16* slices, TO* __restrict__ out,
                                              const bf16* __restrict__ w, int n, int k, const int* __restrict__ sorted, int m0, int n0,
                                              int top, int gather, int act, const PairAct& pa) {
   constexpr int BM = 128 * TILES, BN = 256, BK = LINES_BK, IT = 4, JT = 4 * TILES;
-  constexpr int XL = BM / 8 / 8, WL = BN / 8 / 8, STAGE_ELEMENTS = (BM + BN) * BK;
+  constexpr int HALVES = TILES, XL = BM / 8 / 8 / HALVES, WL = BN / 8 / 8, STAGE_ELEMENTS = (BM + BN) * BK;
   const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int wm = (wave >> 2) * (16 * JT), wn = (wave & 3) * 64;
   const int place_row = lines_place_row(lane), place_chunk = lines_place_chunk(lane);
   const int first_pair = sorted[m0];                                 // a tile in use begins with a row in use
   const int fallback = gather ? first_pair / top : m0;
-  unsigned xoff[XL], woff[WL];
+  unsigned xoff[HALVES][XL], xto[HALVES][XL], woff[WL];
 #pragma unroll
-  for (int i = 0; i < XL; ++i) {
-    const int at = m0 + 8 * (wave + 8 * i) + place_row, pair = sorted[at];
-    const int row = pair < 0 ? fallback : (gather ? pair / top : at);
-    xoff[i] = (unsigned)((row * lda + place_chunk * 8) * 2);
-  }
+  for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+      const int b = wave + 8 * i, first = HALVES == 2 ? ((b / JT) * 2 + h) * 8 * JT + (b % JT) * 8 : b * 8;   // a wave's half is JT blocks
+      const int at = m0 + first + place_row, pair = sorted[at];
+      const int row = pair < 0 ? fallback : (gather ? pair / top : at);
+      xto[h][i] = first * 128;
+      xoff[h][i] = (unsigned)((row * lda + place_chunk * 8) * 2);
+    }
 #pragma unroll
   for (int i = 0; i < WL; ++i) {
     const int row = n0 + 8 * (wave + 8 * i) + place_row;
@@ -840,16 +844,18 @@ __device__ __forceinline__ void experts_tile(bf16* slices, TO* __restrict__ out,
     for (int jt = 0; jt < JT; ++jt) acc[it][jt] = floatx4{0.f, 0.f, 0.f, 0.f};
   const int steps = k / BK;
   const unsigned slices_address = (unsigned)(uintptr_t)(__attribute__((address_space(3))) bf16*)slices;
-  auto fetch = [&](int kt, int stage) {
-    const int at = (kt < steps ? kt : steps - 1) * BK * 2;
-    const unsigned to = slices_address + (unsigned)(stage * STAGE_ELEMENTS * 2 + wave * 1024);
+  auto fetch_x = [&](int h, int s, int stage) {
+    const unsigned to = slices_address + (unsigned)(stage * STAGE_ELEMENTS * 2);
 #pragma unroll
-    for (int i = 0; i < XL; ++i) fetch_to_lds((const char*)x + at, xoff[i], to + (unsigned)(i * 8192));
+    for (int i = 0; i < XL; ++i) fetch_to_lds((const char*)x + s * BK * 2, xoff[h][i], to + xto[h][i]);
+  };
+  auto fetch_w = [&](int s, int stage) {
+    const unsigned to = slices_address + (unsigned)((stage * STAGE_ELEMENTS + BM * BK) * 2 + wave * 1024);
 #pragma unroll
-    for (int i = 0; i < WL; ++i) fetch_to_lds((const char*)w + at, woff[i], to + (unsigned)(BM * BK * 2 + i * 8192));
+    for (int i = 0; i < WL; ++i) fetch_to_lds((const char*)w + s * BK * 2, woff[i], to + (unsigned)(i * 8192));
   };
   int m0_opaque = m0;
-  lines_walk<STAGES, XL + WL>(acc, slices, BM, BN, wm, wn, steps, fetch);
+  walk_in_turns<HALVES, 1, STAGES, XL, WL, false>(acc, slices, BM, BN, wm, wn, steps, false, fetch_x, fetch_w);
   asm volatile("" : "+s"(ldc), "+s"(m0_opaque));
   store_expert_tile<IT, JT>(acc, out, ldc, m0_opaque + wm, n0 + wn, n, sorted, act, pa);
 }
