@@ -1669,11 +1669,14 @@ LRS_API int lrs_gemm_lines_split_pays(int m, int n, int k) {
 //   2  the residual add and a norm: a K of twice the width (more than 1,024 wide), or up to 512 rows where K is divided.  Down 512 rows 1.7B 24.6 /
 //      26.0, 4B 39.7 / 53.7, 8B 60.6 / 86.0, 14B 89.9 / 174; 2,048 rows 59.8 / 66.2, 95.8 / 113, 170 / 189, 291 / 303; o at 512 rows 0.6B 13.0 / 14.0,
 //      1.7B 16.7 / 15.8 (not divided), 4B 24.1 / 25.7, 14B 43.8 / 53.2; at 768 8B 44.9 / 40.3.
+//   3  nothing, stored as float32: from 10,240 outputs on.  10,304 outputs of K 4,096 at 256 rows 37 / 49, 512 54 / 54, 1,024 79 / 84, 2,048 145 / 207, of K 2,560 2,048
+//      104 / 105; 12,288 of 2,048 36 / 39 at 768, 28 / 27 at 512; 151,936 of 4,096 513 / 617 at 512, 301 / 305 at 144; 8,192 between a tenth slower and faster.
 // Not at all for a K of less than 512: eight slices are mostly beginnings and ends.
 LRS_API int lrs_gemm_tiles_pay(int m, int n, int k, int form) {
   if (m <= 128 || n <= NARROW_MAX || n % 4 != 0 || k < 512 || k % 64 != 0) return 0;
   if (form == 0) return m <= 256;
   if (form == 1) return n % 16 == 0;
+  if (form == 3) return n >= 10240;
   if (form != 2 || n > 8192) return 0;
   if (k >= 2 * n && n > 1024) return 1;
   return m <= 512 && choose_tiles(m, n, k, SPLIT_SUMS_BYTES).splits > 1;

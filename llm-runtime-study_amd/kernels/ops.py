@@ -701,10 +701,10 @@ def gemm_tiles_choice(m: int, n: int, k: int, sums_bytes: int | None = None) -> 
 
 @functools.lru_cache(maxsize=4096)
 def gemm_tiles_pay(m: int, n: int, k: int, follows: str) -> bool:
-    """Whether a bfloat16 product of more than 128 rows and what `follows` it ("nothing", "gate": the gated activation, "norm": the
-    residual add and an RMSNorm) are faster by this package's tiles than by the vendor library and a kernel for what follows (a rule
+    """Whether a bfloat16 product of more than 128 rows and what `follows` it ("nothing", of a bfloat16 output, "nothing, float32", "gate": the
+    gated activation, "norm": the residual add and an RMSNorm) are faster by this package's tiles than by the vendor library and a kernel for what follows (a rule
     from measurements, see `lrs_gemm_tiles_pay`)."""
-    return bool(library().lrs_gemm_tiles_pay(m, n, k, ("nothing", "gate", "norm").index(follows)))
+    return bool(library().lrs_gemm_tiles_pay(m, n, k, ("nothing", "gate", "norm", "nothing, float32").index(follows)))
 
 
 def few_rows_capacity() -> int:

@@ -209,8 +209,8 @@ def linear(ctx, out, x, weight, bias=None, accumulate: bool = False, swiglu: boo
         fused = following is not None and out.is_contiguous()
         if not (x.data_ptr() | out.data_ptr() | weight.data_ptr()) % 16 and m * k < 2 ** 31 and n * k < 2 ** 31:
             # what the tiles with the rest in their epilogue are faster at
-            if swiglu or (not accumulate and out.dtype == torch.bfloat16):
-                if ops.gemm_tiles_pay(m, n, k, "gate" if swiglu else "nothing"):
+            if swiglu or not accumulate:
+                if ops.gemm_tiles_pay(m, n, k, "gate" if swiglu else "nothing" if out.dtype == torch.bfloat16 else "nothing, float32"):
                     ops.gemm(out, x, weight, swiglu=swiglu, choice=choice, workspace=workspace_of(ctx))
                     return None
             elif fused and ops.gemm_tiles_pay(m, n, k, "norm"):

@@ -34,6 +34,7 @@ def test_what_goes_to_the_tiles_rather_than_to_the_library():
     assert pay(2048, 24576, 4096, "gate") and pay(129, 6144, 1024, "gate") and not pay(512, 6144, 1056, "gate") and not pay(512, 6152, 1024, "gate")
     assert pay(2048, 4096, 12288, "norm") and not pay(2048, 4096, 4096, "norm") and not pay(300, 64, 4096, "norm") and not pay(300, 8196, 65536, "norm")
     assert not pay(512, 24576, 448, "gate")
+    assert pay(300, 10304, 4096, "nothing, float32") and not pay(2048, 8192, 4096, "nothing, float32")
 
 
 def test_tiles_keep_their_values_in_registers(tmp_path):
