@@ -28,6 +28,11 @@ int lrs_check_launch(const char* what);
     if (!(cond)) return lrs_fail(__VA_ARGS__); \
   } while (0)
 
+// Float32 products add up K in F32_PARTS runs of so many terms (whole 128s; the last run is what is left, runs past K are none): each run a
+// chain of fused multiply-adds in ascending k from zero, the runs' sums added first to last.
+constexpr int F32_PARTS = 4;
+__host__ __device__ inline int f32_part(int k) { return ((k + 127) / 128 + F32_PARTS - 1) / F32_PARTS * 128; }
+
 template <typename T>
 __device__ __forceinline__ float to_float(T v) { return (float)v; }
 template <typename T>

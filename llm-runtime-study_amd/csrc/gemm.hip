@@ -2,8 +2,8 @@
 //   x [M, K] row-major, W [N, K] row-major, both of dtype T (float or bf16).
 // Output modes: store as T, store as float32, or add into a float32 matrix (the residual
 // stream).  Accumulation is float32 in every kernel; float32 products are chains of float32
-// fused multiply-adds (gemm_f32.hip, and the tiled kernel here for what that does not take), so a
-// float32 run is float32 throughout.  The order of the sum over K for one output element of such a
+// fused multiply-adds over runs of K (gemm_f32.hip, and the tiled kernel here for what that does not
+// take), so a float32 run is float32 throughout.  The order of the sum over K for one output element of such a
 // product never depends on M, so a row's result does not depend on what else is in the batch.
 #include "common.h"
 #include "gemm_tiles.h"
@@ -35,8 +35,17 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(void* __restrict__ out,
   const int tid = threadIdx.x;
   const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
   const int tm = (tid / 16) * 4, tn = (tid % 16) * 4;
-  float acc[4][4] = {};
+  float acc[4][4] = {}, total[4][4] = {};
+  const int part = sizeof(T) == sizeof(float) ? f32_part(k) : k;   // float32 sums are made in runs of K
+  int run_end = part;
   for (int k0 = 0; k0 < k; k0 += BK) {
+    if (k0 == run_end) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) total[i][j] += acc[i][j], acc[i][j] = 0.f;
+      run_end += part;
+    }
     for (int e = tid; e < BM * BK; e += 256) {
       const int r = e / BK, c = e % BK;
       const int gm = m0 + r, gn = n0 + r, gk = k0 + c;
@@ -64,7 +73,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(void* __restrict__ out,
     for (int j = 0; j < 4; ++j) {
       const int gn = n0 + tn + j;
       if (gn >= n) continue;
-      float v = acc[i][j];
+      float v = total[i][j] + acc[i][j];
       if (bias) v += to_float(bias[gn]);
       emit<T>(out, mode, (int64_t)gm * ldc + gn, v);
     }

@@ -2,10 +2,14 @@
 //
 // The float32 matrix instruction multiplies and adds float32 values as fused multiply-adds in ascending k, subnormal
 // numbers included: 16x16x4 gives, bit for bit, the chain of fmaf that a thread would make (checked over normal products,
-// subnormal products and subnormal inputs).  So every output here is the sum over k ascending from zero whatever kernel,
-// tile or number of rows made it, and equals the tiled kernel's in gemm.hip, which serves what this file does not take
-// (K no multiple of 32, rows not 16-byte aligned): a row's result does not depend on what else is in the batch.
+// subnormal products and subnormal inputs).  K is divided into F32_PARTS runs of whole 128s (f32_part, common.h), a chain each from
+// zero, whose sums are added first to last: four short chains at once where rows are few, and an error a quarter of one
+// chain's.  So every output here is the same sum whatever kernel, tile or number of rows made it, and equals the tiled
+// kernel's in gemm.hip, which serves what this file does not take (K no multiple of 32, rows not 16-byte aligned): a row's result
+// does not depend on what else is in the batch.
 #include "common.h"
+
+#include <type_traits>
 
 int lrs_gemm_f32(float* out, bool add, const float* a, const float* w, const float* bias, int m, int n, int k, int lda, int ldc, hipStream_t s);
 
@@ -20,25 +24,35 @@ __device__ __forceinline__ void fetch_from(uint64_t base, unsigned lane_offset, 
 // WN x WM waves side by side along weight rows and input rows, TN x TM tiles of 16 x 16 outputs a wave; slices of BK of both
 // operands lie in LDS, written there by memory itself (STAGES slices).  A tile's rows lie piece by piece, the 16 bytes of its
 // rows at one place of K after each other: the 64 single floats that a fragment read takes (16 rows, four consecutive k) meet
-// every bank once, and all of a slice's reads go by one address register.  A slice's fragments are read into registers while
+// every bank once, and all of a slice's reads go by one address register.  QUADS, where memory and not the matrix unit sets the pace: four
+// neighbouring lanes of a fetch bring 64 bytes of one row, since a lane a row costs the compute unit's L1 four times as many looks at its
+// tags (8 rows, N 1,024 K 3,072 11.5 us for 7.6); 64 bytes of all of a tile's rows lie together, and a row's four pieces of 16 bytes are
+// turned round by a quarter of its number, for the banks.  That is four address registers an operand to work out for every slice: 8
+// rows, N 4,096 K 1,024 in one chain 7.6 us so 8.9, 509 rows N 1,024 K 2,048 27 so 29.  A slice's fragments are read into registers while
 // the slice before is multiplied, between the products: what a wave does besides them has to fit the 32 cycles of a 16x16x4,
 // for a wave whose sums are one chain has nothing else to wait for (K = 3,072 in 64 workgroups: 54 cycles a product with an
 // address worked out for every read and fetch).
+// PARTS: 1, or F32_PARTS groups of waves that take a run of K each, one wave a group, with slices of its own that no barrier guards;
+// their sums meet in LDS at the end.  (With 1 a wave adds each run's sum to those before.)  A wave a SIMD: a 16x16x4 is as long in the
+// matrix unit as its sum is on its way, so two chains on a SIMD take turns.
 // WR, AR: 8 where a tile has only 8 rows of weights or inputs to bring (its other outputs are copies that nobody stores).
 // A wave's fragment of the weights is the instruction's first operand: its lanes end with four consecutive output columns.
-template <int BK, int WN, int WM, int TN, int TM, int STAGES, int WR, int AR>
-__global__ __launch_bounds__(WN * WM * WAVE) void gemm_f32_mfma_kernel(const float* __restrict__ a, const float* __restrict__ w, int m, int n, int k,
+template <bool QUADS, int BK, int PARTS, int WN, int WM, int TN, int TM, int STAGES, int WR, int AR>
+__global__ __launch_bounds__(PARTS * WN * WM * WAVE) void gemm_f32_mfma_kernel(const float* __restrict__ a, const float* __restrict__ w, int m, int n, int k,
                                                                        int lda, int tiles_m, int tiles, float* __restrict__ out, int add, int ldc,
                                                                        const float* __restrict__ bias, int wide_stores) {
   // (the arguments that lead to the first fetches come first: they are in registers when a wave begins, the file is compiled so)
   static_assert((BK == 32 || BK == 64) && (WR == 8 || WR == 16) && (AR == 8 || AR == 16), "what the layout is made for");
+  static_assert(PARTS == 1 || (PARTS == F32_PARTS && WN * WM == 1), "one group of waves for all of K, or a wave for each run of it");
   constexpr int WAVES = WN * WM, BN = WN * TN * WR, BM = WM * TM * AR;
   constexpr int CHUNKS = BK / 4;                                           // a row's pieces of 16 bytes
   constexpr int STAGE = (BN + BM) * BK, EACH = (BN + BM) * BK / 256 / WAVES;   // floats; fetches a wave and slice (a fetch brings 64 pieces)
   constexpr int W_FETCHES = CHUNKS * WR / 64, A_FETCHES = CHUNKS * AR / 64;    // for the rows of a tile
   static_assert((BN + BM) * BK / 256 % WAVES == 0 && STAGES * EACH < 64, "every wave brings as much, counted in vmcnt");
-  __shared__ __attribute__((aligned(128))) float slices[STAGES * STAGE];
+  __shared__ __attribute__((aligned(128))) float all_slices[PARTS * STAGES * STAGE];
   const int tid = threadIdx.x, lane = tid % WAVE, wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int part = PARTS == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / WAVE);
+  float* const slices = all_slices + part * (STAGES * STAGE);
   int id = blockIdx.x;
   if (tiles % 8 == 0) id = (id % 8) * (tiles / 8) + id / 8;        // an XCD takes neighbouring weight rows, which it then reads once
   const int m0 = (id % tiles_m) * BM, n0 = (id / tiles_m) * BN;
@@ -47,17 +61,27 @@ __global__ __launch_bounds__(WN * WM * WAVE) void gemm_f32_mfma_kernel(const flo
   for (int i = 0; i < EACH; ++i) {
     const int fetch = wave + i * WAVES;                                    // the weights' tiles first, then the inputs'
     if (fetch < BN / WR * W_FETCHES) {
-      const int row = fetch / W_FETCHES * WR + lane % WR, chunk = fetch % W_FETCHES * (64 / WR) + lane / WR, last = n - 1 - n0;
+      const int of_tile = QUADS ? lane / 4 % WR : lane % WR, last = n - 1 - n0, piece = fetch % W_FETCHES;
+      const int row = fetch / W_FETCHES * WR + of_tile;
+      const int chunk = QUADS ? (piece * (16 / WR) + lane / (4 * WR)) * 4 + (lane % 4 ^ (of_tile >> 2)) : piece * (64 / WR) + lane / WR;
       offset[i] = ((unsigned)(row < last ? row : last) * (unsigned)k + (unsigned)chunk * 4u) * 4u;
     } else {
       const int mine = fetch - BN / WR * W_FETCHES;
-      const int row = mine / A_FETCHES * AR + lane % AR, chunk = mine % A_FETCHES * (64 / AR) + lane / AR, last = m - 1 - m0;
+      const int of_tile = QUADS ? lane / 4 % AR : lane % AR, last = m - 1 - m0, piece = mine % A_FETCHES;
+      const int row = mine / A_FETCHES * AR + of_tile;
+      const int chunk = QUADS ? (piece * (16 / AR) + lane / (4 * AR)) * 4 + (lane % 4 ^ (of_tile >> 2)) : piece * (64 / AR) + lane / AR;
       offset[i] = ((unsigned)(row < last ? row : last) * (unsigned)lda + (unsigned)chunk * 4u) * 4u;
     }
   }
-  const int steps = k / BK;
-  const unsigned slices_address = (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)slices + (unsigned)wave * 1024u;
-  uint64_t w_at = (uint64_t)(uintptr_t)(w + (int64_t)n0 * k), a_at = (uint64_t)(uintptr_t)(a + (int64_t)m0 * lda);   // of the slice to fetch next
+  // this wave's slices: all, or its run's (none where K is too short for so many runs: it fetches the last and multiplies nothing)
+  const int run = f32_part(k) / BK, all = k / BK, first = PARTS == 1 ? 0 : part * run < all ? part * run : all - 1;
+  const int steps = PARTS == 1 ? all : part * run >= all ? 0 : all - first < run ? all - first : run;
+  const unsigned slices_address = (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)all_slices + (unsigned)(part * (STAGES * STAGE * 4) + wave * 1024);
+  uint64_t w_at = (uint64_t)(uintptr_t)(w + (int64_t)n0 * k + first * BK), a_at = (uint64_t)(uintptr_t)(a + (int64_t)m0 * lda + first * BK);   // of the slice to fetch next
+  auto slice_there = [&](auto pending) {                                   // and read by every wave that shares it
+    if constexpr (PARTS == 1) fetched_and_read_then_barrier<decltype(pending)::value>();
+    else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(decltype(pending)::value) : "memory");
+  };
   auto fetch = [&](int stage, int i) {
     const uint64_t base = wave + i * WAVES < BN / WR * W_FETCHES ? w_at : a_at;
     fetch_from(base, offset[i], slices_address + (unsigned)(stage * (STAGE * 4) + i * WAVES * 1024));
@@ -71,19 +95,25 @@ __global__ __launch_bounds__(WN * WM * WAVE) void gemm_f32_mfma_kernel(const flo
   };
   const int r = lane & 15, g = lane >> 4;
   const int wave_n = (wave % WN) * TN * WR, wave_m = (wave / WN) * TM * AR;
-  const float* w_mine = slices + wave_n * BK + (r % WR) * 4 + g;
-  const float* a_mine = slices + (BN + wave_m) * BK + (r % AR) * 4 + g;
+  // this lane's value of a tile's rows in the pieces c, c + 4, .. (QUADS; else in piece 0), in floats from the tile's first
+  int w_at_chunk[QUADS ? 4 : 1], a_at_chunk[QUADS ? 4 : 1];
+#pragma unroll
+  for (int c = 0; c < (QUADS ? 4 : 1); ++c) {
+    const int wr = r % WR, ar = r % AR;
+    w_at_chunk[c] = wave_n * BK + (QUADS ? wr * 16 + (c ^ (wr >> 2)) * 4 : wr * 4) + g;
+    a_at_chunk[c] = (BN + wave_m) * BK + (QUADS ? ar * 16 + (c ^ (ar >> 2)) * 4 : ar * 4) + g;
+  }
   auto read = [&](int stage, int c, Fragments& f) {                       // four k of a slice
 #pragma unroll
-    for (int i = 0; i < TN; ++i) f.w[c][i] = w_mine[stage * STAGE + i * WR * BK + c * WR * 4];
+    for (int i = 0; i < TN; ++i) f.w[c][i] = slices[w_at_chunk[QUADS ? c % 4 : 0] + stage * STAGE + i * WR * BK + (QUADS ? c / 4 * WR * 16 : c * WR * 4)];
 #pragma unroll
-    for (int j = 0; j < TM; ++j) f.a[c][j] = a_mine[stage * STAGE + j * AR * BK + c * AR * 4];
+    for (int j = 0; j < TM; ++j) f.a[c][j] = slices[a_at_chunk[QUADS ? c % 4 : 0] + stage * STAGE + j * AR * BK + (QUADS ? c / 4 * AR * 16 : c * AR * 4)];
   };
-  floatx4 acc[TN][TM];
+  floatx4 acc[TN][TM], total[TN][TM];
 #pragma unroll
   for (int i = 0; i < TN; ++i)
 #pragma unroll
-    for (int j = 0; j < TM; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < TM; ++j) acc[i][j] = total[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int kt = 0; kt < STAGES; ++kt) {
 #pragma unroll
@@ -91,13 +121,13 @@ __global__ __launch_bounds__(WN * WM * WAVE) void gemm_f32_mfma_kernel(const flo
     advance(kt + 1);
   }
   Fragments even, odd;
-  fetched_and_read_then_barrier<(STAGES - 1) * EACH>();
+  slice_there(std::integral_constant<int, (STAGES - 1) * EACH>());
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) read(0, c, even);
   int stage = 0;                                                           // of slice kt
   auto turn = [&](int kt, const Fragments& now, Fragments& next) {
     // slice kt + 1 is there, and every wave holds slice kt in registers: its stage may be filled again
-    fetched_and_read_then_barrier<(STAGES - 2) * EACH>();
+    slice_there(std::integral_constant<int, (STAGES - 2) * EACH>());
     const int free = stage;
     stage = stage == STAGES - 1 ? 0 : stage + 1;
 #pragma unroll
@@ -109,16 +139,46 @@ __global__ __launch_bounds__(WN * WM * WAVE) void gemm_f32_mfma_kernel(const flo
         for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.w[c][i], now.a[c][j], acc[i][j], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
       if (c < CHUNKS / 2) read(stage, 2 * c, next), read(stage, 2 * c + 1, next);
-      if (c < EACH) fetch(free, c);
+#pragma unroll
+      for (int i = c; i < EACH; i += CHUNKS) fetch(free, i);
       __builtin_amdgcn_sched_barrier(0);
     }
     advance(kt + STAGES + 1);
   };
-  for (int kt = 0; kt < steps; kt += 2) {
-    turn(kt, even, odd);
-    if (kt + 1 < steps) turn(kt + 1, odd, even);
+  for (int kt = 0, end = run;; end += run) {                               // a run has an even number of slices, but for the last
+    for (; kt < steps && kt < end; kt += 2) {
+      turn(kt, even, odd);
+      if (kt + 1 < steps) turn(kt + 1, odd, even);
+    }
+    if (kt >= steps) break;
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) total[i][j] += acc[i][j], acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                         // the fetches past K
+  if constexpr (PARTS == 1) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) acc[i][j] = total[i][j] + acc[i][j];    // (zeros where K ends with a run)
+  } else {
+    // every wave's fetches are done and its slices read: its sums go where they were
+    if (part > 0) {
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) *(floatx4*)(slices + ((i * TM + j) * WAVE + lane) * 4) = acc[i][j];
+    }
+    __syncthreads();
+    if (part > 0) return;
+#pragma unroll
+    for (int p = 1; p < PARTS; ++p)
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) acc[i][j] += *(const floatx4*)(all_slices + p * (STAGES * STAGE) + ((i * TM + j) * WAVE + lane) * 4);
+  }
 #pragma unroll
   for (int j = 0; j < TM; ++j) {
     const int token = m0 + wave_m + j * AR + r;
@@ -148,12 +208,12 @@ __global__ __launch_bounds__(WN * WM * WAVE) void gemm_f32_mfma_kernel(const flo
   }
 }
 
-// Measured on the MI355X (us; the FMA kernels that made the same sums before, 64 x 64 tiles and a thread an output):
-//   rows 509: N 4,096 K 1,024 39 (169 before), N 1,024 K 2,048 28 and K 3,072 38 (408 on average), N 6,144 K 1,024 56 (179);
-//   rows 2,048: N 24,576 K 4,096 2,978, 138 TFLOP/s of the 139 that the instruction alone reaches in a loop;
-//   rows 8: N 1,024 K 3,072 15.7 and K 2,048 11.3 (33.5 on average), N 4,096 K 1,024 9.9 (15.1), N 151,936 K 1,024 143 (141).
-// What bounds them: many rows the matrix units; few rows and few weight rows the chain of a sum, 13.3 ns for four k where nothing
-// else is in the way (16.5 here); the head memory.
+// Measured on the MI355X, us now and before runs of K, fetches of four lanes a row and the tiles for them (in a graph, weights in turn):
+//   rows 8: N 4,096 K 1,024 5.7 (7.6), N 1,024 K 2,048 6.5 (11.7) and K 3,072 7.7 (16.0), N 6,144 K 1,024 7.9 (10.5), N 151,936 K 1,024 119 (139);
+//   rows 32: 7.7 (10.1), 9.9 (15.1), 12.7 (20.4), 13.0 (17.1); rows 256: 23 (22), 19 (28), 25 (38), 39 (45);
+//   rows 509: 38 (37), 25 (28), 34 (39), 55 (54); rows 2,048: N 24,576 K 4,096 2,978, 138 TFLOP/s of the 139 that the instruction alone reaches.
+// What bounds them: many rows the matrix units; few rows the node of a graph, a trip for the first slices and the chains of a run, 13.3 ns
+// for four k; the head memory (6.2 TB/s would make 100).
 // What a launch of BN x BM tiles costs, by the outputs of the compute unit that has the most of them; `per_output` is how much
 // longer a small tile takes an output (it reads more from the L2s for each).
 int tile_cost(int m, int n, int bn, int bm, int per_output) {
@@ -175,28 +235,36 @@ LRS_API int lrs_gemm_f32_tile(int m, int n) {
 // K % 32 == 0; a, w and rows of lda floats 16-byte aligned.
 int lrs_gemm_f32(float* out, bool add, const float* a, const float* w, const float* bias, int m, int n, int k, int lda, int ldc, hipStream_t s) {
   const int wide_stores = ldc % 4 == 0 && (uintptr_t)out % 16 == 0;
-#define TILES(BK, WN, WM, TN, TM, STAGES, WR, AR)                                                                                  \
+#define TILES(QUADS, BK, PARTS, WN, WM, TN, TM, STAGES, WR, AR)                                                                           \
   do {                                                                                                                             \
     const int tiles_m = (m + WM * TM * AR - 1) / (WM * TM * AR), tiles_n = (n + WN * TN * WR - 1) / (WN * TN * WR);                \
-    gemm_f32_mfma_kernel<BK, WN, WM, TN, TM, STAGES, WR, AR><<<tiles_m * tiles_n, WN * WM * WAVE, 0, s>>>(                         \
-        a, w, m, n, k, lda, tiles_m, tiles_m * tiles_n, out, add, ldc, bias, wide_stores);                                                         \
+    gemm_f32_mfma_kernel<QUADS, BK, PARTS, WN, WM, TN, TM, STAGES, WR, AR><<<tiles_m * tiles_n, PARTS * WN * WM * WAVE, 0, s>>>(          \
+        a, w, m, n, k, lda, tiles_m, tiles_m * tiles_n, out, add, ldc, bias, wide_stores);                                         \
   } while (0)
   if (m <= 16) {
     // Few rows: memory and the chains bound it.  As many workgroups as there are tiles of 16 weight rows, of 8 where those are
-    // fewer than half the compute units (N under 2,048), with slices of 64 deep in flight; a head's many rows in workgroups of
-    // 64, which share the input rows (one wave a workgroup: 197 us, its tiles of 16 weight rows as half lines 147).
+    // fewer than half the compute units (N under 2,048), a wave for each run of K; a head's many rows in workgroups of
+    // 64, which share the input rows (119 us; a wave for each run and 16 weight rows 137).
     const bool pairs = k % 64 == 0, half = m <= 8;
-    if (n > 16384 && pairs) TILES(64, 4, 1, 2, 1, 4, 8, 16);
-    else if (!pairs) TILES(32, 1, 1, 1, 1, 15, 16, 16);
-    else if (n >= 2048) { if (half) TILES(64, 1, 1, 1, 1, 8, 16, 8); else TILES(64, 1, 1, 1, 1, 7, 16, 16); }
-    else if (half) TILES(64, 1, 1, 1, 1, 15, 8, 8);
-    else TILES(64, 1, 1, 1, 1, 10, 8, 16);
+    if (n > 16384 && pairs) TILES(true, 64, 1, 4, 1, 1, 1, 4, 16, 16);
+    else if (!pairs) TILES(false, 32, 1, 1, 1, 1, 1, 15, 16, 16);
+    else if (n >= 2048) { if (half) TILES(true, 64, 4, 1, 1, 1, 1, 3, 16, 8); else TILES(true, 32, 4, 1, 1, 1, 1, 4, 16, 16); }
+    else if (half) TILES(true, 64, 4, 1, 1, 1, 1, 8, 8, 8);
+    else TILES(true, 64, 4, 1, 1, 1, 1, 6, 8, 16);
   } else {
     switch (lrs_gemm_f32_tile(m, n)) {
-      case 16 * 1024 + 32: TILES(32, 1, 2, 1, 1, 12, 16, 16); break;
-      case 64 * 1024 + 32: TILES(32, 2, 2, 2, 1, 8, 16, 16); break;
-      case 64 * 1024 + 64: TILES(32, 2, 2, 2, 2, 3, 16, 16); break;
-      default: TILES(32, 2, 4, 4, 2, 3, 16, 16);
+      case 16 * 1024 + 32:
+        // a wave for each run of K with two chains, where K is long enough for more than one run (K 3,072, 17 to 128 rows: 12-14 us for 17-21)
+        if (f32_part(k) < k) TILES(true, 32, 4, 1, 1, 1, 2, 6, 16, 16);
+        else TILES(false, 32, 1, 1, 2, 1, 1, 12, 16, 16);
+        break;
+      case 64 * 1024 + 32:
+        // a wave for each run with eight chains, no barrier in the walk: K 3,072, 509 rows 34 us for 39
+        if (f32_part(k) < k) TILES(true, 32, 4, 1, 1, 4, 2, 3, 16, 16);
+        else TILES(false, 32, 1, 2, 2, 2, 1, 8, 16, 16);
+        break;
+      case 64 * 1024 + 64: TILES(false, 32, 1, 2, 2, 2, 2, 3, 16, 16); break;
+      default: TILES(false, 32, 1, 2, 4, 4, 2, 3, 16, 16);
     }
   }
 #undef TILES

@@ -35,7 +35,7 @@ FLAGS = [f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-fvisibility=h
 # are in registers when a wave begins, instead of a trip to memory away.
 ARGUMENTS_IN_REGISTERS = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
 FILE_FLAGS = {**{name: ARGUMENTS_IN_REGISTERS for name in ("gemm.hip", "gemm_tiles.hip", "attention.hip", "elementwise.hip", "gemm_f32.hip", "attention_f32.hip", "moe.hip")}, "latent.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", *ARGUMENTS_IN_REGISTERS],
-              "delta_chunks.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+              "delta_chunks.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "gemm_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", *ARGUMENTS_IN_REGISTERS]}
 # the vendor's matrix library, for bfloat16 products of many rows (csrc/library_gemm.hip)
 ROCM_LIB = Path(os.environ.get("ROCM_PATH", "/opt/rocm")) / "lib"
 LINK_FLAGS = [f"-L{ROCM_LIB}", "-lhipblaslt", f"-Wl,-rpath,{ROCM_LIB}"]
