@@ -9,9 +9,13 @@
 //
 // A piece is 256 products of 32 cycles at 128 dims whatever columns are in use, 6.8 us for the two waves of a SIMD: that bounds a
 // prompt (2,048 tokens, 16 heads of 128: 305 us, 56 TFLOP/s; 3,174 us with a workgroup a (token, head) and plain FMAs) and,
-// with one trip to memory before it, a decode step (8 tokens at 509: 18 us, 35 before).  A block of 16 keys, and one of
-// values, is asked for while the one before is multiplied; the registers this takes leave one workgroup a compute unit.
+// with one trip to memory before it, a decode step (8 tokens at 509: 16.6 us, 18.5 before; 509 tokens of a prompt 33, 39 before).  A block of 16 keys, and one of
+// values, is asked for while the one before is multiplied.  Memory writes it into the wave's part of LDS, 64 bytes of a row by
+// four neighbouring lanes: loaded as the products' operands lie, a lane a row, a block costs the compute unit's L1 four times as many
+// looks at its tags, and a decode step's 512 KB for a compute unit took 15 us to come.
 #include "common.h"
+
+#include <type_traits>
 
 LRS_API int lrs_compute_units();
 
@@ -60,15 +64,22 @@ __global__ __launch_bounds__(WAVES * WAVE, WAVES == 8 ? 1 : 2) void attention_f3
     const float* __restrict__ v_pages, float* __restrict__ out, int out_stride, int nkv, int page_size, float scale, int window) {
   // (what leads to the first keys comes first: those arguments are in registers when a wave begins, the file is compiled so)
   constexpr int PITCH = D + 4, TILES = D / 16;   // floats from column to column of a partial result; its tiles of 16 dims
-  extern __shared__ __attribute__((aligned(16))) float parts[];           // [WAVES][columns][PITCH], then maxima and sums [WAVES][16][2]
+  constexpr int BLOCK = 16 * D, ROOM = 2 * BLOCK > COLUMNS * PITCH ? 2 * BLOCK : COLUMNS * PITCH;   // floats: 16 keys or their values; a wave's two, or its partial result
+  __shared__ __attribute__((aligned(128))) float parts[WAVES * ROOM];
+  __shared__ float maxima[WAVES * COLUMNS * 2];                            // maxima and sums
   const int columns = together * heads;
-  float* maxima = parts + WAVES * columns * PITCH;
   const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int r = lane & 15, g = lane >> 4;
   const int kv_head = blockIdx.y;
   // the last tokens of a prompt, which see most, begin first
   const int begin = (groups - 1 - (int)blockIdx.x) * together, end = begin + together < tokens ? begin + together : tokens;
-  const unsigned key_lane = (unsigned)(r * D + 4 * g), value_lane = (unsigned)(r * page_size + 4 * g);     // floats from a block's first
+  // A fetch brings 16 bytes of each of 16 rows four times over (rows of 16 dims of a key, or of 16 keys of a value's dim): lane l the
+  // piece at place l, row l / 4; a row's pieces are turned round so that 16-byte reads of the operands meet every bank once.
+  const int place_row = lane / 4, place_piece = lane % 4 ^ (place_row >> 2 & 1) << 1;
+  const unsigned key_lane = (unsigned)(place_row * D + 4 * place_piece) * 4u, value_lane = (unsigned)(place_row * page_size + 4 * place_piece) * 4u;   // bytes
+  float* const blocks = parts + wave * ROOM;
+  const unsigned blocks_address = (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)parts + (unsigned)(wave * ROOM * 4);
+  const float* const operand = blocks + r * 16 + (g ^ (r >> 2 & 1) << 1) * 4;
   const int my_token = begin + r / heads;                                  // of this lane's column
   // the thread that merges: column and four dims
   const int item = tid, item_column = item / (D / 4), item_dim = item % (D / 4) * 4;
@@ -93,7 +104,7 @@ __global__ __launch_bounds__(WAVES * WAVE, WAVES == 8 ? 1 : 2) void attention_f3
     for (int piece0 = lowest / PIECE; piece0 <= last_piece; piece0 += WAVES) {
       const int piece = piece0 + wave;
       if (piece <= last_piece) {
-        floatx4 score[4], ahead[2][TILES];                                 // ahead: 16 keys, or their values, asked for a block ahead
+        floatx4 score[4];
         int64_t page[4];                                                   // the (page, kv head) block of 16 keys, and the slot they begin at
         int slot[4];
         bool seen[4];
@@ -106,28 +117,40 @@ __global__ __launch_bounds__(WAVES * WAVE, WAVES == 8 ? 1 : 2) void attention_f3
           page[b] = (int64_t)table[key0 / page_size] * nkv + kv_head;
           slot[b] = key0 % page_size;
         }
+        // 16 keys, or their values, are asked for a block ahead, once the wave has what it read from their place
+        auto have_read = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
         auto load_keys = [&](int b) {
+          have_read();
           const float* keys = k_pages + (page[b] * page_size + slot[b]) * D;
 #pragma unroll
-          for (int j = 0; j < TILES; ++j) ahead[b & 1][j] = *(const floatx4*)(keys + (key_lane + 16 * j));
+          for (int j = 0; j < TILES; ++j) fetch_to_lds(keys + 16 * j, key_lane, blocks_address + (unsigned)(((b & 1) * BLOCK + j * 256) * 4));
         };
         auto load_values = [&](int b) {
+          have_read();
           const float* values = v_pages + page[b] * D * page_size + slot[b];                      // [dim][slot]
 #pragma unroll
-          for (int i = 0; i < TILES; ++i) ahead[b & 1][i] = *(const floatx4*)(values + (int64_t)(16 * i) * page_size + value_lane);
+          for (int i = 0; i < TILES; ++i) fetch_to_lds(values + 16 * i * page_size, value_lane, blocks_address + (unsigned)(((b & 1) * BLOCK + i * 256) * 4));
         };
+        floatx4 now[TILES];
+        auto take = [&](int b, auto pending) {                             // block b, with so many fetches still on their way
+          asm volatile("s_waitcnt vmcnt(%0)" :: "n"(decltype(pending)::value) : "memory");
+#pragma unroll
+          for (int j = 0; j < TILES; ++j) now[j] = *(const floatx4*)(operand + (b & 1) * BLOCK + j * 256);
+        };
+        typedef std::integral_constant<int, TILES> NextBlock;
         load_keys(0);
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
           if (b < 3) load_keys(b + 1);
           else load_values(0);
+          take(b, NextBlock());
           __builtin_amdgcn_sched_barrier(0);
           score[b] = floatx4{0.f, 0.f, 0.f, 0.f};
           if (seen[b])
 #pragma unroll
             for (int j = 0; j < TILES; ++j)
 #pragma unroll
-              for (int t = 0; t < 4; ++t) score[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(ahead[b & 1][j][t], qf[j][t], score[b], 0, 0, 0);
+              for (int t = 0; t < 4; ++t) score[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(now[j][t], qf[j][t], score[b], 0, 0, 0);
           __builtin_amdgcn_sched_barrier(0);
         }
         // this lane: keys 16 b + 4 g + t of its column
@@ -160,10 +183,15 @@ __global__ __launch_bounds__(WAVES * WAVE, WAVES == 8 ? 1 : 2) void attention_f3
         for (int i = 0; i < TILES; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
-          if (b < 3) load_values(b + 1);
+          if (b < 3) {
+            load_values(b + 1);
+            take(b, NextBlock());
+          } else {
+            take(b, std::integral_constant<int, 0>());
+          }
           __builtin_amdgcn_sched_barrier(0);
           if (seen[b]) {
-            const floatx4(&vf)[TILES] = ahead[b & 1];
+            const floatx4(&vf)[TILES] = now;
             float finite = 0.f;
 #pragma unroll
             for (int i = 0; i < TILES; ++i)
@@ -182,7 +210,7 @@ __global__ __launch_bounds__(WAVES * WAVE, WAVES == 8 ? 1 : 2) void attention_f3
           __builtin_amdgcn_sched_barrier(0);
         }
         if (r < columns) {
-          float* to = parts + (wave * columns + r) * PITCH + 4 * g;
+          float* to = blocks + r * PITCH + 4 * g;
 #pragma unroll
           for (int i = 0; i < TILES; ++i) *(floatx4*)(to + 16 * i) = acc[i];
           if (g == 0) maxima[(wave * COLUMNS + r) * 2] = top, maxima[(wave * COLUMNS + r) * 2 + 1] = sum;
@@ -193,7 +221,7 @@ __global__ __launch_bounds__(WAVES * WAVE, WAVES == 8 ? 1 : 2) void attention_f3
         const int here = last_piece - piece0 + 1 < WAVES ? last_piece - piece0 + 1 : WAVES;
         for (int p = 0; p < here; ++p) {
           const float top = maxima[(p * COLUMNS + item_column) * 2], sum = maxima[(p * COLUMNS + item_column) * 2 + 1];
-          const floatx4 part = *(const floatx4*)(parts + (p * columns + item_column) * PITCH + item_dim);
+          const floatx4 part = *(const floatx4*)(parts + p * ROOM + item_column * PITCH + item_dim);
           const float now = fmaxf(run_max, top), keep = moved(run_max, now), take = moved(top, now);
           run_sum = fmaf(run_sum, keep, sum * take);
 #pragma unroll
@@ -217,8 +245,7 @@ void launch(float* out, int out_stride, const float* q, int q_stride, const floa
             const int* token_request, const int* positions, int tokens, int heads, int nkv, int page_size, float scale, int window, int together,
             hipStream_t s) {
   const dim3 grid((tokens + together - 1) / together, nkv);
-  const int columns = together * heads;
-  attention_f32_mfma_kernel<D, WAVES, SHORT><<<grid, WAVES * WAVE, sizeof(float) * WAVES * (columns * (D + 4) + COLUMNS * 2), s>>>(
+  attention_f32_mfma_kernel<D, WAVES, SHORT><<<grid, WAVES * WAVE, 0, s>>>(
       positions, token_request, block_table, q, table_stride, q_stride, tokens, together, heads, (int)grid.x, k_pages, v_pages, out, out_stride, nkv, page_size,
       scale, window);
 }
