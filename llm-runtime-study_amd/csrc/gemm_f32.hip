@@ -40,7 +40,7 @@ __device__ __forceinline__ void fetch_from(uint64_t base, unsigned lane_offset, 
 template <bool QUADS, int BK, int PARTS, int WN, int WM, int TN, int TM, int STAGES, int WR, int AR>
 __global__ __launch_bounds__(PARTS * WN * WM * WAVE) void gemm_f32_mfma_kernel(const float* __restrict__ a, const float* __restrict__ w, int m, int n, int k,
                                                                        int lda, int tiles_m, int tiles, float* __restrict__ out, int add, int ldc,
-                                                                       const float* __restrict__ bias, int wide_stores) {
+                                                                       const float* __restrict__ bias, int wide_stores, int gated) {
   // (the arguments that lead to the first fetches come first: they are in registers when a wave begins, the file is compiled so)
   static_assert((BK == 32 || BK == 64) && (WR == 8 || WR == 16) && (AR == 8 || AR == 16), "what the layout is made for");
   static_assert(PARTS == 1 || (PARTS == F32_PARTS && WN * WM == 1), "one group of waves for all of K, or a wave for each run of it");
@@ -187,8 +187,20 @@ __global__ __launch_bounds__(PARTS * WN * WM * WAVE) void gemm_f32_mfma_kernel(c
     for (int i = 0; i < TN; ++i) {
       const int col = n0 + wave_n + i * WR + 4 * g;
       if (4 * g >= WR) continue;
-      float* to = out + (int64_t)token * ldc + col;
       floatx4 v = acc[i][j];
+      if (gated) {
+        // a tile's 16 weight rows are 8 gate rows and the 8 up rows of the same features, which the lane 32 further on holds (n % 16 == 0)
+        floatx4 up;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) up[e] = __shfl(v[e], (lane + 32) % WAVE, WAVE);
+        if (g < 2 && col < n) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = v[e] / (1.0f + expf(-v[e])) * up[e];
+          *(floatx4*)(out + (int64_t)token * ldc + (col - 4 * g) / 2 + 4 * g) = v;
+        }
+        continue;
+      }
+      float* to = out + (int64_t)token * ldc + col;
       if (wide_stores && col + 3 < n) {
         if (bias)
 #pragma unroll
@@ -232,23 +244,23 @@ LRS_API int lrs_gemm_f32_tile(int m, int n) {
   return large <= largest ? 64 * 1024 + 64 : 128 * 1024 + 128;
 }
 
-// K % 32 == 0; a, w and rows of lda floats 16-byte aligned.
-int lrs_gemm_f32(float* out, bool add, const float* a, const float* w, const float* bias, int m, int n, int k, int lda, int ldc, hipStream_t s) {
+// K % 32 == 0; a, w and rows of lda floats 16-byte aligned.  gated: silu(gate) * up of weight rows interleaved in groups of 8, out [m, n / 2].
+static int launch_f32(float* out, bool add, const float* a, const float* w, const float* bias, int m, int n, int k, int lda, int ldc, int gated, hipStream_t s) {
   const int wide_stores = ldc % 4 == 0 && (uintptr_t)out % 16 == 0;
 #define TILES(QUADS, BK, PARTS, WN, WM, TN, TM, STAGES, WR, AR)                                                                           \
   do {                                                                                                                             \
     const int tiles_m = (m + WM * TM * AR - 1) / (WM * TM * AR), tiles_n = (n + WN * TN * WR - 1) / (WN * TN * WR);                \
     gemm_f32_mfma_kernel<QUADS, BK, PARTS, WN, WM, TN, TM, STAGES, WR, AR><<<tiles_m * tiles_n, PARTS * WN * WM * WAVE, 0, s>>>(          \
-        a, w, m, n, k, lda, tiles_m, tiles_m * tiles_n, out, add, ldc, bias, wide_stores);                                         \
+        a, w, m, n, k, lda, tiles_m, tiles_m * tiles_n, out, add, ldc, bias, wide_stores, gated);                                         \
   } while (0)
   if (m <= 16) {
     // Few rows: memory and the chains bound it.  As many workgroups as there are tiles of 16 weight rows, of 8 where those are
     // fewer than half the compute units (N under 2,048), a wave for each run of K; a head's many rows in workgroups of
     // 64, which share the input rows (119 us; a wave for each run and 16 weight rows 137).
     const bool pairs = k % 64 == 0, half = m <= 8;
-    if (n > 16384 && pairs) TILES(true, 64, 1, 4, 1, 1, 1, 4, 16, 16);
+    if (n > 16384 && pairs && !gated) TILES(true, 64, 1, 4, 1, 1, 1, 4, 16, 16);
     else if (!pairs) TILES(false, 32, 1, 1, 1, 1, 1, 15, 16, 16);
-    else if (n >= 2048) { if (half) TILES(true, 64, 4, 1, 1, 1, 1, 3, 16, 8); else TILES(true, 32, 4, 1, 1, 1, 1, 4, 16, 16); }
+    else if (n >= 2048 || gated) { if (half) TILES(true, 64, 4, 1, 1, 1, 1, 3, 16, 8); else TILES(true, 32, 4, 1, 1, 1, 1, 4, 16, 16); }
     else if (half) TILES(true, 64, 4, 1, 1, 1, 1, 8, 8, 8);
     else TILES(true, 64, 4, 1, 1, 1, 1, 6, 8, 16);
   } else {
@@ -269,4 +281,19 @@ int lrs_gemm_f32(float* out, bool add, const float* a, const float* w, const flo
   }
 #undef TILES
   return 0;
+}
+
+int lrs_gemm_f32(float* out, bool add, const float* a, const float* w, const float* bias, int m, int n, int k, int lda, int ldc, hipStream_t s) {
+  return launch_f32(out, add, a, w, bias, m, n, k, lda, ldc, 0, s);
+}
+
+// out [M, N / 2] (row stride ldc) = silu(gate) * up, float32, where a [M, K] (row stride lda) times w[N, K]^T gives 8 gate columns, then the 8 up
+// columns of the same features, and so on: the sums and the activation of lrs_gemm and lrs_silu_mul, bit for bit, without the
+// kernel between and its two trips through memory (8 rows of N 6,144: 5 us a layer; 509 rows 6).
+LRS_API int lrs_gemm_f32_gated(float* out, const float* a, const float* w, int m, int n, int k, int lda, int ldc, void* stream) {
+  LRS_REQUIRE(m > 0 && n > 0 && k > 0 && n % 16 == 0 && k % 32 == 0 && lda >= k && ldc >= n / 2, "gemm_f32_gated: takes N %% 16 == 0 and K %% 32 == 0, got m=%d n=%d k=%d lda=%d ldc=%d", m, n, k, lda, ldc);
+  LRS_REQUIRE(lda % 4 == 0 && ldc % 4 == 0 && (((uintptr_t)out | (uintptr_t)a | (uintptr_t)w) % 16) == 0 && (int64_t)128 * (lda > k ? lda : k) < (1ll << 30),
+              "gemm_f32_gated: needs 16-byte aligned rows (lda=%d ldc=%d)", lda, ldc);
+  if (int rc = launch_f32(out, false, a, w, nullptr, m, n, k, lda, ldc, 1, (hipStream_t)stream)) return rc;
+  return lrs_check_launch("gemm_f32_gated");
 }

@@ -117,6 +117,7 @@ _SIGNATURES = {
     "lrs_probe_mfma": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p]),
     "lrs_probe_lines": (c_int, [c_void_p, c_size_t, c_void_p, c_int, c_int, c_size_t, c_int, c_void_p]),
     "lrs_gemm_prepare": (c_int, []),
+    "lrs_gemm_f32_gated": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "lrs_library_gemm_prepare": (c_int, []),
     "lrs_library_open": (c_int, [POINTER(c_void_p)]),
     "lrs_library_close": (c_int, [c_void_p]),
@@ -252,7 +253,7 @@ def library():
 # and _SIGNATURES by kernels/plan_codegen.py, is the other side (a test keeps the two in step).
 PLAN_OPS = ("lrs_activation", "lrs_add_gathered", "lrs_add_into", "lrs_add_rmsnorm", "lrs_advance_decode", "lrs_advance_slots", "lrs_attention", "lrs_attention_decode",
             "lrs_attention_mixed", "lrs_attention_prefill", "lrs_axpby", "lrs_choose_tokens", "lrs_choose_tokens_split", "lrs_copy_to_pinned", "lrs_delta_rule", "lrs_delta_rule_channels", "lrs_delta_rule_chunks", "lrs_embed", "lrs_fill_i32",
-            "lrs_filter_logits", "lrs_filter_logits_wide", "lrs_gated_clamped", "lrs_gated_norm_add", "lrs_gather_rows", "lrs_gemm", "lrs_gemm_lines_add_rmsnorm", "lrs_gemm_mid_add_norm_begin", "lrs_gemm_mid_qk_prep", "lrs_gemm_mid_scaled",
+            "lrs_filter_logits", "lrs_filter_logits_wide", "lrs_gated_clamped", "lrs_gated_norm_add", "lrs_gather_rows", "lrs_gemm", "lrs_gemm_f32_gated", "lrs_gemm_lines_add_rmsnorm", "lrs_gemm_mid_add_norm_begin", "lrs_gemm_mid_qk_prep", "lrs_gemm_mid_scaled",
             "lrs_gemm_norm_chain", "lrs_gemm_tiles_add_rmsnorm", "lrs_head_gemm", "lrs_latent_attention", "lrs_latent_attention_groups", "lrs_latent_prep", "lrs_layernorm", "lrs_library_gemm", "lrs_mlstm", "lrs_mlstm_chunks", "lrs_moe_align", "lrs_moe_combine", "lrs_moe_experts", "lrs_moe_route", "lrs_moe_route_align", "lrs_norm_add",
             "lrs_qk_prep", "lrs_qkv_norm_prep", "lrs_rmsnorm", "lrs_rope_table", "lrs_rotate_unit_prep", "lrs_round_rows", "lrs_scale_add_layernorm", "lrs_scale_rows", "lrs_scale_values", "lrs_sigmoid_gate", "lrs_silu_mul", "lrs_soft_cap", "lrs_ssm", "lrs_xielu")
 _PLAN_INDEX = {name: index for index, name in enumerate(PLAN_OPS)}
@@ -910,6 +911,16 @@ def gemm(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor
                               dtype_code(w.dtype), m, n, k, lda, ldc, None if rows is None else _dev(rows, "rows"),
                               None if not normed else _dev(norm_weight, "norm_weight"), dtype_code(norm_weight.dtype) if normed else 0,
                               eps, 1 if swiglu else 0, choice.word, *_workspace(workspace, "gemm"), _stream())
+
+
+def gemm_f32_gated(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> None:
+    """out [M, N / 2] = silu(gate) * up, all float32, with gate and up columns of a @ w.T interleaved in groups of 8: the bits of gemm()
+    and silu_mul().  N a multiple of 16, K of 32, rows 16 bytes aligned."""
+    n, k = w.shape
+    m = a.shape[0]
+    _need(a.dtype == torch.float32 and w.dtype == torch.float32 and out.dtype == torch.float32 and w.is_contiguous() and a.shape == (m, k)
+          and out.shape == (m, n // 2) and n % 16 == 0 and k % 32 == 0, f"gemm_f32_gated: takes float32 [M, {k}] and [M, {n // 2}], N % 16 == 0, K % 32 == 0")
+    _launch("lrs_gemm_f32_gated", _dev(out, "out"), _dev(a, "a"), _dev(w, "w"), m, n, k, _rows(a, "a"), _rows(out, "out"), _stream())
 
 
 def gemm_tiles_add_rmsnorm(residual: torch.Tensor, a: torch.Tensor, w: torch.Tensor, norm_weight: torch.Tensor, eps: float,

@@ -13,7 +13,7 @@ import torch
 
 from ..kernels import ops
 from .base import Part, TensorSpec, register
-from .linear import linear, rows_of
+from .linear import linear, materialize, rows_of
 
 
 class SwiGLU(Part):
@@ -44,16 +44,21 @@ class SwiGLU(Part):
         }
 
     def bind(self, weights, dtype):
-        gate, up = weights["gate_proj.weight"].to(dtype), weights["up_proj.weight"].to(dtype)
+        gate, up = weights["gate_proj.weight"], weights["up_proj.weight"]
         h, i = self.hidden_size, self.intermediate_size
-        # bfloat16: rows interleaved in groups of 8 (8 gate rows, then the 8 up rows of the same
-        # features), so that the product's epilogue has both halves of a feature and writes
-        # silu(gate) * up itself; otherwise gate rows then up rows and a separate activation kernel
-        self.interleaved = dtype == torch.bfloat16 and i % 8 == 0 and h % 8 == 0 and self.clamped is None
-        if self.interleaved:
-            self.gate_up = torch.stack((gate.view(i // 8, 8, h), up.view(i // 8, 8, h)), 1).reshape(2 * i, h).contiguous()
+        # rows interleaved in groups of 8 (8 gate rows, then the 8 up rows of the same features), so that the product's
+        # epilogue has both halves of a feature and writes silu(gate) * up itself (in float32 where the product
+        # runs on the matrix cores); otherwise gate rows then up rows and a separate activation kernel
+        plain = self.clamped is None and i % 8 == 0
+        self.interleaved = plain and dtype == torch.bfloat16 and h % 8 == 0
+        self.gated_f32 = plain and dtype == torch.float32 and h % 32 == 0
+        if self.interleaved or self.gated_f32:
+            self.gate_up = torch.empty(2 * i, h, dtype=dtype, device=gate.device)
+            groups = self.gate_up.view(i // 8, 2, 8, h)
+            for place, rows in enumerate((gate, up)):              # brought to the run's precision on the way
+                groups[:, place].copy_(rows.reshape(i // 8, 8, h))
         else:
-            self.gate_up = torch.cat((gate, up), 0).contiguous()
+            self.gate_up = torch.cat((gate.to(dtype), up.to(dtype)), 0).contiguous()
         self.down = weights["down_proj.weight"].to(dtype).contiguous()
 
     def weight_bytes(self):
@@ -64,6 +69,14 @@ class SwiGLU(Part):
         act = ctx.scratch("ffn_act", (t, self.intermediate_size), ctx.dtype)
         if self.interleaved:
             linear(ctx, act, x, self.gate_up, swiglu=True)
+        elif self.gated_f32:
+            x = materialize(ctx, x)
+            if x.stride(1) == 1 and x.stride(0) % 4 == 0 and not (x.data_ptr() | self.gate_up.data_ptr() | act.data_ptr()) % 16:
+                ops.gemm_f32_gated(act, x, self.gate_up)
+            else:
+                gate_up = ctx.scratch("ffn_gate_up", (t, 2 * self.intermediate_size), ctx.dtype)
+                linear(ctx, gate_up, x, self.gate_up)
+                ops.silu_mul(act, gate_up, interleaved=True)
         else:
             gate_up = ctx.scratch("ffn_gate_up", (t, 2 * self.intermediate_size), ctx.dtype)
             linear(ctx, gate_up, x, self.gate_up)

@@ -29,3 +29,18 @@ def test_sums_in_runs(m, n, k):
     first = torch.empty(1, n, device="cuda")
     ops.gemm(first, a[:1], w)
     assert torch.equal(first, out[:1])
+
+
+@pytest.mark.parametrize("m", [1, 9, 17, 100, 509])
+@pytest.mark.parametrize("n,k", [(16, 32), (48, 64), (6144, 1024), (1040, 96), (2064, 640)])
+def test_gated_product(m, n, k):
+    """The activation in the product's epilogue: the bits of the product and the activation's own kernel."""
+    from llm_runtime_study_amd.kernels import ops
+
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, w = torch.randn(m, k, generator=g, device="cuda"), torch.randn(n, k, generator=g, device="cuda")
+    both, want, got = torch.empty(m, n, device="cuda"), torch.empty(m, n // 2, device="cuda"), torch.full((m + 1, n // 2 + 4), 7.0, device="cuda")
+    ops.gemm(both, a, w)
+    ops.silu_mul(want, both, interleaved=True)
+    ops.gemm_f32_gated(got[:m, :n // 2], a, w)
+    assert torch.equal(got[:m, :n // 2], want) and (got[m:] == 7).all() and (got[:, n // 2:] == 7).all()
