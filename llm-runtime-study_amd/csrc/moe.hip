@@ -807,9 +807,9 @@ __device__ __forceinline__ int pairs_to_keep(const TilesUsed& used, int tiles_n,
 // against 34, measured with nothing but fetches), and its tiles of 128 x 256 take half as much again for every product.  What bounds
 // it: few rows an expert, the weights' way from memory; many, the clock (some 2 GHz with the matrix cores this busy), the rows that
 // pad runs to tiles and the last round of workgroups.  Pairs before tiles alone: in the list's order a late pair made a round of its
-// own (612 tokens 218 us for 160).  32 experts of 8 choices, unequally loaded, 4,096 -> 2,304 features and back, this kernel against
-// that one: 200 tokens 172 / 190 and 131 / 134 us, 500 156 / 179 and 170 / 181, 612 183 / 188 and 194 / 219, 1,200 250 / 303 and 272 / 302,
-// 2,048 352 / 450 and 386 / 466, 4,096 612 / 754 and 710 / 790.
+// own (612 tokens 218 us for 160).  2,048 tokens 336 us and, back, 389; 369 and 412 with all eight waves in step.  In that form, 32 experts of
+// 8 choices, unequally loaded, 4,096 -> 2,304 features and back, against the kernel above: 200 tokens 172 / 190 and 131 / 134 us, 500
+// 156 / 179 and 170 / 181, 1,200 250 / 303 and 272 / 302, 2,048 352 / 450 and 386 / 466, 4,096 612 / 754 and 710 / 790.
 template <int TILES, int STAGES, typename TO>
 __device__ __forceinline__ void experts_tile(bf16* slices, TO* __restrict__ out, int ldc, const bf16* __restrict__ x, int lda,
                                              const bf16* __restrict__ w, int n, int k, const int* __restrict__ sorted, int m0, int n0,
