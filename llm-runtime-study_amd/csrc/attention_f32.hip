@@ -27,7 +27,8 @@ bool lrs_attention_f32_takes(const void* out, int out_stride, const void* q, int
 
 namespace {
 
-constexpr int PIECE = 64, COLUMNS = 16;
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+constexpr int PIECE = 64, COLUMNS = 16, FEW = 4;
 
 // What is left of a partial result when its reference point moves to `top`.
 __device__ __forceinline__ float moved(float from, float top) { return from == -INFINITY ? 0.f : expf(from - top); }
@@ -240,6 +241,258 @@ __global__ __launch_bounds__(WAVES * WAVE, WAVES == 8 ? 1 : 2) void attention_f3
   }
 }
 
+// f(0), f(1) .. f(N - 1), each as a constant.
+template <typename F, int... X>
+__device__ __forceinline__ void each_of(F&& f, std::integer_sequence<int, X...>) { (f(std::integral_constant<int, X>()), ...); }
+template <int N, typename F>
+__device__ __forceinline__ void each(F&& f) { each_of(f, std::make_integer_sequence<int, N>()); }
+
+// acc += column i of `a`'s block ABID (lanes 4 ABID + i) times every lane's b: element i of a lane is its own sum for column i.
+template <int ABID>
+__device__ __forceinline__ void add_few(floatx4& acc, float a, float b) {
+  acc = __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, acc, 4, ABID, 0);
+}
+// 16 keys' weighted values where some are not finite (add_odd_values): key 4 g + t is v[g][t], its weight for column i in lane 16 `block` + 4 g + i of w[t].
+__device__ __forceinline__ void add_few_odd_values(const floatx4 (&v)[4], floatx4 w, int block, floatx4& acc) {
+  for (int i = 0; i < FEW; ++i) {
+    bool plus = false, minus = false, none = false;
+    float sum = acc[i];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float x = v[g][t], weight = __shfl(w[t], 16 * block + 4 * g + i, WAVE);
+        sum = fmaf(isfinite(x) ? x : 0.f, weight, sum);
+        plus |= x == INFINITY && weight != 0.f;
+        minus |= x == -INFINITY && weight != 0.f;
+        none |= x != x && weight != 0.f;
+      }
+    if (plus) sum += INFINITY;
+    if (minus) sum -= INFINITY;
+    if (none) sum = NAN;
+    acc[i] = sum;
+  }
+}
+
+// A step in which every request brings one token and at most four heads share a kv head: the pieces of a (token, kv head) go round `divided`
+// workgroups of one wave, piece p, counted from the first that the token sees, to place p of `slots` of sums [tokens, heads of all, slots, D] and
+// maxima [..., 2], which attention_f32_merge_kernel merges.  The same operations in the same order as above, so the same bits, but on
+// 4x4x1 products, whose sixteen blocks are 64 keys (then 64 dims) for four columns, where 16x16x4 multiplies sixteen whatever is in
+// use: a quarter of the time.  All of a piece is asked for at once (64 KB of LDS at 128 dims, two workgroups a unit), the next
+// one's keys and values as soon as their place is free.
+// What bounds it: one (token, kv head) its trips to memory and the merge's launch (8 of 128 dims at 509 tokens 15.3 -> 10.0 us), many and long ones
+// two waves' fetches a unit (64 at 4,000 tokens 116 -> 73 us, 3.6 TB/s).  With 16x16x4 products instead 91 us, 16.2 for 13.7 at 509.
+template <int D>
+__global__ __launch_bounds__(WAVE, 1) void attention_f32_few_kernel(
+    const int* __restrict__ positions, const int* __restrict__ token_request, const int* __restrict__ block_table, const float* __restrict__ q, int table_stride,
+    int q_stride, int heads, int divided, const float* __restrict__ k_pages, const float* __restrict__ v_pages, float* __restrict__ sums, float* __restrict__ maxima,
+    int slots, int nkv, int page_size, float scale, int window) {
+  constexpr int TILES = D / 16, BLOCK = 16 * D, PITCH = PIECE + 4, HALVES = D / 64;
+  __shared__ __attribute__((aligned(128))) float blocks[8 * BLOCK];        // 16 keys each, then 16 keys' values each
+  __shared__ __attribute__((aligned(16))) float share[FEW * PITCH];        // scores, then weights
+  __shared__ __attribute__((aligned(16))) float queries[FEW * D];
+  const int lane = threadIdx.x, r = lane & 15, g = lane >> 4, column = r & 3;
+  const int token = blockIdx.x, kv_head = blockIdx.y;
+  const int pos = positions[token], from = first_seen(pos, window), last_piece = pos / PIECE, first_piece = from / PIECE;
+  int piece = first_piece + (int)blockIdx.z;
+  if (piece > last_piece) return;
+  const int* table = block_table + (int64_t)token_request[token] * table_stride;
+  // places of a row's pieces of 16 bytes (fetches as above), turned round so that a lane a row meets every bank once
+  const int place_row = lane / 4, place_piece = lane % 4 ^ (place_row >> 2 & 3);
+  const unsigned key_lane = (unsigned)(place_row * D + 4 * place_piece) * 4u, value_lane = (unsigned)(place_row * page_size + 4 * place_piece) * 4u;   // bytes
+  const unsigned blocks_address = (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)blocks;
+  const int turn = r >> 2 & 3;
+  auto have_read = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
+  auto block_of = [&](int at, int b, int64_t& page, int& slot) {           // the (page, kv head) block of 16 keys of piece `at`, and the slot they begin at
+    int key0 = at * PIECE + b * 16;                                        // one that is not seen stands for the nearest that is
+    key0 = key0 < (from & ~15) ? from & ~15 : key0 > (pos & ~15) ? pos & ~15 : key0;
+    page = (int64_t)table[key0 / page_size] * nkv + kv_head;
+    slot = key0 % page_size;
+  };
+  auto load_keys = [&](int at) {                                           // 16 dims of all, then the next
+    const float* keys[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      int64_t page;
+      int slot;
+      block_of(at, b, page, slot);
+      keys[b] = k_pages + (page * page_size + slot) * D;
+    }
+    have_read();
+#pragma unroll
+    for (int j = 0; j < TILES; ++j)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) fetch_to_lds(keys[b] + 16 * j, key_lane, blocks_address + (unsigned)((b * BLOCK + j * 256) * 4));
+  };
+  auto load_values = [&](int at) {
+    const float* values[4];                                                // [dim][slot]
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      int64_t page;
+      int slot;
+      block_of(at, b, page, slot);
+      values[b] = v_pages + page * D * page_size + slot;
+    }
+    have_read();
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int i = 0; i < TILES; ++i) fetch_to_lds(values[b] + 16 * i * page_size, value_lane, blocks_address + (unsigned)(((4 + b) * BLOCK + i * 256) * 4));
+  };
+  // The queries, through LDS as well: a wait of the compiler's for a load of its own would wait for all keys behind it.
+#pragma unroll
+  for (int f = 0; f < FEW * D / 256; ++f) {
+    const int at = f * 256 + 4 * lane, head = kv_head * heads + (at / D < heads ? at / D : 0);
+    fetch_lanes_to_lds((uint64_t)(uintptr_t)(q + (int64_t)token * q_stride + head * D + at % D), (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)queries + (unsigned)(f * 1024));
+  }
+  load_keys(piece);
+  load_values(piece);
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(8 * TILES < 60 ? 8 * TILES : 60) : "memory");
+  float qf[TILES];                                                         // dim 16 j + lane / 4 of this lane's column
+#pragma unroll
+  for (int j = 0; j < TILES; ++j) qf[j] = queries[(lane & 3) * D + 16 * j + lane / 4];
+  for (;;) {
+    const int next = piece + divided;
+    const bool more = next <= last_piece;
+    // scores: this lane's key for every column
+    floatx4 score_of = {0.f, 0.f, 0.f, 0.f};
+    auto score_tile = [&](auto tile) {
+      constexpr int j = decltype(tile)::value;
+      asm volatile("s_waitcnt vmcnt(%0)" :: "n"(4 * TILES + 4 * (TILES - 1 - j)) : "memory");
+      floatx4 key[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) key[c] = *(const floatx4*)(blocks + g * BLOCK + j * 256 + r * 16 + (c ^ turn) * 4);
+      each<16>([&](auto x) {                                               // dims 16 j + 4 c + t, t first to last and c within
+        constexpr int t = x / 4, c = x % 4;
+        add_few<4 * c + t>(score_of, qf[j], key[c][t]);
+      });
+    };
+    each<TILES>(score_tile);
+    if (more) load_keys(next);
+#pragma unroll
+    for (int i = 0; i < FEW; ++i) share[i * PITCH + lane] = score_of[i];
+    __builtin_amdgcn_wave_barrier();
+    // this lane: keys 16 b + 4 g + t of its column, as above
+    floatx4 score[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) score[b] = *(const floatx4*)(share + column * PITCH + 16 * b + 4 * g);
+    float top = -INFINITY;
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int key = piece * PIECE + b * 16 + 4 * g + t;
+        score[b][t] = key <= pos && key >= from ? score[b][t] * scale : -INFINITY;
+        top = fmaxf(top, score[b][t]);
+      }
+    top = fmaxf(top, __shfl_xor(top, 16, WAVE));
+    top = fmaxf(top, __shfl_xor(top, 32, WAVE));
+    const float ref = top == -INFINITY ? 0.f : top;
+    float sum = 0.f;
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int key = piece * PIECE + b * 16 + 4 * g + t;
+        score[b][t] = key <= pos && key >= from ? expf(score[b][t] - ref) : 0.f;
+        sum += score[b][t];
+      }
+    sum += __shfl_xor(sum, 16, WAVE);
+    sum += __shfl_xor(sum, 32, WAVE);
+    __builtin_amdgcn_wave_barrier();
+    if (r < FEW)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) *(floatx4*)(share + r * PITCH + 16 * b + 4 * g) = score[b];
+    __builtin_amdgcn_wave_barrier();
+    const floatx4 weights = *(const floatx4*)(share + (lane & 3) * PITCH + lane / 4 * 4);   // key 4 (lane / 4) + t of column lane % 4
+    floatx4 acc[HALVES];
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h) acc[h] = floatx4{0.f, 0.f, 0.f, 0.f};
+    auto add_block = [&](auto block) {
+      constexpr int b = decltype(block)::value;
+      if (more) asm volatile("s_waitcnt vmcnt(%0)" :: "n"((3 - b) * TILES + 4 * TILES) : "memory");
+      else asm volatile("s_waitcnt vmcnt(%0)" :: "n"((3 - b) * TILES) : "memory");
+      const int key0 = piece * PIECE + b * 16;
+      if (key0 > pos || key0 + 15 < from) return;
+      floatx4 value[HALVES][4];
+      float finite = 0.f;
+#pragma unroll
+      for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          value[h][c] = *(const floatx4*)(blocks + (4 + b) * BLOCK + (4 * h + g) * 256 + r * 16 + (c ^ turn) * 4);
+#pragma unroll
+          for (int t = 0; t < 4; ++t) finite = fmaf(value[h][c][t], 0.f, finite);
+        }
+      if (__any(finite != 0.f)) {
+#pragma unroll
+        for (int h = 0; h < HALVES; ++h) add_few_odd_values(value[h], weights, b, acc[h]);
+      } else {
+        each<16>([&](auto x) {                                             // keys 16 b + 4 c + t, t first to last and c within
+          constexpr int t = x / 4, c = x % 4;
+#pragma unroll
+          for (int h = 0; h < HALVES; ++h) add_few<4 * b + c>(acc[h], weights[t], value[h][c][t]);
+        });
+      }
+    };
+    each<4>(add_block);
+    const int place = piece - first_piece;
+    if (place < slots) {
+      const int64_t row = (int64_t)(token * nkv + kv_head) * heads;
+#pragma unroll
+      for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+        for (int i = 0; i < FEW; ++i)
+          if (i < heads) sums[((row + i) * slots + place) * D + 64 * h + lane] = acc[h][i];
+      if (lane < heads) *(floatx2*)(maxima + ((row + lane) * slots + place) * 2) = floatx2{top, sum};
+    }
+    if (!more) return;
+    load_values(next);
+    piece = next;
+  }
+}
+
+// A thread four dims of a (token, head): its pieces merged as above.  The first eight are asked for before the token's position is known (the
+// buffer has `slots` of each).
+constexpr int MERGE_AHEAD = 8;
+template <int D>
+__global__ __launch_bounds__(WAVE) void attention_f32_merge_kernel(const int* __restrict__ positions, const float* __restrict__ sums, const float* __restrict__ maxima,
+                                                                  int items, int nq, int slots, int window, float* __restrict__ out, int out_stride) {
+  const int item = blockIdx.x * WAVE + threadIdx.x;
+  if (item >= items) return;
+  const int row = item / (D / 4), dim = item % (D / 4) * 4, token = row / nq, head = row % nq;
+  const float* from = sums + (int64_t)row * slots * D + dim;
+  const float* tops = maxima + (int64_t)row * slots * 2;
+  const int pos = positions[token];
+  float run_max = -INFINITY, run_sum = 0.f;
+  floatx4 run = {0.f, 0.f, 0.f, 0.f};
+  int pieces = slots;
+  for (int p0 = 0; p0 < pieces; p0 += MERGE_AHEAD) {
+    floatx4 part[MERGE_AHEAD];
+    floatx2 ml[MERGE_AHEAD];
+#pragma unroll
+    for (int e = 0; e < MERGE_AHEAD; ++e) {
+      const int p = p0 + e < slots ? p0 + e : slots - 1;
+      part[e] = *(const floatx4*)(from + (int64_t)p * D);
+      ml[e] = *(const floatx2*)(tops + 2 * p);
+    }
+    if (p0 == 0) {
+      const int seen = pos / PIECE - first_seen(pos, window) / PIECE + 1;
+      pieces = seen < slots ? seen : slots;
+    }
+#pragma unroll
+    for (int e = 0; e < MERGE_AHEAD; ++e)
+      if (p0 + e < pieces) {
+        const float now = fmaxf(run_max, ml[e][0]), keep = moved(run_max, now), take = moved(ml[e][0], now);
+        run_sum = fmaf(run_sum, keep, ml[e][1] * take);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) run[i] = fmaf(run[i], keep, part[e][i] * take);
+        run_max = now;
+      }
+  }
+  *(floatx4*)(out + (int64_t)token * out_stride + head * D + dim) = run * (1.f / run_sum);
+}
+
 template <int D, int WAVES, bool SHORT>
 void launch(float* out, int out_stride, const float* q, int q_stride, const float* k_pages, const float* v_pages, const int* block_table, int table_stride,
             const int* token_request, const int* positions, int tokens, int heads, int nkv, int page_size, float scale, int window, int together,
@@ -290,4 +543,32 @@ int lrs_attention_f32(float* out, int out_stride, const float* q, int q_stride, 
 #undef SIZE
 #undef CALL
   return lrs_check_launch("attention");
+}
+
+// The same for a step in which every request brings one token, the pieces of a token divided between `splits` workgroups, with the bits of
+// lrs_attention: heads of 64 and 128, at most four a kv head.  No token sees more than `slots` pieces of 64 positions (what lies beyond is
+// left out); part_o holds tokens * nq * slots * d floats and part_ml two for every d.
+LRS_API int lrs_attention_f32_divided(float* out, int out_stride, const float* q, int q_stride, const float* k_pages, const float* v_pages, const int* block_table,
+                                      int table_stride, const int* token_request, const int* positions, int tokens, int nq, int nkv, int d, int page_size,
+                                      float scale, int window, int splits, int slots, float* part_o, float* part_ml, void* stream) {
+  LRS_REQUIRE(tokens > 0 && nq > 0 && nkv > 0 && nq % nkv == 0 && page_size > 0, "attention_f32_divided: bad sizes tokens=%d nq=%d nkv=%d page=%d", tokens, nq, nkv, page_size);
+  LRS_REQUIRE(lrs_attention_f32_takes(out, out_stride, q, q_stride, k_pages, v_pages, nq, nkv, d, d, page_size) && d % 64 == 0 && nq / nkv <= FEW,
+              "attention_f32_divided: takes heads of 64 or 128, at most 4 a kv head, pages of a multiple of 16, 16-byte aligned rows (nq=%d nkv=%d d=%d page=%d)", nq, nkv, d, page_size);
+  LRS_REQUIRE(splits > 0 && splits <= 65535 && slots > 0 && part_o && part_ml && ((uintptr_t)part_o | (uintptr_t)part_ml) % 16 == 0,
+              "attention_f32_divided: needs buffers for the parts' results (splits=%d slots=%d)", splits, slots);
+  LRS_REQUIRE((int64_t)tokens * nq * (d / 4) < (1 << 30) && nkv <= 65535, "attention_f32_divided: too many rows (tokens=%d nq=%d nkv=%d)", tokens, nq, nkv);
+  const hipStream_t s = (hipStream_t)stream;
+  const int items = tokens * nq * (d / 4);
+  const dim3 grid(tokens, nkv, splits);
+#define SIZE(D)                                                                                                                                            \
+  do {                                                                                                                                                     \
+    attention_f32_few_kernel<D><<<grid, WAVE, 0, s>>>(positions, token_request, block_table, q, table_stride, q_stride, nq / nkv, splits, k_pages,        \
+                                                      v_pages, part_o, part_ml, slots, nkv, page_size, scale, window);                                    \
+    if (int rc = lrs_check_launch("attention_f32_divided")) return rc;                                                                                    \
+    attention_f32_merge_kernel<D><<<(items + WAVE - 1) / WAVE, WAVE, 0, s>>>(positions, part_o, part_ml, items, nq, slots, window, out, out_stride);      \
+  } while (0)
+  if (d == 64) SIZE(64);
+  else SIZE(128);
+#undef SIZE
+  return lrs_check_launch("attention_f32_divided");
 }

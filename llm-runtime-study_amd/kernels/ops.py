@@ -132,6 +132,8 @@ _SIGNATURES = {
     "lrs_norm_begin_parts": (c_int, [c_int]),
     "lrs_attention": (c_int, [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                               c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_float, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_void_p]),
+    "lrs_attention_f32_divided": (c_int, [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
+                                          c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "lrs_qkv_norm_prep": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p,
                                   c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_float, c_int, c_void_p, c_void_p, c_void_p]),
     "lrs_gated_norm_add": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_float, c_int, c_int, c_void_p, c_float,
@@ -251,7 +253,7 @@ def library():
 #
 # PLAN_OPS fixes the number of each entry point inside a plan; csrc/plan_dispatch.inc, made from this list
 # and _SIGNATURES by kernels/plan_codegen.py, is the other side (a test keeps the two in step).
-PLAN_OPS = ("lrs_activation", "lrs_add_gathered", "lrs_add_into", "lrs_add_rmsnorm", "lrs_advance_decode", "lrs_advance_slots", "lrs_attention", "lrs_attention_decode",
+PLAN_OPS = ("lrs_activation", "lrs_add_gathered", "lrs_add_into", "lrs_add_rmsnorm", "lrs_advance_decode", "lrs_advance_slots", "lrs_attention", "lrs_attention_decode", "lrs_attention_f32_divided",
             "lrs_attention_mixed", "lrs_attention_prefill", "lrs_axpby", "lrs_choose_tokens", "lrs_choose_tokens_split", "lrs_copy_to_pinned", "lrs_delta_rule", "lrs_delta_rule_channels", "lrs_delta_rule_chunks", "lrs_embed", "lrs_fill_i32",
             "lrs_filter_logits", "lrs_filter_logits_wide", "lrs_gated_clamped", "lrs_gated_norm_add", "lrs_gather_rows", "lrs_gemm", "lrs_gemm_f32_gated", "lrs_gemm_lines_add_rmsnorm", "lrs_gemm_mid_add_norm_begin", "lrs_gemm_mid_qk_prep", "lrs_gemm_mid_scaled",
             "lrs_gemm_norm_chain", "lrs_gemm_tiles_add_rmsnorm", "lrs_head_gemm", "lrs_latent_attention", "lrs_latent_attention_groups", "lrs_latent_prep", "lrs_layernorm", "lrs_library_gemm", "lrs_mlstm", "lrs_mlstm_chunks", "lrs_moe_align", "lrs_moe_combine", "lrs_moe_experts", "lrs_moe_route", "lrs_moe_route_align", "lrs_norm_add",
@@ -1107,6 +1109,29 @@ def attention(out: torch.Tensor, q: torch.Tensor, k_pages: torch.Tensor, v_pages
 def attention_shares(dtype: torch.dtype, nq: int, nkv: int, d: int, dv: int, page_size: int, plain: bool) -> bool:
     """Whether attention() lets tokens share a workgroup (`together`): float32, and `plain`: no kept positions, sinks, cap, gates or bias."""
     return dtype == torch.float32 and plain and d == dv and d in (32, 64, 96, 128) and nq // nkv <= 16 and page_size % 16 == 0
+
+
+def attention_f32_divided(out: torch.Tensor, q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, block_table: torch.Tensor,
+                          token_request: torch.Tensor, positions: torch.Tensor, nq: int, scale: float, window: int, splits: int, slots: int,
+                          part_o: torch.Tensor, part_ml: torch.Tensor) -> None:
+    """attention() (float32, where attention_shares() says yes and q's rows are 16-byte aligned; heads of 64 or 128, at most four a kv head) for a
+    step with one token per request, with its bits: the keys of a token are divided between `splits` workgroups, whose results for every piece of 64 positions
+    meet in part_o [T, nq * slots * d] and part_ml [T, nq * slots * 2]; no token sees more than `slots` pieces."""
+    tokens = out.shape[0]
+    _need(k_pages.dim() == 4 and v_pages.dim() == 4 and k_pages.is_contiguous() and v_pages.is_contiguous(), "attention_f32_divided: pages must be contiguous")
+    _, nkv, page_size, d = k_pages.shape
+    _need(v_pages.shape == (k_pages.shape[0], nkv, d, page_size), "attention_f32_divided: key pages must be [P, nkv, page, d] and value pages [P, nkv, d, page]")
+    _need(out.shape[1] == nq * d and q.shape[0] == tokens and q.shape[1] >= nq * d, "attention_f32_divided: q/out widths do not match nq*d")
+    _need(q.dtype == k_pages.dtype == v_pages.dtype == out.dtype == torch.float32, "attention_f32_divided: q, pages and out must be float32")
+    _need(block_table.dim() == 2 and block_table.dtype == torch.int32 and block_table.stride(1) == 1, "attention_f32_divided: block_table must be int32 [R, blocks]")
+    for name, t in (("token_request", token_request), ("positions", positions)):
+        _need(t.dtype == torch.int32 and t.numel() >= tokens and t.is_contiguous(), f"attention_f32_divided: {name} must be int32 [T]")
+    for name, t, each in (("part_o", part_o, d), ("part_ml", part_ml, 2)):
+        _need(t.dtype == torch.float32 and t.is_contiguous() and t.numel() >= tokens * nq * slots * each, f"attention_f32_divided: {name} too small")
+    _launch("lrs_attention_f32_divided",
+        _dev(out, "out"), _rows(out, "out"), _dev(q, "q"), _rows(q, "q"), _dev(k_pages, "k_pages"), _dev(v_pages, "v_pages"),
+        _dev(block_table, "block_table"), block_table.stride(0), _dev(token_request, "token_request"), _dev(positions, "positions"),
+        tokens, nq, nkv, d, page_size, scale, window, splits, slots, _dev(part_o, "part_o"), _dev(part_ml, "part_ml"), _stream())
 
 
 def qkv_norm_prep(qkv: torch.Tensor, nq: int, nkv: int, d: int, dv: int, q_weight, k_weight, eps: float, cos, sin,

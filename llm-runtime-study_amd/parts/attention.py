@@ -466,21 +466,63 @@ class GQAAttention(Part):
             self._attend(ctx, out, qkv, cache, group)
         return linear(ctx, residual, out, self.w_o, accumulate=accumulate, then_norm=then_norm)
 
+    PIECE_RESULTS = 1 << 25      # floats, 128 MB, that the results of pieces of keys may take before a launch stays undivided
+
+    @staticmethod
+    def _piece_splits(workgroups: int, longest: int) -> int:
+        """Into how many workgroups of one wave attention_f32_divided() divides the keys of a row (1: attention(), which gives a row of a kv head a
+        workgroup of eight waves).  Two to a unit are a full chip; more parts than pieces have nothing to do; a class of lengths has one answer.
+        us, kv heads of 128 dims with two query heads each, attention() / divided [parts], merge counted:
+          * up to a workgroup for every four units: 8 at 509 tokens 15.3 / 10.0 [8], at 2,000 51.2 / 14.1 [32], 32 at 509 15.8 / 10.7 [8], at 4,000 112 / 45 [16],
+            64 at 260 15.0 / 14.8 [4], at 509 16.0 / 13.7 [8], at 1,000 28.4 / 21.5 [8], at 4,000 116 / 73 [8]; 64 of 64 dims 11.0 / 10.1 [8] at 509;
+          * up to one for every two units, four parts to a unit over long contexts: 96 at 4,000 125 / 101 [16] and 113 [8], 128 at 4,000 131 / 127 [8], of 64 dims
+            79 / 69 [8]; but 96 at 509 16.7 / 19.7 [8], 128 at 1,000 36.9 / 39.3 [8];
+          * beyond that attention() fills the chip: 256 at 4,000 185 / 237 [8]."""
+        units, reach = ops.compute_units(), length_class(longest)
+        if reach >= 256 and 4 * workgroups <= units:
+            return min(reach // 32, 2 * units // workgroups)
+        if reach >= 2048 and 2 * workgroups <= units:
+            return 4 * units // workgroups
+        return 1
+
+    def _attend_divided(self, ctx, out, qkv, cache, group) -> bool:
+        """Float32 attention of rows of a request each with the keys of a row divided between workgroups, if that is the faster way."""
+        rows, nq, d = qkv.shape[0], self.num_heads, self.head_dim
+        if d % 64 != 0 or nq > 4 * cache.k_pages.shape[1] or length_class(ctx.max_k) == 0 or qkv.stride(0) % 4 != 0 or qkv.data_ptr() % 16 != 0:
+            return False
+        longest, slots = ctx.max_k, -(-ctx.max_k_bound // 64)              # pieces of 64 positions, the most that a row sees
+        if self.span is not None:
+            longest, slots = min(longest, self.span + 32), min(slots, self.span // 64 + 2)
+        splits = self._piece_splits(rows * cache.k_pages.shape[1], longest)
+        if splits == 1 or rows * nq * slots * (d + 2) > self.PIECE_RESULTS:
+            return False
+        part_o = ctx.scratch("attn_piece_o", (rows * nq * slots, d), torch.float32)        # (rows of the buffer: one, not one for every bound)
+        part_ml = ctx.scratch("attn_piece_ml", (rows * nq * slots, 2), torch.float32)
+        ops.attention_f32_divided(out, qkv, cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot, ctx.positions, nq, self.scale, self.reach,
+                                  splits, slots, part_o, part_ml)
+        return True
+
     def _attend(self, ctx, out, qkv, cache, group, gates=None, **more):
         """Attention by the kernels for any shape and dtype; where tokens can share a workgroup, the single tokens at the head of a
         mixed step (each of a request of its own) go in a launch of their own, so that a prompt's tokens behind them do."""
         singles = 0 if ctx.all_decode else ctx.single_rows
         longest = ctx.max_k if length_class(ctx.max_k) == 0 else 0        # of short contexts, a class that a shape's steps share
         plain = gates is None and not self.keep_first and not more.get("softcap") and more.get("sinks") is None and more.get("distance") is None
-        if not singles or not ops.attention_shares(ctx.dtype, self.num_heads, cache.k_pages.shape[1], self.head_dim, self.value_dim, group.page_size, plain):
+        shares = ops.attention_shares(ctx.dtype, self.num_heads, cache.k_pages.shape[1], self.head_dim, self.value_dim, group.page_size, plain)
+        alone = qkv.shape[0] if ctx.all_decode else singles               # rows of a request of their own
+        if alone and shares and self._attend_divided(ctx, out[:alone], qkv[:alone], cache, group):
+            if alone == qkv.shape[0]:
+                return
+        elif not singles or not shares:
             ops.attention(out, qkv, cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot, ctx.positions, self.num_heads, self.scale,
                           self.reach, self.keep_first, gates=gates, together=1 if ctx.all_decode else 16, longest=longest, **more)
             return
+        else:
+            ops.attention(out[:singles], qkv[:singles], cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot, ctx.positions, self.num_heads,
+                          self.scale, self.reach, together=1, longest=longest)
         rest = ctx.memo.get("rows_after_singles")
         if rest is None:
             rest = ctx.memo["rows_after_singles"] = (ctx.token_slot[singles:], ctx.positions[singles:])
-        ops.attention(out[:singles], qkv[:singles], cache.k_pages, cache.v_pages, group.block_table, ctx.token_slot, ctx.positions, self.num_heads,
-                      self.scale, self.reach, together=1, longest=longest)
         ops.attention(out[singles:], qkv[singles:], cache.k_pages, cache.v_pages, group.block_table, *rest, self.num_heads, self.scale, self.reach, together=16,
                       longest=longest)
 
