@@ -37,10 +37,10 @@ __device__ __forceinline__ void fetch_from(uint64_t base, unsigned lane_offset, 
 // matrix unit as its sum is on its way, so two chains on a SIMD take turns.
 // WR, AR: 8 where a tile has only 8 rows of weights or inputs to bring (its other outputs are copies that nobody stores).
 // A wave's fragment of the weights is the instruction's first operand: its lanes end with four consecutive output columns.
-template <bool QUADS, int BK, int PARTS, int WN, int WM, int TN, int TM, int STAGES, int WR, int AR>
+template <bool GATED, bool QUADS, int BK, int PARTS, int WN, int WM, int TN, int TM, int STAGES, int WR, int AR>
 __global__ __launch_bounds__(PARTS * WN * WM * WAVE) void gemm_f32_mfma_kernel(const float* __restrict__ a, const float* __restrict__ w, int m, int n, int k,
                                                                        int lda, int tiles_m, int tiles, float* __restrict__ out, int add, int ldc,
-                                                                       const float* __restrict__ bias, int wide_stores, int gated) {
+                                                                       const float* __restrict__ bias, int wide_stores) {
   // (the arguments that lead to the first fetches come first: they are in registers when a wave begins, the file is compiled so)
   static_assert((BK == 32 || BK == 64) && (WR == 8 || WR == 16) && (AR == 8 || AR == 16), "what the layout is made for");
   static_assert(PARTS == 1 || (PARTS == F32_PARTS && WN * WM == 1), "one group of waves for all of K, or a wave for each run of it");
@@ -125,7 +125,10 @@ __global__ __launch_bounds__(PARTS * WN * WM * WAVE) void gemm_f32_mfma_kernel(c
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) read(0, c, even);
   int stage = 0;                                                           // of slice kt
-  auto turn = [&](int kt, const Fragments& now, Fragments& next) {
+  // first: slice kt begins a run of K.  What the run before left is added to the sums before it beside the first products, which begin
+  // from zero.  As a pass over the sums between two runs, with the matrix units waiting, and with the gated epilogue's instructions in
+  // every kernel, 2,048 rows of N 4,096 K 1,024 took 140.5 us (134.6 so, 134.3 in one chain) and 509 rows of N 2,048 K 6,144 108.5 (107.1, 106.2).
+  auto turn = [&](int kt, const Fragments& now, Fragments& next, auto first) {
     // slice kt + 1 is there, and every wave holds slice kt in registers: its stage may be filled again
     slice_there(std::integral_constant<int, (STAGES - 2) * EACH>());
     const int free = stage;
@@ -136,7 +139,16 @@ __global__ __launch_bounds__(PARTS * WN * WM * WAVE) void gemm_f32_mfma_kernel(c
 #pragma unroll
       for (int i = 0; i < TN; ++i)
 #pragma unroll
-        for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.w[c][i], now.a[c][j], acc[i][j], 0, 0, 0);
+        for (int j = 0; j < TM; ++j) {
+          if (decltype(first)::value && c == 0) {
+            total[i][j] += acc[i][j];
+            asm volatile("" : "+v"(total[i][j]));                          // here, not in a block between two runs
+            __builtin_amdgcn_sched_barrier(0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.w[c][i], now.a[c][j], floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+          } else {
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.w[c][i], now.a[c][j], acc[i][j], 0, 0, 0);
+          }
+        }
       __builtin_amdgcn_sched_barrier(0);
       if (c < CHUNKS / 2) read(stage, 2 * c, next), read(stage, 2 * c + 1, next);
 #pragma unroll
@@ -145,23 +157,32 @@ __global__ __launch_bounds__(PARTS * WN * WM * WAVE) void gemm_f32_mfma_kernel(c
     }
     advance(kt + STAGES + 1);
   };
-  for (int kt = 0, end = run;; end += run) {                               // a run has an even number of slices, but for the last
-    for (; kt < steps && kt < end; kt += 2) {
-      turn(kt, even, odd);
-      if (kt + 1 < steps) turn(kt + 1, odd, even);
+  const std::true_type begins;
+  const std::false_type goes_on;
+  int kt = 0;
+  auto walk = [&](int end) {
+    for (; kt < end; kt += 2) {
+      turn(kt, even, odd, goes_on);
+      if (kt + 1 < end) turn(kt + 1, odd, even, goes_on);
     }
-    if (kt >= steps) break;
-#pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-      for (int j = 0; j < TM; ++j) total[i][j] += acc[i][j], acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  };
+  if constexpr (PARTS == 1) {
+    while (kt < steps) {                                                   // a run has an even number of slices, but for the last
+      const int end = steps - kt > run ? kt + run : steps;
+      turn(kt, even, odd, begins);
+      if (kt + 1 < end) turn(kt + 1, odd, even, goes_on);
+      kt += 2;
+      walk(end);
+    }
+  } else {
+    walk(steps);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                         // the fetches past K
   if constexpr (PARTS == 1) {
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
-      for (int j = 0; j < TM; ++j) acc[i][j] = total[i][j] + acc[i][j];    // (zeros where K ends with a run)
+      for (int j = 0; j < TM; ++j) acc[i][j] = total[i][j] + acc[i][j];    // the last run's
   } else {
     // every wave's fetches are done and its slices read: its sums go where they were
     if (part > 0) {
@@ -188,7 +209,7 @@ __global__ __launch_bounds__(PARTS * WN * WM * WAVE) void gemm_f32_mfma_kernel(c
       const int col = n0 + wave_n + i * WR + 4 * g;
       if (4 * g >= WR) continue;
       floatx4 v = acc[i][j];
-      if (gated) {
+      if constexpr (GATED) {
         // a tile's 16 weight rows are 8 gate rows and the 8 up rows of the same features, which the lane 32 further on holds (n % 16 == 0)
         floatx4 up;
 #pragma unroll
@@ -222,8 +243,8 @@ __global__ __launch_bounds__(PARTS * WN * WM * WAVE) void gemm_f32_mfma_kernel(c
 
 // Measured on the MI355X, us now and before runs of K, fetches of four lanes a row and the tiles for them (in a graph, weights in turn):
 //   rows 8: N 4,096 K 1,024 5.7 (7.6), N 1,024 K 2,048 6.5 (11.7) and K 3,072 7.7 (16.0), N 6,144 K 1,024 7.9 (10.5), N 151,936 K 1,024 119 (139);
-//   rows 32: 7.7 (10.1), 9.9 (15.1), 12.7 (20.4), 13.0 (17.1); rows 256: 23 (22), 19 (28), 25 (38), 39 (45);
-//   rows 509: 38 (37), 25 (28), 34 (39), 55 (54); rows 2,048: N 24,576 K 4,096 2,978, 138 TFLOP/s of the 139 that the instruction alone reaches.
+//   rows 32: 7.7 (10.1), 9.9 (15.1), 12.7 (20.4), 13.0 (17.1); rows 256: 23 (23), 18 (28), 24 (38), 38 (45);
+//   rows 509: 39 (38), 23 (27), 32 (38), 53 (53); rows 2,048: N 24,576 K 4,096 2,978, 138 TFLOP/s of the 139 that the instruction alone reaches.
 // What bounds them: many rows the matrix units; few rows the node of a graph, a trip for the first slices and the chains of a run, 13.3 ns
 // for four k; the head memory (6.2 TB/s would make 100).
 // What a launch of BN x BM tiles costs, by the outputs of the compute unit that has the most of them; `per_output` is how much
@@ -244,25 +265,28 @@ LRS_API int lrs_gemm_f32_tile(int m, int n) {
   return large <= largest ? 64 * 1024 + 64 : 128 * 1024 + 128;
 }
 
-// K % 32 == 0; a, w and rows of lda floats 16-byte aligned.  gated: silu(gate) * up of weight rows interleaved in groups of 8, out [m, n / 2].
-static int launch_f32(float* out, bool add, const float* a, const float* w, const float* bias, int m, int n, int k, int lda, int ldc, int gated, hipStream_t s) {
+// K % 32 == 0; a, w and rows of lda floats 16-byte aligned.  GATED: silu(gate) * up of weight rows interleaved in groups of 8, out [m, n / 2].
+template <bool GATED>
+static int launch_f32(float* out, bool add, const float* a, const float* w, const float* bias, int m, int n, int k, int lda, int ldc, hipStream_t s) {
   const int wide_stores = ldc % 4 == 0 && (uintptr_t)out % 16 == 0;
 #define TILES(QUADS, BK, PARTS, WN, WM, TN, TM, STAGES, WR, AR)                                                                           \
   do {                                                                                                                             \
     const int tiles_m = (m + WM * TM * AR - 1) / (WM * TM * AR), tiles_n = (n + WN * TN * WR - 1) / (WN * TN * WR);                \
-    gemm_f32_mfma_kernel<QUADS, BK, PARTS, WN, WM, TN, TM, STAGES, WR, AR><<<tiles_m * tiles_n, PARTS * WN * WM * WAVE, 0, s>>>(          \
-        a, w, m, n, k, lda, tiles_m, tiles_m * tiles_n, out, add, ldc, bias, wide_stores, gated);                                         \
+    gemm_f32_mfma_kernel<GATED, QUADS, BK, PARTS, WN, WM, TN, TM, STAGES, WR, AR><<<tiles_m * tiles_n, PARTS * WN * WM * WAVE, 0, s>>>(   \
+        a, w, m, n, k, lda, tiles_m, tiles_m * tiles_n, out, add, ldc, bias, wide_stores);                                                \
   } while (0)
   if (m <= 16) {
     // Few rows: memory and the chains bound it.  As many workgroups as there are tiles of 16 weight rows, of 8 where those are
     // fewer than half the compute units (N under 2,048), a wave for each run of K; a head's many rows in workgroups of
     // 64, which share the input rows (119 us; a wave for each run and 16 weight rows 137).
     const bool pairs = k % 64 == 0, half = m <= 8;
-    if (n > 16384 && pairs && !gated) TILES(true, 64, 1, 4, 1, 1, 1, 4, 16, 16);
+    if (n > 16384 && pairs && !GATED) TILES(true, 64, 1, 4, 1, 1, 1, 4, 16, 16);
     else if (!pairs) TILES(false, 32, 1, 1, 1, 1, 1, 15, 16, 16);
-    else if (n >= 2048 || gated) { if (half) TILES(true, 64, 4, 1, 1, 1, 1, 3, 16, 8); else TILES(true, 32, 4, 1, 1, 1, 1, 4, 16, 16); }
-    else if (half) TILES(true, 64, 4, 1, 1, 1, 1, 8, 8, 8);
-    else TILES(true, 64, 4, 1, 1, 1, 1, 6, 8, 16);
+    else if (n >= 2048 || GATED) { if (half) TILES(true, 64, 4, 1, 1, 1, 1, 3, 16, 8); else TILES(true, 32, 4, 1, 1, 1, 1, 4, 16, 16); }
+    else if constexpr (!GATED) {
+      if (half) TILES(true, 64, 4, 1, 1, 1, 1, 8, 8, 8);
+      else TILES(true, 64, 4, 1, 1, 1, 1, 6, 8, 16);
+    }
   } else {
     switch (lrs_gemm_f32_tile(m, n)) {
       case 16 * 1024 + 32:
@@ -284,7 +308,7 @@ static int launch_f32(float* out, bool add, const float* a, const float* w, cons
 }
 
 int lrs_gemm_f32(float* out, bool add, const float* a, const float* w, const float* bias, int m, int n, int k, int lda, int ldc, hipStream_t s) {
-  return launch_f32(out, add, a, w, bias, m, n, k, lda, ldc, 0, s);
+  return launch_f32<false>(out, add, a, w, bias, m, n, k, lda, ldc, s);
 }
 
 // out [M, N / 2] (row stride ldc) = silu(gate) * up, float32, where a [M, K] (row stride lda) times w[N, K]^T gives 8 gate columns, then the 8 up
@@ -294,6 +318,6 @@ LRS_API int lrs_gemm_f32_gated(float* out, const float* a, const float* w, int m
   LRS_REQUIRE(m > 0 && n > 0 && k > 0 && n % 16 == 0 && k % 32 == 0 && lda >= k && ldc >= n / 2, "gemm_f32_gated: takes N %% 16 == 0 and K %% 32 == 0, got m=%d n=%d k=%d lda=%d ldc=%d", m, n, k, lda, ldc);
   LRS_REQUIRE(lda % 4 == 0 && ldc % 4 == 0 && (((uintptr_t)out | (uintptr_t)a | (uintptr_t)w) % 16) == 0 && (int64_t)128 * (lda > k ? lda : k) < (1ll << 30),
               "gemm_f32_gated: needs 16-byte aligned rows (lda=%d ldc=%d)", lda, ldc);
-  if (int rc = launch_f32(out, false, a, w, nullptr, m, n, k, lda, ldc, 1, (hipStream_t)stream)) return rc;
+  if (int rc = launch_f32<true>(out, false, a, w, nullptr, m, n, k, lda, ldc, (hipStream_t)stream)) return rc;
   return lrs_check_launch("gemm_f32_gated");
 }

@@ -37,3 +37,21 @@ def test_prompt_kernels_of_128_dims_spill_next_to_nothing(tmp_path):
     short = {name: count for name, count in found.items() if re.search(r"kernelILi1E", name) and not re.search(r"Lb[01]ELi[0-3]ELi[45]E", name)}
     assert short and not any(short.values()), {name: count for name, count in short.items() if count}
     assert max(found.values()) <= 10, {name: count for name, count in found.items() if count > 10}
+
+
+def test_float32_products_add_up_runs_beside_their_products(tmp_path):
+    """The large tiles of float32 products: inside the walk over K no block of instructions moves or adds sums while the matrix units wait
+    (what a run of K leaves is added beside the next run's first products)."""
+    from llm_runtime_study_amd.kernels import build
+
+    source, out = build.SOURCE_DIR / "gemm_f32.hip", tmp_path / "gemm_f32.s"
+    subprocess.run([build._hipcc(), *build.FLAGS, *build.FILE_FLAGS[source.name], "--cuda-device-only", "-S", str(source), "-o", str(out)], capture_output=True, check=True)
+    kernels = {name: text for name, text in re.findall(r"^(_Z\w*gemm_f32_mfma_kernel\w*):(.*?)\.Lfunc_end", out.read_text(), re.M | re.S)}
+    large = [text for name, text in kernels.items() if re.search(r"Li2ELi[24]ELi[24]ELi2ELi3ELi16ELi16E", name)]      # 64 x 64 and 128 x 128 outputs
+    assert len(large) >= 2
+    for text in large:
+        walk = [block for block in re.split(r"\n(?=\.LBB)", text) if re.match(r"\.LBB\w+:\s*;.*Loop", block)]
+        assert sum(block.count("v_mfma_f32_16x16x4") for block in walk) >= 128
+        for block in walk:
+            if "v_mfma_f32_16x16x4" not in block:
+                assert len(re.findall(r"^\tv_", block, re.M)) <= 8, block
