@@ -280,7 +280,11 @@ static int launch_f32(float* out, bool add, const float* a, const float* w, cons
     // fewer than half the compute units (N under 2,048), a wave for each run of K; a head's many rows in workgroups of
     // 64, which share the input rows (119 us; a wave for each run and 16 weight rows 137).
     const bool pairs = k % 64 == 0, half = m <= 8;
-    if (n > 16384 && pairs && !GATED) TILES(true, 64, 1, 4, 1, 1, 1, 4, 16, 16);
+    // Gated products take a wave for each run further, until the rows of every workgroup weigh more than the weights (shared / a wave for each
+    // run: N 24,576 K 4,096 8 rows 84.2 / 78.8, 12 81.4 / 80.3, 16 82.6 / 87; N 34,816 K 5,120 8 rows 164 / 148, 12 162 / 165, 16 163 / 181;
+    // N 51,200 K 5,120 4 rows 206 / 195, 8 202 / 206, 16 211 / 262; N 17,408 K 4,096 16 rows 82 / 72).
+    const bool shared = n > 16384 && (!GATED || (int64_t)m * n >= 24 * 16384);
+    if (shared && pairs) TILES(true, 64, 1, 4, 1, 1, 1, 4, 16, 16);
     else if (!pairs) TILES(false, 32, 1, 1, 1, 1, 1, 15, 16, 16);
     else if (n >= 2048 || GATED) { if (half) TILES(true, 64, 4, 1, 1, 1, 1, 3, 16, 8); else TILES(true, 32, 4, 1, 1, 1, 1, 4, 16, 16); }
     else if constexpr (!GATED) {

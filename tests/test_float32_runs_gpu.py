@@ -31,8 +31,9 @@ def test_sums_in_runs(m, n, k):
     assert torch.equal(first, out[:1])
 
 
-@pytest.mark.parametrize("m", [1, 9, 17, 100, 509])
-@pytest.mark.parametrize("n,k", [(16, 32), (48, 64), (6144, 1024), (1040, 96), (2064, 640)])
+# the last five: on either side of 24 x 16,384 outputs, where workgroups of 64 weight rows share the input rows
+@pytest.mark.parametrize("m,n,k", [(m, n, k) for m in (1, 9, 17, 100, 509) for n, k in ((16, 32), (48, 64), (6144, 1024), (1040, 96), (2064, 640))]
+                         + [(16, 24592, 64), (16, 24560, 192), (8, 49168, 640), (15, 26224, 96), (1, 393232, 64)])
 def test_gated_product(m, n, k):
     """The activation in the product's epilogue: the bits of the product and the activation's own kernel."""
     from llm_runtime_study_amd.kernels import ops
