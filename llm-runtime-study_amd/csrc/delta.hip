@@ -139,7 +139,7 @@ __global__ void delta_prepare_kernel(const TP* __restrict__ proj, int ld, const 
 
 // The same for steps with portions, for heads of up to 128 dims, four taps and one decay a head: a wave takes RUN tokens of a unit, so that a
 // token's inputs are read once and not once for every tap, the weights once for all, and the launch has an eighth of the waves in
-// workgroups of four (2,048 tokens of 48 units were 98,304 workgroups of a wave: 68 us, most of it the launching of them; 30 so).  All
+// workgroups of four (2,048 tokens of 48 units were 98,304 workgroups of a wave: 68 us, most of it the launching of them; 30 so; lrs_delta_in_runs says when).  All
 // inputs are asked for before any is used.  Tokens of two requests in one run, and the run that ends the step, are taken one by one.
 // Every value is made as above, bit for bit.
 constexpr int RUN = 8, RUN_TAPS = 4;
@@ -650,6 +650,16 @@ void launch_scan(int rows, bool single, dim3 grid, hipStream_t s, const float* q
 // Rows of a head's matrix that one lane holds: the key size over the 16 lanes of a column, to the next of 4, 8, 16.
 LRS_API int lrs_delta_state_rows(int d) { return d <= 64 ? 4 : d <= 128 ? 8 : 16; }
 
+// Whether a step's tokens are prepared in runs of eight (delta_prepare_runs_kernel): portions, and enough of them.  A wave of a run has a longer
+// chain (a boundary between two requests inside a run costs it eight trips, one after the other); what it saves is the launching of a wave
+// for every (token, unit).  us of the rule, a wave for each / runs, 8 groups and 32 heads of 128 (48 units): one portion of 8 tokens 13.9 / 17.4, 128
+// 51.2 / 51.2, 512 163 / 152; 16 portions of 9 39.9 / 43.7 (bfloat16 42.4 / 50.7), 64 of 5 83.9 / 80.9 (87.0 / 88.6), 100 of 5 149 / 127; 4 groups and
+// 8 heads (16 units): 512 tokens 134 / 134, 4 portions of 150 52.0 / 52.3 (53.8 / 55.8), 64 of 12 27.3 / 27.3 (29.2 / 30.8), 400 of 5 57.5 / 52.6.
+// From 64 waves of the first kind a compute unit on runs are as fast or faster in all of them.
+LRS_API int lrs_delta_in_runs(int tokens, int requests, int taps, int G, int H, int d, int dv, int decay_rank) {
+  return (int64_t)tokens * (2 * G + H) >= 16384 && tokens >= 2 * requests && taps == RUN_TAPS && decay_rank == 0 && d <= 2 * WAVE && dv <= 2 * WAVE;
+}
+
 namespace {
 
 // The gated delta rule's kernels for one step.  gate_at, beta_at, decay_at: columns of proj.  decay_rank > 0: a decay per
@@ -683,9 +693,7 @@ int delta_launch(void* out, int out_dtype, const void* proj, int proj_dtype, int
   dim3 pgrid(tokens, 2 * G + H), kgrid(requests, (channels + 255) / 256), sgrid(requests, H, (dv + COLUMNS - 1) / COLUMNS);
   const int64_t pairs = (int64_t)tokens * H;
   const bool single = tokens == requests;
-  // Runs of tokens where portions have them: with two tokens a request on the mean the waves that take tokens one by one are no slower
-  // than a wave for each, and the launch is shorter.
-  const bool in_runs = tokens >= 2 * requests && tokens >= RUN && taps == RUN_TAPS && decay_rank == 0 && d <= 2 * WAVE && dv <= 2 * WAVE;
+  const bool in_runs = lrs_delta_in_runs(tokens, requests, taps, G, H, d, dv, decay_rank) != 0;
   const bool many_pairs = gate_rank == 0 && dv <= 2 * WAVE && pairs >= 8192;      // 32 waves a compute unit and more one by one
 #define ALL(TP, TO)                                                                                                           \
   do {                                                                                                                        \

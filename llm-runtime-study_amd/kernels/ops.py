@@ -117,6 +117,7 @@ _SIGNATURES = {
     "lrs_probe_mfma": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p]),
     "lrs_probe_lines": (c_int, [c_void_p, c_size_t, c_void_p, c_int, c_int, c_size_t, c_int, c_void_p]),
     "lrs_gemm_prepare": (c_int, []),
+    "lrs_delta_in_runs": (c_int, [c_int] * 8),
     "lrs_gemm_f32_gated": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "lrs_library_gemm_prepare": (c_int, []),
     "lrs_library_open": (c_int, [POINTER(c_void_p)]),
@@ -1596,6 +1597,12 @@ def delta_state_floats(heads: int, kv_heads: int, dim: int, vdim: int, taps: int
 def delta_pack_floats(tokens: int, requests: int, heads: int, dim: int, vdim: int) -> int:
     """Floats of delta_rule()'s packs for a step of so many tokens; requests: those behind the `singles`."""
     return library().lrs_delta_pack_floats(tokens, requests, heads, dim, vdim)
+
+
+def delta_in_runs(tokens: int, requests: int, taps: int, kv_heads: int, heads: int, dim: int, vdim: int) -> bool:
+    """Whether delta_rule() prepares a step's tokens in runs of eight rather than one by one: portions, and enough of them to pay
+    (see `lrs_delta_in_runs`); the same values either way."""
+    return bool(library().lrs_delta_in_runs(tokens, requests, taps, kv_heads, heads, dim, vdim, 0))
 
 
 def delta_rule(out: torch.Tensor, proj: torch.Tensor, state: torch.Tensor, token_request: torch.Tensor, cu_seqlens: torch.Tensor,
