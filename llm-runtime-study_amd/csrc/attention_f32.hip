@@ -56,16 +56,18 @@ __device__ __forceinline__ void add_odd_values(floatx4 values, floatx4 weights, 
 }
 
 // SHORT: blocks of 16 keys that nobody sees are left out rather than multiplied with weights of zero.
+// DIRECT: keys and values into registers as the products' operands lie, not into LDS first: a trip shorter, which a wave of one piece waits
+// for (lrs_attention_f32 says when).
 // One workgroup: `together` tokens (as many as fit 16 columns with the kv group's heads) of one kv head, taken request by
 // request should they not all belong to one.
-template <int D, int WAVES, bool SHORT>
+template <int D, int WAVES, bool SHORT, bool DIRECT>
 __global__ __launch_bounds__(WAVES * WAVE, WAVES == 8 ? 1 : 2) void attention_f32_mfma_kernel(
     const int* __restrict__ positions, const int* __restrict__ token_request, const int* __restrict__ block_table, const float* __restrict__ q,
     int table_stride, int q_stride, int tokens, int together, int heads, int groups, const float* __restrict__ k_pages,
     const float* __restrict__ v_pages, float* __restrict__ out, int out_stride, int nkv, int page_size, float scale, int window) {
   // (what leads to the first keys comes first: those arguments are in registers when a wave begins, the file is compiled so)
   constexpr int PITCH = D + 4, TILES = D / 16;   // floats from column to column of a partial result; its tiles of 16 dims
-  constexpr int BLOCK = 16 * D, ROOM = 2 * BLOCK > COLUMNS * PITCH ? 2 * BLOCK : COLUMNS * PITCH;   // floats: 16 keys or their values; a wave's two, or its partial result
+  constexpr int BLOCK = 16 * D, ROOM = !DIRECT && 2 * BLOCK > COLUMNS * PITCH ? 2 * BLOCK : COLUMNS * PITCH;   // floats: 16 keys or their values; a wave's two, or its partial result
   __shared__ __attribute__((aligned(128))) float parts[WAVES * ROOM];
   __shared__ float maxima[WAVES * COLUMNS * 2];                            // maxima and sums
   const int columns = together * heads;
@@ -118,25 +120,37 @@ __global__ __launch_bounds__(WAVES * WAVE, WAVES == 8 ? 1 : 2) void attention_f3
           page[b] = (int64_t)table[key0 / page_size] * nkv + kv_head;
           slot[b] = key0 % page_size;
         }
-        // 16 keys, or their values, are asked for a block ahead, once the wave has what it read from their place
+        // 16 keys, or their values, are asked for a block ahead, into LDS once the wave has what it read from their place
+        floatx4 held[DIRECT ? 2 : 1][TILES];
         auto have_read = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
         auto load_keys = [&](int b) {
-          have_read();
           const float* keys = k_pages + (page[b] * page_size + slot[b]) * D;
+          if constexpr (DIRECT) {
 #pragma unroll
-          for (int j = 0; j < TILES; ++j) fetch_to_lds(keys + 16 * j, key_lane, blocks_address + (unsigned)(((b & 1) * BLOCK + j * 256) * 4));
+            for (int j = 0; j < TILES; ++j) held[b & 1][j] = *(const floatx4*)(keys + (unsigned)(r * D + 4 * g) + 16 * j);
+          } else {
+            have_read();
+#pragma unroll
+            for (int j = 0; j < TILES; ++j) fetch_to_lds(keys + 16 * j, key_lane, blocks_address + (unsigned)(((b & 1) * BLOCK + j * 256) * 4));
+          }
         };
         auto load_values = [&](int b) {
-          have_read();
           const float* values = v_pages + page[b] * D * page_size + slot[b];                      // [dim][slot]
+          if constexpr (DIRECT) {
 #pragma unroll
-          for (int i = 0; i < TILES; ++i) fetch_to_lds(values + 16 * i * page_size, value_lane, blocks_address + (unsigned)(((b & 1) * BLOCK + i * 256) * 4));
+            for (int i = 0; i < TILES; ++i) held[b & 1][i] = *(const floatx4*)(values + (int64_t)(16 * i) * page_size + (unsigned)(r * page_size + 4 * g));
+          } else {
+            have_read();
+#pragma unroll
+            for (int i = 0; i < TILES; ++i) fetch_to_lds(values + 16 * i * page_size, value_lane, blocks_address + (unsigned)(((b & 1) * BLOCK + i * 256) * 4));
+          }
         };
-        floatx4 now[TILES];
         auto take = [&](int b, auto pending) {                             // block b, with so many fetches still on their way
-          asm volatile("s_waitcnt vmcnt(%0)" :: "n"(decltype(pending)::value) : "memory");
+          if constexpr (!DIRECT) {
+            asm volatile("s_waitcnt vmcnt(%0)" :: "n"(decltype(pending)::value) : "memory");
 #pragma unroll
-          for (int j = 0; j < TILES; ++j) now[j] = *(const floatx4*)(operand + (b & 1) * BLOCK + j * 256);
+            for (int j = 0; j < TILES; ++j) held[0][j] = *(const floatx4*)(operand + (b & 1) * BLOCK + j * 256);
+          }
         };
         typedef std::integral_constant<int, TILES> NextBlock;
         load_keys(0);
@@ -151,7 +165,7 @@ __global__ __launch_bounds__(WAVES * WAVE, WAVES == 8 ? 1 : 2) void attention_f3
 #pragma unroll
             for (int j = 0; j < TILES; ++j)
 #pragma unroll
-              for (int t = 0; t < 4; ++t) score[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(now[j][t], qf[j][t], score[b], 0, 0, 0);
+              for (int t = 0; t < 4; ++t) score[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(held[DIRECT ? b & 1 : 0][j][t], qf[j][t], score[b], 0, 0, 0);
           __builtin_amdgcn_sched_barrier(0);
         }
         // this lane: keys 16 b + 4 g + t of its column
@@ -192,7 +206,7 @@ __global__ __launch_bounds__(WAVES * WAVE, WAVES == 8 ? 1 : 2) void attention_f3
           }
           __builtin_amdgcn_sched_barrier(0);
           if (seen[b]) {
-            const floatx4(&vf)[TILES] = now;
+            const floatx4(&vf)[TILES] = held[DIRECT ? b & 1 : 0];
             float finite = 0.f;
 #pragma unroll
             for (int i = 0; i < TILES; ++i)
@@ -493,12 +507,12 @@ __global__ __launch_bounds__(WAVE) void attention_f32_merge_kernel(const int* __
   *(floatx4*)(out + (int64_t)token * out_stride + head * D + dim) = run * (1.f / run_sum);
 }
 
-template <int D, int WAVES, bool SHORT>
+template <int D, int WAVES, bool SHORT, bool DIRECT>
 void launch(float* out, int out_stride, const float* q, int q_stride, const float* k_pages, const float* v_pages, const int* block_table, int table_stride,
             const int* token_request, const int* positions, int tokens, int heads, int nkv, int page_size, float scale, int window, int together,
             hipStream_t s) {
   const dim3 grid((tokens + together - 1) / together, nkv);
-  attention_f32_mfma_kernel<D, WAVES, SHORT><<<grid, WAVES * WAVE, 0, s>>>(
+  attention_f32_mfma_kernel<D, WAVES, SHORT, DIRECT><<<grid, WAVES * WAVE, 0, s>>>(
       positions, token_request, block_table, q, table_stride, q_stride, tokens, together, heads, (int)grid.x, k_pages, v_pages, out, out_stride, nkv, page_size,
       scale, window);
 }
@@ -509,6 +523,19 @@ bool lrs_attention_f32_takes(const void* out, int out_stride, const void* q, int
                              int d, int dv, int page_size) {
   const uintptr_t places = (uintptr_t)out | (uintptr_t)q | (uintptr_t)k_pages | (uintptr_t)v_pages;
   return d == dv && (d == 32 || d == 64 || d == 96 || d == 128) && nq / nkv <= COLUMNS && page_size % 16 == 0 && places % 16 == 0 && out_stride % 4 == 0 && q_stride % 4 == 0;
+}
+
+// Whether keys and values go straight into registers (DIRECT): where a wave has one piece or two and waits for its first block, which comes a
+// trip through LDS sooner, and where rows of a request each fill nearly one round of the chip over a few hundred keys.  us, direct / through LDS,
+// 8 kv heads of 128: one row at 100 tokens 9.1 / 9.9, at 160 9.9 / 10.4, at 255 10.8 / 10.6; 32 rows at 255 14.5 / 15.1, at 509 27.7 / 28.1; 28 rows at
+// 700 33.8 / 34.4; 32 at 2,000 97.8 / 95.3; 24 at 509 23.5 / 22.9; a prompt of 64 tokens 11.0 / 11.3, of 150 12.7 / 12.4, of 509 39.9 / 34.7.
+LRS_API int lrs_attention_f32_direct(int64_t workgroups, int together, int longest) {
+  const int units = lrs_compute_units() > 0 ? lrs_compute_units() : 256;
+  if (longest <= 0) return 0;
+  if (longest <= 2 * PIECE) return 1;
+  if (together > 1) return 0;
+  if (longest <= 4 * PIECE) return longest <= 3 * PIECE || 2 * workgroups >= units;
+  return longest < 1024 && 4 * workgroups > 3 * units && workgroups <= units;
 }
 
 // together: the most consecutive tokens that may share a workgroup (1: a step in which every request brings one token).
@@ -524,17 +551,18 @@ int lrs_attention_f32(float* out, int out_stride, const float* q, int q_stride, 
   // with nothing to do.  us of 64 tokens at 30 and at 100, eight waves before / now (the kernel for any shape): 32 heads of 128 on 32 58 / 17
   // (15) and 63 / 37 (36), 32 on 8 16 / 8 (12) and 18 / 16 (29), 16 heads of 64 on 16 21 / 7 (8) and 23 / 12 (17); one token at 10, 32 on 8 8.4 / 6.5 (5.3).
   const int64_t workgroups = (int64_t)((tokens + together - 1) / together) * nkv;
-  const bool few_pieces = longest > 0 && longest <= 4 * PIECE;
+  const bool few_pieces = longest > 0 && longest <= 4 * PIECE, direct = lrs_attention_f32_direct(workgroups, together, longest) != 0;
   const int items = together * heads * (d / 4);                            // what the merge has to do, one a thread
-#define CALL(D, WAVES, SHORT)                                                                                                                  \
-  launch<D, WAVES, SHORT>(out, out_stride, q, q_stride, k_pages, v_pages, block_table, table_stride, token_request, positions, tokens, heads, nkv, \
+#define CALL(D, WAVES, SHORT, DIRECT)                                                                                                          \
+  launch<D, WAVES, SHORT, DIRECT>(out, out_stride, q, q_stride, k_pages, v_pages, block_table, table_stride, token_request, positions, tokens, heads, nkv, \
                           page_size, scale, window, together, s)
 #define SIZE(D)                                                  \
   do {                                                           \
-    if (few_pieces && workgroups > 4 * lrs_compute_units() && items <= WAVE) CALL(D, 1, true);     \
-    else if (few_pieces && workgroups > lrs_compute_units() && items <= 2 * WAVE) CALL(D, 2, true); \
-    else if (longest > 0 && longest <= 32) CALL(D, 8, true);     \
-    else CALL(D, 8, false);                                      \
+    if (few_pieces && workgroups > 4 * lrs_compute_units() && items <= WAVE) CALL(D, 1, true, true);     \
+    else if (few_pieces && workgroups > lrs_compute_units() && items <= 2 * WAVE) CALL(D, 2, true, true); \
+    else if (longest > 0 && longest <= 32) CALL(D, 8, true, true);                                      \
+    else if (direct) CALL(D, 8, false, true);                                                           \
+    else CALL(D, 8, false, false);                                                                      \
   } while (0)
   if (d == 32) SIZE(32);
   else if (d == 64) SIZE(64);

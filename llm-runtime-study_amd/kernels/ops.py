@@ -133,6 +133,7 @@ _SIGNATURES = {
     "lrs_norm_begin_parts": (c_int, [c_int]),
     "lrs_attention": (c_int, [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                               c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_float, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_void_p]),
+    "lrs_attention_f32_direct": (c_int, [c_int64, c_int, c_int]),
     "lrs_attention_f32_divided": (c_int, [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                                           c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "lrs_qkv_norm_prep": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_float, c_void_p, c_void_p,
@@ -1110,6 +1111,12 @@ def attention(out: torch.Tensor, q: torch.Tensor, k_pages: torch.Tensor, v_pages
 def attention_shares(dtype: torch.dtype, nq: int, nkv: int, d: int, dv: int, page_size: int, plain: bool) -> bool:
     """Whether attention() lets tokens share a workgroup (`together`): float32, and `plain`: no kept positions, sinks, cap, gates or bias."""
     return dtype == torch.float32 and plain and d == dv and d in (32, 64, 96, 128) and nq // nkv <= 16 and page_size % 16 == 0
+
+
+def attention_f32_direct(workgroups: int, together: int, longest: int) -> bool:
+    """Whether attention() of float32 brings keys and values straight into registers rather than through LDS, for so many workgroups of up to
+    `together` tokens of a kv head over contexts of up to `longest` (see `lrs_attention_f32_direct`); the same bits either way."""
+    return bool(library().lrs_attention_f32_direct(workgroups, together, longest))
 
 
 def attention_f32_divided(out: torch.Tensor, q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, block_table: torch.Tensor,

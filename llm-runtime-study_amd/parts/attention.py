@@ -506,7 +506,8 @@ class GQAAttention(Part):
         """Attention by the kernels for any shape and dtype; where tokens can share a workgroup, the single tokens at the head of a
         mixed step (each of a request of its own) go in a launch of their own, so that a prompt's tokens behind them do."""
         singles = 0 if ctx.all_decode else ctx.single_rows
-        longest = ctx.max_k if length_class(ctx.max_k) == 0 else 0        # of short contexts, a class that a shape's steps share
+        reach = length_class(ctx.max_k)
+        longest = 2 * reach - 1 if reach else ctx.max_k                   # at most; of long contexts their class's, which a shape's steps share
         plain = gates is None and not self.keep_first and not more.get("softcap") and more.get("sinks") is None and more.get("distance") is None
         shares = ops.attention_shares(ctx.dtype, self.num_heads, cache.k_pages.shape[1], self.head_dim, self.value_dim, group.page_size, plain)
         alone = qkv.shape[0] if ctx.all_decode else singles               # rows of a request of their own

@@ -34,3 +34,25 @@ def test_launches(monkeypatch, form, launches):
     assert sum((c[1] for c in calls), []) == of.tolist()
     if launches == 2:
         assert [c[2] for c in calls] == [1, 16]
+
+
+def test_short_contexts_are_told_and_go_straight_into_registers(monkeypatch):
+    """A launch is told a bound of its contexts that all steps of a shape share; a piece or two of keys, and rows that nearly fill the chip over some
+    hundreds, come straight into registers, as every other launch did better through LDS."""
+    direct = ops.attention_f32_direct
+    for workgroups in (1, 8, 64, 200, 256, 2000):
+        assert direct(workgroups, 1, 100) and direct(workgroups, 16, 128) and direct(workgroups, 1, 192)
+        assert not direct(workgroups, 1, 0) and not direct(workgroups, 16, 129) and not direct(workgroups, 1, 2047)
+    if ops.compute_units() in (0, 256):
+        assert not direct(127, 1, 255) and direct(128, 1, 255) and direct(2000, 1, 256)
+        assert [direct(n, 1, 511) for n in (64, 192, 193, 256, 257, 512)] == [False, False, True, True, False, False] and direct(256, 1, 1023)
+    told = []
+    monkeypatch.setattr(ops, "attention", lambda *a, longest=0, **more: told.append(longest))
+    part = GQAAttention.__new__(GQAAttention)
+    part.num_heads, part.head_dim, part.value_dim, part.scale, part.reach, part.keep_first = 16, 96, 96, 0.125, 0, 0
+    of = torch.zeros(7, dtype=torch.int32)
+    cache = SimpleNamespace(k_pages=torch.zeros(1, 8, 16, 96), v_pages=torch.zeros(1, 8, 96, 16))
+    for max_k in (20, 255, 256, 300, 511, 512, 5000):
+        ctx = SimpleNamespace(all_decode=True, single_rows=0, dtype=torch.float32, memo={}, max_k=max_k, token_slot=of, positions=of)
+        part._attend(ctx, torch.zeros(7, 16 * 96), torch.zeros(7, 32 * 96), cache, SimpleNamespace(block_table=None, page_size=16))
+    assert told == [20, 255, 511, 511, 511, 1023, 8191]

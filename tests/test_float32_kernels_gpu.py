@@ -154,6 +154,30 @@ def test_float32_attention_over_short_contexts(ops, nq, nkv, d, batch, window):
         assert all(torch.equal(out, outs[0]) for out in outs[1:])
 
 
+@pytest.mark.parametrize("nq,nkv,d,page", [(4, 2, 128, 16), (8, 2, 64, 48), (3, 1, 96, 16), (16, 1, 32, 32)])
+@pytest.mark.parametrize("window", [0, 70])
+def test_float32_attention_of_keys_straight_into_registers(ops, nq, nkv, d, page, window):
+    """Keys and values through LDS and straight into registers: the same bits, infinities and NaN among the values, whichever the told length chooses."""
+    g = torch.Generator().manual_seed(nq + d)
+    for batch, most, together in ((5, 128, 1), (5, 190, 1), (5, 100, 3), (200, 250, 1), (240 // nkv, 900, 1)):
+        if not ops.attention_f32_direct(batch * nkv, together, most):
+            assert together == 1 and ops.compute_units() != 256
+            continue
+        per = -(-most // page)
+        pages = torch.randn(batch * per, nkv, page, d, generator=g), torch.randn(batch * per, nkv, d, page, generator=g)
+        for at, value in ((3, math.inf), (5, -math.inf), (7, math.nan)):
+            pages[1][:, :, at, at] = torch.where(torch.rand(batch * per, nkv, generator=g) < 0.03, value, 1.0)
+        pages = [p.cuda() for p in pages]
+        table = torch.randperm(batch * per, generator=g).to(torch.int32).view(batch, per).cuda()
+        q = torch.randn(batch, nq * d, generator=g).cuda()
+        of = (torch.arange(batch, dtype=torch.int32) // together).cuda()
+        at = torch.randint(0, most, (batch,), generator=g).to(torch.int32).cuda()
+        outs = [torch.empty(batch, nq * d, device="cuda") for _ in range(2)]
+        for out, longest in zip(outs, (0, most)):
+            ops.attention(out, q, *pages, table, of, at, nq, 1 / math.sqrt(d), window, together=together, longest=longest)
+        assert torch.equal(*(out.view(torch.int32) for out in outs))
+
+
 def test_float32_product_of_rows_far_apart(ops):
     """Rows whose distance, times the rows of a tile, does not fit 32 bits of bytes."""
     m, n, k, stride = 16, 40, 64, 72_000_000
