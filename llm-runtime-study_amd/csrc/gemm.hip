@@ -1788,7 +1788,7 @@ LRS_API int lrs_gemm(void* out, int mode, const void* a, const void* w, const vo
       else launch_skinny_m<false, false>(out, mode, ap, norm, wp, bp, m, n, k, lda, ldc, s, tune);
     } else if (aligned && k % WIDE_BK == 0 && n % 4 == 0 && ldc % 4 == 0 && (uintptr_t)out % 16 == 0 && !bias &&
                (int64_t)m * lda < (1ll << 31) && (int64_t)n * k < (1ll << 31)) {
-      const bool narrow = n <= NARROW_MAX && !swiglu && !lrs_gemm_lines_width(m, n, k) && !lrs_gemm_lines_splits(m, n, k);
+      const bool narrow = n <= NARROW_MAX && !swiglu && (k % 64 != 0 || !tiles_take_few_outputs(m, k));
       if (k % 64 == 0 && !narrow) {
         const TilesChoice choice = choose_tiles(m, n, k, split_sums_bytes());
         if (choice.splits > 1) {

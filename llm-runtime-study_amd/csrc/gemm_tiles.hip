@@ -120,17 +120,25 @@ constexpr TileShape TILES[] = {{256, 256, 1, 12.0f, 0.81f, 0.66f}, {256, 192, 1,
 // Sums of parts: a kernel more, or more work for the one that adds the residual, and every part's sums written and read once, most of it in the caches.
 constexpr float PARTS_FIXED = 2.f, PARTS_BYTES_A_US = 14e6f;
 
-// Few outputs stay undivided: a router's logits (gemm_bf16_narrow) keep the bits they have beside more weight rows.
-constexpr int UNDIVIDED = 128;
+bool tiles_take_few_outputs(int m, int k) { return (m > 4096 && k >= 512) || (m == 4096 && k >= 4096); }
+
+// More than the memory-side cache holds is streamed from memory, which longer walks do better.  16,384 rows of K 8,192 and 192 outputs: 256 x 192
+// in four parts 98 us, 128 x 128 whole 79; 256 outputs 100 and 87; 32,768 rows 168 and 141; of 8,192 rows (134 MB) 192 outputs in parts 45, whole 50.
+constexpr int64_t CACHED_BYTES = 256ll << 20;
 
 TilesChoice choose_tiles(int m, int n, int k, size_t sums_bytes) {
   const int units = lrs_compute_units() > 0 ? lrs_compute_units() : 256, steps = k / 64;
+  // Up to FEW_OUTPUTS have the same parts, those of so many, and none where some of them go to gemm_bf16_narrow: a router's logits keep the bits
+  // that they have beside more weight rows.
+  const bool few = n <= FEW_OUTPUTS;
+  if (few) n = FEW_OUTPUTS;
+  const bool whole = (few && !tiles_take_few_outputs(m, k)) || ((int64_t)m + n) * k * 2 >= CACHED_BYTES;
   TilesChoice best{0, 1, 0.f};
   for (int t = 0; t < (int)(sizeof(TILES) / sizeof(TILES[0])); ++t) {
     const TileShape& shape = TILES[t];
     if (k % (64 * shape.panels) != 0) continue;
     const int64_t tiles = (int64_t)((m + shape.bm - 1) / shape.bm) * ((n + shape.bn - 1) / shape.bn);
-    for (int parts = 1; parts <= (n <= UNDIVIDED ? 1 : 8); ++parts) {
+    for (int parts = 1; parts <= (whole ? 1 : 8); ++parts) {
       const int each = (steps / shape.panels + parts - 1) / parts * shape.panels;   // slices of the longest part
       const double sums = (double)parts * m * n * sizeof(float);
       // every part has work, and eight slices of it: shorter walks are mostly beginnings

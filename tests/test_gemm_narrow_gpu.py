@@ -7,7 +7,8 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("m,n,k", [(65, 4, 32), (17, 16, 256), (128, 64, 4096), (129, 12, 96), (100, 16, 64), (300, 20, 1056), (257, 36, 2016), (511, 64, 544), (2048, 32, 4096), (9000, 60, 160)])
+@pytest.mark.parametrize("m,n,k", [(65, 4, 32), (17, 16, 256), (128, 64, 4096), (129, 12, 96), (100, 16, 64), (300, 20, 1056), (257, 36, 2016), (511, 64, 544), (2048, 32, 4096), (9000, 60, 160),
+                                   (4095, 40, 512), (4096, 36, 4096), (4097, 8, 576), (5000, 64, 512), (6001, 4, 4096)])
 def test_few_outputs_of_many_rows(m, n, k):
     from llm_runtime_study_amd.kernels import ops
 
@@ -28,7 +29,8 @@ def test_few_outputs_of_many_rows(m, n, k):
     assert ((short.double() - want).abs() <= bound + 2.0 ** -8 * (want.abs() + bound)).all()
 
 
-@pytest.mark.parametrize("m,n,k", [(65, 4, 32), (70, 64, 224), (129, 12, 96), (100, 16, 64), (300, 20, 1056), (257, 36, 2016), (2048, 32, 4096), (2048, 64, 2048), (1000, 8, 544)])
+@pytest.mark.parametrize("m,n,k", [(65, 4, 32), (70, 64, 224), (129, 12, 96), (100, 16, 64), (300, 20, 1056), (257, 36, 2016), (2048, 32, 4096), (2048, 64, 2048), (1000, 8, 544),
+                                   (4095, 16, 4096), (4096, 16, 2048), (4096, 64, 4096), (4097, 4, 1024), (6000, 32, 8192), (5003, 8, 4160)])
 def test_few_outputs_have_the_bits_of_many(m, n, k):
     """A row's outputs are the same whether its weight rows stand alone or among more than one such kernel takes."""
     from llm_runtime_study_amd.kernels import ops

@@ -19,10 +19,17 @@ def test_the_choice_of_tile_and_parts():
                 assert k % (64 * panels) == 0 and 1 <= parts <= 8
                 if parts > 1:
                     each = -(-steps // parts)
-                    assert (parts - 1) * each < steps and each * panels >= 8 and parts * m * n * 4 <= room and n > 128
+                    assert (parts - 1) * each < steps and each * panels >= 8 and parts * m * n * 4 <= room
+                    assert n > 128 or m > 4096 or (m == 4096 and k >= 4096)
                 assert ops.gemm_tiles_choice(m, n, k, 0)[2] == 1
     if ops.compute_units() in (0, 256):
         assert ops.gemm_tiles_choice(2048, 24576, 4096) == (256, 256, 1) and ops.gemm_tiles_choice(512, 19456, 2560) == (256, 160, 1)
+        # few outputs: divided from 4,096 rows on, where a router's own kernel has more than a round of the chip, all up to 128 alike
+        assert ops.gemm_tiles_choice(4096, 64, 8192)[2] > 1 and ops.gemm_tiles_choice(8192, 8, 8192)[2] > 1 and ops.gemm_tiles_choice(4095, 64, 8192)[2] == 1
+        assert all(ops.gemm_tiles_choice(m, n, k) == ops.gemm_tiles_choice(m, 128, k) for m in (4096, 5000, 16384) for n in (8, 64, 100) for k in (512, 2048, 8192))
+        # what streams from memory is not divided
+        assert ops.gemm_tiles_choice(16384, 256, 8192) == (128, 128, 1) and ops.gemm_tiles_choice(32768, 192, 8192) == (128, 192, 1)
+        assert ops.gemm_tiles_choice(8192, 256, 8192)[2] > 1
         assert ops.gemm_tiles_choice(256, 1024, 1024) == (64, 64, 1) and ops.gemm_tiles_choice(512, 4096, 12288)[2] > 1
 
 
