@@ -1624,30 +1624,13 @@ LRS_API int lrs_gemm_mid_qk_prep(void* qkv, int row_stride, const void* a, const
                                v_pages, slots, page_size, split_sums_buffer(), splits, stream);
 }
 
-// The width of 256-token tiles, of 256, 192 or 128 weight rows, whose launch takes the fewest rounds of the chip times its width (the
-// wider of two that tie), or 0 unless K is a multiple of 64 and there is a tile of 256 x 128 for every compute unit.  Says which products
-// of few outputs have tiles enough not to go to gemm_bf16_narrow; the tile that is taken is choose_tiles' (gemm_tiles.hip).
-LRS_API int lrs_gemm_lines_width(int m, int n, int k) {
+// Whether a product of more than 128 rows goes to this package's tiles rather than to the vendor library whatever follows it: one of too few tiles of
+// 256 x 128 to go round the chip, which its K in up to eight parts of eight slices or more half fills, with a long K (the feed-forward's second
+// product: 14B at 512 rows 90 us against 174, 8B 61 against 86, norms included), or square and wide ones up to 256 rows in parts of 12
+// slices (14B q/k/v 39 against 52).  lrs_gemm_tiles_pay says more, by what follows; the tile and the parts are choose_tiles'.
+LRS_API int lrs_gemm_split_pays(int m, int n, int k) {
   const int units = lrs_compute_units() > 0 ? lrs_compute_units() : 256;
-  const int big_m = (m + 255) / 256;
-  if (m <= 0 || n <= 0 || k <= 0 || k % 64 != 0 || big_m * ((n + 127) / 128) < units) return 0;
-  int width = 0;
-  int64_t best = 0;
-  for (int candidate : {256, 192, 128}) {
-    const int across = (n + candidate - 1) / candidate;
-    const int64_t cost = (int64_t)((big_m * across + units - 1) / units) * candidate;
-    if (!width || cost < best) width = candidate, best = cost;
-  }
-  return width;
-}
-
-// Into how many parts K would be divided for a product with too few tiles of 256 x 128 to go round the compute units, or 0 if there are
-// enough of them, or too few even so: the number of parts, from 1 (just the tiles, if they fill half the units) to 8, that fills the
-// units best in one round, every part with 8 slices of 64 or more, and the parts' sums within the split buffer.  Says which products
-// lrs_gemm_lines_add_rmsnorm takes; the parts that are made are choose_tiles'.
-LRS_API int lrs_gemm_lines_splits(int m, int n, int k) {
-  const int units = lrs_compute_units() > 0 ? lrs_compute_units() : 256;
-  if (m <= 128 || n <= 0 || k <= 0 || k % 64 != 0) return 0;
+  if (m <= 128 || n <= 0 || k <= 0 || k % 64 != 0 || n % 4 != 0) return 0;
   const int tiles = ((m + 255) / 256) * ((n + 127) / 128), steps = k / 64;
   if (tiles >= units) return 0;
   int splits = 0;
@@ -1656,17 +1639,8 @@ LRS_API int lrs_gemm_lines_splits(int m, int n, int k) {
     if (parts > 1 && (each < 8 || (parts - 1) * each >= steps || (size_t)parts * m * n * sizeof(float) > SPLIT_SUMS_BYTES)) continue;
     splits = parts;
   }
-  return splits && 2 * tiles * splits >= units ? splits : 0;
-}
-
-// Whether such a product goes to this package's tiles rather than to the vendor library whatever follows it: a long K (the feed-forward's second
-// product: 14B at 512 rows 90 us against 174, 8B 61 against 86, norms included), square and wide ones up to 256 rows where every part would
-// have 12 slices (14B q/k/v 39 against 52).  lrs_gemm_tiles_pay says more, by what follows.
-LRS_API int lrs_gemm_lines_split_pays(int m, int n, int k) {
-  const int splits = lrs_gemm_lines_splits(m, n, k);
-  if (splits < 1 || n % 4 != 0) return 0;
-  if (k >= 2 * n) return 1;
-  return m <= 256 && splits >= 2 && (k / 64 + splits - 1) / splits >= 12;
+  if (splits == 0 || 2 * tiles * splits < units) return 0;
+  return k >= 2 * n || (m <= 256 && splits >= 2 && (steps + splits - 1) / splits >= 12);
 }
 
 // Whether the tiles of gemm_tiles.hip, with what follows the product in their epilogue or in the kernel that adds up their parts, are
@@ -1724,15 +1698,6 @@ LRS_API int lrs_gemm_tiles_add_rmsnorm(float* residual, const void* a, const voi
   launch_tiles(choice, sums, TILES_STORE_F32, (const bf16*)a, (const bf16*)w, m, n, k, lda, n, (hipStream_t)stream);
   if (int rc = lrs_check_launch("gemm_tiles_add_rmsnorm")) return rc;
   return lrs_split_add_rmsnorm(normed, normed_dtype, residual, sums, splits, norm_weight, norm_weight_dtype, m, n, eps, stream);
-}
-
-// The same for shapes that lrs_gemm_lines_splits takes, with room for one part's sums.
-LRS_API int lrs_gemm_lines_add_rmsnorm(float* residual, const void* a, const void* w, int m, int n, int k, int lda,
-                                       const void* norm_weight, int norm_weight_dtype, float eps, void* normed, int normed_dtype,
-                                       void* workspace, int64_t workspace_bytes, void* stream) {
-  LRS_REQUIRE(lrs_gemm_lines_splits(m, n, k) >= 1 && (size_t)m * n * sizeof(float) <= SPLIT_SUMS_BYTES,
-              "gemm_lines_add_rmsnorm: the divided product does not take m=%d n=%d k=%d (see lrs_gemm_lines_splits)", m, n, k);
-  return lrs_gemm_tiles_add_rmsnorm(residual, a, w, m, n, k, lda, norm_weight, norm_weight_dtype, eps, normed, normed_dtype, workspace, workspace_bytes, stream);
 }
 
 // out [M, N] (row stride ldc) = a [M, K] (row stride lda) times w[N, K]^T.

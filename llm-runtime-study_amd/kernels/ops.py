@@ -100,8 +100,6 @@ _SIGNATURES = {
                          c_int, c_float, c_int, c_int, c_void_p, c_int64, c_void_p]),
     "lrs_gemm_workspace_bytes": (c_int64, []),
     "lrs_gemm_f32_tile": (c_int, [c_int, c_int]),
-    "lrs_gemm_lines_add_rmsnorm": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_float, c_void_p, c_int,
-                                           c_void_p, c_int64, c_void_p]),
     "lrs_gemm_tiles_add_rmsnorm": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_float, c_void_p, c_int,
                                            c_void_p, c_int64, c_void_p]),
     "lrs_gemm_norm_chain": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
@@ -172,9 +170,7 @@ _SIGNATURES = {
                                     c_int, c_void_p]),
     "lrs_attention_prefill_prepares": (c_int, [c_int]),
     "lrs_compute_units": (c_int, []),
-    "lrs_gemm_lines_width": (c_int, [c_int, c_int, c_int]),
-    "lrs_gemm_lines_splits": (c_int, [c_int, c_int, c_int]),
-    "lrs_gemm_lines_split_pays": (c_int, [c_int, c_int, c_int]),
+    "lrs_gemm_split_pays": (c_int, [c_int, c_int, c_int]),
     "lrs_gemm_tiles_pay": (c_int, [c_int, c_int, c_int, c_int]),
     "lrs_gemm_tiles_choice": (c_int, [c_int, c_int, c_int, c_int64, c_void_p, c_void_p, c_void_p]),
     "lrs_attention_prefill_group": (c_int, []),
@@ -257,7 +253,7 @@ def library():
 # and _SIGNATURES by kernels/plan_codegen.py, is the other side (a test keeps the two in step).
 PLAN_OPS = ("lrs_activation", "lrs_add_gathered", "lrs_add_into", "lrs_add_rmsnorm", "lrs_advance_decode", "lrs_advance_slots", "lrs_attention", "lrs_attention_decode", "lrs_attention_f32_divided",
             "lrs_attention_mixed", "lrs_attention_prefill", "lrs_axpby", "lrs_choose_tokens", "lrs_choose_tokens_split", "lrs_copy_to_pinned", "lrs_delta_rule", "lrs_delta_rule_channels", "lrs_delta_rule_chunks", "lrs_embed", "lrs_fill_i32",
-            "lrs_filter_logits", "lrs_filter_logits_wide", "lrs_gated_clamped", "lrs_gated_norm_add", "lrs_gather_rows", "lrs_gemm", "lrs_gemm_f32_gated", "lrs_gemm_lines_add_rmsnorm", "lrs_gemm_mid_add_norm_begin", "lrs_gemm_mid_qk_prep", "lrs_gemm_mid_scaled",
+            "lrs_filter_logits", "lrs_filter_logits_wide", "lrs_gated_clamped", "lrs_gated_norm_add", "lrs_gather_rows", "lrs_gemm", "lrs_gemm_f32_gated", "lrs_gemm_mid_add_norm_begin", "lrs_gemm_mid_qk_prep", "lrs_gemm_mid_scaled",
             "lrs_gemm_norm_chain", "lrs_gemm_tiles_add_rmsnorm", "lrs_head_gemm", "lrs_latent_attention", "lrs_latent_attention_groups", "lrs_latent_prep", "lrs_layernorm", "lrs_library_gemm", "lrs_mlstm", "lrs_mlstm_chunks", "lrs_moe_align", "lrs_moe_combine", "lrs_moe_experts", "lrs_moe_route", "lrs_moe_route_align", "lrs_norm_add",
             "lrs_qk_prep", "lrs_qkv_norm_prep", "lrs_rmsnorm", "lrs_rope_table", "lrs_rotate_unit_prep", "lrs_round_rows", "lrs_scale_add_layernorm", "lrs_scale_rows", "lrs_scale_values", "lrs_sigmoid_gate", "lrs_silu_mul", "lrs_soft_cap", "lrs_ssm", "lrs_xielu")
 _PLAN_INDEX = {name: index for index, name in enumerate(PLAN_OPS)}
@@ -677,24 +673,10 @@ def add_into(residual: torch.Tensor, y: torch.Tensor) -> None:
 
 
 @functools.lru_cache(maxsize=4096)
-def gemm_lines_width(m: int, n: int, k: int) -> int:
-    """The width (256, 192 or 128 weight rows) of 256-token tiles that takes the fewest rounds of the chip for out [m, n] = x [m, k] w[n, k]^T,
-    or 0 if there is no tile of 256 x 128 for every compute unit (see `lrs_gemm_lines_width`)."""
-    return int(library().lrs_gemm_lines_width(m, n, k))
-
-
-@functools.lru_cache(maxsize=4096)
-def gemm_lines_splits(m: int, n: int, k: int) -> int:
-    """Into how many parts K would be divided for a product with too few tiles of 256 x 128 to go round the compute units (1: the
-    tiles as they are), or 0 if gemm_lines_add_rmsnorm() does not take the product (see `lrs_gemm_lines_splits`)."""
-    return int(library().lrs_gemm_lines_splits(m, n, k))
-
-
-@functools.lru_cache(maxsize=4096)
 def gemm_split_pays(m: int, n: int, k: int) -> bool:
     """Whether a bfloat16 product of more than 128 rows is faster by this package's many-rows kernel with K divided
-    between workgroups than by the vendor library (a rule from measurements, see `lrs_gemm_lines_split_pays`)."""
-    return bool(library().lrs_gemm_lines_split_pays(m, n, k))
+    between workgroups than by the vendor library (a rule from measurements, see `lrs_gemm_split_pays`)."""
+    return bool(library().lrs_gemm_split_pays(m, n, k))
 
 
 def gemm_tiles_choice(m: int, n: int, k: int, sums_bytes: int | None = None) -> tuple[int, int, int]:
@@ -932,29 +914,17 @@ def gemm_tiles_add_rmsnorm(residual: torch.Tensor, a: torch.Tensor, w: torch.Ten
     """residual (float32 [M, N]) += a @ w.T for more than 128 bf16 rows, K a multiple of 64, and normed [M, N] =
     RMSNorm(residual) with `norm_weight` and `eps`, in two kernels; where K is divided between workgroups, the one that adds
     up their sums also adds them to the residual stream and normalises the rows."""
-    _gemm_add_rmsnorm("gemm_tiles_add_rmsnorm", residual, a, w, norm_weight, eps, normed, workspace)
-
-
-def gemm_lines_add_rmsnorm(residual: torch.Tensor, a: torch.Tensor, w: torch.Tensor, norm_weight: torch.Tensor, eps: float,
-                           normed: torch.Tensor, workspace: torch.Tensor | None = None) -> None:
-    """gemm_tiles_add_rmsnorm() for the shapes that gemm_lines_splits() takes."""
-    m, k = a.shape
-    _need(m > 128 and gemm_lines_splits(m, w.shape[0], k) >= 1, "gemm_lines_add_rmsnorm: takes bf16 products of more than 128 rows that gemm_lines_splits() takes")
-    _gemm_add_rmsnorm("gemm_lines_add_rmsnorm", residual, a, w, norm_weight, eps, normed, workspace)
-
-
-def _gemm_add_rmsnorm(name: str, residual, a, w, norm_weight, eps, normed, workspace) -> None:
     m, k = a.shape
     n = w.shape[0]
     _need(a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.shape == (n, k) and w.is_contiguous() and m > 128 and k % 64 == 0,
-          f"{name}: takes bf16 products of more than 128 rows, K a multiple of 64")
-    _need(residual.dtype == torch.float32 and residual.is_contiguous() and residual.shape == (m, n), f"{name}: residual must be contiguous float32 [{m}, {n}]")
-    _need(normed.is_contiguous() and normed.shape == (m, n), f"{name}: normed must be contiguous [{m}, {n}]")
+          "gemm_tiles_add_rmsnorm: takes bf16 products of more than 128 rows, K a multiple of 64")
+    _need(residual.dtype == torch.float32 and residual.is_contiguous() and residual.shape == (m, n), f"gemm_tiles_add_rmsnorm: residual must be contiguous float32 [{m}, {n}]")
+    _need(normed.is_contiguous() and normed.shape == (m, n), f"gemm_tiles_add_rmsnorm: normed must be contiguous [{m}, {n}]")
     _need(norm_weight.is_contiguous() and norm_weight.numel() == n and eps > 0 and n % 4 == 0 and n <= 8192,
-          f"{name}: the norm weight must hold {n} values, eps be positive and N a multiple of 4 up to 8192")
-    _launch("lrs_" + name, _dev(residual, "residual"), _dev(a, "a"), _dev(w, "w"), m, n, k, _rows(a, "a"),
+          f"gemm_tiles_add_rmsnorm: the norm weight must hold {n} values, eps be positive and N a multiple of 4 up to 8192")
+    _launch("lrs_gemm_tiles_add_rmsnorm", _dev(residual, "residual"), _dev(a, "a"), _dev(w, "w"), m, n, k, _rows(a, "a"),
             _dev(norm_weight, "norm_weight"), dtype_code(norm_weight.dtype), eps, _dev(normed, "normed"), dtype_code(normed.dtype),
-            *_workspace(workspace, name), _stream())
+            *_workspace(workspace, "gemm_tiles_add_rmsnorm"), _stream())
 
 
 class LibraryState:

@@ -21,9 +21,9 @@ name of a route and `linear()` runs it.  The routes:
   fused_norm few rows of the float32 residual stream, normalised on the way in (gemm with norm_weight)
   mid_begin  17..128 rows adding into the residual stream and beginning the norm that follows
   mid        17..128 rows, nothing folded in (gemm picks the kernel for them)
-  split_norm more than 128 rows adding into the residual stream before an RMSNorm, of a shape whose K this package's
-             many-rows kernel divides between workgroups: the kernel that adds up their sums also adds the residual
-             and normalises the rows (gemm_lines_add_rmsnorm)
+  split_norm more than 128 rows adding into the residual stream before an RMSNorm, of few outputs and a long K, which this
+             package's tiles are faster at whatever follows (gemm_split_pays): the kernel that adds up the sums of a divided K
+             also adds the residual and normalises the rows (gemm_tiles_add_rmsnorm)
   library    more rows than these kernels are made for, if the step may use the vendor library: where they are faster with
              what follows, this package's tiles all the same (gemm_tiles_pay: gemm, gemm_tiles_add_rmsnorm), else the library,
              where the residual add (with the norm that follows) or the gated activation take one more small kernel
@@ -203,7 +203,7 @@ def linear(ctx, out, x, weight, bias=None, accumulate: bool = False, swiglu: boo
         return begun
     if route == "split_norm":
         normed = ctx.scratch("norm_after_add", (m, n), ctx.dtype)
-        ops.gemm_lines_add_rmsnorm(out, x, weight, following[0], following[1], normed, workspace=workspace_of(ctx))
+        ops.gemm_tiles_add_rmsnorm(out, x, weight, following[0], following[1], normed, workspace=workspace_of(ctx))
         return normed
     if route == "library":
         fused = following is not None and out.is_contiguous()

@@ -212,33 +212,27 @@ def test_a_plan_packs_one_word_per_argument():
     assert words[13:] == [ops.PLAN_OPS.index("lrs_fill_i32"), 0, (1 << 64) - 7, 12]               # None: a null pointer; -7: two's complement
 
 
-def test_the_tile_width_of_the_many_rows_kernel_follows_the_rounds_of_the_chip():
-    """`lrs_gemm_lines_width`: K a multiple of 64 and a 256 x 128 tile for every compute unit, then the width
-    that needs the fewest rounds times its width (the shapes of the 8B layer at 2,048 rows: one round each)."""
+def test_the_tile_of_the_many_rows_kernel_follows_the_rounds_of_the_chip():
+    """`choose_tiles`: the tile and the parts of K that are expected to take least, and the products that go to such tiles rather than to the
+    vendor library whatever follows them (the shapes of the 8B and 14B layers among them)."""
     from llm_runtime_study_amd.kernels import ops
 
     if ops.compute_units() not in (0, 256):
         return
-    assert ops.gemm_lines_width(2048, 24576, 4096) == 256      # 768 tiles: three rounds
-    assert ops.gemm_lines_width(2048, 6144, 4096) == 192       # 256 tiles of 192: one round
-    assert ops.gemm_lines_width(2048, 4096, 12288) == 128      # 256 tiles of 128
-    assert ops.gemm_lines_width(8192, 4096, 4096) == 256       # 512 tiles: two rounds of 256 tie with four of 128
-    assert ops.gemm_lines_width(1024, 4096, 4096) == 0         # not a tile for every compute unit
-    assert ops.gemm_lines_width(2048, 4096, 4000) == 0         # K no multiple of 64
-    assert ops.gemm_lines_width(129, 151936, 4096) == 128      # the LM head of a small step: five rounds of 128 against three of 256
-    # too few tiles for the chip: K in as many parts as fill it in one round, each with 8 slices of 64 or more
-    assert ops.gemm_lines_splits(512, 4096, 4096) == 4         # 64 tiles x 4
-    assert ops.gemm_lines_splits(512, 5120, 17408) == 3        # 80 tiles x 3 = 240
-    assert ops.gemm_lines_splits(512, 7168, 5120) == 2         # 112 tiles x 2
-    assert ops.gemm_lines_splits(300, 9000, 1088) == 1         # 142 tiles, more than half the units: as they are
-    assert ops.gemm_lines_splits(512, 4096, 512) == 0          # one part of 8 slices, 64 tiles: under half the units
-    assert ops.gemm_lines_splits(2048, 4096, 4096) == 0        # a tile for every unit: not divided
-    assert ops.gemm_lines_splits(128, 4096, 4096) == 0         # the kernel for 17..128 rows' size
-    # ... and where that form is taken instead of the vendor library: a long K at any such row count, others up to 256 rows
+    assert ops.gemm_tiles_choice(2048, 24576, 4096) == (256, 256, 1)       # 768 tiles: three rounds
+    assert ops.gemm_tiles_choice(2048, 6144, 4096) == (256, 192, 1)        # 256 tiles of 192: one round
+    assert ops.gemm_tiles_choice(2048, 4096, 12288) == (256, 256, 2)       # 128 tiles, a long K in two parts
+    assert ops.gemm_tiles_choice(8192, 4096, 4096) == (256, 256, 1)        # 512 tiles: two rounds
+    assert ops.gemm_tiles_choice(2048, 4096, 4096) == (256, 128, 1)        # a tile for every unit: not divided
+    assert ops.gemm_tiles_choice(512, 5120, 17408) == (256, 160, 4)        # 64 tiles x 4
+    assert ops.gemm_tiles_choice(512, 7168, 5120) == (256, 128, 2)         # 112 tiles x 2
+    assert ops.gemm_tiles_choice(512, 4096, 512)[2] == 1                   # eight slices: not divided
+    # a long K at any row count that leaves the chip idle, others up to 256 rows
     assert ops.gemm_split_pays(512, 5120, 17408) and ops.gemm_split_pays(1024, 4096, 12288) and ops.gemm_split_pays(300, 4096, 12288)
     assert ops.gemm_split_pays(256, 5120, 5120) and not ops.gemm_split_pays(512, 5120, 5120)
     assert not ops.gemm_split_pays(256, 4096, 4096)            # 8 parts of 8 slices: too short
     assert not ops.gemm_split_pays(2048, 4096, 12288) and not ops.gemm_split_pays(512, 34816, 5120)
+    assert not ops.gemm_split_pays(128, 4096, 12288) and not ops.gemm_split_pays(512, 4096, 12000) and not ops.gemm_split_pays(512, 4098, 12288)
 
 
 def test_a_recording_of_launches_belongs_to_its_thread():

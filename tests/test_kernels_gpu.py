@@ -370,8 +370,6 @@ def test_product_of_many_rows_with_residual_add_and_norm_in_its_finishing_kernel
     """residual += a w^T and the RMSNorm of the result in two kernels (K divided between workgroups or the tiles as
     they are; the kernel that adds up the sums adds the residual and normalises), with the caller's own workspace and
     with the one the process keeps: the same bits, and both as the plain computation."""
-    if ops.gemm_lines_splits(m, n, k) < 1:
-        pytest.skip("the divided product does not take this shape on this device")
     g = torch.Generator().manual_seed(m + n + k)
     a = torch.randn(m, k, generator=g).bfloat16()
     w = (torch.randn(n, k, generator=g) / math.sqrt(k)).bfloat16()
@@ -385,7 +383,7 @@ def test_product_of_many_rows_with_residual_add_and_norm_in_its_finishing_kernel
         residual = dev(res.clone())
         normed = torch.empty(m, n, device="cuda", dtype=torch.bfloat16)
         space = torch.empty(ops.gemm_workspace_bytes() // 4, device="cuda") if own else None
-        ops.gemm_lines_add_rmsnorm(residual, dev(a), dev(w), dev(nw), eps, normed, workspace=space)
+        ops.gemm_tiles_add_rmsnorm(residual, dev(a), dev(w), dev(nw), eps, normed, workspace=space)
         torch.testing.assert_close(residual.cpu().double(), want_res, rtol=1e-4, atol=1e-4)
         close_in_norm(normed, want, rel=5e-3)
         outs.append((residual.cpu(), normed.cpu()))

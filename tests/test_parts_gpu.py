@@ -122,15 +122,15 @@ def test_swiglu_part_adds_into_the_residual(dtype):
 
 
 def test_swiglu_part_of_a_prompt_portion_divides_the_long_k_of_its_second_product():
-    """300 rows, 1,024 wide, 4,096 between: the second product has 16 tiles of 256 x 128 for 256 compute units and a
-    K four times its width, so it goes to this package's kernel with K in 8 parts (the first one to the library)."""
+    """300 rows, 1,024 wide, 4,096 between: the second product has 80 tiles of 64 x 64 for 256 compute units and a
+    K four times its width, so it goes to this package's kernel with K in 3 parts."""
     from llm_runtime_study_amd.kernels import ops
     from llm_runtime_study_amd.parts import PartSpec, create
     from llm_runtime_study_amd.parts.linear import plan
 
     hidden, inter, rows = 1024, 4096, 300
     if ops.compute_units() == 256:
-        assert ops.gemm_lines_splits(rows, hidden, inter) == 8
+        assert ops.gemm_split_pays(rows, hidden, inter) and ops.gemm_tiles_choice(rows, hidden, inter) == (64, 64, 3)
         assert plan(rows, hidden, inter, weight_dtype=torch.bfloat16, run_dtype=torch.bfloat16, out_dtype=torch.float32,
                     arrives="tensor", accumulate=True)[0] == "own"
     part = create("feed_forward", PartSpec("swiglu", {"hidden_size": hidden, "intermediate_size": inter}))
