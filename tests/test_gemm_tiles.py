@@ -50,8 +50,30 @@ def test_tiles_keep_their_values_in_registers(tmp_path):
     assert len(found) == 9 and not any(found.values()), found
 
 
+# every tile, whole and with K in parts, the last of them shorter than the others, with rows and columns that end inside a tile
+EDGES = {(256, 256, 1): (263, 24792, 512), (256, 256, 7): (142, 8400, 9344), (256, 192, 1): (258, 22072, 512), (256, 192, 5): (140, 8664, 5696),
+         (256, 160, 1): (388, 16444, 512), (256, 160, 3): (138, 12348, 2240), (256, 128, 1): (130, 24800, 512), (256, 128, 4): (143, 8080, 1856),
+         (128, 256, 1): (265, 17672, 512), (128, 256, 4): (65, 16376, 2112), (128, 192, 1): (67, 532, 576), (128, 192, 2): (92, 240, 960),
+         (128, 128, 1): (65, 17400, 512), (128, 128, 5): (71, 5636, 3072), (64, 128, 1): (70, 8268, 512), (64, 128, 5): (72, 3036, 2432),
+         (64, 64, 1): (122, 144, 640), (64, 64, 4): (86, 136, 1664)}
+
+
+def test_the_edges_are_of_every_tile():
+    """What the cases below reach follows from the table of costs: one that is fitted anew has to bring cases that reach every tile again."""
+    from llm_runtime_study_amd.kernels import ops
+
+    if ops.compute_units() not in (0, 256):
+        pytest.skip("another number of compute units makes other choices")
+    for (bm, bn, parts), (m, n, k) in EDGES.items():
+        assert ops.gemm_tiles_choice(m, n, k) == (bm, bn, parts) and m % bm and n % bn and n > 128
+        if parts > 1:
+            steps = k // (128 if (bm, bn) in ((128, 128), (64, 128), (64, 64)) else 64)
+            assert steps % -(-steps // parts)
+    assert {tile[:2] for tile in EDGES} == {tile[:2] for tile in EDGES if tile[2] == 1} == {tile[:2] for tile in EDGES if tile[2] > 1} and len(EDGES) == 18
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n,k", [
+@pytest.mark.parametrize("m,n,k", [*EDGES.values(),
     (2047, 24560, 128), (2048, 24576, 64), (1500, 12276, 192), (512, 19452, 320), (257, 19456, 640), (1030, 6148, 1024), (2048, 4096, 128), (1537, 4092, 576),
     (385, 12288, 192), (300, 9000, 1088), (129, 12300, 448), (1020, 4100, 256), (700, 2052, 384), (129, 68, 64), (65, 4096, 128), (191, 1028, 512), (129, 132, 1024),
     (1020, 12272, 320), (512, 4096, 4096), (300, 1024, 3072), (145, 2560, 9728), (1024, 2560, 2816)])
