@@ -56,3 +56,45 @@ def test_short_contexts_are_told_and_go_straight_into_registers(monkeypatch):
         ctx = SimpleNamespace(all_decode=True, single_rows=0, dtype=torch.float32, memo={}, max_k=max_k, token_slot=of, positions=of)
         part._attend(ctx, torch.zeros(7, 16 * 96), torch.zeros(7, 32 * 96), cache, SimpleNamespace(block_table=None, page_size=16))
     assert told == [20, 255, 511, 511, 511, 1023, 8191]
+
+
+@pytest.mark.parametrize("decode", [True, False])
+@pytest.mark.parametrize("span,reach", [(None, 0), (300, 300), (450, -450), (1000, 1000)])
+@pytest.mark.parametrize("max_k", [256, 300, 2000, 9000])
+def test_rows_of_their_own_are_divided(monkeypatch, decode, span, reach, max_k):
+    """Long float32 rows of a request each go to the divided form, a mixed step's other tokens to attention(), every row once, with places for
+    every piece that a row can see; where the places would take too much, everything goes to attention()."""
+    monkeypatch.setattr(ops, "compute_units", lambda: 256)
+    divided, whole = [], []
+    monkeypatch.setattr(ops, "attention_f32_divided", lambda out, q, k, v, table, of, at, nq, scale, window, splits, slots, o, ml: divided.append((of.tolist()[:out.shape[0]], window, splits, slots, o.numel(), ml.numel())))
+    monkeypatch.setattr(ops, "attention", lambda out, q, k, v, table, of, at, nq, scale, window, *a, together=1, **more: whole.append((of.tolist()[:out.shape[0]], window, together)))
+    part = GQAAttention.__new__(GQAAttention)
+    part.num_heads, part.head_dim, part.value_dim, part.scale, part.reach, part.keep_first, part.span = 4, 64, 64, 0.125, reach, 0, span
+    of = torch.tensor([3, 1, 2, 0, 0, 0, 0], dtype=torch.int32)
+    bound = -(-max_k // 256) * 256
+    ctx = SimpleNamespace(all_decode=decode, single_rows=0 if decode else 3, dtype=torch.float32, memo={}, max_k=max_k, max_k_bound=bound, token_slot=of, positions=of,
+                          scratch=lambda name, shape, dtype: torch.empty(shape, dtype=dtype))
+    cache = SimpleNamespace(k_pages=torch.zeros(1, 2, 16, 64), v_pages=torch.zeros(1, 2, 64, 16))
+    out, qkv, alone = torch.zeros(7, 4 * 64), torch.zeros(7, 8 * 64), 7 if decode else 3
+
+    def step():
+        divided.clear(), whole.clear()
+        part._attend(ctx, out, qkv, cache, SimpleNamespace(block_table=None, page_size=16))
+
+    step()
+    (rows, window, splits, slots, sums, maxima), = divided
+    assert rows == of.tolist()[:alone] and window == reach and splits > 1 and (sums, maxima) == (alone * 4 * slots * 64, alone * 4 * slots * 2)
+    assert whole == ([] if decode else [(of.tolist()[3:], reach, 16)])
+    for pos in range(bound):
+        first = 0 if not reach else max(pos - reach + 1, 0) if reach > 0 else pos - pos % -reach
+        assert pos // 64 - first // 64 + 1 <= slots
+    part.PIECE_RESULTS = alone * 4 * slots * (64 + 2) - 1
+    step()
+    assert not divided and whole == ([(of.tolist(), reach, 1)] if decode else [(of.tolist()[:3], reach, 1), (of.tolist()[3:], reach, 16)])
+    part.PIECE_RESULTS += 1
+    for heads, d in ((10, 64), (4, 96)):                   # more than four heads a kv head; heads of another size
+        part.num_heads, part.head_dim, part.value_dim = heads, d, d
+        cache = SimpleNamespace(k_pages=torch.zeros(1, 2, 16, d), v_pages=torch.zeros(1, 2, d, 16))
+        out, qkv = torch.zeros(7, heads * d), torch.zeros(7, (heads + 4) * d)
+        step()
+        assert not divided and sum((rows for rows, *_ in whole), []) == of.tolist()

@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from llm_runtime_study_amd.parts.attention import GQAAttention
+from llm_runtime_study_amd.parts.base import length_class
 
 
 @pytest.fixture(scope="module")
@@ -22,6 +23,19 @@ def ops():
 POSITIONS = [0, 63, 64, 511, 512, 700, 1100]
 
 
+def odd_values(shape, share, generator):
+    """Values of which a `share` each are infinities of either sign and NaN."""
+    values, kind = torch.randn(shape, generator=generator), torch.rand(shape, generator=generator)
+    for value, low in ((math.inf, 0.0), (-math.inf, share), (math.nan, 2 * share)):
+        values[(kind >= low) & (kind < low + share)] = value
+    return values
+
+
+def same(a, b):
+    """The same bits, or NaN in both."""
+    return bool(((a.view(torch.int32) == b.view(torch.int32)) | (a.isnan() & b.isnan())).all())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("nq,nkv,d,page", [(4, 2, 128, 16), (8, 2, 64, 32), (3, 1, 128, 48), (2, 2, 64, 16)])
 @pytest.mark.parametrize("window", [0, 130, -200])
@@ -30,7 +44,10 @@ def test_bits(ops, nq, nkv, d, page, window, splits):
     g = torch.Generator().manual_seed(nq + d)
     n, per = len(POSITIONS), -(-(max(POSITIONS) + 1) // page)
     pages = torch.randn(n * per, nkv, page, d, generator=g), torch.randn(n * per, nkv, d, page, generator=g)
+    # seen and unseen positions among them; the other dims stay finite
     pages[1][:, :, 3, 5] = torch.where(torch.rand(n * per, nkv, generator=g) < 0.1, math.inf, 1.0)
+    pages[1][:, :, 7:d - 1:11] = odd_values(pages[1][:, :, 7:d - 1:11].shape, 0.0005, g)
+    pages[1][:, :, d - 1] = odd_values(pages[1][:, :, d - 1].shape, 0.01, g)
     pages = [p.cuda() for p in pages]
     table = torch.randperm(n * per, generator=g).to(torch.int32).view(n, per).cuda()
     q = torch.randn(n, (nq + 2 * nkv) * d, generator=g).cuda()
@@ -40,17 +57,40 @@ def test_bits(ops, nq, nkv, d, page, window, splits):
     for slots in (18, 40):
         out, part_o, part_ml = torch.empty_like(want), torch.full((n * nq * slots, d), math.nan, device="cuda"), torch.full((n * nq * slots, 2), math.nan, device="cuda")
         ops.attention_f32_divided(out, q, *pages, table, of, at, nq, 1 / math.sqrt(d), window, splits, slots, part_o, part_ml)
-        assert torch.equal(out.view(torch.int32), want.view(torch.int32))
+        assert same(out, want)
+    assert want.isnan().any() and (want == math.inf).any() and (want == -math.inf).any() and want[:, 4:7].isfinite().all()
     with pytest.raises(Exception, match="too small"):
         ops.attention_f32_divided(out, q, *pages, table, of, at, nq, 1 / math.sqrt(d), window, splits, 41, part_o, part_ml)
 
 
+# contexts of some hundred pieces; a window that begins inside a piece
+@pytest.mark.gpu
+@pytest.mark.parametrize("nq,nkv,d,page", [(2, 1, 128, 16), (4, 1, 64, 64)])
+@pytest.mark.parametrize("window", [0, 5000])
+def test_bits_over_long_contexts(ops, nq, nkv, d, page, window):
+    g = torch.Generator().manual_seed(nq + d)
+    positions = [4095, 9000, 4096, 8191]
+    n, per = len(positions), -(-(max(positions) + 1) // page)
+    pages = [torch.randn(shape, generator=g).cuda() for shape in ((n * per, nkv, page, d), (n * per, nkv, d, page))]
+    table = torch.randperm(n * per, generator=g).to(torch.int32).view(n, per).cuda()
+    q = torch.randn(n, nq * d, generator=g).cuda()
+    of, at = torch.arange(n, dtype=torch.int32).cuda(), torch.tensor(positions, dtype=torch.int32).cuda()
+    want = torch.empty(n, nq * d, device="cuda")
+    ops.attention(want, q, *pages, table, of, at, nq, 1 / math.sqrt(d), window)
+    slots = max(positions) // 64 + 1
+    part_o, part_ml = torch.full((n * nq * slots, d), math.nan, device="cuda"), torch.full((n * nq * slots, 2), math.nan, device="cuda")
+    for splits in (16, 100, 200):
+        out = torch.empty_like(want)
+        ops.attention_f32_divided(out, q, *pages, table, of, at, nq, 1 / math.sqrt(d), window, splits, slots, part_o, part_ml)
+        assert torch.equal(out.view(torch.int32), want.view(torch.int32))
+
+
 def test_rule(monkeypatch):
-    """No division of short contexts or of steps that fill the chip; never more parts than pieces."""
+    """No division of short contexts or of steps that fill the chip; never more parts than the longest row of a class of lengths has pieces."""
     from llm_runtime_study_amd.kernels import ops
 
     monkeypatch.setattr(ops, "compute_units", lambda: 256)
     for workgroups in (1, 8, 64, 96, 128, 129, 512):
         for longest in (1, 255, 256, 511, 512, 2000, 40000):
             splits = GQAAttention._piece_splits(workgroups, longest)
-            assert splits >= 1 and (splits == 1 or (longest >= 256 and workgroups <= 128 and splits * 32 <= longest))
+            assert splits >= 1 and (splits == 1 or (longest >= 256 and workgroups <= 128 and splits <= 2 * length_class(longest) // 64))
