@@ -375,7 +375,7 @@ def main() -> int:
             "max_seq_len": max_seq_len, "num_pages": engine.cache_manager.groups[0].pool.num_pages, "page_size": engine.page_size,
             "prefill_tokens": args.prefill_tokens,
             "decode_steps_per_graph_launch": args.decode_steps_per_launch if engine.runner.use_graph else 0,
-            "prefill_gemm": "own" if args.own_gemm else "hipBLASLt", "parallelism": "single GPU",
+            "prefill_gemm": "own" if args.own_gemm else "own and hipBLASLt, by size", "parallelism": "single GPU",
             "sampling": "greedy" if sampling is None else f"temperature {args.temperature} top_k {args.top_k} top_p {args.top_p}",
         },
         "prefill": prefill,

@@ -352,8 +352,8 @@ __global__ __launch_bounds__(256, 2) void delta_pack_kernel(const float* __restr
 // new S go through LDS, a barrier each; half of O's products stand before either barrier, with the old S still in registers.  A
 // chunk's operands (a wave's rows of the packs, 1,024 bytes a load) are asked for a chunk ahead, into a second set of registers: with
 // one wave a SIMD there are enough.  96 matrix instructions a wave and chunk, 3,072 cycles: 47 us for
-// 32 chunks, 95 by itself and 105 inside a prompt: 71 without the loads (96 KB a chunk and compute unit, 44 bytes a nanosecond is the most that any kernel here
-// has been seen to get), the rest the two barriers with a trip through LDS each.  Left to itself the compiler moves the loads to where
+// 32 chunks, 95 by itself and 105 inside a prompt: 71 without the loads (96 KB a chunk and compute unit, 44 bytes a nanosecond; fetches into LDS that the L2s
+// answer bring a unit 86-100 in gemm_tiles.hip, which has not been tried here), the rest the two barriers with a trip through LDS each.  Left to itself the compiler moves the loads to where
 // their registers are cheapest: 106 us.
 template <int DP>
 __global__ __launch_bounds__(256, 1) void delta_walk_kernel(const float* __restrict__ packs, const int* __restrict__ cu,

@@ -3,8 +3,8 @@
 // The float32 matrix instruction multiplies and adds float32 values as fused multiply-adds in ascending k, subnormal
 // numbers included: 16x16x4 gives, bit for bit, the chain of fmaf that a thread would make (checked over normal products,
 // subnormal products and subnormal inputs).  K is divided into F32_PARTS runs of whole 128s (f32_part, common.h), a chain each from
-// zero, whose sums are added first to last: four short chains at once where rows are few, and an error a quarter of one
-// chain's.  So every output here is the same sum whatever kernel, tile or number of rows made it, and equals the tiled
+// zero, whose sums are added first to last: four short chains at once where rows are few, and a bound of the
+// error that is a quarter of one chain's (measured, K up to 3,072: farthest from 64 bits 4.9e-6 for 5.7e-6).  So every output here is the same sum whatever kernel, tile or number of rows made it, and equals the tiled
 // kernel's in gemm.hip, which serves what this file does not take (K no multiple of 32, rows not 16-byte aligned): a row's result
 // does not depend on what else is in the batch.
 #include "common.h"

@@ -23,7 +23,7 @@ __device__ __forceinline__ float silu_of(float v) { return v / (1.f + __expf(-v)
 template <int WM, int JT, int IT, int PANELS, int HALVES, int STAGES>
 __global__ __launch_bounds__(512, 1) void gemm_bf16_tiles_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, int m, int n, int k, int lda,
                                                                  int tiles_m, int tiles_n, int splits, int chunk, void* __restrict__ out, int form, int ldc) {
-  constexpr int WN = 8 / WM, BM = WM * JT * 16, BN = WN * IT * 16, BK = 64 * PANELS, JH = JT / HALVES, STEPS = 2 * PANELS;
+  constexpr int WN = 8 / WM, BM = WM * JT * 16, BN = WN * IT * 16, BK = 64 * PANELS;
   constexpr int X_BLOCKS = BM / 8 / HALVES, W_BLOCKS = BN / 8;   // blocks of 8 rows of a panel: of a part of the tokens, of the weights
   static_assert(X_BLOCKS * PANELS % 8 == 0 && JT % HALVES == 0, "a part of the tokens is dealt evenly to eight waves");
   constexpr int NX = X_BLOCKS * PANELS / 8, NW = W_BLOCKS * PANELS / 8, REST = W_BLOCKS * PANELS % 8;   // fetches a wave; REST: one more of the weights for the first waves

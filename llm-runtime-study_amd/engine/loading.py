@@ -60,7 +60,7 @@ def resolve_dtype(requested="auto") -> torch.dtype:
 # weights, the cache pool and the step's buffers out of it.  Nothing depends on that happening: an allocator that
 # works otherwise (caching switched off, expandable segments) leaves the engine as it was without this.
 RESERVE_AT_LEAST = 1 << 30        # smaller engines are a few mappings anyway
-RESERVE_MARGIN = 3 << 29          # the step's buffers (activations, logits, metadata, a delta layer's packs) beside weights and cache
+RESERVE_MARGIN = 3 << 29          # the step's buffers (activations, logits, metadata, a delta layer's packs, up to 256 MB of divided float32 attention's parts) beside weights and cache
 
 
 def engine_bytes(model: DecoderModel, dtype: torch.dtype, page_size: int, num_pages: int) -> int:
