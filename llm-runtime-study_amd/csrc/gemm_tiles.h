@@ -12,6 +12,7 @@ enum { TILES_STORE = 0, TILES_STORE_F32 = 1, TILES_ADD_F32 = 2, TILES_GATED = 3 
 struct TilesChoice {
   int tile, splits;
   float us;                                                       // what it is expected to take, the kernel that adds up the parts included
+  float useful;                                                   // of what the chip makes in the rounds of such a launch, the product's own outputs
 };
 // Products of up to 64 outputs that tiles take rather than gemm_bf16_narrow, whose workgroups of 16 rows and all outputs are one round of the chip up
 // to 4,096 rows.  us, narrow / tiles: K 4,096 8 outputs 4,096 rows 11.4 / 13.3, 8,192 19.7 / 17.7; 32 outputs 4,096 rows 17.3 / 13.9, 64 24.4 / 14.1; K 2,048

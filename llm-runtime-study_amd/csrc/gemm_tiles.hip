@@ -122,35 +122,50 @@ constexpr float PARTS_FIXED = 2.f, PARTS_BYTES_A_US = 14e6f;
 
 bool tiles_take_few_outputs(int m, int k) { return (m > 4096 && k >= 512) || (m == 4096 && k >= 4096); }
 
-// More than the memory-side cache holds is streamed from memory, which longer walks do better.  16,384 rows of K 8,192 and 192 outputs: 256 x 192
-// in four parts 98 us, 128 x 128 whole 79; 256 outputs 100 and 87; 32,768 rows 168 and 141; of 8,192 rows (134 MB) 192 outputs in parts 45, whole 50.
+// Few outputs (up to STREAM_OUTPUTS) of rows that the memory-side cache does not hold are a matter of reading those rows.  Parts that begin a multiple of 4 KB
+// into a row read them more slowly (K 8,192, 16,384 rows of 192 and 256 outputs in four parts of 4 KB 97 and 108 us, whole 76 and 87; 32,768 rows in two of 8 KB
+// 167 and 180, whole 146 and 170), and parts that promise less than a tenth are no faster (28,000 rows of K 5,120, 128 outputs in two 80, whole 70).  Others
+// are: 17,000 rows of K 8,192 in three parts 85 and 98, whole 97 and 117; 5,000 of K 28,672 in six 86 and 97, whole 133 and 182; 8 outputs 52, whole 108.
 constexpr int64_t CACHED_BYTES = 256ll << 20;
+constexpr int STREAM_OUTPUTS = 256, SLOW_APART = 32;               // SLOW_APART: slices
+constexpr float STREAM_GAIN = 1.1f;
 
 TilesChoice choose_tiles(int m, int n, int k, size_t sums_bytes) {
   const int units = lrs_compute_units() > 0 ? lrs_compute_units() : 256, steps = k / 64;
   // Up to FEW_OUTPUTS have the same parts, those of so many, and none where some of them go to gemm_bf16_narrow: a router's logits keep the bits
   // that they have beside more weight rows.
   const bool few = n <= FEW_OUTPUTS;
-  if (few) n = FEW_OUTPUTS;
-  const bool whole = (few && !tiles_take_few_outputs(m, k)) || ((int64_t)m + n) * k * 2 >= CACHED_BYTES;
-  TilesChoice best{0, 1, 0.f};
-  for (int t = 0; t < (int)(sizeof(TILES) / sizeof(TILES[0])); ++t) {
-    const TileShape& shape = TILES[t];
-    if (k % (64 * shape.panels) != 0) continue;
-    const int64_t tiles = (int64_t)((m + shape.bm - 1) / shape.bm) * ((n + shape.bn - 1) / shape.bn);
-    for (int parts = 1; parts <= (whole ? 1 : 8); ++parts) {
-      const int each = (steps / shape.panels + parts - 1) / parts * shape.panels;   // slices of the longest part
-      const double sums = (double)parts * m * n * sizeof(float);
-      // every part has work, and eight slices of it: shorter walks are mostly beginnings
-      if (parts > 1 && (each < 8 || (parts - 1) * each >= steps || sums > (double)sums_bytes || tiles * parts > units)) continue;
-      const int64_t rounds = (tiles * parts + units - 1) / units;
-      const float share = (float)(tiles * parts) / (float)(rounds * units);
-      float us = (float)rounds * (shape.fixed + (float)each * (shape.slice + shape.crowd * share));
-      if (parts > 1) us += PARTS_FIXED + 2.f * (float)sums / PARTS_BYTES_A_US;
-      if (best.us == 0.f || us < best.us) best = TilesChoice{t, parts, us};
+  const bool whole = few && !tiles_take_few_outputs(m, k), streams = n <= STREAM_OUTPUTS && (int64_t)m * k * 2 >= CACHED_BYTES;
+  // the least for n outputs with 1 to `most` parts
+  auto least = [&](int n, int most) {
+    TilesChoice best{0, 1, 0.f};
+    for (int t = 0; t < (int)(sizeof(TILES) / sizeof(TILES[0])); ++t) {
+      const TileShape& shape = TILES[t];
+      if (k % (64 * shape.panels) != 0) continue;
+      const int64_t tiles = (int64_t)((m + shape.bm - 1) / shape.bm) * ((n + shape.bn - 1) / shape.bn);
+      for (int parts = 1; parts <= most; ++parts) {
+        const int each = (steps / shape.panels + parts - 1) / parts * shape.panels;   // slices of the longest part
+        const double sums = (double)parts * m * n * sizeof(float);
+        // every part has work, and eight slices of it: shorter walks are mostly beginnings
+        if (parts > 1 && (each < 8 || (parts - 1) * each >= steps || sums > (double)sums_bytes || tiles * parts > units || (streams && each % SLOW_APART == 0))) continue;
+        const int64_t rounds = (tiles * parts + units - 1) / units;
+        const float share = (float)(tiles * parts) / (float)(rounds * units);
+        float us = (float)rounds * (shape.fixed + (float)each * (shape.slice + shape.crowd * share));
+        if (parts > 1) us += PARTS_FIXED + 2.f * (float)sums / PARTS_BYTES_A_US;
+        if (best.us == 0.f || us < best.us) {
+          best = TilesChoice{t, parts, us, (float)((double)parts * m * n / ((double)rounds * units * shape.bm * shape.bn))};
+        }
+      }
     }
+    return best;
+  };
+  const int counted = few ? FEW_OUTPUTS : n;
+  TilesChoice best = least(counted, whole ? 1 : 8);
+  if (streams && best.splits > 1) {
+    const TilesChoice undivided = least(counted, 1);
+    if (undivided.us <= STREAM_GAIN * best.us) best = undivided;
   }
-  return best;
+  return few && best.splits == 1 ? least(n, 1) : best;            // (a sum's bits are the parts' alone: undivided, fewer outputs may take smaller tiles)
 }
 
 void launch_tiles(const TilesChoice& choice, void* out, int form, const bf16* x, const bf16* w, int m, int n, int k, int lda, int ldc, hipStream_t s) {

@@ -30,7 +30,7 @@ def test_few_outputs_of_many_rows(m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k", [(65, 4, 32), (70, 64, 224), (129, 12, 96), (100, 16, 64), (300, 20, 1056), (257, 36, 2016), (2048, 32, 4096), (2048, 64, 2048), (1000, 8, 544),
-                                   (4095, 16, 4096), (4096, 16, 2048), (4096, 64, 4096), (4097, 4, 1024), (6000, 32, 8192), (5003, 8, 4160)])
+                                   (4095, 16, 4096), (4096, 16, 2048), (4096, 64, 4096), (4097, 4, 1024), (6000, 32, 8192), (5003, 8, 4160), (5003, 8, 28672), (16400, 12, 8192)])
 def test_few_outputs_have_the_bits_of_many(m, n, k):
     """A row's outputs are the same whether its weight rows stand alone or among more than one such kernel takes."""
     from llm_runtime_study_amd.kernels import ops
