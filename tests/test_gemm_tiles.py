@@ -1,5 +1,7 @@
 """bfloat16 products of many rows in tiles: the choice of tile and parts, registers, and every tile at its edges."""
 
+import itertools
+
 import pytest
 import torch
 
@@ -26,10 +28,15 @@ def test_the_choice_of_tile_and_parts():
         assert ops.gemm_tiles_choice(2048, 24576, 4096) == (256, 256, 1) and ops.gemm_tiles_choice(512, 19456, 2560) == (256, 160, 1)
         # few outputs: divided from 4,096 rows on, where a router's own kernel has more than a round of the chip, all up to 128 alike
         assert ops.gemm_tiles_choice(4096, 64, 8192)[2] > 1 and ops.gemm_tiles_choice(8192, 8, 8192)[2] > 1 and ops.gemm_tiles_choice(4095, 64, 8192)[2] == 1
-        assert all(ops.gemm_tiles_choice(m, n, k) == ops.gemm_tiles_choice(m, 128, k) for m in (4096, 5000, 16384) for n in (8, 64, 100) for k in (512, 2048, 8192))
-        # what streams from memory is not divided
+        for m, n, k in itertools.product((4096, 5000, 16384, 20000), (8, 64, 100), (512, 2048, 8192, 28672)):
+            mine, all_of_them = ops.gemm_tiles_choice(m, n, k), ops.gemm_tiles_choice(m, 128, k)
+            assert mine == all_of_them or mine[2] == all_of_them[2] == 1           # divided: the same tile too, whose slices the parts begin at
+        # rows that stream from memory: no parts a multiple of 4 KB apart, no parts for less than a tenth, others as ever
         assert ops.gemm_tiles_choice(16384, 256, 8192) == (128, 128, 1) and ops.gemm_tiles_choice(32768, 192, 8192) == (128, 192, 1)
-        assert ops.gemm_tiles_choice(8192, 256, 8192)[2] > 1
+        assert ops.gemm_tiles_choice(28000, 128, 5120)[2] == 1 and ops.gemm_tiles_choice(16384, 8, 8192) == (64, 64, 1)
+        assert [ops.gemm_tiles_choice(m, n, k)[2] for m, n, k in ((17000, 192, 8192), (5000, 192, 28672), (5000, 8, 28672), (8192, 256, 8192))] == [3, 6, 6, 4]
+        # weights that the cache does not hold are divided like any
+        assert ops.gemm_tiles_choice(129, 8192, 28672) == (256, 256, 8) and ops.gemm_tiles_choice(256, 5120, 27648) == (256, 160, 8)
         assert ops.gemm_tiles_choice(256, 1024, 1024) == (64, 64, 1) and ops.gemm_tiles_choice(512, 4096, 12288)[2] > 1
 
 
