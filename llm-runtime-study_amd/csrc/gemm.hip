@@ -1647,22 +1647,30 @@ LRS_API int lrs_gemm_split_pays(int m, int n, int k) {
 // faster than the vendor library and a kernel for what follows, for a product of more than 128 rows.  form: what follows.
 //   0  nothing (stored as bf16): up to 256 rows.  us of the tiles / the library at 256 rows: 0.6B q/k/v 8.2 / 9.7, 1.7B 11.5 / 11.3, 4B 17.4 / 24.8,
 //      8B 28.3 / 41.4, 14B 39.2 / 52.1; at 384 to 2,048 rows between a tenth slower and a twentieth faster (4B 384 23.6 / 21.7, 8B 1,536 65.8 / 70.0).
-//   1  the gated activation: always.  512 rows 0.6B 15.1 / 18.3, 1.7B 31.9 / 35.8, 4B 51.4 / 60.2, 8B 81.7 / 89.6, 14B 179 / 193; 2,048 rows 29.4 / 35.4,
-//      92 / 102, 189 / 218, 299 / 314, 579 / 627.
-//   2  the residual add and a norm: a K of twice the width (more than 1,024 wide), or up to 512 rows where K is divided.  Down 512 rows 1.7B 24.6 /
+//   1  the gated activation: where K is not divided (its parts' sums meet in a kernel of single values: 160 rows of K 4,096, 1,536 outputs 20.3 / 13.4), and beyond
+//      256 rows of 16,384 outputs and more where three fifths of what the chip makes are the product's own (rows that end in a tile: 300 of 28,672 x 4,096
+//      97 / 84, 520 of 16,384 x 2,048 54 / 47).  512 rows 0.6B 15.1 / 18.3, 1.7B 31.9 / 35.8, 4B 51.4 / 60.2, 8B 81.7 / 89.6, 14B 179 / 193; 2,048 rows
+//      29.4 / 35.4, 92 / 102, 189 / 218, 299 / 314, 579 / 627; 3,000 to 16,384 rows 47 / 52 to 205 / 214, 14B 830 / 876 to 3,960 / 4,470.
+//   2  the residual add and a norm: a K of twice the width (more than 1,024 wide; beyond 2,048 rows where three quarters of what the chip makes are its own:
+//      4,096 of K 12,288 3,000 rows 251 / 244, 6,000 548 / 496, 7,000 566 / 600, 12,000 919 / 1,272), or up to 512 rows where K is divided.  Down 512 rows 1.7B 24.6 /
 //      26.0, 4B 39.7 / 53.7, 8B 60.6 / 86.0, 14B 89.9 / 174; 2,048 rows 59.8 / 66.2, 95.8 / 113, 170 / 189, 291 / 303; o at 512 rows 0.6B 13.0 / 14.0,
 //      1.7B 16.7 / 15.8 (not divided), 4B 24.1 / 25.7, 14B 43.8 / 53.2; at 768 8B 44.9 / 40.3.
-//   3  nothing, stored as float32: from 10,240 outputs on.  10,304 outputs of K 4,096 at 256 rows 37 / 49, 512 54 / 54, 1,024 79 / 84, 2,048 145 / 207, of K 2,560 2,048
+//   3  nothing, stored as float32: from 10,240 outputs on, beyond 256 rows where three quarters are its own (32,000 of K 4,096 256 rows 83 / 81, 300 104 / 91,
+//      420 107 / 108, 512 110 / 119, 560 176 / 150, 768 171 / 265, 2,048 407 / 428; 151,936 560 rows 713 / 695, 640 732 / 807).  10,304 outputs of K 4,096 at 256 rows 37 / 49, 512 54 / 54, 1,024 79 / 84, 2,048 145 / 207, of K 2,560 2,048
 //      104 / 105; 12,288 of 2,048 36 / 39 at 768, 28 / 27 at 512; 151,936 of 4,096 513 / 617 at 512, 301 / 305 at 144; 8,192 between a tenth slower and faster.
+// The library's own times jump by a third and more from one size to the next and by a tenth between cards: the lines stand where the mean over 970 products
+// (nine layer sizes and LM heads, 129 to 16,384 rows) is best, form 1 0.90 of the library's time, form 2 0.84, form 3 0.96; single ones are up to a fifth slower.
 // Not at all for a K of less than 512: eight slices are mostly beginnings and ends.
 LRS_API int lrs_gemm_tiles_pay(int m, int n, int k, int form) {
   if (m <= 128 || n <= NARROW_MAX || n % 4 != 0 || k < 512 || k % 64 != 0) return 0;
   if (form == 0) return m <= 256;
-  if (form == 1) return n % 16 == 0;
-  if (form == 3) return n >= 10240;
-  if (form != 2 || n > 8192) return 0;
-  if (k >= 2 * n && n > 1024) return 1;
-  return m <= 512 && choose_tiles(m, n, k, SPLIT_SUMS_BYTES).splits > 1;
+  if (form < 1 || form > 3) return 0;
+  const TilesChoice choice = choose_tiles(m, n, k, SPLIT_SUMS_BYTES);
+  if (form == 1) return n % 16 == 0 && choice.splits == 1 && (m <= 256 || n < 16384 || choice.useful >= 0.6f);
+  if (form == 3) return n >= 10240 && (m <= 256 || choice.useful >= 0.73f);
+  if (n > 8192) return 0;
+  if (k >= 2 * n && n > 1024) return m <= 2048 || choice.useful >= 0.74f;
+  return m <= 512 && choice.splits > 1;
 }
 
 // Defined beside the norm kernels: x += the sum of the splits' sums, then out = RMSNorm(x), one pass over the rows.

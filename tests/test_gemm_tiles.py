@@ -48,6 +48,12 @@ def test_what_goes_to_the_tiles_rather_than_to_the_library():
     assert pay(2048, 24576, 4096, "gate") and pay(129, 6144, 1024, "gate") and not pay(512, 6144, 1056, "gate") and not pay(512, 6152, 1024, "gate")
     assert pay(2048, 4096, 12288, "norm") and not pay(2048, 4096, 4096, "norm") and not pay(300, 64, 4096, "norm") and not pay(300, 8196, 65536, "norm")
     assert not pay(512, 24576, 448, "gate")
+    if ops.compute_units() in (0, 256):
+        # tiles that rows or columns leave half empty: by the library
+        assert [pay(m, 32000, 4096, "nothing, float32") for m in (256, 300, 420, 512, 560, 768, 2048)] == [True, False, True, True, False, True, True]
+        assert [pay(m, 4096, 12288, "norm") for m in (2049, 3000, 3500, 6000, 7000)] == [True, False, True, False, True]
+        assert [pay(m, 28672, 4096, "gate") for m in (129, 256, 300, 512, 2048)] == [True, True, False, True, True] and pay(300, 12288, 2048, "gate")
+        assert not pay(160, 1536, 4096, "gate") and pay(160, 1536, 4096, "nothing")              # divided: the gate behind it is a kernel of single values
     assert pay(300, 10304, 4096, "nothing, float32") and not pay(2048, 8192, 4096, "nothing, float32")
 
 
