@@ -466,18 +466,23 @@ class GQAAttention(Part):
             self._attend(ctx, out, qkv, cache, group)
         return linear(ctx, residual, out, self.w_o, accumulate=accumulate, then_norm=then_norm)
 
-    PIECE_RESULTS = 1 << 25      # floats, 128 MB, that the results of pieces of keys may take before a launch stays undivided
+    # floats, 128 MB, that the results of pieces of keys may take before a launch stays undivided (of the buffers a step keeps, which grow by doubling)
+    PIECE_RESULTS = 1 << 25
 
     @staticmethod
     def _piece_splits(workgroups: int, longest: int) -> int:
         """Into how many workgroups of one wave attention_f32_divided() divides the keys of a row (1: attention(), which gives a row of a kv head a
-        workgroup of eight waves).  Two to a unit are a full chip; more parts than pieces have nothing to do; a class of lengths has one answer.
-        us, kv heads of 128 dims with two query heads each, attention() / divided [parts], merge counted:
-          * up to a workgroup for every four units: 8 at 509 tokens 15.3 / 10.0 [8], at 2,000 51.2 / 14.1 [32], 32 at 509 15.8 / 10.7 [8], at 4,000 112 / 45 [16],
-            64 at 260 15.0 / 14.8 [4], at 509 16.0 / 13.7 [8], at 1,000 28.4 / 21.5 [8], at 4,000 116 / 73 [8]; 64 of 64 dims 11.0 / 10.1 [8] at 509;
-          * up to one for every two units, four parts to a unit over long contexts: 96 at 4,000 125 / 101 [16] and 113 [8], 128 at 4,000 131 / 127 [8], of 64 dims
-            79 / 69 [8]; but 96 at 509 16.7 / 19.7 [8], 128 at 1,000 36.9 / 39.3 [8];
-          * beyond that attention() fills the chip: 256 at 4,000 185 / 237 [8]."""
+        workgroup of eight waves).  A class of lengths has one answer: at most as many parts as the longest of them has pieces (where a row has fewer,
+        some have nothing to do), at most two to a unit, which are a full chip.
+        us, rows of 8 kv heads with two query heads each, attention() / divided into what the rule says [parts], merge counted:
+          * up to a workgroup for every four units, 128 dims: one row at 256 tokens 10.3 / 9.4 [8], at 300 14.2 / 9.4, at 511 14.9 / 9.7, at 700 22.0 / 10.6 [16], at
+            2,000 50.9 / 13.8 [32], at 4,000 99 / 23 [64]; eight at 256 11.0 / 10.0 [8], at 300 14.7 / 11.5, at 511 15.9 / 13.3, at 700 23.1 / 19.7, at 1,000 28.2 / 21.4,
+            at 4,000 116 / 72; 64 dims: one at 256 7.3 / 7.8, at 300 9.4 / 7.9, at 511 9.9 / 8.4, eight at 256 7.8 / 8.1, at 300 9.9 / 8.7, at 4,000 73 / 50 (at 256 itself,
+            four pieces, attention() has one trip; from 257 on two);
+          * up to one for every two units, over long contexts: 12 rows at 4,000 126 / 104 [10], 16 133 / 128 [8], of 64 dims 80 / 70; at 509 and 1,000 tokens 96
+            and 128 workgroups lost by it (16.7 / 19.7, 36.9 / 39.3);
+          * beyond that attention() fills the chip: 256 workgroups at 4,000 185 / 237 [8].
+        One, three and four query heads a kv head take the same times to 0.5 us (16 rows at 4,000 133 / 126, 131 and 133)."""
         units, reach = ops.compute_units(), length_class(longest)
         if reach >= 256 and 4 * workgroups <= units:
             return min(reach // 32, 2 * units // workgroups)
