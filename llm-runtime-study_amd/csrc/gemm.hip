@@ -1646,7 +1646,9 @@ LRS_API int lrs_gemm_split_pays(int m, int n, int k) {
 // Whether the tiles of gemm_tiles.hip, with what follows the product in their epilogue or in the kernel that adds up their parts, are
 // faster than the vendor library and a kernel for what follows, for a product of more than 128 rows.  form: what follows.
 //   0  nothing (stored as bf16): up to 256 rows.  us of the tiles / the library at 256 rows: 0.6B q/k/v 8.2 / 9.7, 1.7B 11.5 / 11.3, 4B 17.4 / 24.8,
-//      8B 28.3 / 41.4, 14B 39.2 / 52.1; at 384 to 2,048 rows between a tenth slower and a twentieth faster (4B 384 23.6 / 21.7, 8B 1,536 65.8 / 70.0).
+//      8B 28.3 / 41.4, 14B 39.2 / 52.1; but from 161 on not where more than 4,096 outputs meet a K of 2,048 to 4,095, but for whole 32s of rows, at which the library
+//      falls back by a third (6,144 of K 2,560, 4B q/k/v: 150 rows 21.5 / 26.7, 160 22.1 / 22.5, 176 22.6 / 19.3, 192 23.2 / 25.1, 200 21.3 / 19.8, 224 22.1 / 29.4, 240 22.8 / 20.7; 6,144 of
+//      K 2,048, 3,072 and 7,680 of K 2,560 likewise; of K 1,536 0.8 throughout, 8B 27.2 / 26.7 at 185, 14B 36.0 / 36.6 at 200); at 384 to 2,048 rows between a tenth slower and a twentieth faster (4B 384 23.6 / 21.7, 8B 1,536 65.8 / 70.0).
 //   1  the gated activation: where K is not divided (its parts' sums meet in a kernel of single values: 160 rows of K 4,096, 1,536 outputs 20.3 / 13.4), and beyond
 //      256 rows of 16,384 outputs and more where three fifths of what the chip makes are the product's own (rows that end in a tile: 300 of 28,672 x 4,096
 //      97 / 84, 520 of 16,384 x 2,048 54 / 47).  512 rows 0.6B 15.1 / 18.3, 1.7B 31.9 / 35.8, 4B 51.4 / 60.2, 8B 81.7 / 89.6, 14B 179 / 193; 2,048 rows
@@ -1663,7 +1665,7 @@ LRS_API int lrs_gemm_split_pays(int m, int n, int k) {
 // Not at all for a K of less than 512: eight slices are mostly beginnings and ends.
 LRS_API int lrs_gemm_tiles_pay(int m, int n, int k, int form) {
   if (m <= 128 || n <= NARROW_MAX || n % 4 != 0 || k < 512 || k % 64 != 0) return 0;
-  if (form == 0) return m <= 256;
+  if (form == 0) return m <= 160 || (m <= 256 && (m % 32 == 0 || n <= 4096 || k < 2048 || k >= 4096));
   if (form < 1 || form > 3) return 0;
   const TilesChoice choice = choose_tiles(m, n, k, SPLIT_SUMS_BYTES);
   if (form == 1) return n % 16 == 0 && choice.splits == 1 && (m <= 256 || n < 16384 || choice.useful >= 0.6f);

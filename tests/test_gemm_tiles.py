@@ -44,6 +44,8 @@ def test_what_goes_to_the_tiles_rather_than_to_the_library():
     from llm_runtime_study_amd.kernels import ops
 
     pay = ops.gemm_tiles_pay
+    assert [pay(m, 6144, 2560, "nothing") for m in (129, 160, 161, 191, 192, 200, 224, 255, 256)] == [True, True, False, False, True, False, True, False, True]
+    assert pay(200, 4096, 2560, "nothing") and pay(200, 6144, 1536, "nothing") and pay(200, 6144, 4096, "nothing")
     assert pay(256, 6144, 4096, "nothing") and not pay(257, 6144, 4096, "nothing") and not pay(128, 6144, 4096, "nothing")
     assert pay(2048, 24576, 4096, "gate") and pay(129, 6144, 1024, "gate") and not pay(512, 6144, 1056, "gate") and not pay(512, 6152, 1024, "gate")
     assert pay(2048, 4096, 12288, "norm") and not pay(2048, 4096, 4096, "norm") and not pay(300, 64, 4096, "norm") and not pay(300, 8196, 65536, "norm")
