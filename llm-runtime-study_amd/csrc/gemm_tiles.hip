@@ -112,8 +112,8 @@ __global__ __launch_bounds__(512, 1) void gemm_bf16_tiles_kernel(const bf16* __r
 // The tiles, and what a launch of them takes: us = rounds of the chip * (fixed + slices of 64 k * (slice + crowd * share of the chip in use)),
 // fitted to 106 to 617 launches of each, at 144 to 2,048 rows of the 0.6B, 1.7B, 4B and 8B layers' products with K in 1 to 8 parts (half
 // of them within 5 %, nine in ten within 12 %; a fuller chip runs slower: its clock).  What the least of these takes is within 0.3 % of
-// the best of all launches on the mean, 6 % at most (weights from memory, 140 to 256 rows of q/k/v and o: 3 % on the mean, 10 % at most).  Outside the fit: 65 to 143
-// rows of nine sizes that the kernels before took in slices of 32 1.1 to 7 times as fast as those; beyond 2,048 rows see lrs_gemm_tiles_pay.  panels: slices of 64 k
+// the best of all launches on the mean, 6 % at most (weights from memory, 140 to 256 rows of q/k/v and o: 4 % on the mean, 13 % at most).  Outside the fit: 65 to 128
+// rows of seven sizes whose K is no multiple of 256, 1.3 to 7 times as fast as in the slices of 32 of gemm_bf16_wide; beyond 2,048 rows see lrs_gemm_tiles_pay.  panels: slices of 64 k
 // a step (K a multiple of so many).  Worked out at every launch that is not recorded: under 1 us of the host.
 struct TileShape { int bm, bn, panels; float fixed, slice, crowd; };
 constexpr TileShape TILES[] = {{256, 256, 1, 12.0f, 0.81f, 0.66f}, {256, 192, 1, 9.7f, 0.69f, 0.51f}, {256, 160, 1, 8.9f, 0.58f, 0.45f},
